@@ -5,6 +5,7 @@
 #include "fm_tok.h"
 #include "fm_norm.h"
 #include "fm_split.h"
+#include "fm_few.h"
 #include "fm_decode.h"
 #include "fm_o1.h"
 #include "fm_pointwise.h"
@@ -622,6 +623,40 @@ int add_rows(const FastmaxDesc* d, const SplitPlan& sp, const void* dqa, void* d
   return fm_launch_status();
 }
 
+// ---- a few queries against many keys (fm_few.h) ----------------------------------------------
+// Forward only, and nothing is left for a backward: a forward that is to keep its workspace takes the general
+// route (causal problems with nk > nq keep nothing there either and come here).
+inline bool is_few(const FastmaxDesc* d) {
+  return fm_few_pays(d->bh, d->nq) && d->d <= 64 && (is_split(d) || !(d->flags & FASTMAX_FLAG_SAVE_FOR_BACKWARD)) &&
+         !(d->flags & (FASTMAX_FLAG_FORCE_MOMENTS | FASTMAX_FLAG_FORCE_DENSE));
+}
+inline size_t few_bytes(const FastmaxDesc* d) {
+  const int s = fm_few_splits(d->bh, d->nq, d->nk);
+  return s > 1 ? align256(size_t(d->bh) * d->nq * s * (d->d + 1) * 4) : 256;
+}
+
+template <typename TIO, int DH>
+int run_few(const FastmaxDesc* d, const void* q, const void* k, const void* v, void* o, float* g, char* ws, fm_stream_t stream) {
+  FewArgs<TIO> a;
+  a.q = cref<TIO>(q, d->sq); a.k = cref<TIO>(k, d->sk); a.v = cref<TIO>(v, d->sv);
+  a.o = mref<TIO>(o, d->so); a.g = mref<float>(g, d->sg);
+  a.nq = d->nq; a.nk = d->nk; a.causal = d->mask != 0;
+  a.a0 = d->a0; a.a1 = d->a1; a.a2 = d->p == 2 ? d->a2 : 0.0f; a.inv_tau = d->inv_tau;
+  a.q_fold = q_fold(d); a.k_fold = k_fold(d);
+  const int splits = fm_few_splits(d->bh, d->nq, d->nk), grp = fm_few_group(d->nq);
+  a.part = splits > 1 ? reinterpret_cast<float*>(ws) : nullptr;
+  const fm_dim3 grid(splits * ((d->nq + grp - 1) / grp), d->bh);
+  ProfScope prof(FM_K_FWD, stream);
+  if (grp == 1) FM_KERNEL_LAUNCH((k_few<TIO, DH, 1>), grid, fm_dim3(FM_THREADS), 0, stream, a, splits);
+  else if (grp == 2) FM_KERNEL_LAUNCH((k_few<TIO, DH, 2>), grid, fm_dim3(FM_THREADS), 0, stream, a, splits);
+  else if (grp == 3) FM_KERNEL_LAUNCH((k_few<TIO, DH, 3>), grid, fm_dim3(FM_THREADS), 0, stream, a, splits);
+  else FM_KERNEL_LAUNCH((k_few<TIO, DH, 4>), grid, fm_dim3(FM_THREADS), 0, stream, a, splits);
+  const int st = fm_launch_status();
+  if (st || splits == 1) return st;
+  FM_KERNEL_LAUNCH((k_few_merge<TIO, DH>), fm_dim3(d->nq, d->bh), fm_dim3(256), 0, stream, a, splits);
+  return fm_launch_status();
+}
+
 }  // namespace
 
 #include "fastmax_api_bwd.inc"
@@ -658,9 +693,26 @@ int fastmax_workspace_bytes(const FastmaxDesc* desc, size_t* forward_bytes, size
     f = p.fwd_bytes; b = p.bwd_bytes;
   }
   if (st) return st;
+  if (is_few(desc)) f = few_bytes(desc);
   if (forward_bytes) *forward_bytes = f;
   if (backward_bytes) *backward_bytes = b;
   return FASTMAX_OK;
+}
+
+static int forward_few(const FastmaxDesc* desc, const void* q, const void* k, const void* v, void* o, float* g,
+                       void* workspace, size_t workspace_bytes, void* hip_stream) {
+  if (!q || !k || !v || !o || !g) return FASTMAX_ERR_NULL;
+  if (!strides_ok(desc->sq, desc->bh, desc->nq, desc->d) || !strides_ok(desc->sk, desc->bh, desc->nk, desc->d) ||
+      !strides_ok(desc->sv, desc->bh, desc->nk, desc->d) || !strides_ok(desc->so, desc->bh, desc->nq, desc->d) ||
+      !strides_ok(desc->sg, desc->bh, desc->nq, 1))
+    return FASTMAX_ERR_SHAPE;
+  if (!workspace || workspace_bytes < few_bytes(desc) || reinterpret_cast<uintptr_t>(workspace) % 256)
+    return FASTMAX_ERR_WORKSPACE;
+  char* ws = static_cast<char*>(workspace);
+  fm_stream_t stream = static_cast<fm_stream_t>(hip_stream);
+  if (desc->dtype == FASTMAX_BF16)
+    return desc->d == 64 ? run_few<fm_bf16, 64>(desc, q, k, v, o, g, ws, stream) : run_few<fm_bf16, 32>(desc, q, k, v, o, g, ws, stream);
+  return desc->d == 64 ? run_few<float, 64>(desc, q, k, v, o, g, ws, stream) : run_few<float, 32>(desc, q, k, v, o, g, ws, stream);
 }
 
 static int forward_one(const FastmaxDesc* desc, const void* q, const void* k, const void* v, void* o, float* g,
@@ -694,6 +746,7 @@ int fastmax_forward(const FastmaxDesc* desc, const void* q, const void* k, const
                     void* workspace, size_t workspace_bytes, void* hip_stream) {
   const int st = validate(desc);
   if (st) return st;
+  if (is_few(desc)) return forward_few(desc, q, k, v, o, g, workspace, workspace_bytes, hip_stream);
   if (!is_split(desc)) return forward_one(desc, q, k, v, o, g, workspace, workspace_bytes, hip_stream);
   // causal with nk > nq: the keys every query sees, then the square causal part, then the merge
   SplitPlan sp;

@@ -69,6 +69,10 @@ FM_DEVICE fm_f32x16 fm_mfma_f32(float a, float b, fm_f32x16 c) {
 }
 FM_DEVICE float fm_shfl_xor(float v, int m) { return hostsim::shfl(v, hostsim::g_t.lane ^ m); }
 FM_DEVICE int fm_shfl_xor_i(int v, int m) { return hostsim::shfl(v, hostsim::g_t.lane ^ m); }
+template <int N> FM_DEVICE float fm_group_sum(float v) {
+  for (int m = 1; m < N; m <<= 1) v += hostsim::shfl(v, hostsim::g_t.lane ^ m);
+  return v;
+}
 FM_DEVICE float fm_dot2(fm_half2 a, fm_half2 b, float c) { return float(a[0]) * float(b[0]) + float(a[1]) * float(b[1]) + c; }
 // Transposing LDS read (ds_read_b64_tr_b16): every lane names four consecutive halves; inside each
 // group of 16 lanes, lane i receives element i % 4 of the words named by lanes i/4, 4 + i/4,
@@ -155,6 +159,18 @@ FM_DEVICE fm_f32x16 fm_mfma_f32(float a, float b, fm_f32x16 c) {
 }
 FM_DEVICE float fm_shfl_xor(float v, int m) { return __shfl_xor(v, m, 64); }
 FM_DEVICE int fm_shfl_xor_i(int v, int m) { return __shfl_xor(v, m, 64); }
+// Sum over groups of N = 4 or 8 consecutive lanes, in every lane of the group: data-parallel-primitive adds (a lane
+// exchange through the LDS pipe, what __shfl_xor compiles to, costs its latency each time).
+template <int N> FM_DEVICE float fm_group_sum(float v) {
+  static_assert(N == 4 || N == 8, "groups of four or eight lanes");
+#define FM_DPP_ADD(ctrl) \
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), (ctrl), 0xf, 0xf, true))
+  FM_DPP_ADD(0xB1);                  // quad_perm [1,0,3,2]
+  FM_DPP_ADD(0x4E);                  // quad_perm [2,3,0,1]
+  if (N == 8) FM_DPP_ADD(0x141);     // row_half_mirror: the other quad of the eight
+#undef FM_DPP_ADD
+  return v;
+}
 FM_DEVICE float fm_dot2(fm_half2 a, fm_half2 b, float c) { return __builtin_amdgcn_fdot2(a, b, c, false); }
 // Transposing LDS read (ds_read_b64_tr_b16): every lane names four consecutive halves; inside each
 // group of 16 lanes, lane i receives element i % 4 of the words named by lanes i/4, 4 + i/4,

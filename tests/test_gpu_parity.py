@@ -248,6 +248,19 @@ def test_causal_more_keys_than_queries(lib, dtype, p, nq, nk):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("d", [32, 64])
+@pytest.mark.parametrize("nq,nk", [(1, 1), (1, 64), (1, 65), (2, 4097), (3, 130), (5, 8192), (16, 16), (64, 64), (64, 1000)])
+def test_few_queries(lib, dtype, d, nq, nk):
+    """The route for a few queries (fm_few.h): group remainders, one part and many parts of the keys, queries that do not
+    see the last keys, unmasked with both normalisation folds."""
+    print(f"case few queries dtype={dtype} d={d} nq={nq} nk={nk}", flush=True)
+    check_forward(lib, 3, nq, d, dtype, DEV, mask=True, p=2, nk=nk, seed=120)
+    check_forward(lib, 2, nq, d, dtype, DEV, mask=False, p=1, nk=nk, seed=121)
+    if nk > 1:                                           # (a single key: dq and dk cancel to zero exactly)
+        check_norm_fold(lib, 2, nq, d, dtype, DEV, mask=False, p=2, nk=nk, seed=122, saved=False)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("jacobian", [True, False])
 def test_normalisation_folded_into_the_loads(lib, dtype, jacobian):
     """lim * x / max-norm of q and k applied as the kernels load the rows (one statistics pass, one read of q and

@@ -153,6 +153,13 @@ def test_causal_with_more_keys_than_queries(sim):
 
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_few_queries(sim, dtype):
+    check_forward(sim, 2, 1, 64, dtype, "cpu", mask=True, p=2, nk=65, seed=24)
+    check_forward(sim, 1, 6, 32, dtype, "cpu", mask=True, p=2, nk=150, seed=25)
+    check_forward(sim, 1, 3, 64, dtype, "cpu", mask=False, p=1, nk=30, seed=26)
+
+
 def test_segment_length_sentinels(sim):
     # a segment length at or beyond the sequence means "one segment", whatever its size; beyond 2^30 it is rejected
     import ctypes as C
