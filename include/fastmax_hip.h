@@ -58,7 +58,9 @@ enum {
  * wrong numbers.  FASTMAX_FLAG_F32_COMPUTE lifts the limits at fp32 speed.  The size of dO is free (the
  * backward rescales dO / g per batch*head to the _Float16 range and back).  The 2e-2 accuracy of this
  * path also rests on weights f(s) that add up without cancelling, as the Taylor weights do (f > 0):
- * with a0 <= 0 the library computes bf16 tensors in fp32 on its own, as if the flag were set. */
+ * with a0 <= 0 the library computes bf16 tensors in fp32 on its own, as if the flag were set.
+ * fp32 tensors: every magnitude of fp32, with the full 24 bits for entries of v and of dO / g above about 1e-34 (below, 16:
+ * the dense tiles form fp32 products from three bf16 parts of each factor). */
 
 /* Where slice i of the batch*head axis, token t, feature f of a tensor lives:
  *   heads <= 1:  i * bh + t * n + f

@@ -10,6 +10,7 @@
 #include "fm_o1.h"
 #include "fm_pointwise.h"
 #include "fm_walk_sym.h"
+#include "fm_x3.h"
 #if defined(FM_BENCH_AIDS)
 #include "fm_bench_aids.h"
 #endif
@@ -113,6 +114,7 @@ struct Plan {
   // workspace offsets (bytes)
   size_t kt, vt, kr, vr, big, big2, small, run, runh, ores, fwd_bytes;
   bool keep_resid;      // the forward leaves o - bf16(o) for the backward (see TokArgs::out_resid)
+  bool x3;              // fp32 arithmetic without states: the kernels of fm_x3.h (read the caller's tensors, no copies)
   bool sym;             // order-2 states are built by the walk per value column (k_walk_sym): one layout, no transposed copy   // run, runh: see k_o1_sums
   bool save;
   size_t b_kr, b_vr, b_qr, b_kt, b_vt, b_qt, b_qct, b_gh, b_ght, b_cv, b_bigq, b_smallq, b_bigk, b_smallk, b_bigv, b_gpart, b_bq, b_bk, b_runq, b_runqh, b_runk, b_runkh, bwd_bytes;
@@ -203,6 +205,7 @@ int make_plan(const FastmaxDesc* d, Plan& p) {
     p.use_state = force_m || (!force_dense && int64_t(d->nk) > int64_t(d->d) * d->d + d->d);
     p.nslots = p.use_state ? 1 : 0;
   }
+  p.x3 = !p.half && !p.use_state;
   p.o1 = p.half && p.use_state && !p.quad && d->mask && p.L == FM_O1_SEG && d->nq == d->nk;
   p.rows_build = p.half && p.use_state && !p.quad && d->mask;
   {
@@ -221,8 +224,8 @@ int make_plan(const FastmaxDesc* d, Plan& p) {
   const size_t bigarr = d->d == 64 ? big_array_bytes<64>(p.esz, p.quad, slots) : big_array_bytes<32>(p.esz, p.quad, slots);
   // fp32 part of a slot: Z and the two vector sums; the order-1 path of fm_o1.h keeps the two vectors only
   const size_t smallsz = p.o1 ? size_t(2) * d->d * 4 : size_t(d->d == 64 ? StateDims<64>::SMALL : StateDims<32>::SMALL) * 4;
-  const size_t tq = p.o1 ? 0 : size_t(d->bh) * d->d * p.npad_q * p.esz;
-  const size_t tk = p.o1 ? 0 : size_t(d->bh) * d->d * p.npad_k * p.esz;
+  const size_t tq = p.o1 || p.x3 ? 0 : size_t(d->bh) * d->d * p.npad_q * p.esz;
+  const size_t tk = p.o1 || p.x3 ? 0 : size_t(d->bh) * d->d * p.npad_k * p.esz;
   size_t off = 0;
   auto take = [&](size_t bytes) { size_t o = off; off = align256(off + bytes); return o; };
   // transposed copies: only the order-2 state walk, the one-total order-1 walk and the fp32 kernels read them
@@ -254,10 +257,10 @@ int make_plan(const FastmaxDesc* d, Plan& p) {
   p.b_bigk = take(bigarr); p.b_smallk = take(size_t(d->bh) * p.nslots * smallsz);
   p.b_bigv = take(p.o1 ? 0 : bigarr);
   p.b_gpart = take(p.half ? size_t(d->bh) * fm_grad_scale_blocks(d->nq) * 4 : 0);   // see k_grad_scale
-  // parts of B = sum dy . y per workgroup of the dQ and dK kernels (128 own tokens at least), see k_norm_fix
+  // parts of B = sum dy . y per workgroup of the dQ and dK kernels (32 own tokens at least), see k_norm_fix
   const bool jac = d->norm.grad != 0;
-  p.b_bq = take(jac && d->norm.q_keys ? size_t(d->bh) * ((d->nq + 127) / 128) * 4 : 0);
-  p.b_bk = take(jac && d->norm.k_keys ? size_t(d->bh) * ((d->nk + 127) / 128) * 4 : 0);
+  p.b_bq = take(jac && d->norm.q_keys ? size_t(d->bh) * ((d->nq + 31) / 32) * 4 : 0);
+  p.b_bk = take(jac && d->norm.k_keys ? size_t(d->bh) * ((d->nk + 31) / 32) * 4 : 0);
   p.b_runq = take(runarr); p.b_runqh = take(runharr); p.b_runk = take(runarr); p.b_runkh = take(runharr);
   p.bwd_bytes = off ? off : 256;
   return FASTMAX_OK;
@@ -490,11 +493,62 @@ int run_forward_o1(const FastmaxDesc* d, const Plan& p, const void* q, const voi
   return fm_launch_status();
 }
 
+// ---- fp32 arithmetic on dense tiles (fm_x3.h) ------------------------------------------------
+// How many wavefronts share an own tile: with one each, a launch has blocks of 128 own tokens (256 for dK + dV); below
+// two workgroups per CU the own tiles are spread over twice or four times as many.
+inline int x3_split(int bh, int n_own, int tokens) {
+  const int blocks = bh * ((n_own + tokens - 1) / tokens);
+  return blocks >= 512 ? 1 : blocks >= 256 ? 2 : 4;
+}
+template <typename TIO> X3Args<TIO> x3_args(const FastmaxDesc* d, const Plan& p, const void* q, const void* k, const void* v) {
+  X3Args<TIO> a;
+  a.q = cref<TIO>(q, d->sq); a.k = cref<TIO>(k, d->sk); a.v = cref<TIO>(v, d->sv);
+  a.o = TRef<const TIO>{nullptr, 0, 0, 0, 0, 0}; a.d_o = a.o; a.out = TRef<TIO>{nullptr, 0, 0, 0, 0, 0}; a.out2 = a.out;
+  a.g = TRef<float>{nullptr, 0, 0, 0, 0, 0};
+  a.cv = nullptr; a.out_resid = nullptr; a.ores = nullptr; a.bpart = nullptr;
+  a.nq = d->nq; a.nk = d->nk; a.npad_q = p.npad_q; a.causal = d->mask != 0;
+  a.a0 = p.a0; a.a1 = p.a1; a.a2 = p.a2; a.sc = p.sc;
+  a.q_fold = q_fold(d); a.k_fold = k_fold(d);
+  return a;
+}
+// KIND 0: forward, 1: dQ, 2: dK + dV
+template <typename TIO, int DH, int KIND, int SPLIT>
+int launch_x3_cfg(const X3Args<TIO>& a, int n_own, int bh, fm_stream_t stream) {
+  typedef X3Cfg<DH, KIND == 2 ? 8 : 4, SPLIT> C;
+  const size_t lds = C::lds(KIND == 2);
+  ProfScope prof(KIND == 0 ? FM_K_FWD : KIND == 1 ? FM_K_DQ : FM_K_DKV, stream);
+  const fm_dim3 grid((n_own + C::QW - 1) / C::QW, bh), block(C::NTH);
+  if constexpr (KIND == 0) {
+    fm_allow_lds(reinterpret_cast<const void*>(&k_x3_fwd<TIO, DH, SPLIT>), lds);
+    FM_KERNEL_LAUNCH((k_x3_fwd<TIO, DH, SPLIT>), grid, block, lds, stream, a);
+  } else if constexpr (KIND == 1) {
+    fm_allow_lds(reinterpret_cast<const void*>(&k_x3_dq<TIO, DH, SPLIT>), lds);
+    FM_KERNEL_LAUNCH((k_x3_dq<TIO, DH, SPLIT>), grid, block, lds, stream, a);
+  } else {
+    fm_allow_lds(reinterpret_cast<const void*>(&k_x3_dkv<TIO, DH, SPLIT>), lds);
+    FM_KERNEL_LAUNCH((k_x3_dkv<TIO, DH, SPLIT>), grid, block, lds, stream, a);
+  }
+  return fm_launch_status();
+}
+template <typename TIO, int DH, int KIND>
+int launch_x3(const X3Args<TIO>& a, int split, int n_own, int bh, fm_stream_t stream) {
+  if (split == 1) return launch_x3_cfg<TIO, DH, KIND, 1>(a, n_own, bh, stream);
+  if (split == 2) return launch_x3_cfg<TIO, DH, KIND, 2>(a, n_own, bh, stream);
+  return launch_x3_cfg<TIO, DH, KIND, 4>(a, n_own, bh, stream);
+}
+
 template <typename TIO, typename E, int DH, int QT>
 int run_forward(const FastmaxDesc* d, const Plan& p, const void* q, const void* k, const void* v, void* o,
                 float* g, char* ws, fm_stream_t stream) {
   if constexpr (sizeof(E) == 2 && DH <= 64) {
     if (p.o1) return run_forward_o1<TIO, DH>(d, p, q, k, v, o, g, ws, stream);
+  } else if constexpr (sizeof(E) == 4) {
+    if (p.x3) {
+      X3Args<TIO> a = x3_args<TIO>(d, p, q, k, v);
+      a.out = mref<TIO>(o, d->so); a.g = mref<float>(g, d->sg);
+      if (p.keep_resid) a.out_resid = reinterpret_cast<fm_half*>(ws + p.ores);
+      return launch_x3<TIO, DH, 0>(a, x3_split(d->bh, d->nq, 128), d->nq, d->bh, stream);
+    }
   }
   E* kt = reinterpret_cast<E*>(ws + p.kt);
   E* vt = reinterpret_cast<E*>(ws + p.vt);

@@ -18,6 +18,8 @@ typedef float fm_f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t fm_u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t fm_u32x2 __attribute__((ext_vector_type(2)));
 typedef uint16_t fm_bf16;  // raw storage of a bfloat16
+typedef uint16_t fm_u16x8 __attribute__((ext_vector_type(8)));   // eight of them: one matrix operand of a lane
+typedef uint16_t fm_u16x4 __attribute__((ext_vector_type(4)));
 
 #if defined(FM_HOSTSIM)
 // ------------------------------------------------------------------ host simulator
@@ -67,6 +69,18 @@ FM_DEVICE fm_f32x16 fm_mfma_f32(float a, float b, fm_f32x16 c) {
   for (int i = 0; i < 16; ++i) c[i] = cv[i];
   return c;
 }
+struct fm_host_bf16 {
+  uint16_t u;
+  operator float() const { const uint32_t w = uint32_t(u) << 16; float f; __builtin_memcpy(&f, &w, 4); return f; }
+};
+FM_DEVICE fm_f32x16 fm_mfma_bf16(fm_u16x8 a, fm_u16x8 b, fm_f32x16 c) {
+  fm_host_bf16 av[8], bv[8]; float cv[16];
+  for (int i = 0; i < 8; ++i) { av[i].u = a[i]; bv[i].u = b[i]; }
+  for (int i = 0; i < 16; ++i) cv[i] = c[i];
+  hostsim::mfma_32x32<fm_host_bf16, 8>(av, bv, cv);
+  for (int i = 0; i < 16; ++i) c[i] = cv[i];
+  return c;
+}
 FM_DEVICE float fm_shfl_xor(float v, int m) { return hostsim::shfl(v, hostsim::g_t.lane ^ m); }
 FM_DEVICE int fm_shfl_xor_i(int v, int m) { return hostsim::shfl(v, hostsim::g_t.lane ^ m); }
 template <int N> FM_DEVICE float fm_group_sum(float v) {
@@ -77,17 +91,19 @@ FM_DEVICE float fm_dot2(fm_half2 a, fm_half2 b, float c) { return float(a[0]) * 
 // Transposing LDS read (ds_read_b64_tr_b16): every lane names four consecutive halves; inside each
 // group of 16 lanes, lane i receives element i % 4 of the words named by lanes i/4, 4 + i/4,
 // 8 + i/4 and 12 + i/4 (layout read off the instruction on an MI355X by a probe kernel).
-FM_DEVICE fm_half4 fm_lds_tr4(const fm_half* p) {
-  fm_half4 w;
+template <typename V4, typename T> inline V4 fm_lds_tr4_any(const T* p) {
+  V4 w;
   __builtin_memcpy(&w, p, 8);
   const int lane = hostsim::g_t.lane, g = lane & ~15, i = lane & 15;
-  fm_half4 r;
+  V4 r;
   for (int t = 0; t < 4; ++t) {
-    const fm_half4 o = hostsim::shfl(w, g + 4 * t + i / 4);
+    const V4 o = hostsim::shfl(w, g + 4 * t + i / 4);
     r[t] = o[i % 4];
   }
   return r;
 }
+FM_DEVICE fm_half4 fm_lds_tr4(const fm_half* p) { return fm_lds_tr4_any<fm_half4>(p); }
+FM_DEVICE fm_u16x4 fm_lds_tr4(const uint16_t* p) { return fm_lds_tr4_any<fm_u16x4>(p); }
 FM_DEVICE float fm_fmaxf(float a, float b) { return a != a ? b : (b != b ? a : (a > b ? a : b)); }   // drops a NaN, like fmaxf
 FM_DEVICE float fm_clampf(float x, float lim) { return x > lim ? lim : (x < -lim ? -lim : x); }
 FM_DEVICE float fm_rsqrtf(float a) { return 1.0f / std::sqrt(a); }
@@ -157,6 +173,12 @@ FM_DEVICE fm_f32x16 fm_mfma_f16(fm_half8 a, fm_half8 b, fm_f32x16 c) {
 FM_DEVICE fm_f32x16 fm_mfma_f32(float a, float b, fm_f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
 }
+FM_DEVICE fm_f32x16 fm_mfma_bf16(fm_u16x8 a, fm_u16x8 b, fm_f32x16 c) {
+  typedef __bf16 fm_bf16x8 __attribute__((ext_vector_type(8)));
+  fm_bf16x8 av, bv;
+  __builtin_memcpy(&av, &a, 16); __builtin_memcpy(&bv, &b, 16);
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, bv, c, 0, 0, 0);
+}
 FM_DEVICE float fm_shfl_xor(float v, int m) { return __shfl_xor(v, m, 64); }
 FM_DEVICE int fm_shfl_xor_i(int v, int m) { return __shfl_xor(v, m, 64); }
 // Sum over groups of N = 4 or 8 consecutive lanes, in every lane of the group: data-parallel-primitive adds (a lane
@@ -182,6 +204,13 @@ FM_DEVICE fm_half4 fm_lds_tr4(const fm_half* p) {
   __builtin_memcpy(&r, &v, 8);
   return r;
 }
+FM_DEVICE fm_u16x4 fm_lds_tr4(const uint16_t* p) {
+  typedef short fm_s16x4 __attribute__((ext_vector_type(4)));
+  const fm_s16x4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) fm_s16x4*)(p));
+  fm_u16x4 r;
+  __builtin_memcpy(&r, &v, 8);
+  return r;
+}
 FM_DEVICE float fm_fmaxf(float a, float b) { return fmaxf(a, b); }
 // clamp to [-lim, lim] in one instruction (v_med3_f32)
 FM_DEVICE float fm_clampf(float x, float lim) { return __builtin_amdgcn_fmed3f(x, -lim, lim); }
@@ -203,3 +232,17 @@ FM_DEVICE fm_bf16 fm_f32_to_bf16(float f) {
   u += 0x7fffu + ((u >> 16) & 1u);
   return fm_bf16(u >> 16);
 }
+// two floats -> two bfloat16 (round to nearest even) in one register, the first in the low half
+FM_DEVICE uint32_t fm_cvt_pk_bf16(float a, float b) {
+#if defined(FM_HOSTSIM)
+  return uint32_t(fm_f32_to_bf16(a)) | (uint32_t(fm_f32_to_bf16(b)) << 16);
+#else
+  typedef __bf16 fm_bf16x2 __attribute__((ext_vector_type(2)));
+  const fm_f32x2 v = {a, b};
+  const fm_bf16x2 h = __builtin_convertvector(v, fm_bf16x2);   // v_cvt_pk_bf16_f32
+  uint32_t u;
+  __builtin_memcpy(&u, &h, 4);
+  return u;
+#endif
+}
+FM_DEVICE float fm_bits_f32(uint32_t u) { float f; __builtin_memcpy(&f, &u, 4); return f; }

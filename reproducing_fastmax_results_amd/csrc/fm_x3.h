@@ -1,0 +1,574 @@
+// Dense fp32 attention on the bf16 matrix pipes, at fp32 accuracy.
+//
+// An fp32 number is the exact sum of three bfloat16 numbers, x = h + m + l: h is x rounded to 8 bits, m what is left
+// rounded to 8 bits, l the rest (24 significant bits in all, each remainder formed exactly in fp32; bf16 has fp32's
+// exponents, so nothing overflows).  A product of two such numbers is taken as
+//     h h + (h m + m h) + (m m + h l + l h),
+// six v_mfma_f32_32x32x16_bf16 with fp32 accumulation; the three products left out are below 2^-26 of |x y|, less than
+// the 2^-24 of one fp32 rounding, and the pipe's rate is 16 / 6 of the fp32 instruction's.  N = 4096, D = 64, causal,
+// relative error of o, dq, dk, dv against 64-bit results: v_mfma_f32_32x32x2_f32 3.9e-7, 4.7e-7, 4.8e-7, 4.0e-7; here 3.6e-7,
+// 4.4e-7, 3.4e-7, 2.8e-7 (a sixth of the accumulator's roundings are fp32-sized, sixteen products to each).  Times at
+// B*H = 32: forward 711 -> 370 us, dQ 1040 -> 520, dK and dV 1760 (two launches) -> 780, and the copies of 80 us are gone.
+// The lowest plane of a number below 2^-110 (1e-33) lies under bf16's smallest normal number and is lost to the matrix
+// instruction's flush: such entries keep 16 bits (1e-36: 3e-5), and everything from 1e-34 up all 24.
+//
+// Three kernels for problems without moment states: the forward, dQ (which first makes c = (dO / g) . o of its queries
+// and leaves it for the next), dK and dV in one pass.  All read the caller's tensors; rows are scaled and split into
+// the three planes on their way from registers to LDS, so nothing is converted in memory beforehand.
+//
+// A wavefront holds a tile of 32 own tokens (its fragments split once, in registers) and multiplies it with 32-token
+// tiles of the other side staged in LDS as rows of three planes; transposed fragments come from transposing LDS reads.
+// SPLIT: how many wavefronts share an own tile, each taking every SPLIT-th stream tile of a stage; their sums meet in
+// LDS in a fixed order.  1 gives the fewest bytes per product, 2 and 4 spread a problem with few own tiles over more
+// workgroups and wavefronts (see x3_split).
+// What bounds them is the matrix pipe and the vector work beside it: per 32 x 32 tile pair and wavefront (D = 64) the
+// forward issues 48 matrix instructions (1536 cycles) and about 140 vector instructions for the weights and their split.
+#pragma once
+#include "fm_kernels.h"
+#include "fm_tok.h"
+
+struct X3 { fm_u16x8 p[3]; };                          // eight numbers as three bf16 planes: h, m, l
+
+// Splits eight floats (or eight accumulator entries).
+FM_DEVICE X3 fm_x3_split(const float v[8]) {
+  fm_u32x4 w[3];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    float a = v[2 * i], b = v[2 * i + 1];
+#pragma unroll
+    for (int pl = 0; pl < 3; ++pl) {
+      const uint32_t u = fm_cvt_pk_bf16(a, b);
+      w[pl][i] = u;
+      a -= fm_bits_f32(u << 16);
+      b -= fm_bits_f32(u & 0xffff0000u);
+    }
+  }
+  X3 r;
+#pragma unroll
+  for (int pl = 0; pl < 3; ++pl) __builtin_memcpy(&r.p[pl], &w[pl], 16);
+  return r;
+}
+FM_DEVICE X3 fm_x3_split_acc(const fm_f32x16& s, int half) {
+  float v[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) v[i] = s[8 * half + i];
+  return fm_x3_split(v);
+}
+// small terms first
+static constexpr int FM_X3_TERMS = 6;
+FM_DEVICE constexpr int fm_x3_pa(int t) { return t == 0 ? 2 : t == 1 ? 0 : t == 2 ? 1 : t == 3 ? 1 : 0; }
+FM_DEVICE constexpr int fm_x3_pb(int t) { return t == 0 ? 0 : t == 1 ? 2 : t == 2 ? 1 : t == 3 ? 0 : t == 4 ? 1 : 0; }
+FM_DEVICE fm_f32x16 fm_x3_mma(const X3& a, const X3& b, fm_f32x16 c) {
+#pragma unroll
+  for (int t = 0; t < FM_X3_TERMS; ++t) c = fm_mfma_bf16(a.p[fm_x3_pa(t)], b.p[fm_x3_pb(t)], c);
+  return c;
+}
+
+template <int DH> struct X3Row {
+  static constexpr int PQ = 3 * DH + 8;                // pitch of a staged row: three planes and 16 bytes of padding
+  static FM_DEVICE X3 load(const uint16_t* p) {        // fragment of a row tile (p: the lane's row and features)
+    X3 f;
+#pragma unroll
+    for (int pl = 0; pl < 3; ++pl) f.p[pl] = *reinterpret_cast<const fm_u16x8*>(p + pl * DH);
+    return f;
+  }
+  // transposed fragment: see Mma<fm_half>::load_tr
+  static FM_DEVICE X3 load_tr(const uint16_t* tile, int tok0, int col0, int lane) {
+    const int lh = lane >> 5, half16 = (lane >> 4) & 1, s = (lane & 15) >> 2, q = lane & 3;
+    const uint16_t* p = tile + (tok0 + 4 * lh + s) * PQ + col0 + 16 * half16 + 4 * q;
+    X3 f;
+#pragma unroll
+    for (int pl = 0; pl < 3; ++pl) {
+      const fm_u16x4 lo = fm_lds_tr4(p + pl * DH), hi = fm_lds_tr4(p + pl * DH + 8 * PQ);
+      fm_u16x8 r = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+      f.p[pl] = r;
+    }
+    return f;
+  }
+  static FM_DEVICE void store(uint16_t* p, const X3& f) {
+#pragma unroll
+    for (int pl = 0; pl < 3; ++pl) *reinterpret_cast<fm_u16x8*>(p + pl * DH) = f.p[pl];
+  }
+};
+
+template <typename TIO> struct X3Args {
+  TRef<const TIO> q, k, v, o, d_o;
+  TRef<float> g;                        // written by the forward, read by the backward
+  TRef<TIO> out, out2;                  // o | dq | dk and dv
+  float* cv;                            // [bh][npad_q] c per query: written by dQ, read by dK + dV
+  fm_half* out_resid; const fm_half* ores;   // bf16 tensors computed in fp32: what rounding takes from o (see TokArgs)
+  int nq, nk, npad_q, causal;
+  float a0, a1, a2, sc;                 // sc = sqrt(1/tau), on q and on k
+  NormFold q_fold, k_fold;
+  float* bpart;                         // the Jacobian's partial sums (see TokArgs::bpart), or null
+};
+
+// Stage of ROWS stream rows of two tensors: caller's rows -> registers -> LDS planes.
+template <typename TIO, int DH, int ROWS, int NTH> struct X3Stage {
+  static constexpr int CPR = DH / 8, PER = ROWS * CPR, TOT = 2 * PER, N = (TOT + NTH - 1) / NTH;
+  float r[N][8];
+  float gi[N];
+  // gb: y rows are divided by g (null: not)
+  FM_DEVICE void load(const TRef<const TIO>& x, const TRef<const TIO>& y, const TRef<float>* g, int bh, int row0, int n, int tid) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const int c = tid + NTH * i;
+      if (TOT % NTH != 0 && c >= TOT) break;
+      const bool second = c >= PER;                    // the same for a whole wavefront: PER is a multiple of 64
+      const int cc = second ? c - PER : c, row = row0 + cc / CPR, col = (cc % CPR) * 8;
+      gi[i] = 1.0f;
+      if (row >= 0 && row < n) {
+        const TRef<const TIO>& t = second ? y : x;
+        IO<TIO>::ld8(t.base(bh) + int64_t(row) * t.s_n + col, t.vec != 0, r[i]);
+        if (g && second) gi[i] = g->base(bh)[int64_t(row) * g->s_n];
+      } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) r[i][j] = 0.f;
+      }
+    }
+  }
+  FM_DEVICE void store(uint16_t* X, uint16_t* Y, float xs, bool div, int tid) const {
+    constexpr int PQ = X3Row<DH>::PQ;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const int c = tid + NTH * i;
+      if (TOT % NTH != 0 && c >= TOT) break;
+      const bool second = c >= PER;
+      const int cc = second ? c - PER : c;
+      const float f = second ? (div ? 1.0f / gi[i] : 1.0f) : xs;
+      float w[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) w[j] = r[i][j] * f;
+      X3Row<DH>::store((second ? Y : X) + (cc / CPR) * PQ + (cc % CPR) * 8, fm_x3_split(w));
+    }
+  }
+};
+
+// Block of own tokens and batch*head of a workgroup: heaviest blocks first (late queries, early keys under the causal
+// mask); with a multiple of eight batch*heads all blocks of one run behind one L2, dealt as in TokGeom.
+FM_DEVICE void fm_x3_place(bool late_first, int& blk, int& bh) {
+  const int nblk = FM_GDIM_X, nbh = FM_GDIM_Y, id = FM_BID_X + nblk * FM_BID_Y;
+  int unit;
+  if ((nbh & 7) == 0) {
+    const int nb = nbh >> 3, rank = fm_snake_rank(id >> 3, nblk * nb);
+    unit = rank / nb;
+    bh = (id & 7) + 8 * (rank % nb);
+  } else {
+    unit = id / nbh;
+    bh = id % nbh;
+  }
+  blk = late_first ? nblk - 1 - unit : unit;
+}
+
+// rows of the stream tile (starting at s0) that the lane's own token (lo + lr) may see
+template <int OWN> FM_DEVICE void fm_x3_window(fm_f32x16& p, bool causal, int s0, int lo, int lr, int lh, int n_str) {
+  int wlo, whi;
+  fm_tile_window<OWN>(causal, s0, lo, lr, n_str, wlo, whi);
+#pragma unroll
+  for (int e = 0; e < 16; ++e) { const int r = fm_acc_row(e, lh); if (r < wlo || r > whi) p[e] = 0.f; }
+}
+
+// Accumulators of all wavefronts -> Os [SPLIT][QW][DH + 4], rows summed over the SPLIT parts by x3_sum8.
+template <int DH, int QW>
+FM_DEVICE void fm_x3_put(const fm_f32x16* acc, float* Os, int sub, int row, int lh) {
+  constexpr int OP = DH + 4;
+#pragma unroll
+  for (int ct = 0; ct < DH / 32; ++ct)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const fm_f32x4 w = {acc[ct][4 * g], acc[ct][4 * g + 1], acc[ct][4 * g + 2], acc[ct][4 * g + 3]};
+      *reinterpret_cast<fm_f32x4*>(Os + (sub * QW + row) * OP + 32 * ct + fm_acc_row(4 * g, lh)) = w;
+    }
+}
+template <int DH, int QW, int SPLIT> FM_DEVICE void fm_x3_sum8(const float* Os, int row, int col, float v[8]) {
+  constexpr int OP = DH + 4;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) v[i] = 0.f;
+#pragma unroll
+  for (int s = 0; s < SPLIT; ++s) {
+    const float* p = Os + (s * QW + row) * OP + col;
+    const fm_f32x4 a = *reinterpret_cast<const fm_f32x4*>(p), b = *reinterpret_cast<const fm_f32x4*>(p + 4);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) { v[i] += a[i]; v[4 + i] += b[i]; }
+  }
+}
+// Gradient rows of the workgroup -> caller's tensor, times scale.  bout: the sum of stored value times raw row (the
+// normalisation's B: stored = fac dy, y = fac x, so dy . y = stored . x), one float per workgroup, or null.
+template <typename TIO, int DH, int QW, int SPLIT, int NTH>
+FM_DEVICE void fm_x3_store(const fm_f32x16* acc, float* Os, int sub, int row, int lh, float scale, const TRef<TIO>& out,
+                           int bh, int t0, int n, int tid, const TRef<const TIO>& raw, float* bout) {
+  FM_SYNC();                                           // whatever lay there has been read
+  fm_x3_put<DH, QW>(acc, Os, sub, row, lh);
+  FM_SYNC();
+  float bsum = 0.f;
+  for (int c = tid; c < QW * (DH / 8); c += NTH) {
+    const int r = c / (DH / 8), col = (c % (DH / 8)) * 8;
+    if (t0 + r >= n) continue;
+    float v[8];
+    fm_x3_sum8<DH, QW, SPLIT>(Os, r, col, v);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] *= scale;
+    if (bout) {
+      float x[8];
+      IO<TIO>::ld8(raw.base(bh) + int64_t(t0 + r) * raw.s_n + col, raw.vec != 0, x);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) bsum += v[i] * x[i];
+    }
+    IO<TIO>::st8(out.base(bh) + int64_t(t0 + r) * out.s_n + col, out.vec != 0, v);
+  }
+  if (bout) {
+#pragma unroll
+    for (int m = 1; m < 64; m <<= 1) bsum += fm_shfl_xor(bsum, m);
+    FM_SYNC();
+    if ((tid & 63) == 0) Os[tid >> 6] = bsum;
+    FM_SYNC();
+    if (tid == 0) {
+      float b = 0.f;
+      for (int w = 0; w < NTH / 64; ++w) b += Os[w];
+      *bout = b;
+    }
+  }
+}
+
+template <int DH, int NW, int SPLIT> struct X3Cfg {
+  static constexpr int NTH = 64 * NW, OT = NW / SPLIT, QW = 32 * OT, KT = 32 * SPLIT, PQ = X3Row<DH>::PQ;
+  static constexpr int STAGE = 2 * KT * PQ;            // u16 elements of one stage buffer
+  static constexpr int NBUF = 2 * STAGE * 2 <= 112 * 1024 ? 2 : 1;
+  static constexpr size_t OS = size_t(SPLIT) * QW * (DH + 4) * 4 + size_t(SPLIT) * QW * 4;
+  // kind 0: forward, dQ; 1: dK + dV (own v rows and the stages' c values as well)
+  static constexpr size_t lds(int kind) {
+    const size_t a = size_t(NBUF) * STAGE * 2 + (kind ? size_t(QW) * PQ * 2 + size_t(NBUF) * KT * 4 : 0);
+    return a > OS ? a : OS;
+  }
+  static constexpr int OCC = NW == 8 || NBUF == 1 || 2 * (NBUF * STAGE * 2) > 150 * 1024 ? NW / 4 : 2;   // wavefronts per SIMD
+};
+
+// ------------------------------------------------------------------------------
+// forward.  grid (ceil(nq / QW), bh), 256 threads.
+// ------------------------------------------------------------------------------
+template <typename TIO, int DH, int SPLIT>
+FM_GLOBAL void FM_LAUNCH_BOUNDS2(256, (X3Cfg<DH, 4, SPLIT>::OCC)) k_x3_fwd(X3Args<TIO> A) {
+  typedef X3Cfg<DH, 4, SPLIT> C;
+  typedef X3Row<DH> R;
+  constexpr int NT = DH / 32, NKS = DH / 16, PQ = C::PQ, KT = C::KT, QW = C::QW;
+  FM_DYN_SMEM(smem);
+  uint16_t* st = reinterpret_cast<uint16_t*>(smem);
+  const int tid = FM_TID_X, lane = tid & 63, lr = lane & 31, lh = lane >> 5;
+  const int wave = FM_UNIFORM(tid >> 6), own = wave / SPLIT, sub = wave % SPLIT;
+  const bool causal = A.causal != 0;
+  int blk, bh;
+  fm_x3_place(causal, blk, bh);
+  const int t0 = blk * QW, lo = t0 + 32 * own;
+  const float qs = A.sc * fm_norm_factor(A.q_fold, bh, lane), ks_ = A.sc * fm_norm_factor(A.k_fold, bh, lane);
+  const int send = causal && t0 + QW < A.nk ? t0 + QW : A.nk;
+  X3Stage<TIO, DH, KT, C::NTH> sg;
+  sg.load(A.k, A.v, nullptr, bh, 0, A.nk, tid);
+  X3 of[NKS];
+  {
+    const bool in = lo + lr < A.nq;
+    const TIO* qr = A.q.base(bh) + int64_t(in ? lo + lr : A.nq - 1) * A.q.s_n + lh * 8;
+#pragma unroll
+    for (int ks = 0; ks < NKS; ++ks) {
+      float v[8];
+      IO<TIO>::ld8(qr + 16 * ks, A.q.vec != 0, v);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v[i] = in ? v[i] * qs : 0.f;
+      of[ks] = fm_x3_split(v);
+    }
+  }
+  fm_f32x16 acc[NT];
+#pragma unroll
+  for (int ct = 0; ct < NT; ++ct) acc[ct] = fm_zero16();
+  float gs = 0.f;
+  int buf = 0;
+  if (C::NBUF == 2) {
+    sg.store(st, st + KT * PQ, ks_, false, tid);
+    sg.load(A.k, A.v, nullptr, bh, KT, A.nk, tid);
+  }
+  for (int s0 = 0; s0 < send; s0 += KT) {
+    uint16_t* X = st + buf * C::STAGE;
+    uint16_t* Y = X + KT * PQ;
+    if (C::NBUF == 1) sg.store(X, Y, ks_, false, tid);
+    FM_SYNC();
+    if (C::NBUF == 1) sg.load(A.k, A.v, nullptr, bh, s0 + KT, A.nk, tid);
+    const int ss0 = s0 + 32 * sub;
+    if (ss0 < A.nk && !(causal && ss0 > lo + 31)) {
+      fm_f32x16 s = fm_zero16();
+#pragma unroll
+      for (int ks = 0; ks < NKS; ++ks) s = fm_x3_mma(R::load(X + (32 * sub + lr) * PQ + 16 * ks + 8 * lh), of[ks], s);
+#pragma unroll
+      for (int e = 0; e < 16; ++e) s[e] = A.a0 + s[e] * (A.a1 + A.a2 * s[e]);
+      if (fm_tile_edge<FM_OWN_Q>(causal, ss0, lo, A.nk)) { FM_KEEP_BRANCH(); fm_x3_window<FM_OWN_Q>(s, causal, ss0, lo, lr, lh, A.nk); }
+#pragma unroll
+      for (int e = 0; e < 16; ++e) gs += s[e];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const X3 pb = fm_x3_split_acc(s, h);
+        X3 zf[NT];
+#pragma unroll
+        for (int ct = 0; ct < NT; ++ct) zf[ct] = R::load_tr(Y, 32 * sub + 16 * h, 32 * ct, lane);
+#pragma unroll
+        for (int t = 0; t < FM_X3_TERMS; ++t)
+#pragma unroll
+          for (int ct = 0; ct < NT; ++ct) acc[ct] = fm_mfma_bf16(zf[ct].p[fm_x3_pa(t)], pb.p[fm_x3_pb(t)], acc[ct]);
+      }
+    }
+    if (C::NBUF == 2) {
+      buf ^= 1;
+      if (s0 + KT < send) {
+        sg.store(st + buf * C::STAGE, st + buf * C::STAGE + KT * PQ, ks_, false, tid);
+        sg.load(A.k, A.v, nullptr, bh, s0 + 2 * KT, A.nk, tid);
+      }
+    } else FM_SYNC();
+  }
+  float* Os = reinterpret_cast<float*>(smem);
+  float* Gs = Os + SPLIT * QW * (DH + 4);              // [SPLIT][QW]
+  FM_SYNC();
+  fm_x3_put<DH, QW>(acc, Os, sub, 32 * own + lr, lh);
+  gs += fm_shfl_xor(gs, 32);
+  if (lh == 0) Gs[sub * QW + 32 * own + lr] = gs;
+  FM_SYNC();
+  for (int c = tid; c < QW * (DH / 8); c += C::NTH) {
+    const int r = c / (DH / 8), col = (c % (DH / 8)) * 8, qi = t0 + r;
+    if (qi >= A.nq) continue;
+    float v[8], gt = 0.f;
+    fm_x3_sum8<DH, QW, SPLIT>(Os, r, col, v);
+#pragma unroll
+    for (int s = 0; s < SPLIT; ++s) gt += Gs[s * QW + r];
+    const float gi = 1.0f / gt;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] *= gi;
+    IO<TIO>::st8(A.out.base(bh) + int64_t(qi) * A.out.s_n + col, A.out.vec != 0, v);
+    if (A.out_resid) {
+      float sv[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) sv[i] = fm_as_stored<TIO>(v[i]);
+      fm_store_resid8(A.out_resid + (int64_t(bh) * A.npad_q + qi) * DH + col, v, sv);
+    }
+    if (col == 0) A.g.base(bh)[int64_t(qi) * A.g.s_n] = gt;
+  }
+}
+
+// ------------------------------------------------------------------------------
+// dQ.  grid (ceil(nq / QW), bh), 256 threads.  dS = (a1 + 2 a2 s) (gh . v - c), gh = dO / g, c = gh . o.
+// ------------------------------------------------------------------------------
+template <typename TIO, int DH, int SPLIT>
+FM_GLOBAL void FM_LAUNCH_BOUNDS2(256, (X3Cfg<DH, 4, SPLIT>::OCC)) k_x3_dq(X3Args<TIO> A) {
+  typedef X3Cfg<DH, 4, SPLIT> C;
+  typedef X3Row<DH> R;
+  constexpr int NT = DH / 32, NKS = DH / 16, PQ = C::PQ, KT = C::KT, QW = C::QW;
+  FM_DYN_SMEM(smem);
+  uint16_t* st = reinterpret_cast<uint16_t*>(smem);
+  const int tid = FM_TID_X, lane = tid & 63, lr = lane & 31, lh = lane >> 5;
+  const int wave = FM_UNIFORM(tid >> 6), own = wave / SPLIT, sub = wave % SPLIT;
+  const bool causal = A.causal != 0;
+  int blk, bh;
+  fm_x3_place(causal, blk, bh);
+  const int t0 = blk * QW, lo = t0 + 32 * own;
+  const float qf = fm_norm_factor(A.q_fold, bh, lane), qs = A.sc * qf, ks_ = A.sc * fm_norm_factor(A.k_fold, bh, lane);
+  const int send = causal && t0 + QW < A.nk ? t0 + QW : A.nk;
+  X3Stage<TIO, DH, KT, C::NTH> sg;
+  sg.load(A.k, A.v, nullptr, bh, 0, A.nk, tid);
+  X3 of[NKS], of2[NKS];
+  float cs = 0.f;
+  {
+    const bool in = lo + lr < A.nq;
+    const int64_t row = in ? lo + lr : A.nq - 1;
+    const float ginv = in ? 1.0f / A.g.base(bh)[row * A.g.s_n] : 0.f;
+#pragma unroll
+    for (int ks = 0; ks < NKS; ++ks) {
+      const int f = 16 * ks + 8 * lh;
+      float v[8], w[8], o[8];
+      IO<TIO>::ld8(A.q.base(bh) + row * A.q.s_n + f, A.q.vec != 0, v);
+      IO<TIO>::ld8(A.d_o.base(bh) + row * A.d_o.s_n + f, A.d_o.vec != 0, w);
+      IO<TIO>::ld8(A.o.base(bh) + row * A.o.s_n + f, A.o.vec != 0, o);
+      if (A.ores) {
+        const fm_half8 rs = *reinterpret_cast<const fm_half8*>(A.ores + (int64_t(bh) * A.npad_q + row) * DH + f);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) o[i] += float(rs[i]);
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) { v[i] = in ? v[i] * qs : 0.f; w[i] = in ? w[i] * ginv : 0.f; cs += w[i] * o[i]; }
+      of[ks] = fm_x3_split(v);
+      of2[ks] = fm_x3_split(w);
+    }
+    cs += fm_shfl_xor(cs, 32);
+    if (sub == 0 && lh == 0 && in) A.cv[int64_t(bh) * A.npad_q + row] = cs;
+  }
+  const float ta2 = 2.0f * A.a2;
+  fm_f32x16 acc[NT];
+#pragma unroll
+  for (int ct = 0; ct < NT; ++ct) acc[ct] = fm_zero16();
+  int buf = 0;
+  if (C::NBUF == 2) {
+    sg.store(st, st + KT * PQ, ks_, false, tid);
+    sg.load(A.k, A.v, nullptr, bh, KT, A.nk, tid);
+  }
+  for (int s0 = 0; s0 < send; s0 += KT) {
+    uint16_t* X = st + buf * C::STAGE;
+    uint16_t* Y = X + KT * PQ;
+    if (C::NBUF == 1) sg.store(X, Y, ks_, false, tid);
+    FM_SYNC();
+    if (C::NBUF == 1) sg.load(A.k, A.v, nullptr, bh, s0 + KT, A.nk, tid);
+    const int ss0 = s0 + 32 * sub;
+    if (ss0 < A.nk && !(causal && ss0 > lo + 31)) {
+      fm_f32x16 s = fm_zero16(), dp = fm_zero16();
+#pragma unroll
+      for (int ks = 0; ks < NKS; ++ks) {
+        const X3 xf = R::load(X + (32 * sub + lr) * PQ + 16 * ks + 8 * lh), yf = R::load(Y + (32 * sub + lr) * PQ + 16 * ks + 8 * lh);
+#pragma unroll
+        for (int t = 0; t < FM_X3_TERMS; ++t) {
+          s = fm_mfma_bf16(xf.p[fm_x3_pa(t)], of[ks].p[fm_x3_pb(t)], s);
+          dp = fm_mfma_bf16(yf.p[fm_x3_pa(t)], of2[ks].p[fm_x3_pb(t)], dp);
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < 16; ++e) s[e] = (A.a1 + ta2 * s[e]) * (dp[e] - cs);
+      if (fm_tile_edge<FM_OWN_Q>(causal, ss0, lo, A.nk)) { FM_KEEP_BRANCH(); fm_x3_window<FM_OWN_Q>(s, causal, ss0, lo, lr, lh, A.nk); }
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const X3 db = fm_x3_split_acc(s, h);
+        X3 zf[NT];
+#pragma unroll
+        for (int ct = 0; ct < NT; ++ct) zf[ct] = R::load_tr(X, 32 * sub + 16 * h, 32 * ct, lane);
+#pragma unroll
+        for (int t = 0; t < FM_X3_TERMS; ++t)
+#pragma unroll
+          for (int ct = 0; ct < NT; ++ct) acc[ct] = fm_mfma_bf16(zf[ct].p[fm_x3_pa(t)], db.p[fm_x3_pb(t)], acc[ct]);
+      }
+    }
+    if (C::NBUF == 2) {
+      buf ^= 1;
+      if (s0 + KT < send) {
+        sg.store(st + buf * C::STAGE, st + buf * C::STAGE + KT * PQ, ks_, false, tid);
+        sg.load(A.k, A.v, nullptr, bh, s0 + 2 * KT, A.nk, tid);
+      }
+    } else FM_SYNC();
+  }
+  fm_x3_store<TIO, DH, QW, SPLIT, C::NTH>(acc, reinterpret_cast<float*>(smem), sub, 32 * own + lr, lh, A.sc * (A.bpart ? qf : 1.0f), A.out,
+                                          bh, t0, A.nq, tid, A.q, A.bpart ? A.bpart + int64_t(bh) * FM_GDIM_X + blk : nullptr);
+}
+
+// ------------------------------------------------------------------------------
+// dK and dV.  grid (ceil(nk / QW), bh), 512 threads: eight wavefronts share the staged queries, so that two per SIMD
+// leave 256 registers each; own k in registers, own v (read once per tile) in LDS.
+// ------------------------------------------------------------------------------
+template <typename TIO, int DH, int SPLIT>
+FM_GLOBAL void FM_LAUNCH_BOUNDS2(512, 2) k_x3_dkv(X3Args<TIO> A) {
+  typedef X3Cfg<DH, 8, SPLIT> C;
+  typedef X3Row<DH> R;
+  constexpr int NT = DH / 32, NKS = DH / 16, PQ = C::PQ, KT = C::KT, QW = C::QW;
+  FM_DYN_SMEM(smem);
+  uint16_t* Vs = reinterpret_cast<uint16_t*>(smem);    // own v rows [QW][PQ]
+  uint16_t* st = Vs + QW * PQ;
+  float* cst = reinterpret_cast<float*>(st + C::NBUF * C::STAGE);   // c of the staged queries [NBUF][KT]
+  const int tid = FM_TID_X, lane = tid & 63, lr = lane & 31, lh = lane >> 5;
+  const int wave = FM_UNIFORM(tid >> 6), own = wave / SPLIT, sub = wave % SPLIT;
+  const bool causal = A.causal != 0;
+  int blk, bh;
+  fm_x3_place(false, blk, bh);
+  const int t0 = blk * QW, lo = t0 + 32 * own;
+  const float kf = fm_norm_factor(A.k_fold, bh, lane), ks_ = A.sc * kf, qs = A.sc * fm_norm_factor(A.q_fold, bh, lane);
+  const int sbeg = causal ? t0 : 0, nst = (A.nq - sbeg + KT - 1) / KT;
+  const int s_last = sbeg + (nst - 1) * KT;            // the stream is walked from its end: see k_ds
+  X3Stage<TIO, DH, KT, C::NTH> sg;
+  float creg = 0.f;
+  const float* cvb = A.cv + int64_t(bh) * A.npad_q;
+  auto fetch = [&](int s) {
+    sg.load(A.q, A.d_o, &A.g, bh, s, A.nq, tid);
+    const int r = s + tid % KT;
+    creg = r >= 0 && r < A.nq ? cvb[r] : 0.f;
+  };
+  auto put = [&](int b) {
+    uint16_t* X = st + b * C::STAGE;
+    sg.store(X, X + KT * PQ, qs, true, tid);
+    if (tid < KT) cst[b * KT + tid] = creg;
+  };
+  fetch(s_last);
+  for (int c = tid; c < QW * (DH / 8); c += C::NTH) {
+    const int r = c / (DH / 8), col = (c % (DH / 8)) * 8, row = t0 + r;
+    float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    if (row < A.nk) IO<TIO>::ld8(A.v.base(bh) + int64_t(row) * A.v.s_n + col, A.v.vec != 0, v);
+    R::store(Vs + r * PQ + col, fm_x3_split(v));
+  }
+  X3 of[NKS];
+  {
+    const bool in = lo + lr < A.nk;
+    const TIO* kr = A.k.base(bh) + int64_t(in ? lo + lr : A.nk - 1) * A.k.s_n + lh * 8;
+#pragma unroll
+    for (int ks = 0; ks < NKS; ++ks) {
+      float v[8];
+      IO<TIO>::ld8(kr + 16 * ks, A.k.vec != 0, v);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v[i] = in ? v[i] * ks_ : 0.f;
+      of[ks] = fm_x3_split(v);
+    }
+  }
+  const float ta2 = 2.0f * A.a2;
+  fm_f32x16 acc[NT], av[NT];
+#pragma unroll
+  for (int ct = 0; ct < NT; ++ct) { acc[ct] = fm_zero16(); av[ct] = fm_zero16(); }
+  int buf = 0;
+  if (C::NBUF == 2) { put(0); fetch(s_last - KT); }
+  const uint16_t* vrow = Vs + (32 * own + lr) * PQ + 8 * lh;
+  for (int s0 = s_last; s0 >= sbeg; s0 -= KT) {
+    uint16_t* X = st + buf * C::STAGE;
+    uint16_t* Y = X + KT * PQ;
+    if (C::NBUF == 1) put(0);
+    FM_SYNC();
+    if (C::NBUF == 1) fetch(s0 - KT);
+    const int ss0 = s0 + 32 * sub;
+    if (ss0 < A.nq && !(causal && ss0 + 31 < lo)) {
+      fm_f32x16 s = fm_zero16(), dp = fm_zero16();
+#pragma unroll
+      for (int ks = 0; ks < NKS; ++ks) {
+        const X3 xf = R::load(X + (32 * sub + lr) * PQ + 16 * ks + 8 * lh), yf = R::load(Y + (32 * sub + lr) * PQ + 16 * ks + 8 * lh);
+        const X3 vf = R::load(vrow + 16 * ks);
+#pragma unroll
+        for (int t = 0; t < FM_X3_TERMS; ++t) {
+          s = fm_mfma_bf16(xf.p[fm_x3_pa(t)], of[ks].p[fm_x3_pb(t)], s);
+          dp = fm_mfma_bf16(yf.p[fm_x3_pa(t)], vf.p[fm_x3_pb(t)], dp);
+        }
+      }
+      const float* cf = cst + buf * KT + 32 * sub + 4 * lh;
+      // dp becomes dS, s becomes P
+#pragma unroll
+      for (int g4 = 0; g4 < 4; ++g4) {
+        const fm_f32x4 c4 = *reinterpret_cast<const fm_f32x4*>(cf + 8 * g4);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int e = 4 * g4 + i;
+          const float x = s[e];
+          dp[e] = (A.a1 + ta2 * x) * (dp[e] - c4[i]);
+          s[e] = A.a0 + x * (A.a1 + A.a2 * x);
+        }
+      }
+      if (fm_tile_edge<FM_OWN_K>(causal, ss0, lo, A.nq)) {
+        FM_KEEP_BRANCH();
+        fm_x3_window<FM_OWN_K>(s, causal, ss0, lo, lr, lh, A.nq);
+        fm_x3_window<FM_OWN_K>(dp, causal, ss0, lo, lr, lh, A.nq);
+      }
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const X3 pb = fm_x3_split_acc(s, h), db = fm_x3_split_acc(dp, h);
+#pragma unroll
+        for (int ct = 0; ct < NT; ++ct) {
+          const X3 yt = R::load_tr(Y, 32 * sub + 16 * h, 32 * ct, lane), xt = R::load_tr(X, 32 * sub + 16 * h, 32 * ct, lane);
+#pragma unroll
+          for (int t = 0; t < FM_X3_TERMS; ++t) {
+            av[ct] = fm_mfma_bf16(yt.p[fm_x3_pa(t)], pb.p[fm_x3_pb(t)], av[ct]);
+            acc[ct] = fm_mfma_bf16(xt.p[fm_x3_pa(t)], db.p[fm_x3_pb(t)], acc[ct]);
+          }
+        }
+      }
+    }
+    if (C::NBUF == 2) {
+      buf ^= 1;
+      if (s0 - KT >= sbeg) { put(buf); fetch(s0 - 2 * KT); }
+    } else FM_SYNC();
+  }
+  float* Os = reinterpret_cast<float*>(smem);
+  fm_x3_store<TIO, DH, QW, SPLIT, C::NTH>(acc, Os, sub, 32 * own + lr, lh, A.sc * (A.bpart ? kf : 1.0f), A.out, bh, t0, A.nk, tid, A.k,
+                                          A.bpart ? A.bpart + int64_t(bh) * FM_GDIM_X + blk : nullptr);
+  fm_x3_store<TIO, DH, QW, SPLIT, C::NTH>(av, Os, sub, 32 * own + lr, lh, 1.0f, A.out2, bh, t0, A.nk, tid, A.k, nullptr);
+}

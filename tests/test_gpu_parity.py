@@ -6,7 +6,7 @@ import torch
 
 from tests.parity import (check_batch_head_strides, check_decode, check_forward, check_forward_backward,
                           check_norm_fold, make_inputs)
-from reproducing_fastmax_results_amd._capi import FLAG_FORCE_DENSE, FLAG_FORCE_MOMENTS
+from reproducing_fastmax_results_amd._capi import FLAG_F32_COMPUTE, FLAG_FORCE_DENSE, FLAG_FORCE_MOMENTS
 
 pytestmark = pytest.mark.gpu
 
@@ -245,6 +245,21 @@ def test_causal_more_keys_than_queries(lib, dtype, p, nq, nk):
     print(f"case causal nk>nq dtype={dtype} p={p} nq={nq} nk={nk}", flush=True)
     d = 64 if nq != 300 else 32
     check_forward_backward(lib, 3, nq, d, dtype, DEV, mask=True, p=p, nk=nk, seed=50)
+
+
+@pytest.mark.parametrize("d", [32, 64])
+@pytest.mark.parametrize("bh,n", [(1, 1), (3, 31), (2, 129), (1, 1025), (256, 40), (600, 33)])
+def test_fp32_dense_tiles(lib, d, bh, n):
+    """fp32 products as six bf16 ones (fm_x3.h): tile edges, own tiles shared by four, two and one wavefronts, more keys
+    than queries, bf16 tensors computed in fp32.  The bar is four times the 4.8e-7 measured at 4096 tokens against
+    64-bit results with v_mfma_f32_32x32x2_f32: one fp32 rounding per product sum, whichever instruction forms it."""
+    print(f"case fp32 dense d={d} bh={bh} n={n}", flush=True)
+    f = torch.float32
+    for e in (check_forward_backward(lib, bh, n, d, f, DEV, mask=True, p=2, seed=130, saved=True, flags=FLAG_FORCE_DENSE),
+              check_forward_backward(lib, bh, n, d, f, DEV, mask=False, p=2, nk=n + 37, seed=131)):
+        assert n == 1 or max(e.values()) < 2e-6, e
+    check_forward_backward(lib, min(bh, 3), n, d, torch.bfloat16, DEV, mask=True, p=2, seed=132, saved=True,
+                           flags=FLAG_F32_COMPUTE)
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
