@@ -34,27 +34,22 @@ __all__ = [
 ]
 
 CENTRE_NONE, CENTRE_FEATURE, CENTRE_TOKEN = 0, 1, 2
+_NORM_OFF, _GRAD_OF_NORMALISED, _GRAD_OF_RAW = 0, 1, 2   # the binding's `attention`: max-norm scaling of q and k, and which gradients
 
 
-_HEAD_SIZES = (32, 64)      # what every kernel is built for
-_WIDE_HEAD = 128            # bf16 attention alone also runs at this width (dense tiles; no normalisation or decoding kernels)
+_HEAD_SIZES = (32, 64)      # what every kernel is built for (bf16 attention also 128: see the binding)
 
 
-def _pad_features(x, wide=False):
+def _pad_features(x):
     """x itself, or a copy zero-padded along the feature axis to the next head size the kernels
-    are built for.  Zero features change neither q.k nor any norm, padded value columns come out
-    as zero output columns, and the padded columns of every gradient are zero as well, so callers
-    pad on the way in and slice on the way out.  ``wide``: the caller's kernels also exist at 128
-    (attention on bf16 tensors)."""
+    are built for (the binding does the same for ``attention``)."""
     d = x.shape[-1]
-    sizes = _HEAD_SIZES + ((_WIDE_HEAD,) if wide and x.dtype == torch.bfloat16 else ())
-    for size in sizes:
+    for size in _HEAD_SIZES:
         if d == size:
             return x
         if d < size:
             return torch.nn.functional.pad(x, (0, size - d))
-    raise RuntimeError(f"fastmax: unsupported head size {d} for {x.dtype} (the kernels cover up to {_HEAD_SIZES[-1]}, "
-                       f"attention on bfloat16 tensors up to {_WIDE_HEAD})")
+    raise RuntimeError(f"fastmax: unsupported head size {d} for {x.dtype} (these kernels cover up to {_HEAD_SIZES[-1]})")
 
 
 class FastmaxNormalize(torch.autograd.Function):
@@ -86,35 +81,20 @@ def _fold_possible(q, k, mask):
     return not (mask and k.shape[-2] > q.shape[-2])
 
 
-class FastmaxNormAttention(torch.autograd.Function):
+class FastmaxNormAttention:
     """Fastmax attention on ``lim * x / max_n ||x_n||_2`` of q and k (per batch and head), the
     normalisation folded into the kernels: one statistics pass reads q and k once, the attention
     kernels scale the rows as they load them, and the backward returns the gradients with respect to
     the RAW q and k, the normalisation's own Jacobian included (the dQ / dK kernels scale what they
     store and one small kernel adds the rank-one term of the row with the largest norm).  Replaces the
     reference's ``apply_norm`` pass (``fastmax_cuda_forward.cu:326-338``) and the autograd graph of its
-    Python variants (``score_function.py:40-55``); semantics of ``transformer/model.py:97-102``."""
+    Python variants (``score_function.py:40-55``); semantics of ``transformer/model.py:97-102``.  The
+    autograd node is the binding's (``attention``)."""
 
     @staticmethod
-    def forward(ctx, q, k, v, mask=False, lim=1.0, temperature=1.0, a0=1.0, a1=1.0, a2=0.5, p=2):
-        d = q.shape[-1]
-        q, k, v = _pad_features(q), _pad_features(k), _pad_features(v)
-        qk, kk = _ext.maxnorm_stats(q, k)
-        cfg = (bool(mask), 1.0 / float(temperature), float(a0), float(a1), float(a2), int(p))
-        o, g, saved = _ext.forward_norm(q, k, v, qk, kk, float(lim), *cfg, 0, 0)
-        if any(ctx.needs_input_grad[:3]):
-            ctx.save_for_backward(q, k, v, o, g, saved, qk, kk)
-        ctx.cfg, ctx.lim, ctx.d = cfg, float(lim), d
-        return o[..., :d]
-
-    @staticmethod
-    def backward(ctx, grad_output):
-        q, k, v, o, g, saved, qk, kk = ctx.saved_tensors
-        if q.shape[-1] != ctx.d:
-            grad_output = _pad_features(grad_output)
-        gq, gk, gv = _ext.backward_norm(q, k, v, o, g, grad_output, saved, qk, kk, ctx.lim, True, *ctx.cfg, 0, 0)
-        d = ctx.d
-        return (gq[..., :d], gk[..., :d], gv[..., :d]) + (None,) * 7
+    def apply(q, k, v, mask=False, lim=1.0, temperature=1.0, a0=1.0, a1=1.0, a2=0.5, p=2):
+        return _ext.attention(q, k, v, bool(mask), _GRAD_OF_RAW, float(temperature), float(a0), float(a1), float(a2), float(lim),
+                              int(p))
 
 
 class FastmaxOutputNoise(torch.autograd.Function):
@@ -172,71 +152,23 @@ def fastmax_with_dormant_steps(q, k, v, drop_noise=None, rpe_matrix=None, mask=F
     return o
 
 
-class FASTMultiHeadAttention_Function(torch.autograd.Function):
+class FASTMultiHeadAttention_Function:
     """Same call as reference ``transformer/model.py:16``.  q, k, v: ``(b, h, n, d)`` or
     ``(b*h, n, d)``.  ``drop_noise``, ``rpe_matrix`` and ``dropout`` are accepted and unused,
     as in the reference extension (``fastmax_cuda_forward.cu:289, 443``).  With
     ``normalize`` the tensors are first mapped to ``lim * x / max_n ||x_n||`` (the
-    semantics spelled out in ``transformer/model.py:97-102``) and, like the reference,
-    the returned gradients are those with respect to the normalised q and k.  Head sizes other
-    than 32 and 64 (up to 64; on bfloat16 tensors up to 128) run zero-padded to the next size the kernels have.
+    semantics spelled out in ``transformer/model.py:97-102``) and, like the reference (its extension
+    has no backward of apply_norm), the returned gradients are those with respect to the normalised q and k.
+    Head sizes other than 32 and 64 (up to 64; on bfloat16 tensors up to 128) run zero-padded to the next
+    size the kernels have.  The autograd node is the binding's (``attention``): where a gradient is asked for it keeps
+    the key-side copies and prefix states the forward built, and the backward reuses them.
     """
 
     @staticmethod
-    def forward(ctx, q, k, v, drop_noise=None, rpe_matrix=None, mask=False, dropout=0.0, normalize=False,
-                temperature=1.0, a0=1.0, a1=1.0, a2=0.5, lim=1.0, p=2):
-        if q.dim() not in (3, 4):
-            raise ValueError("q, k, and v should be either 3 or 4 dimensional tensors. "
-                             "If 3D: (b*h,n,d), if 4D: (b,h,n,d).")
-        d = q.shape[-1]
-        q, k, v = _pad_features(q, True), _pad_features(k, True), _pad_features(v, True)
-        inv_tau = 1.0 / float(temperature)
-        ctx.fold = None
-        if normalize and q.shape[-1] > _HEAD_SIZES[-1]:
-            # no normalisation kernels at that width: the scaling itself (lim * x / max_n ||x_n||, transformer/model.py:97-102)
-            # as tensor operations; like the reference, the gradients returned are those of the normalised q and k
-            q = q * (float(lim) / q.float().norm(dim=-1).amax(dim=-1)[..., None, None]).to(q.dtype)
-            k = k * (float(lim) / k.float().norm(dim=-1).amax(dim=-1)[..., None, None]).to(k.dtype)
-            normalize = False
-        if normalize and _fold_possible(q, k, mask):
-            # normalised on load; like the reference, the backward returns the gradients with respect to the
-            # normalised q and k (its extension has no backward of apply_norm)
-            qk, kk = _ext.maxnorm_stats(q, k)
-            o, g, saved = _ext.forward_norm(q, k, v, qk, kk, float(lim), bool(mask), inv_tau, float(a0), float(a1),
-                                            float(a2), int(p), 0, 0)
-            if any(ctx.needs_input_grad[:3]):
-                ctx.save_for_backward(q, k, v, o, g, saved, qk, kk)
-            ctx.fold = float(lim)
-            ctx.cfg = (bool(mask), inv_tau, float(a0), float(a1), float(a2), int(p), d)
-            return o[..., :d]
-        if normalize:
-            q = _ext.normalize(q, CENTRE_NONE, True, float(lim))
-            k = _ext.normalize(k, CENTRE_NONE, True, float(lim))
-        needs_grad = any(ctx.needs_input_grad[:3])
-        if needs_grad:
-            # keep the key-side copies and prefix states the forward built: the backward reuses them
-            o, g, saved = _ext.forward_save(q, k, v, bool(mask), inv_tau, float(a0), float(a1), float(a2), int(p), 0, 0)
-            ctx.save_for_backward(q, k, v, o, g, saved)
-        else:
-            o, g = _ext.forward_ex(q, k, v, bool(mask), inv_tau, float(a0), float(a1), float(a2), int(p), 0, 0)
-        ctx.cfg = (bool(mask), inv_tau, float(a0), float(a1), float(a2), int(p), d)
-        return o[..., :d]
-
-    @staticmethod
-    def backward(ctx, grad_output):
-        mask, inv_tau, a0, a1, a2, p, d = ctx.cfg
-        if ctx.fold is not None:
-            q, k, v, o, g, saved, qk, kk = ctx.saved_tensors
-            if q.shape[-1] != d:
-                grad_output = _pad_features(grad_output)
-            gq, gk, gv = _ext.backward_norm(q, k, v, o, g, grad_output, saved, qk, kk, ctx.fold, False, mask, inv_tau,
-                                            a0, a1, a2, p, 0, 0)
-            return (gq[..., :d], gk[..., :d], gv[..., :d]) + (None,) * 11
-        q, k, v, o, g, saved = ctx.saved_tensors
-        if q.shape[-1] != d:
-            grad_output = _pad_features(grad_output, True)
-        gq, gk, gv = _ext.backward_saved(q, k, v, o, g, grad_output, saved, mask, inv_tau, a0, a1, a2, p, 0, 0)
-        return (gq[..., :d], gk[..., :d], gv[..., :d]) + (None,) * 11
+    def apply(q, k, v, drop_noise=None, rpe_matrix=None, mask=False, dropout=0.0, normalize=False,
+              temperature=1.0, a0=1.0, a1=1.0, a2=0.5, lim=1.0, p=2):
+        return _ext.attention(q, k, v, bool(mask), _GRAD_OF_NORMALISED if normalize else _NORM_OFF, float(temperature), float(a0),
+                              float(a1), float(a2), float(lim), int(p))
 
 
 class FastmaxDecodeState:

@@ -497,9 +497,115 @@ torch::Tensor output_noise(torch::Tensor o_, torch::Tensor noise_, double scale)
   return y;
 }
 
+// ---------------------------------------------------------------------------------
+// The operator with its gradient, as a C++ autograd node: the backward runs on the engine's thread without the
+// interpreter.  (As a Python autograd function a training call of a small problem cost 64 - 125 us of host time, most
+// of it in the engine's hand-over and the interpreter; a forward with its backward is two to five launches.)
+// ---------------------------------------------------------------------------------
+constexpr int64_t kHeadSizes[] = {32, 64};             // what every kernel is built for
+constexpr int64_t kWideHead = 128;                     // bf16 attention alone (dense tiles; no normalisation, no decoding kernels)
+
+// t itself, or a copy zero-padded along the feature axis to the next head size the kernels are built for.  Zero features
+// change neither q.k nor any norm, padded value columns come out as zero output columns, and the padded columns of every
+// gradient are zero as well, so callers pad on the way in and slice on the way out.
+torch::Tensor pad_features(const torch::Tensor& t, bool wide) {
+  const int64_t d = t.size(-1);
+  wide = wide && t.scalar_type() == torch::kBFloat16;
+  for (int64_t size : {kHeadSizes[0], kHeadSizes[1], wide ? kWideHead : int64_t(0)}) {
+    if (d == size) return t;
+    if (d < size) return at::constant_pad_nd(t, {0, size - d});
+  }
+  TORCH_CHECK(false, "fastmax: unsupported head size ", d, " for ", t.scalar_type(), " (the kernels cover up to ", kHeadSizes[1],
+              ", attention on bfloat16 tensors up to ", kWideHead, ")");
+}
+torch::Tensor first_features(const torch::Tensor& t, int64_t d) { return t.size(-1) == d ? t : t.narrow(-1, 0, d); }
+
+enum { kNormNone = 0, kNormGradOfNormalised = 1, kNormGradOfRaw = 2 };
+
+struct AttnConfig {
+  bool mask;
+  int64_t norm;              // max-norm scaling of q and k: off, or on with gradients of the scaled / of the raw tensors
+  double inv_tau, a0, a1, a2, lim;
+  int64_t p;
+};
+
+// More keys than queries under the causal mask run in two parts that would share one Jacobian: no fold there.
+bool fold_possible(const torch::Tensor& q, const torch::Tensor& k, bool mask) { return !(mask && k.size(-2) > q.size(-2)); }
+
+struct AttnResult { torch::Tensor q, k, v, o, g, saved, qk, kk; bool fold = false; };
+
+// q, k, v in any head size; `save`: a backward follows
+AttnResult attention_forward(const torch::Tensor& q_, const torch::Tensor& k_, const torch::Tensor& v_, const AttnConfig& c, bool save) {
+  TORCH_CHECK_VALUE(q_.dim() == 3 || q_.dim() == 4, "q, k, and v should be either 3 or 4 dimensional tensors. "
+                    "If 3D: (b*h,n,d), if 4D: (b,h,n,d).");
+  AttnResult r;
+  const bool wide = c.norm != kNormGradOfRaw;          // the folded kernels stop at 64
+  r.q = pad_features(q_, wide); r.k = pad_features(k_, wide); r.v = pad_features(v_, wide);
+  NormArgs na;
+  if (c.norm != kNormNone) {
+    if (r.q.size(-1) > kHeadSizes[1]) {
+      // no normalisation kernels at that width: the scaling itself (lim * x / max_n ||x_n||, transformer/model.py:97-102)
+      // as tensor operations
+      auto scaled = [&](const torch::Tensor& x) {
+        const torch::Tensor m = x.to(torch::kFloat32).norm(2, {-1}).amax({-1}).unsqueeze(-1).unsqueeze(-1);
+        return x * (c.lim / m).to(x.scalar_type());
+      };
+      r.q = scaled(r.q); r.k = scaled(r.k);
+    } else if (fold_possible(r.q, r.k, c.mask)) {
+      std::tie(r.qk, r.kk) = maxnorm_stats(r.q, r.k);
+      na = NormArgs{r.qk, r.kk, c.lim, false};
+      r.fold = true;
+    } else {
+      r.q = normalize(r.q, 0, true, c.lim);
+      r.k = normalize(r.k, 0, true, c.lim);
+    }
+  }
+  std::vector<torch::Tensor> f = forward_any(r.q, r.k, r.v, c.mask, c.inv_tau, c.a0, c.a1, c.a2, c.p, 0,
+                                             save ? FASTMAX_FLAG_SAVE_FOR_BACKWARD : 0, r.fold ? &na : nullptr);
+  r.o = f[0]; r.g = f[1]; r.saved = f[2];
+  return r;
+}
+
+struct AttentionNode : public torch::autograd::Function<AttentionNode> {
+  static torch::Tensor forward(torch::autograd::AutogradContext* ctx, const torch::Tensor& q, const torch::Tensor& k,
+                               const torch::Tensor& v, const AttnConfig& c) {
+    AttnResult r = attention_forward(q, k, v, c, true);
+    ctx->save_for_backward({r.q, r.k, r.v, r.o, r.g, r.saved, r.qk, r.kk});
+    ctx->saved_data["d"] = q.size(-1);
+    ctx->saved_data["fold"] = r.fold;
+    ctx->saved_data["mask"] = c.mask;
+    ctx->saved_data["ip"] = std::vector<int64_t>{c.norm, c.p};
+    ctx->saved_data["fp"] = std::vector<double>{c.inv_tau, c.a0, c.a1, c.a2, c.lim};
+    return first_features(r.o, q.size(-1));
+  }
+  static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx, torch::autograd::variable_list grads) {
+    const torch::autograd::variable_list s = ctx->get_saved_variables();
+    const int64_t d = ctx->saved_data["d"].toInt();
+    const bool fold = ctx->saved_data["fold"].toBool(), mask = ctx->saved_data["mask"].toBool();
+    const std::vector<int64_t> ip = ctx->saved_data["ip"].toIntVector();
+    const std::vector<double> fp = ctx->saved_data["fp"].toDoubleVector();
+    const torch::Tensor go = s[0].size(-1) == d ? grads[0] : pad_features(grads[0], true);
+    NormArgs na{s[6], s[7], fp[4], ip[0] == kNormGradOfRaw};
+    std::vector<torch::Tensor> r = backward_any(s[0], s[1], s[2], s[3], s[4], go, &s[5], mask, fp[0], fp[1], fp[2], fp[3], ip[1], 0,
+                                                FASTMAX_FLAG_SAVE_FOR_BACKWARD, fold ? &na : nullptr);
+    return {first_features(r[0], d), first_features(r[1], d), first_features(r[2], d), torch::Tensor()};
+  }
+};
+
+// Attention with autograd.  norm: kNorm* above.
+torch::Tensor attention(const torch::Tensor& q, const torch::Tensor& k, const torch::Tensor& v, bool mask, int64_t norm, double temperature,
+                        double a0, double a1, double a2, double lim, int64_t p) {
+  const AttnConfig c{mask, norm, 1.0 / temperature, a0, a1, a2, lim, p};
+  if (at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad()))
+    return AttentionNode::apply(q, k, v, c);
+  at::NoGradGuard guard;
+  return first_features(attention_forward(q, k, v, c, false).o, q.size(-1));
+}
+
 }  // namespace
 
 PYBIND11_MODULE(fastmax_cuda, m) {
+  m.def("attention", &attention, "attention with its gradient (autograd): returns o");
   m.def("forwardpass", &forwardpass, "forwardpass");
   m.def("backwardpass", &backwardpass, "backwardpass");
   m.def("forward_ex", &forward_ex, "strided forward: returns (o, g)");
