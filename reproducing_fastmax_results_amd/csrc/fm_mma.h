@@ -142,7 +142,7 @@ template <> struct IO<fm_bf16> {
       fm_u32x4 u;
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        u[i] = uint32_t(fm_f32_to_bf16(in[2 * i])) | (uint32_t(fm_f32_to_bf16(in[2 * i + 1])) << 16);
+        u[i] = fm_cvt_pk_bf16(in[2 * i], in[2 * i + 1]);
       *reinterpret_cast<fm_u32x4*>(p) = u;
     } else {
 #pragma unroll

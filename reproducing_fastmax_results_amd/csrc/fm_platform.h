@@ -225,6 +225,7 @@ FM_DEVICE float fm_bf16_to_f32(fm_bf16 v) {
   __builtin_memcpy(&f, &u, 4);
   return f;
 }
+#if defined(FM_HOSTSIM)
 FM_DEVICE fm_bf16 fm_f32_to_bf16(float f) {
   uint32_t u;
   __builtin_memcpy(&u, &f, 4);
@@ -232,7 +233,8 @@ FM_DEVICE fm_bf16 fm_f32_to_bf16(float f) {
   u += 0x7fffu + ((u >> 16) & 1u);
   return fm_bf16(u >> 16);
 }
-// two floats -> two bfloat16 (round to nearest even) in one register, the first in the low half
+#endif
+// two floats -> two bfloat16 in one register, the first in the low half
 FM_DEVICE uint32_t fm_cvt_pk_bf16(float a, float b) {
 #if defined(FM_HOSTSIM)
   return uint32_t(fm_f32_to_bf16(a)) | (uint32_t(fm_f32_to_bf16(b)) << 16);
@@ -245,4 +247,9 @@ FM_DEVICE uint32_t fm_cvt_pk_bf16(float a, float b) {
   return u;
 #endif
 }
+#if !defined(FM_HOSTSIM)
+// (the conversion instruction: rounding spelt out in integer arithmetic was five instructions per element and up to half of
+// the code of the kernels that store bf16)
+FM_DEVICE fm_bf16 fm_f32_to_bf16(float f) { return fm_bf16(fm_cvt_pk_bf16(f, f)); }
+#endif
 FM_DEVICE float fm_bits_f32(uint32_t u) { float f; __builtin_memcpy(&f, &u, 4); return f; }
