@@ -39,9 +39,11 @@ enum {
   FASTMAX_FLAG_SAVE_FOR_BACKWARD = 4, /* forward: also leave in its workspace what the backward of the same
                                         problem can reuse (converted k, v and the key-side moment states);
                                         forward_bytes grows accordingly */
-  FASTMAX_FLAG_F32_COMPUTE = 8       /* bf16 tensors: do all arithmetic in fp32 (matrix products included)
+  FASTMAX_FLAG_F32_COMPUTE = 8,      /* bf16 tensors: do all arithmetic in fp32 (matrix products included)
                                         instead of _Float16; for inputs outside the range stated below.
                                         Many times slower; workspace sizes grow.  Ignored for fp32 tensors. */
+  FASTMAX_FLAG_NORM_SELF = 16        /* nq, nk <= 64 (and not causal with nk > nq): q and k are max-normalised with norm.lim and
+                                        the kernels find the norms themselves; norm.q_keys and norm.k_keys are null */
 };
 
 /* Numeric range of the bf16 interface.  bf16 tensors are computed in _Float16 with fp32 accumulation

@@ -21,7 +21,7 @@ LIB_NAME = "libfastmax_hip.so"
 BENCH_LIB_NAME = "libfastmax_hip_bench.so"
 
 F32, BF16 = 0, 1
-FLAG_FORCE_MOMENTS, FLAG_FORCE_DENSE, FLAG_SAVE_FOR_BACKWARD, FLAG_F32_COMPUTE = 1, 2, 4, 8
+FLAG_FORCE_MOMENTS, FLAG_FORCE_DENSE, FLAG_SAVE_FOR_BACKWARD, FLAG_F32_COMPUTE, FLAG_NORM_SELF = 1, 2, 4, 8, 16
 STATUS_OK = 0
 
 

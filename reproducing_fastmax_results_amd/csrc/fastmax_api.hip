@@ -11,6 +11,7 @@
 #include "fm_pointwise.h"
 #include "fm_walk_sym.h"
 #include "fm_x3.h"
+#include "fm_small.h"
 #if defined(FM_BENCH_AIDS)
 #include "fm_bench_aids.h"
 #endif
@@ -114,6 +115,7 @@ struct Plan {
   // workspace offsets (bytes)
   size_t kt, vt, kr, vr, big, big2, small, run, runh, ores, fwd_bytes;
   bool keep_resid;      // the forward leaves o - bf16(o) for the backward (see TokArgs::out_resid)
+  bool tiny;            // at most 64 tokens: fm_small.h
   bool x3;              // fp32 arithmetic without states: the kernels of fm_x3.h (read the caller's tensors, no copies)
   bool sym;             // order-2 states are built by the walk per value column (k_walk_sym): one layout, no transposed copy   // run, runh: see k_o1_sums
   bool save;
@@ -130,6 +132,11 @@ bool strides_ok(const FastmaxStrides& s, int bh, int n, int d) {
     return false;
   }
   return s.n > 0 || n <= 1;
+}
+
+// Whole batch*heads of at most 64 tokens on either side (fm_small.h).
+inline bool is_small(const FastmaxDesc* d) {
+  return d->nq <= FM_SMALL_TOKENS && d->nk <= FM_SMALL_TOKENS && d->d <= 64 && !(d->flags & FASTMAX_FLAG_FORCE_MOMENTS);
 }
 
 int validate(const FastmaxDesc* d) {
@@ -152,6 +159,10 @@ int validate(const FastmaxDesc* d) {
   if (d->mask && d->nq > d->nk) return FASTMAX_ERR_UNSUPPORTED;   // nk > nq: see SplitPlan
   if (d->chunk < 0) return FASTMAX_ERR_SHAPE;
   if (!(d->inv_tau > 0.0f) || !(d->inv_tau < 3.0e38f)) return FASTMAX_ERR_SHAPE;   // also rejects NaN
+  if (d->flags & FASTMAX_FLAG_NORM_SELF) {
+    if (!is_small(d) || (d->mask && d->nk > d->nq)) return FASTMAX_ERR_UNSUPPORTED;
+    if (d->norm.q_keys || d->norm.k_keys || !(d->norm.lim > 0.0f) || !(d->norm.lim < 3.0e38f)) return FASTMAX_ERR_SHAPE;
+  }
   if (d->norm.q_keys || d->norm.k_keys) {
     if (d->mask && d->nk > d->nq) return FASTMAX_ERR_UNSUPPORTED;                    // two parts would share one Jacobian
     if (!(d->norm.lim > 0.0f) || !(d->norm.lim < 3.0e38f)) return FASTMAX_ERR_SHAPE;
@@ -205,7 +216,8 @@ int make_plan(const FastmaxDesc* d, Plan& p) {
     p.use_state = force_m || (!force_dense && int64_t(d->nk) > int64_t(d->d) * d->d + d->d);
     p.nslots = p.use_state ? 1 : 0;
   }
-  p.x3 = !p.half && !p.use_state;
+  p.tiny = is_small(d);
+  p.x3 = !p.half && !p.use_state && !p.tiny;
   p.o1 = p.half && p.use_state && !p.quad && d->mask && p.L == FM_O1_SEG && d->nq == d->nk;
   p.rows_build = p.half && p.use_state && !p.quad && d->mask;
   {
@@ -224,8 +236,9 @@ int make_plan(const FastmaxDesc* d, Plan& p) {
   const size_t bigarr = d->d == 64 ? big_array_bytes<64>(p.esz, p.quad, slots) : big_array_bytes<32>(p.esz, p.quad, slots);
   // fp32 part of a slot: Z and the two vector sums; the order-1 path of fm_o1.h keeps the two vectors only
   const size_t smallsz = p.o1 ? size_t(2) * d->d * 4 : size_t(d->d == 64 ? StateDims<64>::SMALL : StateDims<32>::SMALL) * 4;
-  const size_t tq = p.o1 || p.x3 ? 0 : size_t(d->bh) * d->d * p.npad_q * p.esz;
-  const size_t tk = p.o1 || p.x3 ? 0 : size_t(d->bh) * d->d * p.npad_k * p.esz;
+  const bool no_copies = p.o1 || p.x3 || p.tiny;
+  const size_t tq = no_copies ? 0 : size_t(d->bh) * d->d * p.npad_q * p.esz;
+  const size_t tk = no_copies ? 0 : size_t(d->bh) * d->d * p.npad_k * p.esz;
   size_t off = 0;
   auto take = [&](size_t bytes) { size_t o = off; off = align256(off + bytes); return o; };
   // transposed copies: only the order-2 state walk, the one-total order-1 walk and the fp32 kernels read them
@@ -246,17 +259,17 @@ int make_plan(const FastmaxDesc* d, Plan& p) {
   const size_t runharr = size_t(d->bh) * nruns * d->d * d->d * 2;
   p.run = take(runarr); p.runh = take(runharr);
   p.keep_resid = p.save && d->dtype == FASTMAX_BF16 && !p.o1;
-  p.ores = take(p.keep_resid ? size_t(d->bh) * p.npad_q * d->d * 2 : 0);
+  p.ores = take(p.keep_resid ? size_t(d->bh) * (p.tiny ? d->nq : p.npad_q) * d->d * 2 : 0);
   p.fwd_bytes = off ? off : 256;
   off = 0;
   p.b_kt = take(tkt); p.b_vt = take(tkt); p.b_qt = take(tqt); p.b_qct = take(tqt);
   p.b_kr = take(tk); p.b_vr = take(tk); p.b_qr = take(tq);
   p.b_gh = take(tq); p.b_ght = take(tqt);
-  p.b_cv = take(p.o1 ? 0 : size_t(d->bh) * p.npad_q * 4);
+  p.b_cv = take(p.o1 || p.tiny ? 0 : size_t(d->bh) * p.npad_q * 4);
   p.b_bigq = take(bigarr); p.b_smallq = take(size_t(d->bh) * p.nslots * smallsz);
   p.b_bigk = take(bigarr); p.b_smallk = take(size_t(d->bh) * p.nslots * smallsz);
   p.b_bigv = take(p.o1 ? 0 : bigarr);
-  p.b_gpart = take(p.half ? size_t(d->bh) * fm_grad_scale_blocks(d->nq) * 4 : 0);   // see k_grad_scale
+  p.b_gpart = take(p.half && !p.tiny ? size_t(d->bh) * fm_grad_scale_blocks(d->nq) * 4 : 0);   // see k_grad_scale
   // parts of B = sum dy . y per workgroup of the dQ and dK kernels (32 own tokens at least), see k_norm_fix
   const bool jac = d->norm.grad != 0;
   p.b_bq = take(jac && d->norm.q_keys ? size_t(d->bh) * ((d->nq + 31) / 32) * 4 : 0);
@@ -537,6 +550,46 @@ int launch_x3(const X3Args<TIO>& a, int split, int n_own, int bh, fm_stream_t st
   return launch_x3_cfg<TIO, DH, KIND, 4>(a, n_own, bh, stream);
 }
 
+// ---- at most 64 tokens (fm_small.h) ----------------------------------------------------------
+template <typename TIO> SmallArgs<TIO> small_args(const FastmaxDesc* d, const Plan& p, const void* q, const void* k, const void* v) {
+  SmallArgs<TIO> a;
+  a.q = cref<TIO>(q, d->sq); a.k = cref<TIO>(k, d->sk); a.v = cref<TIO>(v, d->sv);
+  a.o = TRef<const TIO>{nullptr, 0, 0, 0, 0, 0}; a.d_o = a.o;
+  a.out = TRef<TIO>{nullptr, 0, 0, 0, 0, 0}; a.dk = a.out; a.dv = a.out;
+  a.g = TRef<float>{nullptr, 0, 0, 0, 0, 0};
+  a.out_resid = nullptr; a.ores = nullptr; a.npad_q = d->nq;
+  a.nq = d->nq; a.nk = d->nk; a.causal = d->mask != 0;
+  a.a0 = p.a0; a.a1 = p.a1; a.a2 = p.a2; a.sc = p.sc;
+  const bool self = (d->flags & FASTMAX_FLAG_NORM_SELF) != 0;
+  a.norm_q = self || d->norm.q_keys; a.norm_k = self || d->norm.k_keys; a.jac = d->norm.grad != 0; a.lim = d->norm.lim;
+  return a;
+}
+template <typename TIO, int DH>
+int run_small_fwd(const FastmaxDesc* d, const Plan& p, const void* q, const void* k, const void* v, void* o, float* g, char* ws,
+                  fm_stream_t stream) {
+  SmallArgs<TIO> a = small_args<TIO>(d, p, q, k, v);
+  a.out = mref<TIO>(o, d->so); a.g = mref<float>(g, d->sg);
+  if (p.keep_resid) a.out_resid = reinterpret_cast<fm_half*>(ws + p.ores);
+  const size_t lds = SmallCfg<TIO, DH>::fwd_lds();
+  fm_allow_lds(reinterpret_cast<const void*>(&k_small_fwd<TIO, DH>), lds);
+  ProfScope prof(FM_K_FWD, stream);
+  FM_KERNEL_LAUNCH((k_small_fwd<TIO, DH>), fm_dim3(1, d->bh), fm_dim3(256), lds, stream, a);
+  return fm_launch_status();
+}
+template <typename TIO, int DH>
+int run_small_bwd(const FastmaxDesc* d, const Plan& p, const void* q, const void* k, const void* v, const void* o, const float* g,
+                  const void* d_o, void* dq, void* dk, void* dv, const char* fws, fm_stream_t stream) {
+  SmallArgs<TIO> a = small_args<TIO>(d, p, q, k, v);
+  a.o = cref<TIO>(o, d->so); a.d_o = cref<TIO>(d_o, d->sdo); a.g = fm_ref<float>(const_cast<float*>(g), d->sg);   // read only
+  a.out = mref<TIO>(dq, d->sdq); a.dk = mref<TIO>(dk, d->sdk); a.dv = mref<TIO>(dv, d->sdv);
+  if (fws && p.keep_resid) a.ores = reinterpret_cast<const fm_half*>(fws + p.ores);
+  const size_t lds = SmallCfg<TIO, DH>::bwd_lds();
+  fm_allow_lds(reinterpret_cast<const void*>(&k_small_bwd<TIO, DH>), lds);
+  ProfScope prof(FM_K_DKV, stream);
+  FM_KERNEL_LAUNCH((k_small_bwd<TIO, DH>), fm_dim3(1, d->bh), fm_dim3(256), lds, stream, a);
+  return fm_launch_status();
+}
+
 template <typename TIO, typename E, int DH, int QT>
 int run_forward(const FastmaxDesc* d, const Plan& p, const void* q, const void* k, const void* v, void* o,
                 float* g, char* ws, fm_stream_t stream) {
@@ -681,7 +734,7 @@ int add_rows(const FastmaxDesc* d, const SplitPlan& sp, const void* dqa, void* d
 // Forward only, and nothing is left for a backward: a forward that is to keep its workspace takes the general
 // route (causal problems with nk > nq keep nothing there either and come here).
 inline bool is_few(const FastmaxDesc* d) {
-  return fm_few_pays(d->bh, d->nq) && d->d <= 64 && (is_split(d) || !(d->flags & FASTMAX_FLAG_SAVE_FOR_BACKWARD)) &&
+  return fm_few_pays(d->bh, d->nq) && d->d <= 64 && !(d->nq > 16 && is_small(d)) && !(d->flags & FASTMAX_FLAG_NORM_SELF) && (is_split(d) || !(d->flags & FASTMAX_FLAG_SAVE_FOR_BACKWARD)) &&
          !(d->flags & (FASTMAX_FLAG_FORCE_MOMENTS | FASTMAX_FLAG_FORCE_DENSE));
 }
 inline size_t few_bytes(const FastmaxDesc* d) {
@@ -737,7 +790,7 @@ int fastmax_workspace_bytes(const FastmaxDesc* desc, size_t* forward_bytes, size
   int st = validate(desc);
   if (st) return st;
   size_t f = 0, b = 0;
-  if (is_split(desc)) {
+  if (is_split(desc) && !is_small(desc)) {
     SplitPlan sp;
     st = make_split(desc, sp);
     f = sp.fwd_bytes; b = sp.bwd_bytes;
@@ -783,6 +836,11 @@ static int forward_one(const FastmaxDesc* desc, const void* q, const void* k, co
     return FASTMAX_ERR_WORKSPACE;
   char* ws = static_cast<char*>(workspace);
   fm_stream_t stream = static_cast<fm_stream_t>(hip_stream);
+  if (p.tiny) {
+    if (desc->dtype == FASTMAX_BF16)
+      return desc->d == 64 ? run_small_fwd<fm_bf16, 64>(desc, p, q, k, v, o, g, ws, stream) : run_small_fwd<fm_bf16, 32>(desc, p, q, k, v, o, g, ws, stream);
+    return desc->d == 64 ? run_small_fwd<float, 64>(desc, p, q, k, v, o, g, ws, stream) : run_small_fwd<float, 32>(desc, p, q, k, v, o, g, ws, stream);
+  }
   if (p.half) {
     if (desc->d == FM_WIDE_HEAD) return run_forward<fm_bf16, fm_half, FM_WIDE_HEAD, 1>(desc, p, q, k, v, o, g, ws, stream);
     if (desc->d == 64) return run_forward<fm_bf16, fm_half, 64, 1>(desc, p, q, k, v, o, g, ws, stream);
@@ -801,7 +859,7 @@ int fastmax_forward(const FastmaxDesc* desc, const void* q, const void* k, const
   const int st = validate(desc);
   if (st) return st;
   if (is_few(desc)) return forward_few(desc, q, k, v, o, g, workspace, workspace_bytes, hip_stream);
-  if (!is_split(desc)) return forward_one(desc, q, k, v, o, g, workspace, workspace_bytes, hip_stream);
+  if (!is_split(desc) || is_small(desc)) return forward_one(desc, q, k, v, o, g, workspace, workspace_bytes, hip_stream);
   // causal with nk > nq: the keys every query sees, then the square causal part, then the merge
   SplitPlan sp;
   int s2 = make_split(desc, sp);
@@ -862,6 +920,13 @@ static int backward_one(const FastmaxDesc* desc, const void* q, const void* k, c
   char* ws = static_cast<char*>(workspace);
   const char* fws = static_cast<const char*>(fwd_ws);
   fm_stream_t stream = static_cast<fm_stream_t>(hip_stream);
+  if (p.tiny) {
+    if (desc->dtype == FASTMAX_BF16)
+      return desc->d == 64 ? run_small_bwd<fm_bf16, 64>(desc, p, q, k, v, o, g, d_o, dq, dk, dv, fws, stream)
+                           : run_small_bwd<fm_bf16, 32>(desc, p, q, k, v, o, g, d_o, dq, dk, dv, fws, stream);
+    return desc->d == 64 ? run_small_bwd<float, 64>(desc, p, q, k, v, o, g, d_o, dq, dk, dv, fws, stream)
+                         : run_small_bwd<float, 32>(desc, p, q, k, v, o, g, d_o, dq, dk, dv, fws, stream);
+  }
   if (p.half) {
     if (desc->d == FM_WIDE_HEAD) return run_backward_wide<fm_bf16, fm_half, FM_WIDE_HEAD>(desc, p, q, k, v, o, g, d_o, dq, dk, dv, fws, ws, stream);
     if (desc->d == 64) return run_backward<fm_bf16, fm_half, 64, 1>(desc, p, q, k, v, o, g, d_o, dq, dk, dv, fws, ws, stream);
@@ -880,11 +945,11 @@ static int backward_impl(const FastmaxDesc* desc, const void* q, const void* k, 
                          size_t fwd_ws_bytes, void* workspace, size_t workspace_bytes, void* hip_stream) {
   const int st = validate(desc);
   if (st) return st;
-  if (!is_split(desc))
+  // causal with nk > nq: the forward keeps nothing
+  if (fwd_ws && is_split(desc)) return FASTMAX_ERR_UNSUPPORTED;
+  if (!is_split(desc) || is_small(desc))
     return backward_one(desc, q, k, v, o, g, d_o, dq, dk, dv, fwd_ws, fwd_ws_bytes, workspace, workspace_bytes, hip_stream);
-  // causal with nk > nq: both parts take the final o and g; dk and dv of the two parts are
-  // disjoint key ranges, dq is their sum.  The forward keeps nothing for this case.
-  if (fwd_ws) return FASTMAX_ERR_UNSUPPORTED;
+  // both parts take the final o and g; dk and dv of the two parts are disjoint key ranges, dq is their sum
   SplitPlan sp;
   int s2 = make_split(desc, sp);
   if (s2) return s2;

@@ -205,6 +205,7 @@ struct NormArgs {
   torch::Tensor q_keys, k_keys;
   double lim = 1.0;
   bool grad = false;
+  bool self = false;         // short sequences: the kernels find the norms themselves (FASTMAX_FLAG_NORM_SELF)
 };
 
 void apply_norm_args(FastmaxDesc& d, const NormArgs* na) {
@@ -220,6 +221,7 @@ void apply_norm_args(FastmaxDesc& d, const NormArgs* na) {
   d.norm.k_keys = check(na->k_keys, d.nk, "k_keys");
   d.norm.lim = float(na->lim);
   d.norm.grad = na->grad ? 1 : 0;
+  if (na->self) d.flags |= FASTMAX_FLAG_NORM_SELF;
 }
 
 FastmaxDesc ex_desc(const View& q, const View& k, const View& v, bool mask, double inv_tau, double a0, double a1,
@@ -532,7 +534,7 @@ struct AttnConfig {
 // More keys than queries under the causal mask run in two parts that would share one Jacobian: no fold there.
 bool fold_possible(const torch::Tensor& q, const torch::Tensor& k, bool mask) { return !(mask && k.size(-2) > q.size(-2)); }
 
-struct AttnResult { torch::Tensor q, k, v, o, g, saved, qk, kk; bool fold = false; };
+struct AttnResult { torch::Tensor q, k, v, o, g, saved, qk, kk; bool fold = false, self = false; };
 
 // q, k, v in any head size; `save`: a backward follows
 AttnResult attention_forward(const torch::Tensor& q_, const torch::Tensor& k_, const torch::Tensor& v_, const AttnConfig& c, bool save) {
@@ -552,9 +554,10 @@ AttnResult attention_forward(const torch::Tensor& q_, const torch::Tensor& k_, c
       };
       r.q = scaled(r.q); r.k = scaled(r.k);
     } else if (fold_possible(r.q, r.k, c.mask)) {
-      std::tie(r.qk, r.kk) = maxnorm_stats(r.q, r.k);
-      na = NormArgs{r.qk, r.kk, c.lim, false};
       r.fold = true;
+      r.self = r.q.size(-2) <= 64 && r.k.size(-2) <= 64;
+      if (!r.self) std::tie(r.qk, r.kk) = maxnorm_stats(r.q, r.k);
+      na = NormArgs{r.qk, r.kk, c.lim, false, r.self};
     } else {
       r.q = normalize(r.q, 0, true, c.lim);
       r.k = normalize(r.k, 0, true, c.lim);
@@ -572,20 +575,18 @@ struct AttentionNode : public torch::autograd::Function<AttentionNode> {
     AttnResult r = attention_forward(q, k, v, c, true);
     ctx->save_for_backward({r.q, r.k, r.v, r.o, r.g, r.saved, r.qk, r.kk});
     ctx->saved_data["d"] = q.size(-1);
-    ctx->saved_data["fold"] = r.fold;
-    ctx->saved_data["mask"] = c.mask;
-    ctx->saved_data["ip"] = std::vector<int64_t>{c.norm, c.p};
+    ctx->saved_data["ip"] = std::vector<int64_t>{c.norm, c.p, r.fold, r.self, c.mask};
     ctx->saved_data["fp"] = std::vector<double>{c.inv_tau, c.a0, c.a1, c.a2, c.lim};
     return first_features(r.o, q.size(-1));
   }
   static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx, torch::autograd::variable_list grads) {
     const torch::autograd::variable_list s = ctx->get_saved_variables();
     const int64_t d = ctx->saved_data["d"].toInt();
-    const bool fold = ctx->saved_data["fold"].toBool(), mask = ctx->saved_data["mask"].toBool();
     const std::vector<int64_t> ip = ctx->saved_data["ip"].toIntVector();
+    const bool fold = ip[2] != 0, mask = ip[4] != 0;
     const std::vector<double> fp = ctx->saved_data["fp"].toDoubleVector();
     const torch::Tensor go = s[0].size(-1) == d ? grads[0] : pad_features(grads[0], true);
-    NormArgs na{s[6], s[7], fp[4], ip[0] == kNormGradOfRaw};
+    NormArgs na{s[6], s[7], fp[4], ip[0] == kNormGradOfRaw, ip[3] != 0};
     std::vector<torch::Tensor> r = backward_any(s[0], s[1], s[2], s[3], s[4], go, &s[5], mask, fp[0], fp[1], fp[2], fp[3], ip[1], 0,
                                                 FASTMAX_FLAG_SAVE_FOR_BACKWARD, fold ? &na : nullptr);
     return {first_features(r[0], d), first_features(r[1], d), first_features(r[2], d), torch::Tensor()};

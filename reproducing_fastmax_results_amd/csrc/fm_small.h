@@ -1,0 +1,356 @@
+// Sequences of at most 64 queries and 64 keys: a whole batch*head is one workgroup's work, forward one launch, backward
+// (dQ, dK and dV) one launch, the max-norm normalisation of q and k and its Jacobian inside both.
+//
+// Such problems (an image classifier: thousands of heads of 50 tokens) are bound by their bytes and by launches; the general
+// kernels padded 50 tokens to blocks of 128 and 256, read every tensor two to four times and took a launch each for the
+// norms, dQ, dK + dV and the Jacobian's row.  Here every tensor is read once and every result written once.
+// fp32 tensors: products of three bf16 planes (fm_x3.h).  bf16 tensors: the operands are the caller's numbers themselves (one
+// plane, exact), every factor (temperature, norms, 1 / g) is applied in fp32 to what the products give, and the weights
+// are split in two planes (16 bits), so no range but fp32's applies here.  Wavefront (i, j) of the four works on the 32 x 32 tile of query tile i and key tile j; two sums per
+// result meet in LDS.  The backward forms the scores twice, keys along the accumulator rows for dQ and queries along
+// them for dK and dV: each is then the operand of the product that follows, without a transposition.
+// B*H = 1024, 50 tokens, D = 32, normalised (26 MB forward, 53 MB backward): fp32 forward with its norms 23 -> 11.3 us, backward
+// with its Jacobian 77 -> 24.6 (160 in six launches before fm_x3.h), bf16 73 -> 30 in all; 1024 heads of 64 x 64, bf16: 82 -> 44.
+// The kernels run once through straight code, so its length counts: half of the bf16 code was rounding spelt out in integer
+// arithmetic, and taking it out brought forward and backward of the last shape from 56 to 44 us.
+#pragma once
+#include "fm_x3.h"
+
+static constexpr int FM_SMALL_TOKENS = 64;
+
+template <typename TIO> struct SmallArgs {
+  TRef<const TIO> q, k, v, o, d_o;
+  TRef<float> g;
+  TRef<TIO> out, dk, dv;                // out: o | dq
+  fm_half* out_resid; const fm_half* ores; int npad_q;   // see TokArgs
+  int nq, nk, causal;
+  float a0, a1, a2, sc;
+  int norm_q, norm_k, jac; float lim;   // max-norm scaling of q / k; jac: gradients with respect to the raw tensors
+};
+
+template <typename TIO, int DH> struct SmallCfg {
+  static constexpr bool RAW = sizeof(TIO) == 2;        // operands are the caller's numbers
+  static constexpr int PL = RAW ? 1 : 3, PP = RAW ? 2 : 3;          // planes of an operand in LDS, of a weight
+  static constexpr int N = DH / 32;                    // eight-feature items of a tensor per thread
+  static constexpr int PQ = PL * DH + 8, TILE = 64 * PQ, OP = DH + 4;
+  static constexpr size_t OS = size_t(2) * 64 * OP * 4;            // one result's two parts
+  static constexpr size_t fwd_lds() { const size_t a = size_t(3) * TILE * 2, b = OS + 2 * 64 * 4; return a > b ? a : b; }
+  static constexpr size_t bwd_lds() { const size_t a = size_t(4) * TILE * 2 + 2 * 64 * 4; return a > OS ? a : OS; }
+};
+
+template <typename TIO, int DH>
+FM_DEVICE void fm_small_load(const TRef<const TIO>& t, int bh, int n, int tid, float (*r)[8]) {
+#pragma unroll
+  for (int i = 0; i < DH / 32; ++i) {
+    const int c = tid + 256 * i, row = c / (DH / 8), col = (c % (DH / 8)) * 8;
+    if (row < n) {
+      IO<TIO>::ld8(t.base(bh) + int64_t(row) * t.s_n + col, t.vec != 0, r[i]);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) r[i][j] = 0.f;
+    }
+  }
+}
+template <typename TIO, int DH> FM_DEVICE void fm_small_stage(uint16_t* tile, const float (*r)[8], const float* f, int tid) {
+  typedef SmallCfg<TIO, DH> C;
+#pragma unroll
+  for (int i = 0; i < DH / 32; ++i) {
+    const int c = tid + 256 * i, row = c / (DH / 8), col = (c % (DH / 8)) * 8;
+    uint16_t* p = tile + row * C::PQ + col;
+    if constexpr (C::RAW) {
+      IO<fm_bf16>::st8(p, true, r[i]);                 // exact: they came from bf16
+    } else {
+      float w[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) w[j] = r[i][j] * f[i];
+      X3Row<DH>::store(p, fm_x3_split(w));
+    }
+  }
+}
+// largest squared row norm of the thread's wavefront with its row, as in k_maxnorm_keys: the first row among equal norms
+template <int DH> FM_DEVICE unsigned long long fm_small_norm_key(const float (*r)[8], int n, int tid) {
+  unsigned long long key = 0;
+#pragma unroll
+  for (int i = 0; i < DH / 32; ++i) {
+    const int row = (tid + 256 * i) / (DH / 8);
+    float s = 0.f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) s += r[i][j] * r[i][j];
+    s = fm_group_sum<DH / 8>(s);
+    uint32_t bits;
+    __builtin_memcpy(&bits, &s, 4);
+    const unsigned long long k = row < n ? (static_cast<unsigned long long>(bits) << 32) | uint32_t(~row) : 0ull;
+    key = k > key ? k : key;
+  }
+#pragma unroll
+  for (int m = DH / 8; m < 64; m <<= 1) { const unsigned long long o = fm_shfl_xor_u64(key, m); key = o > key ? o : key; }
+  return key;
+}
+// factor lim / norm, squared norm and its row from the four wavefronts' keys
+FM_DEVICE float fm_small_factor(const unsigned long long* keys, bool on, float lim, float& m2, int& nstar) {
+  m2 = 0.f; nstar = -1;
+  if (!on) return 1.0f;
+  unsigned long long k = keys[0];
+#pragma unroll
+  for (int w = 1; w < 4; ++w) k = keys[w] > k ? keys[w] : k;
+  m2 = fm_bits_f32(uint32_t(k >> 32));
+  nstar = int(~uint32_t(k));
+  return m2 > FM_MAXNORM_FLOOR ? lim * fm_rsqrtf(m2) : 0.0f;
+}
+
+// 32 x 32 tile of rows `a` and columns `b` (tiles of 32 rows in LDS)
+template <typename TIO, int DH> FM_DEVICE fm_f32x16 fm_small_tile(const uint16_t* a, const uint16_t* b, int lr, int lh) {
+  typedef SmallCfg<TIO, DH> C;
+  fm_f32x16 s = fm_zero16();
+#pragma unroll
+  for (int ks = 0; ks < DH / 16; ++ks) {
+    const uint16_t *pa = a + lr * C::PQ + 16 * ks + 8 * lh, *pb = b + lr * C::PQ + 16 * ks + 8 * lh;
+    if constexpr (C::RAW) s = fm_mfma_bf16(*reinterpret_cast<const fm_u16x8*>(pa), *reinterpret_cast<const fm_u16x8*>(pb), s);
+    else s = fm_x3_mma(X3Row<DH>::load(pa), X3Row<DH>::load(pb), s);
+  }
+  return s;
+}
+// acc (rows = features, column = the lane's token) += sum over the 32 rows r of tile: tile[r][.] p[r]
+template <typename TIO, int DH> FM_DEVICE void fm_small_acc(fm_f32x16* acc, const uint16_t* tile, const fm_f32x16& p, int lane) {
+  typedef SmallCfg<TIO, DH> C;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const X3 pb = fm_x3_split_acc(p, h);
+#pragma unroll
+    for (int ct = 0; ct < DH / 32; ++ct) {
+      if constexpr (C::RAW) {
+        const fm_u16x8 t = fm_bf16_load_tr(tile, C::PQ, 16 * h, 32 * ct, lane);
+        acc[ct] = fm_mfma_bf16(t, pb.p[1], acc[ct]);   // (the third plane is not used: the optimiser drops its making)
+        acc[ct] = fm_mfma_bf16(t, pb.p[0], acc[ct]);
+      } else {
+        acc[ct] = fm_x3_mma(X3Row<DH>::load_tr(tile, 16 * h, 32 * ct, lane), pb, acc[ct]);
+      }
+    }
+  }
+}
+
+// grid (1, bh), 256 threads
+template <typename TIO, int DH>
+FM_GLOBAL void FM_LAUNCH_BOUNDS2(256, 2) k_small_fwd(SmallArgs<TIO> A) {
+  typedef SmallCfg<TIO, DH> C;
+  constexpr int NT = DH / 32, N = C::N;
+  FM_DYN_SMEM(smem);
+  FM_SHARED unsigned long long keys[2][4];
+  uint16_t* Q = reinterpret_cast<uint16_t*>(smem);
+  uint16_t* K = Q + C::TILE;
+  uint16_t* V = K + C::TILE;
+  const int tid = FM_TID_X, lane = tid & 63, lr = lane & 31, lh = lane >> 5, bh = FM_BID_Y;
+  const int wave = FM_UNIFORM(tid >> 6), ti = wave >> 1, tj = wave & 1, off = A.nk - A.nq;
+  float rq[N][8], rk[N][8], rv[N][8];
+  fm_small_load<TIO, DH>(A.q, bh, A.nq, tid, rq);
+  fm_small_load<TIO, DH>(A.k, bh, A.nk, tid, rk);
+  fm_small_load<TIO, DH>(A.v, bh, A.nk, tid, rv);
+  float fq = A.sc, fk = A.sc;
+  if (A.norm_q | A.norm_k) {
+    const unsigned long long a = fm_small_norm_key<DH>(rq, A.nq, tid), b = fm_small_norm_key<DH>(rk, A.nk, tid);
+    if (lane == 0) { keys[0][wave] = a; keys[1][wave] = b; }
+    FM_SYNC();
+    float m2; int ns;
+    fq *= fm_small_factor(keys[0], A.norm_q != 0, A.lim, m2, ns);
+    fk *= fm_small_factor(keys[1], A.norm_k != 0, A.lim, m2, ns);
+  }
+  const float sq[2] = {fq, fq}, sk[2] = {fk, fk}, one[2] = {1.0f, 1.0f};
+  fm_small_stage<TIO, DH>(Q, rq, sq, tid);
+  fm_small_stage<TIO, DH>(K, rk, sk, tid);
+  fm_small_stage<TIO, DH>(V, rv, one, tid);
+  FM_SYNC();
+  fm_f32x16 acc[NT];
+#pragma unroll
+  for (int ct = 0; ct < NT; ++ct) acc[ct] = fm_zero16();
+  float gs = 0.f;
+  if (32 * ti < A.nq && 32 * tj < A.nk && !(A.causal && 32 * tj > 32 * ti + 31 + off)) {
+    fm_f32x16 s = fm_small_tile<TIO, DH>(K + 32 * tj * C::PQ, Q + 32 * ti * C::PQ, lr, lh);
+    int last = A.nk - 1 - 32 * tj;                     // last key row the lane's query sees
+    if (A.causal) { const int l = 32 * ti + lr + off - 32 * tj; last = l < last ? l : last; }
+    const float ss = C::RAW ? fq * fk : 1.0f;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const float x = C::RAW ? s[e] * ss : s[e], p = A.a0 + x * (A.a1 + A.a2 * x);
+      s[e] = fm_acc_row(e, lh) <= last ? p : 0.f;
+      gs += s[e];
+    }
+    fm_small_acc<TIO, DH>(acc, V + 32 * tj * C::PQ, s, lane);
+  }
+  FM_SYNC();
+  float* Os = reinterpret_cast<float*>(smem);
+  float* Gs = Os + 2 * 64 * C::OP;
+  fm_x3_put<DH, 64>(acc, Os, tj, 32 * ti + lr, lh);
+  gs += fm_shfl_xor(gs, 32);
+  if (lh == 0) Gs[tj * 64 + 32 * ti + lr] = gs;
+  FM_SYNC();
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const int c = tid + 256 * i, row = c / (DH / 8), col = (c % (DH / 8)) * 8;
+    if (row >= A.nq) continue;
+    float v[8];
+    fm_x3_sum8<DH, 64, 2>(Os, row, col, v);
+    const float gt = Gs[row] + Gs[64 + row], gi = 1.0f / gt;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] *= gi;
+    IO<TIO>::st8(A.out.base(bh) + int64_t(row) * A.out.s_n + col, A.out.vec != 0, v);
+    if (A.out_resid) {
+      float sv[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) sv[j] = fm_as_stored<TIO>(v[j]);
+      fm_store_resid8(A.out_resid + (int64_t(bh) * A.npad_q + row) * DH + col, v, sv);
+    }
+    if (col == 0) A.g.base(bh)[int64_t(row) * A.g.s_n] = gt;
+  }
+}
+
+// one result's rows: the two parts summed and scaled; returns the thread's share of sum value * raw
+template <int DH> FM_DEVICE float fm_small_result(const float* Os, float scale, const float (*raw)[8], int tid, float (*v)[8]) {
+  float b = 0.f;
+#pragma unroll
+  for (int i = 0; i < DH / 32; ++i) {
+    const int c = tid + 256 * i, row = c / (DH / 8), col = (c % (DH / 8)) * 8;
+    fm_x3_sum8<DH, 64, 2>(Os, row, col, v[i]);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) { v[i][j] *= scale; b += v[i][j] * raw[i][j]; }
+  }
+  return b;
+}
+// stores it, less the Jacobian's rank-one term in row nstar (see k_norm_fix)
+template <typename TIO, int DH>
+FM_DEVICE void fm_small_store(const TRef<TIO>& t, int bh, int n, int nstar, float coef, const float (*raw)[8], int tid, float (*v)[8]) {
+#pragma unroll
+  for (int i = 0; i < DH / 32; ++i) {
+    const int c = tid + 256 * i, row = c / (DH / 8), col = (c % (DH / 8)) * 8;
+    if (row >= n) continue;
+    if (row == nstar) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[i][j] -= coef * raw[i][j];
+    }
+    IO<TIO>::st8(t.base(bh) + int64_t(row) * t.s_n + col, t.vec != 0, v[i]);
+  }
+}
+
+// grid (1, bh), 256 threads
+template <typename TIO, int DH>
+FM_GLOBAL void FM_LAUNCH_BOUNDS2(256, (DH == 64 ? (sizeof(TIO) == 4 ? 1 : 2) : (sizeof(TIO) == 4 ? 2 : 3))) k_small_bwd(SmallArgs<TIO> A) {
+  typedef SmallCfg<TIO, DH> C;
+  constexpr int NT = DH / 32, N = C::N;
+  FM_DYN_SMEM(smem);
+  FM_SHARED unsigned long long keys[2][4];
+  FM_SHARED float bsum[2][4];
+  uint16_t* Q = reinterpret_cast<uint16_t*>(smem);
+  uint16_t* K = Q + C::TILE;
+  uint16_t* V = K + C::TILE;
+  uint16_t* G = V + C::TILE;                           // gh = dO / g (bf16 tensors: dO)
+  float* cs = reinterpret_cast<float*>(G + C::TILE);   // c = gh . o
+  float* gr = cs + 64;                                 // 1 / g
+  const int tid = FM_TID_X, lane = tid & 63, lr = lane & 31, lh = lane >> 5, bh = FM_BID_Y;
+  const int wave = FM_UNIFORM(tid >> 6), ti = wave >> 1, tj = wave & 1, off = A.nk - A.nq;
+  float rq[N][8], rk[N][8];
+  float fq = 1.0f, fk = 1.0f, m2q = 0.f, m2k = 0.f;
+  int nsq = -1, nsk = -1;
+  {
+    float rv[N][8], ro[N][8], rd[N][8], gi[N];
+    fm_small_load<TIO, DH>(A.q, bh, A.nq, tid, rq);
+    fm_small_load<TIO, DH>(A.k, bh, A.nk, tid, rk);
+    fm_small_load<TIO, DH>(A.v, bh, A.nk, tid, rv);
+    fm_small_load<TIO, DH>(A.o, bh, A.nq, tid, ro);
+    fm_small_load<TIO, DH>(A.d_o, bh, A.nq, tid, rd);
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const int c = tid + 256 * i, row = c / (DH / 8), col = (c % (DH / 8)) * 8;
+      gi[i] = row < A.nq ? 1.0f / A.g.base(bh)[int64_t(row) * A.g.s_n] : 0.f;
+      if (A.ores && row < A.nq) {
+        const fm_half8 rs = *reinterpret_cast<const fm_half8*>(A.ores + (int64_t(bh) * A.npad_q + row) * DH + col);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) ro[i][j] += float(rs[j]);
+      }
+    }
+    if (A.norm_q | A.norm_k) {
+      const unsigned long long a = fm_small_norm_key<DH>(rq, A.nq, tid), b = fm_small_norm_key<DH>(rk, A.nk, tid);
+      if (lane == 0) { keys[0][wave] = a; keys[1][wave] = b; }
+      FM_SYNC();
+      fq = fm_small_factor(keys[0], A.norm_q != 0, A.lim, m2q, nsq);
+      fk = fm_small_factor(keys[1], A.norm_k != 0, A.lim, m2k, nsk);
+    }
+    const float sq[2] = {A.sc * fq, A.sc * fq}, sk[2] = {A.sc * fk, A.sc * fk}, one[2] = {1.0f, 1.0f};
+    fm_small_stage<TIO, DH>(Q, rq, sq, tid);
+    fm_small_stage<TIO, DH>(K, rk, sk, tid);
+    fm_small_stage<TIO, DH>(V, rv, one, tid);
+    fm_small_stage<TIO, DH>(G, rd, gi, tid);
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const int c = tid + 256 * i;
+      float s = 0.f;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) s += rd[i][j] * ro[i][j];
+      s = fm_group_sum<DH / 8>(s * gi[i]);
+      if (c % (DH / 8) == 0) { cs[c / (DH / 8)] = s; gr[c / (DH / 8)] = gi[i]; }
+    }
+  }
+  FM_SYNC();
+  fm_f32x16 aq[NT], ak[NT], av[NT];
+#pragma unroll
+  for (int ct = 0; ct < NT; ++ct) { aq[ct] = fm_zero16(); ak[ct] = fm_zero16(); av[ct] = fm_zero16(); }
+  if (32 * ti < A.nq && 32 * tj < A.nk && !(A.causal && 32 * tj > 32 * ti + 31 + off)) {
+    const uint16_t *Qt = Q + 32 * ti * C::PQ, *Kt = K + 32 * tj * C::PQ, *Vt = V + 32 * tj * C::PQ, *Gt = G + 32 * ti * C::PQ;
+    const float ta2 = 2.0f * A.a2;
+    const float ss = C::RAW ? A.sc * A.sc * fq * fk : 1.0f;
+    const int diag = 32 * (ti - tj) + off;             // query row r sees key rows 0 .. r + diag
+    {
+      // rows = keys, column = the lane's query
+      fm_f32x16 s = fm_small_tile<TIO, DH>(Kt, Qt, lr, lh);
+      const fm_f32x16 dp = fm_small_tile<TIO, DH>(Vt, Gt, lr, lh);
+      const float c = cs[32 * ti + lr], gi = C::RAW ? gr[32 * ti + lr] : 1.0f;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const float ds = (A.a1 + ta2 * (s[e] * ss)) * (dp[e] * gi - c);
+        s[e] = A.causal && fm_acc_row(e, lh) > lr + diag ? 0.f : ds;
+      }
+      fm_small_acc<TIO, DH>(aq, Kt, s, lane);
+    }
+    {
+      // rows = queries, column = the lane's key (rows past the last query: gh = c = 0, they add nothing)
+      fm_f32x16 s = fm_small_tile<TIO, DH>(Qt, Kt, lr, lh);
+      fm_f32x16 dp = fm_small_tile<TIO, DH>(Gt, Vt, lr, lh);
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int r = fm_acc_row(e, lh);
+        const float gi = C::RAW ? gr[32 * ti + r] : 1.0f, x = s[e] * ss;
+        const float ds = (A.a1 + ta2 * x) * (dp[e] * gi - cs[32 * ti + r]), p = (A.a0 + x * (A.a1 + A.a2 * x)) * gi;
+        const bool hid = A.causal && lr > r + diag;
+        dp[e] = hid ? 0.f : ds;
+        s[e] = hid ? 0.f : p;
+      }
+      fm_small_acc<TIO, DH>(ak, Qt, dp, lane);
+      fm_small_acc<TIO, DH>(av, Gt, s, lane);
+    }
+  }
+  // the three results in turn through one region (two parts each), so that two to four workgroups share a CU
+  float* Os = reinterpret_cast<float*>(smem);
+  float vq[N][8], vk[N][8], vv[N][8];
+  FM_SYNC();
+  fm_x3_put<DH, 64>(aq, Os, tj, 32 * ti + lr, lh);
+  FM_SYNC();
+  float bq = fm_small_result<DH>(Os, A.sc * (A.jac ? fq : 1.0f) * (C::RAW ? A.sc * fk : 1.0f), rq, tid, vq);
+  FM_SYNC();
+  fm_x3_put<DH, 64>(ak, Os, ti, 32 * tj + lr, lh);
+  FM_SYNC();
+  float bk = fm_small_result<DH>(Os, A.sc * (A.jac ? fk : 1.0f) * (C::RAW ? A.sc * fq : 1.0f), rk, tid, vk);
+  FM_SYNC();
+  fm_x3_put<DH, 64>(av, Os, ti, 32 * tj + lr, lh);
+  FM_SYNC();
+  (void)fm_small_result<DH>(Os, 1.0f, rk, tid, vv);
+  float cq = 0.f, ck = 0.f;
+  if (A.jac) {
+#pragma unroll
+    for (int m = 1; m < 64; m <<= 1) { bq += fm_shfl_xor(bq, m); bk += fm_shfl_xor(bk, m); }
+    if (lane == 0) { bsum[0][wave] = bq; bsum[1][wave] = bk; }
+    FM_SYNC();
+    if (m2q > FM_MAXNORM_FLOOR) cq = ((bsum[0][0] + bsum[0][1]) + (bsum[0][2] + bsum[0][3])) / m2q;
+    if (m2k > FM_MAXNORM_FLOOR) ck = ((bsum[1][0] + bsum[1][1]) + (bsum[1][2] + bsum[1][3])) / m2k;
+  }
+  fm_small_store<TIO, DH>(A.out, bh, A.nq, cq != 0.f ? nsq : -1, cq, rq, tid, vq);
+  fm_small_store<TIO, DH>(A.dk, bh, A.nk, ck != 0.f ? nsk : -1, ck, rk, tid, vk);
+  fm_small_store<TIO, DH>(A.dv, bh, A.nk, -1, 0.f, rk, tid, vv);
+}

@@ -64,6 +64,15 @@ FM_DEVICE fm_f32x16 fm_x3_mma(const X3& a, const X3& b, fm_f32x16 c) {
   return c;
 }
 
+// transposed fragment of a row tile of 16-bit numbers: see Mma<fm_half>::load_tr
+FM_DEVICE fm_u16x8 fm_bf16_load_tr(const uint16_t* tile, int pitch, int tok0, int col0, int lane) {
+  const int lh = lane >> 5, half16 = (lane >> 4) & 1, s = (lane & 15) >> 2, q = lane & 3;
+  const uint16_t* p = tile + (tok0 + 4 * lh + s) * pitch + col0 + 16 * half16 + 4 * q;
+  const fm_u16x4 lo = fm_lds_tr4(p), hi = fm_lds_tr4(p + 8 * pitch);
+  fm_u16x8 r = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+  return r;
+}
+
 template <int DH> struct X3Row {
   static constexpr int PQ = 3 * DH + 8;                // pitch of a staged row: three planes and 16 bytes of padding
   static FM_DEVICE X3 load(const uint16_t* p) {        // fragment of a row tile (p: the lane's row and features)
@@ -72,17 +81,10 @@ template <int DH> struct X3Row {
     for (int pl = 0; pl < 3; ++pl) f.p[pl] = *reinterpret_cast<const fm_u16x8*>(p + pl * DH);
     return f;
   }
-  // transposed fragment: see Mma<fm_half>::load_tr
   static FM_DEVICE X3 load_tr(const uint16_t* tile, int tok0, int col0, int lane) {
-    const int lh = lane >> 5, half16 = (lane >> 4) & 1, s = (lane & 15) >> 2, q = lane & 3;
-    const uint16_t* p = tile + (tok0 + 4 * lh + s) * PQ + col0 + 16 * half16 + 4 * q;
     X3 f;
 #pragma unroll
-    for (int pl = 0; pl < 3; ++pl) {
-      const fm_u16x4 lo = fm_lds_tr4(p + pl * DH), hi = fm_lds_tr4(p + pl * DH + 8 * PQ);
-      fm_u16x8 r = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-      f.p[pl] = r;
-    }
+    for (int pl = 0; pl < 3; ++pl) f.p[pl] = fm_bf16_load_tr(tile + pl * DH, PQ, tok0, col0, lane);
     return f;
   }
   static FM_DEVICE void store(uint16_t* p, const X3& f) {

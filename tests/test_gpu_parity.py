@@ -6,7 +6,7 @@ import torch
 
 from tests.parity import (check_batch_head_strides, check_decode, check_forward, check_forward_backward,
                           check_norm_fold, make_inputs)
-from reproducing_fastmax_results_amd._capi import FLAG_F32_COMPUTE, FLAG_FORCE_DENSE, FLAG_FORCE_MOMENTS
+from reproducing_fastmax_results_amd._capi import FLAG_F32_COMPUTE, FLAG_FORCE_DENSE, FLAG_FORCE_MOMENTS, FLAG_NORM_SELF
 
 pytestmark = pytest.mark.gpu
 
@@ -245,6 +245,29 @@ def test_causal_more_keys_than_queries(lib, dtype, p, nq, nk):
     print(f"case causal nk>nq dtype={dtype} p={p} nq={nq} nk={nk}", flush=True)
     d = 64 if nq != 300 else 32
     check_forward_backward(lib, 3, nq, d, dtype, DEV, mask=True, p=p, nk=nk, seed=50)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("d", [32, 64])
+@pytest.mark.parametrize("nq,nk", [(32, 32), (33, 33), (64, 64), (17, 64), (64, 3), (20, 31)])
+def test_sequences_of_at_most_64_tokens(lib, dtype, d, nq, nk):
+    """One workgroup per batch*head (fm_small.h): one and two tiles each way, causal with the queries at the end of the
+    keys, norms found by the kernels themselves (the same bits as with the keys given: either way this route finds them itself)."""
+    print(f"case short sequences dtype={dtype} d={d} nq={nq} nk={nk}", flush=True)
+    check_forward_backward(lib, 3, nq, d, dtype, DEV, mask=False, p=2, nk=nk, seed=140)
+    if nq <= nk:
+        check_forward_backward(lib, 20, nq, d, dtype, DEV, mask=True, p=2, nk=nk, seed=141, saved=nq == nk)
+    check_norm_fold(lib, 3, nq, d, dtype, DEV, mask=False, p=1, nk=nk, seed=142, saved=False)
+    q, k, v, go = make_inputs(3, nq, nk, d, dtype, DEV, seed=143)
+    keys = lib.maxnorm_stats(q, k)
+    res = []
+    for flags, norm in ((0, (*keys, 1.5, True)), (FLAG_NORM_SELF, (None, None, 1.5, True))):
+        kw = dict(mask=False, inv_tau=0.5, p=2, flags=flags, norm=norm)
+        o, g = lib.forward(q, k, v, **kw)
+        res.append((o, g, *lib.backward(q, k, v, o, g, go, **kw)))
+    for a, b in zip(*res):
+        if nq > 16:                                      # (fewer queries: the forwards are different kernels)
+            assert torch.equal(a, b)
 
 
 @pytest.mark.parametrize("d", [32, 64])
