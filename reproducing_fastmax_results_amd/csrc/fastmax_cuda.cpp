@@ -6,6 +6,7 @@
 // from torch's caching allocator, work is enqueued on torch's current HIP
 // stream, and nothing synchronises.
 #include <torch/extension.h>
+#include <ATen/FuncTorchTLS.h>
 #include <c10/hip/HIPStream.h>
 
 #include <cmath>
@@ -596,6 +597,10 @@ struct AttentionNode : public torch::autograd::Function<AttentionNode> {
 // Attention with autograd.  norm: kNorm* above.
 torch::Tensor attention(const torch::Tensor& q, const torch::Tensor& k, const torch::Tensor& v, bool mask, int64_t norm, double temperature,
                         double a0, double a1, double a2, double lim, int64_t p) {
+  // refused here because a call without reverse-mode gradients passes the node, which would refuse these, by
+  if (const auto& transforms = at::functorch::functorchTLSAccessor()) transforms->checkSupportsCppAutogradFunction();
+  for (const torch::Tensor* t : {&q, &k, &v})
+    TORCH_CHECK(!t->defined() || !t->_fw_grad(/*level=*/0).defined(), "fastmax: forward-mode derivatives are not supported");
   const AttnConfig c{mask, norm, 1.0 / temperature, a0, a1, a2, lim, p};
   if (at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad()))
     return AttentionNode::apply(q, k, v, c);

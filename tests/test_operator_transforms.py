@@ -1,0 +1,32 @@
+"""What the attention operator refuses before it looks at devices: forward-mode derivatives and function transforms,
+of which its results would carry no trace."""
+import pytest
+import torch
+
+from reproducing_fastmax_results_amd.attention_mechanisms.score_function import (FASTMultiHeadAttention_Function,
+                                                                                 FastmaxNormAttention)
+
+CALLS = [lambda q, k, v: FASTMultiHeadAttention_Function.apply(q, k, v), FastmaxNormAttention.apply]
+
+
+@pytest.mark.parametrize("call", CALLS)
+@pytest.mark.parametrize("which", [0, 1, 2])
+def test_forward_mode_is_refused(call, which):
+    x = [torch.randn(1, 2, 8, 32) for _ in range(3)]
+    with torch.autograd.forward_ad.dual_level():
+        x[which] = torch.autograd.forward_ad.make_dual(x[which], torch.ones_like(x[which]))
+        with pytest.raises(RuntimeError, match="forward-mode"):
+            call(*x)
+        with torch.no_grad(), pytest.raises(RuntimeError, match="forward-mode"):
+            call(*x)
+
+
+@pytest.mark.parametrize("call", CALLS)
+def test_function_transforms_are_refused(call):
+    x = [torch.randn(3, 1, 2, 8, 32) for _ in range(3)]
+    with pytest.raises(RuntimeError, match="functorch transforms"):
+        torch.func.vmap(call)(*x)
+    with pytest.raises(RuntimeError, match="functorch transforms"):
+        torch.func.grad(lambda q: call(q, x[1][0], x[2][0]).sum())(x[0][0])
+    with pytest.raises(RuntimeError, match="CUDA|cuda|device|GPU"):     # afterwards a call gets as far as the device check
+        call(*(t[0] for t in x))
