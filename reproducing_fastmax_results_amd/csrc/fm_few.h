@@ -80,6 +80,10 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS(FM_THREADS) k_few(FewArgs<TIO> A, int nsplit) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int t = b + u * RPW + row;
+      if (t >= ke) {                                   // past the part's end: zero times an infinite entry would be NaN
+#pragma unroll
+        for (int j = 0; j < 8; ++j) vx[u][j] = 0.f;
+      }
 #pragma unroll
       for (int i = 0; i < NQ; ++i) {
         float s = 0.f;

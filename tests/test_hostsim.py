@@ -315,3 +315,12 @@ def test_kernel_sources_under_address_sanitizer(tmp_path):
     run = subprocess.run([exe], capture_output=True, text=True, env=dict(os.environ, ASAN_OPTIONS="detect_leaks=0"))
     assert run.returncode == 0, run.stdout[-2000:] + run.stderr[-4000:]
     assert "AddressSanitizer" not in run.stderr
+
+
+def test_few_queries_keep_infinities(sim):
+    # the last rows of a part are loaded by several lanes; those past its end must not add zero times infinity
+    q, k, v, _ = make_inputs(1, 1, 60, 64, torch.float32, "cpu", seed=27)
+    k = k.abs() * torch.sign(q)                          # all weights positive
+    v[:, -1, 5] = float("inf")
+    o, _ = sim.forward(q, k, v, mask=False, inv_tau=1.0, p=2)
+    assert o[0, 0, 5] == float("inf") and torch.isfinite(o[0, 0, :5]).all()
