@@ -564,29 +564,29 @@ template <typename TIO> SmallArgs<TIO> small_args(const FastmaxDesc* d, const Pl
   a.norm_q = self || d->norm.q_keys; a.norm_k = self || d->norm.k_keys; a.jac = d->norm.grad != 0; a.lim = d->norm.lim;
   return a;
 }
-template <typename TIO, int DH>
+template <typename TIO, int DH, bool FULL>
 int run_small_fwd(const FastmaxDesc* d, const Plan& p, const void* q, const void* k, const void* v, void* o, float* g, char* ws,
                   fm_stream_t stream) {
   SmallArgs<TIO> a = small_args<TIO>(d, p, q, k, v);
   a.out = mref<TIO>(o, d->so); a.g = mref<float>(g, d->sg);
   if (p.keep_resid) a.out_resid = reinterpret_cast<fm_half*>(ws + p.ores);
-  const size_t lds = SmallCfg<TIO, DH>::fwd_lds();
-  fm_allow_lds(reinterpret_cast<const void*>(&k_small_fwd<TIO, DH>), lds);
+  const size_t lds = SmallCfg<TIO, DH, FULL>::fwd_lds();
+  fm_allow_lds(reinterpret_cast<const void*>(&k_small_fwd<TIO, DH, FULL>), lds);
   ProfScope prof(FM_K_FWD, stream);
-  FM_KERNEL_LAUNCH((k_small_fwd<TIO, DH>), fm_dim3(1, d->bh), fm_dim3(256), lds, stream, a);
+  FM_KERNEL_LAUNCH((k_small_fwd<TIO, DH, FULL>), fm_dim3(1, d->bh), fm_dim3(256), lds, stream, a);
   return fm_launch_status();
 }
-template <typename TIO, int DH>
+template <typename TIO, int DH, bool FULL>
 int run_small_bwd(const FastmaxDesc* d, const Plan& p, const void* q, const void* k, const void* v, const void* o, const float* g,
                   const void* d_o, void* dq, void* dk, void* dv, const char* fws, fm_stream_t stream) {
   SmallArgs<TIO> a = small_args<TIO>(d, p, q, k, v);
   a.o = cref<TIO>(o, d->so); a.d_o = cref<TIO>(d_o, d->sdo); a.g = fm_ref<float>(const_cast<float*>(g), d->sg);   // read only
   a.out = mref<TIO>(dq, d->sdq); a.dk = mref<TIO>(dk, d->sdk); a.dv = mref<TIO>(dv, d->sdv);
   if (fws && p.keep_resid) a.ores = reinterpret_cast<const fm_half*>(fws + p.ores);
-  const size_t lds = SmallCfg<TIO, DH>::bwd_lds();
-  fm_allow_lds(reinterpret_cast<const void*>(&k_small_bwd<TIO, DH>), lds);
+  const size_t lds = SmallCfg<TIO, DH, FULL>::bwd_lds();
+  fm_allow_lds(reinterpret_cast<const void*>(&k_small_bwd<TIO, DH, FULL>), lds);
   ProfScope prof(FM_K_DKV, stream);
-  FM_KERNEL_LAUNCH((k_small_bwd<TIO, DH>), fm_dim3(1, d->bh), fm_dim3(256), lds, stream, a);
+  FM_KERNEL_LAUNCH((k_small_bwd<TIO, DH, FULL>), fm_dim3(1, d->bh), fm_dim3(256), lds, stream, a);
   return fm_launch_status();
 }
 
@@ -837,9 +837,11 @@ static int forward_one(const FastmaxDesc* desc, const void* q, const void* k, co
   char* ws = static_cast<char*>(workspace);
   fm_stream_t stream = static_cast<fm_stream_t>(hip_stream);
   if (p.tiny) {
+    if (p.half)
+      return desc->d == 64 ? run_small_fwd<fm_bf16, 64, false>(desc, p, q, k, v, o, g, ws, stream) : run_small_fwd<fm_bf16, 32, false>(desc, p, q, k, v, o, g, ws, stream);
     if (desc->dtype == FASTMAX_BF16)
-      return desc->d == 64 ? run_small_fwd<fm_bf16, 64>(desc, p, q, k, v, o, g, ws, stream) : run_small_fwd<fm_bf16, 32>(desc, p, q, k, v, o, g, ws, stream);
-    return desc->d == 64 ? run_small_fwd<float, 64>(desc, p, q, k, v, o, g, ws, stream) : run_small_fwd<float, 32>(desc, p, q, k, v, o, g, ws, stream);
+      return desc->d == 64 ? run_small_fwd<fm_bf16, 64, true>(desc, p, q, k, v, o, g, ws, stream) : run_small_fwd<fm_bf16, 32, true>(desc, p, q, k, v, o, g, ws, stream);
+    return desc->d == 64 ? run_small_fwd<float, 64, true>(desc, p, q, k, v, o, g, ws, stream) : run_small_fwd<float, 32, true>(desc, p, q, k, v, o, g, ws, stream);
   }
   if (p.half) {
     if (desc->d == FM_WIDE_HEAD) return run_forward<fm_bf16, fm_half, FM_WIDE_HEAD, 1>(desc, p, q, k, v, o, g, ws, stream);
@@ -921,11 +923,14 @@ static int backward_one(const FastmaxDesc* desc, const void* q, const void* k, c
   const char* fws = static_cast<const char*>(fwd_ws);
   fm_stream_t stream = static_cast<fm_stream_t>(hip_stream);
   if (p.tiny) {
+    if (p.half)
+      return desc->d == 64 ? run_small_bwd<fm_bf16, 64, false>(desc, p, q, k, v, o, g, d_o, dq, dk, dv, fws, stream)
+                           : run_small_bwd<fm_bf16, 32, false>(desc, p, q, k, v, o, g, d_o, dq, dk, dv, fws, stream);
     if (desc->dtype == FASTMAX_BF16)
-      return desc->d == 64 ? run_small_bwd<fm_bf16, 64>(desc, p, q, k, v, o, g, d_o, dq, dk, dv, fws, stream)
-                           : run_small_bwd<fm_bf16, 32>(desc, p, q, k, v, o, g, d_o, dq, dk, dv, fws, stream);
-    return desc->d == 64 ? run_small_bwd<float, 64>(desc, p, q, k, v, o, g, d_o, dq, dk, dv, fws, stream)
-                         : run_small_bwd<float, 32>(desc, p, q, k, v, o, g, d_o, dq, dk, dv, fws, stream);
+      return desc->d == 64 ? run_small_bwd<fm_bf16, 64, true>(desc, p, q, k, v, o, g, d_o, dq, dk, dv, fws, stream)
+                           : run_small_bwd<fm_bf16, 32, true>(desc, p, q, k, v, o, g, d_o, dq, dk, dv, fws, stream);
+    return desc->d == 64 ? run_small_bwd<float, 64, true>(desc, p, q, k, v, o, g, d_o, dq, dk, dv, fws, stream)
+                         : run_small_bwd<float, 32, true>(desc, p, q, k, v, o, g, d_o, dq, dk, dv, fws, stream);
   }
   if (p.half) {
     if (desc->d == FM_WIDE_HEAD) return run_backward_wide<fm_bf16, fm_half, FM_WIDE_HEAD>(desc, p, q, k, v, o, g, d_o, dq, dk, dv, fws, ws, stream);

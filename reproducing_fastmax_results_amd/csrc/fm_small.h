@@ -6,7 +6,8 @@
 // norms, dQ, dK + dV and the Jacobian's row.  Here every tensor is read once and every result written once.
 // fp32 tensors: products of three bf16 planes (fm_x3.h).  bf16 tensors: the operands are the caller's numbers themselves (one
 // plane, exact), every factor (temperature, norms, 1 / g) is applied in fp32 to what the products give, and the weights
-// are split in two planes (16 bits), so no range but fp32's applies here.  Wavefront (i, j) of the four works on the 32 x 32 tile of query tile i and key tile j; two sums per
+// are split in two planes (16 bits; the general kernels' _Float16 weights have 11), or in three (FULL, all 24 bits) where
+// the caller asked for fp32 arithmetic or the weights may cancel; no range but fp32's applies here.  Wavefront (i, j) of the four works on the 32 x 32 tile of query tile i and key tile j; two sums per
 // result meet in LDS.  The backward forms the scores twice, keys along the accumulator rows for dQ and queries along
 // them for dK and dV: each is then the operand of the product that follows, without a transposition.
 // B*H = 1024, 50 tokens, D = 32, normalised (26 MB forward, 53 MB backward): fp32 forward with its norms 23 -> 11.3 us, backward
@@ -28,9 +29,10 @@ template <typename TIO> struct SmallArgs {
   int norm_q, norm_k, jac; float lim;   // max-norm scaling of q / k; jac: gradients with respect to the raw tensors
 };
 
-template <typename TIO, int DH> struct SmallCfg {
+template <typename TIO, int DH, bool FULL> struct SmallCfg {
   static constexpr bool RAW = sizeof(TIO) == 2;        // operands are the caller's numbers
-  static constexpr int PL = RAW ? 1 : 3, PP = RAW ? 2 : 3;          // planes of an operand in LDS, of a weight
+  static constexpr int PP = RAW && !FULL ? 2 : 3;      // planes of a weight
+  static constexpr int PL = RAW ? 1 : 3;        // planes of an operand in LDS
   static constexpr int N = DH / 32;                    // eight-feature items of a tensor per thread
   static constexpr int PQ = PL * DH + 8, TILE = 64 * PQ, OP = DH + 4;
   static constexpr size_t OS = size_t(2) * 64 * OP * 4;            // one result's two parts
@@ -51,8 +53,8 @@ FM_DEVICE void fm_small_load(const TRef<const TIO>& t, int bh, int n, int tid, f
     }
   }
 }
-template <typename TIO, int DH> FM_DEVICE void fm_small_stage(uint16_t* tile, const float (*r)[8], const float* f, int tid) {
-  typedef SmallCfg<TIO, DH> C;
+template <typename TIO, int DH, bool FULL> FM_DEVICE void fm_small_stage(uint16_t* tile, const float (*r)[8], const float* f, int tid) {
+  typedef SmallCfg<TIO, DH, FULL> C;
 #pragma unroll
   for (int i = 0; i < DH / 32; ++i) {
     const int c = tid + 256 * i, row = c / (DH / 8), col = (c % (DH / 8)) * 8;
@@ -99,8 +101,8 @@ FM_DEVICE float fm_small_factor(const unsigned long long* keys, bool on, float l
 }
 
 // 32 x 32 tile of rows `a` and columns `b` (tiles of 32 rows in LDS)
-template <typename TIO, int DH> FM_DEVICE fm_f32x16 fm_small_tile(const uint16_t* a, const uint16_t* b, int lr, int lh) {
-  typedef SmallCfg<TIO, DH> C;
+template <typename TIO, int DH, bool FULL> FM_DEVICE fm_f32x16 fm_small_tile(const uint16_t* a, const uint16_t* b, int lr, int lh) {
+  typedef SmallCfg<TIO, DH, FULL> C;
   fm_f32x16 s = fm_zero16();
 #pragma unroll
   for (int ks = 0; ks < DH / 16; ++ks) {
@@ -111,8 +113,8 @@ template <typename TIO, int DH> FM_DEVICE fm_f32x16 fm_small_tile(const uint16_t
   return s;
 }
 // acc (rows = features, column = the lane's token) += sum over the 32 rows r of tile: tile[r][.] p[r]
-template <typename TIO, int DH> FM_DEVICE void fm_small_acc(fm_f32x16* acc, const uint16_t* tile, const fm_f32x16& p, int lane) {
-  typedef SmallCfg<TIO, DH> C;
+template <typename TIO, int DH, bool FULL> FM_DEVICE void fm_small_acc(fm_f32x16* acc, const uint16_t* tile, const fm_f32x16& p, int lane) {
+  typedef SmallCfg<TIO, DH, FULL> C;
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
     const X3 pb = fm_x3_split_acc(p, h);
@@ -120,7 +122,8 @@ template <typename TIO, int DH> FM_DEVICE void fm_small_acc(fm_f32x16* acc, cons
     for (int ct = 0; ct < DH / 32; ++ct) {
       if constexpr (C::RAW) {
         const fm_u16x8 t = fm_bf16_load_tr(tile, C::PQ, 16 * h, 32 * ct, lane);
-        acc[ct] = fm_mfma_bf16(t, pb.p[1], acc[ct]);   // (the third plane is not used: the optimiser drops its making)
+        if constexpr (C::PP == 3) acc[ct] = fm_mfma_bf16(t, pb.p[2], acc[ct]);   // (else the optimiser drops its making)
+        acc[ct] = fm_mfma_bf16(t, pb.p[1], acc[ct]);
         acc[ct] = fm_mfma_bf16(t, pb.p[0], acc[ct]);
       } else {
         acc[ct] = fm_x3_mma(X3Row<DH>::load_tr(tile, 16 * h, 32 * ct, lane), pb, acc[ct]);
@@ -130,9 +133,9 @@ template <typename TIO, int DH> FM_DEVICE void fm_small_acc(fm_f32x16* acc, cons
 }
 
 // grid (1, bh), 256 threads
-template <typename TIO, int DH>
+template <typename TIO, int DH, bool FULL>
 FM_GLOBAL void FM_LAUNCH_BOUNDS2(256, 2) k_small_fwd(SmallArgs<TIO> A) {
-  typedef SmallCfg<TIO, DH> C;
+  typedef SmallCfg<TIO, DH, FULL> C;
   constexpr int NT = DH / 32, N = C::N;
   FM_DYN_SMEM(smem);
   FM_SHARED unsigned long long keys[2][4];
@@ -155,16 +158,16 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(256, 2) k_small_fwd(SmallArgs<TIO> A) {
     fk *= fm_small_factor(keys[1], A.norm_k != 0, A.lim, m2, ns);
   }
   const float sq[2] = {fq, fq}, sk[2] = {fk, fk}, one[2] = {1.0f, 1.0f};
-  fm_small_stage<TIO, DH>(Q, rq, sq, tid);
-  fm_small_stage<TIO, DH>(K, rk, sk, tid);
-  fm_small_stage<TIO, DH>(V, rv, one, tid);
+  fm_small_stage<TIO, DH, FULL>(Q, rq, sq, tid);
+  fm_small_stage<TIO, DH, FULL>(K, rk, sk, tid);
+  fm_small_stage<TIO, DH, FULL>(V, rv, one, tid);
   FM_SYNC();
   fm_f32x16 acc[NT];
 #pragma unroll
   for (int ct = 0; ct < NT; ++ct) acc[ct] = fm_zero16();
   float gs = 0.f;
   if (32 * ti < A.nq && 32 * tj < A.nk && !(A.causal && 32 * tj > 32 * ti + 31 + off)) {
-    fm_f32x16 s = fm_small_tile<TIO, DH>(K + 32 * tj * C::PQ, Q + 32 * ti * C::PQ, lr, lh);
+    fm_f32x16 s = fm_small_tile<TIO, DH, FULL>(K + 32 * tj * C::PQ, Q + 32 * ti * C::PQ, lr, lh);
     int last = A.nk - 1 - 32 * tj;                     // last key row the lane's query sees
     if (A.causal) { const int l = 32 * ti + lr + off - 32 * tj; last = l < last ? l : last; }
     const float ss = C::RAW ? fq * fk : 1.0f;
@@ -174,7 +177,7 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(256, 2) k_small_fwd(SmallArgs<TIO> A) {
       s[e] = fm_acc_row(e, lh) <= last ? p : 0.f;
       gs += s[e];
     }
-    fm_small_acc<TIO, DH>(acc, V + 32 * tj * C::PQ, s, lane);
+    fm_small_acc<TIO, DH, FULL>(acc, V + 32 * tj * C::PQ, s, lane);
   }
   FM_SYNC();
   float* Os = reinterpret_cast<float*>(smem);
@@ -231,9 +234,9 @@ FM_DEVICE void fm_small_store(const TRef<TIO>& t, int bh, int n, int nstar, floa
 }
 
 // grid (1, bh), 256 threads
-template <typename TIO, int DH>
+template <typename TIO, int DH, bool FULL>
 FM_GLOBAL void FM_LAUNCH_BOUNDS2(256, (DH == 64 ? (sizeof(TIO) == 4 ? 1 : 2) : (sizeof(TIO) == 4 ? 2 : 3))) k_small_bwd(SmallArgs<TIO> A) {
-  typedef SmallCfg<TIO, DH> C;
+  typedef SmallCfg<TIO, DH, FULL> C;
   constexpr int NT = DH / 32, N = C::N;
   FM_DYN_SMEM(smem);
   FM_SHARED unsigned long long keys[2][4];
@@ -274,10 +277,10 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(256, (DH == 64 ? (sizeof(TIO) == 4 ? 1 : 2) : (
       fk = fm_small_factor(keys[1], A.norm_k != 0, A.lim, m2k, nsk);
     }
     const float sq[2] = {A.sc * fq, A.sc * fq}, sk[2] = {A.sc * fk, A.sc * fk}, one[2] = {1.0f, 1.0f};
-    fm_small_stage<TIO, DH>(Q, rq, sq, tid);
-    fm_small_stage<TIO, DH>(K, rk, sk, tid);
-    fm_small_stage<TIO, DH>(V, rv, one, tid);
-    fm_small_stage<TIO, DH>(G, rd, gi, tid);
+    fm_small_stage<TIO, DH, FULL>(Q, rq, sq, tid);
+    fm_small_stage<TIO, DH, FULL>(K, rk, sk, tid);
+    fm_small_stage<TIO, DH, FULL>(V, rv, one, tid);
+    fm_small_stage<TIO, DH, FULL>(G, rd, gi, tid);
 #pragma unroll
     for (int i = 0; i < N; ++i) {
       const int c = tid + 256 * i;
@@ -299,20 +302,20 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(256, (DH == 64 ? (sizeof(TIO) == 4 ? 1 : 2) : (
     const int diag = 32 * (ti - tj) + off;             // query row r sees key rows 0 .. r + diag
     {
       // rows = keys, column = the lane's query
-      fm_f32x16 s = fm_small_tile<TIO, DH>(Kt, Qt, lr, lh);
-      const fm_f32x16 dp = fm_small_tile<TIO, DH>(Vt, Gt, lr, lh);
+      fm_f32x16 s = fm_small_tile<TIO, DH, FULL>(Kt, Qt, lr, lh);
+      const fm_f32x16 dp = fm_small_tile<TIO, DH, FULL>(Vt, Gt, lr, lh);
       const float c = cs[32 * ti + lr], gi = C::RAW ? gr[32 * ti + lr] : 1.0f;
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
         const float ds = (A.a1 + ta2 * (s[e] * ss)) * (dp[e] * gi - c);
         s[e] = A.causal && fm_acc_row(e, lh) > lr + diag ? 0.f : ds;
       }
-      fm_small_acc<TIO, DH>(aq, Kt, s, lane);
+      fm_small_acc<TIO, DH, FULL>(aq, Kt, s, lane);
     }
     {
       // rows = queries, column = the lane's key (rows past the last query: gh = c = 0, they add nothing)
-      fm_f32x16 s = fm_small_tile<TIO, DH>(Qt, Kt, lr, lh);
-      fm_f32x16 dp = fm_small_tile<TIO, DH>(Gt, Vt, lr, lh);
+      fm_f32x16 s = fm_small_tile<TIO, DH, FULL>(Qt, Kt, lr, lh);
+      fm_f32x16 dp = fm_small_tile<TIO, DH, FULL>(Gt, Vt, lr, lh);
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
         const int r = fm_acc_row(e, lh);
@@ -322,8 +325,8 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(256, (DH == 64 ? (sizeof(TIO) == 4 ? 1 : 2) : (
         dp[e] = hid ? 0.f : ds;
         s[e] = hid ? 0.f : p;
       }
-      fm_small_acc<TIO, DH>(ak, Qt, dp, lane);
-      fm_small_acc<TIO, DH>(av, Gt, s, lane);
+      fm_small_acc<TIO, DH, FULL>(ak, Qt, dp, lane);
+      fm_small_acc<TIO, DH, FULL>(av, Gt, s, lane);
     }
   }
   // the three results in turn through one region (two parts each), so that two to four workgroups share a CU

@@ -324,3 +324,17 @@ def test_few_queries_keep_infinities(sim):
     v[:, -1, 5] = float("inf")
     o, _ = sim.forward(q, k, v, mask=False, inv_tau=1.0, p=2)
     assert o[0, 0, 5] == float("inf") and torch.isfinite(o[0, 0, :5]).all()
+
+
+def test_short_sequences_of_bf16_tensors_in_fp32(sim):
+    """F32_COMPUTE keeps all 24 bits of the weights: f1 - f2 = 1.5 * 2^-17 of two keys with values 1 and -1.  Each weight
+    (between 1 and 2) is rounded by 2^-24 at most, twice; so is the score: 4 * 2^-24 / (1.5 * 2^-17) = 2.1 %, the store 0.4 %."""
+    n, d = 17, 32
+    q = torch.zeros(1, n, d); k = torch.zeros(1, 2, d); v = torch.zeros(1, 2, d)
+    q[..., :3] = 1.0
+    k[..., 0], k[..., 1], k[0, 0, 2] = 0.3828125, 2.0 ** -9 * 1.9453125, 2.0 ** -17 * 1.5
+    v[0, 0, :], v[0, 1, :] = 1.0, -1.0
+    f = 1.0 + k.double().sum(-1)
+    want = float((f[0, 0] - f[0, 1]) / f.sum())
+    o, _ = sim.forward(q.bfloat16(), k.bfloat16(), v.bfloat16(), mask=False, inv_tau=1.0, p=1, flags=_capi.FLAG_F32_COMPUTE)
+    assert ((o.double() - want).abs() <= 0.025 * want).all(), (o[0, 0, 0], want)
