@@ -54,26 +54,6 @@ static inline int fm_static_scratch(void** out) {
 namespace {
 
 inline int fm_launch_status() { return fm_after_launch() ? FASTMAX_ERR_LAUNCH : FASTMAX_OK; }
-#if defined(FM_HOSTSIM)
-inline void fm_allow_lds(const void*, size_t) {}
-#else
-// Dynamic LDS above the 64 KiB default has to be allowed once per kernel function (and device); the
-// attribute call costs microseconds of host time, so it is made the first time a kernel asks for more
-// than it has been granted so far and skipped afterwards.
-inline void fm_allow_lds(const void* fn, size_t bytes) {
-  if (bytes <= 64 * 1024) return;
-  struct Key { const void* fn; int dev; bool operator==(const Key& o) const { return fn == o.fn && dev == o.dev; } };
-  struct Hash { size_t operator()(const Key& k) const { return std::hash<const void*>()(k.fn) ^ (size_t(k.dev) * 0x9e3779b97f4a7c15ull); } };
-  static std::mutex mu;
-  static std::unordered_map<Key, size_t, Hash> granted;
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) dev = 0;
-  std::lock_guard<std::mutex> lock(mu);
-  size_t& have = granted[Key{fn, dev}];
-  if (bytes <= have) return;
-  if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, int(bytes)) == hipSuccess) have = bytes;
-}
-#endif
 
 // ---- per-kernel timing: compiled only into the bench build of this file (-DFM_BENCH_AIDS); in the product
 // library a ProfScope is an empty object and no launch touches any process-wide state ---------------------

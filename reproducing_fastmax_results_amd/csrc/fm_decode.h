@@ -163,8 +163,9 @@ k_decode(TRef<const TIO> k, TRef<const TIO> v, TRef<const TIO> q, int n_new, int
 // per token and workgroup, 1.7 ms for 4 096 tokens at 16 batch*heads; the same sums are three 32 x 32 x 16 products
 // per 16 tokens and value column.
 //
-// grid (D / 4, bh), 256 threads: the workgroup owns the same [R][4] block of the state as in k_decode, wavefront w its
-// value column c = 4 cb + w.  Per tile of 128 tokens the keys (times inv_tau, as _Float16) are staged row-major and
+// grid (D / 4, bh), 512 threads: the workgroup owns the same [R][4] block of the state as in k_decode.  Two groups of four
+// wavefronts take every other tile of 128 tokens, wavefront w of a group the value column c = 4 cb + w.  Per tile
+// the keys (times inv_tau, as _Float16) are staged row-major and
 // the four value columns, a row of ones (zero past the end of the prompt) and three rows of zeros as rows over the
 // tokens.  Per k-step of 16 tokens a wavefront reads the two key fragments with transposing LDS reads and uses them
 // as B operand and, times its value column's fragment, as A operand: the slice  sum_t v_tc k'_ta k'_tb  of its column
@@ -172,9 +173,15 @@ k_decode(TRef<const TIO> k, TRef<const TIO> v, TRef<const TIO> q, int n_new, int
 // columns share is dealt by k-step, wavefront w taking the k-steps u = w (mod 4): the denominators' order-2 sums
 // (the same three products with the bare key fragments), and the rows 0 .. D of numerators and denominators in one go
 // as  sum_t z_tn' x_tn  with z = (k', then the rows of x) and x = (the four value columns, ones, zeros): three more
-// products.  At the end the four wavefronts' parts of the shared sums meet in LDS and are added in a fixed order, and
+// products.  At the end the wavefronts' parts meet in LDS and are added in a fixed order, and
 // every sum is ADDED to the state in memory (each address by exactly one lane: no atomics, the same bits every run).
 // Operands are rounded to _Float16 (k', and the products v k'), the sums are fp32.
+//
+// What bounds it is latency: 16 batch*heads are one workgroup per CU, each a chain over the tiles (fetch, LDS, products).
+// Two groups halve the chain (LDS and 256 registers per lane leave no room for more).  At the end every state entry is
+// read before the first is written: as read-modify-writes one after the other they were up to 72 memory latencies in a
+// row.  One group and read-modify-writes, then this, microseconds per call at 64, 1024 and 4096 tokens:
+// B*H = 1: 17, 32, 81 and 11, 20, 50;  B*H = 16: 19, 35, 86 and 13, 24, 58;  B*H = 64: 100, 187, 474 and 46, 96, 262.
 template <int DH> struct DecAbsCfg {
   typedef Mma<fm_half> M;
   static constexpr int TT = 128;                       // tokens per tile
@@ -183,12 +190,14 @@ template <int DH> struct DecAbsCfg {
   static constexpr int XP = TT + M::PAD;
   static constexpr int TILE_E = TT * PQ + XR * XP;
   static constexpr int NSH = 6;                        // accumulator tiles of the shared sums per wavefront
-  static constexpr size_t RED_BYTES = size_t(4) * (NSH / 2) * 16 * 64 * 4;   // they meet in LDS three tiles at a time
-  static constexpr size_t lds_bytes() { return size_t(2) * TILE_E * 2 > RED_BYTES ? size_t(2) * TILE_E * 2 : RED_BYTES; }
+  static constexpr int NG = 2, NTH = NG * 256;         // groups of four wavefronts
+  static constexpr size_t RED_BYTES = size_t(4) * NG * (NSH / 2) * 16 * 64 * 4;   // they meet in LDS three tiles at a time
+  static constexpr size_t STAGE_BYTES = size_t(NG) * 2 * TILE_E * 2;
+  static constexpr size_t lds_bytes() { return STAGE_BYTES > RED_BYTES ? STAGE_BYTES : RED_BYTES; }
 };
 
 template <typename TIO, int DH>
-FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_THREADS, 1)
+FM_GLOBAL void FM_LAUNCH_BOUNDS2((DecAbsCfg<DH>::NTH), 2)
 k_decode_absorb_mma(TRef<const TIO> k, TRef<const TIO> v, int n_new, float inv_tau, float* FM_RESTRICT state) {
   static_assert(DH == 64, "two 32-row tiles per feature axis");
   typedef fm_half E;
@@ -197,10 +206,11 @@ k_decode_absorb_mma(TRef<const TIO> k, TRef<const TIO> v, int n_new, float inv_t
   typedef DecAbsCfg<DH> C;
   constexpr int TT = C::TT, PQ = C::PQ, XP = C::XP, NSTEP = TT / M::KSTEP;
   FM_DYN_SMEM(smem);
-  E* const buf0 = reinterpret_cast<E*>(smem);
+  const int lane = FM_TID_X & 63, lr = lane & 31, lh = lane >> 5;
+  const int wave8 = FM_UNIFORM(FM_TID_X >> 6), wave = wave8 & 3, grp = wave8 >> 2;
+  const int tid = FM_TID_X & 255;                        // within the group
+  E* const buf0 = reinterpret_cast<E*>(smem) + grp * 2 * C::TILE_E;
   E* const buf1 = buf0 + C::TILE_E;
-  const int tid = FM_TID_X, lane = tid & 63, lr = lane & 31, lh = lane >> 5;
-  const int wave = FM_UNIFORM(tid >> 6);
   // the sixteen workgroups of a batch*head read the same keys: behind one L2 (145 -> 28 MB fetched for 4 096 tokens at 16 heads, 0.125 -> 0.097 ms)
   int cb, bh;
   fm_xcd_map(FM_GDIM_X, FM_GDIM_Y, cb, bh);
@@ -212,12 +222,12 @@ k_decode_absorb_mma(TRef<const TIO> k, TRef<const TIO> v, int n_new, float inv_t
   const TIO* vb = v.base(bh);
 
   // global memory -> registers: a thread's four 16-byte pieces of the key rows, and (threads below TT) a token's four values
-  constexpr int CPR = DH / 8, NK = TT * CPR / FM_THREADS;
+  constexpr int CPR = DH / 8, NK = TT * CPR / 256;
   float kreg[NK][8], vreg[4];
   auto fetch = [&](int t0) FM_ALWAYS_INLINE {
 #pragma unroll
     for (int i = 0; i < NK; ++i) {
-      const int c = tid + FM_THREADS * i, row = t0 + c / CPR, f0 = (c % CPR) * 8;
+      const int c = tid + 256 * i, row = t0 + c / CPR, f0 = (c % CPR) * 8;
       if (row < n_new) IO<TIO>::ld8(kb + int64_t(row) * k.s_n + f0, k.vec != 0, kreg[i]);
       else {
 #pragma unroll
@@ -232,7 +242,7 @@ k_decode_absorb_mma(TRef<const TIO> k, TRef<const TIO> v, int n_new, float inv_t
   auto put = [&](E* b, int t0) FM_ALWAYS_INLINE {
 #pragma unroll
     for (int i = 0; i < NK; ++i) {
-      const int c = tid + FM_THREADS * i;
+      const int c = tid + 256 * i;
       float sc[8];
 #pragma unroll
       for (int j = 0; j < 8; ++j) sc[j] = kreg[i][j] * inv_tau;
@@ -246,7 +256,7 @@ k_decode_absorb_mma(TRef<const TIO> k, TRef<const TIO> v, int n_new, float inv_t
     }
   };
   // rows 5 .. 7 of both buffers: zeros, written once
-  for (int i = tid; i < 2 * 3 * XP; i += FM_THREADS) {
+  for (int i = tid; i < 2 * 3 * XP; i += 256) {
     E* b = i < 3 * XP ? buf0 : buf1;
     b[TT * PQ + 5 * XP + (i % (3 * XP))] = E(0.0f);
   }
@@ -256,14 +266,16 @@ k_decode_absorb_mma(TRef<const TIO> k, TRef<const TIO> v, int n_new, float inv_t
 #pragma unroll
   for (int i = 0; i < C::NSH; ++i) sh[i] = fm_zero16();
 
-  fetch(0);
-  put(buf0, 0);
-  if (TT < n_new) fetch(TT);
+  const int g0 = grp * TT;                               // tiles past the end of the prompt are zeros
+  fetch(g0);
+  put(buf0, g0);
+  if (C::NG * TT < n_new) fetch(C::NG * TT + g0);
   FM_SYNC();
   int par = 0;
-  for (int t0 = 0; t0 < n_new; t0 += TT) {
+  for (int tb = 0; tb < n_new; tb += C::NG * TT) {
     const E* cbuf = par ? buf1 : buf0;
     const E* xt = cbuf + TT * PQ;
+    if (tb + g0 < n_new) {
 #pragma unroll
     for (int u = 0; u < NSTEP; ++u) {
       const frag k0 = M::load_tr(cbuf, PQ, 16 * u, 0, lane), k1 = M::load_tr(cbuf, PQ, 16 * u, 32, lane);
@@ -282,61 +294,93 @@ k_decode_absorb_mma(TRef<const TIO> k, TRef<const TIO> v, int n_new, float inv_t
         sh[5] = M::mma(xs, xs, sh[5]);
       }
     }
-    if (t0 + TT < n_new) {
-      put(par ? buf0 : buf1, t0 + TT);
-      if (t0 + 2 * TT < n_new) fetch(t0 + 2 * TT);
+    }
+    if (tb + C::NG * TT < n_new) {
+      put(par ? buf0 : buf1, tb + C::NG * TT + g0);
+      if (tb + 2 * C::NG * TT < n_new) fetch(tb + 2 * C::NG * TT + g0);
     }
     FM_SYNC();
     par ^= 1;
   }
 
-  // the wavefront's own column: entries (a, b) with a <= b go to their pair rows
+  float* red = reinterpret_cast<float*>(smem);           // the staging buffers are spent: the loop ended on a barrier
   auto pair_row = [&](int a, int b) { return 1 + DH + a * DH - a * (a - 1) / 2 + (b - a); };
+  // the value columns: entries (a, b) with a <= b go to their pair rows; group 0 writes accumulator entries 0 .. 7 of its
+  // column's three tiles, group 1 entries 8 .. 15 (16 rows further down), each with the other group's part from LDS
+  {
+    float old[3][8];
+    float* at[3][8];
+    bool live[3][8];
 #pragma unroll
-  for (int e = 0; e < 16; ++e) {
-    const int ra = fm_acc_row(e, lh);
-    if (ra <= lr) num[int64_t(pair_row(ra, lr)) * 4 + wave] += a00[e];
-    num[int64_t(pair_row(ra, 32 + lr)) * 4 + wave] += a01[e];
-    if (ra <= lr) num[int64_t(pair_row(32 + ra, 32 + lr)) * 4 + wave] += a11[e];
+    for (int e = 0; e < 8; ++e) {
+      const int ra = fm_acc_row(e, lh) + 16 * grp;
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        live[i][e] = i == 1 || ra <= lr;
+        at[i][e] = num + (live[i][e] ? int64_t(pair_row(i == 2 ? 32 + ra : ra, i == 0 ? lr : 32 + lr)) * 4 + wave : wave);
+        old[i][e] = *at[i][e];
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const fm_f32x16& a = i == 0 ? a00 : i == 1 ? a01 : a11;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) red[((wave8 * 3 + i) * 8 + e) * 64 + lane] = grp ? a[e] : a[8 + e];
+    }
+    FM_SYNC();
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const fm_f32x16& a = i == 0 ? a00 : i == 1 ? a01 : a11;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float other = red[(((wave8 ^ 4) * 3 + i) * 8 + e) * 64 + lane];
+        if (live[i][e]) *at[i][e] = old[i][e] + ((grp ? other : a[e]) + (grp ? a[8 + e] : other));
+      }
+    }
   }
-  // the shared sums: the four parts through LDS (the staging buffers are spent: the loop ended on a barrier), three
-  // tiles at a time; wavefront w adds entries 4 w .. 4 w + 3 of every tile in the order of the wavefronts
-  float* red = reinterpret_cast<float*>(smem);           // [wave][tile of the round][e][lane]
-  constexpr int HALF = C::NSH / 2;
+  // the shared sums: the eight parts through LDS, three tiles at a time; wavefront w adds entries 2 w and 2 w + 1 of every
+  // tile in the order of the wavefronts
+  constexpr int HALF = C::NSH / 2, NW = 4 * C::NG, EPW = 16 / NW;
+  float* sat[C::NSH][EPW];                               // where they go; null: nowhere
+  float sold[C::NSH][EPW];
+#pragma unroll
+  for (int i = 0; i < C::NSH; ++i)
+#pragma unroll
+    for (int x = 0; x < EPW; ++x) {
+      const int ra = fm_acc_row(EPW * wave8 + x, lh);
+      float* p = nullptr;
+      if (i == 0) { if (ra <= lr) p = den + pair_row(ra, lr); }            // denominators of the pair rows
+      else if (i == 1) p = den + pair_row(ra, 32 + lr);
+      else if (i == 2) { if (ra <= lr) p = den + pair_row(32 + ra, 32 + lr); }
+      else if (i < 5) {                                  // rows 1 + a: column n < 4 a numerator, n = 4 the denominator
+        const int a = 32 * (i - 3) + ra;
+        if (lr < 4) p = num + int64_t(1 + a) * 4 + lr;
+        else if (lr == 4) p = den + 1 + a;
+      } else if (ra == 4) {                              // row 0: the ones row of z against the columns of x
+        if (lr < 4) p = num + lr;
+        else if (lr == 4) p = den;
+      }
+      sat[i][x] = p;
+      sold[i][x] = *(p ? p : den);
+    }
 #pragma unroll
   for (int rnd = 0; rnd < 2; ++rnd) {
-    if (rnd) FM_SYNC();
+    FM_SYNC();                                           // what lay there has been read
 #pragma unroll
     for (int i = 0; i < HALF; ++i)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) red[((wave * HALF + i) * 16 + e) * 64 + lane] = sh[rnd * HALF + i][e];
+      for (int e = 0; e < 16; ++e) red[((wave8 * HALF + i) * 16 + e) * 64 + lane] = sh[rnd * HALF + i][e];
     FM_SYNC();
 #pragma unroll
-    for (int i = 0; i < HALF; ++i) {
+    for (int i = 0; i < HALF; ++i)
 #pragma unroll
-      for (int e4 = 0; e4 < 4; ++e4) {
-        const int e = 4 * wave + e4;
+      for (int x = 0; x < EPW; ++x) {
         float sum = 0.f;
 #pragma unroll
-        for (int w = 0; w < 4; ++w) sum += red[((w * HALF + i) * 16 + e) * 64 + lane];
-        const int ra = fm_acc_row(e, lh);
-        if (rnd == 0) {
-          // denominators of the pair rows: tiles (0,0), (0,1), (1,1)
-          if (i == 0) { if (ra <= lr) den[pair_row(ra, lr)] += sum; }
-          else if (i == 1) den[pair_row(ra, 32 + lr)] += sum;
-          else if (ra <= lr) den[pair_row(32 + ra, 32 + lr)] += sum;
-        } else if (i < 2) {
-          // rows 1 + a: column n < 4 a numerator, n = 4 the denominator
-          const int a = 32 * i + ra;
-          if (lr < 4) num[int64_t(1 + a) * 4 + lr] += sum;
-          else if (lr == 4) den[1 + a] += sum;
-        } else if (ra == 4) {
-          // row 0: the ones row of z against the columns of x
-          if (lr < 4) num[lr] += sum;
-          else if (lr == 4) den[0] += sum;
-        }
+        for (int w = 0; w < NW; ++w) sum += red[((w * HALF + i) * 16 + EPW * wave8 + x) * 64 + lane];
+        float* p = sat[rnd * HALF + i][x];
+        if (p) *p = sold[rnd * HALF + i][x] + sum;
       }
-    }
   }
 }
 
@@ -358,7 +402,8 @@ int fm_decode_run(const FastmaxDesc* d, const void* q, const void* k, const void
   if constexpr (sizeof(TIO) == 2 && DH == 64) {
     if (fm_decode_absorb_mma_applies<TIO, DH>(quad, q != nullptr, n_new)) {
       typedef DecAbsCfg<DH> C;
-      FM_KERNEL_LAUNCH((k_decode_absorb_mma<TIO, DH>), fm_dim3(DH / 4, d->bh), fm_dim3(FM_THREADS), C::lds_bytes(), stream, kr, vr,
+      fm_allow_lds(reinterpret_cast<const void*>(&k_decode_absorb_mma<TIO, DH>), C::lds_bytes());
+      FM_KERNEL_LAUNCH((k_decode_absorb_mma<TIO, DH>), fm_dim3(DH / 4, d->bh), fm_dim3(C::NTH), C::lds_bytes(), stream, kr, vr,
                        n_new, d->inv_tau, state);
       return fm_after_launch() ? FASTMAX_ERR_LAUNCH : FASTMAX_OK;
     }

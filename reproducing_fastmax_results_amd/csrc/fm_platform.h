@@ -5,6 +5,9 @@
 // the same names onto a host-thread simulator so that indexing and lane layouts
 // can be checked without a GPU; the shipped library never defines FM_HOSTSIM.
 #pragma once
+#include <functional>
+#include <mutex>
+#include <unordered_map>
 #include <cstddef>
 #include <cstdint>
 
@@ -253,3 +256,24 @@ FM_DEVICE uint32_t fm_cvt_pk_bf16(float a, float b) {
 FM_DEVICE fm_bf16 fm_f32_to_bf16(float f) { return fm_bf16(fm_cvt_pk_bf16(f, f)); }
 #endif
 FM_DEVICE float fm_bits_f32(uint32_t u) { float f; __builtin_memcpy(&f, &u, 4); return f; }
+
+#if defined(FM_HOSTSIM)
+static inline void fm_allow_lds(const void*, size_t) {}
+#else
+// Dynamic LDS above the 64 KiB default has to be allowed once per kernel function (and device); the
+// attribute call costs microseconds of host time, so it is made the first time a kernel asks for more
+// than it has been granted so far and skipped afterwards.
+static inline void fm_allow_lds(const void* fn, size_t bytes) {
+  if (bytes <= 64 * 1024) return;
+  struct Key { const void* fn; int dev; bool operator==(const Key& o) const { return fn == o.fn && dev == o.dev; } };
+  struct Hash { size_t operator()(const Key& k) const { return std::hash<const void*>()(k.fn) ^ (size_t(k.dev) * 0x9e3779b97f4a7c15ull); } };
+  static std::mutex mu;
+  static std::unordered_map<Key, size_t, Hash> granted;
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) dev = 0;
+  std::lock_guard<std::mutex> lock(mu);
+  size_t& have = granted[Key{fn, dev}];
+  if (bytes <= have) return;
+  if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, int(bytes)) == hipSuccess) have = bytes;
+}
+#endif
