@@ -46,7 +46,6 @@ PEAK_HBM_GBS = 8000.0
 # were when the named summary was made.
 TRAFFIC = {
     (4096, 2, "bf16", 0, "dkv"): {"bytes": int((42622.6 * 2 + 32768.1) * 1024), "source": "profiles/c2_bf16_hbm_traffic.md"},
-    (4096, 2, "f32", 0, "dk"): {"bytes": int((324657.1 * 2 + 32768.9) * 1024), "source": "profiles/c2_fp32_kernel_trace.md"},
     (65536, 1, "bf16", 0, "dkv"): {"bytes": int((402949.3 * 2 + 393223.9) * 1024), "source": "profiles/long_order1_bf16_hbm_traffic.md"},
     (65536, 2, "bf16", 0, "build"): {"bytes": int((130128.6 * 2 + 544747.5) * 1024), "source": "profiles/long_order2_bf16_hbm_traffic.md"},
     (65536, 2, "bf16", 0, "dkv"): {"bytes": int((609337.0 * 2 + 262146.4) * 1024), "source": "profiles/long_order2_bf16_hbm_traffic.md"},
@@ -307,7 +306,7 @@ def c1_line(lib, dev, with_cpu):
     gpu_us = 1e3 * e0.elapsed_time(e1) / 20
     out = {"workload": "configs[0]: order-2 forward, unmasked, fp32, B=1 H=2 N=256 D=Dv=32", "gpu_us_per_call": gpu_us,
            "gpu_tokens_per_s": 256 / (gpu_us * 1e-6),
-           "note": "a call of 512 (b,h,token) rows: launch-bound on the GPU (two launches, host side of the Python front included)"}
+           "note": "a call of 512 (b,h,token) rows: launch-bound on the GPU (one launch, host side of the Python front included)"}
     if with_cpu:
         O.factorised_forward(q, k, v, mask=False, tau=tau, p=2)
         t0 = time.perf_counter()
