@@ -541,6 +541,10 @@ struct AttnResult { torch::Tensor q, k, v, o, g, saved, qk, kk; bool fold = fals
 AttnResult attention_forward(const torch::Tensor& q_, const torch::Tensor& k_, const torch::Tensor& v_, const AttnConfig& c, bool save) {
   TORCH_CHECK_VALUE(q_.dim() == 3 || q_.dim() == 4, "q, k, and v should be either 3 or 4 dimensional tensors. "
                     "If 3D: (b*h,n,d), if 4D: (b,h,n,d).");
+  // Gradients of the raw tensors come from the folded kernels alone; the separate pass below would hand out those of the
+  // normalised ones.
+  TORCH_CHECK(c.norm != kNormGradOfRaw || fold_possible(q_, k_, c.mask), "fastmax: no folded normalisation for causal attention with "
+              "more keys than queries (normalise q and k with FastmaxNormalize first)");
   AttnResult r;
   const bool wide = c.norm != kNormGradOfRaw;          // the folded kernels stop at 64
   r.q = pad_features(q_, wide); r.k = pad_features(k_, wide); r.v = pad_features(v_, wide);

@@ -1,5 +1,5 @@
 """What the attention operator refuses before it looks at devices: forward-mode derivatives and function transforms,
-of which its results would carry no trace."""
+of which its results would carry no trace, and the one problem whose folded normalisation has no gradient."""
 import pytest
 import torch
 
@@ -30,3 +30,14 @@ def test_function_transforms_are_refused(call):
         torch.func.grad(lambda q: call(q, x[1][0], x[2][0]).sum())(x[0][0])
     with pytest.raises(RuntimeError, match="CUDA|cuda|device|GPU"):     # afterwards a call gets as far as the device check
         call(*(t[0] for t in x))
+
+
+@pytest.mark.parametrize("grad", [False, True])
+def test_folded_normalisation_refuses_more_keys_than_queries_under_the_mask(grad):
+    """Two sub-problems would share one Jacobian: refused, with or without gradients, and not answered with the gradients
+    of the normalised tensors.  (Unmasked, such a call gets as far as the device check.)"""
+    q, k, v = (torch.randn(1, 2, n, 32, requires_grad=grad) for n in (8, 12, 12))
+    with pytest.raises(RuntimeError, match="more keys than queries"):
+        FastmaxNormAttention.apply(q, k, v, True)
+    with pytest.raises(RuntimeError, match="CUDA|cuda|device|GPU"):
+        FastmaxNormAttention.apply(q, k, v, False)
