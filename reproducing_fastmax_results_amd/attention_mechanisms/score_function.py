@@ -37,19 +37,23 @@ CENTRE_NONE, CENTRE_FEATURE, CENTRE_TOKEN = 0, 1, 2
 _NORM_OFF, _GRAD_OF_NORMALISED, _GRAD_OF_RAW = 0, 1, 2   # the binding's `attention`: max-norm scaling of q and k, and which gradients
 
 
-_HEAD_SIZES = (32, 64)      # what every kernel is built for (bf16 attention also 128: see the binding)
+_HEAD_SIZES = (32, 64)      # what every kernel is built for
+_WIDE_HEAD = 128            # bf16 attention alone also runs at this width (dense tiles; no normalisation or decoding kernels)
 
 
-def _pad_features(x):
+def _pad_features(x, wide=False):
     """x itself, or a copy zero-padded along the feature axis to the next head size the kernels
-    are built for (the binding does the same for ``attention``)."""
+    are built for (the binding does the same for ``attention``).  ``wide``: the caller's kernels also exist at 128
+    (attention on bf16 tensors)."""
     d = x.shape[-1]
-    for size in _HEAD_SIZES:
+    sizes = _HEAD_SIZES + ((_WIDE_HEAD,) if wide and x.dtype == torch.bfloat16 else ())
+    for size in sizes:
         if d == size:
             return x
         if d < size:
             return torch.nn.functional.pad(x, (0, size - d))
-    raise RuntimeError(f"fastmax: unsupported head size {d} for {x.dtype} (these kernels cover up to {_HEAD_SIZES[-1]})")
+    raise RuntimeError(f"fastmax: unsupported head size {d} for {x.dtype} (the kernels cover up to {_HEAD_SIZES[-1]}, "
+                       f"attention on bfloat16 tensors up to {_WIDE_HEAD})")
 
 
 class FastmaxNormalize(torch.autograd.Function):
@@ -81,20 +85,42 @@ def _fold_possible(q, k, mask):
     return not (mask and k.shape[-2] > q.shape[-2])
 
 
-class FastmaxNormAttention:
+class FastmaxNormAttention(torch.autograd.Function):
     """Fastmax attention on ``lim * x / max_n ||x_n||_2`` of q and k (per batch and head), the
     normalisation folded into the kernels: one statistics pass reads q and k once, the attention
     kernels scale the rows as they load them, and the backward returns the gradients with respect to
     the RAW q and k, the normalisation's own Jacobian included (the dQ / dK kernels scale what they
     store and one small kernel adds the rank-one term of the row with the largest norm).  Replaces the
     reference's ``apply_norm`` pass (``fastmax_cuda_forward.cu:326-338``) and the autograd graph of its
-    Python variants (``score_function.py:40-55``); semantics of ``transformer/model.py:97-102``.  The
-    autograd node is the binding's (``attention``)."""
+    Python variants (``score_function.py:40-55``); semantics of ``transformer/model.py:97-102``.  ``apply``
+    goes to the binding's autograd node (``attention``); ``forward`` and ``backward`` are the same two steps for
+    a function of the caller's own that brings its ``ctx``."""
 
     @staticmethod
     def apply(q, k, v, mask=False, lim=1.0, temperature=1.0, a0=1.0, a1=1.0, a2=0.5, p=2):
         return _ext.attention(q, k, v, bool(mask), _GRAD_OF_RAW, float(temperature), float(a0), float(a1), float(a2), float(lim),
                               int(p))
+
+    @staticmethod
+    def forward(ctx, q, k, v, mask=False, lim=1.0, temperature=1.0, a0=1.0, a1=1.0, a2=0.5, p=2):
+        d = q.shape[-1]
+        q, k, v = _pad_features(q), _pad_features(k), _pad_features(v)
+        qk, kk = _ext.maxnorm_stats(q, k)
+        cfg = (bool(mask), 1.0 / float(temperature), float(a0), float(a1), float(a2), int(p))
+        o, g, saved = _ext.forward_norm(q, k, v, qk, kk, float(lim), *cfg, 0, 0)
+        if any(ctx.needs_input_grad[:3]):
+            ctx.save_for_backward(q, k, v, o, g, saved, qk, kk)
+        ctx.cfg, ctx.lim, ctx.d = cfg, float(lim), d
+        return o[..., :d]
+
+    @staticmethod
+    def backward(ctx, grad_output):
+        q, k, v, o, g, saved, qk, kk = ctx.saved_tensors
+        d = ctx.d
+        if q.shape[-1] != d:
+            grad_output = _pad_features(grad_output)
+        gq, gk, gv = _ext.backward_norm(q, k, v, o, g, grad_output, saved, qk, kk, ctx.lim, True, *ctx.cfg, 0, 0)
+        return (gq[..., :d], gk[..., :d], gv[..., :d]) + (None,) * 7
 
 
 class FastmaxOutputNoise(torch.autograd.Function):
@@ -152,7 +178,7 @@ def fastmax_with_dormant_steps(q, k, v, drop_noise=None, rpe_matrix=None, mask=F
     return o
 
 
-class FASTMultiHeadAttention_Function:
+class FASTMultiHeadAttention_Function(torch.autograd.Function):
     """Same call as reference ``transformer/model.py:16``.  q, k, v: ``(b, h, n, d)`` or
     ``(b*h, n, d)``.  ``drop_noise``, ``rpe_matrix`` and ``dropout`` are accepted and unused,
     as in the reference extension (``fastmax_cuda_forward.cu:289, 443``).  With
@@ -160,8 +186,9 @@ class FASTMultiHeadAttention_Function:
     semantics spelled out in ``transformer/model.py:97-102``) and, like the reference (its extension
     has no backward of apply_norm), the returned gradients are those with respect to the normalised q and k.
     Head sizes other than 32 and 64 (up to 64; on bfloat16 tensors up to 128) run zero-padded to the next
-    size the kernels have.  The autograd node is the binding's (``attention``): where a gradient is asked for it keeps
-    the key-side copies and prefix states the forward built, and the backward reuses them.
+    size the kernels have.  ``apply`` goes to the binding's autograd node (``attention``): where a gradient is asked
+    for it keeps the key-side copies and prefix states the forward built, and the backward reuses them.  ``forward`` and
+    ``backward`` are the same two steps for a function of the caller's own that brings its ``ctx``.
     """
 
     @staticmethod
@@ -169,6 +196,46 @@ class FASTMultiHeadAttention_Function:
               temperature=1.0, a0=1.0, a1=1.0, a2=0.5, lim=1.0, p=2):
         return _ext.attention(q, k, v, bool(mask), _GRAD_OF_NORMALISED if normalize else _NORM_OFF, float(temperature), float(a0),
                               float(a1), float(a2), float(lim), int(p))
+
+    @staticmethod
+    def forward(ctx, q, k, v, drop_noise=None, rpe_matrix=None, mask=False, dropout=0.0, normalize=False,
+                temperature=1.0, a0=1.0, a1=1.0, a2=0.5, lim=1.0, p=2):
+        if q.dim() not in (3, 4):
+            raise ValueError("q, k, and v should be either 3 or 4 dimensional tensors. "
+                             "If 3D: (b*h,n,d), if 4D: (b,h,n,d).")
+        d = q.shape[-1]
+        q, k, v = _pad_features(q, True), _pad_features(k, True), _pad_features(v, True)
+        ctx.cfg, ctx.d, ctx.fold = (bool(mask), 1.0 / float(temperature), float(a0), float(a1), float(a2), int(p)), d, None
+        keys = ()
+        if normalize and q.shape[-1] > _HEAD_SIZES[-1]:
+            q = q * (float(lim) / q.float().norm(dim=-1).amax(dim=-1)[..., None, None]).to(q.dtype)
+            k = k * (float(lim) / k.float().norm(dim=-1).amax(dim=-1)[..., None, None]).to(k.dtype)
+        elif normalize and _fold_possible(q, k, mask):
+            keys, ctx.fold = _ext.maxnorm_stats(q, k), float(lim)
+        elif normalize:
+            q = _ext.normalize(q, CENTRE_NONE, True, float(lim))
+            k = _ext.normalize(k, CENTRE_NONE, True, float(lim))
+        if keys:
+            o, g, saved = _ext.forward_norm(q, k, v, *keys, ctx.fold, *ctx.cfg, 0, 0)
+        elif any(ctx.needs_input_grad[:3]):
+            o, g, saved = _ext.forward_save(q, k, v, *ctx.cfg, 0, 0)
+        else:
+            return _ext.forward_ex(q, k, v, *ctx.cfg, 0, 0)[0][..., :d]
+        if any(ctx.needs_input_grad[:3]):
+            ctx.save_for_backward(q, k, v, o, g, saved, *keys)
+        return o[..., :d]
+
+    @staticmethod
+    def backward(ctx, grad_output):
+        q, k, v, o, g, saved, *keys = ctx.saved_tensors
+        d = ctx.d
+        if q.shape[-1] != d:
+            grad_output = _pad_features(grad_output, True)
+        if keys:
+            grads = _ext.backward_norm(q, k, v, o, g, grad_output, saved, *keys, ctx.fold, False, *ctx.cfg, 0, 0)
+        else:
+            grads = _ext.backward_saved(q, k, v, o, g, grad_output, saved, *ctx.cfg, 0, 0)
+        return tuple(x[..., :d] for x in grads) + (None,) * 11
 
 
 class FastmaxDecodeState:

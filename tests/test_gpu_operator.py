@@ -458,3 +458,42 @@ def test_operator_with_dormant_steps(sf, dtype, d):
     o_plain = sf.fastmax_with_dormant_steps(qd, kd, vd, noise.to(DEV), rpe.to(DEV), mask=True, temperature=t, p=2)
     o_ref = sf.FASTMultiHeadAttention_Function.apply(qd, kd, vd, None, None, True, 0.0, False, t, 1.0, 1.0, 0.5, 1.0, 2)
     assert torch.equal(o_plain, o_ref)
+
+
+class _Doubled(torch.autograd.Function):
+    """A function of a caller's own around an attention class: forward and backward with its ctx, outputs doubled."""
+
+    @staticmethod
+    def forward(ctx, cls, *args):
+        class Ctx:
+            needs_input_grad = ctx.needs_input_grad[1:]
+
+            def save_for_backward(self, *tensors):
+                self.saved_tensors = tensors
+        ctx.inner, ctx.cls = Ctx(), cls
+        return 2.0 * cls.forward(ctx.inner, *args)
+
+    @staticmethod
+    def backward(ctx, go):
+        return (None,) + ctx.cls.backward(ctx.inner, 2.0 * go)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n,nk,d", [(50, 50, 32), (70, 70, 64), (70, 70, 48), (70, 90, 64)])
+def test_forward_and_backward_of_the_attention_classes(sf, dtype, n, nk, d):
+    """The classes' own forward and backward give what their apply gives, bit for bit (factors of two are exact)."""
+    print(f"case attention classes {dtype} {n} {nk} {d}", flush=True)
+    F, N = sf.FASTMultiHeadAttention_Function, sf.FastmaxNormAttention
+    calls = [(F, (None, None, True, 0.0, normalize, 4.0, 1.0, 1.0, 0.5, 1.5, 2)) for normalize in (False, True)]
+    if n == nk:
+        calls.append((N, (True, 1.5, 2.0)))
+    x = [rnd(2, 2, m, d, seed=60 + i).to(dtype).to(DEV).requires_grad_(True) for i, m in enumerate((n, nk, nk))]
+    go = rnd(2, 2, n, d, seed=64).to(dtype).to(DEV)
+    for cls, args in calls:
+        o = cls.apply(*x, *args)
+        grads = torch.autograd.grad(o, x, go)
+        o2 = _Doubled.apply(cls, *x, *args)
+        for a, b in zip((o2, *torch.autograd.grad(o2, x, go)), (o, *grads)):
+            assert torch.equal(a, 2 * b)
+        with torch.no_grad():
+            assert torch.equal(_Doubled.apply(cls, *x, *args), 2 * cls.apply(*x, *args))

@@ -1,5 +1,8 @@
 """What the attention operator refuses before it looks at devices: forward-mode derivatives and function transforms,
-of which its results would carry no trace, and the one problem whose folded normalisation has no gradient."""
+of which its results would carry no trace, and the one problem whose folded normalisation has no gradient; and that the
+attention classes are autograd functions."""
+import types
+
 import pytest
 import torch
 
@@ -41,3 +44,11 @@ def test_folded_normalisation_refuses_more_keys_than_queries_under_the_mask(grad
         FastmaxNormAttention.apply(q, k, v, True)
     with pytest.raises(RuntimeError, match="CUDA|cuda|device|GPU"):
         FastmaxNormAttention.apply(q, k, v, False)
+
+
+@pytest.mark.parametrize("cls", [FASTMultiHeadAttention_Function, FastmaxNormAttention])
+def test_the_attention_classes_are_autograd_functions(cls):
+    assert issubclass(cls, torch.autograd.Function)
+    x = torch.randn(1, 2, 8, 32)
+    with pytest.raises(RuntimeError, match="CUDA|cuda|device|GPU"):
+        cls.forward(types.SimpleNamespace(needs_input_grad=(True,) * 3), x, x, x)
