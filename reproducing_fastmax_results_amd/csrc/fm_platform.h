@@ -37,6 +37,7 @@ typedef uint16_t fm_u16x4 __attribute__((ext_vector_type(4)));
 #define FM_RESTRICT
 #define FM_UNIFORM(x) (x)
 #define FM_OPAQUE_ZERO() 0
+#define FM_ARGS_AGAIN(a) (a)
 #define FM_SCHED_FENCE()
 #define FM_SCHED_MFMA_DS(n)
 #define FM_KEEP_BRANCH()
@@ -108,6 +109,7 @@ template <typename V4, typename T> inline V4 fm_lds_tr4_any(const T* p) {
 FM_DEVICE fm_half4 fm_lds_tr4(const fm_half* p) { return fm_lds_tr4_any<fm_half4>(p); }
 FM_DEVICE fm_u16x4 fm_lds_tr4(const uint16_t* p) { return fm_lds_tr4_any<fm_u16x4>(p); }
 FM_DEVICE float fm_fmaxf(float a, float b) { return a != a ? b : (b != b ? a : (a > b ? a : b)); }   // drops a NaN, like fmaxf
+FM_DEVICE float fm_absf(float x) { return __builtin_fabsf(x); }
 FM_DEVICE float fm_clampf(float x, float lim) { return x > lim ? lim : (x < -lim ? -lim : x); }
 FM_DEVICE float fm_rsqrtf(float a) { return 1.0f / std::sqrt(a); }
 FM_DEVICE float fm_sqrtf(float a) { return std::sqrt(a); }
@@ -129,6 +131,14 @@ FM_DEVICE float fm_sqrtf(float a) { return std::sqrt(a); }
 // same tile apart, so the second is a fresh read instead of 16 more live registers.
 static __device__ __forceinline__ int fm_opaque_zero() { int z = 0; asm volatile("" : "+v"(z)); return z; }
 #define FM_OPAQUE_ZERO() fm_opaque_zero()
+// A kernel's only argument, read from memory again: what a rarely taken second pass needs of it stays out of the registers
+// of the first (as FM_TID_X + FM_OPAQUE_ZERO() keeps out what is made from the thread index).
+template <typename T> static __device__ __forceinline__ const T& fm_args_again(const T&) {
+  const __attribute__((address_space(4))) void* p = (const __attribute__((address_space(4))) void*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return *(const T*)p;
+}
+#define FM_ARGS_AGAIN(a) fm_args_again(a)
 // Nothing is scheduled across this point (keeps the live ranges of one phase out of the next).
 #define FM_SCHED_FENCE() __builtin_amdgcn_sched_barrier(0)
 // Asks the instruction scheduler to interleave the LDS reads of this block with its matrix
@@ -215,6 +225,7 @@ FM_DEVICE fm_u16x4 fm_lds_tr4(const uint16_t* p) {
   return r;
 }
 FM_DEVICE float fm_fmaxf(float a, float b) { return fmaxf(a, b); }
+FM_DEVICE float fm_absf(float x) { return __builtin_fabsf(x); }
 // clamp to [-lim, lim] in one instruction (v_med3_f32)
 FM_DEVICE float fm_clampf(float x, float lim) { return __builtin_amdgcn_fmed3f(x, -lim, lim); }
 FM_DEVICE float fm_rsqrtf(float a) { return rsqrtf(a); }

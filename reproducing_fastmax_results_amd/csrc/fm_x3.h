@@ -73,8 +73,25 @@ FM_DEVICE fm_u16x8 fm_bf16_load_tr(const uint16_t* tile, int pitch, int tok0, in
   return r;
 }
 
+// How a kernel holds and multiplies its rows.  X3Row: three planes, the products above.  F32Row: fp32 rows and
+// v_mfma_f32_32x32x2_f32, for the workgroups whose sums came out non-finite (see fm_x3_look).
+//   Own              the lane's own token: CH features from feat(c, lh) in chunk c of NOWN
+//   score, score2    score tile (rows = stream tokens, column = own token), and the second one beside it
+//   accum, accum2    acc (rows = features) += rows of a stream tile times a weight tile, one product and two
 template <int DH> struct X3Row {
   static constexpr int PQ = 3 * DH + 8;                // pitch of a staged row: three planes and 16 bytes of padding
+  static constexpr bool PIPE = true;                   // the next stage is loaded while one is multiplied
+  static constexpr int CH = 8, NOWN = DH / 16, NT = DH / 32;
+  struct Own { X3 f[NOWN]; };
+  static FM_DEVICE int feat(int c, int lh) { return 16 * c + 8 * lh; }
+  template <typename TIO> static FM_DEVICE void ld(const TIO* p, bool vec, float v[CH]) { IO<TIO>::ld8(p, vec, v); }
+  static FM_DEVICE void add_half(const fm_half* p, float v[CH]) {
+    const fm_half8 h = *reinterpret_cast<const fm_half8*>(p);
+#pragma unroll
+    for (int i = 0; i < CH; ++i) v[i] += float(h[i]);
+  }
+  static FM_DEVICE void set(Own& o, int c, const float v[CH]) { o.f[c] = fm_x3_split(v); }
+  static FM_DEVICE void fence(int) {}
   static FM_DEVICE X3 load(const uint16_t* p) {        // fragment of a row tile (p: the lane's row and features)
     X3 f;
 #pragma unroll
@@ -91,7 +108,132 @@ template <int DH> struct X3Row {
 #pragma unroll
     for (int pl = 0; pl < 3; ++pl) *reinterpret_cast<fm_u16x8*>(p + pl * DH) = f.p[pl];
   }
+  static FM_DEVICE void put8(uint16_t* tile, int row, int col, const float w[8]) { store(tile + row * PQ + col, fm_x3_split(w)); }
+  static FM_DEVICE void score(const uint16_t* X, int row, int lh, const Own& of, fm_f32x16& s) {
+#pragma unroll
+    for (int ks = 0; ks < NOWN; ++ks) s = fm_x3_mma(load(X + row * PQ + feat(ks, lh)), of.f[ks], s);
+  }
+  static FM_DEVICE void score2(const uint16_t* X, const uint16_t* Y, int row, int lh, const Own& of, const Own& of2, fm_f32x16& s,
+                               fm_f32x16& dp) {
+#pragma unroll
+    for (int ks = 0; ks < NOWN; ++ks) terms2(load(X + row * PQ + feat(ks, lh)), of.f[ks], load(Y + row * PQ + feat(ks, lh)), of2.f[ks], s, dp);
+  }
+  // the second own row in LDS
+  static FM_DEVICE void score2(const uint16_t* X, const uint16_t* Y, int row, int lh, const Own& of, const uint16_t* V, int vrow,
+                               fm_f32x16& s, fm_f32x16& dp) {
+#pragma unroll
+    for (int ks = 0; ks < NOWN; ++ks)
+      terms2(load(X + row * PQ + feat(ks, lh)), of.f[ks], load(Y + row * PQ + feat(ks, lh)), load(V + vrow * PQ + feat(ks, lh)), s, dp);
+  }
+  static FM_DEVICE void terms2(const X3& xf, const X3& of, const X3& yf, const X3& of2, fm_f32x16& s, fm_f32x16& dp) {
+#pragma unroll
+    for (int t = 0; t < FM_X3_TERMS; ++t) {
+      s = fm_mfma_bf16(xf.p[fm_x3_pa(t)], of.p[fm_x3_pb(t)], s);
+      dp = fm_mfma_bf16(yf.p[fm_x3_pa(t)], of2.p[fm_x3_pb(t)], dp);
+    }
+  }
+  static FM_DEVICE void accum(fm_f32x16* acc, const uint16_t* Y, int tok0, const fm_f32x16& s, int lane) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const X3 pb = fm_x3_split_acc(s, h);
+      X3 zf[NT];
+#pragma unroll
+      for (int ct = 0; ct < NT; ++ct) zf[ct] = load_tr(Y, tok0 + 16 * h, 32 * ct, lane);
+#pragma unroll
+      for (int t = 0; t < FM_X3_TERMS; ++t)
+#pragma unroll
+        for (int ct = 0; ct < NT; ++ct) acc[ct] = fm_mfma_bf16(zf[ct].p[fm_x3_pa(t)], pb.p[fm_x3_pb(t)], acc[ct]);
+    }
+  }
+  // av += Y s, ak += X dp
+  static FM_DEVICE void accum2(fm_f32x16* av, const uint16_t* Y, const fm_f32x16& s, fm_f32x16* ak, const uint16_t* X, const fm_f32x16& dp,
+                               int tok0, int lane) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const X3 pb = fm_x3_split_acc(s, h), db = fm_x3_split_acc(dp, h);
+#pragma unroll
+      for (int ct = 0; ct < NT; ++ct) {
+        const X3 yt = load_tr(Y, tok0 + 16 * h, 32 * ct, lane), xt = load_tr(X, tok0 + 16 * h, 32 * ct, lane);
+#pragma unroll
+        for (int t = 0; t < FM_X3_TERMS; ++t) {
+          av[ct] = fm_mfma_bf16(yt.p[fm_x3_pa(t)], pb.p[fm_x3_pb(t)], av[ct]);
+          ak[ct] = fm_mfma_bf16(xt.p[fm_x3_pa(t)], db.p[fm_x3_pb(t)], ak[ct]);
+        }
+      }
+    }
+  }
 };
+template <int DH> struct F32Row {
+  static constexpr int PQ = X3Row<DH>::PQ;             // the tiles lie where the planes lay
+  static constexpr int PF = DH + 1;                    // a row in floats
+  static_assert(2 * PF <= PQ, "a row of floats fits a row of planes");
+  static constexpr bool PIPE = false;                  // few registers: this code shares the allocation of the one above
+  static constexpr int CH = 1, NOWN = DH / 2, NT = DH / 32;
+  struct Own { float f[NOWN]; };
+  static FM_DEVICE int feat(int c, int lh) { return 2 * c + lh; }
+  template <typename TIO> static FM_DEVICE void ld(const TIO* p, bool, float v[CH]) { v[0] = IO<TIO>::ld(p); }
+  static FM_DEVICE void add_half(const fm_half* p, float v[CH]) { v[0] += float(*p); }
+  static FM_DEVICE void set(Own& o, int c, const float v[CH]) { o.f[c] = v[0]; }
+  static FM_DEVICE void fence(int c) { if (c % 4 == 0) FM_SCHED_FENCE(); }
+  static FM_DEVICE const float* at(const uint16_t* tile, int row) { return reinterpret_cast<const float*>(tile) + row * PF; }
+  static FM_DEVICE void put8(uint16_t* tile, int row, int col, const float w[8]) {
+    float* p = reinterpret_cast<float*>(tile) + row * PF + col;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) p[i] = w[i];
+  }
+  static FM_DEVICE void score(const uint16_t* X, int row, int lh, const Own& of, fm_f32x16& s) {
+    const float* x = at(X, row) + lh;
+#pragma unroll
+    for (int c = 0; c < NOWN; ++c) {
+      fence(c);
+      s = fm_mfma_f32(x[2 * c], of.f[c], s);
+    }
+  }
+  static FM_DEVICE void score2(const uint16_t* X, const uint16_t* Y, int row, int lh, const Own& of, const Own& of2, fm_f32x16& s,
+                               fm_f32x16& dp) {
+    score(X, row, lh, of, s);
+    score(Y, row, lh, of2, dp);
+  }
+  static FM_DEVICE void score2(const uint16_t* X, const uint16_t* Y, int row, int lh, const Own& of, const uint16_t* V, int vrow,
+                               fm_f32x16& s, fm_f32x16& dp) {
+    score(X, row, lh, of, s);
+    const float *y = at(Y, row) + lh, *v = at(V, vrow) + lh;
+#pragma unroll
+    for (int c = 0; c < NOWN; ++c) {
+      fence(c);
+      dp = fm_mfma_f32(y[2 * c], v[2 * c], dp);
+    }
+  }
+  static FM_DEVICE void accum(fm_f32x16* acc, const uint16_t* Y, int tok0, const fm_f32x16& s, int lane) {
+    const float* y = at(Y, tok0) + (lane & 31);
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      fence(e);
+#pragma unroll
+      for (int ct = 0; ct < NT; ++ct) acc[ct] = fm_mfma_f32(y[fm_acc_row(e, lane >> 5) * PF + 32 * ct], s[e], acc[ct]);
+    }
+  }
+  static FM_DEVICE void accum2(fm_f32x16* av, const uint16_t* Y, const fm_f32x16& s, fm_f32x16* ak, const uint16_t* X, const fm_f32x16& dp,
+                               int tok0, int lane) {
+    accum(av, Y, tok0, s, lane);
+    accum(ak, X, tok0, dp, lane);
+  }
+};
+
+// Three planes hold every finite number below 3.3953e38 (what bf16's largest number rounds down from); an infinity, a NaN
+// or a number above comes out of the split as infinity and NaN, and whatever sum it enters as NaN.  So the wavefronts look
+// at their sums before the workgroup adds and stores them and, if one is not finite (or so large that the parts' sum might
+// not be), the workgroup makes its rows again with fp32 matrix products: an infinite value then gives the infinities and NaN
+// that fp32 arithmetic gives.  bad: one flag in LDS, cleared at the kernel's start; the barrier before the sums are read
+// is the one that shows it to everybody (one of its own behind the stores would wait for them: 0.4 us).
+template <int NT> FM_DEVICE void fm_x3_look(int* bad, const fm_f32x16* acc, float g) {
+  float z[4] = {fm_absf(g), 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int ct = 0; ct < NT; ++ct)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) z[e % 4] += fm_absf(acc[ct][e]);
+  if (!((z[0] + z[1]) + (z[2] + z[3]) < 0x1p125f)) *bad = 1;
+}
 
 template <typename TIO> struct X3Args {
   TRef<const TIO> q, k, v, o, d_o;
@@ -106,10 +248,9 @@ template <typename TIO> struct X3Args {
 };
 
 // Stage of ROWS stream rows of two tensors: caller's rows -> registers -> LDS planes.
-template <typename TIO, int DH, int ROWS, int NTH> struct X3Stage {
+template <typename TIO, int DH, typename R, int ROWS, int NTH> struct X3Stage {
   static constexpr int CPR = DH / 8, PER = ROWS * CPR, TOT = 2 * PER, N = (TOT + NTH - 1) / NTH;
-  float r[N][8];
-  float gi[N];
+  float r[N][8], gi[N];
   // gb: y rows are divided by g (null: not)
   FM_DEVICE void load(const TRef<const TIO>& x, const TRef<const TIO>& y, const TRef<float>* g, int bh, int row0, int n, int tid) {
 #pragma unroll
@@ -130,7 +271,6 @@ template <typename TIO, int DH, int ROWS, int NTH> struct X3Stage {
     }
   }
   FM_DEVICE void store(uint16_t* X, uint16_t* Y, float xs, bool div, int tid) const {
-    constexpr int PQ = X3Row<DH>::PQ;
 #pragma unroll
     for (int i = 0; i < N; ++i) {
       const int c = tid + NTH * i;
@@ -141,7 +281,25 @@ template <typename TIO, int DH, int ROWS, int NTH> struct X3Stage {
       float w[8];
 #pragma unroll
       for (int j = 0; j < 8; ++j) w[j] = r[i][j] * f;
-      X3Row<DH>::store((second ? Y : X) + (cc / CPR) * PQ + (cc % CPR) * 8, fm_x3_split(w));
+      R::put8(second ? Y : X, cc / CPR, (cc % CPR) * 8, w);
+    }
+  }
+  // both steps at once, one piece after the other (few registers)
+  static FM_DEVICE void copy(uint16_t* X, uint16_t* Y, const TRef<const TIO>& x, const TRef<const TIO>& y, const TRef<float>* g, int bh,
+                             int row0, int n, float xs, int tid) {
+#pragma unroll 1
+    for (int c = tid; c < TOT; c += NTH) {
+      const bool second = c >= PER;
+      const int cc = second ? c - PER : c, row = row0 + cc / CPR, col = (cc % CPR) * 8;
+      float w[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+      if (row >= 0 && row < n) {
+        const TRef<const TIO>& t = second ? y : x;
+        IO<TIO>::ld8(t.base(bh) + int64_t(row) * t.s_n + col, t.vec != 0, w);
+        const float f = second ? (g ? 1.0f / g->base(bh)[int64_t(row) * g->s_n] : 1.0f) : xs;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) w[j] *= f;
+      }
+      R::put8(second ? Y : X, cc / CPR, col, w);
     }
   }
 };
@@ -195,13 +353,15 @@ template <int DH, int QW, int SPLIT> FM_DEVICE void fm_x3_sum8(const float* Os, 
   }
 }
 // Gradient rows of the workgroup -> caller's tensor, times scale.  bout: the sum of stored value times raw row (the
-// normalisation's B: stored = fac dy, y = fac x, so dy . y = stored . x), one float per workgroup, or null.
-template <typename TIO, int DH, int QW, int SPLIT, int NTH>
-FM_DEVICE void fm_x3_store(const fm_f32x16* acc, float* Os, int sub, int row, int lh, float scale, const TRef<TIO>& out,
-                           int bh, int t0, int n, int tid, const TRef<const TIO>& raw, float* bout) {
+// normalisation's B: stored = fac dy, y = fac x, so dy . y = stored . x), one float per workgroup, or null.  bad: see
+// fm_x3_look; false if it is set.
+template <typename TIO, int DH, int QW, int SPLIT, int NTH, typename R>
+FM_DEVICE bool fm_x3_store(const fm_f32x16* acc, float* Os, int sub, int row, int lh, float scale, const TRef<TIO>& out,
+                           int bh, int t0, int n, int tid, const TRef<const TIO>& raw, float* bout, const int* bad) {
   FM_SYNC();                                           // whatever lay there has been read
   fm_x3_put<DH, QW>(acc, Os, sub, row, lh);
   FM_SYNC();
+  if (R::PIPE && __builtin_expect(*bad != 0, 0)) return false;
   float bsum = 0.f;
   for (int c = tid; c < QW * (DH / 8); c += NTH) {
     const int r = c / (DH / 8), col = (c % (DH / 8)) * 8;
@@ -230,6 +390,7 @@ FM_DEVICE void fm_x3_store(const fm_f32x16* acc, float* Os, int sub, int row, in
       *bout = b;
     }
   }
+  return true;
 }
 
 template <int DH, int NW, int SPLIT> struct X3Cfg {
@@ -242,20 +403,17 @@ template <int DH, int NW, int SPLIT> struct X3Cfg {
     const size_t a = size_t(NBUF) * STAGE * 2 + (kind ? size_t(QW) * PQ * 2 + size_t(NBUF) * KT * 4 : 0);
     return a > OS ? a : OS;
   }
-  static constexpr int OCC = NW == 8 || NBUF == 1 || 2 * (NBUF * STAGE * 2) > 150 * 1024 ? NW / 4 : 2;   // wavefronts per SIMD
+  static constexpr int OCC = NW == 8 || NBUF == 1 || 2 * (NBUF * STAGE * 2) > 150 * 1024 ? NW / 4 : DH == 32 && SPLIT == 1 ? 3 : 2;   // wavefronts per SIMD
 };
 
 // ------------------------------------------------------------------------------
 // forward.  grid (ceil(nq / QW), bh), 256 threads.
 // ------------------------------------------------------------------------------
-template <typename TIO, int DH, int SPLIT>
-FM_GLOBAL void FM_LAUNCH_BOUNDS2(256, (X3Cfg<DH, 4, SPLIT>::OCC)) k_x3_fwd(X3Args<TIO> A) {
+template <typename TIO, int DH, int SPLIT, typename R>
+FM_DEVICE bool fm_x3_fwd(const X3Args<TIO>& A, uint16_t* st, int* bad, const int tid) {
   typedef X3Cfg<DH, 4, SPLIT> C;
-  typedef X3Row<DH> R;
-  constexpr int NT = DH / 32, NKS = DH / 16, PQ = C::PQ, KT = C::KT, QW = C::QW;
-  FM_DYN_SMEM(smem);
-  uint16_t* st = reinterpret_cast<uint16_t*>(smem);
-  const int tid = FM_TID_X, lane = tid & 63, lr = lane & 31, lh = lane >> 5;
+  constexpr int NT = DH / 32, PQ = C::PQ, KT = C::KT, QW = C::QW;
+  const int lane = tid & 63, lr = lane & 31, lh = lane >> 5;
   const int wave = FM_UNIFORM(tid >> 6), own = wave / SPLIT, sub = wave % SPLIT;
   const bool causal = A.causal != 0;
   int blk, bh;
@@ -263,59 +421,52 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(256, (X3Cfg<DH, 4, SPLIT>::OCC)) k_x3_fwd(X3Arg
   const int t0 = blk * QW, lo = t0 + 32 * own;
   const float qs = A.sc * fm_norm_factor(A.q_fold, bh, lane), ks_ = A.sc * fm_norm_factor(A.k_fold, bh, lane);
   const int send = causal && t0 + QW < A.nk ? t0 + QW : A.nk;
-  X3Stage<TIO, DH, KT, C::NTH> sg;
-  sg.load(A.k, A.v, nullptr, bh, 0, A.nk, tid);
-  X3 of[NKS];
+  typedef X3Stage<TIO, DH, R, KT, C::NTH> Stage;
+  Stage sg;
+  if (R::PIPE) sg.load(A.k, A.v, nullptr, bh, 0, A.nk, tid);
+  typename R::Own of;
   {
     const bool in = lo + lr < A.nq;
-    const TIO* qr = A.q.base(bh) + int64_t(in ? lo + lr : A.nq - 1) * A.q.s_n + lh * 8;
+    const TIO* qr = A.q.base(bh) + int64_t(in ? lo + lr : A.nq - 1) * A.q.s_n;
 #pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) {
-      float v[8];
-      IO<TIO>::ld8(qr + 16 * ks, A.q.vec != 0, v);
+    for (int c = 0; c < R::NOWN; ++c) {
+      R::fence(c);
+      float v[R::CH];
+      R::ld(qr + R::feat(c, lh), A.q.vec != 0, v);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) v[i] = in ? v[i] * qs : 0.f;
-      of[ks] = fm_x3_split(v);
+      for (int i = 0; i < R::CH; ++i) v[i] = in ? v[i] * qs : 0.f;
+      R::set(of, c, v);
     }
   }
   fm_f32x16 acc[NT];
 #pragma unroll
   for (int ct = 0; ct < NT; ++ct) acc[ct] = fm_zero16();
   float gs = 0.f;
+  constexpr bool TWO = R::PIPE && C::NBUF == 2;
   int buf = 0;
-  if (C::NBUF == 2) {
+  if (TWO) {
     sg.store(st, st + KT * PQ, ks_, false, tid);
     sg.load(A.k, A.v, nullptr, bh, KT, A.nk, tid);
   }
   for (int s0 = 0; s0 < send; s0 += KT) {
     uint16_t* X = st + buf * C::STAGE;
     uint16_t* Y = X + KT * PQ;
-    if (C::NBUF == 1) sg.store(X, Y, ks_, false, tid);
+    if (!R::PIPE) Stage::copy(X, Y, A.k, A.v, nullptr, bh, s0, A.nk, ks_, tid);
+    else if (!TWO) sg.store(X, Y, ks_, false, tid);
     FM_SYNC();
-    if (C::NBUF == 1) sg.load(A.k, A.v, nullptr, bh, s0 + KT, A.nk, tid);
+    if (R::PIPE && !TWO) sg.load(A.k, A.v, nullptr, bh, s0 + KT, A.nk, tid);
     const int ss0 = s0 + 32 * sub;
     if (ss0 < A.nk && !(causal && ss0 > lo + 31)) {
       fm_f32x16 s = fm_zero16();
-#pragma unroll
-      for (int ks = 0; ks < NKS; ++ks) s = fm_x3_mma(R::load(X + (32 * sub + lr) * PQ + 16 * ks + 8 * lh), of[ks], s);
+      R::score(X, 32 * sub + lr, lh, of, s);
 #pragma unroll
       for (int e = 0; e < 16; ++e) s[e] = A.a0 + s[e] * (A.a1 + A.a2 * s[e]);
       if (fm_tile_edge<FM_OWN_Q>(causal, ss0, lo, A.nk)) { FM_KEEP_BRANCH(); fm_x3_window<FM_OWN_Q>(s, causal, ss0, lo, lr, lh, A.nk); }
 #pragma unroll
       for (int e = 0; e < 16; ++e) gs += s[e];
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const X3 pb = fm_x3_split_acc(s, h);
-        X3 zf[NT];
-#pragma unroll
-        for (int ct = 0; ct < NT; ++ct) zf[ct] = R::load_tr(Y, 32 * sub + 16 * h, 32 * ct, lane);
-#pragma unroll
-        for (int t = 0; t < FM_X3_TERMS; ++t)
-#pragma unroll
-          for (int ct = 0; ct < NT; ++ct) acc[ct] = fm_mfma_bf16(zf[ct].p[fm_x3_pa(t)], pb.p[fm_x3_pb(t)], acc[ct]);
-      }
+      R::accum(acc, Y, 32 * sub, s, lane);
     }
-    if (C::NBUF == 2) {
+    if (TWO) {
       buf ^= 1;
       if (s0 + KT < send) {
         sg.store(st + buf * C::STAGE, st + buf * C::STAGE + KT * PQ, ks_, false, tid);
@@ -323,13 +474,15 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(256, (X3Cfg<DH, 4, SPLIT>::OCC)) k_x3_fwd(X3Arg
       }
     } else FM_SYNC();
   }
-  float* Os = reinterpret_cast<float*>(smem);
+  float* Os = reinterpret_cast<float*>(st);
   float* Gs = Os + SPLIT * QW * (DH + 4);              // [SPLIT][QW]
+  if (R::PIPE) fm_x3_look<NT>(bad, acc, gs);
   FM_SYNC();
   fm_x3_put<DH, QW>(acc, Os, sub, 32 * own + lr, lh);
   gs += fm_shfl_xor(gs, 32);
   if (lh == 0) Gs[sub * QW + 32 * own + lr] = gs;
   FM_SYNC();
+  if (R::PIPE && __builtin_expect(*bad != 0, 0)) return false;
   for (int c = tid; c < QW * (DH / 8); c += C::NTH) {
     const int r = c / (DH / 8), col = (c % (DH / 8)) * 8, qi = t0 + r;
     if (qi >= A.nq) continue;
@@ -349,19 +502,26 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(256, (X3Cfg<DH, 4, SPLIT>::OCC)) k_x3_fwd(X3Arg
     }
     if (col == 0) A.g.base(bh)[int64_t(qi) * A.g.s_n] = gt;
   }
+  return true;
+}
+template <typename TIO, int DH, int SPLIT>
+FM_GLOBAL void FM_LAUNCH_BOUNDS2(256, (X3Cfg<DH, 4, SPLIT>::OCC)) k_x3_fwd(X3Args<TIO> A) {
+  FM_DYN_SMEM(smem);
+  FM_SHARED int bad;
+  uint16_t* st = reinterpret_cast<uint16_t*>(smem);
+  if (FM_TID_X == 0) bad = 0;
+  if (fm_x3_fwd<TIO, DH, SPLIT, X3Row<DH>>(A, st, &bad, FM_TID_X)) return;
+  (void)fm_x3_fwd<TIO, DH, SPLIT, F32Row<DH>>(FM_ARGS_AGAIN(A), st, &bad, FM_TID_X + FM_OPAQUE_ZERO());
 }
 
 // ------------------------------------------------------------------------------
 // dQ.  grid (ceil(nq / QW), bh), 256 threads.  dS = (a1 + 2 a2 s) (gh . v - c), gh = dO / g, c = gh . o.
 // ------------------------------------------------------------------------------
-template <typename TIO, int DH, int SPLIT>
-FM_GLOBAL void FM_LAUNCH_BOUNDS2(256, (X3Cfg<DH, 4, SPLIT>::OCC)) k_x3_dq(X3Args<TIO> A) {
+template <typename TIO, int DH, int SPLIT, typename R>
+FM_DEVICE bool fm_x3_dq(const X3Args<TIO>& A, uint16_t* st, int* bad, const int tid) {
   typedef X3Cfg<DH, 4, SPLIT> C;
-  typedef X3Row<DH> R;
-  constexpr int NT = DH / 32, NKS = DH / 16, PQ = C::PQ, KT = C::KT, QW = C::QW;
-  FM_DYN_SMEM(smem);
-  uint16_t* st = reinterpret_cast<uint16_t*>(smem);
-  const int tid = FM_TID_X, lane = tid & 63, lr = lane & 31, lh = lane >> 5;
+  constexpr int NT = DH / 32, PQ = C::PQ, KT = C::KT, QW = C::QW;
+  const int lane = tid & 63, lr = lane & 31, lh = lane >> 5;
   const int wave = FM_UNIFORM(tid >> 6), own = wave / SPLIT, sub = wave % SPLIT;
   const bool causal = A.causal != 0;
   int blk, bh;
@@ -369,30 +529,28 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(256, (X3Cfg<DH, 4, SPLIT>::OCC)) k_x3_dq(X3Args
   const int t0 = blk * QW, lo = t0 + 32 * own;
   const float qf = fm_norm_factor(A.q_fold, bh, lane), qs = A.sc * qf, ks_ = A.sc * fm_norm_factor(A.k_fold, bh, lane);
   const int send = causal && t0 + QW < A.nk ? t0 + QW : A.nk;
-  X3Stage<TIO, DH, KT, C::NTH> sg;
-  sg.load(A.k, A.v, nullptr, bh, 0, A.nk, tid);
-  X3 of[NKS], of2[NKS];
+  typedef X3Stage<TIO, DH, R, KT, C::NTH> Stage;
+  Stage sg;
+  if (R::PIPE) sg.load(A.k, A.v, nullptr, bh, 0, A.nk, tid);
+  typename R::Own of, of2;
   float cs = 0.f;
   {
     const bool in = lo + lr < A.nq;
     const int64_t row = in ? lo + lr : A.nq - 1;
     const float ginv = in ? 1.0f / A.g.base(bh)[row * A.g.s_n] : 0.f;
 #pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) {
-      const int f = 16 * ks + 8 * lh;
-      float v[8], w[8], o[8];
-      IO<TIO>::ld8(A.q.base(bh) + row * A.q.s_n + f, A.q.vec != 0, v);
-      IO<TIO>::ld8(A.d_o.base(bh) + row * A.d_o.s_n + f, A.d_o.vec != 0, w);
-      IO<TIO>::ld8(A.o.base(bh) + row * A.o.s_n + f, A.o.vec != 0, o);
-      if (A.ores) {
-        const fm_half8 rs = *reinterpret_cast<const fm_half8*>(A.ores + (int64_t(bh) * A.npad_q + row) * DH + f);
+    for (int c = 0; c < R::NOWN; ++c) {
+      R::fence(c);
+      const int f = R::feat(c, lh);
+      float v[R::CH], w[R::CH], o[R::CH];
+      R::ld(A.q.base(bh) + row * A.q.s_n + f, A.q.vec != 0, v);
+      R::ld(A.d_o.base(bh) + row * A.d_o.s_n + f, A.d_o.vec != 0, w);
+      R::ld(A.o.base(bh) + row * A.o.s_n + f, A.o.vec != 0, o);
+      if (A.ores) R::add_half(A.ores + (int64_t(bh) * A.npad_q + row) * DH + f, o);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) o[i] += float(rs[i]);
-      }
-#pragma unroll
-      for (int i = 0; i < 8; ++i) { v[i] = in ? v[i] * qs : 0.f; w[i] = in ? w[i] * ginv : 0.f; cs += w[i] * o[i]; }
-      of[ks] = fm_x3_split(v);
-      of2[ks] = fm_x3_split(w);
+      for (int i = 0; i < R::CH; ++i) { v[i] = in ? v[i] * qs : 0.f; w[i] = in ? w[i] * ginv : 0.f; cs += w[i] * o[i]; }
+      R::set(of, c, v);
+      R::set(of2, c, w);
     }
     cs += fm_shfl_xor(cs, 32);
     if (sub == 0 && lh == 0 && in) A.cv[int64_t(bh) * A.npad_q + row] = cs;
@@ -401,45 +559,29 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(256, (X3Cfg<DH, 4, SPLIT>::OCC)) k_x3_dq(X3Args
   fm_f32x16 acc[NT];
 #pragma unroll
   for (int ct = 0; ct < NT; ++ct) acc[ct] = fm_zero16();
+  constexpr bool TWO = R::PIPE && C::NBUF == 2;
   int buf = 0;
-  if (C::NBUF == 2) {
+  if (TWO) {
     sg.store(st, st + KT * PQ, ks_, false, tid);
     sg.load(A.k, A.v, nullptr, bh, KT, A.nk, tid);
   }
   for (int s0 = 0; s0 < send; s0 += KT) {
     uint16_t* X = st + buf * C::STAGE;
     uint16_t* Y = X + KT * PQ;
-    if (C::NBUF == 1) sg.store(X, Y, ks_, false, tid);
+    if (!R::PIPE) Stage::copy(X, Y, A.k, A.v, nullptr, bh, s0, A.nk, ks_, tid);
+    else if (!TWO) sg.store(X, Y, ks_, false, tid);
     FM_SYNC();
-    if (C::NBUF == 1) sg.load(A.k, A.v, nullptr, bh, s0 + KT, A.nk, tid);
+    if (R::PIPE && !TWO) sg.load(A.k, A.v, nullptr, bh, s0 + KT, A.nk, tid);
     const int ss0 = s0 + 32 * sub;
     if (ss0 < A.nk && !(causal && ss0 > lo + 31)) {
       fm_f32x16 s = fm_zero16(), dp = fm_zero16();
-#pragma unroll
-      for (int ks = 0; ks < NKS; ++ks) {
-        const X3 xf = R::load(X + (32 * sub + lr) * PQ + 16 * ks + 8 * lh), yf = R::load(Y + (32 * sub + lr) * PQ + 16 * ks + 8 * lh);
-#pragma unroll
-        for (int t = 0; t < FM_X3_TERMS; ++t) {
-          s = fm_mfma_bf16(xf.p[fm_x3_pa(t)], of[ks].p[fm_x3_pb(t)], s);
-          dp = fm_mfma_bf16(yf.p[fm_x3_pa(t)], of2[ks].p[fm_x3_pb(t)], dp);
-        }
-      }
+      R::score2(X, Y, 32 * sub + lr, lh, of, of2, s, dp);
 #pragma unroll
       for (int e = 0; e < 16; ++e) s[e] = (A.a1 + ta2 * s[e]) * (dp[e] - cs);
       if (fm_tile_edge<FM_OWN_Q>(causal, ss0, lo, A.nk)) { FM_KEEP_BRANCH(); fm_x3_window<FM_OWN_Q>(s, causal, ss0, lo, lr, lh, A.nk); }
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const X3 db = fm_x3_split_acc(s, h);
-        X3 zf[NT];
-#pragma unroll
-        for (int ct = 0; ct < NT; ++ct) zf[ct] = R::load_tr(X, 32 * sub + 16 * h, 32 * ct, lane);
-#pragma unroll
-        for (int t = 0; t < FM_X3_TERMS; ++t)
-#pragma unroll
-          for (int ct = 0; ct < NT; ++ct) acc[ct] = fm_mfma_bf16(zf[ct].p[fm_x3_pa(t)], db.p[fm_x3_pb(t)], acc[ct]);
-      }
+      R::accum(acc, X, 32 * sub, s, lane);
     }
-    if (C::NBUF == 2) {
+    if (TWO) {
       buf ^= 1;
       if (s0 + KT < send) {
         sg.store(st + buf * C::STAGE, st + buf * C::STAGE + KT * PQ, ks_, false, tid);
@@ -447,24 +589,31 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(256, (X3Cfg<DH, 4, SPLIT>::OCC)) k_x3_dq(X3Args
       }
     } else FM_SYNC();
   }
-  fm_x3_store<TIO, DH, QW, SPLIT, C::NTH>(acc, reinterpret_cast<float*>(smem), sub, 32 * own + lr, lh, A.sc * (A.bpart ? qf : 1.0f), A.out,
-                                          bh, t0, A.nq, tid, A.q, A.bpart ? A.bpart + int64_t(bh) * FM_GDIM_X + blk : nullptr);
+  if (R::PIPE) fm_x3_look<NT>(bad, acc, 0.f);
+  return fm_x3_store<TIO, DH, QW, SPLIT, C::NTH, R>(acc, reinterpret_cast<float*>(st), sub, 32 * own + lr, lh, A.sc * (A.bpart ? qf : 1.0f), A.out,
+                                          bh, t0, A.nq, tid, A.q, A.bpart ? A.bpart + int64_t(bh) * FM_GDIM_X + blk : nullptr, bad);
+}
+template <typename TIO, int DH, int SPLIT>
+FM_GLOBAL void FM_LAUNCH_BOUNDS2(256, (X3Cfg<DH, 4, SPLIT>::OCC)) k_x3_dq(X3Args<TIO> A) {
+  FM_DYN_SMEM(smem);
+  FM_SHARED int bad;
+  uint16_t* st = reinterpret_cast<uint16_t*>(smem);
+  if (FM_TID_X == 0) bad = 0;
+  if (fm_x3_dq<TIO, DH, SPLIT, X3Row<DH>>(A, st, &bad, FM_TID_X)) return;
+  (void)fm_x3_dq<TIO, DH, SPLIT, F32Row<DH>>(FM_ARGS_AGAIN(A), st, &bad, FM_TID_X + FM_OPAQUE_ZERO());
 }
 
 // ------------------------------------------------------------------------------
 // dK and dV.  grid (ceil(nk / QW), bh), 512 threads: eight wavefronts share the staged queries, so that two per SIMD
 // leave 256 registers each; own k in registers, own v (read once per tile) in LDS.
 // ------------------------------------------------------------------------------
-template <typename TIO, int DH, int SPLIT>
-FM_GLOBAL void FM_LAUNCH_BOUNDS2(512, 2) k_x3_dkv(X3Args<TIO> A) {
+template <typename TIO, int DH, int SPLIT, typename R>
+FM_DEVICE bool fm_x3_dkv(const X3Args<TIO>& A, uint16_t* Vs, int* bad, const int tid) {
   typedef X3Cfg<DH, 8, SPLIT> C;
-  typedef X3Row<DH> R;
-  constexpr int NT = DH / 32, NKS = DH / 16, PQ = C::PQ, KT = C::KT, QW = C::QW;
-  FM_DYN_SMEM(smem);
-  uint16_t* Vs = reinterpret_cast<uint16_t*>(smem);    // own v rows [QW][PQ]
-  uint16_t* st = Vs + QW * PQ;
+  constexpr int NT = DH / 32, PQ = C::PQ, KT = C::KT, QW = C::QW;
+  uint16_t* st = Vs + QW * PQ;                         // Vs: own v rows [QW][PQ]
   float* cst = reinterpret_cast<float*>(st + C::NBUF * C::STAGE);   // c of the staged queries [NBUF][KT]
-  const int tid = FM_TID_X, lane = tid & 63, lr = lane & 31, lh = lane >> 5;
+  const int lane = tid & 63, lr = lane & 31, lh = lane >> 5;
   const int wave = FM_UNIFORM(tid >> 6), own = wave / SPLIT, sub = wave % SPLIT;
   const bool causal = A.causal != 0;
   int blk, bh;
@@ -473,65 +622,61 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(512, 2) k_x3_dkv(X3Args<TIO> A) {
   const float kf = fm_norm_factor(A.k_fold, bh, lane), ks_ = A.sc * kf, qs = A.sc * fm_norm_factor(A.q_fold, bh, lane);
   const int sbeg = causal ? t0 : 0, nst = (A.nq - sbeg + KT - 1) / KT;
   const int s_last = sbeg + (nst - 1) * KT;            // the stream is walked from its end: see k_ds
-  X3Stage<TIO, DH, KT, C::NTH> sg;
+  typedef X3Stage<TIO, DH, R, KT, C::NTH> Stage;
+  Stage sg;
   float creg = 0.f;
   const float* cvb = A.cv + int64_t(bh) * A.npad_q;
-  auto fetch = [&](int s) {
+  auto fetch = [&](int s) FM_ALWAYS_INLINE {
     sg.load(A.q, A.d_o, &A.g, bh, s, A.nq, tid);
     const int r = s + tid % KT;
     creg = r >= 0 && r < A.nq ? cvb[r] : 0.f;
   };
-  auto put = [&](int b) {
+  auto put = [&](int b) FM_ALWAYS_INLINE {
     uint16_t* X = st + b * C::STAGE;
     sg.store(X, X + KT * PQ, qs, true, tid);
     if (tid < KT) cst[b * KT + tid] = creg;
   };
-  fetch(s_last);
+  if (R::PIPE) fetch(s_last);
   for (int c = tid; c < QW * (DH / 8); c += C::NTH) {
     const int r = c / (DH / 8), col = (c % (DH / 8)) * 8, row = t0 + r;
     float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     if (row < A.nk) IO<TIO>::ld8(A.v.base(bh) + int64_t(row) * A.v.s_n + col, A.v.vec != 0, v);
-    R::store(Vs + r * PQ + col, fm_x3_split(v));
+    R::put8(Vs, r, col, v);
   }
-  X3 of[NKS];
+  typename R::Own of;
   {
     const bool in = lo + lr < A.nk;
-    const TIO* kr = A.k.base(bh) + int64_t(in ? lo + lr : A.nk - 1) * A.k.s_n + lh * 8;
+    const TIO* kr = A.k.base(bh) + int64_t(in ? lo + lr : A.nk - 1) * A.k.s_n;
 #pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) {
-      float v[8];
-      IO<TIO>::ld8(kr + 16 * ks, A.k.vec != 0, v);
+    for (int c = 0; c < R::NOWN; ++c) {
+      R::fence(c);
+      float v[R::CH];
+      R::ld(kr + R::feat(c, lh), A.k.vec != 0, v);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) v[i] = in ? v[i] * ks_ : 0.f;
-      of[ks] = fm_x3_split(v);
+      for (int i = 0; i < R::CH; ++i) v[i] = in ? v[i] * ks_ : 0.f;
+      R::set(of, c, v);
     }
   }
   const float ta2 = 2.0f * A.a2;
   fm_f32x16 acc[NT], av[NT];
 #pragma unroll
   for (int ct = 0; ct < NT; ++ct) { acc[ct] = fm_zero16(); av[ct] = fm_zero16(); }
+  constexpr bool TWO = R::PIPE && C::NBUF == 2;
   int buf = 0;
-  if (C::NBUF == 2) { put(0); fetch(s_last - KT); }
-  const uint16_t* vrow = Vs + (32 * own + lr) * PQ + 8 * lh;
+  if (TWO) { put(0); fetch(s_last - KT); }
   for (int s0 = s_last; s0 >= sbeg; s0 -= KT) {
     uint16_t* X = st + buf * C::STAGE;
     uint16_t* Y = X + KT * PQ;
-    if (C::NBUF == 1) put(0);
+    if (!R::PIPE) {
+      Stage::copy(X, Y, A.q, A.d_o, &A.g, bh, s0, A.nq, qs, tid);
+      if (tid < KT) cst[tid] = s0 + tid < A.nq ? cvb[s0 + tid] : 0.f;
+    } else if (!TWO) put(0);
     FM_SYNC();
-    if (C::NBUF == 1) fetch(s0 - KT);
+    if (R::PIPE && !TWO) fetch(s0 - KT);
     const int ss0 = s0 + 32 * sub;
     if (ss0 < A.nq && !(causal && ss0 + 31 < lo)) {
       fm_f32x16 s = fm_zero16(), dp = fm_zero16();
-#pragma unroll
-      for (int ks = 0; ks < NKS; ++ks) {
-        const X3 xf = R::load(X + (32 * sub + lr) * PQ + 16 * ks + 8 * lh), yf = R::load(Y + (32 * sub + lr) * PQ + 16 * ks + 8 * lh);
-        const X3 vf = R::load(vrow + 16 * ks);
-#pragma unroll
-        for (int t = 0; t < FM_X3_TERMS; ++t) {
-          s = fm_mfma_bf16(xf.p[fm_x3_pa(t)], of[ks].p[fm_x3_pb(t)], s);
-          dp = fm_mfma_bf16(yf.p[fm_x3_pa(t)], vf.p[fm_x3_pb(t)], dp);
-        }
-      }
+      R::score2(X, Y, 32 * sub + lr, lh, of, Vs, 32 * own + lr, s, dp);
       const float* cf = cst + buf * KT + 32 * sub + 4 * lh;
       // dp becomes dS, s becomes P
 #pragma unroll
@@ -550,27 +695,26 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(512, 2) k_x3_dkv(X3Args<TIO> A) {
         fm_x3_window<FM_OWN_K>(s, causal, ss0, lo, lr, lh, A.nq);
         fm_x3_window<FM_OWN_K>(dp, causal, ss0, lo, lr, lh, A.nq);
       }
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const X3 pb = fm_x3_split_acc(s, h), db = fm_x3_split_acc(dp, h);
-#pragma unroll
-        for (int ct = 0; ct < NT; ++ct) {
-          const X3 yt = R::load_tr(Y, 32 * sub + 16 * h, 32 * ct, lane), xt = R::load_tr(X, 32 * sub + 16 * h, 32 * ct, lane);
-#pragma unroll
-          for (int t = 0; t < FM_X3_TERMS; ++t) {
-            av[ct] = fm_mfma_bf16(yt.p[fm_x3_pa(t)], pb.p[fm_x3_pb(t)], av[ct]);
-            acc[ct] = fm_mfma_bf16(xt.p[fm_x3_pa(t)], db.p[fm_x3_pb(t)], acc[ct]);
-          }
-        }
-      }
+      R::accum2(av, Y, s, acc, X, dp, 32 * sub, lane);
     }
-    if (C::NBUF == 2) {
+    if (TWO) {
       buf ^= 1;
       if (s0 - KT >= sbeg) { put(buf); fetch(s0 - 2 * KT); }
     } else FM_SYNC();
   }
-  float* Os = reinterpret_cast<float*>(smem);
-  fm_x3_store<TIO, DH, QW, SPLIT, C::NTH>(acc, Os, sub, 32 * own + lr, lh, A.sc * (A.bpart ? kf : 1.0f), A.out, bh, t0, A.nk, tid, A.k,
-                                          A.bpart ? A.bpart + int64_t(bh) * FM_GDIM_X + blk : nullptr);
-  fm_x3_store<TIO, DH, QW, SPLIT, C::NTH>(av, Os, sub, 32 * own + lr, lh, 1.0f, A.out2, bh, t0, A.nk, tid, A.k, nullptr);
+  float* Os = reinterpret_cast<float*>(Vs);
+  if (R::PIPE) { fm_x3_look<NT>(bad, acc, 0.f); fm_x3_look<NT>(bad, av, 0.f); }
+  if (!fm_x3_store<TIO, DH, QW, SPLIT, C::NTH, R>(acc, Os, sub, 32 * own + lr, lh, A.sc * (A.bpart ? kf : 1.0f), A.out, bh, t0, A.nk, tid, A.k,
+                                          A.bpart ? A.bpart + int64_t(bh) * FM_GDIM_X + blk : nullptr, bad))
+    return false;
+  return fm_x3_store<TIO, DH, QW, SPLIT, C::NTH, R>(av, Os, sub, 32 * own + lr, lh, 1.0f, A.out2, bh, t0, A.nk, tid, A.k, nullptr, bad);
+}
+template <typename TIO, int DH, int SPLIT>
+FM_GLOBAL void FM_LAUNCH_BOUNDS2(512, 2) k_x3_dkv(X3Args<TIO> A) {
+  FM_DYN_SMEM(smem);
+  FM_SHARED int bad;
+  uint16_t* st = reinterpret_cast<uint16_t*>(smem);
+  if (FM_TID_X == 0) bad = 0;
+  if (fm_x3_dkv<TIO, DH, SPLIT, X3Row<DH>>(A, st, &bad, FM_TID_X)) return;
+  (void)fm_x3_dkv<TIO, DH, SPLIT, F32Row<DH>>(FM_ARGS_AGAIN(A), st, &bad, FM_TID_X + FM_OPAQUE_ZERO());
 }

@@ -162,3 +162,59 @@ def check_decode(lib, bh, n, n0, d, dtype, device, *, p, tau_mult=8.0, a=(1.0, 1
     eo, eg = rel_err(o, ro[:, n0:]), rel_err(g, rg[:, n0:])
     assert eo < TOL[dtype] and eg < TOL[dtype], f"decode o {eo:.3e} g {eg:.3e}"
     return eo, eg
+
+
+def check_infinite_and_largest_values(lib, bh, n, d, dtype, device, *, flags=0, seed=0, largest=None):
+    """One infinite entry, one NaN and one entry at the top of the type's range, in v and in dO: what IEEE arithmetic gives.
+    All weights are positive, so an infinite v is an infinite output column, and its neighbours do not change; an infinite
+    dO is an infinite column of dv, and the other queries' dq do not change.  The largest entry's key is zero (its weight
+    1), so nothing overflows.  Unmasked, plain weights; every other number against the fp64 closed form."""
+    q, k, v, go = make_inputs(bh, n, n, d, dtype, device, seed)
+    t, f, tau = n - 2, 5, 8.0 * math.sqrt(d)
+    k[:, t] = 0.0
+    kw = dict(mask=False, inv_tau=1.0 / tau, p=2, flags=flags)
+    tol = 1.5 * TOL[dtype] if dtype == torch.bfloat16 else 2e-6
+    rest = [i for i in range(d) if i != f]
+    ref = oracle_all(q, k, v, go, mask=False, tau=tau, p=2)
+    o0, g0 = lib.forward(q, k, v, **kw)
+    for x in (float("inf"), float("-inf"), float("nan")):
+        w = v.clone(); w[:, t, f] = x
+        o, g = lib.forward(q, k, w, **kw)
+        same = torch.isnan(o[..., f]) if x != x else o[..., f] == x
+        assert bool(same.all()), f"v = {x}: {o[0, :, f]}"
+        assert rel_err(o[..., rest], ref[0][..., rest]) < tol and rel_err(g, ref[1]) < tol
+        w = go.clone(); w[:, t, f] = x
+        dq, dk, dv = lib.backward(q, k, v, o0, g0, w, **kw)
+        same = torch.isnan(dv[..., f]) if x != x else dv[..., f] == x
+        assert bool(same.all()), f"dO = {x}: {dv[0, :, f]}"
+        assert rel_err(dv[..., rest], ref[4][..., rest]) < tol
+        others = [i for i in range(n) if i != t]
+        assert rel_err(dq[:, others], ref[2][:, others]) < tol
+        assert not bool(torch.isfinite(dq[:, t]).any()) and not bool(torch.isfinite(dk).any())
+    for x in (largest or (3.0e38, 3.4e38)):
+        w = v.clone(); w[:, t, f] = x
+        o, g = lib.forward(q, k, w, **kw)
+        big = oracle_all(q, k, w, go, mask=False, tau=tau, p=2)
+        assert rel_err(o[..., f], big[0][..., f]) < tol, f"v = {x}: {o[0, :3, f]}"
+        assert rel_err(o[..., rest], big[0][..., rest]) < tol
+        w = go.clone(); w[:, t, f] = x
+        dq, dk, dv = lib.backward(q, k, v, o0, g0, w, **kw)
+        big = oracle_all(q, k, v, w, mask=False, tau=tau, p=2)
+        assert rel_err(dv[..., f], big[4][..., f]) < tol and rel_err(dq[:, t], big[2][:, t]) < tol
+        assert rel_err(dk.double() / 1e38, big[3] / 1e38) < tol
+
+
+def check_tiny_values(lib, bh, n, d, dtype, device, *, tol, flags=0, seed=0):
+    """One of v, dO, q and k far below 1e-30, at the same bar as ordinary numbers: everything here is linear in v and in dO,
+    and dq and dk in the other factor.  (The results stay above fp32's subnormal numbers.)"""
+    tau = 8.0 * math.sqrt(d)
+    for which, scale in ((2, 3e-36), (3, 1e-34), (0, 1e-35), (1, 1e-35)):
+        x = list(make_inputs(bh, n, n, d, torch.float32, device, seed + which, go_scale=1.0 if which == 3 else 1e4))
+        x[which] = x[which] * scale
+        q, k, v, go = (t.to(dtype) for t in x)
+        kw = dict(mask=True, inv_tau=1.0 / tau, p=2, flags=flags)
+        o, g = lib.forward(q, k, v, **kw)
+        grads = lib.backward(q, k, v, o, g, go, **kw)
+        ref = oracle_all(q, k, v, go, mask=True, tau=tau, p=2)
+        errs = {m: rel_err(a, b) for m, a, b in zip(("o", "g", "dq", "dk", "dv"), (o, g, *grads), ref)}
+        assert max(errs.values()) < tol, f"tiny {'q k v dO'.split()[which]}: {errs}"

@@ -4,7 +4,7 @@ bf16-rounded inputs)."""
 import pytest
 import torch
 
-from tests.parity import (check_batch_head_strides, check_decode, check_forward, check_forward_backward,
+from tests.parity import (check_infinite_and_largest_values, check_batch_head_strides, check_decode, check_forward, check_forward_backward,
                           check_norm_fold, make_inputs)
 from reproducing_fastmax_results_amd._capi import FLAG_F32_COMPUTE, FLAG_FORCE_DENSE, FLAG_FORCE_MOMENTS, FLAG_NORM_SELF
 
@@ -283,6 +283,14 @@ def test_fp32_dense_tiles(lib, d, bh, n):
         assert n == 1 or max(e.values()) < 2e-6, e
     check_forward_backward(lib, min(bh, 3), n, d, torch.bfloat16, DEV, mask=True, p=2, seed=132, saved=True,
                            flags=FLAG_F32_COMPUTE)
+
+
+@pytest.mark.parametrize("d", [32, 64])
+@pytest.mark.parametrize("bh", [3, 256, 512])
+def test_infinite_and_largest_values_on_fp32_dense_tiles(lib, d, bh):
+    """Own tiles shared by four, two and one wavefronts; a workgroup that meets such a value makes its rows again."""
+    print(f"case infinite values d={d} bh={bh}", flush=True)
+    check_infinite_and_largest_values(lib, bh, 70, d, torch.float32, DEV, seed=150)
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])

@@ -16,7 +16,7 @@ import pytest
 import torch
 
 from reproducing_fastmax_results_amd import _capi
-from tests.parity import (TOL, check_batch_head_strides, check_decode, check_norm_fold, check_forward, check_forward_backward, make_inputs, oracle_all,
+from tests.parity import (TOL, check_infinite_and_largest_values, check_tiny_values, check_batch_head_strides, check_decode, check_norm_fold, check_forward, check_forward_backward, make_inputs, oracle_all,
                           rel_err)
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -338,3 +338,16 @@ def test_short_sequences_of_bf16_tensors_in_fp32(sim):
     want = float((f[0, 0] - f[0, 1]) / f.sum())
     o, _ = sim.forward(q.bfloat16(), k.bfloat16(), v.bfloat16(), mask=False, inv_tau=1.0, p=1, flags=_capi.FLAG_F32_COMPUTE)
     assert ((o.double() - want).abs() <= 0.025 * want).all(), (o[0, 0, 0], want)
+
+
+def test_infinite_and_largest_values_on_fp32_dense_tiles(sim):
+    # three bf16 parts hold neither (fm_x3.h): such workgroups make their rows again in fp32
+    check_infinite_and_largest_values(sim, 1, 66, 32, torch.float32, "cpu", seed=60)
+
+
+def test_tiny_values_on_fp32_dense_tiles(sim):
+    n, d = 66, 32
+    # the matrix instruction flushes bf16 parts under 2^-126 (the simulator's does too); the bar of test_fp32_dense_tiles
+    check_tiny_values(sim, 1, n, d, torch.float32, "cpu", tol=2e-6, seed=61)
+    # a coefficient that scaling would take out of the normal range: fp32 products from the start
+    check_forward_backward(sim, 1, n, d, torch.float32, "cpu", mask=True, p=2, a=(1.0, 1.0, 1e-20), seed=62)
