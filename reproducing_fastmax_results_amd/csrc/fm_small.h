@@ -35,6 +35,8 @@ template <typename TIO, int DH, bool FULL> struct SmallCfg {
   static constexpr int PL = RAW ? 1 : 3;        // planes of an operand in LDS
   static constexpr int N = DH / 32;                    // eight-feature items of a tensor per thread
   static constexpr int PQ = PL * DH + 8, TILE = 64 * PQ, OP = DH + 4;
+  static constexpr int PF = DH + 1;                    // PLAIN: pitch of a row of floats (fp32 tensors)
+  static_assert(RAW || 2 * PF <= PQ, "a row of floats fits a row of planes");
   static constexpr size_t OS = size_t(2) * 64 * OP * 4;            // one result's two parts
   static constexpr size_t fwd_lds() { const size_t a = size_t(3) * TILE * 2, b = OS + 2 * 64 * 4; return a > b ? a : b; }
   static constexpr size_t bwd_lds() { const size_t a = size_t(4) * TILE * 2 + 2 * 64 * 4; return a > OS ? a : OS; }
@@ -53,7 +55,10 @@ FM_DEVICE void fm_small_load(const TRef<const TIO>& t, int bh, int n, int tid, f
     }
   }
 }
-template <typename TIO, int DH, bool FULL> FM_DEVICE void fm_small_stage(uint16_t* tile, const float (*r)[8], const float* f, int tid) {
+// PLAIN, here and below: the second pass of a workgroup whose sums came out non-finite (the lower planes of a weight are
+// zero or of either sign, so an infinite factor makes NaN or the other infinity of them; and see fm_x3_look): rows as
+// floats (bf16 tensors: their own rows) and sums on the vector units, term by term, over the keys a query sees.
+template <typename TIO, int DH, bool FULL, bool PLAIN> FM_DEVICE void fm_small_stage(uint16_t* tile, const float (*r)[8], const float* f, int tid) {
   typedef SmallCfg<TIO, DH, FULL> C;
 #pragma unroll
   for (int i = 0; i < DH / 32; ++i) {
@@ -61,6 +66,10 @@ template <typename TIO, int DH, bool FULL> FM_DEVICE void fm_small_stage(uint16_
     uint16_t* p = tile + row * C::PQ + col;
     if constexpr (C::RAW) {
       IO<fm_bf16>::st8(p, true, r[i]);                 // exact: they came from bf16
+    } else if constexpr (PLAIN) {
+      float* q = reinterpret_cast<float*>(tile) + row * C::PF + col;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) q[j] = r[i][j] * f[i];
     } else {
       float w[8];
 #pragma unroll
@@ -100,6 +109,22 @@ FM_DEVICE float fm_small_factor(const unsigned long long* keys, bool on, float l
   return m2 > FM_MAXNORM_FLOOR ? lim * fm_rsqrtf(m2) : 0.0f;
 }
 
+template <typename TIO, int DH, bool FULL> FM_DEVICE float fm_small_at(const uint16_t* tile, int row, int col) {   // PLAIN
+  typedef SmallCfg<TIO, DH, FULL> C;
+  if constexpr (C::RAW) return fm_bf16_to_f32(tile[row * C::PQ + col]);
+  else return reinterpret_cast<const float*>(tile)[row * C::PF + col];
+}
+template <typename TIO, int DH, bool FULL> FM_DEVICE float fm_small_dot(const uint16_t* a, int ra, const uint16_t* b, int rb) {
+  float s = 0.f;
+#pragma unroll 1
+  for (int f = 0; f < DH; ++f) s += fm_small_at<TIO, DH, FULL>(a, ra, f) * fm_small_at<TIO, DH, FULL>(b, rb, f);
+  return s;
+}
+template <typename TIO, int DH, bool FULL> FM_DEVICE void fm_small_add8(float v[8], float w, const uint16_t* tile, int row, int col) {
+#pragma unroll
+  for (int j = 0; j < 8; ++j) v[j] += w * fm_small_at<TIO, DH, FULL>(tile, row, col + j);
+}
+
 // 32 x 32 tile of rows `a` and columns `b` (tiles of 32 rows in LDS)
 template <typename TIO, int DH, bool FULL> FM_DEVICE fm_f32x16 fm_small_tile(const uint16_t* a, const uint16_t* b, int lr, int lh) {
   typedef SmallCfg<TIO, DH, FULL> C;
@@ -132,17 +157,15 @@ template <typename TIO, int DH, bool FULL> FM_DEVICE void fm_small_acc(fm_f32x16
   }
 }
 
-// grid (1, bh), 256 threads
-template <typename TIO, int DH, bool FULL>
-FM_GLOBAL void FM_LAUNCH_BOUNDS2(256, 2) k_small_fwd(SmallArgs<TIO> A) {
+// false: a sum is not finite, nothing is stored (bad: one flag in LDS, see fm_x3_look; keys: two times four, in LDS)
+template <typename TIO, int DH, bool FULL, bool PLAIN>
+FM_DEVICE bool fm_small_fwd(const SmallArgs<TIO>& A, unsigned char* smem, unsigned long long (*keys)[4], int* bad, const int tid) {
   typedef SmallCfg<TIO, DH, FULL> C;
   constexpr int NT = DH / 32, N = C::N;
-  FM_DYN_SMEM(smem);
-  FM_SHARED unsigned long long keys[2][4];
   uint16_t* Q = reinterpret_cast<uint16_t*>(smem);
   uint16_t* K = Q + C::TILE;
   uint16_t* V = K + C::TILE;
-  const int tid = FM_TID_X, lane = tid & 63, lr = lane & 31, lh = lane >> 5, bh = FM_BID_Y;
+  const int lane = tid & 63, lr = lane & 31, lh = lane >> 5, bh = FM_BID_Y;
   const int wave = FM_UNIFORM(tid >> 6), ti = wave >> 1, tj = wave & 1, off = A.nk - A.nq;
   float rq[N][8], rk[N][8], rv[N][8];
   fm_small_load<TIO, DH>(A.q, bh, A.nq, tid, rq);
@@ -158,41 +181,58 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(256, 2) k_small_fwd(SmallArgs<TIO> A) {
     fk *= fm_small_factor(keys[1], A.norm_k != 0, A.lim, m2, ns);
   }
   const float sq[2] = {fq, fq}, sk[2] = {fk, fk}, one[2] = {1.0f, 1.0f};
-  fm_small_stage<TIO, DH, FULL>(Q, rq, sq, tid);
-  fm_small_stage<TIO, DH, FULL>(K, rk, sk, tid);
-  fm_small_stage<TIO, DH, FULL>(V, rv, one, tid);
+  fm_small_stage<TIO, DH, FULL, PLAIN>(Q, rq, sq, tid);
+  fm_small_stage<TIO, DH, FULL, PLAIN>(K, rk, sk, tid);
+  fm_small_stage<TIO, DH, FULL, PLAIN>(V, rv, one, tid);
   FM_SYNC();
-  fm_f32x16 acc[NT];
-#pragma unroll
-  for (int ct = 0; ct < NT; ++ct) acc[ct] = fm_zero16();
-  float gs = 0.f;
-  if (32 * ti < A.nq && 32 * tj < A.nk && !(A.causal && 32 * tj > 32 * ti + 31 + off)) {
-    fm_f32x16 s = fm_small_tile<TIO, DH, FULL>(K + 32 * tj * C::PQ, Q + 32 * ti * C::PQ, lr, lh);
-    int last = A.nk - 1 - 32 * tj;                     // last key row the lane's query sees
-    if (A.causal) { const int l = 32 * ti + lr + off - 32 * tj; last = l < last ? l : last; }
-    const float ss = C::RAW ? fq * fk : 1.0f;
-#pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const float x = C::RAW ? s[e] * ss : s[e], p = A.a0 + x * (A.a1 + A.a2 * x);
-      s[e] = fm_acc_row(e, lh) <= last ? p : 0.f;
-      gs += s[e];
-    }
-    fm_small_acc<TIO, DH, FULL>(acc, V + 32 * tj * C::PQ, s, lane);
-  }
-  FM_SYNC();
+  const float ss = C::RAW ? fq * fk : 1.0f;
   float* Os = reinterpret_cast<float*>(smem);
   float* Gs = Os + 2 * 64 * C::OP;
-  fm_x3_put<DH, 64>(acc, Os, tj, 32 * ti + lr, lh);
-  gs += fm_shfl_xor(gs, 32);
-  if (lh == 0) Gs[tj * 64 + 32 * ti + lr] = gs;
-  FM_SYNC();
+  if constexpr (!PLAIN) {
+    fm_f32x16 acc[NT];
+#pragma unroll
+    for (int ct = 0; ct < NT; ++ct) acc[ct] = fm_zero16();
+    float gs = 0.f;
+    if (32 * ti < A.nq && 32 * tj < A.nk && !(A.causal && 32 * tj > 32 * ti + 31 + off)) {
+      fm_f32x16 s = fm_small_tile<TIO, DH, FULL>(K + 32 * tj * C::PQ, Q + 32 * ti * C::PQ, lr, lh);
+      int last = A.nk - 1 - 32 * tj;                     // last key row the lane's query sees
+      if (A.causal) { const int l = 32 * ti + lr + off - 32 * tj; last = l < last ? l : last; }
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const float x = C::RAW ? s[e] * ss : s[e], p = A.a0 + x * (A.a1 + A.a2 * x);
+        s[e] = fm_acc_row(e, lh) <= last ? p : 0.f;
+        gs += s[e];
+      }
+      fm_small_acc<TIO, DH, FULL>(acc, V + 32 * tj * C::PQ, s, lane);
+    }
+    fm_x3_look<NT>(bad, acc, gs);
+    FM_SYNC();
+    fm_x3_put<DH, 64>(acc, Os, tj, 32 * ti + lr, lh);
+    gs += fm_shfl_xor(gs, 32);
+    if (lh == 0) Gs[tj * 64 + 32 * ti + lr] = gs;
+    FM_SYNC();
+    if (__builtin_expect(*bad != 0, 0)) return false;
+  }
 #pragma unroll
   for (int i = 0; i < N; ++i) {
     const int c = tid + 256 * i, row = c / (DH / 8), col = (c % (DH / 8)) * 8;
     if (row >= A.nq) continue;
-    float v[8];
-    fm_x3_sum8<DH, 64, 2>(Os, row, col, v);
-    const float gt = Gs[row] + Gs[64 + row], gi = 1.0f / gt;
+    float v[8], gt = 0.f;
+    if constexpr (PLAIN) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] = 0.f;
+      const int ke = A.causal && row + off + 1 < A.nk ? row + off + 1 : A.nk;
+#pragma unroll 1
+      for (int t = 0; t < ke; ++t) {
+        const float x = fm_small_dot<TIO, DH, FULL>(Q, row, K, t) * ss, p = A.a0 + x * (A.a1 + A.a2 * x);
+        gt += p;
+        fm_small_add8<TIO, DH, FULL>(v, p, V, t, col);
+      }
+    } else {
+      fm_x3_sum8<DH, 64, 2>(Os, row, col, v);
+      gt = Gs[row] + Gs[64 + row];
+    }
+    const float gi = 1.0f / gt;
 #pragma unroll
     for (int j = 0; j < 8; ++j) v[j] *= gi;
     IO<TIO>::st8(A.out.base(bh) + int64_t(row) * A.out.s_n + col, A.out.vec != 0, v);
@@ -204,15 +244,27 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(256, 2) k_small_fwd(SmallArgs<TIO> A) {
     }
     if (col == 0) A.g.base(bh)[int64_t(row) * A.g.s_n] = gt;
   }
+  return true;
+}
+// grid (1, bh), 256 threads
+template <typename TIO, int DH, bool FULL>
+FM_GLOBAL void FM_LAUNCH_BOUNDS2(256, 2) k_small_fwd(SmallArgs<TIO> A) {
+  FM_DYN_SMEM(smem);
+  FM_SHARED unsigned long long keys[2][4];
+  FM_SHARED int bad;
+  if (FM_TID_X == 0) bad = 0;
+  if (fm_small_fwd<TIO, DH, FULL, false>(A, smem, keys, &bad, FM_TID_X)) return;
+  (void)fm_small_fwd<TIO, DH, FULL, true>(FM_ARGS_AGAIN(A), smem, keys, &bad, FM_TID_X + FM_OPAQUE_ZERO());
 }
 
 // one result's rows: the two parts summed and scaled; returns the thread's share of sum value * raw
+// (Os null: the sums are in v)
 template <int DH> FM_DEVICE float fm_small_result(const float* Os, float scale, const float (*raw)[8], int tid, float (*v)[8]) {
   float b = 0.f;
 #pragma unroll
   for (int i = 0; i < DH / 32; ++i) {
     const int c = tid + 256 * i, row = c / (DH / 8), col = (c % (DH / 8)) * 8;
-    fm_x3_sum8<DH, 64, 2>(Os, row, col, v[i]);
+    if (Os) fm_x3_sum8<DH, 64, 2>(Os, row, col, v[i]);
 #pragma unroll
     for (int j = 0; j < 8; ++j) { v[i][j] *= scale; b += v[i][j] * raw[i][j]; }
   }
@@ -233,21 +285,19 @@ FM_DEVICE void fm_small_store(const TRef<TIO>& t, int bh, int n, int nstar, floa
   }
 }
 
-// grid (1, bh), 256 threads
-template <typename TIO, int DH, bool FULL>
-FM_GLOBAL void FM_LAUNCH_BOUNDS2(256, (DH == 64 ? (sizeof(TIO) == 4 ? 1 : 2) : (sizeof(TIO) == 4 ? 2 : 3))) k_small_bwd(SmallArgs<TIO> A) {
+// false: as fm_small_fwd (bsum: two times four floats in LDS)
+template <typename TIO, int DH, bool FULL, bool PLAIN>
+FM_DEVICE bool fm_small_bwd(const SmallArgs<TIO>& A, unsigned char* smem, unsigned long long (*keys)[4], float (*bsum)[4], int* bad,
+                            const int tid) {
   typedef SmallCfg<TIO, DH, FULL> C;
   constexpr int NT = DH / 32, N = C::N;
-  FM_DYN_SMEM(smem);
-  FM_SHARED unsigned long long keys[2][4];
-  FM_SHARED float bsum[2][4];
   uint16_t* Q = reinterpret_cast<uint16_t*>(smem);
   uint16_t* K = Q + C::TILE;
   uint16_t* V = K + C::TILE;
   uint16_t* G = V + C::TILE;                           // gh = dO / g (bf16 tensors: dO)
   float* cs = reinterpret_cast<float*>(G + C::TILE);   // c = gh . o
   float* gr = cs + 64;                                 // 1 / g
-  const int tid = FM_TID_X, lane = tid & 63, lr = lane & 31, lh = lane >> 5, bh = FM_BID_Y;
+  const int lane = tid & 63, lr = lane & 31, lh = lane >> 5, bh = FM_BID_Y;
   const int wave = FM_UNIFORM(tid >> 6), ti = wave >> 1, tj = wave & 1, off = A.nk - A.nq;
   float rq[N][8], rk[N][8];
   float fq = 1.0f, fk = 1.0f, m2q = 0.f, m2k = 0.f;
@@ -277,10 +327,10 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(256, (DH == 64 ? (sizeof(TIO) == 4 ? 1 : 2) : (
       fk = fm_small_factor(keys[1], A.norm_k != 0, A.lim, m2k, nsk);
     }
     const float sq[2] = {A.sc * fq, A.sc * fq}, sk[2] = {A.sc * fk, A.sc * fk}, one[2] = {1.0f, 1.0f};
-    fm_small_stage<TIO, DH, FULL>(Q, rq, sq, tid);
-    fm_small_stage<TIO, DH, FULL>(K, rk, sk, tid);
-    fm_small_stage<TIO, DH, FULL>(V, rv, one, tid);
-    fm_small_stage<TIO, DH, FULL>(G, rd, gi, tid);
+    fm_small_stage<TIO, DH, FULL, PLAIN>(Q, rq, sq, tid);
+    fm_small_stage<TIO, DH, FULL, PLAIN>(K, rk, sk, tid);
+    fm_small_stage<TIO, DH, FULL, PLAIN>(V, rv, one, tid);
+    fm_small_stage<TIO, DH, FULL, PLAIN>(G, rd, gi, tid);
 #pragma unroll
     for (int i = 0; i < N; ++i) {
       const int c = tid + 256 * i;
@@ -292,58 +342,85 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(256, (DH == 64 ? (sizeof(TIO) == 4 ? 1 : 2) : (
     }
   }
   FM_SYNC();
-  fm_f32x16 aq[NT], ak[NT], av[NT];
-#pragma unroll
-  for (int ct = 0; ct < NT; ++ct) { aq[ct] = fm_zero16(); ak[ct] = fm_zero16(); av[ct] = fm_zero16(); }
-  if (32 * ti < A.nq && 32 * tj < A.nk && !(A.causal && 32 * tj > 32 * ti + 31 + off)) {
-    const uint16_t *Qt = Q + 32 * ti * C::PQ, *Kt = K + 32 * tj * C::PQ, *Vt = V + 32 * tj * C::PQ, *Gt = G + 32 * ti * C::PQ;
-    const float ta2 = 2.0f * A.a2;
-    const float ss = C::RAW ? A.sc * A.sc * fq * fk : 1.0f;
-    const int diag = 32 * (ti - tj) + off;             // query row r sees key rows 0 .. r + diag
-    {
-      // rows = keys, column = the lane's query
-      fm_f32x16 s = fm_small_tile<TIO, DH, FULL>(Kt, Qt, lr, lh);
-      const fm_f32x16 dp = fm_small_tile<TIO, DH, FULL>(Vt, Gt, lr, lh);
-      const float c = cs[32 * ti + lr], gi = C::RAW ? gr[32 * ti + lr] : 1.0f;
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const float ds = (A.a1 + ta2 * (s[e] * ss)) * (dp[e] * gi - c);
-        s[e] = A.causal && fm_acc_row(e, lh) > lr + diag ? 0.f : ds;
-      }
-      fm_small_acc<TIO, DH, FULL>(aq, Kt, s, lane);
-    }
-    {
-      // rows = queries, column = the lane's key (rows past the last query: gh = c = 0, they add nothing)
-      fm_f32x16 s = fm_small_tile<TIO, DH, FULL>(Qt, Kt, lr, lh);
-      fm_f32x16 dp = fm_small_tile<TIO, DH, FULL>(Gt, Vt, lr, lh);
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const int r = fm_acc_row(e, lh);
-        const float gi = C::RAW ? gr[32 * ti + r] : 1.0f, x = s[e] * ss;
-        const float ds = (A.a1 + ta2 * x) * (dp[e] * gi - cs[32 * ti + r]), p = (A.a0 + x * (A.a1 + A.a2 * x)) * gi;
-        const bool hid = A.causal && lr > r + diag;
-        dp[e] = hid ? 0.f : ds;
-        s[e] = hid ? 0.f : p;
-      }
-      fm_small_acc<TIO, DH, FULL>(ak, Qt, dp, lane);
-      fm_small_acc<TIO, DH, FULL>(av, Gt, s, lane);
-    }
-  }
-  // the three results in turn through one region (two parts each), so that two to four workgroups share a CU
-  float* Os = reinterpret_cast<float*>(smem);
+  const float ta2 = 2.0f * A.a2, ss = C::RAW ? A.sc * A.sc * fq * fk : 1.0f;
+  const float scale_q = A.sc * (A.jac ? fq : 1.0f) * (C::RAW ? A.sc * fk : 1.0f), scale_k = A.sc * (A.jac ? fk : 1.0f) * (C::RAW ? A.sc * fq : 1.0f);
   float vq[N][8], vk[N][8], vv[N][8];
-  FM_SYNC();
-  fm_x3_put<DH, 64>(aq, Os, tj, 32 * ti + lr, lh);
-  FM_SYNC();
-  float bq = fm_small_result<DH>(Os, A.sc * (A.jac ? fq : 1.0f) * (C::RAW ? A.sc * fk : 1.0f), rq, tid, vq);
-  FM_SYNC();
-  fm_x3_put<DH, 64>(ak, Os, ti, 32 * tj + lr, lh);
-  FM_SYNC();
-  float bk = fm_small_result<DH>(Os, A.sc * (A.jac ? fk : 1.0f) * (C::RAW ? A.sc * fq : 1.0f), rk, tid, vk);
-  FM_SYNC();
-  fm_x3_put<DH, 64>(av, Os, ti, 32 * tj + lr, lh);
-  FM_SYNC();
-  (void)fm_small_result<DH>(Os, 1.0f, rk, tid, vv);
+  float bq, bk;
+  if constexpr (PLAIN) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const int c = tid + 256 * i, row = c / (DH / 8), col = (c % (DH / 8)) * 8;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) { vq[i][j] = 0.f; vk[i][j] = 0.f; vv[i][j] = 0.f; }
+      const int ke = row >= A.nq ? 0 : A.causal && row + off + 1 < A.nk ? row + off + 1 : A.nk;
+#pragma unroll 1
+      for (int t = 0; t < ke; ++t) {
+        const float x = fm_small_dot<TIO, DH, FULL>(Q, row, K, t) * ss, dp = fm_small_dot<TIO, DH, FULL>(G, row, V, t) * (C::RAW ? gr[row] : 1.0f);
+        fm_small_add8<TIO, DH, FULL>(vq[i], (A.a1 + ta2 * x) * (dp - cs[row]), K, t, col);
+      }
+      const int qb = A.causal && row > off ? row - off : 0;
+#pragma unroll 1
+      for (int t = row < A.nk ? qb : A.nq; t < A.nq; ++t) {
+        const float gi = C::RAW ? gr[t] : 1.0f, x = fm_small_dot<TIO, DH, FULL>(Q, t, K, row) * ss, dp = fm_small_dot<TIO, DH, FULL>(G, t, V, row) * gi;
+        fm_small_add8<TIO, DH, FULL>(vk[i], (A.a1 + ta2 * x) * (dp - cs[t]), Q, t, col);
+        fm_small_add8<TIO, DH, FULL>(vv[i], (A.a0 + x * (A.a1 + A.a2 * x)) * gi, G, t, col);
+      }
+    }
+    bq = fm_small_result<DH>(nullptr, scale_q, rq, tid, vq);
+    bk = fm_small_result<DH>(nullptr, scale_k, rk, tid, vk);
+  } else {
+    fm_f32x16 aq[NT], ak[NT], av[NT];
+#pragma unroll
+    for (int ct = 0; ct < NT; ++ct) { aq[ct] = fm_zero16(); ak[ct] = fm_zero16(); av[ct] = fm_zero16(); }
+    if (32 * ti < A.nq && 32 * tj < A.nk && !(A.causal && 32 * tj > 32 * ti + 31 + off)) {
+      const uint16_t *Qt = Q + 32 * ti * C::PQ, *Kt = K + 32 * tj * C::PQ, *Vt = V + 32 * tj * C::PQ, *Gt = G + 32 * ti * C::PQ;
+      const int diag = 32 * (ti - tj) + off;             // query row r sees key rows 0 .. r + diag
+      {
+        // rows = keys, column = the lane's query
+        fm_f32x16 s = fm_small_tile<TIO, DH, FULL>(Kt, Qt, lr, lh);
+        const fm_f32x16 dp = fm_small_tile<TIO, DH, FULL>(Vt, Gt, lr, lh);
+        const float c = cs[32 * ti + lr], gi = C::RAW ? gr[32 * ti + lr] : 1.0f;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const float ds = (A.a1 + ta2 * (s[e] * ss)) * (dp[e] * gi - c);
+          s[e] = A.causal && fm_acc_row(e, lh) > lr + diag ? 0.f : ds;
+        }
+        fm_small_acc<TIO, DH, FULL>(aq, Kt, s, lane);
+      }
+      {
+        // rows = queries, column = the lane's key (rows past the last query: gh = c = 0, they add nothing)
+        fm_f32x16 s = fm_small_tile<TIO, DH, FULL>(Qt, Kt, lr, lh);
+        fm_f32x16 dp = fm_small_tile<TIO, DH, FULL>(Gt, Vt, lr, lh);
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const int r = fm_acc_row(e, lh);
+          const float gi = C::RAW ? gr[32 * ti + r] : 1.0f, x = s[e] * ss;
+          const float ds = (A.a1 + ta2 * x) * (dp[e] * gi - cs[32 * ti + r]), p = (A.a0 + x * (A.a1 + A.a2 * x)) * gi;
+          const bool hid = A.causal && lr > r + diag;
+          dp[e] = hid ? 0.f : ds;
+          s[e] = hid ? 0.f : p;
+        }
+        fm_small_acc<TIO, DH, FULL>(ak, Qt, dp, lane);
+        fm_small_acc<TIO, DH, FULL>(av, Gt, s, lane);
+      }
+    }
+    // the three results in turn through one region (two parts each), so that two to four workgroups share a CU
+    float* Os = reinterpret_cast<float*>(smem);
+    fm_x3_look<NT>(bad, aq, 0.f); fm_x3_look<NT>(bad, ak, 0.f); fm_x3_look<NT>(bad, av, 0.f);
+    FM_SYNC();
+    fm_x3_put<DH, 64>(aq, Os, tj, 32 * ti + lr, lh);
+    FM_SYNC();
+    if (__builtin_expect(*bad != 0, 0)) return false;
+    bq = fm_small_result<DH>(Os, scale_q, rq, tid, vq);
+    FM_SYNC();
+    fm_x3_put<DH, 64>(ak, Os, ti, 32 * tj + lr, lh);
+    FM_SYNC();
+    bk = fm_small_result<DH>(Os, scale_k, rk, tid, vk);
+    FM_SYNC();
+    fm_x3_put<DH, 64>(av, Os, ti, 32 * tj + lr, lh);
+    FM_SYNC();
+    (void)fm_small_result<DH>(Os, 1.0f, rk, tid, vv);
+  }
   float cq = 0.f, ck = 0.f;
   if (A.jac) {
 #pragma unroll
@@ -356,4 +433,17 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(256, (DH == 64 ? (sizeof(TIO) == 4 ? 1 : 2) : (
   fm_small_store<TIO, DH>(A.out, bh, A.nq, cq != 0.f ? nsq : -1, cq, rq, tid, vq);
   fm_small_store<TIO, DH>(A.dk, bh, A.nk, ck != 0.f ? nsk : -1, ck, rk, tid, vk);
   fm_small_store<TIO, DH>(A.dv, bh, A.nk, -1, 0.f, rk, tid, vv);
+  return true;
+}
+// grid (1, bh), 256 threads
+template <typename TIO, int DH, bool FULL>
+FM_GLOBAL void FM_LAUNCH_BOUNDS2(256, (DH == 64 ? (sizeof(TIO) == 4 ? 1 : 2) : (sizeof(TIO) == 4 ? 2 : 3))) k_small_bwd(SmallArgs<TIO> A) {
+  FM_DYN_SMEM(smem);
+  FM_SHARED unsigned long long keys[2][4];
+  FM_SHARED float bsum[2][4];
+  FM_SHARED int bad;
+  if (FM_TID_X == 0) bad = 0;
+  if (fm_small_bwd<TIO, DH, FULL, false>(A, smem, keys, bsum, &bad, FM_TID_X)) return;
+  FM_SYNC();                                           // (the first result's region becomes tiles again)
+  (void)fm_small_bwd<TIO, DH, FULL, true>(FM_ARGS_AGAIN(A), smem, keys, bsum, &bad, FM_TID_X + FM_OPAQUE_ZERO());
 }

@@ -191,7 +191,7 @@ def check_infinite_and_largest_values(lib, bh, n, d, dtype, device, *, flags=0, 
         others = [i for i in range(n) if i != t]
         assert rel_err(dq[:, others], ref[2][:, others]) < tol
         assert not bool(torch.isfinite(dq[:, t]).any()) and not bool(torch.isfinite(dk).any())
-    for x in (largest or (3.0e38, 3.4e38)):
+    for x in ((3.0e38, 3.4e38) if largest is None else largest):
         w = v.clone(); w[:, t, f] = x
         o, g = lib.forward(q, k, w, **kw)
         big = oracle_all(q, k, w, go, mask=False, tau=tau, p=2)

@@ -293,6 +293,15 @@ def test_infinite_and_largest_values_on_fp32_dense_tiles(lib, d, bh):
     check_infinite_and_largest_values(lib, bh, 70, d, torch.float32, DEV, seed=150)
 
 
+@pytest.mark.parametrize("dtype,flags", [(torch.float32, 0), (torch.bfloat16, 0), (torch.bfloat16, FLAG_F32_COMPUTE)])
+@pytest.mark.parametrize("d", [32, 64])
+@pytest.mark.parametrize("n", [20, 50, 64])
+def test_infinite_and_largest_values_in_short_sequences(lib, dtype, flags, d, n):
+    print(f"case infinite values, short dtype={dtype} flags={flags} d={d} n={n}", flush=True)
+    check_infinite_and_largest_values(lib, 5, n, d, dtype, DEV, flags=flags, seed=151,
+                                      largest=None if dtype == torch.float32 else (1e30,))
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("d", [32, 64])
 @pytest.mark.parametrize("nq,nk", [(1, 1), (1, 64), (1, 65), (2, 4097), (3, 130), (5, 8192), (16, 16), (64, 64), (64, 1000)])

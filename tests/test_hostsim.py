@@ -351,3 +351,9 @@ def test_tiny_values_on_fp32_dense_tiles(sim):
     check_tiny_values(sim, 1, n, d, torch.float32, "cpu", tol=2e-6, seed=61)
     # a coefficient that scaling would take out of the normal range: fp32 products from the start
     check_forward_backward(sim, 1, n, d, torch.float32, "cpu", mask=True, p=2, a=(1.0, 1.0, 1e-20), seed=62)
+
+
+def test_infinite_and_largest_values_in_short_sequences(sim):
+    for dtype, flags in ((torch.float32, 0), (torch.bfloat16, 0), (torch.bfloat16, _capi.FLAG_F32_COMPUTE)):
+        check_infinite_and_largest_values(sim, 1, 20, 32, dtype, "cpu", flags=flags, seed=63,
+                                          largest=None if dtype == torch.float32 else (1e30,))
