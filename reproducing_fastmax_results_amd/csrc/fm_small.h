@@ -157,9 +157,9 @@ template <typename TIO, int DH, bool FULL> FM_DEVICE void fm_small_acc(fm_f32x16
   }
 }
 
-// false: a sum is not finite, nothing is stored (bad: one flag in LDS, see fm_x3_look; keys: two times four, in LDS)
+// bad: one flag in LDS, see fm_x3_look; keys: two times four, in LDS
 template <typename TIO, int DH, bool FULL, bool PLAIN>
-FM_DEVICE bool fm_small_fwd(const SmallArgs<TIO>& A, unsigned char* smem, unsigned long long (*keys)[4], int* bad, const int tid) {
+FM_DEVICE void fm_small_fwd(const SmallArgs<TIO>& A, unsigned char* smem, unsigned long long (*keys)[4], int* bad, const int tid) {
   typedef SmallCfg<TIO, DH, FULL> C;
   constexpr int NT = DH / 32, N = C::N;
   uint16_t* Q = reinterpret_cast<uint16_t*>(smem);
@@ -205,13 +205,11 @@ FM_DEVICE bool fm_small_fwd(const SmallArgs<TIO>& A, unsigned char* smem, unsign
       }
       fm_small_acc<TIO, DH, FULL>(acc, V + 32 * tj * C::PQ, s, lane);
     }
-    fm_x3_look<NT>(bad, acc, gs);
     FM_SYNC();
     fm_x3_put<DH, 64>(acc, Os, tj, 32 * ti + lr, lh);
     gs += fm_shfl_xor(gs, 32);
     if (lh == 0) Gs[tj * 64 + 32 * ti + lr] = gs;
     FM_SYNC();
-    if (__builtin_expect(*bad != 0, 0)) return false;
   }
 #pragma unroll
   for (int i = 0; i < N; ++i) {
@@ -231,6 +229,7 @@ FM_DEVICE bool fm_small_fwd(const SmallArgs<TIO>& A, unsigned char* smem, unsign
     } else {
       fm_x3_sum8<DH, 64, 2>(Os, row, col, v);
       gt = Gs[row] + Gs[64 + row];
+      fm_x3_look(bad, v, gt);
     }
     const float gi = 1.0f / gt;
 #pragma unroll
@@ -244,7 +243,6 @@ FM_DEVICE bool fm_small_fwd(const SmallArgs<TIO>& A, unsigned char* smem, unsign
     }
     if (col == 0) A.g.base(bh)[int64_t(row) * A.g.s_n] = gt;
   }
-  return true;
 }
 // grid (1, bh), 256 threads
 template <typename TIO, int DH, bool FULL>
@@ -253,8 +251,8 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(256, 2) k_small_fwd(SmallArgs<TIO> A) {
   FM_SHARED unsigned long long keys[2][4];
   FM_SHARED int bad;
   if (FM_TID_X == 0) bad = 0;
-  if (fm_small_fwd<TIO, DH, FULL, false>(A, smem, keys, &bad, FM_TID_X)) return;
-  (void)fm_small_fwd<TIO, DH, FULL, true>(FM_ARGS_AGAIN(A), smem, keys, &bad, FM_TID_X + FM_OPAQUE_ZERO());
+  fm_small_fwd<TIO, DH, FULL, false>(A, smem, keys, &bad, FM_TID_X);
+  if (fm_x3_again(&bad)) fm_small_fwd<TIO, DH, FULL, true>(FM_ARGS_AGAIN(A), smem, keys, &bad, FM_TID_X + FM_OPAQUE_ZERO());
 }
 
 // one result's rows: the two parts summed and scaled; returns the thread's share of sum value * raw
@@ -285,9 +283,9 @@ FM_DEVICE void fm_small_store(const TRef<TIO>& t, int bh, int n, int nstar, floa
   }
 }
 
-// false: as fm_small_fwd (bsum: two times four floats in LDS)
+// bsum: two times four floats in LDS
 template <typename TIO, int DH, bool FULL, bool PLAIN>
-FM_DEVICE bool fm_small_bwd(const SmallArgs<TIO>& A, unsigned char* smem, unsigned long long (*keys)[4], float (*bsum)[4], int* bad,
+FM_DEVICE void fm_small_bwd(const SmallArgs<TIO>& A, unsigned char* smem, unsigned long long (*keys)[4], float (*bsum)[4], int* bad,
                             const int tid) {
   typedef SmallCfg<TIO, DH, FULL> C;
   constexpr int NT = DH / 32, N = C::N;
@@ -406,11 +404,9 @@ FM_DEVICE bool fm_small_bwd(const SmallArgs<TIO>& A, unsigned char* smem, unsign
     }
     // the three results in turn through one region (two parts each), so that two to four workgroups share a CU
     float* Os = reinterpret_cast<float*>(smem);
-    fm_x3_look<NT>(bad, aq, 0.f); fm_x3_look<NT>(bad, ak, 0.f); fm_x3_look<NT>(bad, av, 0.f);
     FM_SYNC();
     fm_x3_put<DH, 64>(aq, Os, tj, 32 * ti + lr, lh);
     FM_SYNC();
-    if (__builtin_expect(*bad != 0, 0)) return false;
     bq = fm_small_result<DH>(Os, scale_q, rq, tid, vq);
     FM_SYNC();
     fm_x3_put<DH, 64>(ak, Os, ti, 32 * tj + lr, lh);
@@ -419,7 +415,9 @@ FM_DEVICE bool fm_small_bwd(const SmallArgs<TIO>& A, unsigned char* smem, unsign
     FM_SYNC();
     fm_x3_put<DH, 64>(av, Os, ti, 32 * tj + lr, lh);
     FM_SYNC();
-    (void)fm_small_result<DH>(Os, 1.0f, rk, tid, vv);
+    // a sum that is not finite makes its b that, whatever the row it is multiplied by
+    const float bv = fm_small_result<DH>(Os, 1.0f, rk, tid, vv);
+    if (!(fm_absf(bq) + fm_absf(bk) + fm_absf(bv) < 0x1p127f)) *bad = 1;
   }
   float cq = 0.f, ck = 0.f;
   if (A.jac) {
@@ -433,7 +431,6 @@ FM_DEVICE bool fm_small_bwd(const SmallArgs<TIO>& A, unsigned char* smem, unsign
   fm_small_store<TIO, DH>(A.out, bh, A.nq, cq != 0.f ? nsq : -1, cq, rq, tid, vq);
   fm_small_store<TIO, DH>(A.dk, bh, A.nk, ck != 0.f ? nsk : -1, ck, rk, tid, vk);
   fm_small_store<TIO, DH>(A.dv, bh, A.nk, -1, 0.f, rk, tid, vv);
-  return true;
 }
 // grid (1, bh), 256 threads
 template <typename TIO, int DH, bool FULL>
@@ -443,7 +440,6 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(256, (DH == 64 ? (sizeof(TIO) == 4 ? 1 : 2) : (
   FM_SHARED float bsum[2][4];
   FM_SHARED int bad;
   if (FM_TID_X == 0) bad = 0;
-  if (fm_small_bwd<TIO, DH, FULL, false>(A, smem, keys, bsum, &bad, FM_TID_X)) return;
-  FM_SYNC();                                           // (the first result's region becomes tiles again)
-  (void)fm_small_bwd<TIO, DH, FULL, true>(FM_ARGS_AGAIN(A), smem, keys, bsum, &bad, FM_TID_X + FM_OPAQUE_ZERO());
+  fm_small_bwd<TIO, DH, FULL, false>(A, smem, keys, bsum, &bad, FM_TID_X);
+  if (fm_x3_again(&bad)) fm_small_bwd<TIO, DH, FULL, true>(FM_ARGS_AGAIN(A), smem, keys, bsum, &bad, FM_TID_X + FM_OPAQUE_ZERO());
 }

@@ -221,19 +221,18 @@ template <int DH> struct F32Row {
 };
 
 // Three planes hold every finite number below 3.3953e38 (what bf16's largest number rounds down from); an infinity, a NaN
-// or a number above comes out of the split as infinity and NaN, and whatever sum it enters as NaN.  So the wavefronts look
-// at their sums before the workgroup adds and stores them and, if one is not finite (or so large that the parts' sum might
-// not be), the workgroup makes its rows again with fp32 matrix products: an infinite value then gives the infinities and NaN
-// that fp32 arithmetic gives.  bad: one flag in LDS, cleared at the kernel's start; the barrier before the sums are read
-// is the one that shows it to everybody (one of its own behind the stores would wait for them: 0.4 us).
-template <int NT> FM_DEVICE void fm_x3_look(int* bad, const fm_f32x16* acc, float g) {
-  float z[4] = {fm_absf(g), 0.f, 0.f, 0.f};
+// or a number above comes out of the split as infinity and NaN, and whatever sum it enters as NaN.  So a thread looks at the
+// sums it stores and, if one of the workgroup's is not finite, the workgroup makes its rows again with fp32 matrix products,
+// over what it stored: an infinite value then gives the infinities and NaN that fp32 arithmetic gives.  bad: one flag in
+// LDS, cleared at the kernel's start.  (A call of 8 us is bound by the length of its straight code: eight additions per
+// eight sums and a barrier that does not wait for the stores.)
+FM_DEVICE void fm_x3_look(int* bad, const float v[8], float g) {
+  float z = fm_absf(g);
 #pragma unroll
-  for (int ct = 0; ct < NT; ++ct)
-#pragma unroll
-    for (int e = 0; e < 16; ++e) z[e % 4] += fm_absf(acc[ct][e]);
-  if (!((z[0] + z[1]) + (z[2] + z[3]) < 0x1p125f)) *bad = 1;
+  for (int i = 0; i < 8; ++i) z += fm_absf(v[i]);
+  if (!(z < 0x1p127f)) *bad = 1;
 }
+FM_DEVICE bool fm_x3_again(const int* bad) { FM_SYNC_LDS(); return __builtin_expect(*bad != 0, 0); }
 
 template <typename TIO> struct X3Args {
   TRef<const TIO> q, k, v, o, d_o;
@@ -354,20 +353,20 @@ template <int DH, int QW, int SPLIT> FM_DEVICE void fm_x3_sum8(const float* Os, 
 }
 // Gradient rows of the workgroup -> caller's tensor, times scale.  bout: the sum of stored value times raw row (the
 // normalisation's B: stored = fac dy, y = fac x, so dy . y = stored . x), one float per workgroup, or null.  bad: see
-// fm_x3_look; false if it is set.
+// fm_x3_look.
 template <typename TIO, int DH, int QW, int SPLIT, int NTH, typename R>
-FM_DEVICE bool fm_x3_store(const fm_f32x16* acc, float* Os, int sub, int row, int lh, float scale, const TRef<TIO>& out,
-                           int bh, int t0, int n, int tid, const TRef<const TIO>& raw, float* bout, const int* bad) {
+FM_DEVICE void fm_x3_store(const fm_f32x16* acc, float* Os, int sub, int row, int lh, float scale, const TRef<TIO>& out,
+                           int bh, int t0, int n, int tid, const TRef<const TIO>& raw, float* bout, int* bad) {
   FM_SYNC();                                           // whatever lay there has been read
   fm_x3_put<DH, QW>(acc, Os, sub, row, lh);
   FM_SYNC();
-  if (R::PIPE && __builtin_expect(*bad != 0, 0)) return false;
   float bsum = 0.f;
   for (int c = tid; c < QW * (DH / 8); c += NTH) {
     const int r = c / (DH / 8), col = (c % (DH / 8)) * 8;
     if (t0 + r >= n) continue;
     float v[8];
     fm_x3_sum8<DH, QW, SPLIT>(Os, r, col, v);
+    if (R::PIPE) fm_x3_look(bad, v, 0.f);
 #pragma unroll
     for (int i = 0; i < 8; ++i) v[i] *= scale;
     if (bout) {
@@ -390,7 +389,6 @@ FM_DEVICE bool fm_x3_store(const fm_f32x16* acc, float* Os, int sub, int row, in
       *bout = b;
     }
   }
-  return true;
 }
 
 template <int DH, int NW, int SPLIT> struct X3Cfg {
@@ -410,7 +408,7 @@ template <int DH, int NW, int SPLIT> struct X3Cfg {
 // forward.  grid (ceil(nq / QW), bh), 256 threads.
 // ------------------------------------------------------------------------------
 template <typename TIO, int DH, int SPLIT, typename R>
-FM_DEVICE bool fm_x3_fwd(const X3Args<TIO>& A, uint16_t* st, int* bad, const int tid) {
+FM_DEVICE void fm_x3_fwd(const X3Args<TIO>& A, uint16_t* st, int* bad, const int tid) {
   typedef X3Cfg<DH, 4, SPLIT> C;
   constexpr int NT = DH / 32, PQ = C::PQ, KT = C::KT, QW = C::QW;
   const int lane = tid & 63, lr = lane & 31, lh = lane >> 5;
@@ -476,13 +474,11 @@ FM_DEVICE bool fm_x3_fwd(const X3Args<TIO>& A, uint16_t* st, int* bad, const int
   }
   float* Os = reinterpret_cast<float*>(st);
   float* Gs = Os + SPLIT * QW * (DH + 4);              // [SPLIT][QW]
-  if (R::PIPE) fm_x3_look<NT>(bad, acc, gs);
   FM_SYNC();
   fm_x3_put<DH, QW>(acc, Os, sub, 32 * own + lr, lh);
   gs += fm_shfl_xor(gs, 32);
   if (lh == 0) Gs[sub * QW + 32 * own + lr] = gs;
   FM_SYNC();
-  if (R::PIPE && __builtin_expect(*bad != 0, 0)) return false;
   for (int c = tid; c < QW * (DH / 8); c += C::NTH) {
     const int r = c / (DH / 8), col = (c % (DH / 8)) * 8, qi = t0 + r;
     if (qi >= A.nq) continue;
@@ -490,6 +486,7 @@ FM_DEVICE bool fm_x3_fwd(const X3Args<TIO>& A, uint16_t* st, int* bad, const int
     fm_x3_sum8<DH, QW, SPLIT>(Os, r, col, v);
 #pragma unroll
     for (int s = 0; s < SPLIT; ++s) gt += Gs[s * QW + r];
+    if (R::PIPE) fm_x3_look(bad, v, gt);
     const float gi = 1.0f / gt;
 #pragma unroll
     for (int i = 0; i < 8; ++i) v[i] *= gi;
@@ -502,7 +499,6 @@ FM_DEVICE bool fm_x3_fwd(const X3Args<TIO>& A, uint16_t* st, int* bad, const int
     }
     if (col == 0) A.g.base(bh)[int64_t(qi) * A.g.s_n] = gt;
   }
-  return true;
 }
 template <typename TIO, int DH, int SPLIT>
 FM_GLOBAL void FM_LAUNCH_BOUNDS2(256, (X3Cfg<DH, 4, SPLIT>::OCC)) k_x3_fwd(X3Args<TIO> A) {
@@ -510,15 +506,15 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(256, (X3Cfg<DH, 4, SPLIT>::OCC)) k_x3_fwd(X3Arg
   FM_SHARED int bad;
   uint16_t* st = reinterpret_cast<uint16_t*>(smem);
   if (FM_TID_X == 0) bad = 0;
-  if (fm_x3_fwd<TIO, DH, SPLIT, X3Row<DH>>(A, st, &bad, FM_TID_X)) return;
-  (void)fm_x3_fwd<TIO, DH, SPLIT, F32Row<DH>>(FM_ARGS_AGAIN(A), st, &bad, FM_TID_X + FM_OPAQUE_ZERO());
+  fm_x3_fwd<TIO, DH, SPLIT, X3Row<DH>>(A, st, &bad, FM_TID_X);
+  if (fm_x3_again(&bad)) fm_x3_fwd<TIO, DH, SPLIT, F32Row<DH>>(FM_ARGS_AGAIN(A), st, &bad, FM_TID_X + FM_OPAQUE_ZERO());
 }
 
 // ------------------------------------------------------------------------------
 // dQ.  grid (ceil(nq / QW), bh), 256 threads.  dS = (a1 + 2 a2 s) (gh . v - c), gh = dO / g, c = gh . o.
 // ------------------------------------------------------------------------------
 template <typename TIO, int DH, int SPLIT, typename R>
-FM_DEVICE bool fm_x3_dq(const X3Args<TIO>& A, uint16_t* st, int* bad, const int tid) {
+FM_DEVICE void fm_x3_dq(const X3Args<TIO>& A, uint16_t* st, int* bad, const int tid) {
   typedef X3Cfg<DH, 4, SPLIT> C;
   constexpr int NT = DH / 32, PQ = C::PQ, KT = C::KT, QW = C::QW;
   const int lane = tid & 63, lr = lane & 31, lh = lane >> 5;
@@ -589,8 +585,7 @@ FM_DEVICE bool fm_x3_dq(const X3Args<TIO>& A, uint16_t* st, int* bad, const int 
       }
     } else FM_SYNC();
   }
-  if (R::PIPE) fm_x3_look<NT>(bad, acc, 0.f);
-  return fm_x3_store<TIO, DH, QW, SPLIT, C::NTH, R>(acc, reinterpret_cast<float*>(st), sub, 32 * own + lr, lh, A.sc * (A.bpart ? qf : 1.0f), A.out,
+  fm_x3_store<TIO, DH, QW, SPLIT, C::NTH, R>(acc, reinterpret_cast<float*>(st), sub, 32 * own + lr, lh, A.sc * (A.bpart ? qf : 1.0f), A.out,
                                           bh, t0, A.nq, tid, A.q, A.bpart ? A.bpart + int64_t(bh) * FM_GDIM_X + blk : nullptr, bad);
 }
 template <typename TIO, int DH, int SPLIT>
@@ -599,8 +594,8 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(256, (X3Cfg<DH, 4, SPLIT>::OCC)) k_x3_dq(X3Args
   FM_SHARED int bad;
   uint16_t* st = reinterpret_cast<uint16_t*>(smem);
   if (FM_TID_X == 0) bad = 0;
-  if (fm_x3_dq<TIO, DH, SPLIT, X3Row<DH>>(A, st, &bad, FM_TID_X)) return;
-  (void)fm_x3_dq<TIO, DH, SPLIT, F32Row<DH>>(FM_ARGS_AGAIN(A), st, &bad, FM_TID_X + FM_OPAQUE_ZERO());
+  fm_x3_dq<TIO, DH, SPLIT, X3Row<DH>>(A, st, &bad, FM_TID_X);
+  if (fm_x3_again(&bad)) fm_x3_dq<TIO, DH, SPLIT, F32Row<DH>>(FM_ARGS_AGAIN(A), st, &bad, FM_TID_X + FM_OPAQUE_ZERO());
 }
 
 // ------------------------------------------------------------------------------
@@ -608,7 +603,7 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(256, (X3Cfg<DH, 4, SPLIT>::OCC)) k_x3_dq(X3Args
 // leave 256 registers each; own k in registers, own v (read once per tile) in LDS.
 // ------------------------------------------------------------------------------
 template <typename TIO, int DH, int SPLIT, typename R>
-FM_DEVICE bool fm_x3_dkv(const X3Args<TIO>& A, uint16_t* Vs, int* bad, const int tid) {
+FM_DEVICE void fm_x3_dkv(const X3Args<TIO>& A, uint16_t* Vs, int* bad, const int tid) {
   typedef X3Cfg<DH, 8, SPLIT> C;
   constexpr int NT = DH / 32, PQ = C::PQ, KT = C::KT, QW = C::QW;
   uint16_t* st = Vs + QW * PQ;                         // Vs: own v rows [QW][PQ]
@@ -703,11 +698,9 @@ FM_DEVICE bool fm_x3_dkv(const X3Args<TIO>& A, uint16_t* Vs, int* bad, const int
     } else FM_SYNC();
   }
   float* Os = reinterpret_cast<float*>(Vs);
-  if (R::PIPE) { fm_x3_look<NT>(bad, acc, 0.f); fm_x3_look<NT>(bad, av, 0.f); }
-  if (!fm_x3_store<TIO, DH, QW, SPLIT, C::NTH, R>(acc, Os, sub, 32 * own + lr, lh, A.sc * (A.bpart ? kf : 1.0f), A.out, bh, t0, A.nk, tid, A.k,
-                                          A.bpart ? A.bpart + int64_t(bh) * FM_GDIM_X + blk : nullptr, bad))
-    return false;
-  return fm_x3_store<TIO, DH, QW, SPLIT, C::NTH, R>(av, Os, sub, 32 * own + lr, lh, 1.0f, A.out2, bh, t0, A.nk, tid, A.k, nullptr, bad);
+  fm_x3_store<TIO, DH, QW, SPLIT, C::NTH, R>(acc, Os, sub, 32 * own + lr, lh, A.sc * (A.bpart ? kf : 1.0f), A.out, bh, t0, A.nk, tid, A.k,
+                                          A.bpart ? A.bpart + int64_t(bh) * FM_GDIM_X + blk : nullptr, bad);
+  fm_x3_store<TIO, DH, QW, SPLIT, C::NTH, R>(av, Os, sub, 32 * own + lr, lh, 1.0f, A.out2, bh, t0, A.nk, tid, A.k, nullptr, bad);
 }
 template <typename TIO, int DH, int SPLIT>
 FM_GLOBAL void FM_LAUNCH_BOUNDS2(512, 2) k_x3_dkv(X3Args<TIO> A) {
@@ -715,6 +708,6 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(512, 2) k_x3_dkv(X3Args<TIO> A) {
   FM_SHARED int bad;
   uint16_t* st = reinterpret_cast<uint16_t*>(smem);
   if (FM_TID_X == 0) bad = 0;
-  if (fm_x3_dkv<TIO, DH, SPLIT, X3Row<DH>>(A, st, &bad, FM_TID_X)) return;
-  (void)fm_x3_dkv<TIO, DH, SPLIT, F32Row<DH>>(FM_ARGS_AGAIN(A), st, &bad, FM_TID_X + FM_OPAQUE_ZERO());
+  fm_x3_dkv<TIO, DH, SPLIT, X3Row<DH>>(A, st, &bad, FM_TID_X);
+  if (fm_x3_again(&bad)) fm_x3_dkv<TIO, DH, SPLIT, F32Row<DH>>(FM_ARGS_AGAIN(A), st, &bad, FM_TID_X + FM_OPAQUE_ZERO());
 }
