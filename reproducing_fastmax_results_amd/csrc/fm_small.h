@@ -252,7 +252,8 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(256, 2) k_small_fwd(SmallArgs<TIO> A) {
   FM_SHARED int bad;
   if (FM_TID_X == 0) bad = 0;
   fm_small_fwd<TIO, DH, FULL, false>(A, smem, keys, &bad, FM_TID_X);
-  if (fm_x3_again(&bad)) fm_small_fwd<TIO, DH, FULL, true>(FM_ARGS_AGAIN(A), smem, keys, &bad, FM_TID_X + FM_OPAQUE_ZERO());
+  if (!fm_x3_again(&bad)) FM_END();
+  fm_small_fwd<TIO, DH, FULL, true>(FM_ARGS_AGAIN(A), smem, keys, &bad, FM_TID_X + FM_OPAQUE_ZERO());
 }
 
 // one result's rows: the two parts summed and scaled; returns the thread's share of sum value * raw
@@ -441,5 +442,6 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(256, (DH == 64 ? (sizeof(TIO) == 4 ? 1 : 2) : (
   FM_SHARED int bad;
   if (FM_TID_X == 0) bad = 0;
   fm_small_bwd<TIO, DH, FULL, false>(A, smem, keys, bsum, &bad, FM_TID_X);
-  if (fm_x3_again(&bad)) fm_small_bwd<TIO, DH, FULL, true>(FM_ARGS_AGAIN(A), smem, keys, bsum, &bad, FM_TID_X + FM_OPAQUE_ZERO());
+  if (!fm_x3_again(&bad)) FM_END();
+  fm_small_bwd<TIO, DH, FULL, true>(FM_ARGS_AGAIN(A), smem, keys, bsum, &bad, FM_TID_X + FM_OPAQUE_ZERO());
 }

@@ -232,7 +232,7 @@ FM_DEVICE void fm_x3_look(int* bad, const float v[8], float g) {
   for (int i = 0; i < 8; ++i) z += fm_absf(v[i]);
   if (!(z < 0x1p127f)) *bad = 1;
 }
-FM_DEVICE bool fm_x3_again(const int* bad) { FM_SYNC_LDS(); return __builtin_expect(*bad != 0, 0); }
+FM_DEVICE bool fm_x3_again(const int* bad) { FM_SYNC_LDS(); return __builtin_expect(FM_UNIFORM(*bad) != 0, 0); }
 
 template <typename TIO> struct X3Args {
   TRef<const TIO> q, k, v, o, d_o;
@@ -507,7 +507,8 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(256, (X3Cfg<DH, 4, SPLIT>::OCC)) k_x3_fwd(X3Arg
   uint16_t* st = reinterpret_cast<uint16_t*>(smem);
   if (FM_TID_X == 0) bad = 0;
   fm_x3_fwd<TIO, DH, SPLIT, X3Row<DH>>(A, st, &bad, FM_TID_X);
-  if (fm_x3_again(&bad)) fm_x3_fwd<TIO, DH, SPLIT, F32Row<DH>>(FM_ARGS_AGAIN(A), st, &bad, FM_TID_X + FM_OPAQUE_ZERO());
+  if (!fm_x3_again(&bad)) FM_END();
+  fm_x3_fwd<TIO, DH, SPLIT, F32Row<DH>>(FM_ARGS_AGAIN(A), st, &bad, FM_TID_X + FM_OPAQUE_ZERO());
 }
 
 // ------------------------------------------------------------------------------
@@ -595,7 +596,8 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(256, (X3Cfg<DH, 4, SPLIT>::OCC)) k_x3_dq(X3Args
   uint16_t* st = reinterpret_cast<uint16_t*>(smem);
   if (FM_TID_X == 0) bad = 0;
   fm_x3_dq<TIO, DH, SPLIT, X3Row<DH>>(A, st, &bad, FM_TID_X);
-  if (fm_x3_again(&bad)) fm_x3_dq<TIO, DH, SPLIT, F32Row<DH>>(FM_ARGS_AGAIN(A), st, &bad, FM_TID_X + FM_OPAQUE_ZERO());
+  if (!fm_x3_again(&bad)) FM_END();
+  fm_x3_dq<TIO, DH, SPLIT, F32Row<DH>>(FM_ARGS_AGAIN(A), st, &bad, FM_TID_X + FM_OPAQUE_ZERO());
 }
 
 // ------------------------------------------------------------------------------
@@ -709,5 +711,6 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(512, 2) k_x3_dkv(X3Args<TIO> A) {
   uint16_t* st = reinterpret_cast<uint16_t*>(smem);
   if (FM_TID_X == 0) bad = 0;
   fm_x3_dkv<TIO, DH, SPLIT, X3Row<DH>>(A, st, &bad, FM_TID_X);
-  if (fm_x3_again(&bad)) fm_x3_dkv<TIO, DH, SPLIT, F32Row<DH>>(FM_ARGS_AGAIN(A), st, &bad, FM_TID_X + FM_OPAQUE_ZERO());
+  if (!fm_x3_again(&bad)) FM_END();
+  fm_x3_dkv<TIO, DH, SPLIT, F32Row<DH>>(FM_ARGS_AGAIN(A), st, &bad, FM_TID_X + FM_OPAQUE_ZERO());
 }
