@@ -501,6 +501,7 @@ template <typename TIO> X3Args<TIO> x3_args(const FastmaxDesc* d, const Plan& p,
   a.cv = nullptr; a.out_resid = nullptr; a.ores = nullptr; a.bpart = nullptr;
   a.nq = d->nq; a.nk = d->nk; a.npad_q = p.npad_q; a.causal = d->mask != 0;
   a.a0 = p.a0; a.a1 = p.a1; a.a2 = p.a2; a.sc = p.sc;
+  a.plain = fm_x3_coef_lost(p.a1, p.a2);
   a.q_fold = q_fold(d); a.k_fold = k_fold(d);
   return a;
 }

@@ -9,8 +9,11 @@
 // relative error of o, dq, dk, dv against 64-bit results: v_mfma_f32_32x32x2_f32 3.9e-7, 4.7e-7, 4.8e-7, 4.0e-7; here 3.6e-7,
 // 4.4e-7, 3.4e-7, 2.8e-7 (a sixth of the accumulator's roundings are fp32-sized, sixteen products to each).  Times at
 // B*H = 32: forward 711 -> 370 us, dQ 1040 -> 520, dK and dV 1760 (two launches) -> 780, and the copies of 80 us are gone.
-// The lowest plane of a number below 2^-110 (1e-33) lies under bf16's smallest normal number and is lost to the matrix
-// instruction's flush: such entries keep 16 bits (1e-36: 3e-5), and everything from 1e-34 up all 24.
+// The matrix instruction takes a bf16 number under 2^-126 for zero, which would cost a number below 2^-103 its lowest plane.
+// So every operand, the weights and score gradients among them, is multiplied by UP = 2^24 before it is split: every fp32
+// number, the subnormal ones included, then keeps all its bits.  The powers are taken out of the polynomials'
+// coefficients and of the sums, all exactly: results are what they are without, bit for bit, wherever those keep 24 bits.
+// At the other end an operand or a sum beyond 2^79 to 2^104 overflows; such workgroups work in fp32 (see fm_x3_look).
 //
 // Three kernels for problems without moment states: the forward, dQ (which first makes c = (dO / g) . o of its queries
 // and leaves it for the next), dK and dV in one pass.  All read the caller's tensors; rows are scaled and split into
@@ -80,6 +83,7 @@ FM_DEVICE fm_u16x8 fm_bf16_load_tr(const uint16_t* tile, int pitch, int tok0, in
 //   accum, accum2    acc (rows = features) += rows of a stream tile times a weight tile, one product and two
 template <int DH> struct X3Row {
   static constexpr int PQ = 3 * DH + 8;                // pitch of a staged row: three planes and 16 bytes of padding
+  static constexpr float UP = 0x1p24f;                 // factor on every operand
   static constexpr bool PIPE = true;                   // the next stage is loaded while one is multiplied
   static constexpr int CH = 8, NOWN = DH / 16, NT = DH / 32;
   struct Own { X3 f[NOWN]; };
@@ -167,6 +171,7 @@ template <int DH> struct F32Row {
   static constexpr int PQ = X3Row<DH>::PQ;             // the tiles lie where the planes lay
   static constexpr int PF = DH + 1;                    // a row in floats
   static_assert(2 * PF <= PQ, "a row of floats fits a row of planes");
+  static constexpr float UP = 1.0f;
   static constexpr bool PIPE = false;                  // few registers: this code shares the allocation of the one above
   static constexpr int CH = 1, NOWN = DH / 2, NT = DH / 32;
   struct Own { float f[NOWN]; };
@@ -220,8 +225,8 @@ template <int DH> struct F32Row {
   }
 };
 
-// Three planes hold every finite number below 3.3953e38 (what bf16's largest number rounds down from); an infinity, a NaN
-// or a number above comes out of the split as infinity and NaN, and whatever sum it enters as NaN.  So a thread looks at the
+// An infinity, a NaN or a number that UP takes beyond bf16's largest comes out of the split as infinity and NaN, and
+// whatever sum it enters as NaN.  So a thread looks at the
 // sums it stores and, if one of the workgroup's is not finite, the workgroup makes its rows again with fp32 matrix products,
 // over what it stored: an infinite value then gives the infinities and NaN that fp32 arithmetic gives.  bad: one flag in
 // LDS, cleared at the kernel's start.  (A call of 8 us is bound by the length of its straight code: eight additions per
@@ -234,6 +239,19 @@ FM_DEVICE void fm_x3_look(int* bad, const float v[8], float g) {
 }
 FM_DEVICE bool fm_x3_again(const int* bad) { FM_SYNC_LDS(); return __builtin_expect(FM_UNIFORM(*bad) != 0, 0); }
 
+// The polynomials' coefficients where the score carries UP^2 and the result is to carry UP.
+struct X3Coef { float a0, a1, a2; };                   // f(s) = a0 + s (a1 + a2 s)
+template <typename R> FM_DEVICE X3Coef fm_x3_coef(float a0, float a1, float a2) {
+  const X3Coef c = {a0 * R::UP, a1 / R::UP, a2 / (R::UP * R::UP * R::UP)};
+  return c;
+}
+// A coefficient that this would take under fp32's normal numbers: fp32 matrix products from the start (X3Args::plain).
+inline bool fm_x3_coef_lost(float a1, float a2) {
+  typedef X3Row<64> R;
+  const float least = 0x1p-126f, b1 = (a1 < 0 ? -a1 : a1) / R::UP, b2 = (a2 < 0 ? -a2 : a2) / (R::UP * R::UP * R::UP);
+  return (a1 != 0.0f && b1 < least) || (a2 != 0.0f && b2 < least);
+}
+
 template <typename TIO> struct X3Args {
   TRef<const TIO> q, k, v, o, d_o;
   TRef<float> g;                        // written by the forward, read by the backward
@@ -242,6 +260,7 @@ template <typename TIO> struct X3Args {
   fm_half* out_resid; const fm_half* ores;   // bf16 tensors computed in fp32: what rounding takes from o (see TokArgs)
   int nq, nk, npad_q, causal;
   float a0, a1, a2, sc;                 // sc = sqrt(1/tau), on q and on k
+  int plain;                            // see fm_x3_coef_lost
   NormFold q_fold, k_fold;
   float* bpart;                         // the Jacobian's partial sums (see TokArgs::bpart), or null
 };
@@ -276,7 +295,7 @@ template <typename TIO, int DH, typename R, int ROWS, int NTH> struct X3Stage {
       if (TOT % NTH != 0 && c >= TOT) break;
       const bool second = c >= PER;
       const int cc = second ? c - PER : c;
-      const float f = second ? (div ? 1.0f / gi[i] : 1.0f) : xs;
+      const float f = second ? (div ? R::UP / gi[i] : R::UP) : xs;   // (xs has the factor already)
       float w[8];
 #pragma unroll
       for (int j = 0; j < 8; ++j) w[j] = r[i][j] * f;
@@ -294,7 +313,7 @@ template <typename TIO, int DH, typename R, int ROWS, int NTH> struct X3Stage {
       if (row >= 0 && row < n) {
         const TRef<const TIO>& t = second ? y : x;
         IO<TIO>::ld8(t.base(bh) + int64_t(row) * t.s_n + col, t.vec != 0, w);
-        const float f = second ? (g ? 1.0f / g->base(bh)[int64_t(row) * g->s_n] : 1.0f) : xs;
+        const float f = second ? (g ? R::UP / g->base(bh)[int64_t(row) * g->s_n] : R::UP) : xs;
 #pragma unroll
         for (int j = 0; j < 8; ++j) w[j] *= f;
       }
@@ -368,7 +387,7 @@ FM_DEVICE void fm_x3_store(const fm_f32x16* acc, float* Os, int sub, int row, in
     fm_x3_sum8<DH, QW, SPLIT>(Os, r, col, v);
     if (R::PIPE) fm_x3_look(bad, v, 0.f);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] *= scale;
+    for (int i = 0; i < 8; ++i) v[i] = v[i] * (1.0f / (R::UP * R::UP)) * scale;
     if (bout) {
       float x[8];
       IO<TIO>::ld8(raw.base(bh) + int64_t(t0 + r) * raw.s_n + col, raw.vec != 0, x);
@@ -417,7 +436,8 @@ FM_DEVICE void fm_x3_fwd(const X3Args<TIO>& A, uint16_t* st, int* bad, const int
   int blk, bh;
   fm_x3_place(causal, blk, bh);
   const int t0 = blk * QW, lo = t0 + 32 * own;
-  const float qs = A.sc * fm_norm_factor(A.q_fold, bh, lane), ks_ = A.sc * fm_norm_factor(A.k_fold, bh, lane);
+  const float qs = A.sc * fm_norm_factor(A.q_fold, bh, lane) * R::UP, ks_ = A.sc * fm_norm_factor(A.k_fold, bh, lane) * R::UP;
+  const X3Coef cf = fm_x3_coef<R>(A.a0, A.a1, A.a2);
   const int send = causal && t0 + QW < A.nk ? t0 + QW : A.nk;
   typedef X3Stage<TIO, DH, R, KT, C::NTH> Stage;
   Stage sg;
@@ -458,7 +478,7 @@ FM_DEVICE void fm_x3_fwd(const X3Args<TIO>& A, uint16_t* st, int* bad, const int
       fm_f32x16 s = fm_zero16();
       R::score(X, 32 * sub + lr, lh, of, s);
 #pragma unroll
-      for (int e = 0; e < 16; ++e) s[e] = A.a0 + s[e] * (A.a1 + A.a2 * s[e]);
+      for (int e = 0; e < 16; ++e) s[e] = cf.a0 + s[e] * (cf.a1 + cf.a2 * s[e]);
       if (fm_tile_edge<FM_OWN_Q>(causal, ss0, lo, A.nk)) { FM_KEEP_BRANCH(); fm_x3_window<FM_OWN_Q>(s, causal, ss0, lo, lr, lh, A.nk); }
 #pragma unroll
       for (int e = 0; e < 16; ++e) gs += s[e];
@@ -487,9 +507,10 @@ FM_DEVICE void fm_x3_fwd(const X3Args<TIO>& A, uint16_t* st, int* bad, const int
 #pragma unroll
     for (int s = 0; s < SPLIT; ++s) gt += Gs[s * QW + r];
     if (R::PIPE) fm_x3_look(bad, v, gt);
+    gt *= 1.0f / R::UP;
     const float gi = 1.0f / gt;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] *= gi;
+    for (int i = 0; i < 8; ++i) v[i] = v[i] * (1.0f / (R::UP * R::UP)) * gi;
     IO<TIO>::st8(A.out.base(bh) + int64_t(qi) * A.out.s_n + col, A.out.vec != 0, v);
     if (A.out_resid) {
       float sv[8];
@@ -506,8 +527,10 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(256, (X3Cfg<DH, 4, SPLIT>::OCC)) k_x3_fwd(X3Arg
   FM_SHARED int bad;
   uint16_t* st = reinterpret_cast<uint16_t*>(smem);
   if (FM_TID_X == 0) bad = 0;
-  fm_x3_fwd<TIO, DH, SPLIT, X3Row<DH>>(A, st, &bad, FM_TID_X);
-  if (!fm_x3_again(&bad)) FM_END();
+  if (!A.plain) {
+    fm_x3_fwd<TIO, DH, SPLIT, X3Row<DH>>(A, st, &bad, FM_TID_X);
+    if (!fm_x3_again(&bad)) FM_END();
+  }
   fm_x3_fwd<TIO, DH, SPLIT, F32Row<DH>>(FM_ARGS_AGAIN(A), st, &bad, FM_TID_X + FM_OPAQUE_ZERO());
 }
 
@@ -524,7 +547,7 @@ FM_DEVICE void fm_x3_dq(const X3Args<TIO>& A, uint16_t* st, int* bad, const int 
   int blk, bh;
   fm_x3_place(causal, blk, bh);
   const int t0 = blk * QW, lo = t0 + 32 * own;
-  const float qf = fm_norm_factor(A.q_fold, bh, lane), qs = A.sc * qf, ks_ = A.sc * fm_norm_factor(A.k_fold, bh, lane);
+  const float qf = fm_norm_factor(A.q_fold, bh, lane), qs = A.sc * qf * R::UP, ks_ = A.sc * fm_norm_factor(A.k_fold, bh, lane) * R::UP;
   const int send = causal && t0 + QW < A.nk ? t0 + QW : A.nk;
   typedef X3Stage<TIO, DH, R, KT, C::NTH> Stage;
   Stage sg;
@@ -534,7 +557,7 @@ FM_DEVICE void fm_x3_dq(const X3Args<TIO>& A, uint16_t* st, int* bad, const int 
   {
     const bool in = lo + lr < A.nq;
     const int64_t row = in ? lo + lr : A.nq - 1;
-    const float ginv = in ? 1.0f / A.g.base(bh)[row * A.g.s_n] : 0.f;
+    const float ginv = in ? R::UP / A.g.base(bh)[row * A.g.s_n] : 0.f;
 #pragma unroll
     for (int c = 0; c < R::NOWN; ++c) {
       R::fence(c);
@@ -550,9 +573,10 @@ FM_DEVICE void fm_x3_dq(const X3Args<TIO>& A, uint16_t* st, int* bad, const int 
       R::set(of2, c, w);
     }
     cs += fm_shfl_xor(cs, 32);
-    if (sub == 0 && lh == 0 && in) A.cv[int64_t(bh) * A.npad_q + row] = cs;
+    if (sub == 0 && lh == 0 && in) A.cv[int64_t(bh) * A.npad_q + row] = cs * (1.0f / R::UP);
+    cs *= R::UP;                                       // as gh . v
   }
-  const float ta2 = 2.0f * A.a2;
+  const X3Coef cf = fm_x3_coef<R>(0.0f, A.a1, 2.0f * A.a2);
   fm_f32x16 acc[NT];
 #pragma unroll
   for (int ct = 0; ct < NT; ++ct) acc[ct] = fm_zero16();
@@ -574,7 +598,7 @@ FM_DEVICE void fm_x3_dq(const X3Args<TIO>& A, uint16_t* st, int* bad, const int 
       fm_f32x16 s = fm_zero16(), dp = fm_zero16();
       R::score2(X, Y, 32 * sub + lr, lh, of, of2, s, dp);
 #pragma unroll
-      for (int e = 0; e < 16; ++e) s[e] = (A.a1 + ta2 * s[e]) * (dp[e] - cs);
+      for (int e = 0; e < 16; ++e) s[e] = (cf.a1 + cf.a2 * s[e]) * (dp[e] - cs);
       if (fm_tile_edge<FM_OWN_Q>(causal, ss0, lo, A.nk)) { FM_KEEP_BRANCH(); fm_x3_window<FM_OWN_Q>(s, causal, ss0, lo, lr, lh, A.nk); }
       R::accum(acc, X, 32 * sub, s, lane);
     }
@@ -595,8 +619,10 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(256, (X3Cfg<DH, 4, SPLIT>::OCC)) k_x3_dq(X3Args
   FM_SHARED int bad;
   uint16_t* st = reinterpret_cast<uint16_t*>(smem);
   if (FM_TID_X == 0) bad = 0;
-  fm_x3_dq<TIO, DH, SPLIT, X3Row<DH>>(A, st, &bad, FM_TID_X);
-  if (!fm_x3_again(&bad)) FM_END();
+  if (!A.plain) {
+    fm_x3_dq<TIO, DH, SPLIT, X3Row<DH>>(A, st, &bad, FM_TID_X);
+    if (!fm_x3_again(&bad)) FM_END();
+  }
   fm_x3_dq<TIO, DH, SPLIT, F32Row<DH>>(FM_ARGS_AGAIN(A), st, &bad, FM_TID_X + FM_OPAQUE_ZERO());
 }
 
@@ -616,7 +642,7 @@ FM_DEVICE void fm_x3_dkv(const X3Args<TIO>& A, uint16_t* Vs, int* bad, const int
   int blk, bh;
   fm_x3_place(false, blk, bh);
   const int t0 = blk * QW, lo = t0 + 32 * own;
-  const float kf = fm_norm_factor(A.k_fold, bh, lane), ks_ = A.sc * kf, qs = A.sc * fm_norm_factor(A.q_fold, bh, lane);
+  const float kf = fm_norm_factor(A.k_fold, bh, lane), ks_ = A.sc * kf * R::UP, qs = A.sc * fm_norm_factor(A.q_fold, bh, lane) * R::UP;
   const int sbeg = causal ? t0 : 0, nst = (A.nq - sbeg + KT - 1) / KT;
   const int s_last = sbeg + (nst - 1) * KT;            // the stream is walked from its end: see k_ds
   typedef X3Stage<TIO, DH, R, KT, C::NTH> Stage;
@@ -631,13 +657,15 @@ FM_DEVICE void fm_x3_dkv(const X3Args<TIO>& A, uint16_t* Vs, int* bad, const int
   auto put = [&](int b) FM_ALWAYS_INLINE {
     uint16_t* X = st + b * C::STAGE;
     sg.store(X, X + KT * PQ, qs, true, tid);
-    if (tid < KT) cst[b * KT + tid] = creg;
+    if (tid < KT) cst[b * KT + tid] = creg * (R::UP * R::UP);
   };
   if (R::PIPE) fetch(s_last);
   for (int c = tid; c < QW * (DH / 8); c += C::NTH) {
     const int r = c / (DH / 8), col = (c % (DH / 8)) * 8, row = t0 + r;
     float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     if (row < A.nk) IO<TIO>::ld8(A.v.base(bh) + int64_t(row) * A.v.s_n + col, A.v.vec != 0, v);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] *= R::UP;
     R::put8(Vs, r, col, v);
   }
   typename R::Own of;
@@ -654,7 +682,7 @@ FM_DEVICE void fm_x3_dkv(const X3Args<TIO>& A, uint16_t* Vs, int* bad, const int
       R::set(of, c, v);
     }
   }
-  const float ta2 = 2.0f * A.a2;
+  const X3Coef cp = fm_x3_coef<R>(A.a0, A.a1, A.a2), cd = fm_x3_coef<R>(0.0f, A.a1, 2.0f * A.a2);
   fm_f32x16 acc[NT], av[NT];
 #pragma unroll
   for (int ct = 0; ct < NT; ++ct) { acc[ct] = fm_zero16(); av[ct] = fm_zero16(); }
@@ -683,8 +711,8 @@ FM_DEVICE void fm_x3_dkv(const X3Args<TIO>& A, uint16_t* Vs, int* bad, const int
         for (int i = 0; i < 4; ++i) {
           const int e = 4 * g4 + i;
           const float x = s[e];
-          dp[e] = (A.a1 + ta2 * x) * (dp[e] - c4[i]);
-          s[e] = A.a0 + x * (A.a1 + A.a2 * x);
+          dp[e] = (cd.a1 + cd.a2 * x) * (dp[e] - c4[i]);
+          s[e] = cp.a0 + x * (cp.a1 + cp.a2 * x);
         }
       }
       if (fm_tile_edge<FM_OWN_K>(causal, ss0, lo, A.nq)) {
@@ -710,7 +738,9 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(512, 2) k_x3_dkv(X3Args<TIO> A) {
   FM_SHARED int bad;
   uint16_t* st = reinterpret_cast<uint16_t*>(smem);
   if (FM_TID_X == 0) bad = 0;
-  fm_x3_dkv<TIO, DH, SPLIT, X3Row<DH>>(A, st, &bad, FM_TID_X);
-  if (!fm_x3_again(&bad)) FM_END();
+  if (!A.plain) {
+    fm_x3_dkv<TIO, DH, SPLIT, X3Row<DH>>(A, st, &bad, FM_TID_X);
+    if (!fm_x3_again(&bad)) FM_END();
+  }
   fm_x3_dkv<TIO, DH, SPLIT, F32Row<DH>>(FM_ARGS_AGAIN(A), st, &bad, FM_TID_X + FM_OPAQUE_ZERO());
 }

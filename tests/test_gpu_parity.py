@@ -4,7 +4,7 @@ bf16-rounded inputs)."""
 import pytest
 import torch
 
-from tests.parity import (check_infinite_and_largest_values, check_batch_head_strides, check_decode, check_forward, check_forward_backward,
+from tests.parity import (check_infinite_and_largest_values, check_tiny_values, check_batch_head_strides, check_decode, check_forward, check_forward_backward,
                           check_norm_fold, make_inputs)
 from reproducing_fastmax_results_amd._capi import FLAG_F32_COMPUTE, FLAG_FORCE_DENSE, FLAG_FORCE_MOMENTS, FLAG_NORM_SELF
 
@@ -291,6 +291,16 @@ def test_infinite_and_largest_values_on_fp32_dense_tiles(lib, d, bh):
     """Own tiles shared by four, two and one wavefronts; a workgroup that meets such a value makes its rows again."""
     print(f"case infinite values d={d} bh={bh}", flush=True)
     check_infinite_and_largest_values(lib, bh, 70, d, torch.float32, DEV, seed=150)
+
+
+@pytest.mark.parametrize("d", [32, 64])
+@pytest.mark.parametrize("bh", [3, 256, 512])
+def test_tiny_values_on_fp32_dense_tiles(lib, d, bh):
+    """Numbers whose lower bf16 parts the matrix instruction would take for zero; and a coefficient under the range of the
+    scaled polynomial, where the kernels use fp32 products from the start.  The bar of test_fp32_dense_tiles."""
+    print(f"case tiny values d={d} bh={bh}", flush=True)
+    check_tiny_values(lib, bh, 70, d, torch.float32, DEV, tol=2e-6, seed=152)
+    check_forward_backward(lib, bh, 70, d, torch.float32, DEV, mask=True, p=2, a=(1.0, 1.0, 1e-20), seed=153)
 
 
 @pytest.mark.parametrize("dtype,flags", [(torch.float32, 0), (torch.bfloat16, 0), (torch.bfloat16, FLAG_F32_COMPUTE)])
