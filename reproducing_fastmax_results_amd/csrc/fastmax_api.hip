@@ -541,6 +541,7 @@ template <typename TIO> SmallArgs<TIO> small_args(const FastmaxDesc* d, const Pl
   a.out_resid = nullptr; a.ores = nullptr; a.npad_q = d->nq;
   a.nq = d->nq; a.nk = d->nk; a.causal = d->mask != 0;
   a.a0 = p.a0; a.a1 = p.a1; a.a2 = p.a2; a.sc = p.sc;
+  a.plain = !p.half && fm_x3_coef_lost(p.a1, p.a2);    // (two planes: no factor on the scores)
   const bool self = (d->flags & FASTMAX_FLAG_NORM_SELF) != 0;
   a.norm_q = self || d->norm.q_keys; a.norm_k = self || d->norm.k_keys; a.jac = d->norm.grad != 0; a.lim = d->norm.lim;
   return a;

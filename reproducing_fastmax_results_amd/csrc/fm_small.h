@@ -7,7 +7,8 @@
 // fp32 tensors: products of three bf16 planes (fm_x3.h).  bf16 tensors: the operands are the caller's numbers themselves (one
 // plane, exact), every factor (temperature, norms, 1 / g) is applied in fp32 to what the products give, and the weights
 // are split in two planes (16 bits; the general kernels' _Float16 weights have 11), or in three (FULL, all 24 bits) where
-// the caller asked for fp32 arithmetic or the weights may cancel; no range but fp32's applies here.  Wavefront (i, j) of the four works on the 32 x 32 tile of query tile i and key tile j; two sums per
+// the caller asked for fp32 arithmetic or the weights may cancel; no range but fp32's applies here.  As in fm_x3.h the operands
+// carry a power of two, so that the planes of the smallest numbers stay normal ones (dO always, the rest but for two planes).  Wavefront (i, j) of the four works on the 32 x 32 tile of query tile i and key tile j; two sums per
 // result meet in LDS.  The backward forms the scores twice, keys along the accumulator rows for dQ and queries along
 // them for dK and dV: each is then the operand of the product that follows, without a transposition.
 // B*H = 1024, 50 tokens, D = 32, normalised (26 MB forward, 53 MB backward): fp32 forward with its norms 23 -> 11.3 us, backward
@@ -26,6 +27,7 @@ template <typename TIO> struct SmallArgs {
   fm_half* out_resid; const fm_half* ores; int npad_q;   // see TokArgs
   int nq, nk, causal;
   float a0, a1, a2, sc;
+  int plain;                            // see fm_x3_coef_lost
   int norm_q, norm_k, jac; float lim;   // max-norm scaling of q / k; jac: gradients with respect to the raw tensors
 };
 
@@ -37,6 +39,8 @@ template <typename TIO, int DH, bool FULL> struct SmallCfg {
   static constexpr int PQ = PL * DH + 8, TILE = 64 * PQ, OP = DH + 4;
   static constexpr int PF = DH + 1;                    // PLAIN: pitch of a row of floats (fp32 tensors)
   static_assert(RAW || 2 * PF <= PQ, "a row of floats fits a row of planes");
+  // factors on q, k and v, on dO, and on the weights
+  static constexpr float UQ = FULL ? 0x1p24f : 1.0f, UG = 0x1p24f, UW = UQ;
   static constexpr size_t OS = size_t(2) * 64 * OP * 4;            // one result's two parts
   static constexpr size_t fwd_lds() { const size_t a = size_t(3) * TILE * 2, b = OS + 2 * 64 * 4; return a > b ? a : b; }
   static constexpr size_t bwd_lds() { const size_t a = size_t(4) * TILE * 2 + 2 * 64 * 4; return a > OS ? a : OS; }
@@ -58,22 +62,25 @@ FM_DEVICE void fm_small_load(const TRef<const TIO>& t, int bh, int n, int tid, f
 // PLAIN, here and below: the second pass of a workgroup whose sums came out non-finite (the lower planes of a weight are
 // zero or of either sign, so an infinite factor makes NaN or the other infinity of them; and see fm_x3_look): rows as
 // floats (bf16 tensors: their own rows) and sums on the vector units, term by term, over the keys a query sees.
-template <typename TIO, int DH, bool FULL, bool PLAIN> FM_DEVICE void fm_small_stage(uint16_t* tile, const float (*r)[8], const float* f, int tid) {
+template <typename TIO, int DH, bool FULL, bool PLAIN> FM_DEVICE void fm_small_stage(uint16_t* tile, const float (*r)[8], const float* f, float up, int tid) {
   typedef SmallCfg<TIO, DH, FULL> C;
 #pragma unroll
   for (int i = 0; i < DH / 32; ++i) {
     const int c = tid + 256 * i, row = c / (DH / 8), col = (c % (DH / 8)) * 8;
     uint16_t* p = tile + row * C::PQ + col;
     if constexpr (C::RAW) {
-      IO<fm_bf16>::st8(p, true, r[i]);                 // exact: they came from bf16
+      float w[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) w[j] = r[i][j] * up;
+      IO<fm_bf16>::st8(p, true, w);                    // exact: they came from bf16
     } else if constexpr (PLAIN) {
       float* q = reinterpret_cast<float*>(tile) + row * C::PF + col;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) q[j] = r[i][j] * f[i];
+      for (int j = 0; j < 8; ++j) q[j] = r[i][j] * (f[i] * up);
     } else {
       float w[8];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) w[j] = r[i][j] * f[i];
+      for (int j = 0; j < 8; ++j) w[j] = r[i][j] * (f[i] * up);
       X3Row<DH>::store(p, fm_x3_split(w));
     }
   }
@@ -162,11 +169,13 @@ template <typename TIO, int DH, bool FULL, bool PLAIN>
 FM_DEVICE void fm_small_fwd(const SmallArgs<TIO>& A, unsigned char* smem, unsigned long long (*keys)[4], int* bad, const int tid) {
   typedef SmallCfg<TIO, DH, FULL> C;
   constexpr int NT = DH / 32, N = C::N;
+  constexpr float UQ = PLAIN ? 1.0f : C::UQ, UW = PLAIN ? 1.0f : C::UW;
   uint16_t* Q = reinterpret_cast<uint16_t*>(smem);
   uint16_t* K = Q + C::TILE;
   uint16_t* V = K + C::TILE;
   const int lane = tid & 63, lr = lane & 31, lh = lane >> 5, bh = FM_BID_Y;
   const int wave = FM_UNIFORM(tid >> 6), ti = wave >> 1, tj = wave & 1, off = A.nk - A.nq;
+  const float a0 = A.a0 * UW, a1 = A.a1 * (UW / (UQ * UQ)), a2 = A.a2 * (UW / (UQ * UQ * UQ * UQ));   // on scores that carry UQ^2
   float rq[N][8], rk[N][8], rv[N][8];
   fm_small_load<TIO, DH>(A.q, bh, A.nq, tid, rq);
   fm_small_load<TIO, DH>(A.k, bh, A.nk, tid, rk);
@@ -181,9 +190,9 @@ FM_DEVICE void fm_small_fwd(const SmallArgs<TIO>& A, unsigned char* smem, unsign
     fk *= fm_small_factor(keys[1], A.norm_k != 0, A.lim, m2, ns);
   }
   const float sq[2] = {fq, fq}, sk[2] = {fk, fk}, one[2] = {1.0f, 1.0f};
-  fm_small_stage<TIO, DH, FULL, PLAIN>(Q, rq, sq, tid);
-  fm_small_stage<TIO, DH, FULL, PLAIN>(K, rk, sk, tid);
-  fm_small_stage<TIO, DH, FULL, PLAIN>(V, rv, one, tid);
+  fm_small_stage<TIO, DH, FULL, PLAIN>(Q, rq, sq, UQ, tid);
+  fm_small_stage<TIO, DH, FULL, PLAIN>(K, rk, sk, UQ, tid);
+  fm_small_stage<TIO, DH, FULL, PLAIN>(V, rv, one, UQ, tid);
   FM_SYNC();
   const float ss = C::RAW ? fq * fk : 1.0f;
   float* Os = reinterpret_cast<float*>(smem);
@@ -199,7 +208,7 @@ FM_DEVICE void fm_small_fwd(const SmallArgs<TIO>& A, unsigned char* smem, unsign
       if (A.causal) { const int l = 32 * ti + lr + off - 32 * tj; last = l < last ? l : last; }
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
-        const float x = C::RAW ? s[e] * ss : s[e], p = A.a0 + x * (A.a1 + A.a2 * x);
+        const float x = C::RAW ? s[e] * ss : s[e], p = a0 + x * (a1 + a2 * x);
         s[e] = fm_acc_row(e, lh) <= last ? p : 0.f;
         gs += s[e];
       }
@@ -222,7 +231,7 @@ FM_DEVICE void fm_small_fwd(const SmallArgs<TIO>& A, unsigned char* smem, unsign
       const int ke = A.causal && row + off + 1 < A.nk ? row + off + 1 : A.nk;
 #pragma unroll 1
       for (int t = 0; t < ke; ++t) {
-        const float x = fm_small_dot<TIO, DH, FULL>(Q, row, K, t) * ss, p = A.a0 + x * (A.a1 + A.a2 * x);
+        const float x = fm_small_dot<TIO, DH, FULL>(Q, row, K, t) * ss, p = a0 + x * (a1 + a2 * x);
         gt += p;
         fm_small_add8<TIO, DH, FULL>(v, p, V, t, col);
       }
@@ -231,9 +240,10 @@ FM_DEVICE void fm_small_fwd(const SmallArgs<TIO>& A, unsigned char* smem, unsign
       gt = Gs[row] + Gs[64 + row];
       fm_x3_look(bad, v, gt);
     }
+    gt *= 1.0f / UW;
     const float gi = 1.0f / gt;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] *= gi;
+    for (int j = 0; j < 8; ++j) v[j] = v[j] * (1.0f / (UW * UQ)) * gi;
     IO<TIO>::st8(A.out.base(bh) + int64_t(row) * A.out.s_n + col, A.out.vec != 0, v);
     if (A.out_resid) {
       float sv[8];
@@ -251,21 +261,23 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(256, 2) k_small_fwd(SmallArgs<TIO> A) {
   FM_SHARED unsigned long long keys[2][4];
   FM_SHARED int bad;
   if (FM_TID_X == 0) bad = 0;
-  fm_small_fwd<TIO, DH, FULL, false>(A, smem, keys, &bad, FM_TID_X);
-  if (!fm_x3_again(&bad)) FM_END();
+  if (!A.plain) {
+    fm_small_fwd<TIO, DH, FULL, false>(A, smem, keys, &bad, FM_TID_X);
+    if (!fm_x3_again(&bad)) FM_END();
+  }
   fm_small_fwd<TIO, DH, FULL, true>(FM_ARGS_AGAIN(A), smem, keys, &bad, FM_TID_X + FM_OPAQUE_ZERO());
 }
 
-// one result's rows: the two parts summed and scaled; returns the thread's share of sum value * raw
+// one result's rows: the two parts summed, multiplied by down and by scale; returns the thread's share of sum value * raw
 // (Os null: the sums are in v)
-template <int DH> FM_DEVICE float fm_small_result(const float* Os, float scale, const float (*raw)[8], int tid, float (*v)[8]) {
+template <int DH> FM_DEVICE float fm_small_result(const float* Os, float down, float scale, const float (*raw)[8], int tid, float (*v)[8]) {
   float b = 0.f;
 #pragma unroll
   for (int i = 0; i < DH / 32; ++i) {
     const int c = tid + 256 * i, row = c / (DH / 8), col = (c % (DH / 8)) * 8;
     if (Os) fm_x3_sum8<DH, 64, 2>(Os, row, col, v[i]);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) { v[i][j] *= scale; b += v[i][j] * raw[i][j]; }
+    for (int j = 0; j < 8; ++j) { v[i][j] = v[i][j] * down * scale; b += v[i][j] * raw[i][j]; }
   }
   return b;
 }
@@ -290,6 +302,8 @@ FM_DEVICE void fm_small_bwd(const SmallArgs<TIO>& A, unsigned char* smem, unsign
                             const int tid) {
   typedef SmallCfg<TIO, DH, FULL> C;
   constexpr int NT = DH / 32, N = C::N;
+  constexpr float UQ = PLAIN ? 1.0f : C::UQ, UW = PLAIN ? 1.0f : C::UW;
+  float ug = C::UG, down = 1.0f;                       // factor on dO; what takes it out again
   uint16_t* Q = reinterpret_cast<uint16_t*>(smem);
   uint16_t* K = Q + C::TILE;
   uint16_t* V = K + C::TILE;
@@ -318,6 +332,30 @@ FM_DEVICE void fm_small_bwd(const SmallArgs<TIO>& A, unsigned char* smem, unsign
         for (int j = 0; j < 8; ++j) ro[i][j] += float(rs[j]);
       }
     }
+    if constexpr (PLAIN) {
+      // dO of any size: its largest finite entry between 1 and 2 (a sum of products with dO itself may overflow else)
+      float m = 0.f;
+#pragma unroll
+      for (int i = 0; i < N; ++i)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) { const float x = fm_absf(rd[i][j]); m = x < 0x1p127f * 1.9999999f && x > m ? x : m; }
+#pragma unroll
+      for (int w = 1; w < 64; w <<= 1) m = fm_fmaxf(m, fm_shfl_xor(m, w));
+      if (lane == 0) bsum[0][wave] = m;
+      FM_SYNC();
+      m = fm_fmaxf(fm_fmaxf(bsum[0][0], bsum[0][1]), fm_fmaxf(bsum[0][2], bsum[0][3]));
+      uint32_t e;
+      __builtin_memcpy(&e, &m, 4);
+      e >>= 23;
+      e = e < 1 ? 1 : e > 253 ? 253 : e;
+      ug = fm_bits_f32((254 - e) << 23);
+      down = fm_bits_f32(e << 23);
+      FM_SYNC();
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) rd[i][j] *= ug;
     if (A.norm_q | A.norm_k) {
       const unsigned long long a = fm_small_norm_key<DH>(rq, A.nq, tid), b = fm_small_norm_key<DH>(rk, A.nk, tid);
       if (lane == 0) { keys[0][wave] = a; keys[1][wave] = b; }
@@ -326,22 +364,25 @@ FM_DEVICE void fm_small_bwd(const SmallArgs<TIO>& A, unsigned char* smem, unsign
       fk = fm_small_factor(keys[1], A.norm_k != 0, A.lim, m2k, nsk);
     }
     const float sq[2] = {A.sc * fq, A.sc * fq}, sk[2] = {A.sc * fk, A.sc * fk}, one[2] = {1.0f, 1.0f};
-    fm_small_stage<TIO, DH, FULL, PLAIN>(Q, rq, sq, tid);
-    fm_small_stage<TIO, DH, FULL, PLAIN>(K, rk, sk, tid);
-    fm_small_stage<TIO, DH, FULL, PLAIN>(V, rv, one, tid);
-    fm_small_stage<TIO, DH, FULL, PLAIN>(G, rd, gi, tid);
+    fm_small_stage<TIO, DH, FULL, PLAIN>(Q, rq, sq, UQ, tid);
+    fm_small_stage<TIO, DH, FULL, PLAIN>(K, rk, sk, UQ, tid);
+    fm_small_stage<TIO, DH, FULL, PLAIN>(V, rv, one, UQ, tid);
+    fm_small_stage<TIO, DH, FULL, PLAIN>(G, rd, gi, 1.0f, tid);
 #pragma unroll
     for (int i = 0; i < N; ++i) {
       const int c = tid + 256 * i;
       float s = 0.f;
 #pragma unroll
       for (int j = 0; j < 8; ++j) s += rd[i][j] * ro[i][j];
-      s = fm_group_sum<DH / 8>(s * gi[i]);
+      s = fm_group_sum<DH / 8>(s * gi[i] * UQ);        // carries UQ UG, as dO . v
       if (c % (DH / 8) == 0) { cs[c / (DH / 8)] = s; gr[c / (DH / 8)] = gi[i]; }
     }
   }
   FM_SYNC();
-  const float ta2 = 2.0f * A.a2, ss = C::RAW ? A.sc * A.sc * fq * fk : 1.0f;
+  const float ss = C::RAW ? A.sc * A.sc * fq * fk : 1.0f;
+  // on scores that carry UQ^2; dS carries UG
+  const float d1 = A.a1 * (1.0f / UQ), d2 = 2.0f * A.a2 * (1.0f / (UQ * UQ * UQ));
+  const float a0 = A.a0 * UW, a1 = A.a1 * (UW / (UQ * UQ)), a2 = A.a2 * (UW / (UQ * UQ * UQ * UQ));
   const float scale_q = A.sc * (A.jac ? fq : 1.0f) * (C::RAW ? A.sc * fk : 1.0f), scale_k = A.sc * (A.jac ? fk : 1.0f) * (C::RAW ? A.sc * fq : 1.0f);
   float vq[N][8], vk[N][8], vv[N][8];
   float bq, bk;
@@ -355,18 +396,19 @@ FM_DEVICE void fm_small_bwd(const SmallArgs<TIO>& A, unsigned char* smem, unsign
 #pragma unroll 1
       for (int t = 0; t < ke; ++t) {
         const float x = fm_small_dot<TIO, DH, FULL>(Q, row, K, t) * ss, dp = fm_small_dot<TIO, DH, FULL>(G, row, V, t) * (C::RAW ? gr[row] : 1.0f);
-        fm_small_add8<TIO, DH, FULL>(vq[i], (A.a1 + ta2 * x) * (dp - cs[row]), K, t, col);
+        fm_small_add8<TIO, DH, FULL>(vq[i], (d1 + d2 * x) * (dp - cs[row]), K, t, col);
       }
       const int qb = A.causal && row > off ? row - off : 0;
 #pragma unroll 1
       for (int t = row < A.nk ? qb : A.nq; t < A.nq; ++t) {
         const float gi = C::RAW ? gr[t] : 1.0f, x = fm_small_dot<TIO, DH, FULL>(Q, t, K, row) * ss, dp = fm_small_dot<TIO, DH, FULL>(G, t, V, row) * gi;
-        fm_small_add8<TIO, DH, FULL>(vk[i], (A.a1 + ta2 * x) * (dp - cs[t]), Q, t, col);
-        fm_small_add8<TIO, DH, FULL>(vv[i], (A.a0 + x * (A.a1 + A.a2 * x)) * gi, G, t, col);
+        fm_small_add8<TIO, DH, FULL>(vk[i], (d1 + d2 * x) * (dp - cs[t]), Q, t, col);
+        fm_small_add8<TIO, DH, FULL>(vv[i], (a0 + x * (a1 + a2 * x)) * gi, G, t, col);
       }
     }
-    bq = fm_small_result<DH>(nullptr, scale_q, rq, tid, vq);
-    bk = fm_small_result<DH>(nullptr, scale_k, rk, tid, vk);
+    bq = fm_small_result<DH>(nullptr, scale_q, down, rq, tid, vq);
+    bk = fm_small_result<DH>(nullptr, scale_k, down, rk, tid, vk);
+    (void)fm_small_result<DH>(nullptr, 1.0f, down, rk, tid, vv);
   } else {
     fm_f32x16 aq[NT], ak[NT], av[NT];
 #pragma unroll
@@ -381,7 +423,7 @@ FM_DEVICE void fm_small_bwd(const SmallArgs<TIO>& A, unsigned char* smem, unsign
         const float c = cs[32 * ti + lr], gi = C::RAW ? gr[32 * ti + lr] : 1.0f;
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
-          const float ds = (A.a1 + ta2 * (s[e] * ss)) * (dp[e] * gi - c);
+          const float ds = (d1 + d2 * (s[e] * ss)) * (dp[e] * gi - c);
           s[e] = A.causal && fm_acc_row(e, lh) > lr + diag ? 0.f : ds;
         }
         fm_small_acc<TIO, DH, FULL>(aq, Kt, s, lane);
@@ -394,7 +436,7 @@ FM_DEVICE void fm_small_bwd(const SmallArgs<TIO>& A, unsigned char* smem, unsign
         for (int e = 0; e < 16; ++e) {
           const int r = fm_acc_row(e, lh);
           const float gi = C::RAW ? gr[32 * ti + r] : 1.0f, x = s[e] * ss;
-          const float ds = (A.a1 + ta2 * x) * (dp[e] * gi - cs[32 * ti + r]), p = (A.a0 + x * (A.a1 + A.a2 * x)) * gi;
+          const float ds = (d1 + d2 * x) * (dp[e] * gi - cs[32 * ti + r]), p = (a0 + x * (a1 + a2 * x)) * gi;
           const bool hid = A.causal && lr > r + diag;
           dp[e] = hid ? 0.f : ds;
           s[e] = hid ? 0.f : p;
@@ -408,16 +450,16 @@ FM_DEVICE void fm_small_bwd(const SmallArgs<TIO>& A, unsigned char* smem, unsign
     FM_SYNC();
     fm_x3_put<DH, 64>(aq, Os, tj, 32 * ti + lr, lh);
     FM_SYNC();
-    bq = fm_small_result<DH>(Os, scale_q, rq, tid, vq);
+    bq = fm_small_result<DH>(Os, 1.0f / (C::UG * UQ), scale_q, rq, tid, vq);
     FM_SYNC();
     fm_x3_put<DH, 64>(ak, Os, ti, 32 * tj + lr, lh);
     FM_SYNC();
-    bk = fm_small_result<DH>(Os, scale_k, rk, tid, vk);
+    bk = fm_small_result<DH>(Os, 1.0f / (C::UG * UQ), scale_k, rk, tid, vk);
     FM_SYNC();
     fm_x3_put<DH, 64>(av, Os, ti, 32 * tj + lr, lh);
     FM_SYNC();
     // a sum that is not finite makes its b that, whatever the row it is multiplied by
-    const float bv = fm_small_result<DH>(Os, 1.0f, rk, tid, vv);
+    const float bv = fm_small_result<DH>(Os, 1.0f / (C::UG * UW), 1.0f, rk, tid, vv);
     if (!(fm_absf(bq) + fm_absf(bk) + fm_absf(bv) < 0x1p127f)) *bad = 1;
   }
   float cq = 0.f, ck = 0.f;
@@ -441,7 +483,9 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(256, (DH == 64 ? (sizeof(TIO) == 4 ? 1 : 2) : (
   FM_SHARED float bsum[2][4];
   FM_SHARED int bad;
   if (FM_TID_X == 0) bad = 0;
-  fm_small_bwd<TIO, DH, FULL, false>(A, smem, keys, bsum, &bad, FM_TID_X);
-  if (!fm_x3_again(&bad)) FM_END();
+  if (!A.plain) {
+    fm_small_bwd<TIO, DH, FULL, false>(A, smem, keys, bsum, &bad, FM_TID_X);
+    if (!fm_x3_again(&bad)) FM_END();
+  }
   fm_small_bwd<TIO, DH, FULL, true>(FM_ARGS_AGAIN(A), smem, keys, bsum, &bad, FM_TID_X + FM_OPAQUE_ZERO());
 }

@@ -218,3 +218,18 @@ def check_tiny_values(lib, bh, n, d, dtype, device, *, tol, flags=0, seed=0):
         ref = oracle_all(q, k, v, go, mask=True, tau=tau, p=2)
         errs = {m: rel_err(a, b) for m, a, b in zip(("o", "g", "dq", "dk", "dv"), (o, g, *grads), ref)}
         assert max(errs.values()) < tol, f"tiny {'q k v dO'.split()[which]}: {errs}"
+
+
+def check_upstream_gradients_at_the_ends_of_the_range(lib, bh, n, d, device, *, flags=0, seed=0):
+    """bf16 tensors, dO near the smallest and the largest numbers of its type (gradients are linear in dO): dq and dv at the
+    bf16 bar.  Small q and large k keep the scores ordinary and dq far enough from the subnormal numbers."""
+    tau = 8.0 * math.sqrt(d)
+    for go_scale in (2e-37, 3e37):
+        q, k, v, go = make_inputs(bh, n, n, d, torch.float32, device, seed, go_scale=go_scale)
+        q, k, v, go = (t.bfloat16() for t in (0.02 * q, 50.0 * k, v, go))
+        kw = dict(mask=False, inv_tau=1.0 / tau, p=2, flags=flags)
+        o, g = lib.forward(q, k, v, **kw)
+        dq, _, dv = lib.backward(q, k, v, o, g, go, **kw)
+        ref = oracle_all(q, k, v, go, mask=False, tau=tau, p=2)
+        eq, ev = rel_err(dq, ref[2]), rel_err(dv, ref[4])
+        assert eq < TOL[torch.bfloat16] and ev < TOL[torch.bfloat16], f"dO x {go_scale:g}: dq {eq:.3e}, dv {ev:.3e}"

@@ -4,7 +4,7 @@ bf16-rounded inputs)."""
 import pytest
 import torch
 
-from tests.parity import (check_infinite_and_largest_values, check_tiny_values, check_batch_head_strides, check_decode, check_forward, check_forward_backward,
+from tests.parity import (check_infinite_and_largest_values, check_tiny_values, check_upstream_gradients_at_the_ends_of_the_range, check_batch_head_strides, check_decode, check_forward, check_forward_backward,
                           check_norm_fold, make_inputs)
 from reproducing_fastmax_results_amd._capi import FLAG_F32_COMPUTE, FLAG_FORCE_DENSE, FLAG_FORCE_MOMENTS, FLAG_NORM_SELF
 
@@ -301,6 +301,16 @@ def test_tiny_values_on_fp32_dense_tiles(lib, d, bh):
     print(f"case tiny values d={d} bh={bh}", flush=True)
     check_tiny_values(lib, bh, 70, d, torch.float32, DEV, tol=2e-6, seed=152)
     check_forward_backward(lib, bh, 70, d, torch.float32, DEV, mask=True, p=2, a=(1.0, 1.0, 1e-20), seed=153)
+
+
+@pytest.mark.parametrize("d", [32, 64])
+@pytest.mark.parametrize("n", [20, 50, 64])
+def test_tiny_values_in_short_sequences(lib, d, n):
+    print(f"case tiny values, short d={d} n={n}", flush=True)
+    check_tiny_values(lib, 5, n, d, torch.float32, DEV, tol=2e-6, seed=154)
+    for flags in (0, FLAG_F32_COMPUTE):
+        check_upstream_gradients_at_the_ends_of_the_range(lib, 5, n, d, DEV, flags=flags, seed=155)
+    check_forward_backward(lib, 5, n, d, torch.float32, DEV, mask=True, p=2, a=(1.0, 1.0, 1e-20), seed=156)
 
 
 @pytest.mark.parametrize("dtype,flags", [(torch.float32, 0), (torch.bfloat16, 0), (torch.bfloat16, FLAG_F32_COMPUTE)])

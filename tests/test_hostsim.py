@@ -16,7 +16,7 @@ import pytest
 import torch
 
 from reproducing_fastmax_results_amd import _capi
-from tests.parity import (TOL, check_infinite_and_largest_values, check_tiny_values, check_batch_head_strides, check_decode, check_norm_fold, check_forward, check_forward_backward, make_inputs, oracle_all,
+from tests.parity import (TOL, check_upstream_gradients_at_the_ends_of_the_range, check_infinite_and_largest_values, check_tiny_values, check_batch_head_strides, check_decode, check_norm_fold, check_forward, check_forward_backward, make_inputs, oracle_all,
                           rel_err)
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -357,3 +357,11 @@ def test_infinite_and_largest_values_in_short_sequences(sim):
     for dtype, flags in ((torch.float32, 0), (torch.bfloat16, 0), (torch.bfloat16, _capi.FLAG_F32_COMPUTE)):
         check_infinite_and_largest_values(sim, 1, 20, 32, dtype, "cpu", flags=flags, seed=63,
                                           largest=None if dtype == torch.float32 else (1e30,))
+
+
+def test_tiny_values_in_short_sequences(sim):
+    # the bars: fp32's; bf16 tensors the type's, with dO down to its smallest normal numbers and up to its largest
+    check_tiny_values(sim, 1, 20, 32, torch.float32, "cpu", tol=2e-6, seed=64)
+    for flags in (0, _capi.FLAG_F32_COMPUTE):
+        check_upstream_gradients_at_the_ends_of_the_range(sim, 1, 20, 32, "cpu", flags=flags, seed=65)
+    check_forward_backward(sim, 1, 20, 32, torch.float32, "cpu", mask=True, p=2, a=(1.0, 1.0, 1e-20), seed=66)
