@@ -85,7 +85,8 @@ template <typename TIO, int DH, bool FULL, bool PLAIN> FM_DEVICE void fm_small_s
     }
   }
 }
-// largest squared row norm of the thread's wavefront with its row, as in k_maxnorm_keys: the first row among equal norms
+// largest squared row norm of the thread's wavefront with its row, as in k_maxnorm_keys: the first row among equal norms,
+// a row whose norm is NaN left out
 template <int DH> FM_DEVICE unsigned long long fm_small_norm_key(const float (*r)[8], int n, int tid) {
   unsigned long long key = 0;
 #pragma unroll
@@ -97,7 +98,7 @@ template <int DH> FM_DEVICE unsigned long long fm_small_norm_key(const float (*r
     s = fm_group_sum<DH / 8>(s);
     uint32_t bits;
     __builtin_memcpy(&bits, &s, 4);
-    const unsigned long long k = row < n ? (static_cast<unsigned long long>(bits) << 32) | uint32_t(~row) : 0ull;
+    const unsigned long long k = row < n && s == s ? (static_cast<unsigned long long>(bits) << 32) | uint32_t(~row) : 0ull;
     key = k > key ? k : key;
   }
 #pragma unroll

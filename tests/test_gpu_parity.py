@@ -293,6 +293,25 @@ def test_infinite_and_largest_values_on_fp32_dense_tiles(lib, d, bh):
     check_infinite_and_largest_values(lib, bh, 70, d, torch.float32, DEV, seed=150)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n", [40, 64])
+def test_short_sequences_normalised_with_a_nan_row(lib, dtype, n):
+    """The norm leaves such a row out (as fastmax_maxnorm_stats does for long sequences): the others keep their results."""
+    q, k, v, _ = make_inputs(5, n, n, 64, dtype, DEV, seed=157)
+    kw = dict(mask=False, inv_tau=1.0, p=2, flags=FLAG_NORM_SELF, norm=(None, None, 1.5, True))
+    small = q.clone()
+    small[:, 3] = 0.0                                    # takes no part in the norm either
+    want = lib.forward(small, k, v, **kw)
+    q[:, 3] = float("nan")
+    got = lib.forward(q, k, v, **kw)
+    rest = [i for i in range(n) if i != 3]
+    # (a workgroup with a NaN among its sums makes its rows again in fp32)
+    tol = 2e-6 if dtype == torch.float32 else 4e-3       # fp32 sums in another order; stored as bf16
+    for a, b in zip(got, want):
+        assert float((a[:, rest].double() - b[:, rest].double()).norm() / b[:, rest].double().norm()) < tol
+    assert bool(torch.isnan(got[0][:, 3]).all())
+
+
 @pytest.mark.parametrize("d", [32, 64])
 @pytest.mark.parametrize("bh", [3, 256, 512])
 def test_tiny_values_on_fp32_dense_tiles(lib, d, bh):

@@ -365,3 +365,18 @@ def test_tiny_values_in_short_sequences(sim):
     for flags in (0, _capi.FLAG_F32_COMPUTE):
         check_upstream_gradients_at_the_ends_of_the_range(sim, 1, 20, 32, "cpu", flags=flags, seed=65)
     check_forward_backward(sim, 1, 20, 32, torch.float32, "cpu", mask=True, p=2, a=(1.0, 1.0, 1e-20), seed=66)
+
+
+def test_short_sequences_normalised_with_a_nan_row(sim):
+    """A row that is NaN takes no part in the norm, as in fastmax_maxnorm_stats: the other queries' results are those of the
+    largest norm among them (and not of a factor zero)."""
+    from oracle import fastmax_oracle as O
+    q, k, v, _ = make_inputs(1, 20, 20, 32, torch.float32, "cpu", seed=67)
+    q[0, 3] = float("nan")
+    rest = [i for i in range(20) if i != 3]
+    want = O.closed_form_forward(O.normalize_lim(q[:, rest].double(), 1.5), O.normalize_lim(k.double(), 1.5), v.double(), mask=False,
+                                 tau=1.0, p=2)
+    for flags, keys in ((0, sim.maxnorm_stats(q, k)), (_capi.FLAG_NORM_SELF, (None, None))):
+        o, g = sim.forward(q, k, v, mask=False, inv_tau=1.0, p=2, flags=flags, norm=(*keys, 1.5, True))
+        assert rel_err(o[:, rest], want[0]) < 2e-6 and rel_err(g[:, rest], want[1]) < 2e-6
+        assert bool(torch.isnan(o[:, 3]).all())
