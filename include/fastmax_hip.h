@@ -41,7 +41,8 @@ enum {
                                         forward_bytes grows accordingly */
   FASTMAX_FLAG_F32_COMPUTE = 8,      /* bf16 tensors: do all arithmetic in fp32 (matrix products included)
                                         instead of _Float16; for inputs outside the range stated below.
-                                        Many times slower; workspace sizes grow.  Ignored for fp32 tensors. */
+                                        A training step takes four to five times as long; workspace sizes differ.
+                                        Ignored for fp32 tensors. */
   FASTMAX_FLAG_NORM_SELF = 16        /* nq, nk <= 64 (and not causal with nk > nq): q and k are max-normalised with norm.lim and
                                         the kernels find the norms themselves; norm.q_keys and norm.k_keys are null */
 };
@@ -61,8 +62,9 @@ enum {
  * backward rescales dO / g per batch*head to the _Float16 range and back).  The 2e-2 accuracy of this
  * path also rests on weights f(s) that add up without cancelling, as the Taylor weights do (f > 0):
  * with a0 <= 0 the library computes bf16 tensors in fp32 on its own, as if the flag were set.
- * fp32 tensors: every magnitude of fp32, with the full 24 bits for entries of v and of dO / g above about 1e-34 (below, 16:
- * the dense tiles form fp32 products from three bf16 parts of each factor). */
+ * fp32 tensors: every magnitude of fp32, infinities and NaN included, with fp32's 24 bits throughout.  (Dense tiles form fp32
+ * products from three bf16 parts of each factor; a workgroup that meets a number the parts cannot hold, beyond about 1e31,
+ * makes its rows a second time with fp32 products.) */
 
 /* Where slice i of the batch*head axis, token t, feature f of a tensor lives:
  *   heads <= 1:  i * bh + t * n + f

@@ -119,6 +119,13 @@ inline bool is_small(const FastmaxDesc* d) {
   return d->nq <= FM_SMALL_TOKENS && d->nk <= FM_SMALL_TOKENS && d->d <= 64 && !(d->flags & FASTMAX_FLAG_FORCE_MOMENTS);
 }
 
+// _Float16 arithmetic: bf16 tensors (see make_plan)
+inline bool half_arithmetic(const FastmaxDesc* d) {
+  return d->dtype == FASTMAX_BF16 && !(d->flags & FASTMAX_FLAG_F32_COMPUTE) && d->a0 > 0.0f;
+}
+// Unmasked attention: one total of the moments costs less than products with every key.
+inline bool states_pay_unmasked(const FastmaxDesc* d) { return int64_t(d->nk) > int64_t(d->d) * d->d + d->d; }
+
 int validate(const FastmaxDesc* d) {
   if (!d) return FASTMAX_ERR_NULL;
   if (d->dtype != FASTMAX_F32 && d->dtype != FASTMAX_BF16) return FASTMAX_ERR_DTYPE;
@@ -164,7 +171,7 @@ int make_plan(const FastmaxDesc* d, Plan& p) {
   // _Float16 arithmetic serves weights that are positive sums: with a0 <= 0 the weights f(s) change sign
   // around s = 0, numerator and denominator cancel, and 11 bits per weight no longer bound the error of
   // their ratio; such problems are computed in fp32 like the ones that ask for it
-  p.half = d->dtype == FASTMAX_BF16 && !(d->flags & FASTMAX_FLAG_F32_COMPUTE) && d->a0 > 0.0f;
+  p.half = half_arithmetic(d);
   p.esz = p.half ? 2 : 4;
   p.npad_q = int(round_up(d->nq, 256));
   p.npad_k = int(round_up(d->nk, 256));
@@ -181,6 +188,8 @@ int make_plan(const FastmaxDesc* d, Plan& p) {
     // beyond; order 1 (one D x D state per segment): one segment up to 1024 tokens (0.150 against 0.159 ms
     // per step at B*H = 128; at 1536 tokens, B*H = 96: 0.209 against 0.190),
     // 256-token segments beyond.
+    // fp32 arithmetic keeps the same limits: they were not measured for it (its dense tiles, fm_x3.h, run at about a quarter
+    // of the _Float16 rate, its state kernels at fp32's).
     // Order 1 on _Float16: 128-token segments, so that the backward of a segment is one workgroup's work (k_o1_bwd).
     const int auto_L = p.quad ? (d->nq > 6144 ? 1024 : p.npad_q) : (d->nq > 1024 ? (p.half ? 128 : 256) : p.npad_q);
     int L = d->chunk > 0 ? (d->chunk >= d->nq ? p.npad_q : int(round_up(d->chunk, 256))) : auto_L;
@@ -193,7 +202,7 @@ int make_plan(const FastmaxDesc* d, Plan& p) {
     p.L = p.npad_k;
     p.nseg = 1;
     const bool force_m = (d->flags & FASTMAX_FLAG_FORCE_MOMENTS) != 0;
-    p.use_state = force_m || (!force_dense && int64_t(d->nk) > int64_t(d->d) * d->d + d->d);
+    p.use_state = force_m || (!force_dense && states_pay_unmasked(d));
     p.nslots = p.use_state ? 1 : 0;
   }
   p.tiny = is_small(d);
@@ -716,8 +725,9 @@ int add_rows(const FastmaxDesc* d, const SplitPlan& sp, const void* dqa, void* d
 // Forward only, and nothing is left for a backward: a forward that is to keep its workspace takes the general
 // route (causal problems with nk > nq keep nothing there either and come here).
 inline bool is_few(const FastmaxDesc* d) {
-  return fm_few_pays(d->bh, d->nq) && d->d <= 64 && !(d->nq > 16 && is_small(d)) && !(d->flags & FASTMAX_FLAG_NORM_SELF) && (is_split(d) || !(d->flags & FASTMAX_FLAG_SAVE_FOR_BACKWARD)) &&
-         !(d->flags & (FASTMAX_FLAG_FORCE_MOMENTS | FASTMAX_FLAG_FORCE_DENSE));
+  if (d->d > 64 || (d->flags & (FASTMAX_FLAG_NORM_SELF | FASTMAX_FLAG_FORCE_MOMENTS | FASTMAX_FLAG_FORCE_DENSE))) return false;
+  if (!is_split(d) && (d->flags & FASTMAX_FLAG_SAVE_FOR_BACKWARD)) return false;
+  return fm_few_pays(d->bh, d->nq, d->nk, d->d, half_arithmetic(d), is_small(d), is_split(d), !d->mask && states_pay_unmasked(d));
 }
 inline size_t few_bytes(const FastmaxDesc* d) {
   const int s = fm_few_splits(d->bh, d->nq, d->nk);

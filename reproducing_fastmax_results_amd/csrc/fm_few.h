@@ -12,25 +12,43 @@
 #pragma once
 #include "fm_kernels.h"
 
-// Queries the route takes.  Its work per key grows with the queries while the general route's does not until 128, but
-// the general route has one workgroup per batch*head.  bf16, D = 64, general route and this one, microseconds:
-//   B*H = 32, 4097 keys:    1 query 73.9, 11.5;   16 queries 74.1, 27.7
-//   B*H = 64, 16384 keys:   1 query 657, 43 (6.2 TB/s);   16 queries 657, 146
-//   B*H = 1024, 300 keys, D = 32:   1 query 51, 10;   16 queries 50, 46
-//   B*H = 8, 1024 keys:     64 queries 30, 14.7;     B*H = 16, 16384 keys:   64 queries 186, 139;   B*H = 32, 4097 keys:   74, 77
-// so sixteen queries everywhere, and up to 64 while there are few batch*heads.
-inline bool fm_few_pays(int bh, int nq) { return nq <= 16 || (nq <= 64 && bh * nq <= 1024); }
 static constexpr int FM_FEW_MAX_SPLITS = 64;
 // queries that share one pass over the keys: registers 16 per query
 inline int fm_few_group(int nq) { return nq >= 4 ? 4 : nq; }
-// Parts the keys of a batch*head are cut into: enough workgroups for four per CU, none with less than 64 keys, and
-// no more than one wavefront of the merge reads in one go.
+inline int fm_few_groups(int nq) { return (nq + fm_few_group(nq) - 1) / fm_few_group(nq); }
+// Queries the route takes.  Its work per key grows with the query groups while the general route's does not until 128
+// queries, but the general route has one workgroup per batch*head.  bf16, D = 64, general route and this one, microseconds:
+//   B*H = 32, 4097 keys:    1 query 73.9, 11.5;   16 queries 74.1, 27.7
+//   B*H = 64, 16384 keys:   1 query 657, 43 (6.2 TB/s);   16 queries 657, 146
+//   B*H = 8, 1024 keys:     64 queries 30, 14.7;     B*H = 16, 16384 keys:   64 queries 186, 139;   B*H = 32, 4097 keys:   74, 77
+// So up to 64 queries while there are few batch*heads, and otherwise, on _Float16 arithmetic (`half`), what pays on a full chip:
+// up to eight queries, and up to sixteen where the general route walks moment states or, under the mask, runs in two parts on
+// few keys.  Times there of this route over the general one's (whole calls, B*H = 128 .. 4096, 17 .. 16384 keys): 1 to 4 queries
+// 0.07 .. 0.9; 8 queries 0.15 .. 0.99; 16 queries on dense tiles 1.05 .. 1.5 (D = 32, B*H = 128: 0.83 .. 0.91, but 12 queries 0.92 .. 1.08), on states 0.26 .. 0.9,
+// under the mask 0.35 .. 1.0 up to 1024 groups or 300 keys and 1.1 .. 1.2 beyond, 12 queries 0.7 .. 0.96 up to 1024 keys and 1.09 at
+// 4096.  Up to 64 keys (`tiny`) the general route is fm_small.h, one launch: more than one group pays up to 1024 groups.
+// fp32 arithmetic takes the route up to sixteen queries everywhere.
+inline bool fm_few_pays(int bh, int nq, int nk, int d, bool half, bool tiny, bool split, bool states) {
+  if (nq > 16 || !half) return nq <= 16 || (nq <= 64 && !tiny && bh * nq <= 1024);
+  const int groups = fm_few_groups(nq);
+  if (groups == 1) return true;
+  if (tiny) return bh * groups <= 1024;
+  if (groups == 2) return true;
+  if (split) return bh * groups <= 1024 || nk <= (groups == 3 ? 2048 : 512);
+  return states || bh * nq <= (d == 32 && groups == 4 ? 2048 : 1024);
+}
+// Parts the keys of a batch*head are cut into: enough workgroups for four per CU, about 64 keys or more in each (a count is
+// rounded up: 577 keys may go in 16 parts of 37), and no more than one wavefront of the merge reads in one go.
 inline int fm_few_splits(int bh, int nq, int nk) {
-  const int g = fm_few_group(nq), groups = (nq + g - 1) / g;
+  const int groups = fm_few_groups(nq);
   int s = (1024 + bh * groups - 1) / (bh * groups);
   const int most = (nk + 63) / 64;
   if (s > most) s = most;
-  if (s > 8) s = (s + 7) / 8 * 8;                       // a multiple of the XCDs: see k_few's grid
+  // a power of two or a multiple of the eight XCDs: the groups that read the same keys then run behind one L2, or two (see
+  // k_few's grid; B*H = 64, 12 queries on 1024 keys, whole call: 6 parts 28.1 us, 8 parts 23.4); up to eight parts not at
+  // the price of shorter ones (300 keys: 5 parts 15.7 us, 8 parts 19.6)
+  const int even = s > 4 ? (s + 7) / 8 * 8 : s == 3 ? 4 : s;
+  if (s > 8 || even <= most) s = even;
   if (s > FM_FEW_MAX_SPLITS) s = FM_FEW_MAX_SPLITS;
   return s < 1 ? 1 : s;
 }
@@ -128,7 +146,8 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS(FM_THREADS) k_few(FewArgs<TIO> A, int nsplit) {
   }
 }
 
-// Sums the parts of one query in a fixed order and divides.  grid (nq, bh), 64 threads x (DH / 64 or fewer lanes busy).
+// Sums the parts of one query in a fixed order and divides.  grid (nq, bh), 256 threads: 256 / DH groups of
+// DH lanes, a lane one feature of every 256 / DH-th part.
 template <typename TIO, int DH>
 FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_few_merge(FewArgs<TIO> A, int nsplit) {
   constexpr int NG = 256 / DH;                         // groups of lanes, each sums every NG-th part

@@ -194,3 +194,32 @@ def test_normalize_backward_arguments(lib):
     nd.d, nd.centre = 64, 5
     assert lib.lib.fastmax_normalize_backward(C.byref(nd), one, one, one, one, None) == 3
 
+
+
+def forward_bytes(lib, bh, nq, nk, **kw):
+    d = base_desc()
+    d.bh, d.nq, d.nk = bh, nq, nk
+    for k, v in kw.items():
+        setattr(d, k, v)
+    f = C.c_size_t()
+    assert lib.lib.fastmax_workspace_bytes(C.byref(d), C.byref(f), None) == 0
+    return f.value
+
+
+def test_route_for_a_few_queries(lib):
+    """Where the route for a few queries pays (seen in the workspace it asks for: parts of 65 floats per query, or 256 bytes for
+    one part): up to eight queries everywhere; beyond, on a full chip, not on dense _Float16 tiles and not on many keys in two parts."""
+    def parts(bh, nq, nk, **kw):
+        per = bh * nq * 65 * 4
+        b = forward_bytes(lib, bh, nq, nk, **kw)
+        return 1 if b == 256 else b // per if b <= 64 * per and b - b // per * per < 256 else None
+
+    assert parts(1024, 8, 300, mask=0) == 1 and parts(64, 16, 1024, mask=0) == 4
+    for bh, nq, nk in ((128, 16, 1024), (1024, 16, 300), (512, 12, 1024)):
+        assert parts(bh, nq, nk, mask=0) is None, (bh, nq, nk)
+    assert parts(1024, 16, 5000, mask=0) == 1                            # the general route would walk moment states
+    assert parts(1024, 16, 300) == 1 and parts(512, 12, 1024) == 1       # under the mask: one launch for two parts and a merge
+    assert parts(512, 16, 1024) is None and parts(512, 12, 4096) is None
+    assert parts(1024, 16, 300, mask=0, dtype=_capi.F32) == 1
+    # part counts: powers of two or multiples of eight, unless the parts would fall short of 64 keys
+    assert parts(64, 12, 1024, mask=0) == 8 and parts(64, 12, 300, mask=0) == 5 and parts(32, 1, 4097) == 32
