@@ -9,30 +9,43 @@
 #include "fastmax_hip.h"
 static uint16_t bf16(float x) { uint32_t u; memcpy(&u, &x, 4); return uint16_t((u + 0x7fff + ((u >> 16) & 1)) >> 16); }
 static float frand() { return float(rand()) / RAND_MAX * 2.f - 1.f; }
-static int run(int bh, int n, int d, int p, int chunk, int dtype, int save) {
+// nk 0: as many keys as queries.  norm: q and k max-normalised by the kernels themselves, gradients of the raw tensors.
+// inf: an infinite value, which sends the dense fp32 kernels and the short sequences through their second pass.
+struct Opt { int nk = 0, mask = 1, flags = 0, norm = 0, inf = 0, backward = 1; };
+static int run(int bh, int n, int d, int p, int chunk, int dtype, int save, Opt x = Opt()) {
+  const int nk = x.nk ? x.nk : n;
   FastmaxDesc D; memset(&D, 0, sizeof D);
-  D.bh = bh; D.nq = D.nk = n; D.d = d; D.dtype = dtype; D.mask = 1; D.p = p; D.a0 = 1; D.a1 = 1; D.a2 = .5f;
-  D.inv_tau = 1.f / (2.f * std::sqrt(float(d))); D.chunk = chunk; D.flags = save ? FASTMAX_FLAG_SAVE_FOR_BACKWARD : 0;
-  FastmaxStrides s = {int64_t(n) * d, d, 0, 0};
-  D.sq = D.sk = D.sv = D.so = D.sdo = D.sdq = D.sdk = D.sdv = s;
+  D.bh = bh; D.nq = n; D.nk = nk; D.d = d; D.dtype = dtype; D.mask = x.mask; D.p = p; D.a0 = 1; D.a1 = 1; D.a2 = .5f;
+  D.inv_tau = 1.f / (2.f * std::sqrt(float(d))); D.chunk = chunk; D.flags = x.flags | (save ? FASTMAX_FLAG_SAVE_FOR_BACKWARD : 0);
+  if (x.norm) { D.flags |= FASTMAX_FLAG_NORM_SELF; D.norm.lim = 1.5f; D.norm.grad = 1; }
+  FastmaxStrides sq = {int64_t(n) * d, d, 0, 0}, sk = {int64_t(nk) * d, d, 0, 0};
+  D.sq = D.so = D.sdo = D.sdq = sq;
+  D.sk = D.sv = D.sdk = D.sdv = sk;
   D.sg.bh = n; D.sg.n = 1;
   size_t fb, bb; int st = fastmax_workspace_bytes(&D, &fb, &bb); if (st) return st;
-  const size_t esz = dtype == FASTMAX_BF16 ? 2 : 4, ne = size_t(bh) * n * d;
-  std::vector<char> q(ne * esz), k(ne * esz), v(ne * esz), go(ne * esz), o(ne * esz), dq(ne * esz), dk(ne * esz), dv(ne * esz);
+  const size_t esz = dtype == FASTMAX_BF16 ? 2 : 4, ne = size_t(bh) * n * d, nke = size_t(bh) * nk * d;
+  std::vector<char> q(ne * esz), k(nke * esz), v(nke * esz), go(ne * esz), o(ne * esz), dq(ne * esz), dk(nke * esz), dv(nke * esz);
   std::vector<float> g(size_t(bh) * n);
-  for (size_t i = 0; i < ne; ++i)
-    for (char* b : {q.data(), k.data(), v.data(), go.data()}) {
-      const float x = frand();
-      if (esz == 2) reinterpret_cast<uint16_t*>(b)[i] = bf16(x); else reinterpret_cast<float*>(b)[i] = x;
+  for (std::vector<char>* b : {&q, &k, &v, &go})
+    for (size_t i = 0; i < b->size() / esz; ++i) {
+      const float r = frand();
+      if (esz == 2) reinterpret_cast<uint16_t*>(b->data())[i] = bf16(r); else reinterpret_cast<float*>(b->data())[i] = r;
     }
+  if (x.inf) { if (esz == 2) reinterpret_cast<uint16_t*>(v.data())[3] = 0x7f80; else reinterpret_cast<float*>(v.data())[3] = INFINITY; }
+  // exactly the bytes the library names (a multiple of the alignment)
   void* fws = aligned_alloc(256, (fb + 255) / 256 * 256); void* bws = aligned_alloc(256, (bb + 255) / 256 * 256);
   st = fastmax_forward(&D, q.data(), k.data(), v.data(), o.data(), g.data(), fws, fb, nullptr);
-  if (!st) st = save ? fastmax_backward_saved(&D, q.data(), k.data(), v.data(), o.data(), g.data(), go.data(), dq.data(), dk.data(), dv.data(), fws, fb, bws, bb, nullptr)
+  if (!st && x.backward) st = save ? fastmax_backward_saved(&D, q.data(), k.data(), v.data(), o.data(), g.data(), go.data(), dq.data(), dk.data(), dv.data(), fws, fb, bws, bb, nullptr)
                      : fastmax_backward(&D, q.data(), k.data(), v.data(), o.data(), g.data(), go.data(), dq.data(), dk.data(), dv.data(), bws, bb, nullptr);
   free(fws); free(bws);
-  double sum = 0; for (float x : g) sum += x;
-  printf("bh=%d n=%d d=%d p=%d chunk=%d dtype=%d save=%d -> status %d, sum g %.3f\n", bh, n, d, p, chunk, dtype, save, st, sum);
+  double sum = 0; for (float y : g) sum += y;
+  printf("bh=%d n=%d nk=%d d=%d p=%d mask=%d chunk=%d dtype=%d save=%d flags=%d norm=%d inf=%d -> status %d, sum g %.3f\n", bh, n, nk, d, p,
+         x.mask, chunk, dtype, save, x.flags, x.norm, x.inf, st, sum);
+  fflush(stdout);
   return st;
+}
+static Opt opt(int nk, int mask, int flags = 0, int norm = 0, int inf = 0, int backward = 1) {
+  Opt x; x.nk = nk; x.mask = mask; x.flags = flags; x.norm = norm; x.inf = inf; x.backward = backward; return x;
 }
 // the two element-wise passes (key RPE, output noise) on a ragged shape, in place
 static int run_pointwise(int bh, int n, int d, int dtype) {
@@ -95,5 +108,27 @@ int main() {
   bad |= run(1, 200, 128, 2, 0, FASTMAX_BF16, 1);     // heads of 128: four accumulator tiles per feature axis
   bad |= run(1, 150, 128, 1, 0, FASTMAX_BF16, 0);
   bad |= run(1, 300, 32, 2, 256, FASTMAX_F32, 1);
+  // fp32 on dense tiles (fm_x3.h): square and not, saved and not, bf16 tensors computed in fp32, the second pass
+  bad |= run(1, 70, 64, 2, 0, FASTMAX_F32, 1);
+  bad |= run(1, 130, 32, 2, 0, FASTMAX_F32, 0);
+  bad |= run(1, 40, 64, 1, 0, FASTMAX_F32, 0, opt(75, 0));
+  bad |= run(1, 75, 32, 2, 0, FASTMAX_F32, 0, opt(40, 0));
+  bad |= run(1, 70, 64, 2, 0, FASTMAX_BF16, 1, opt(0, 1, FASTMAX_FLAG_F32_COMPUTE));
+  bad |= run(1, 70, 64, 2, 0, FASTMAX_F32, 1, opt(0, 1, 0, 0, 1));
+  bad |= run(1, 70, 32, 2, 0, FASTMAX_F32, 0, opt(0, 0, 0, 0, 1));
+  // at most 64 tokens (fm_small.h): normalised by the kernels, causal with more keys, fp32 arithmetic, the second pass
+  for (int dtype : {FASTMAX_F32, FASTMAX_BF16})
+    for (int n : {1, 33, 50, 64}) bad |= run(2, n, n == 50 ? 32 : 64, 2, 0, dtype, 1, opt(0, 0, 0, 1));
+  bad |= run(1, 17, 64, 2, 0, FASTMAX_F32, 0, opt(64, 1));
+  bad |= run(1, 17, 32, 2, 0, FASTMAX_BF16, 0, opt(64, 1));
+  bad |= run(1, 50, 64, 2, 0, FASTMAX_BF16, 1, opt(0, 1, FASTMAX_FLAG_F32_COMPUTE, 0, 1));
+  bad |= run(1, 33, 32, 2, 0, FASTMAX_BF16, 1, opt(0, 1, 0, 1, 1));
+  bad |= run(1, 33, 64, 2, 0, FASTMAX_F32, 0, opt(20, 0, 0, 1, 1));
+  // a few queries (fm_few.h): forward alone
+  for (int dtype : {FASTMAX_F32, FASTMAX_BF16}) {
+    bad |= run(2, 1, 64, 2, 0, dtype, 0, opt(65, 1, 0, 0, 0, 0));
+    bad |= run(1, 6, 32, 2, 0, dtype, 0, opt(577, 1, 0, 0, 0, 0));
+    bad |= run(1, 3, 64, 1, 0, dtype, 0, opt(30, 0, 0, 0, 0, 0));
+  }
   return bad;
 }

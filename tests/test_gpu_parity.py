@@ -271,18 +271,19 @@ def test_sequences_of_at_most_64_tokens(lib, dtype, d, nq, nk):
 
 
 @pytest.mark.parametrize("d", [32, 64])
-@pytest.mark.parametrize("bh,n", [(1, 1), (3, 31), (2, 129), (1, 1025), (256, 40), (600, 33)])
+@pytest.mark.parametrize("bh,n", [(1, 65), (3, 95), (2, 129), (1, 1025), (256, 70), (600, 65), (90, 520), (180, 520)])
 def test_fp32_dense_tiles(lib, d, bh, n):
-    """fp32 products as six bf16 ones (fm_x3.h): tile edges, own tiles shared by four, two and one wavefronts, more keys
-    than queries, bf16 tensors computed in fp32.  The bar is four times the 4.8e-7 measured at 4096 tokens against
+    """fp32 products as six bf16 ones (fm_x3.h): tile edges, more keys than queries, bf16 tensors computed in fp32 with what
+    rounding takes from o kept.  Own tiles are shared by four wavefronts below 256 workgroups (B*H times blocks of 128 own tokens,
+    of 256 for dK + dV), by two below 512 and by one from there: (256, 70) and (90, 520) two, (600, 65) and (180, 520) one, with one
+    stage and with several.  Up to 64 tokens run fm_small.h.  The bar is four times the 4.8e-7 measured at 4096 tokens against
     64-bit results with v_mfma_f32_32x32x2_f32: one fp32 rounding per product sum, whichever instruction forms it."""
     print(f"case fp32 dense d={d} bh={bh} n={n}", flush=True)
     f = torch.float32
     for e in (check_forward_backward(lib, bh, n, d, f, DEV, mask=True, p=2, seed=130, saved=True, flags=FLAG_FORCE_DENSE),
               check_forward_backward(lib, bh, n, d, f, DEV, mask=False, p=2, nk=n + 37, seed=131)):
-        assert n == 1 or max(e.values()) < 2e-6, e
-    check_forward_backward(lib, min(bh, 3), n, d, torch.bfloat16, DEV, mask=True, p=2, seed=132, saved=True,
-                           flags=FLAG_F32_COMPUTE)
+        assert max(e.values()) < 2e-6, e
+    check_forward_backward(lib, bh, n, d, torch.bfloat16, DEV, mask=True, p=2, seed=132, saved=True, flags=FLAG_F32_COMPUTE)
 
 
 @pytest.mark.parametrize("d", [32, 64])
@@ -348,7 +349,10 @@ def test_few_queries(lib, dtype, d, nq, nk):
     """The route for a few queries (fm_few.h): group remainders, one part and many parts of the keys, queries that do not
     see the last keys, unmasked with both normalisation folds."""
     print(f"case few queries dtype={dtype} d={d} nq={nq} nk={nk}", flush=True)
-    check_forward(lib, 3, nq, d, dtype, DEV, mask=True, p=2, nk=nk, seed=120)
+    eo, _ = check_forward(lib, 3, nq, d, dtype, DEV, mask=True, p=2, nk=nk, seed=120)
+    # fp32 arithmetic, rounded once to 8 bits: rounding errors of 2^-8 / sqrt(3) of the binade's start, 1.5e-3 to 1.7e-3 of the
+    # norm (measured the same for the 64-bit result rounded; two roundings measured 2.3e-3)
+    assert dtype == torch.float32 or eo < 2.1e-3
     check_forward(lib, 2, nq, d, dtype, DEV, mask=False, p=1, nk=nk, seed=121)
     if nk > 1:                                           # (a single key: dq and dk cancel to zero exactly)
         check_norm_fold(lib, 2, nq, d, dtype, DEV, mask=False, p=2, nk=nk, seed=122, saved=False)

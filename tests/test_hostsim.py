@@ -354,9 +354,8 @@ def test_tiny_values_on_fp32_dense_tiles(sim):
 
 
 def test_infinite_and_largest_values_in_short_sequences(sim):
-    for dtype, flags in ((torch.float32, 0), (torch.bfloat16, 0), (torch.bfloat16, _capi.FLAG_F32_COMPUTE)):
-        check_infinite_and_largest_values(sim, 1, 20, 32, dtype, "cpu", flags=flags, seed=63,
-                                          largest=None if dtype == torch.float32 else (1e30,))
+    for dtype, largest in ((torch.float32, None), (torch.bfloat16, (1e30,))):
+        check_infinite_and_largest_values(sim, 1, 20, 32, dtype, "cpu", seed=63, largest=largest)
 
 
 def test_tiny_values_in_short_sequences(sim):
