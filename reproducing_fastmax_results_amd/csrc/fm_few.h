@@ -24,9 +24,11 @@ inline int fm_few_groups(int nq) { return (nq + fm_few_group(nq) - 1) / fm_few_g
 // So up to 64 queries while there are few batch*heads, and otherwise, on _Float16 arithmetic (`half`), what pays on a full chip:
 // up to eight queries, and up to sixteen where the general route walks moment states or, under the mask, runs in two parts on
 // few keys.  Times there of this route over the general one's (whole calls, B*H = 128 .. 4096, 17 .. 16384 keys): 1 to 4 queries
-// 0.07 .. 0.9; 8 queries 0.15 .. 0.99; 16 queries on dense tiles 1.05 .. 1.5 (D = 32, B*H = 128: 0.83 .. 0.91, but 12 queries 0.92 .. 1.08), on states 0.26 .. 0.9,
-// under the mask 0.35 .. 1.0 up to 1024 groups or 300 keys and 1.1 .. 1.2 beyond, 12 queries 0.7 .. 0.96 up to 1024 keys and 1.09 at
-// 4096.  Up to 64 keys (`tiny`) the general route is fm_small.h, one launch: more than one group pays up to 1024 groups.
+// 0.07 .. 0.9; 8 queries 0.15 .. 0.99; 16 queries on dense tiles 1.05 .. 1.5 (D = 32, B*H = 128: 0.83 .. 0.91, 12 queries there
+// 0.92 .. 1.08), on states 0.26 .. 0.9, under the mask 0.35 .. 1.0 up to 1024 groups or 300 keys and 1.1 .. 1.2 beyond, 12 queries
+// 0.7 .. 0.96 up to 1024 keys and 1.09 at
+// 4096.  Up to 64 keys (`tiny`) the general route is fm_small.h, one launch: more than one group up to 1024 groups
+// (B*H = 4096, 16 queries on 17 keys, D = 32: 117 us here, 12 there).
 // fp32 arithmetic takes the route up to sixteen queries everywhere.
 inline bool fm_few_pays(int bh, int nq, int nk, int d, bool half, bool tiny, bool split, bool states) {
   if (nq > 16 || !half) return nq <= 16 || (nq <= 64 && !tiny && bh * nq <= 1024);
