@@ -63,8 +63,8 @@ enum {
  * path also rests on weights f(s) that add up without cancelling, as the Taylor weights do (f > 0):
  * with a0 <= 0 the library computes bf16 tensors in fp32 on its own, as if the flag were set.
  * fp32 tensors: every magnitude of fp32, infinities and NaN included, with fp32's 24 bits throughout.  (Dense tiles form fp32
- * products from three bf16 parts of each factor; a workgroup that meets a number the parts cannot hold, beyond about 1e31,
- * makes its rows a second time with fp32 products.) */
+ * products from three bf16 parts of each factor; a workgroup that meets an entry beyond about 1e31 or a sum beyond 1e23, which the
+ * parts cannot hold, makes its rows a second time with fp32 products.) */
 
 /* Where slice i of the batch*head axis, token t, feature f of a tensor lives:
  *   heads <= 1:  i * bh + t * n + f

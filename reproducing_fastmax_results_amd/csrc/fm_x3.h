@@ -2,7 +2,7 @@
 //
 // An fp32 number is the exact sum of three bfloat16 numbers, x = h + m + l: h is x rounded to 8 bits, m what is left
 // rounded to 8 bits, l the rest (24 significant bits in all, each remainder formed exactly in fp32; bf16 has fp32's
-// exponents, so nothing overflows).  A product of two such numbers is taken as
+// exponents).  A product of two such numbers is taken as
 //     h h + (h m + m h) + (m m + h l + l h),
 // six v_mfma_f32_32x32x16_bf16 with fp32 accumulation; the three products left out are below 2^-26 of |x y|, less than
 // the 2^-24 of one fp32 rounding, and the pipe's rate is 16 / 6 of the fp32 instruction's.  N = 4096, D = 64, causal,
@@ -13,7 +13,7 @@
 // So every operand, the weights and score gradients among them, is multiplied by UP = 2^24 before it is split: every fp32
 // number, the subnormal ones included, then keeps all its bits.  The powers are taken out of the polynomials'
 // coefficients and of the sums, all exactly: results are what they are without, bit for bit, wherever those keep 24 bits.
-// At the other end an operand or a sum beyond 2^79 to 2^104 overflows; such workgroups work in fp32 (see fm_x3_look).
+// At the other end an operand beyond 2^104 or a sum beyond 2^79 overflows; such workgroups work in fp32 (see fm_x3_look).
 //
 // Three kernels for problems without moment states: the forward, dQ (which first makes c = (dO / g) . o of its queries
 // and leaves it for the next), dK and dV in one pass.  All read the caller's tensors; rows are scaled and split into
@@ -346,7 +346,7 @@ template <int OWN> FM_DEVICE void fm_x3_window(fm_f32x16& p, bool causal, int s0
   for (int e = 0; e < 16; ++e) { const int r = fm_acc_row(e, lh); if (r < wlo || r > whi) p[e] = 0.f; }
 }
 
-// Accumulators of all wavefronts -> Os [SPLIT][QW][DH + 4], rows summed over the SPLIT parts by x3_sum8.
+// Accumulators of all wavefronts -> Os [SPLIT][QW][DH + 4], rows summed over the SPLIT parts by fm_x3_sum8.
 template <int DH, int QW>
 FM_DEVICE void fm_x3_put(const fm_f32x16* acc, float* Os, int sub, int row, int lh) {
   constexpr int OP = DH + 4;
