@@ -724,10 +724,12 @@ int add_rows(const FastmaxDesc* d, const SplitPlan& sp, const void* dqa, void* d
 // ---- a few queries against many keys (fm_few.h) ----------------------------------------------
 // Forward only, and nothing is left for a backward: a forward that is to keep its workspace takes the general
 // route (causal problems with nk > nq keep nothing there either and come here).
-inline bool is_few(const FastmaxDesc* d) {
+inline bool few_possible(const FastmaxDesc* d) {
   if (d->d > 64 || (d->flags & (FASTMAX_FLAG_NORM_SELF | FASTMAX_FLAG_FORCE_MOMENTS | FASTMAX_FLAG_FORCE_DENSE))) return false;
-  if (!is_split(d) && (d->flags & FASTMAX_FLAG_SAVE_FOR_BACKWARD)) return false;
-  return fm_few_pays(d->bh, d->nq, d->nk, d->d, half_arithmetic(d), is_small(d), is_split(d), !d->mask && states_pay_unmasked(d));
+  return is_split(d) || !(d->flags & FASTMAX_FLAG_SAVE_FOR_BACKWARD);
+}
+inline bool is_few(const FastmaxDesc* d) {
+  return few_possible(d) && fm_few_pays(d->bh, d->nq, d->nk, d->d, half_arithmetic(d), is_small(d), is_split(d), !d->mask && states_pay_unmasked(d));
 }
 inline size_t few_bytes(const FastmaxDesc* d) {
   const int s = fm_few_splits(d->bh, d->nq, d->nk);
@@ -884,11 +886,15 @@ int fastmax_forward_static(const FastmaxDesc* desc, const void* q, const void* k
   size_t need = 0;
   const int st = fastmax_workspace_bytes(desc, &need, nullptr);
   if (st) return st;
-  if (need > size_t(FASTMAX_STATIC_SCRATCH_BYTES)) return FASTMAX_ERR_TOO_LARGE;
+  // a few queries whose general route needs more than the buffer take theirs, which needs next to nothing
+  const bool few = need > size_t(FASTMAX_STATIC_SCRATCH_BYTES) && desc->nq <= 16 && few_possible(desc) &&
+                   few_bytes(desc) <= size_t(FASTMAX_STATIC_SCRATCH_BYTES);
+  if (need > size_t(FASTMAX_STATIC_SCRATCH_BYTES) && !few) return FASTMAX_ERR_TOO_LARGE;
   void* ws = nullptr;
   const int sa = fm_static_scratch(&ws);
   if (sa) return sa;
   // nothing in the scratch has to start at zero: every kernel of the forward writes what a later one reads
+  if (few) return forward_few(desc, q, k, v, o, g, ws, size_t(FASTMAX_STATIC_SCRATCH_BYTES), hip_stream);
   return fastmax_forward(desc, q, k, v, o, g, ws, size_t(FASTMAX_STATIC_SCRATCH_BYTES), hip_stream);
 }
 

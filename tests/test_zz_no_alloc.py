@@ -57,3 +57,20 @@ def test_static_scratch_limit(lib):
     o, g = torch.empty_like(q), torch.empty(16, 65536, device=DEV)
     with pytest.raises(_capi.FastmaxError, match="static buffer"):
         lib.forward_static(q, q, q, o, g, mask=True, inv_tau=0.1, p=2)
+
+
+def test_static_scratch_takes_a_few_queries_on_many_keys(lib):
+    """Sixteen queries of each of 1024 batch*heads: the general route, the faster one there, would need 134 MB; the static
+    buffer serves the call on the route for a few queries, with the same results up to one rounding to bf16 on each side
+    (2^-8 of the binade's start, rms 1.7e-3 of the norm, twice) and the general route's _Float16 weights."""
+    print("case no-alloc few queries", flush=True)
+    gen = torch.Generator().manual_seed(6)
+    q, k, v = (torch.randn(1024, n, 64, generator=gen).to(torch.bfloat16).to(DEV) for n in (16, 300, 300))
+    kw = dict(mask=False, inv_tau=1.0 / 64.0, p=2)
+    d = lib.make_desc(q, k, v, a0=1.0, a1=1.0, a2=0.5, **kw)
+    assert lib.workspace_bytes(d)[0] > _capi.STATIC_SCRATCH_BYTES
+    o1, g1 = lib.forward(q, k, v, **kw)
+    o2, g2 = torch.full_like(o1, float("nan")), torch.full_like(g1, float("nan"))
+    lib.forward_static(q, k, v, o2, g2, **kw)
+    assert float((o1.double() - o2.double()).norm() / o1.double().norm()) < 4e-3
+    assert float((g1.double() - g2.double()).norm() / g1.double().norm()) < 1e-3
