@@ -139,7 +139,8 @@ int fastmax_forward(const FastmaxDesc* desc, const void* q, const void* k, const
  * FASTMAX_STATIC_SCRATCH_BYTES that is part of the loaded library (one copy per GPU, held until the
  * process ends); the call allocates and frees nothing.  A problem whose forward_bytes
  * (fastmax_workspace_bytes) exceed that size is refused with FASTMAX_ERR_TOO_LARGE before anything is
- * launched.  All calls on one GPU share that GPU's buffer: calls that overlap in time on one GPU (two
+ * launched, unless it has at most 16 queries (nq) and takes the kernels for a few queries, which need no
+ * such workspace.  All calls on one GPU share that GPU's buffer: calls that overlap in time on one GPU (two
  * streams, two threads) race and give wrong results; calls on one stream are ordered and safe.  The
  * buffer keeps the last call's contents; nothing in it needs clearing between calls.
  * FASTMAX_FLAG_SAVE_FOR_BACKWARD is honoured (the saved data then lives in the static buffer, until the
