@@ -228,11 +228,7 @@ k_decode_absorb_mma(TRef<const TIO> k, TRef<const TIO> v, int n_new, float inv_t
 #pragma unroll
     for (int i = 0; i < NK; ++i) {
       const int c = tid + 256 * i, row = t0 + c / CPR, f0 = (c % CPR) * 8;
-      if (row < n_new) IO<TIO>::ld8(kb + int64_t(row) * k.s_n + f0, k.vec != 0, kreg[i]);
-      else {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) kreg[i][j] = 0.f;
-      }
+      fm_ld8_row<TIO>(kb, k.s_n, row, n_new, f0, kreg[i]);
     }
     if (tid < TT) {
 #pragma unroll

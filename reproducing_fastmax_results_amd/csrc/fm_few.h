@@ -81,7 +81,7 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS(FM_THREADS) k_few(FewArgs<TIO> A, int nsplit) {
 #pragma unroll
   for (int i = 0; i < NQ; ++i) {
     const int qi = q0 + i < A.nq ? q0 + i : A.nq - 1;
-    IO<TIO>::ld8(A.q.base(bh) + int64_t(qi) * A.q.s_n + d0, A.q.vec != 0, qv[i]);
+    IO<TIO>::ld8(A.q.base(bh) + int64_t(qi) * A.q.s_n + d0, qv[i]);
 #pragma unroll
     for (int j = 0; j < 8; ++j) { qv[i][j] *= sc; acc[i][j] = 0.f; }
     gs[i] = 0.f;
@@ -94,8 +94,8 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS(FM_THREADS) k_few(FewArgs<TIO> A, int nsplit) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int t = b + u * RPW + row, tc = t < ke ? t : ke - 1;
-      IO<TIO>::ld8(kp + int64_t(tc) * A.k.s_n, A.k.vec != 0, kx[u]);
-      IO<TIO>::ld8(vp + int64_t(tc) * A.v.s_n, A.v.vec != 0, vx[u]);
+      IO<TIO>::ld8(kp + int64_t(tc) * A.k.s_n, kx[u]);
+      IO<TIO>::ld8(vp + int64_t(tc) * A.v.s_n, vx[u]);
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {

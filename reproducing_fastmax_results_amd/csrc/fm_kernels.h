@@ -99,6 +99,15 @@ struct TileRegs {
   }
 };
 
+// Eight elements of row `row` of a caller tensor of n rows; a row outside it reads the nearest one and becomes zeros.  (A branch per
+// row would hold the load and its conversion, and every load would wait for the one before it.)
+template <typename TIO> FM_DEVICE void fm_ld8_row(const TIO* base, int64_t s_n, int row, int n, int col, float v[8]) {
+  const int rc = row < n ? row : n - 1;
+  IO<TIO>::ld8(base + int64_t(rc) * s_n + col, v);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) v[j] = row < n ? v[j] : 0.f;
+}
+
 // Rows of a caller tensor (interface type, strided, bounds-checked) -> LDS in the
 // compute type.  ROWS x DH elements, eight elements per chunk.
 template <typename TIO, typename E, int ROWS, int DH>
@@ -108,18 +117,14 @@ struct RowRegs {
   static constexpr int N = (TOTAL + FM_THREADS - 1) / FM_THREADS;
   float v[N][8];
   // base points at (token 0, feature 0) of this batch*head; rows row0..row0+ROWS-1
-  FM_DEVICE void load(const TIO* base, int64_t s_n, bool vec, int row0, int nrows, int tid) {
+  // (rows past the end read the last one and become zeros: no branch between the loads)
+  FM_DEVICE void load(const TIO* base, int64_t s_n, int row0, int nrows, int tid) {
 #pragma unroll
     for (int i = 0; i < N; ++i) {
       const int c = tid + FM_THREADS * i;
       if (TOTAL % FM_THREADS == 0 || c < TOTAL) {
         const int row = row0 + c / CPR, col = (c % CPR) * 8;
-        if (row < nrows) {
-          IO<TIO>::ld8(base + int64_t(row) * s_n + col, vec, v[i]);
-        } else {
-#pragma unroll
-          for (int j = 0; j < 8; ++j) v[i][j] = 0.f;
-        }
+        fm_ld8_row<TIO>(base, s_n, row, nrows, col, v[i]);
       }
     }
   }
@@ -232,16 +237,10 @@ k_transpose(TransposeJob<TIO, E> j0, TransposeJob<TIO, E> j1, int n, int npad) {
   const float scale = (second ? j1.scale : j0.scale) * fm_norm_factor(second ? j1.fold : j0.fold, bh, tid & 63);
   const TIO* xb = x.base(bh);
   const int64_t s_n = x.s_n;
-  const int vec = x.vec;
   for (int c = tid; c < 64 * (DH / 8); c += FM_THREADS) {
     const int tok = c / (DH / 8), d0 = (c % (DH / 8)) * 8;
     float v[8];
-    if (t0 + tok < n) {
-      IO<TIO>::ld8(xb + int64_t(t0 + tok) * s_n + d0, vec != 0, v);
-    } else {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) v[j] = 0.f;
-    }
+    fm_ld8_row<TIO>(xb, s_n, t0 + tok, n, d0, v);
 #pragma unroll
     for (int j = 0; j < 8; ++j) v[j] *= scale;
     if (xr) CE<E>::st8(xr + (int64_t(bh) * npad + t0 + tok) * DH + d0, v);
@@ -288,7 +287,7 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS(FM_THREADS) k_grad_scale(TRef<const TIO> d_o, TR
     const int tok = tok0 + 64 * p, tk = tok < n ? tok : n - 1;
     gi[p] = g.base(bh)[int64_t(tk) * g.s_n];
 #pragma unroll
-    for (int j = 0; j < EPT; j += 8) IO<TIO>::ld8(d_o.base(bh) + int64_t(tk) * d_o.s_n + d0 + j, d_o.vec != 0, &v[p][j]);
+    for (int j = 0; j < EPT; j += 8) IO<TIO>::ld8(d_o.base(bh) + int64_t(tk) * d_o.s_n + d0 + j, &v[p][j]);
   }
   float mx = 0.f;
 #pragma unroll
@@ -370,29 +369,34 @@ k_prep_bwd(TRef<const TIO> q, TRef<const TIO> o, TRef<const TIO> d_o, TRef<const
   const float qscale = qscale0 * fm_norm_factor(qfold, bh, tid & 63);
   float vg[EPT], vq[EPT];
   float csum = 0.f;
-  if (row < n) {
-    // every load of the thread is issued before the first result is used
+  {
+    // every load of the thread is issued before the first result is used (rows past the end read the last one and become zeros)
+    const bool in = row < n;
+    const int rc = in ? row : n - 1;
     float a[EPT], b[EPT], c[EPT];
     fm_half8 r[EPT / 8];
-    const float gi = g.base(bh)[int64_t(row) * g.s_n];
+    const float gi = g.base(bh)[int64_t(rc) * g.s_n];
+#pragma unroll
+    for (int j = 0; j < EPT / 8; ++j) r[j] = Mma<fm_half>::splat(fm_half(0.f));
+    if (ores) {
+#pragma unroll
+      for (int j = 0; j < EPT; j += 8) r[j / 8] = *reinterpret_cast<const fm_half8*>(ores + (int64_t(bh) * npad + rc) * DH + d0 + j);
+    }
 #pragma unroll
     for (int j = 0; j < EPT; j += 8) {
-      IO<TIO>::ld8(d_o.base(bh) + int64_t(row) * d_o.s_n + d0 + j, d_o.vec != 0, &a[j]);
-      IO<TIO>::ld8(o.base(bh) + int64_t(row) * o.s_n + d0 + j, o.vec != 0, &b[j]);
-      IO<TIO>::ld8(q.base(bh) + int64_t(row) * q.s_n + d0 + j, q.vec != 0, &c[j]);
-      r[j / 8] = ores ? *reinterpret_cast<const fm_half8*>(ores + (int64_t(bh) * npad + row) * DH + d0 + j)
-                      : Mma<fm_half>::splat(fm_half(0.f));
+      IO<TIO>::ld8(d_o.base(bh) + int64_t(rc) * d_o.s_n + d0 + j, &a[j]);
+      IO<TIO>::ld8(o.base(bh) + int64_t(rc) * o.s_n + d0 + j, &b[j]);
+      IO<TIO>::ld8(q.base(bh) + int64_t(rc) * q.s_n + d0 + j, &c[j]);
     }
     const float ginv = gscale / gi;
 #pragma unroll
     for (int j = 0; j < EPT; ++j) {
       vg[j] = a[j] * ginv;
       csum += vg[j] * (b[j] + float(r[j / 8][j % 8]));
-      vq[j] = c[j] * qscale;
+      vq[j] = in ? c[j] * qscale : 0.f;
+      vg[j] = in ? vg[j] : 0.f;
     }
-  } else {
-#pragma unroll
-    for (int j = 0; j < EPT; ++j) { vg[j] = 0.f; vq[j] = 0.f; }
+    csum = in ? csum : 0.f;
   }
   csum += fm_shfl_xor(csum, 1);
   csum += fm_shfl_xor(csum, 2);

@@ -93,61 +93,30 @@ FM_DEVICE fm_f32x16 fm_zero16() {
 }
 
 // ---- interface element types (what the caller's tensors hold) -----------------
+// ld8, st8: eight consecutive elements at any address an element may lie at.  The copies are of unaligned type, for which
+// gfx950 code has the 16-byte instructions too (the target runs with unaligned access); a test of the alignment ahead of
+// them would put every load in a branch of its own, with its conversion, so that each waits for the one before it.
 template <typename T> struct IO;
 template <> struct IO<float> {
   static FM_DEVICE float ld(const float* p) { return *p; }
   static FM_DEVICE void st(float* p, float v) { *p = v; }
-  // eight consecutive elements; `vec` says the address is 16-byte aligned
-  static FM_DEVICE void ld8(const float* p, bool vec, float out[8]) {
-    if (vec) {
-      const fm_f32x4 a = *reinterpret_cast<const fm_f32x4*>(p);
-      const fm_f32x4 b = *reinterpret_cast<const fm_f32x4*>(p + 4);
-      out[0] = a[0]; out[1] = a[1]; out[2] = a[2]; out[3] = a[3];
-      out[4] = b[0]; out[5] = b[1]; out[6] = b[2]; out[7] = b[3];
-    } else {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) out[i] = p[i];
-    }
-  }
-  static FM_DEVICE void st8(float* p, bool vec, const float in[8]) {
-    if (vec) {
-      fm_f32x4 a = {in[0], in[1], in[2], in[3]}, b = {in[4], in[5], in[6], in[7]};
-      *reinterpret_cast<fm_f32x4*>(p) = a;
-      *reinterpret_cast<fm_f32x4*>(p + 4) = b;
-    } else {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) p[i] = in[i];
-    }
-  }
+  static FM_DEVICE void ld8(const float* p, float out[8]) { __builtin_memcpy(out, p, 32); }
+  static FM_DEVICE void st8(float* p, const float in[8]) { __builtin_memcpy(p, in, 32); }
 };
 template <> struct IO<fm_bf16> {
   static FM_DEVICE float ld(const fm_bf16* p) { return fm_bf16_to_f32(*p); }
   static FM_DEVICE void st(fm_bf16* p, float v) { *p = fm_f32_to_bf16(v); }
-  static FM_DEVICE void ld8(const fm_bf16* p, bool vec, float out[8]) {
-    if (vec) {
-      const fm_u32x4 u = *reinterpret_cast<const fm_u32x4*>(p);
+  static FM_DEVICE void ld8(const fm_bf16* p, float out[8]) {
+    fm_u32x4 u;
+    __builtin_memcpy(&u, p, 16);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        uint32_t lo = u[i] << 16, hi = u[i] & 0xffff0000u;
-        __builtin_memcpy(&out[2 * i], &lo, 4);
-        __builtin_memcpy(&out[2 * i + 1], &hi, 4);
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) out[i] = fm_bf16_to_f32(p[i]);
-    }
+    for (int i = 0; i < 4; ++i) { out[2 * i] = fm_bits_f32(u[i] << 16); out[2 * i + 1] = fm_bits_f32(u[i] & 0xffff0000u); }
   }
-  static FM_DEVICE void st8(fm_bf16* p, bool vec, const float in[8]) {
-    if (vec) {
-      fm_u32x4 u;
+  static FM_DEVICE void st8(fm_bf16* p, const float in[8]) {
+    fm_u32x4 u;
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        u[i] = fm_cvt_pk_bf16(in[2 * i], in[2 * i + 1]);
-      *reinterpret_cast<fm_u32x4*>(p) = u;
-    } else {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) p[i] = fm_f32_to_bf16(in[i]);
-    }
+    for (int i = 0; i < 4; ++i) u[i] = fm_cvt_pk_bf16(in[2 * i], in[2 * i + 1]);
+    __builtin_memcpy(p, &u, 16);
   }
 };
 

@@ -32,9 +32,9 @@ inline int64_t fm_norm_stride(int dh, int n, int centre) {
 // A thread's quarter of one token row, and the centring of it (the feature mean needs the four
 // threads of the token: every lane of the wavefront must call fm_norm_centre).
 template <typename TIO, int DH>
-FM_DEVICE void fm_norm_load(const TIO* row, bool vec, int d0, float v[DH / 4]) {
+FM_DEVICE void fm_norm_load(const TIO* row, int d0, float v[DH / 4]) {
 #pragma unroll
-  for (int j = 0; j < DH / 4; j += 8) IO<TIO>::ld8(row + d0 + j, vec, &v[j]);
+  for (int j = 0; j < DH / 4; j += 8) IO<TIO>::ld8(row + d0 + j, &v[j]);
 }
 template <int DH>
 FM_DEVICE void fm_norm_centre(float v[DH / 4], int d0, int centre, const float* mean) {
@@ -54,8 +54,8 @@ FM_DEVICE void fm_norm_centre(float v[DH / 4], int d0, int centre, const float* 
   }
 }
 template <typename TIO, int DH>
-FM_DEVICE void fm_norm_load_centred(const TIO* row, bool vec, int d0, int centre, const float* mean, float v[DH / 4]) {
-  fm_norm_load<TIO, DH>(row, vec, d0, v);
+FM_DEVICE void fm_norm_load_centred(const TIO* row, int d0, int centre, const float* mean, float v[DH / 4]) {
+  fm_norm_load<TIO, DH>(row, d0, v);
   fm_norm_centre<DH>(v, d0, centre, mean);
 }
 
@@ -74,12 +74,8 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_norm_colsum(TRef<const TIO> x0, TRef<cons
 #pragma unroll
   for (int p = 0; p < NP; ++p) {
     const int tok = tok0 + 64 * p;
-    if (tok < n) {
-      fm_norm_load<TIO, DH>(x.base(bh) + int64_t(tok) * x.s_n, x.vec != 0, d0, v[p]);
-    } else {
 #pragma unroll
-      for (int j = 0; j < EPT; ++j) v[p][j] = 0.f;
-    }
+    for (int j = 0; j < EPT; j += 8) fm_ld8_row<TIO>(x.base(bh), x.s_n, tok, n, d0 + j, &v[p][j]);
   }
 #pragma unroll
   for (int j = 0; j < EPT; ++j) {
@@ -134,7 +130,7 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_norm_maxnorm(TRef<const TIO> x, int n, in
 #pragma unroll
   for (int p = 0; p < NP; ++p) {
     const int tok = tok0 + 64 * p, tk = tok < n ? tok : n - 1;
-    fm_norm_load<TIO, DH>(x.base(bh) + int64_t(tk) * x.s_n, x.vec != 0, d0, v[p]);
+    fm_norm_load<TIO, DH>(x.base(bh) + int64_t(tk) * x.s_n, d0, v[p]);
   }
   float mx = 0.f;
 #pragma unroll
@@ -165,7 +161,7 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_norm_apply(TRef<const TIO> x, TRef<TIO> y
 #pragma unroll
   for (int p = 0; p < NP; ++p) {
     const int tok = tok0 + 64 * p, tk = tok < n ? tok : n - 1;
-    fm_norm_load<TIO, DH>(x.base(bh) + int64_t(tk) * x.s_n, x.vec != 0, d0, v[p]);
+    fm_norm_load<TIO, DH>(x.base(bh) + int64_t(tk) * x.s_n, d0, v[p]);
   }
   float f = scale;
   if (max_norm) {
@@ -185,7 +181,7 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_norm_apply(TRef<const TIO> x, TRef<TIO> y
 #pragma unroll
       for (int j = 0; j < EPT; ++j) v[p][j] *= f;
 #pragma unroll
-      for (int j = 0; j < EPT; j += 8) IO<TIO>::st8(y.base(bh) + int64_t(tok) * y.s_n + d0 + j, y.vec != 0, &v[p][j]);
+      for (int j = 0; j < EPT; j += 8) IO<TIO>::st8(y.base(bh) + int64_t(tok) * y.s_n + d0 + j, &v[p][j]);
     }
   }
 }
@@ -261,8 +257,8 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_normb_stats(TRef<const TIO> x, TRef<const
 #pragma unroll
   for (int p = 0; p < NP; ++p) {
     const int tok = tok0 + 64 * p, tk = tok < n ? tok : n - 1;
-    fm_norm_load<TIO, DH>(x.base(bh) + int64_t(tk) * x.s_n, x.vec != 0, d0, c[p]);
-    fm_norm_load<TIO, DH>(dy.base(bh) + int64_t(tk) * dy.s_n, dy.vec != 0, d0, g[p]);
+    fm_norm_load<TIO, DH>(x.base(bh) + int64_t(tk) * x.s_n, d0, c[p]);
+    fm_norm_load<TIO, DH>(dy.base(bh) + int64_t(tk) * dy.s_n, d0, g[p]);
   }
   float mx = -1.0f;
   int cand = 0x7fffffff;
@@ -320,7 +316,7 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_normb_apply(TRef<const TIO> x, TRef<const
 #pragma unroll
   for (int p = 0; p < NP; ++p) {
     const int tok = tok0 + 64 * p, tk = tok < n ? tok : n - 1;
-    fm_norm_load<TIO, DH>(dy.base(bh) + int64_t(tk) * dy.s_n, dy.vec != 0, d0, g[p]);
+    fm_norm_load<TIO, DH>(dy.base(bh) + int64_t(tk) * dy.s_n, d0, g[p]);
   }
   float f = scale, kf = 0.f;
   int nstar = -1;
@@ -354,7 +350,7 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_normb_apply(TRef<const TIO> x, TRef<const
     f = some ? scale / fm_sqrtf(m2) : 0.0f;
     kf = some ? red[0] / m2 : 0.0f;
     // every lane takes part in the shuffles of the centring
-    fm_norm_load_centred<TIO, DH>(x.base(bh) + int64_t(nstar) * x.s_n, x.vec != 0, d0, centre, st + 4, cs);
+    fm_norm_load_centred<TIO, DH>(x.base(bh) + int64_t(nstar) * x.s_n, d0, centre, st + 4, cs);
   }
 #pragma unroll
   for (int p = 0; p < NP; ++p) {
@@ -369,7 +365,7 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_normb_apply(TRef<const TIO> x, TRef<const
 #pragma unroll
       for (int j = 0; j < EPT; ++j) g[p][j] *= f;
 #pragma unroll
-      for (int j = 0; j < EPT; j += 8) IO<TIO>::st8(dx.base(bh) + int64_t(tok) * dx.s_n + d0 + j, dx.vec != 0, &g[p][j]);
+      for (int j = 0; j < EPT; j += 8) IO<TIO>::st8(dx.base(bh) + int64_t(tok) * dx.s_n + d0 + j, &g[p][j]);
     }
   }
 }
@@ -438,7 +434,7 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_maxnorm_keys(MaxnormJob<TIO> j0, MaxnormJ
 #pragma unroll
   for (int p = 0; p < NP; ++p) {
     const int tok = tok0 + 64 * p, tk = tok < n ? tok : n - 1;
-    fm_norm_load<TIO, DH>(J.x.base(bh) + int64_t(tk) * J.x.s_n, J.x.vec != 0, d0, v[p]);
+    fm_norm_load<TIO, DH>(J.x.base(bh) + int64_t(tk) * J.x.s_n, d0, v[p]);
   }
   float mx = -1.0f;
   int cand = 0x7fffffff;

@@ -31,22 +31,27 @@ static constexpr int FM_O1_DQ_PITCH = 40;   // elements per row of k_o1_bwd's pe
 template <int DH> struct O1Raw {
   static constexpr int CPR = DH / 8, N = FM_O1_SEG * CPR / FM_THREADS, RSTEP = FM_THREADS / CPR;
   fm_u32x4 r[N];
-  FM_DEVICE void load(const TRef<const fm_bf16>& x, int bh, int t0, int n, int tid) {
+  // AHEAD: for loads that travel while other work is done: rows past the end are skipped (a branch; nothing here waits for what was
+  // loaded).  Otherwise they read the last row and are cleared behind all loads.
+  template <bool AHEAD = false> FM_DEVICE void load(const TRef<const fm_bf16>& x, int bh, int t0, int n, int tid) {
     const fm_bf16* base = x.base(bh);
     const int col = (tid % CPR) * 8;
 #pragma unroll
     for (int i = 0; i < N; ++i) {
       const int row = t0 + tid / CPR + RSTEP * i;
-      fm_u32x4 z = {0u, 0u, 0u, 0u};
-      if (row < n) {
-        const fm_bf16* p = base + int64_t(row) * x.s_n + col;
-        if (x.vec) z = *reinterpret_cast<const fm_u32x4*>(p);
-        else {
+      if (AHEAD) {
+        fm_u32x4 z = {0u, 0u, 0u, 0u};
+        if (row < n) __builtin_memcpy(&z, base + int64_t(row) * x.s_n + col, 16);
+        r[i] = z;
+      } else __builtin_memcpy(&r[i], base + int64_t(row < n ? row : n - 1) * x.s_n + col, 16);
+    }
+    if (!AHEAD) {
 #pragma unroll
-          for (int j = 0; j < 4; ++j) z[j] = uint32_t(p[2 * j]) | (uint32_t(p[2 * j + 1]) << 16);
-        }
+      for (int i = 0; i < N; ++i) {
+        const bool in = t0 + tid / CPR + RSTEP * i < n;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) r[i][j] = in ? r[i][j] : 0u;
       }
-      r[i] = z;
     }
   }
   // chunk i as eight floats
@@ -163,10 +168,10 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_THREADS, 2) k_o1_sums(O1SumArgs<TIO> A) {
   float gi[R::N];
   auto fetch = [&](int seg) FM_ALWAYS_INLINE {
     const int tb = seg * TT;
-    r0.load(A.x0, bh, tb, A.n, tid);
-    r1.load(A.x1, bh, tb, A.n, tid);
+    r0.template load<true>(A.x0, bh, tb, A.n, tid);
+    r1.template load<true>(A.x1, bh, tb, A.n, tid);
     if (QG) {
-      ro.load(A.o, bh, tb, A.n, tid);
+      ro.template load<true>(A.o, bh, tb, A.n, tid);
 #pragma unroll
       for (int i = 0; i < R::N; ++i) {
         const int row = tb + R::row_of(i, tid);
@@ -407,7 +412,7 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_THREADS, 3) k_o1_fwd(O1FwdArgs<TIO> A) {
       const fm_f32x4 lo = *reinterpret_cast<const fm_f32x4*>(Os + row * OP + col);
       const fm_f32x4 hi = *reinterpret_cast<const fm_f32x4*>(Os + row * OP + col + 4);
       const float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-      IO<TIO>::st8(ob + int64_t(t0 + row) * A.o.s_n + col, A.o.vec != 0, v);
+      IO<TIO>::st8(ob + int64_t(t0 + row) * A.o.s_n + col, v);
     }
   }
 }

@@ -29,18 +29,18 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_pointwise(TRef<const TIO> x, TRef<const T
     const int tok = tok0 + 64 * p;
     if (tok >= a.n) continue;
     float v[EPT], w[EPT];
-    fm_norm_load<TIO, DH>(x.base(bh) + int64_t(tok) * x.s_n, x.vec != 0, d0, v);
+    fm_norm_load<TIO, DH>(x.base(bh) + int64_t(tok) * x.s_n, d0, v);
     if (a.mode == 0) {
       const float* row = a.table + int64_t((tok + a.n) % (2 * a.n - 1)) * DH + d0;
 #pragma unroll
       for (int j = 0; j < EPT; ++j) v[j] += a.factor * row[j];
     } else {
-      fm_norm_load<TIO, DH>(noise.base(bh) + int64_t(tok) * noise.s_n, noise.vec != 0, d0, w);
+      fm_norm_load<TIO, DH>(noise.base(bh) + int64_t(tok) * noise.s_n, d0, w);
 #pragma unroll
       for (int j = 0; j < EPT; ++j) v[j] *= 1.0f + a.factor * w[j];
     }
 #pragma unroll
-    for (int j = 0; j < EPT; j += 8) IO<TIO>::st8(y.base(bh) + int64_t(tok) * y.s_n + d0 + j, y.vec != 0, &v[j]);
+    for (int j = 0; j < EPT; j += 8) IO<TIO>::st8(y.base(bh) + int64_t(tok) * y.s_n + d0 + j, &v[j]);
   }
 }
 

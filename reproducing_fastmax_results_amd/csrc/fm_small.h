@@ -51,12 +51,7 @@ FM_DEVICE void fm_small_load(const TRef<const TIO>& t, int bh, int n, int tid, f
 #pragma unroll
   for (int i = 0; i < DH / 32; ++i) {
     const int c = tid + 256 * i, row = c / (DH / 8), col = (c % (DH / 8)) * 8;
-    if (row < n) {
-      IO<TIO>::ld8(t.base(bh) + int64_t(row) * t.s_n + col, t.vec != 0, r[i]);
-    } else {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) r[i][j] = 0.f;
-    }
+    fm_ld8_row<TIO>(t.base(bh), t.s_n, row, n, col, r[i]);
   }
 }
 // PLAIN, here and below: the second pass of a workgroup whose sums came out non-finite (the lower planes of a weight are
@@ -72,7 +67,7 @@ template <typename TIO, int DH, bool FULL, bool PLAIN> FM_DEVICE void fm_small_s
       float w[8];
 #pragma unroll
       for (int j = 0; j < 8; ++j) w[j] = r[i][j] * up;
-      IO<fm_bf16>::st8(p, true, w);                    // exact: they came from bf16
+      IO<fm_bf16>::st8(p, w);                    // exact: they came from bf16
     } else if constexpr (PLAIN) {
       float* q = reinterpret_cast<float*>(tile) + row * C::PF + col;
 #pragma unroll
@@ -245,7 +240,7 @@ FM_DEVICE void fm_small_fwd(const SmallArgs<TIO>& A, unsigned char* smem, unsign
     const float gi = 1.0f / gt;
 #pragma unroll
     for (int j = 0; j < 8; ++j) v[j] = v[j] * (1.0f / (UW * UQ)) * gi;
-    IO<TIO>::st8(A.out.base(bh) + int64_t(row) * A.out.s_n + col, A.out.vec != 0, v);
+    IO<TIO>::st8(A.out.base(bh) + int64_t(row) * A.out.s_n + col, v);
     if (A.out_resid) {
       float sv[8];
 #pragma unroll
@@ -293,7 +288,7 @@ FM_DEVICE void fm_small_store(const TRef<TIO>& t, int bh, int n, int nstar, floa
 #pragma unroll
       for (int j = 0; j < 8; ++j) v[i][j] -= coef * raw[i][j];
     }
-    IO<TIO>::st8(t.base(bh) + int64_t(row) * t.s_n + col, t.vec != 0, v[i]);
+    IO<TIO>::st8(t.base(bh) + int64_t(row) * t.s_n + col, v[i]);
   }
 }
 

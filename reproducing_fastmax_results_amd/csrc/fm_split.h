@@ -20,11 +20,11 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_merge_parts(TRef<const TIO> oa, TRef<cons
   const float wa = ga.base(bh)[int64_t(tok) * ga.s_n], wb = g.base(bh)[int64_t(tok) * g.s_n];
   const float inv = 1.0f / (wa + wb);
   float a[8], b[8];
-  IO<TIO>::ld8(oa.base(bh) + int64_t(tok) * oa.s_n + d0, oa.vec != 0, a);
-  IO<TIO>::ld8(o.base(bh) + int64_t(tok) * o.s_n + d0, o.vec != 0, b);
+  IO<TIO>::ld8(oa.base(bh) + int64_t(tok) * oa.s_n + d0, a);
+  IO<TIO>::ld8(o.base(bh) + int64_t(tok) * o.s_n + d0, b);
 #pragma unroll
   for (int j = 0; j < 8; ++j) b[j] = (a[j] * wa + b[j] * wb) * inv;
-  IO<TIO>::st8(o.base(bh) + int64_t(tok) * o.s_n + d0, o.vec != 0, b);
+  IO<TIO>::st8(o.base(bh) + int64_t(tok) * o.s_n + d0, b);
 }
 
 // g += ga, after every thread of k_merge_parts has read the old g (a launch of its own).
@@ -42,9 +42,9 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_add_rows(TRef<const TIO> a, TRef<TIO> out
   const int tok = int(i / PER), d0 = int(i % PER) * 8;
   if (tok >= n) return;
   float x[8], y[8];
-  IO<TIO>::ld8(a.base(bh) + int64_t(tok) * a.s_n + d0, a.vec != 0, x);
-  IO<TIO>::ld8(out.base(bh) + int64_t(tok) * out.s_n + d0, out.vec != 0, y);
+  IO<TIO>::ld8(a.base(bh) + int64_t(tok) * a.s_n + d0, x);
+  IO<TIO>::ld8(out.base(bh) + int64_t(tok) * out.s_n + d0, y);
 #pragma unroll
   for (int j = 0; j < 8; ++j) y[j] += x[j];
-  IO<TIO>::st8(out.base(bh) + int64_t(tok) * out.s_n + d0, out.vec != 0, y);
+  IO<TIO>::st8(out.base(bh) + int64_t(tok) * out.s_n + d0, y);
 }

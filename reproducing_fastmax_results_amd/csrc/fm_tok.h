@@ -149,7 +149,7 @@ FM_DEVICE void fm_store_tokens(fm_f32x16 (*acc)[DH / 32], const int* xrow, const
 #pragma unroll
         for (int i = 0; i < 8; ++i) bsum += v[i] * float(br[i]);
       }
-      IO<TIO>::st8(ob + int64_t(row0 + row) * out.s_n + col, out.vec != 0, v);
+      IO<TIO>::st8(ob + int64_t(row0 + row) * out.s_n + col, v);
     }
   }
   FM_SYNC();
@@ -291,7 +291,7 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_THREADS, (TokCfg<E, DH, QT>::OCC_PV)) k_pv(T
   // ---- stage the own rows (and the small states) ----
   if (OWN == FM_OWN_Q) {
     RowRegs<TIO, E, QW, DH> rq;
-    rq.load(A.own_io.base(bh), A.own_io.s_n, A.own_io.vec != 0, t0, A.n_own, tid);
+    rq.load(A.own_io.base(bh), A.own_io.s_n, t0, A.n_own, tid);
     rq.store(Own, PQ, tid, A.sc * fm_norm_factor(A.own_fold, bh, lane));
   } else {
     TileRegs<E, QW, DH> ro;
@@ -492,7 +492,7 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_THREADS, (TokCfg<E, DH, QT>::OCC_PV)) k_pv(T
         const fm_f32x4 lo = *reinterpret_cast<const fm_f32x4*>(Os + row * OP + col);
         const fm_f32x4 hi = *reinterpret_cast<const fm_f32x4*>(Os + row * OP + col + 4);
         const float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-        IO<TIO>::st8(ob + int64_t(t0 + row) * A.out.s_n + col, A.out.vec != 0, v);
+        IO<TIO>::st8(ob + int64_t(t0 + row) * A.out.s_n + col, v);
         if (A.out_resid) {
           float sv[8];
 #pragma unroll
@@ -627,22 +627,14 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_THREADS, (DV ? TokCfg<E, DH, QT>::OCC_DV : T
     // every load of the block is issued before the first result is used
 #pragma unroll
     for (int h = 0; h < NH; ++h) {
-      const int row = t0 + 64 * h + (tid >> 2);
-      if (row < A.n_own) {
-        gi[h] = A.g.base(bh)[int64_t(row) * A.g.s_n];
+      const int row = t0 + 64 * h + (tid >> 2), rw = row < A.n_own ? row : A.n_own - 1;   // (rows past the end: the last one's, made zeros below)
+      gi[h] = A.g.base(bh)[int64_t(rw) * A.g.s_n];
 #pragma unroll
-        for (int j = 0; j < EPT; j += 8) {
-          IO<TIO>::ld8(A.own_do.base(bh) + int64_t(row) * A.own_do.s_n + d0 + j, A.own_do.vec != 0, &ra[h][j]);
-          IO<TIO>::ld8(A.own_o.base(bh) + int64_t(row) * A.own_o.s_n + d0 + j, A.own_o.vec != 0, &rb[h][j]);
-          IO<TIO>::ld8(A.own_io.base(bh) + int64_t(row) * A.own_io.s_n + d0 + j, A.own_io.vec != 0, &rc[h][j]);
-          if (PREP == 2) rr[h][j / 8] = *reinterpret_cast<const fm_half8*>(A.own_ores + (int64_t(bh) * A.npad_own + row) * DH + d0 + j);
-        }
-      } else {
-        gi[h] = 1.0f;
-#pragma unroll
-        for (int j = 0; j < EPT; ++j) { ra[h][j] = 0.f; rb[h][j] = 0.f; rc[h][j] = 0.f; }
-#pragma unroll
-        for (int j = 0; j < EPT / 8; ++j) rr[h][j] = Mma<fm_half>::splat(fm_half(0.f));
+      for (int j = 0; j < EPT; j += 8) {
+        IO<TIO>::ld8(A.own_do.base(bh) + int64_t(rw) * A.own_do.s_n + d0 + j, &ra[h][j]);
+        IO<TIO>::ld8(A.own_o.base(bh) + int64_t(rw) * A.own_o.s_n + d0 + j, &rb[h][j]);
+        IO<TIO>::ld8(A.own_io.base(bh) + int64_t(rw) * A.own_io.s_n + d0 + j, &rc[h][j]);
+        if (PREP == 2) rr[h][j / 8] = *reinterpret_cast<const fm_half8*>(A.own_ores + (int64_t(bh) * A.npad_own + rw) * DH + d0 + j);
       }
     }
 #pragma unroll
@@ -655,8 +647,10 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_THREADS, (DV ? TokCfg<E, DH, QT>::OCC_DV : T
       for (int j = 0; j < EPT; ++j) {
         vg[j] = ra[h][j] * ginv;
         csum += vg[j] * (PREP == 2 ? rb[h][j] + float(rr[h][j / 8][j % 8]) : rb[h][j]);   // PREP = 2: o = bf16 o + what its rounding took
-        vq[j] = rc[h][j] * qsc;
+        vq[j] = row < A.n_own ? rc[h][j] * qsc : 0.f;
+        vg[j] = row < A.n_own ? vg[j] : 0.f;
       }
+      csum = row < A.n_own ? csum : 0.f;
       csum += fm_shfl_xor(csum, 1);
       csum += fm_shfl_xor(csum, 2);
       if (part == 0) {

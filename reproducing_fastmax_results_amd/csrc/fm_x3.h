@@ -88,7 +88,7 @@ template <int DH> struct X3Row {
   static constexpr int CH = 8, NOWN = DH / 16, NT = DH / 32;
   struct Own { X3 f[NOWN]; };
   static FM_DEVICE int feat(int c, int lh) { return 16 * c + 8 * lh; }
-  template <typename TIO> static FM_DEVICE void ld(const TIO* p, bool vec, float v[CH]) { IO<TIO>::ld8(p, vec, v); }
+  template <typename TIO> static FM_DEVICE void ld(const TIO* p, float v[CH]) { IO<TIO>::ld8(p, v); }
   static FM_DEVICE void add_half(const fm_half* p, float v[CH]) {
     const fm_half8 h = *reinterpret_cast<const fm_half8*>(p);
 #pragma unroll
@@ -176,7 +176,7 @@ template <int DH> struct F32Row {
   static constexpr int CH = 1, NOWN = DH / 2, NT = DH / 32;
   struct Own { float f[NOWN]; };
   static FM_DEVICE int feat(int c, int lh) { return 2 * c + lh; }
-  template <typename TIO> static FM_DEVICE void ld(const TIO* p, bool, float v[CH]) { v[0] = IO<TIO>::ld(p); }
+  template <typename TIO> static FM_DEVICE void ld(const TIO* p, float v[CH]) { v[0] = IO<TIO>::ld(p); }
   static FM_DEVICE void add_half(const fm_half* p, float v[CH]) { v[0] += float(*p); }
   static FM_DEVICE void set(Own& o, int c, const float v[CH]) { o.f[c] = v[0]; }
   static FM_DEVICE void fence(int c) { if (c % 4 == 0) FM_SCHED_FENCE(); }
@@ -280,7 +280,7 @@ template <typename TIO, int DH, typename R, int ROWS, int NTH> struct X3Stage {
       gi[i] = 1.0f;
       if (row >= 0 && row < n) {
         const TRef<const TIO>& t = second ? y : x;
-        IO<TIO>::ld8(t.base(bh) + int64_t(row) * t.s_n + col, t.vec != 0, r[i]);
+        IO<TIO>::ld8(t.base(bh) + int64_t(row) * t.s_n + col, r[i]);
         if (g && second) gi[i] = g->base(bh)[int64_t(row) * g->s_n];
       } else {
 #pragma unroll
@@ -312,7 +312,7 @@ template <typename TIO, int DH, typename R, int ROWS, int NTH> struct X3Stage {
       float w[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
       if (row >= 0 && row < n) {
         const TRef<const TIO>& t = second ? y : x;
-        IO<TIO>::ld8(t.base(bh) + int64_t(row) * t.s_n + col, t.vec != 0, w);
+        IO<TIO>::ld8(t.base(bh) + int64_t(row) * t.s_n + col, w);
         const float f = second ? (g ? R::UP / g->base(bh)[int64_t(row) * g->s_n] : R::UP) : xs;
 #pragma unroll
         for (int j = 0; j < 8; ++j) w[j] *= f;
@@ -390,11 +390,11 @@ FM_DEVICE void fm_x3_store(const fm_f32x16* acc, float* Os, int sub, int row, in
     for (int i = 0; i < 8; ++i) v[i] = v[i] * (1.0f / (R::UP * R::UP)) * scale;
     if (bout) {
       float x[8];
-      IO<TIO>::ld8(raw.base(bh) + int64_t(t0 + r) * raw.s_n + col, raw.vec != 0, x);
+      IO<TIO>::ld8(raw.base(bh) + int64_t(t0 + r) * raw.s_n + col, x);
 #pragma unroll
       for (int i = 0; i < 8; ++i) bsum += v[i] * x[i];
     }
-    IO<TIO>::st8(out.base(bh) + int64_t(t0 + r) * out.s_n + col, out.vec != 0, v);
+    IO<TIO>::st8(out.base(bh) + int64_t(t0 + r) * out.s_n + col, v);
   }
   if (bout) {
 #pragma unroll
@@ -450,7 +450,7 @@ FM_DEVICE void fm_x3_fwd(const X3Args<TIO>& A, uint16_t* st, int* bad, const int
     for (int c = 0; c < R::NOWN; ++c) {
       R::fence(c);
       float v[R::CH];
-      R::ld(qr + R::feat(c, lh), A.q.vec != 0, v);
+      R::ld(qr + R::feat(c, lh), v);
 #pragma unroll
       for (int i = 0; i < R::CH; ++i) v[i] = in ? v[i] * qs : 0.f;
       R::set(of, c, v);
@@ -516,7 +516,7 @@ FM_DEVICE void fm_x3_fwd(const X3Args<TIO>& A, uint16_t* st, int* bad, const int
     const float gi = 1.0f / gt;
 #pragma unroll
     for (int i = 0; i < 8; ++i) v[i] = v[i] * (1.0f / (R::UP * R::UP)) * gi;
-    IO<TIO>::st8(A.out.base(bh) + int64_t(qi) * A.out.s_n + col, A.out.vec != 0, v);
+    IO<TIO>::st8(A.out.base(bh) + int64_t(qi) * A.out.s_n + col, v);
     if (A.out_resid) {
       float sv[8];
 #pragma unroll
@@ -568,9 +568,9 @@ FM_DEVICE void fm_x3_dq(const X3Args<TIO>& A, uint16_t* st, int* bad, const int 
       R::fence(c);
       const int f = R::feat(c, lh);
       float v[R::CH], w[R::CH], o[R::CH];
-      R::ld(A.q.base(bh) + row * A.q.s_n + f, A.q.vec != 0, v);
-      R::ld(A.d_o.base(bh) + row * A.d_o.s_n + f, A.d_o.vec != 0, w);
-      R::ld(A.o.base(bh) + row * A.o.s_n + f, A.o.vec != 0, o);
+      R::ld(A.q.base(bh) + row * A.q.s_n + f, v);
+      R::ld(A.d_o.base(bh) + row * A.d_o.s_n + f, w);
+      R::ld(A.o.base(bh) + row * A.o.s_n + f, o);
       if (A.ores) R::add_half(A.ores + (int64_t(bh) * A.npad_q + row) * DH + f, o);
 #pragma unroll
       for (int i = 0; i < R::CH; ++i) { v[i] = in ? v[i] * qs : 0.f; w[i] = in ? w[i] * ginv : 0.f; cs += w[i] * o[i]; }
@@ -668,7 +668,7 @@ FM_DEVICE void fm_x3_dkv(const X3Args<TIO>& A, uint16_t* Vs, int* bad, const int
   for (int c = tid; c < QW * (DH / 8); c += C::NTH) {
     const int r = c / (DH / 8), col = (c % (DH / 8)) * 8, row = t0 + r;
     float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    if (row < A.nk) IO<TIO>::ld8(A.v.base(bh) + int64_t(row) * A.v.s_n + col, A.v.vec != 0, v);
+    if (row < A.nk) IO<TIO>::ld8(A.v.base(bh) + int64_t(row) * A.v.s_n + col, v);
 #pragma unroll
     for (int i = 0; i < 8; ++i) v[i] *= R::UP;
     R::put8(Vs, r, col, v);
@@ -681,7 +681,7 @@ FM_DEVICE void fm_x3_dkv(const X3Args<TIO>& A, uint16_t* Vs, int* bad, const int
     for (int c = 0; c < R::NOWN; ++c) {
       R::fence(c);
       float v[R::CH];
-      R::ld(kr + R::feat(c, lh), A.k.vec != 0, v);
+      R::ld(kr + R::feat(c, lh), v);
 #pragma unroll
       for (int i = 0; i < R::CH; ++i) v[i] = in ? v[i] * ks_ : 0.f;
       R::set(of, c, v);
