@@ -378,8 +378,8 @@ inline int launch_walk_sym(const WalkSymArgs& a, int bh, fm_stream_t stream) {
 }
 
 // Dynamic LDS of a token kernel (kind 0: k_pv, 1: k_ds, 2: k_ds with dV, 3: k_ds with the fused
-// preparation, 4: k_ds with dV and states): va, vb | own rows | region, where the dense stages and the output staging lie over
-// the own rows and the region.
+// preparation, 4: k_ds with dV and states): va, vb | own rows | region, where the dense stages lie over the own rows and
+// the region.
 template <typename E, int DH, int QT> size_t tok_lds_bytes(int kind) {
   typedef TokCfg<E, DH, QT> C;
   size_t region = size_t(2) * (kind == 0 ? C::SLAB_SYM : C::SLAB) * sizeof(E);   // k_pv reads its states with fm_readout_sym
@@ -387,12 +387,10 @@ template <typename E, int DH, int QT> size_t tok_lds_bytes(int kind) {
   if (zs > region) region = zs;
   if (C::WIDE) region = 0;                             // no states at that width
   size_t body = size_t(C::QW) * C::PQ * sizeof(E) + region;
-  const size_t outst = size_t(C::QW) * fm_store_pitch(DH) * 4;
   const size_t stage = kind == 0 ? size_t(2) * C::PV_STAGE * sizeof(E)
                                  : size_t(C::DS_NBUF) * (kind == 2 || kind == 4 ? C::DV_STAGE : C::DS_STAGE) * sizeof(E);
   if (kind == 4) body += size_t(C::QW) * (DH + 1) * 4;      // dK of the fused state readout, behind the slabs
   const size_t prep = size_t(2) * C::QW * C::PQ * sizeof(E) + size_t(C::QW) * 4;   // own q' rows, gh rows, c
-  if (outst > body) body = outst;
   if (stage > body) body = stage;
   if (kind == 3 && prep > body) body = prep;
   return size_t(2 * DH) * 4 + body;

@@ -239,13 +239,15 @@ template <> struct TileMath<fm_half> {
   }
   static FM_DEVICE void put2(fm_half8& v, int i, fm_half2 x) { v[2 * i] = x[0]; v[2 * i + 1] = x[1]; }
   // zero the entries of both fragments whose accumulator row is outside [lo, hi]
+  // (the lane's part of a row is taken off the bounds: what is left of the rows are constants, not sixteen registers)
   static FM_DEVICE void window_frags(frag* f, int lo, int hi, int lh) {
+    const int l = lo - 4 * lh, h = hi - 4 * lh;
 #pragma unroll
     for (int ss = 0; ss < 2; ++ss)
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        const int r = fm_acc_row(8 * ss + i, lh);
-        if (r < lo || r > hi) f[ss][i] = fm_half(0.f);
+        const int r = fm_acc_row(8 * ss + i, 0);
+        if (r < l || r > h) f[ss][i] = fm_half(0.f);
       }
   }
   static FM_DEVICE float fwd(const fm_f32x16& s, const Coef& k, bool edge, int lo, int hi, int lh, frag* pb) {

@@ -24,7 +24,6 @@
 #include "fm_tok.h"
 
 static constexpr int FM_O1_SEG = 128;
-static constexpr int FM_O1_DQ_PITCH = 40;   // elements per row of k_o1_bwd's per-wavefront output staging (32 features, rows 16-byte aligned)
 
 // One 128-token segment of a bf16 caller tensor as raw 16-byte chunks: with CPR = DH / 8 chunks per row,
 // thread t holds chunk t % CPR of the rows t / CPR + (256 / CPR) i.  Rows past the end are zeros.
@@ -388,36 +387,19 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_THREADS, 3) k_o1_fwd(O1FwdArgs<TIO> A) {
 #pragma unroll
       for (int ct = 0; ct < NT; ++ct) acc[ct] = M::mma(M::load_tr(Vs, PQ, 32 * jt + 16 * ss, 32 * ct, lane), pb[ss], acc[ct]);
   }
-  FM_SYNC();                                             // the tiles are spent: the output staging lies over them
-  float* Os = reinterpret_cast<float*>(smem);           // [QW][fm_store_pitch]
   float gt = gsum + fm_shfl_xor(gsum, 32) + A.a0 * float(t0);
   const float ginv = 1.0f / gt;
-  constexpr int OP = fm_store_pitch(DH);
+  const bool in = t0 + own < A.n;
+  if (lh == 0 && in) A.g.base(bh)[int64_t(t0 + own) * A.g.s_n] = gt;
+  TIO* orow = A.o.base(bh) + int64_t(t0 + own) * A.o.s_n;
+  fm_each_octet<NT>(acc, lh, [&](int c, float* v) FM_ALWAYS_INLINE {
 #pragma unroll
-  for (int ct = 0; ct < NT; ++ct)
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const int c = 32 * ct + fm_acc_row(4 * g, lh);
-      fm_f32x4 w;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) w[i] = (acc[ct][4 * g + i] + vecs[DH + c + i]) * ginv;
-      *reinterpret_cast<fm_f32x4*>(Os + own * OP + c) = w;
-    }
-  if (lh == 0 && t0 + own < A.n) A.g.base(bh)[int64_t(t0 + own) * A.g.s_n] = gt;
-  FM_SYNC();
-  TIO* ob = A.o.base(bh);
-  for (int c = tid; c < QW * (DH / 8); c += FM_THREADS) {
-    const int row = c / (DH / 8), col = (c % (DH / 8)) * 8;
-    if (t0 + row < A.n) {
-      const fm_f32x4 lo = *reinterpret_cast<const fm_f32x4*>(Os + row * OP + col);
-      const fm_f32x4 hi = *reinterpret_cast<const fm_f32x4*>(Os + row * OP + col + 4);
-      const float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-      IO<TIO>::st8(ob + int64_t(t0 + row) * A.o.s_n + col, v);
-    }
-  }
+    for (int i = 0; i < 8; ++i) v[i] = (v[i] + vecs[DH + c + i]) * ginv;
+    if (in) IO<TIO>::st8(orow + c, v);
+  });
 }
 template <int DH> inline size_t fm_o1_fwd_lds() {
-  // two row tiles, the two vectors and the prefix slab behind them; the output staging lies over the tiles
+  // two row tiles, the two vectors and the prefix slab behind them
   const size_t tiles = size_t(2) * FM_O1_SEG * (DH + Mma<fm_half>::PAD) * 2 + size_t(2) * DH * 4 +
                        size_t(DH) * (DH + Mma<fm_half>::PAD) * 2;
   return tiles;
@@ -504,7 +486,8 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_THREADS, 2) k_o1_bwd(O1BwdArgs<TIO> A) {
 #pragma unroll
     for (int i = 0; i < O1Raw<DH>::N; ++i) {
       const int row = t0 + O1Raw<DH>::row_of(i, tid);
-      gi[i] = row < A.n ? A.g.base(bh)[int64_t(row) * A.g.s_n] : 1.0f;
+      const float x = A.g.base(bh)[int64_t(row < A.n ? row : A.n - 1) * A.g.s_n];
+      gi[i] = row < A.n ? x : 1.0f;
     }
     float vsum = 0.f;
     if (tid < 3 * DH) {
@@ -568,42 +551,13 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_THREADS, 2) k_o1_bwd(O1BwdArgs<TIO> A) {
 #pragma unroll
       for (int mt = 0; mt < NT; ++mt) dq[mt] = M::mma(M::load_tr(Ks, PQ, 32 * jt + 16 * ss, 32 * mt, lane), db[ss], dq[mt]);
   }
-  // A gradient leaves through an LDS region of the wavefront's own (its 32 tokens, 32 features at a time, already in
-  // the output type): no barrier, so dq goes out right after its phase (its stores travel while dk and dv are
-  // computed) and a wavefront that is done with dk and dv (the later its tokens, the fewer dense tiles) stores them
-  // without waiting for the others.  (With the Jacobian of a folded normalisation, or rows that are not 16-byte
-  // aligned, a gradient goes through the workgroup's fp32 staging at the end.)
+  // A gradient leaves straight from the registers (fm_store_tokens): no barrier, so dq goes out right after its phase (its stores
+  // travel while dk and dv are computed) and a wavefront that is done with dk and dv (the later its tokens, the fewer
+  // dense tiles) stores them without waiting for the others.  (With the Jacobian of a folded normalisation dq goes
+  // out at the end: it meets the rows of Q', which take the place of K'.)
   const float ginv = 1.0f / gsc;
-  auto store_own = [&](const fm_f32x16* acc, float f, const TRef<TIO>& out) FM_ALWAYS_INLINE {
-    if constexpr (sizeof(TIO) == 2) {
-      constexpr int DP = FM_O1_DQ_PITCH;
-      TIO* st = reinterpret_cast<TIO*>(Sl + DH * PS) + wave * 32 * DP;
-      TIO* ob = out.base(bh);
-#pragma unroll
-      for (int mt = 0; mt < NT; ++mt) {
-#pragma unroll
-        for (int g4 = 0; g4 < 4; ++g4) {
-          fm_u32x2 w;
-          w[0] = uint32_t(fm_f32_to_bf16(f * acc[mt][4 * g4])) | (uint32_t(fm_f32_to_bf16(f * acc[mt][4 * g4 + 1])) << 16);
-          w[1] = uint32_t(fm_f32_to_bf16(f * acc[mt][4 * g4 + 2])) | (uint32_t(fm_f32_to_bf16(f * acc[mt][4 * g4 + 3])) << 16);
-          *reinterpret_cast<fm_u32x2*>(st + lr * DP + fm_acc_row(4 * g4, lh)) = w;
-        }
-        FM_WAVE_SYNC();
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          const int c = lane + 64 * i, row = c >> 2, col = (c & 3) * 8;
-          const int tok = t0 + wave * 32 + row;
-          if (tok < A.n)
-            *reinterpret_cast<fm_u32x4*>(ob + int64_t(tok) * out.s_n + 32 * mt + col) = *reinterpret_cast<const fm_u32x4*>(st + row * DP + col);
-        }
-        FM_WAVE_SYNC();
-      }
-    }
-  };
-  const bool dq_own = sizeof(TIO) == 2 && !A.bq && A.dq.vec != 0;
-  const bool dk_own = sizeof(TIO) == 2 && !A.bk && A.dk.vec != 0;
-  const bool dv_own = sizeof(TIO) == 2 && A.dv.vec != 0;
-  if (dq_own) store_own(dq, A.sc * ginv, A.dq);
+  const int xrow[1] = {own};
+  if (!A.bq) fm_store_tokens<TIO, E, DH, 1>(&dq, xrow, nullptr, A.sc * ginv, nullptr, A.dq, bh, t0, A.n, tid);
   FM_SYNC();                                             // K' and the prefix slab are spent
   rq.store(Qs, PQ, tid, qsc);
   slab_store(rs, rs2);
@@ -653,40 +607,32 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_THREADS, 2) k_o1_bwd(O1BwdArgs<TIO> A) {
       }
     }
   }
-  // ---- stores, through LDS.  With the Jacobian of a folded normalisation (bq / bk): the stored gradient carries
+  // ---- stores.  With the Jacobian of a folded normalisation (bq / bk): the stored gradient carries
   // lim / max-norm and the workgroup's part of B = sum dy . y is left for k_norm_fix; the rows y * sc are the tiles
   // still in LDS (Q', and K' which is written back first) ----
-  if (dk_own) store_own(dk, A.sc * ginv, A.dk);
-  if (dv_own) store_own(dv, ginv, A.dv);
-  if (dq_own && dk_own && dv_own) return;
+  if (!A.bk) fm_store_tokens<TIO, E, DH, 1>(&dk, xrow, nullptr, A.sc * ginv, nullptr, A.dk, bh, t0, A.n, tid);
+  fm_store_tokens<TIO, E, DH, 1>(&dv, xrow, nullptr, ginv, nullptr, A.dv, bh, t0, A.n, tid);
+  if (!A.bq && !A.bk) return;
   const int nblk = (A.n + QW - 1) / QW;
-  const int xrow[1] = {own};
-  float* Os = reinterpret_cast<float*>(Vs);              // over V and GH: [QW][fm_store_pitch] floats
+  float* red = reinterpret_cast<float*>(Vs);
   FM_SYNC();                                             // GH, V and c are spent
-  if (!dq_own) {
-    const float fac = A.bq ? fm_norm_factor(A.q_fold, bh, lane) : 1.0f;
-    fm_store_tokens<TIO, E, DH, 1>(&dq, xrow, nullptr, A.sc * ginv * fac, Os, A.dq, bh, t0, A.n, tid,
-                                   A.bq ? Qs : nullptr, fac > 0.f ? 1.0f / (fac * A.sc) : 0.f,
-                                   A.bq ? A.bq + int64_t(bh) * nblk + seg : nullptr, PQ, t0);
+  if (A.bq) {
+    const float fac = fm_norm_factor(A.q_fold, bh, lane);
+    fm_store_tokens<TIO, E, DH, 1>(&dq, xrow, nullptr, A.sc * ginv * fac, red, A.dq, bh, t0, A.n, tid, Qs,
+                                   fac > 0.f ? 1.0f / (fac * A.sc) : 0.f, A.bq + int64_t(bh) * nblk + seg, PQ, t0);
   }
   if (A.bk) {
     // K' rows back into the tile (from the fragments every lane kept): the Jacobian part of dk needs them
+    FM_SYNC();                                           // the rows of Q' have been read, and red
 #pragma unroll
     for (int ks = 0; ks < NKS; ++ks) *reinterpret_cast<frag*>(Ks + own * PQ + ks * M::KSTEP + lh * M::KPL) = kf[ks];
     FM_SYNC();
+    const float fac = fm_norm_factor(A.k_fold, bh, lane);
+    fm_store_tokens<TIO, E, DH, 1>(&dk, xrow, nullptr, A.sc * ginv * fac, red, A.dk, bh, t0, A.n, tid, Ks,
+                                   fac > 0.f ? 1.0f / (fac * A.sc) : 0.f, A.bk + int64_t(bh) * nblk + seg, PQ, t0);
   }
-  if (!dk_own) {
-    const float fac = A.bk ? fm_norm_factor(A.k_fold, bh, lane) : 1.0f;
-    fm_store_tokens<TIO, E, DH, 1>(&dk, xrow, nullptr, A.sc * ginv * fac, Os, A.dk, bh, t0, A.n, tid,
-                                   A.bk ? Ks : nullptr, fac > 0.f ? 1.0f / (fac * A.sc) : 0.f,
-                                   A.bk ? A.bk + int64_t(bh) * nblk + seg : nullptr, PQ, t0);
-  }
-  if (!dv_own) fm_store_tokens<TIO, E, DH, 1>(&dv, xrow, nullptr, ginv, Os, A.dv, bh, t0, A.n, tid);
 }
 template <int DH> inline size_t fm_o1_bwd_lds() {
   const size_t tile = size_t(FM_O1_SEG) * (DH + Mma<fm_half>::PAD) * 2;
-  const size_t tiles = 3 * tile + size_t(FM_O1_SEG) * 4 + size_t(3) * DH * 4 + size_t(DH) * (DH + Mma<fm_half>::PAD) * 2 +
-                       size_t(FM_THREADS / 64) * 32 * FM_O1_DQ_PITCH * 2;            // and the wavefronts' own output staging
-  const size_t outst = tile + size_t(FM_O1_SEG) * fm_store_pitch(DH) * 4;      // Q' / K' tile kept, staging over V and GH
-  return tiles > outst ? tiles : outst;
+  return 3 * tile + size_t(FM_O1_SEG) * 4 + size_t(3) * DH * 4 + size_t(DH) * (DH + Mma<fm_half>::PAD) * 2;
 }

@@ -111,6 +111,12 @@ template <typename V4, typename T> inline V4 fm_lds_tr4_any(const T* p) {
 }
 FM_DEVICE fm_half4 fm_lds_tr4(const fm_half* p) { return fm_lds_tr4_any<fm_half4>(p); }
 FM_DEVICE fm_u16x4 fm_lds_tr4(const uint16_t* p) { return fm_lds_tr4_any<fm_u16x4>(p); }
+// the upper 32 lanes' a and the lower 32 lanes' b change places
+FM_DEVICE void fm_swap_halves(uint32_t& a, uint32_t& b) {
+  const int l = hostsim::g_t.lane;
+  const uint32_t oa = hostsim::shfl(a, l ^ 32), ob = hostsim::shfl(b, l ^ 32);
+  if (l < 32) b = oa; else a = ob;
+}
 FM_DEVICE float fm_fmaxf(float a, float b) { return a != a ? b : (b != b ? a : (a > b ? a : b)); }   // drops a NaN, like fmaxf
 FM_DEVICE float fm_absf(float x) { return __builtin_fabsf(x); }
 FM_DEVICE float fm_clampf(float x, float lim) { return x > lim ? lim : (x < -lim ? -lim : x); }
@@ -230,6 +236,12 @@ FM_DEVICE fm_u16x4 fm_lds_tr4(const uint16_t* p) {
   fm_u16x4 r;
   __builtin_memcpy(&r, &v, 8);
   return r;
+}
+// the upper 32 lanes' a and the lower 32 lanes' b change places (v_permlane32_swap_b32)
+FM_DEVICE void fm_swap_halves(uint32_t& a, uint32_t& b) {
+  typedef uint32_t fm_u2 __attribute__((ext_vector_type(2)));
+  const fm_u2 r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+  a = r[0]; b = r[1];
 }
 FM_DEVICE float fm_fmaxf(float a, float b) { return fmaxf(a, b); }
 FM_DEVICE float fm_absf(float x) { return __builtin_fabsf(x); }

@@ -110,56 +110,67 @@ FM_DEVICE fm_f32x16 fm_zy(const E* Zs, const typename Mma<E>::frag* tf, int mt, 
   return y;
 }
 
-// Accumulators (rows = feature, column = token of tile j) -> caller tensor rows, through LDS.
+// A 32-token tile of accumulators (rows = feature, column = the lane's token) to the token's row, straight from the registers: of two
+// groups of eight features the halves of the wavefront exchange four each (fm_swap_halves), so that a lane holds eight consecutive
+// ones and a store instruction covers 32 bytes of each of the 32 rows.  (Through LDS, with its barriers and one more pass over the
+// values: forward at 4 x 8 heads of 4096 tokens 90 us, so 85; order 1 at 65536 tokens, backward 324, so 303.)
+// f(c, v): the stored values v[8] of the features c .. c + 7 of the lane's token; it stores them where the token exists.
+template <int NT, typename F> FM_DEVICE void fm_each_octet(const fm_f32x16* acc, int lh, F f) {
+#pragma unroll
+  for (int ct = 0; ct < NT; ++ct)
+#pragma unroll
+    for (int g = 0; g < 4; g += 2) {
+      float v[8];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        uint32_t x, y;
+        const float a = acc[ct][4 * g + i], b = acc[ct][4 * g + 4 + i];
+        __builtin_memcpy(&x, &a, 4); __builtin_memcpy(&y, &b, 4);
+        fm_swap_halves(x, y);
+        v[i] = fm_bits_f32(x); v[4 + i] = fm_bits_f32(y);
+      }
+      f(32 * ct + 8 * (g + lh), v);
+    }
+}
+
+// Accumulators (rows = feature, column = token of tile j) times scale -> caller tensor rows.
 // brows (optional): compute-type rows of the same tokens (row t at brows + (t - brow0) * bpitch: a copy in
 // memory, or a tile still in LDS); the workgroup's sum over its stored values times those rows, times bscale,
-// goes to *bout (one workgroup-uniform address).
-// pitch (floats) of the fp32 staging of fm_store_tokens: rows stay 16-byte aligned
-constexpr int fm_store_pitch(int dh) { return dh + 4; }
+// goes to *bout (one workgroup-uniform address).  red: four floats of LDS, used with brows only.
 template <typename TIO, typename E, int DH, int QT>
-FM_DEVICE void fm_store_tokens(fm_f32x16 (*acc)[DH / 32], const int* xrow, const float* addvec, float scale, float* Os,
+FM_DEVICE void fm_store_tokens(fm_f32x16 (*acc)[DH / 32], const int* xrow, const float* addvec, float scale, float* red,
                                TRef<TIO> out, int bh, int row0, int nrows, int tid, const E* brows = nullptr,
                                float bscale = 0.f, float* bout = nullptr, int bpitch = DH, int brow0 = 0) {
   typedef TokCfg<E, DH, QT> C;
-  constexpr int OP = fm_store_pitch(DH);                 // rows of the staging 16-byte aligned: four entries per LDS write
   const int lane = tid & 63, lh = lane >> 5;
-#pragma unroll
-  for (int j = 0; j < QT; ++j)
-#pragma unroll
-    for (int ct = 0; ct < C::NT; ++ct)
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int c = 32 * ct + fm_acc_row(4 * g, lh);
-        fm_f32x4 w;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) w[i] = scale * (acc[j][ct][4 * g + i] + (addvec ? addvec[c + i] : 0.f));
-        *reinterpret_cast<fm_f32x4*>(Os + xrow[j] * OP + c) = w;
-      }
-  FM_SYNC();
   TIO* ob = out.base(bh);
   float bsum = 0.f;
-  for (int c = tid; c < C::QW * (DH / 8); c += FM_THREADS) {
-    const int row = c / (DH / 8), col = (c % (DH / 8)) * 8;
-    if (row0 + row < nrows) {
-      const fm_f32x4 lo = *reinterpret_cast<const fm_f32x4*>(Os + row * OP + col);
-      const fm_f32x4 hi = *reinterpret_cast<const fm_f32x4*>(Os + row * OP + col + 4);
-      const float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-      if (brows) {
-        const E* br = brows + int64_t(row0 + row - brow0) * bpitch + col;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) bsum += v[i] * float(br[i]);
+  for (int j = 0; j < QT; ++j) {
+    const int row = row0 + xrow[j];
+    const bool in = row < nrows;
+    TIO* orow = ob + int64_t(row) * out.s_n;
+    const E* br = brows ? brows + int64_t(row - brow0) * bpitch : nullptr;
+    fm_each_octet<C::NT>(acc[j], lh, [&](int c, float* v) FM_ALWAYS_INLINE {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v[i] = scale * (v[i] + (addvec ? addvec[c + i] : 0.f));
+      if (in) {
+        if (brows) {
+          struct alignas(16) Oct { E e[8]; };
+          const Oct y = *reinterpret_cast<const Oct*>(br + c);
+#pragma unroll
+          for (int i = 0; i < 8; ++i) bsum += v[i] * float(y.e[i]);
+        }
+        IO<TIO>::st8(orow + c, v);
       }
-      IO<TIO>::st8(ob + int64_t(row0 + row) * out.s_n + col, v);
-    }
+    });
   }
-  FM_SYNC();
   if (bout) {
 #pragma unroll
     for (int m = 1; m < 64; m <<= 1) bsum += fm_shfl_xor(bsum, m);
-    if (lane == 0) Os[tid >> 6] = bsum;
+    if (lane == 0) red[tid >> 6] = bsum;
     FM_SYNC();
-    if (tid == 0) *bout = bscale * ((Os[0] + Os[1]) + (Os[2] + Os[3]));
-    FM_SYNC();
+    if (tid == 0) *bout = bscale * ((red[0] + red[1]) + (red[2] + red[3]));
   }
 }
 
@@ -228,7 +239,7 @@ struct TokGeom {
     // the L2 for the others (ordered by weight, the blocks of a segment ran far apart and each fetched it
     // again).  With hundreds of blocks per batch*head the dispatcher evens the weights out by itself.
     const bool seg_major = A.causal && A.use_state && A.nseg >= 8;
-    const int blk = !A.causal ? unit : seg_major ? (OWN == FM_OWN_Q ? nblk - 1 - unit : unit)
+    const int blk = !A.causal ? unit : seg_major || nblk * QW <= A.L ? (OWN == FM_OWN_Q ? nblk - 1 - unit : unit)   // (or one segment)
                                                  : fm_block_of_rank<OWN>(unit, nblk, A.L / QW);
     t0 = blk * QW;
     seg = A.causal ? t0 / A.L : 0;
@@ -459,52 +470,40 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_THREADS, (TokCfg<E, DH, QT>::OCC_PV)) k_pv(T
     FM_SYNC();
   }
 
-  // ---- epilogue, staged through LDS for coalesced stores ----
-  float* Os = reinterpret_cast<float*>(Own);           // [QW][fm_store_pitch]
-  constexpr int OP = fm_store_pitch(DH);
+  // ---- epilogue ----
   if (OWN == FM_OWN_Q) {
     // o = (F + vb) / g
     const float cnt = causal ? float(G.sbeg) : float(A.n_str);   // keys covered by the state
+    TIO* ob = A.out.base(bh);
 #pragma unroll
     for (int j = 0; j < QT; ++j) {
       float gt = gsum[j] + fm_shfl_xor(gsum[j], 32);
       if (G.use_state) gt += A.a0 * cnt;
       const float ginv = 1.0f / gt;
       if (QF) gt *= 1.0f / (4.0f * A.a2);              // the constant taken out of the weights (o does not see it)
-#pragma unroll
-      for (int ct = 0; ct < NT; ++ct)
-#pragma unroll
-        for (int g4 = 0; g4 < 4; ++g4) {
-          const int c = 32 * ct + fm_acc_row(4 * g4, lh);
-          fm_f32x4 w;
-#pragma unroll
-          for (int i = 0; i < 4; ++i) w[i] = (acc[j][ct][4 * g4 + i] + (G.use_state ? vecs[DH + c + i] : 0.f)) * ginv;
-          *reinterpret_cast<fm_f32x4*>(Os + xrow[j] * OP + c) = w;
-        }
       const int qi = t0 + xrow[j];
-      if (lh == 0 && qi < A.n_own) A.g.base(bh)[int64_t(qi) * A.g.s_n] = gt;
-    }
-    FM_SYNC();
-    TIO* ob = A.out.base(bh);
-    for (int c = tid; c < QW * (DH / 8); c += FM_THREADS) {
-      const int row = c / (DH / 8), col = (c % (DH / 8)) * 8;
-      if (t0 + row < A.n_own) {
-        const fm_f32x4 lo = *reinterpret_cast<const fm_f32x4*>(Os + row * OP + col);
-        const fm_f32x4 hi = *reinterpret_cast<const fm_f32x4*>(Os + row * OP + col + 4);
-        const float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-        IO<TIO>::st8(ob + int64_t(t0 + row) * A.out.s_n + col, v);
-        if (A.out_resid) {
-          float sv[8];
+      const bool in = qi < A.n_own;
+      if (lh == 0 && in) A.g.base(bh)[int64_t(qi) * A.g.s_n] = gt;
+      TIO* orow = ob + int64_t(qi) * A.out.s_n;
+      fm_half* rrow = A.out_resid ? A.out_resid + (int64_t(bh) * A.npad_own + qi) * DH : nullptr;
+      fm_each_octet<NT>(acc[j], lh, [&](int c, float* v) FM_ALWAYS_INLINE {
 #pragma unroll
-          for (int i = 0; i < 8; ++i) sv[i] = fm_as_stored<TIO>(v[i]);
-          fm_store_resid8(A.out_resid + (int64_t(bh) * A.npad_own + t0 + row) * DH + col, v, sv);
+        for (int i = 0; i < 8; ++i) v[i] = (v[i] + (G.use_state ? vecs[DH + c + i] : 0.f)) * ginv;
+        if (in) {
+          IO<TIO>::st8(orow + c, v);
+          if (rrow) {
+            float sv[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) sv[i] = fm_as_stored<TIO>(v[i]);
+            fm_store_resid8(rrow + c, v, sv);
+          }
         }
-      }
+      });
     }
   } else {
     // dV = (sums + vb) * out_scale; keys past n_own are discarded by the bounds check
     const float gsc = fm_grad_scale(A.gpart ? A.gpart + int64_t(bh) * A.gnblk : nullptr, A.gnblk, lane);
-    fm_store_tokens<TIO, E, DH, QT>(acc, xrow, G.use_state ? vecs + DH : nullptr, A.out_scale / gsc, Os, A.out, bh, t0,
+    fm_store_tokens<TIO, E, DH, QT>(acc, xrow, G.use_state ? vecs + DH : nullptr, A.out_scale / gsc, nullptr, A.out, bh, t0,
                                     A.n_own, tid);
   }
 }
