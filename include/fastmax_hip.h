@@ -43,8 +43,10 @@ enum {
                                         instead of _Float16; for inputs outside the range stated below.
                                         A training step takes four to five times as long; workspace sizes differ.
                                         Ignored for fp32 tensors. */
-  FASTMAX_FLAG_NORM_SELF = 16        /* nq, nk <= 64 (and not causal with nk > nq): q and k are max-normalised with norm.lim and
+  FASTMAX_FLAG_NORM_SELF = 16,       /* nq, nk <= 64 (and not causal with nk > nq): q and k are max-normalised with norm.lim and
                                         the kernels find the norms themselves; norm.q_keys and norm.k_keys are null */
+  FASTMAX_FLAG_NEW_STATE = 32        /* fastmax_decode_absorb: the state is taken for empty whatever its memory holds, and every
+                                        byte of it is written */
 };
 
 /* Numeric range of the bf16 interface.  bf16 tensors are computed in _Float16 with fp32 accumulation
@@ -176,13 +178,13 @@ int fastmax_backward_saved(const FastmaxDesc* desc, const void* q, const void* k
  * fastmax_decode_state_bytes(desc) bytes for desc->bh of them (0.70 MB per batch*head at d = 64, order 2;
  * 41 KB at order 1), whatever the number of keys.  The layout is the library's own (a state is only ever
  * passed back to these two calls).  A zero-filled buffer
- * is the empty state.  desc: bh, d, dtype, p, a0..a2, inv_tau and the strides named below are used; mask,
- * chunk, flags and norm are ignored (decoding is causal by construction and needs unnormalised q, k: the
+ * is the empty state.  desc: bh, d, dtype, p, a0..a2, inv_tau, FASTMAX_FLAG_NEW_STATE and the strides named below are used;
+ * mask, chunk, the other flags and norm are ignored (decoding is causal by construction and needs unnormalised q, k: the
  * max-norm depends on every token).
  *   fastmax_decode_absorb: adds desc->nk tokens (k, v: strides sk, sv) to the state, e.g. a prompt whose
- *     own outputs come from fastmax_forward.  One launch.  bf16 tensors at d = 64, order 2, 64 tokens or more:
- *     summed with matrix instructions on _Float16 operands (k', and the products v k'), fp32 sums (4 096 tokens
- *     at 16 batch*heads: 0.10 ms); otherwise token after token in fp32.
+ *     own outputs come from fastmax_forward.  One launch.  64 tokens or more are summed with matrix instructions, on
+ *     _Float16 operands (k', and the products v k') with fp32 sums for bf16 tensors at d = 64, order 2, on fp32 operands
+ *     otherwise; fewer token after token in fp32.
  *   fastmax_decode_step: adds one token (k, v) and reads the state out for its query q (strides sq; the
  *     query sees its own key, as in causal attention): o (strides so, one token) and g (sg).  scratch is
  *     not used any more (a step is one launch; the argument and fastmax_decode_scratch_bytes stay for

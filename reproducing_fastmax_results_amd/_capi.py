@@ -22,6 +22,7 @@ BENCH_LIB_NAME = "libfastmax_hip_bench.so"
 
 F32, BF16 = 0, 1
 FLAG_FORCE_MOMENTS, FLAG_FORCE_DENSE, FLAG_SAVE_FOR_BACKWARD, FLAG_F32_COMPUTE, FLAG_NORM_SELF = 1, 2, 4, 8, 16
+FLAG_NEW_STATE = 32
 STATUS_OK = 0
 
 
@@ -295,9 +296,11 @@ class FastmaxLib:
         desc = self.make_desc(k, k, k, mask=True, inv_tau=inv_tau, a0=a0, a1=a1, a2=a2, p=p)
         return torch.zeros(self.lib.fastmax_decode_state_bytes(C.byref(desc)) // 4, dtype=torch.float32, device=k.device)
 
-    def decode_absorb(self, k, v, state, *, inv_tau, p=2, a0=1.0, a1=1.0, a2=0.5):
-        """Adds all tokens of k, v to the state."""
+    def decode_absorb(self, k, v, state, *, inv_tau, p=2, a0=1.0, a1=1.0, a2=0.5, new=False):
+        """Adds all tokens of k, v to the state (``new``: to an empty one, whatever its memory holds)."""
         desc = self.make_desc(k, k, v, mask=True, inv_tau=inv_tau, a0=a0, a1=a1, a2=a2, p=p)
+        if new:
+            desc.flags |= FLAG_NEW_STATE
         st = self.lib.fastmax_decode_absorb(C.byref(desc), k.data_ptr(), v.data_ptr(), state.data_ptr(), self._stream(k))
         self.check(st, "fastmax_decode_absorb")
 

@@ -253,8 +253,9 @@ class FastmaxDecodeState:
 
     def _absorb(self, k, v):
         if self.state is None:
-            self.state = _ext.decode_state(k, *self.args)
-        _ext.decode_absorb(k, v, self.state, *self.args)
+            self.state = _ext.decode_prompt(k, v, *self.args)
+        else:
+            _ext.decode_absorb(k, v, self.state, *self.args)
         self.tokens += k.shape[-2]
 
     @torch.no_grad()

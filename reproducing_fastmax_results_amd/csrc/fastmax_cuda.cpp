@@ -401,6 +401,17 @@ void decode_absorb(torch::Tensor k_, torch::Tensor v_, torch::Tensor state, doub
                "fastmax_decode_absorb");
 }
 
+// the state of a sequence that begins with the tokens of k, v (its memory need not be cleared first)
+torch::Tensor decode_prompt(torch::Tensor k_, torch::Tensor v_, double inv_tau, double a0, double a1, double a2, int64_t p) {
+  const View k = view_of(k_, "k"), v = view_of(v_, "v");
+  FastmaxDesc d = decode_desc(k, k, v, inv_tau, a0, a1, a2, p);
+  d.flags |= FASTMAX_FLAG_NEW_STATE;
+  torch::Tensor state = torch::empty({int64_t(fastmax_decode_state_bytes(&d) / 4)}, k.t.options().dtype(torch::kFloat32));
+  check_status(fastmax_decode_absorb(&d, k.t.data_ptr(), v.t.data_ptr(), state.data_ptr<float>(), stream_of(k.t)),
+               "fastmax_decode_absorb");
+  return state;
+}
+
 std::tuple<torch::Tensor, torch::Tensor> decode_step(torch::Tensor q_, torch::Tensor k_, torch::Tensor v_, torch::Tensor state,
                                                     double inv_tau, double a0, double a1, double a2, int64_t p) {
   const View q = view_of(q_, "q"), k = view_of(k_, "k"), v = view_of(v_, "v");
@@ -627,6 +638,7 @@ PYBIND11_MODULE(fastmax_cuda, m) {
   m.def("backward_norm", &backward_norm, "backward of forward_norm: returns [dq, dk, dv]");
   m.def("decode_state", &decode_state, "empty decoding state (zeros) for keys shaped like k");
   m.def("decode_absorb", &decode_absorb, "add all tokens of k, v to a decoding state");
+  m.def("decode_prompt", &decode_prompt, "decoding state of a sequence that begins with the tokens of k, v");
   m.def("decode_step", &decode_step, "one decoding step on the state: returns (o, g) of the new token");
   m.def("normalize", &normalize, "fused normalisation pass");
   m.def("normalize_backward", &normalize_backward, "gradient of the normalisation pass with respect to its input");

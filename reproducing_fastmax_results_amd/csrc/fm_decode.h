@@ -24,8 +24,9 @@
 // outputs.  Bandwidth and latency bound: a step reads and writes the state once (the denominators once per
 // workgroup: 5 floats per row and workgroup instead of 4).
 //
-// k_decode_absorb_mma (further down): the same sums for a whole prompt with matrix instructions, one launch.
+// k_decode_absorb_mma, k_decode_absorb_f32 (further down): the same sums for a whole prompt with matrix instructions, one launch.
 #pragma once
+#include <type_traits>
 #include "fm_kernels.h"
 
 static constexpr int FM_DEC_ROWS = 64;      // the moment rows of a state are padded to a multiple of this
@@ -59,7 +60,7 @@ template <int DH> FM_DEVICE void fm_decode_row(int r, bool quad, int& m, int& l,
 template <typename TIO, int DH>
 FM_GLOBAL void FM_LAUNCH_BOUNDS(FM_DEC_THREADS)
 k_decode(TRef<const TIO> k, TRef<const TIO> v, TRef<const TIO> q, int n_new, int quad, float inv_tau, float a0,
-         float a1, float a2, float* FM_RESTRICT state, TRef<TIO> o, TRef<float> g, int has_q) {
+         float a1, float a2, float* FM_RESTRICT state, TRef<TIO> o, TRef<float> g, int has_q, int fresh) {
   constexpr int TB = 16;                                 // new tokens staged at a time
   constexpr int NI = (int(fm_decode_rows(DH, true)) + FM_DEC_THREADS - 1) / FM_DEC_THREADS;   // rows per thread at most
   FM_SHARED float ks[TB][DH + 1];                        // k' of the staged tokens, [DH] = 1
@@ -84,8 +85,10 @@ k_decode(TRef<const TIO> k, TRef<const TIO> v, TRef<const TIO> q, int n_new, int
     rlive[i] = false; rm[i] = DH; rl[i] = DH; rmult[i] = 1.0f; dsum[i] = 0.f;
     acc[i] = fm_f32x4{0.f, 0.f, 0.f, 0.f};
     if (r < R) {
-      acc[i] = *reinterpret_cast<const fm_f32x4*>(num + int64_t(r) * 4);
-      dsum[i] = den[r];
+      if (!fresh) {
+        acc[i] = *reinterpret_cast<const fm_f32x4*>(num + int64_t(r) * 4);
+        dsum[i] = den[r];
+      }
       fm_decode_row<DH>(r, quad != 0, rm[i], rl[i], rlive[i], rmult[i]);
     }
   }
@@ -123,6 +126,12 @@ k_decode(TRef<const TIO> k, TRef<const TIO> v, TRef<const TIO> q, int n_new, int
       den[r] = dsum[i];
     }
   }
+  if (fresh) {                                           // the padding behind the last row
+    for (int64_t r = R + tid; r < Rp; r += FM_DEC_THREADS) {
+      *reinterpret_cast<fm_f32x4*>(num + r * 4) = fm_f32x4{0.f, 0.f, 0.f, 0.f};
+      den[r] = 0.f;
+    }
+  }
   if (!has_q) return;
   // readout of the new token's query: the thread's rows, then the wavefront (a butterfly: every lane ends with the
   // same sum), then the wavefronts in order
@@ -158,53 +167,179 @@ k_decode(TRef<const TIO> k, TRef<const TIO> v, TRef<const TIO> q, int n_new, int
 }
 
 // ------------------------------------------------------------------------------
-// k_decode_absorb_mma: a prompt's keys and values added to the state with matrix instructions (bf16 tensors, D = 64,
-// order 2).  k_decode adds tokens one after the other on the vector units: 2 145 rows x 4 columns of multiply-adds
-// per token and workgroup, 1.7 ms for 4 096 tokens at 16 batch*heads; the same sums are three 32 x 32 x 16 products
-// per 16 tokens and value column.
+// Prompts: their keys and values added to the state with matrix instructions.  k_decode adds tokens one after the other on the
+// vector units: 2 145 rows x 4 columns of multiply-adds per token and workgroup, 1.7 ms for 4 096 tokens at 16 batch*heads.
 //
 // grid (D / 4, bh), 512 threads: the workgroup owns the same [R][4] block of the state as in k_decode.  Two groups of four
-// wavefronts take every other tile of 128 tokens, wavefront w of a group the value column c = 4 cb + w.  Per tile
-// the keys (times inv_tau, as _Float16) are staged row-major and
-// the four value columns, a row of ones (zero past the end of the prompt) and three rows of zeros as rows over the
-// tokens.  Per k-step of 16 tokens a wavefront reads the two key fragments with transposing LDS reads and uses them
-// as B operand and, times its value column's fragment, as A operand: the slice  sum_t v_tc k'_ta k'_tb  of its column
-// on the three 32 x 32 tiles on and above the diagonal (it is symmetric in a, b), as k_walk_sym does.  What all four
-// columns share is dealt by k-step, wavefront w taking the k-steps u = w (mod 4): the denominators' order-2 sums
-// (the same three products with the bare key fragments), and the rows 0 .. D of numerators and denominators in one go
-// as  sum_t z_tn' x_tn  with z = (k', then the rows of x) and x = (the four value columns, ones, zeros): three more
-// products.  At the end the wavefronts' parts meet in LDS and are added in a fixed order, and
-// every sum is ADDED to the state in memory (each address by exactly one lane: no atomics, the same bits every run).
-// Operands are rounded to _Float16 (k', and the products v k'), the sums are fp32.
+// wavefronts take every other tile of tokens, wavefront w of a group the value column c = 4 cb + w: the slice
+// sum_t v_tc k'_ta k'_tb of its column on the 32 x 32 tiles on and above the diagonal (it is symmetric in a, b).  What all four
+// columns share is dealt by k-step: the denominators' order-2 sums, and the rows 0 .. D of numerators and denominators in one go
+// as  sum_t z_tn' x_tn  with z = (k', then the rows of x) and x = (the four value columns, ones, zeros).  At the end the wavefronts'
+// parts meet in LDS and are added in a fixed order, and every sum goes to the state in memory, added to what is there or (fresh) in
+// its place: each address by exactly one lane, no atomics, the same bits every run.
+//   k_decode_absorb_mma  bf16 tensors, D = 64, order 2: operands rounded to _Float16 (k', and the products v k'), fp32 sums
+//   k_decode_absorb_f32  everything else: fp32 products (v_mfma_f32_32x32x2_f32)
+// ------------------------------------------------------------------------------
+static constexpr int FM_ABS_GROUPS = 2, FM_ABS_THREADS = FM_ABS_GROUPS * 256, FM_ABS_XR = 8;   // XR: rows of x
+template <int DH, bool QUAD> struct AbsSums {
+  static constexpr int NT = DH / 32;
+  static constexpr int NP = QUAD ? NT * (NT + 1) / 2 : 0;        // pair tiles (a <= b): (0,0) or (0,0), (0,1), (1,1)
+  static constexpr int NSH = NP + NT + 1;                        // shared: denominators of the pairs, rows 1 .. D, row 0
+  static constexpr int RT = 3;                                   // tiles that meet in LDS at a time
+  static constexpr size_t red_bytes() { return size_t(4) * FM_ABS_GROUPS * RT * 16 * 64 * 4; }
+  static constexpr int pa(int i) { return i == 2 ? 1 : 0; }      // row tile and column tile of pair tile i
+  static constexpr int pb(int i) { return i == 0 ? 0 : 1; }
+};
+// N elements of a caller's row as they lie in memory, in whole registers: loads that travel while other work is done wait for nothing
+template <typename TIO, int N> struct Raw {
+  static constexpr int NW = N * int(sizeof(TIO)) / 4;
+  uint32_t w[NW];
+  FM_DEVICE void zero() {
+#pragma unroll
+    for (int i = 0; i < NW; ++i) w[i] = 0u;
+  }
+  FM_DEVICE void ld(const TIO* p) { __builtin_memcpy(w, p, sizeof(w)); }
+  FM_DEVICE float get(int i) const {
+    if (sizeof(TIO) == 4) return fm_bits_f32(w[i % NW]);
+    return fm_bits_f32((i & 1) ? (w[i / 2] & 0xffff0000u) : (w[i / 2] << 16));
+  }
+};
+
+// Everything accumulated -> state.  col: the wavefront's pair tiles, sh: its part of the shared sums; all LDS from red on is free.
+template <int DH, bool QUAD>
+FM_DEVICE void fm_absorb_finish(const fm_f32x16* col, const fm_f32x16* sh, float* red, float* num, float* den, bool fresh) {
+  typedef AbsSums<DH, QUAD> C;
+  constexpr int NP = C::NP, NSH = C::NSH, NW = 4 * FM_ABS_GROUPS;
+  const int lane = FM_TID_X & 63, lr = lane & 31, lh = lane >> 5;
+  const int wave8 = FM_UNIFORM(FM_TID_X >> 6), wave = wave8 & 3, grp = wave8 >> 2;
+  auto pair_row = [&](int a, int b) { return 1 + DH + a * DH - a * (a - 1) / 2 + (b - a); };
+  // the value columns: entries (a, b) with a <= b go to their pair rows; group 0 writes accumulator entries 0 .. 7 of its
+  // column's tiles, group 1 entries 8 .. 15 (16 rows further down), each with the other group's part from LDS.  Every state entry
+  // is read before the first is written: as read-modify-writes one after the other they were up to 72 memory latencies in a row.
+  if constexpr (NP > 0) {
+    float old[NP][8];
+    float* at[NP][8];
+    bool live[NP][8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int ra = fm_acc_row(e, lh) + 16 * grp;
+#pragma unroll
+      for (int i = 0; i < NP; ++i) {
+        live[i][e] = C::pa(i) != C::pb(i) || ra <= lr;
+        at[i][e] = num + (live[i][e] ? int64_t(pair_row(32 * C::pa(i) + ra, 32 * C::pb(i) + lr)) * 4 + wave : wave);
+        old[i][e] = 0.f;
+      }
+    }
+    if (!fresh) {
+#pragma unroll
+      for (int i = 0; i < NP; ++i)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) old[i][e] = *at[i][e];
+    }
+#pragma unroll
+    for (int i = 0; i < NP; ++i)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) red[((wave8 * NP + i) * 8 + e) * 64 + lane] = grp ? col[i][e] : col[i][8 + e];
+    FM_SYNC();
+#pragma unroll
+    for (int i = 0; i < NP; ++i)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float other = red[(((wave8 ^ 4) * NP + i) * 8 + e) * 64 + lane];
+        if (live[i][e]) *at[i][e] = old[i][e] + ((grp ? other : col[i][e]) + (grp ? col[i][8 + e] : other));
+      }
+  }
+  // the shared sums: the eight parts through LDS, RT tiles at a time; wavefront w adds entries 2 w and 2 w + 1 of every
+  // tile in the order of the wavefronts
+  constexpr int RT = C::RT, EPW = 16 / NW;
+  float* sat[NSH][EPW];                                  // where they go; null: nowhere
+  float sold[NSH][EPW];
+#pragma unroll
+  for (int i = 0; i < NSH; ++i)
+#pragma unroll
+    for (int x = 0; x < EPW; ++x) {
+      const int ra = fm_acc_row(EPW * wave8 + x, lh);
+      float* p = nullptr;
+      if (i < NP) {                                      // denominators of the pair rows
+        if (C::pa(i) != C::pb(i) || ra <= lr) p = den + pair_row(32 * C::pa(i) + ra, 32 * C::pb(i) + lr);
+      } else if (i < NSH - 1) {                          // rows 1 + a: column n < 4 a numerator, n = 4 the denominator
+        const int a = 32 * (i - NP) + ra;
+        if (lr < 4) p = num + int64_t(1 + a) * 4 + lr;
+        else if (lr == 4) p = den + 1 + a;
+      } else if (ra == 4) {                              // row 0: the ones row of z against the columns of x
+        if (lr < 4) p = num + lr;
+        else if (lr == 4) p = den;
+      }
+      sat[i][x] = p;
+      sold[i][x] = 0.f;
+    }
+  if (!fresh) {
+#pragma unroll
+    for (int i = 0; i < NSH; ++i)
+#pragma unroll
+      for (int x = 0; x < EPW; ++x) sold[i][x] = *(sat[i][x] ? sat[i][x] : den);
+  } else {
+    // the padding behind the last row
+    constexpr int R = int(fm_decode_rows(DH, QUAD)), RP = int(fm_decode_rows_padded(DH, QUAD));
+    for (int r = R + FM_TID_X; r < RP; r += FM_ABS_THREADS) {
+      *reinterpret_cast<fm_f32x4*>(num + int64_t(r) * 4) = fm_f32x4{0.f, 0.f, 0.f, 0.f};
+      den[r] = 0.f;
+    }
+  }
+#pragma unroll
+  for (int i0 = 0; i0 < NSH; i0 += RT) {
+    FM_SYNC();                                           // what lay there has been read
+#pragma unroll
+    for (int i = 0; i < RT; ++i)
+      if (i0 + i < NSH) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) red[((wave8 * RT + i) * 16 + e) * 64 + lane] = sh[i0 + i][e];
+      }
+    FM_SYNC();
+#pragma unroll
+    for (int i = 0; i < RT; ++i)
+      if (i0 + i < NSH) {
+#pragma unroll
+        for (int x = 0; x < EPW; ++x) {
+          float sum = 0.f;
+#pragma unroll
+          for (int w = 0; w < NW; ++w) sum += red[((w * RT + i) * 16 + EPW * wave8 + x) * 64 + lane];
+          float* p = sat[i0 + i][x];
+          if (p) *p = sold[i0 + i][x] + sum;
+        }
+      }
+  }
+}
+
+// Per tile of 128 tokens the keys (times inv_tau, as _Float16) are staged row-major and the four value columns, a row of ones (zero
+// past the end of the prompt) and three rows of zeros as rows over the tokens.  Per k-step of 16 tokens a wavefront reads the two key
+// fragments with transposing LDS reads and uses them as B operand and, times its value column's fragment, as A operand.
 //
-// What bounds it is latency: 16 batch*heads are one workgroup per CU, each a chain over the tiles (fetch, LDS, products).
-// Two groups halve the chain (LDS and 256 registers per lane leave no room for more).  At the end every state entry is
-// read before the first is written: as read-modify-writes one after the other they were up to 72 memory latencies in a
-// row.  One group and read-modify-writes, then this, microseconds per call at 64, 1024 and 4096 tokens:
-// B*H = 1: 17, 32, 81 and 11, 20, 50;  B*H = 16: 19, 35, 86 and 13, 24, 58;  B*H = 64: 100, 187, 474 and 46, 96, 262.
+// What bounds it is latency: 16 batch*heads are one workgroup per CU, each a chain over the tiles (fetch, LDS, products); two groups
+// halve it (LDS and 256 registers per lane leave no room for more).  The rows on their way to LDS wait in registers as they came:
+// converted as they were loaded, they made every tile wait for its loads.
 template <int DH> struct DecAbsCfg {
   typedef Mma<fm_half> M;
   static constexpr int TT = 128;                       // tokens per tile
   static constexpr int PQ = DH + M::PAD;               // pitch of the key rows
-  static constexpr int XR = 8;                         // rows over tokens: four value columns, ones, three of zeros
   static constexpr int XP = TT + M::PAD;
-  static constexpr int TILE_E = TT * PQ + XR * XP;
-  static constexpr int NSH = 6;                        // accumulator tiles of the shared sums per wavefront
-  static constexpr int NG = 2, NTH = NG * 256;         // groups of four wavefronts
-  static constexpr size_t RED_BYTES = size_t(4) * NG * (NSH / 2) * 16 * 64 * 4;   // they meet in LDS three tiles at a time
-  static constexpr size_t STAGE_BYTES = size_t(NG) * 2 * TILE_E * 2;
-  static constexpr size_t lds_bytes() { return STAGE_BYTES > RED_BYTES ? STAGE_BYTES : RED_BYTES; }
+  static constexpr int TILE_E = TT * PQ + FM_ABS_XR * XP;
+  static constexpr size_t lds_bytes() {
+    const size_t st = size_t(FM_ABS_GROUPS) * 2 * TILE_E * 2, red = AbsSums<DH, true>::red_bytes();
+    return st > red ? st : red;
+  }
 };
 
 template <typename TIO, int DH>
-FM_GLOBAL void FM_LAUNCH_BOUNDS2((DecAbsCfg<DH>::NTH), 2)
-k_decode_absorb_mma(TRef<const TIO> k, TRef<const TIO> v, int n_new, float inv_tau, float* FM_RESTRICT state) {
+FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_ABS_THREADS, 2)
+k_decode_absorb_mma(TRef<const TIO> k, TRef<const TIO> v, int n_new, float inv_tau, float* FM_RESTRICT state, int fresh) {
   static_assert(DH == 64, "two 32-row tiles per feature axis");
   typedef fm_half E;
   typedef Mma<E> M;
   typedef typename M::frag frag;
   typedef DecAbsCfg<DH> C;
-  constexpr int TT = C::TT, PQ = C::PQ, XP = C::XP, NSTEP = TT / M::KSTEP;
+  typedef AbsSums<DH, true> S;
+  constexpr int TT = C::TT, PQ = C::PQ, XP = C::XP, NSTEP = TT / M::KSTEP, XR = FM_ABS_XR, NG = FM_ABS_GROUPS;
   FM_DYN_SMEM(smem);
   const int lane = FM_TID_X & 63, lr = lane & 31, lh = lane >> 5;
   const int wave8 = FM_UNIFORM(FM_TID_X >> 6), wave = wave8 & 3, grp = wave8 >> 2;
@@ -221,18 +356,20 @@ k_decode_absorb_mma(TRef<const TIO> k, TRef<const TIO> v, int n_new, float inv_t
   const TIO* kb = k.base(bh);
   const TIO* vb = v.base(bh);
 
-  // global memory -> registers: a thread's four 16-byte pieces of the key rows, and (threads below TT) a token's four values
+  // global memory -> registers: a thread's four pieces of the key rows, and (threads below TT) a token's four values
   constexpr int CPR = DH / 8, NK = TT * CPR / 256;
-  float kreg[NK][8], vreg[4];
+  Raw<TIO, 8> kreg[NK];
+  Raw<TIO, 4> vreg;
   auto fetch = [&](int t0) FM_ALWAYS_INLINE {
 #pragma unroll
     for (int i = 0; i < NK; ++i) {
       const int c = tid + 256 * i, row = t0 + c / CPR, f0 = (c % CPR) * 8;
-      fm_ld8_row<TIO>(kb, k.s_n, row, n_new, f0, kreg[i]);
+      if (row < n_new) kreg[i].ld(kb + int64_t(row) * k.s_n + f0);
+      else kreg[i].zero();
     }
     if (tid < TT) {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) vreg[j] = (t0 + tid < n_new) ? IO<TIO>::ld(vb + int64_t(t0 + tid) * v.s_n + c4 + j) : 0.f;
+      if (t0 + tid < n_new) vreg.ld(vb + int64_t(t0 + tid) * v.s_n + c4);
+      else vreg.zero();
     }
   };
   auto put = [&](E* b, int t0) FM_ALWAYS_INLINE {
@@ -241,173 +378,232 @@ k_decode_absorb_mma(TRef<const TIO> k, TRef<const TIO> v, int n_new, float inv_t
       const int c = tid + 256 * i;
       float sc[8];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) sc[j] = kreg[i][j] * inv_tau;
+      for (int j = 0; j < 8; ++j) sc[j] = kreg[i].get(j) * inv_tau;
       CE<E>::st8(b + (c / CPR) * PQ + (c % CPR) * 8, sc);
     }
     if (tid < TT) {
       E* x = b + TT * PQ + tid;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) x[j * XP] = E(vreg[j]);
+      for (int j = 0; j < 4; ++j) x[j * XP] = E(vreg.get(j));
       x[4 * XP] = E(t0 + tid < n_new ? 1.0f : 0.0f);
     }
   };
+  const int g0 = grp * TT;                               // tiles past the end of the prompt are zeros
+  fetch(g0);
   // rows 5 .. 7 of both buffers: zeros, written once
   for (int i = tid; i < 2 * 3 * XP; i += 256) {
     E* b = i < 3 * XP ? buf0 : buf1;
     b[TT * PQ + 5 * XP + (i % (3 * XP))] = E(0.0f);
   }
 
-  fm_f32x16 a00 = fm_zero16(), a01 = fm_zero16(), a11 = fm_zero16();       // the wavefront's value column
-  fm_f32x16 sh[C::NSH];                                                     // its part of the shared sums: d00, d01, d11, l0, l1, r0
+  fm_f32x16 col[S::NP], sh[S::NSH];                      // the wavefront's value column; its part of the shared sums
 #pragma unroll
-  for (int i = 0; i < C::NSH; ++i) sh[i] = fm_zero16();
+  for (int i = 0; i < S::NP; ++i) col[i] = fm_zero16();
+#pragma unroll
+  for (int i = 0; i < S::NSH; ++i) sh[i] = fm_zero16();
 
-  const int g0 = grp * TT;                               // tiles past the end of the prompt are zeros
-  fetch(g0);
   put(buf0, g0);
-  if (C::NG * TT < n_new) fetch(C::NG * TT + g0);
-  FM_SYNC();
+  if (NG * TT < n_new) fetch(NG * TT + g0);
+  FM_SYNC_LDS();
   int par = 0;
-  for (int tb = 0; tb < n_new; tb += C::NG * TT) {
+  for (int tb = 0; tb < n_new; tb += NG * TT) {
     const E* cbuf = par ? buf1 : buf0;
     const E* xt = cbuf + TT * PQ;
+    if (tb + NG * TT < n_new) {
+      put(par ? buf0 : buf1, tb + NG * TT + g0);
+      if (tb + 2 * NG * TT < n_new) fetch(tb + 2 * NG * TT + g0);
+    }
     if (tb + g0 < n_new) {
+      // the wavefront's own quarter of the k-steps first (no branch around the shared sums); the fragments of the next k-step are
+      // on their way while one is multiplied
+      frag k0, k1, xv;
+      auto load = [&](int j) FM_ALWAYS_INLINE {
+        const int u = (j + NSTEP / 4 * wave) % NSTEP;
+        const E* kt = cbuf + 16 * u * PQ;
+        k0 = M::load_tr(kt, PQ, 0, 0, lane); k1 = M::load_tr(kt, PQ, 0, 32, lane);
+        xv = M::load_nat_perm(xt + wave * XP, u, lh);
+      };
+      load(0);
 #pragma unroll
-    for (int u = 0; u < NSTEP; ++u) {
-      const frag k0 = M::load_tr(cbuf, PQ, 16 * u, 0, lane), k1 = M::load_tr(cbuf, PQ, 16 * u, 32, lane);
-      const frag xv = M::load_nat_perm(xt + wave * XP, u, lh);
-      const frag f0 = k0 * xv, f1 = k1 * xv;
-      a00 = M::mma(f0, k0, a00);
-      a01 = M::mma(f0, k1, a01);
-      a11 = M::mma(f1, k1, a11);
-      if ((u & 3) == wave) {
-        const frag xs = M::load_nat_perm(xt + (lr < C::XR ? lr : C::XR - 1) * XP, u, lh);   // rows past the eighth: zeros
-        sh[0] = M::mma(k0, k0, sh[0]);
-        sh[1] = M::mma(k0, k1, sh[1]);
-        sh[2] = M::mma(k1, k1, sh[2]);
-        sh[3] = M::mma(k0, xs, sh[3]);
-        sh[4] = M::mma(k1, xs, sh[4]);
-        sh[5] = M::mma(xs, xs, sh[5]);
+      for (int j = 0; j < NSTEP; ++j) {
+        const frag c0 = k0, c1 = k1, f0 = k0 * xv, f1 = k1 * xv;
+        if (j + 1 < NSTEP) load(j + 1);
+        FM_SCHED_FENCE();
+        col[0] = M::mma(f0, c0, col[0]);
+        col[1] = M::mma(f0, c1, col[1]);
+        col[2] = M::mma(f1, c1, col[2]);
+        if (j < NSTEP / 4) {
+          const frag xs = M::load_nat_perm(xt + (lr < XR ? lr : XR - 1) * XP, (j + NSTEP / 4 * wave) % NSTEP, lh);   // rows past the eighth: zeros
+          sh[0] = M::mma(c0, c0, sh[0]);
+          sh[1] = M::mma(c0, c1, sh[1]);
+          sh[2] = M::mma(c1, c1, sh[2]);
+          sh[3] = M::mma(c0, xs, sh[3]);
+          sh[4] = M::mma(c1, xs, sh[4]);
+          sh[5] = M::mma(xs, xs, sh[5]);
+        }
       }
     }
-    }
-    if (tb + C::NG * TT < n_new) {
-      put(par ? buf0 : buf1, tb + C::NG * TT + g0);
-      if (tb + 2 * C::NG * TT < n_new) fetch(tb + 2 * C::NG * TT + g0);
-    }
-    FM_SYNC();
+    FM_SYNC_LDS();
     par ^= 1;
   }
-
-  float* red = reinterpret_cast<float*>(smem);           // the staging buffers are spent: the loop ended on a barrier
-  auto pair_row = [&](int a, int b) { return 1 + DH + a * DH - a * (a - 1) / 2 + (b - a); };
-  // the value columns: entries (a, b) with a <= b go to their pair rows; group 0 writes accumulator entries 0 .. 7 of its
-  // column's three tiles, group 1 entries 8 .. 15 (16 rows further down), each with the other group's part from LDS
-  {
-    float old[3][8];
-    float* at[3][8];
-    bool live[3][8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const int ra = fm_acc_row(e, lh) + 16 * grp;
-#pragma unroll
-      for (int i = 0; i < 3; ++i) {
-        live[i][e] = i == 1 || ra <= lr;
-        at[i][e] = num + (live[i][e] ? int64_t(pair_row(i == 2 ? 32 + ra : ra, i == 0 ? lr : 32 + lr)) * 4 + wave : wave);
-        old[i][e] = *at[i][e];
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-      const fm_f32x16& a = i == 0 ? a00 : i == 1 ? a01 : a11;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) red[((wave8 * 3 + i) * 8 + e) * 64 + lane] = grp ? a[e] : a[8 + e];
-    }
-    FM_SYNC();
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-      const fm_f32x16& a = i == 0 ? a00 : i == 1 ? a01 : a11;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float other = red[(((wave8 ^ 4) * 3 + i) * 8 + e) * 64 + lane];
-        if (live[i][e]) *at[i][e] = old[i][e] + ((grp ? other : a[e]) + (grp ? a[8 + e] : other));
-      }
-    }
-  }
-  // the shared sums: the eight parts through LDS, three tiles at a time; wavefront w adds entries 2 w and 2 w + 1 of every
-  // tile in the order of the wavefronts
-  constexpr int HALF = C::NSH / 2, NW = 4 * C::NG, EPW = 16 / NW;
-  float* sat[C::NSH][EPW];                               // where they go; null: nowhere
-  float sold[C::NSH][EPW];
-#pragma unroll
-  for (int i = 0; i < C::NSH; ++i)
-#pragma unroll
-    for (int x = 0; x < EPW; ++x) {
-      const int ra = fm_acc_row(EPW * wave8 + x, lh);
-      float* p = nullptr;
-      if (i == 0) { if (ra <= lr) p = den + pair_row(ra, lr); }            // denominators of the pair rows
-      else if (i == 1) p = den + pair_row(ra, 32 + lr);
-      else if (i == 2) { if (ra <= lr) p = den + pair_row(32 + ra, 32 + lr); }
-      else if (i < 5) {                                  // rows 1 + a: column n < 4 a numerator, n = 4 the denominator
-        const int a = 32 * (i - 3) + ra;
-        if (lr < 4) p = num + int64_t(1 + a) * 4 + lr;
-        else if (lr == 4) p = den + 1 + a;
-      } else if (ra == 4) {                              // row 0: the ones row of z against the columns of x
-        if (lr < 4) p = num + lr;
-        else if (lr == 4) p = den;
-      }
-      sat[i][x] = p;
-      sold[i][x] = *(p ? p : den);
-    }
-#pragma unroll
-  for (int rnd = 0; rnd < 2; ++rnd) {
-    FM_SYNC();                                           // what lay there has been read
-#pragma unroll
-    for (int i = 0; i < HALF; ++i)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) red[((wave8 * HALF + i) * 16 + e) * 64 + lane] = sh[rnd * HALF + i][e];
-    FM_SYNC();
-#pragma unroll
-    for (int i = 0; i < HALF; ++i)
-#pragma unroll
-      for (int x = 0; x < EPW; ++x) {
-        float sum = 0.f;
-#pragma unroll
-        for (int w = 0; w < NW; ++w) sum += red[((w * HALF + i) * 16 + EPW * wave8 + x) * 64 + lane];
-        float* p = sat[rnd * HALF + i][x];
-        if (p) *p = sold[rnd * HALF + i][x] + sum;
-      }
-  }
+  // the staging buffers are spent: the loop ended on a barrier
+  fm_absorb_finish<DH, true>(col, sh, reinterpret_cast<float*>(smem), num, den, fresh != 0);
 }
 
-// prompts of bf16 tensors at D = 64, order 2, from this many tokens on go through k_decode_absorb_mma (below it the
-// one launch of k_decode is as quick, and it keeps fp32 products)
+// The same sums from fp32 products, for fp32 tensors, order 1 and heads of 32.  A matrix instruction takes two tokens; its operands
+// are single floats of the staged rows (key rows [token][feature], x rows [token][8]), read across the lanes without conflicts.
+// The matrix pipe bounds it: 4.5 instructions of 64 cycles per two tokens, wavefront and order-2 problem at D = 64.
+template <int DH> struct DecAbsF32Cfg {
+  static constexpr int TT = 64;                        // tokens per tile
+  static constexpr int PQ = DH + 4;
+  static constexpr int TILE = TT * PQ + TT * FM_ABS_XR;
+  static constexpr size_t lds_bytes() {
+    const size_t st = size_t(FM_ABS_GROUPS) * 2 * TILE * 4, red = AbsSums<DH, true>::red_bytes();
+    return st > red ? st : red;
+  }
+};
+template <typename TIO, int DH, bool QUAD>
+FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_ABS_THREADS, 2)
+k_decode_absorb_f32(TRef<const TIO> k, TRef<const TIO> v, int n_new, float inv_tau, float* FM_RESTRICT state, int fresh) {
+  typedef Mma<float> M;
+  typedef DecAbsF32Cfg<DH> C;
+  typedef AbsSums<DH, QUAD> S;
+  constexpr int TT = C::TT, PQ = C::PQ, XR = FM_ABS_XR, NT = DH / 32, NG = FM_ABS_GROUPS;
+  FM_DYN_SMEM(smem);
+  const int lane = FM_TID_X & 63, lr = lane & 31, lh = lane >> 5;
+  const int wave8 = FM_UNIFORM(FM_TID_X >> 6), wave = wave8 & 3, grp = wave8 >> 2;
+  const int tid = FM_TID_X & 255;
+  float* const buf0 = reinterpret_cast<float*>(smem) + grp * 2 * C::TILE;
+  int cb, bh;
+  fm_xcd_map(FM_GDIM_X, FM_GDIM_Y, cb, bh);
+  const int c4 = 4 * cb;
+  const int64_t Rp = fm_decode_rows_padded(DH, QUAD);
+  float* num = state + (int64_t(bh) * (DH / 4) + cb) * Rp * 5;
+  float* den = num + Rp * 4;
+  const TIO* kb = k.base(bh);
+  const TIO* vb = v.base(bh);
+  constexpr int CPR = DH / 8, NK = TT * CPR / 256;
+  static_assert(TT * CPR % 256 == 0, "whole pieces per thread");
+  Raw<TIO, 8> kreg[NK];
+  Raw<TIO, 4> vreg;
+  auto fetch = [&](int t0) FM_ALWAYS_INLINE {
+#pragma unroll
+    for (int i = 0; i < NK; ++i) {
+      const int c = tid + 256 * i, row = t0 + c / CPR, f0 = (c % CPR) * 8;
+      if (row < n_new) kreg[i].ld(kb + int64_t(row) * k.s_n + f0);
+      else kreg[i].zero();
+    }
+    if (tid < TT) {
+      if (t0 + tid < n_new) vreg.ld(vb + int64_t(t0 + tid) * v.s_n + c4);
+      else vreg.zero();
+    }
+  };
+  auto put = [&](float* b, int t0) FM_ALWAYS_INLINE {
+#pragma unroll
+    for (int i = 0; i < NK; ++i) {
+      const int c = tid + 256 * i;
+      float sc[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) sc[j] = kreg[i].get(j) * inv_tau;
+      CE<float>::st8(b + (c / CPR) * PQ + (c % CPR) * 8, sc);
+    }
+    if (tid < TT) {
+      const float x[8] = {vreg.get(0), vreg.get(1), vreg.get(2), vreg.get(3), t0 + tid < n_new ? 1.0f : 0.0f, 0.f, 0.f, 0.f};
+      CE<float>::st8(b + TT * PQ + tid * XR, x);
+    }
+  };
+  fm_f32x16 col[S::NP > 0 ? S::NP : 1], sh[S::NSH];
+#pragma unroll
+  for (int i = 0; i < S::NP; ++i) col[i] = fm_zero16();
+#pragma unroll
+  for (int i = 0; i < S::NSH; ++i) sh[i] = fm_zero16();
+  const int g0 = grp * TT;
+  fetch(g0);
+  put(buf0, g0);
+  if (NG * TT < n_new) fetch(NG * TT + g0);
+  FM_SYNC_LDS();
+  int par = 0;
+  for (int tb = 0; tb < n_new; tb += NG * TT) {
+    const float* kt = buf0 + par * C::TILE;
+    const float* xt = kt + TT * PQ;
+    if (tb + NG * TT < n_new) {
+      put(buf0 + (par ^ 1) * C::TILE, tb + NG * TT + g0);
+      if (tb + 2 * NG * TT < n_new) fetch(tb + 2 * NG * TT + g0);
+    }
+    if (tb + g0 < n_new) {
+      constexpr int NU = TT / 2;
+      auto step = [&](int j, auto shared_tag) FM_ALWAYS_INLINE {
+        const int t = 2 * ((j + NU / 4 * wave) % NU) + lh;   // the wavefront's own quarter of the steps first
+        float kf[NT], f[NT];
+#pragma unroll
+        for (int i = 0; i < NT; ++i) kf[i] = kt[t * PQ + 32 * i + lr];
+        if constexpr (QUAD) {
+          const float x = xt[t * XR + wave];
+#pragma unroll
+          for (int i = 0; i < NT; ++i) f[i] = kf[i] * x;
+#pragma unroll
+          for (int i = 0; i < S::NP; ++i) col[i] = M::mma(f[S::pa(i)], kf[S::pb(i)], col[i]);
+        }
+        if constexpr (decltype(shared_tag)::value) {
+          const float xr = xt[t * XR + (lr & (XR - 1))], xs = lr < XR ? xr : 0.f;
+#pragma unroll
+          for (int i = 0; i < S::NP; ++i) sh[i] = M::mma(kf[S::pa(i)], kf[S::pb(i)], sh[i]);
+#pragma unroll
+          for (int i = 0; i < NT; ++i) sh[S::NP + i] = M::mma(kf[i], xs, sh[S::NP + i]);
+          sh[S::NSH - 1] = M::mma(xs, xs, sh[S::NSH - 1]);
+        }
+      };
+#pragma unroll
+      for (int j = 0; j < NU / 4; ++j) step(j, std::true_type());
+      if constexpr (QUAD) {
+#pragma unroll 8
+        for (int j = NU / 4; j < NU; ++j) step(j, std::false_type());
+      }
+    }
+    FM_SYNC_LDS();
+    par ^= 1;
+  }
+  fm_absorb_finish<DH, QUAD>(col, sh, reinterpret_cast<float*>(smem), num, den, fresh != 0);
+}
+
+// prompts from this many tokens on are summed with matrix instructions (below it the one launch of k_decode is as quick)
 static constexpr int FM_DEC_MMA_MIN = 64;
-template <typename TIO, int DH> inline bool fm_decode_absorb_mma_applies(bool quad, bool has_q, int n_new) {
-  return sizeof(TIO) == 2 && DH == 64 && quad && !has_q && n_new >= FM_DEC_MMA_MIN;
+template <typename TIO, int DH, bool QUAD>
+int fm_absorb_launch_f32(const FastmaxDesc* d, const TRef<const TIO>& kr, const TRef<const TIO>& vr, int n_new, float* state, int fresh, fm_stream_t stream) {
+  const size_t lds = DecAbsF32Cfg<DH>::lds_bytes();
+  fm_allow_lds(reinterpret_cast<const void*>(&k_decode_absorb_f32<TIO, DH, QUAD>), lds);
+  FM_KERNEL_LAUNCH((k_decode_absorb_f32<TIO, DH, QUAD>), fm_dim3(DH / 4, d->bh), fm_dim3(FM_ABS_THREADS), lds, stream, kr, vr, n_new,
+                   d->inv_tau, state, fresh);
+  return fm_after_launch() ? FASTMAX_ERR_LAUNCH : FASTMAX_OK;
 }
 
 template <typename TIO, int DH>
 int fm_decode_run(const FastmaxDesc* d, const void* q, const void* k, const void* v, int n_new, float* state, void* o,
                   float* g, float* scratch, fm_stream_t stream) {
   const bool quad = d->p == 2 && d->a2 != 0.0f;
-  const int nblk = fm_decode_blocks(DH, quad);
   const TRef<const TIO> kr = fm_ref<const TIO>(static_cast<const TIO*>(k), d->sk), vr = fm_ref<const TIO>(static_cast<const TIO*>(v), d->sv);
   const TRef<const TIO> qr = q ? fm_ref<const TIO>(static_cast<const TIO*>(q), d->sq) : kr;
-  (void)scratch; (void)nblk;
-  if constexpr (sizeof(TIO) == 2 && DH == 64) {
-    if (fm_decode_absorb_mma_applies<TIO, DH>(quad, q != nullptr, n_new)) {
-      typedef DecAbsCfg<DH> C;
-      fm_allow_lds(reinterpret_cast<const void*>(&k_decode_absorb_mma<TIO, DH>), C::lds_bytes());
-      FM_KERNEL_LAUNCH((k_decode_absorb_mma<TIO, DH>), fm_dim3(DH / 4, d->bh), fm_dim3(C::NTH), C::lds_bytes(), stream, kr, vr,
-                       n_new, d->inv_tau, state);
-      return fm_after_launch() ? FASTMAX_ERR_LAUNCH : FASTMAX_OK;
+  (void)scratch;
+  const int fresh = !q && (d->flags & FASTMAX_FLAG_NEW_STATE) ? 1 : 0;
+  if (!q && n_new >= FM_DEC_MMA_MIN) {
+    if constexpr (sizeof(TIO) == 2 && DH == 64) {
+      if (quad) {
+        const size_t lds = DecAbsCfg<DH>::lds_bytes();
+        fm_allow_lds(reinterpret_cast<const void*>(&k_decode_absorb_mma<TIO, DH>), lds);
+        FM_KERNEL_LAUNCH((k_decode_absorb_mma<TIO, DH>), fm_dim3(DH / 4, d->bh), fm_dim3(FM_ABS_THREADS), lds, stream, kr, vr, n_new,
+                         d->inv_tau, state, fresh);
+        return fm_after_launch() ? FASTMAX_ERR_LAUNCH : FASTMAX_OK;
+      }
     }
+    if constexpr (sizeof(TIO) == 4 || DH != 64) {
+      if (quad) return fm_absorb_launch_f32<TIO, DH, true>(d, kr, vr, n_new, state, fresh, stream);
+    }
+    return fm_absorb_launch_f32<TIO, DH, false>(d, kr, vr, n_new, state, fresh, stream);
   }
   const TRef<TIO> orf = q ? fm_ref<TIO>(static_cast<TIO*>(o), d->so) : TRef<TIO>{nullptr, 0, 0, 0, 0, 0};
   const TRef<float> grf = q ? fm_ref<float>(g, d->sg) : TRef<float>{nullptr, 0, 0, 0, 0, 0};
   FM_KERNEL_LAUNCH((k_decode<TIO, DH>), fm_dim3(DH / 4, d->bh), fm_dim3(FM_DEC_THREADS), 0, stream, kr, vr, qr, n_new, quad ? 1 : 0,
-                   d->inv_tau, d->a0, d->a1, quad ? d->a2 : 0.0f, state, orf, grf, q ? 1 : 0);
+                   d->inv_tau, d->a0, d->a1, quad ? d->a2 : 0.0f, state, orf, grf, q ? 1 : 0, fresh);
   return fm_after_launch() ? FASTMAX_ERR_LAUNCH : FASTMAX_OK;
 }
 

@@ -444,6 +444,41 @@ def test_prompt_absorbed_with_matrix_instructions(lib):
     assert float(((one - small).abs() / small.abs().clamp_min(1e-30))[live].max()) < 5e-3
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("p", [1, 2])
+@pytest.mark.parametrize("d", [32, 64])
+@pytest.mark.parametrize("n", [64, 65, 127, 129, 255, 257, 700])
+def test_prompt_sums(lib, dtype, p, d, n):
+    """Prompts of 64 tokens and more against the state k_decode builds token after token; a new state in memory full of NaN against
+    one added to zeros, bit by bit; and rows that begin at odd elements.  fp32 products: n terms in another order, off by at
+    most n 2^-24 of the sum of their sizes, which is below 1e3 times a sum that is compared by itself."""
+    import math
+    from tests.parity import make_inputs
+    print(f"case prompt sums {dtype} p={p} d={d} n={n}", flush=True)
+    bh = 3
+    q, k, v, _ = make_inputs(bh, n, n, d, dtype, DEV, 11 + n)
+    kw = dict(inv_tau=1.0 / (8.0 * math.sqrt(d)), p=p, a0=1.0, a1=1.0, a2=0.5)
+    one, small = lib.decode_state(k, **kw), lib.decode_state(k, **kw)
+    new = torch.full_like(one, float("nan"))
+    lib.decode_absorb(k, v, one, **kw)
+    lib.decode_absorb(k, v, new, new=True, **kw)
+    for t0 in range(0, n, 48):
+        lib.decode_absorb(k[:, t0:t0 + 48], v[:, t0:t0 + 48], small, **kw)
+    few = torch.full_like(one, float("nan"))
+    lib.decode_absorb(k[:, :40], v[:, :40], few, new=True, **kw)              # below the threshold: k_decode
+    few2 = lib.decode_state(k, **kw)
+    lib.decode_absorb(k[:, :40], v[:, :40], few2, **kw)
+    odd = [torch.empty(bh, n, d + 1, dtype=dtype, device=DEV)[..., 1:].copy_(x) for x in (k, v)]
+    skew = lib.decode_state(k, **kw)
+    lib.decode_absorb(*odd, skew, **kw)
+    torch.cuda.synchronize()
+    assert torch.equal(new, one) and torch.equal(skew, one) and torch.equal(few, few2)
+    half = dtype == torch.bfloat16 and d == 64 and p == 2                     # operands rounded to _Float16
+    assert float((one - small).norm() / small.norm()) < (1e-4 if half else 1e-6)
+    live = small.abs() > 1e-3 * small.abs().max()
+    assert float(((one - small).abs() / small.abs().clamp_min(1e-30))[live].max()) < (5e-3 if half else n * 2.0 ** -24 * 1e3)
+
+
 
 @pytest.mark.parametrize("go_scale", [1e-7, 1e-4, 3e4])
 def test_upstream_gradient_of_any_size(lib, go_scale):

@@ -268,6 +268,18 @@ def test_prompt_absorbed_with_matrix_instructions(sim):
     assert float((s1 - s2).norm() / s2.norm()) < 1e-5
     live = s2.abs() > 1e-3 * s2.abs().max()
     assert float(((s1 - s2).abs() / s2.abs().clamp_min(1e-30))[live].max()) < 5e-3      # operands rounded to _Float16
+    # a new state in memory that is not clear; fp32 products (fp32 tensors, order 1, heads of 32), two tiles per group and a ragged one
+    for dtype, p, d, n in ((torch.bfloat16, 2, 64, 70), (torch.float32, 2, 64, 70), (torch.bfloat16, 1, 64, 195), (torch.float32, 2, 32, 66)):
+        q, k, v, _ = make_inputs(1, n, n, d, dtype, "cpu", 6)
+        kw = dict(inv_tau=1.0 / (8 * math.sqrt(d)), p=p, a0=1.0, a1=1.0, a2=0.5)
+        s1, s2 = sim.decode_state(k, **kw), sim.decode_state(k, **kw)
+        s3 = torch.full_like(s1, float("nan"))
+        sim.decode_absorb(k, v, s1, **kw)
+        sim.decode_absorb(k, v, s3, new=True, **kw)
+        for t0 in range(0, n, 48):
+            sim.decode_absorb(k[:, t0:t0 + 48], v[:, t0:t0 + 48], s2, **kw)
+        assert torch.equal(s1, s3)
+        assert float((s1 - s2).norm() / s2.norm()) < (1e-5 if dtype == torch.bfloat16 and p == 2 else 1e-6)
 
 
 def test_bf16_value_range_on_the_cpu(sim):
