@@ -219,6 +219,14 @@ typedef struct FastmaxNormDesc {
 size_t fastmax_normalize_stats_bytes(const FastmaxNormDesc* desc);
 int fastmax_normalize(const FastmaxNormDesc* desc, const void* x, void* y, float* stats,
                       void* hip_stream);
+/* The same pass over two tensors (q and k) in the same launches: equal but for n, strides and pointers. */
+int fastmax_normalize_pair(const FastmaxNormDesc* desc0, const void* x0, void* y0, float* stats0,
+                           const FastmaxNormDesc* desc1, const void* x1, void* y1, float* stats1, void* hip_stream);
+
+/* Up to three tensors of bh x n rows of desc->d elements (any d below dpad; sx) copied to rows of dpad (32, 64 or 128; sy) with
+ * zeros behind them, in one launch: head sizes the other entry points do not have.  The tensors agree in bh, d and dtype. */
+int fastmax_pad_features(const FastmaxNormDesc* const* descs, const void* const* x, void* const* y, int32_t count,
+                         int32_t dpad, void* hip_stream);
 
 /* Statistics for FastmaxNormFold: one read of x (desc->bh, n, d, dtype, sx are used), leaving
  * fastmax_maxnorm_stats_bytes(bh, n) bytes in `keys` (8-byte aligned device memory): per 256 tokens the
@@ -243,6 +251,10 @@ int fastmax_maxnorm_stats(const FastmaxNormDesc* desc0, const void* x0, void* ke
 size_t fastmax_normalize_backward_stats_bytes(const FastmaxNormDesc* desc);
 int fastmax_normalize_backward(const FastmaxNormDesc* desc, const void* x, const void* dy, void* dx,
                                float* stats, void* hip_stream);
+/* The same for two tensors in the same launches (see fastmax_normalize_pair). */
+int fastmax_normalize_backward_pair(const FastmaxNormDesc* desc0, const void* x0, const void* dy0, void* dx0, float* stats0,
+                                    const FastmaxNormDesc* desc1, const void* x1, const void* dy1, void* dx1,
+                                    float* stats1, void* hip_stream);
 
 /* The two element-wise steps the reference's forward_cuda carries switched off, for callers that switch
  * them on.  desc: bh, n, d, dtype; sx: strides of the input (and of `noise`), sy: strides of the output,

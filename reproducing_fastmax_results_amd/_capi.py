@@ -65,6 +65,7 @@ EXPORTS = (
     "fastmax_status_string", "fastmax_version", "fastmax_probe_mfma", "fastmax_probe_lds_transpose",
     "fastmax_key_rpe", "fastmax_output_noise", "fastmax_forward_static",
     "fastmax_maxnorm_stats", "fastmax_maxnorm_stats_bytes",
+    "fastmax_normalize_pair", "fastmax_normalize_backward_pair", "fastmax_pad_features",
     "fastmax_decode_state_bytes", "fastmax_decode_scratch_bytes", "fastmax_decode_absorb", "fastmax_decode_step",
 )
 BENCH_EXPORTS = ("fastmax_profile_begin", "fastmax_profile_end", "fastmax_probe_mfma_rate", "fastmax_probe_mix_rate")
@@ -147,6 +148,13 @@ class FastmaxLib:
         L.fastmax_normalize_backward.restype = C.c_int
         L.fastmax_normalize_backward_stats_bytes.argtypes = [C.POINTER(NormDesc)]
         L.fastmax_normalize_backward_stats_bytes.restype = C.c_size_t
+        L.fastmax_normalize_pair.argtypes = [C.POINTER(NormDesc), C.c_void_p, C.c_void_p, C.c_void_p] * 2 + [C.c_void_p]
+        L.fastmax_normalize_pair.restype = C.c_int
+        L.fastmax_normalize_backward_pair.argtypes = [C.POINTER(NormDesc), C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p] * 2 + [C.c_void_p]
+        L.fastmax_normalize_backward_pair.restype = C.c_int
+        L.fastmax_pad_features.argtypes = [C.POINTER(C.POINTER(NormDesc)), C.POINTER(C.c_void_p), C.POINTER(C.c_void_p), C.c_int32,
+                                           C.c_int32, C.c_void_p]
+        L.fastmax_pad_features.restype = C.c_int
         L.fastmax_maxnorm_stats_bytes.argtypes = [C.c_int32, C.c_int32]
         L.fastmax_maxnorm_stats_bytes.restype = C.c_size_t
         L.fastmax_maxnorm_stats.argtypes = [C.POINTER(NormDesc), C.c_void_p, C.c_void_p, C.POINTER(NormDesc), C.c_void_p,
@@ -385,6 +393,43 @@ class FastmaxLib:
                                                  self._stream(x))
         self.check(st, "fastmax_normalize_backward")
         return dx
+
+    def normalize_pair(self, x0, x1, dy0=None, dy1=None, *, centre=0, max_norm=True, scale=1.0):
+        """normalize() of two tensors in common launches; with dy0 and dy1 normalize_backward() of both."""
+        args, keep = [], []
+        for x, dy in ((x0, dy0), (x1, dy1)):
+            nd = NormDesc()
+            nd.bh, nd.n, nd.d = _dims(x)
+            nd.dtype = _dtype_code(x)
+            nd.centre, nd.max_norm, nd.scale = int(centre), int(bool(max_norm)), float(scale)
+            x = x.contiguous()
+            out = torch.empty_like(x)
+            nd.sx, nd.sy = _strides(x), _strides(out if dy is None else dy)
+            size = self.lib.fastmax_normalize_stats_bytes if dy is None else self.lib.fastmax_normalize_backward_stats_bytes
+            stats = torch.empty(max(size(C.byref(nd)) // 4, 1), dtype=torch.float32, device=x.device)
+            args += [C.byref(nd), x.data_ptr(), *([] if dy is None else [dy.data_ptr()]), out.data_ptr(), stats.data_ptr()]
+            keep.append((nd, x, out, stats))
+        fn = self.lib.fastmax_normalize_pair if dy0 is None else self.lib.fastmax_normalize_backward_pair
+        self.check(fn(*args, self._stream(x0)), "fastmax_normalize_pair")
+        return keep[0][2], keep[1][2]
+
+    def pad_features(self, xs, dpad):
+        """Views (bh, n, d) or (b, h, n, d), d < dpad, zero-padded to dpad features in one launch."""
+        descs, outs = [], []
+        for x in xs:
+            nd = NormDesc()
+            nd.bh, nd.n, nd.d = _dims(x)
+            nd.dtype = _dtype_code(x)
+            out = torch.empty(*x.shape[:-1], dpad, dtype=x.dtype, device=x.device)
+            nd.sx, nd.sy = _strides(x), _strides(out)
+            descs.append(nd)
+            outs.append(out)
+        n = len(descs)
+        st = self.lib.fastmax_pad_features((C.POINTER(NormDesc) * n)(*[C.pointer(d) for d in descs]),
+                                           (C.c_void_p * n)(*[x.data_ptr() for x in xs]),
+                                           (C.c_void_p * n)(*[o.data_ptr() for o in outs]), n, dpad, self._stream(xs[0]))
+        self.check(st, "fastmax_pad_features")
+        return outs
 
     def _pointwise_desc(self, x, out):
         nd = NormDesc()

@@ -34,7 +34,8 @@ __all__ = [
 ]
 
 CENTRE_NONE, CENTRE_FEATURE, CENTRE_TOKEN = 0, 1, 2
-_NORM_OFF, _GRAD_OF_NORMALISED, _GRAD_OF_RAW = 0, 1, 2   # the binding's `attention`: max-norm scaling of q and k, and which gradients
+# the binding's `attention`: max-norm scaling of q and k (centred over tokens before it, for the last), and which gradients
+_NORM_OFF, _GRAD_OF_NORMALISED, _GRAD_OF_RAW, _CENTRED = 0, 1, 2, 3
 
 
 _HEAD_SIZES = (32, 64)      # what every kernel is built for
@@ -352,11 +353,8 @@ def fastmax(q, k, v, mask=None, denum_term=8, normalize=0, p=1, create_attn_matr
         return torch.matmul(a, v.float()).to(q.dtype), a
     masked = False if mask is None else bool(mask)      # reference: `if mask is None or not mask` -> unmasked
     if normalize == 1:
-        q = FastmaxNormalize.apply(q, CENTRE_TOKEN, 1.0)
-        k = FastmaxNormalize.apply(k, CENTRE_TOKEN, 1.0)
-        temperature = 1.0
-    else:
-        temperature = denum_term * math.sqrt(d)
+        return _ext.attention(q, k, v, masked, _CENTRED, 1.0, 1.0, 1.0, 0.5, 1.0, int(p))
+    temperature = denum_term * math.sqrt(d)
     return FASTMultiHeadAttention_Function.apply(q, k, v, None, None, masked, 0.0, False, temperature,
                                                  1.0, 1.0, 0.5, 1.0, int(p))
 

@@ -998,7 +998,19 @@ size_t fastmax_normalize_stats_bytes(const FastmaxNormDesc* desc) {
 
 int fastmax_normalize(const FastmaxNormDesc* desc, const void* x, void* y, float* stats, void* hip_stream) {
   ProfScope prof(FM_K_NORM, static_cast<fm_stream_t>(hip_stream));   // the whole pass (its kernels together)
-  return fm_normalize_dispatch(desc, x, y, stats, static_cast<fm_stream_t>(hip_stream));
+  return fm_normalize_dispatch(desc, x, y, stats, nullptr, nullptr, nullptr, nullptr, static_cast<fm_stream_t>(hip_stream));
+}
+
+int fastmax_normalize_pair(const FastmaxNormDesc* desc0, const void* x0, void* y0, float* stats0, const FastmaxNormDesc* desc1,
+                           const void* x1, void* y1, float* stats1, void* hip_stream) {
+  if (!desc1) return FASTMAX_ERR_NULL;
+  ProfScope prof(FM_K_NORM, static_cast<fm_stream_t>(hip_stream));
+  return fm_normalize_dispatch(desc0, x0, y0, stats0, desc1, x1, y1, stats1, static_cast<fm_stream_t>(hip_stream));
+}
+
+int fastmax_pad_features(const FastmaxNormDesc* const* descs, const void* const* x, void* const* y, int32_t count, int32_t dpad,
+                         void* hip_stream) {
+  return fm_pad_dispatch(descs, x, y, count, dpad, static_cast<fm_stream_t>(hip_stream));
 }
 
 int fastmax_key_rpe(const FastmaxNormDesc* desc, const void* k, const float* rpe, void* k_out, float temperature,
@@ -1091,7 +1103,16 @@ size_t fastmax_normalize_backward_stats_bytes(const FastmaxNormDesc* desc) {
 int fastmax_normalize_backward(const FastmaxNormDesc* desc, const void* x, const void* dy, void* dx, float* stats,
                                void* hip_stream) {
   ProfScope prof(FM_K_NORM, static_cast<fm_stream_t>(hip_stream));
-  return fm_normalize_bwd_dispatch(desc, x, dy, dx, stats, static_cast<fm_stream_t>(hip_stream));
+  return fm_normalize_bwd_dispatch(desc, x, dy, dx, stats, nullptr, nullptr, nullptr, nullptr, nullptr,
+                                   static_cast<fm_stream_t>(hip_stream));
+}
+
+int fastmax_normalize_backward_pair(const FastmaxNormDesc* desc0, const void* x0, const void* dy0, void* dx0, float* stats0,
+                                    const FastmaxNormDesc* desc1, const void* x1, const void* dy1, void* dx1, float* stats1,
+                                    void* hip_stream) {
+  if (!desc1) return FASTMAX_ERR_NULL;
+  ProfScope prof(FM_K_NORM, static_cast<fm_stream_t>(hip_stream));
+  return fm_normalize_bwd_dispatch(desc0, x0, dy0, dx0, stats0, desc1, x1, dy1, dx1, stats1, static_cast<fm_stream_t>(hip_stream));
 }
 
 int fastmax_probe_mfma(float* out_f16, float* out_f32, void* hip_stream) {

@@ -430,51 +430,88 @@ std::tuple<torch::Tensor, torch::Tensor> decode_step(torch::Tensor q_, torch::Te
   return {o, g};
 }
 
-// y = scale * (x - centre) / max_n ||x_n - centre||  (see fastmax_normalize in the C header)
-torch::Tensor normalize(torch::Tensor x_, int64_t centre, bool max_norm, double scale) {
-  const View x = view_of(x_, "x");
-  FM_CHECK_CUDA(x.t);
+// One tensor's part of the normalisation passes: tensors, descriptor and scratch.
+struct NormPass {
+  torch::Tensor in, dy, out, stats;
   FastmaxNormDesc nd{};
-  nd.bh = static_cast<int32_t>(x.bh); nd.n = static_cast<int32_t>(x.n); nd.d = static_cast<int32_t>(x.d);
-  nd.dtype = dtype_code(x.t); nd.centre = static_cast<int32_t>(centre); nd.max_norm = max_norm ? 1 : 0;
-  nd.scale = float(scale);
-  torch::Tensor y = empty_like_layout(x.t, x.n, x.t.scalar_type());
-  nd.sx = x.s; nd.sy = view_of(y, "y").s;
-  torch::Tensor stats = torch::empty({int64_t(fastmax_normalize_stats_bytes(&nd) / sizeof(float))},
-                                     x.t.options().dtype(torch::kFloat32));
-  check_status(fastmax_normalize(&nd, x.t.data_ptr(), y.data_ptr(), stats.data_ptr<float>(), stream_of(x.t)),
-               "fastmax_normalize");
-  return y;
+  NormPass(const View& x, int64_t centre, bool max_norm, double scale) : in(x.t) {
+    FM_CHECK_CUDA(x.t);
+    nd.bh = static_cast<int32_t>(x.bh); nd.n = static_cast<int32_t>(x.n); nd.d = static_cast<int32_t>(x.d);
+    nd.dtype = dtype_code(x.t); nd.centre = static_cast<int32_t>(centre); nd.max_norm = max_norm ? 1 : 0;
+    nd.scale = float(scale);
+    nd.sx = x.s;
+  }
+  void scratch(size_t bytes) { stats = torch::empty({int64_t(bytes / 4 + 1)}, in.options().dtype(torch::kFloat32)); }
+  bool shares_launches(const NormPass& o) const { return nd.bh == o.nd.bh && nd.d == o.nd.d && nd.dtype == o.nd.dtype; }
+};
+
+NormPass forward_pass(const torch::Tensor& x_, int64_t centre, bool max_norm, double scale) {
+  const View x = view_of(x_, "x");
+  NormPass p(x, centre, max_norm, scale);
+  p.out = empty_like_layout(x.t, x.n, x.t.scalar_type());
+  p.nd.sy = view_of(p.out, "y").s;
+  p.scratch(fastmax_normalize_stats_bytes(&p.nd));
+  return p;
 }
 
-// gradient of normalize() with respect to x (see fastmax_normalize_backward in the C header)
-torch::Tensor normalize_backward(torch::Tensor x_, torch::Tensor dy_, int64_t centre, bool max_norm, double scale) {
-  const View x = view_of(x_, "x");
-  const View dy = view_of(dy_, "dy");
-  FM_CHECK_CUDA(x.t);
+NormPass backward_pass(const torch::Tensor& x_, const torch::Tensor& dy_, int64_t centre, bool max_norm, double scale) {
+  const View x = view_of(x_, "x"), dy = view_of(dy_, "dy");
+  NormPass p(x, centre, max_norm, scale);
   FM_CHECK_CUDA(dy.t);
   TORCH_CHECK(dy.bh == x.bh && dy.n == x.n && dy.d == x.d && dy.t.scalar_type() == x.t.scalar_type(),
               "dy must have x's shape and dtype");
-  FastmaxNormDesc nd{};
-  nd.bh = static_cast<int32_t>(x.bh); nd.n = static_cast<int32_t>(x.n); nd.d = static_cast<int32_t>(x.d);
-  nd.dtype = dtype_code(x.t); nd.centre = static_cast<int32_t>(centre); nd.max_norm = max_norm ? 1 : 0;
-  nd.scale = float(scale);
+  p.dy = dy.t;
   // dx shares x's strides: lay it out like x, and if that is not possible take a packed copy of x
-  torch::Tensor xs = x.t;
-  torch::Tensor dx = empty_like_layout(xs, x.n, xs.scalar_type());
-  View dxv = view_of(dx, "dx");
-  View xv = x;
+  p.out = empty_like_layout(x.t, x.n, x.t.scalar_type());
+  const View dxv = view_of(p.out, "dx");
   if (dxv.s.bh != x.s.bh || dxv.s.n != x.s.n || dxv.s.b != x.s.b || dxv.s.heads != x.s.heads) {
-    xs = x.t.contiguous();
-    xv = view_of(xs, "x");
-    dx = torch::empty_like(xs);
+    p.in = x.t.contiguous();
+    p.nd.sx = view_of(p.in, "x").s;
+    p.out = torch::empty_like(p.in);
   }
-  nd.sx = xv.s; nd.sy = dy.s;
-  const size_t nbytes = fastmax_normalize_backward_stats_bytes(&nd);
-  torch::Tensor stats = torch::empty({int64_t(nbytes / 4 + 1)}, x.t.options().dtype(torch::kFloat32));
-  check_status(fastmax_normalize_backward(&nd, xs.data_ptr(), dy.t.data_ptr(), dx.data_ptr(), stats.data_ptr<float>(),
-                                          stream_of(x.t)), "fastmax_normalize_backward");
-  return dx;
+  p.nd.sy = dy.s;
+  p.scratch(fastmax_normalize_backward_stats_bytes(&p.nd));
+  return p;
+}
+
+void run(NormPass& p) {
+  void* stream = stream_of(p.in);
+  if (!p.dy.defined())
+    check_status(fastmax_normalize(&p.nd, p.in.data_ptr(), p.out.data_ptr(), p.stats.data_ptr<float>(), stream), "fastmax_normalize");
+  else
+    check_status(fastmax_normalize_backward(&p.nd, p.in.data_ptr(), p.dy.data_ptr(), p.out.data_ptr(), p.stats.data_ptr<float>(),
+                                            stream), "fastmax_normalize_backward");
+}
+
+// two passes of the same kind, in common launches where the shapes allow
+void run(NormPass& a, NormPass& b) {
+  if (!a.shares_launches(b)) {
+    run(a);
+    run(b);
+    return;
+  }
+  void* stream = stream_of(a.in);
+  float *sa = a.stats.data_ptr<float>(), *sb = b.stats.data_ptr<float>();
+  if (!a.dy.defined())
+    check_status(fastmax_normalize_pair(&a.nd, a.in.data_ptr(), a.out.data_ptr(), sa, &b.nd, b.in.data_ptr(), b.out.data_ptr(), sb,
+                                        stream), "fastmax_normalize_pair");
+  else
+    check_status(fastmax_normalize_backward_pair(&a.nd, a.in.data_ptr(), a.dy.data_ptr(), a.out.data_ptr(), sa, &b.nd, b.in.data_ptr(),
+                                                 b.dy.data_ptr(), b.out.data_ptr(), sb, stream), "fastmax_normalize_backward_pair");
+}
+
+// y = scale * (x - centre) / max_n ||x_n - centre||  (see fastmax_normalize in the C header)
+torch::Tensor normalize(torch::Tensor x, int64_t centre, bool max_norm, double scale) {
+  NormPass p = forward_pass(x, centre, max_norm, scale);
+  run(p);
+  return p.out;
+}
+
+// gradient of normalize() with respect to x (see fastmax_normalize_backward in the C header)
+torch::Tensor normalize_backward(torch::Tensor x, torch::Tensor dy, int64_t centre, bool max_norm, double scale) {
+  NormPass p = backward_pass(x, dy, centre, max_norm, scale);
+  run(p);
+  return p.out;
 }
 
 // k + temperature * rpe[(l + n) % (2n - 1)]  (see fastmax_key_rpe in the C header)
@@ -522,19 +559,62 @@ constexpr int64_t kWideHead = 128;                     // bf16 attention alone (
 // t itself, or a copy zero-padded along the feature axis to the next head size the kernels are built for.  Zero features
 // change neither q.k nor any norm, padded value columns come out as zero output columns, and the padded columns of every
 // gradient are zero as well, so callers pad on the way in and slice on the way out.
-torch::Tensor pad_features(const torch::Tensor& t, bool wide) {
+int64_t head_size(const torch::Tensor& t, bool wide) {
   const int64_t d = t.size(-1);
   wide = wide && t.scalar_type() == torch::kBFloat16;
-  for (int64_t size : {kHeadSizes[0], kHeadSizes[1], wide ? kWideHead : int64_t(0)}) {
-    if (d == size) return t;
-    if (d < size) return at::constant_pad_nd(t, {0, size - d});
-  }
+  for (int64_t size : {kHeadSizes[0], kHeadSizes[1], wide ? kWideHead : int64_t(0)})
+    if (d <= size) return size;
   TORCH_CHECK(false, "fastmax: unsupported head size ", d, " for ", t.scalar_type(), " (the kernels cover up to ", kHeadSizes[1],
               ", attention on bfloat16 tensors up to ", kWideHead, ")");
 }
+// `ts` (q, k and v, or dO), each padded where it needs it; those that agree in batch*heads, head size and type in one launch.
+void pad_features(std::initializer_list<torch::Tensor*> ts, bool wide) {
+  std::vector<View> views;
+  std::vector<FastmaxNormDesc> nds;
+  std::vector<torch::Tensor*> todo;
+  int64_t size = 0;
+  auto flush = [&]() {
+    const FastmaxNormDesc* descs[3];
+    const void* x[3];
+    void* y[3];
+    std::vector<torch::Tensor> out;
+    for (size_t i = 0; i < todo.size(); ++i) {
+      const torch::Tensor& t = views[i].t;
+      std::vector<int64_t> shape = t.sizes().vec();
+      shape.back() = size;
+      out.push_back(torch::empty(shape, t.options()));
+      nds[i].sy = view_of(out[i], "padded").s;
+      descs[i] = &nds[i]; x[i] = t.data_ptr(); y[i] = out[i].data_ptr();
+    }
+    if (!todo.empty())
+      check_status(fastmax_pad_features(descs, x, y, int32_t(todo.size()), int32_t(size), stream_of(views[0].t)), "fastmax_pad_features");
+    for (size_t i = 0; i < todo.size(); ++i) *todo[i] = out[i];
+    views.clear(); nds.clear(); todo.clear();
+  };
+  for (torch::Tensor* t : ts) {
+    const int64_t want = head_size(*t, wide);
+    if (t->size(-1) == want) continue;
+    if (t->numel() == 0) {                               // no rows or no features: nothing for a kernel to read
+      *t = at::constant_pad_nd(*t, {0, want - t->size(-1)});
+      continue;
+    }
+    View v = view_of(*t, "tensor");
+    FM_CHECK_CUDA(v.t);
+    FastmaxNormDesc nd{};
+    nd.bh = static_cast<int32_t>(v.bh); nd.n = static_cast<int32_t>(v.n); nd.d = static_cast<int32_t>(v.d);
+    nd.dtype = dtype_code(v.t); nd.sx = v.s;
+    if (!todo.empty() && (nds[0].bh != nd.bh || nds[0].d != nd.d || nds[0].dtype != nd.dtype || views[0].t.device() != v.t.device())) flush();
+    size = want;
+    views.push_back(std::move(v)); nds.push_back(nd); todo.push_back(t);
+  }
+  flush();
+}
 torch::Tensor first_features(const torch::Tensor& t, int64_t d) { return t.size(-1) == d ? t : t.narrow(-1, 0, d); }
 
-enum { kNormNone = 0, kNormGradOfNormalised = 1, kNormGradOfRaw = 2 };
+// kNormCentred: q and k centred over their tokens, then max-norm scaled, in passes of their own; gradients of the raw tensors
+// (the score-function front, score_function.py:40-55)
+enum { kNormNone = 0, kNormGradOfNormalised = 1, kNormGradOfRaw = 2, kNormCentred = 3 };
+constexpr int64_t kCentreToken = 2;
 
 struct AttnConfig {
   bool mask;
@@ -546,7 +626,7 @@ struct AttnConfig {
 // More keys than queries under the causal mask run in two parts that would share one Jacobian: no fold there.
 bool fold_possible(const torch::Tensor& q, const torch::Tensor& k, bool mask) { return !(mask && k.size(-2) > q.size(-2)); }
 
-struct AttnResult { torch::Tensor q, k, v, o, g, saved, qk, kk; bool fold = false, self = false; };
+struct AttnResult { torch::Tensor q, k, v, o, g, saved, qk, kk, rq, rk; bool fold = false, self = false; };   // rq, rk: kNormCentred, the raw tensors
 
 // q, k, v in any head size; `save`: a backward follows
 AttnResult attention_forward(const torch::Tensor& q_, const torch::Tensor& k_, const torch::Tensor& v_, const AttnConfig& c, bool save) {
@@ -557,10 +637,16 @@ AttnResult attention_forward(const torch::Tensor& q_, const torch::Tensor& k_, c
   TORCH_CHECK(c.norm != kNormGradOfRaw || fold_possible(q_, k_, c.mask), "fastmax: no folded normalisation for causal attention with "
               "more keys than queries (normalise q and k with FastmaxNormalize first)");
   AttnResult r;
-  const bool wide = c.norm != kNormGradOfRaw;          // the folded kernels stop at 64
-  r.q = pad_features(q_, wide); r.k = pad_features(k_, wide); r.v = pad_features(v_, wide);
+  const bool wide = c.norm < kNormGradOfRaw;           // the folded kernels and the centring ones stop at 64
+  r.q = q_; r.k = k_; r.v = v_;
+  pad_features({&r.q, &r.k, &r.v}, wide);
   NormArgs na;
-  if (c.norm != kNormNone) {
+  if (c.norm == kNormCentred) {
+    r.rq = r.q; r.rk = r.k;
+    NormPass a = forward_pass(r.rq, kCentreToken, true, c.lim), b = forward_pass(r.rk, kCentreToken, true, c.lim);
+    run(a, b);
+    r.q = a.out; r.k = b.out;
+  } else if (c.norm != kNormNone) {
     if (r.q.size(-1) > kHeadSizes[1]) {
       // no normalisation kernels at that width: the scaling itself (lim * x / max_n ||x_n||, transformer/model.py:97-102)
       // as tensor operations
@@ -589,7 +675,7 @@ struct AttentionNode : public torch::autograd::Function<AttentionNode> {
   static torch::Tensor forward(torch::autograd::AutogradContext* ctx, const torch::Tensor& q, const torch::Tensor& k,
                                const torch::Tensor& v, const AttnConfig& c) {
     AttnResult r = attention_forward(q, k, v, c, true);
-    ctx->save_for_backward({r.q, r.k, r.v, r.o, r.g, r.saved, r.qk, r.kk});
+    ctx->save_for_backward({r.q, r.k, r.v, r.o, r.g, r.saved, r.qk, r.kk, r.rq, r.rk});
     ctx->saved_data["d"] = q.size(-1);
     ctx->saved_data["ip"] = std::vector<int64_t>{c.norm, c.p, r.fold, r.self, c.mask};
     ctx->saved_data["fp"] = std::vector<double>{c.inv_tau, c.a0, c.a1, c.a2, c.lim};
@@ -601,10 +687,16 @@ struct AttentionNode : public torch::autograd::Function<AttentionNode> {
     const std::vector<int64_t> ip = ctx->saved_data["ip"].toIntVector();
     const bool fold = ip[2] != 0, mask = ip[4] != 0;
     const std::vector<double> fp = ctx->saved_data["fp"].toDoubleVector();
-    const torch::Tensor go = s[0].size(-1) == d ? grads[0] : pad_features(grads[0], true);
+    torch::Tensor go = grads[0];
+    if (s[0].size(-1) != d) pad_features({&go}, true);
     NormArgs na{s[6], s[7], fp[4], ip[0] == kNormGradOfRaw, ip[3] != 0};
     std::vector<torch::Tensor> r = backward_any(s[0], s[1], s[2], s[3], s[4], go, &s[5], mask, fp[0], fp[1], fp[2], fp[3], ip[1], 0,
                                                 FASTMAX_FLAG_SAVE_FOR_BACKWARD, fold ? &na : nullptr);
+    if (ip[0] == kNormCentred && (ctx->needs_input_grad(0) || ctx->needs_input_grad(1))) {
+      NormPass a = backward_pass(s[8], r[0], kCentreToken, true, fp[4]), b = backward_pass(s[9], r[1], kCentreToken, true, fp[4]);
+      run(a, b);
+      r[0] = a.out; r[1] = b.out;
+    }
     return {first_features(r[0], d), first_features(r[1], d), first_features(r[2], d), torch::Tensor()};
   }
 };

@@ -23,7 +23,7 @@ static constexpr float FM_NORM_FLOOR = 1e-30f;
 // forward scratch per batch*head (floats): [0], [1] unused; [2 .. 2+d) token mean; then one largest
 // squared norm per workgroup of k_norm_maxnorm; then, with the token-mean centring, d column sums per
 // workgroup of k_norm_colsum
-inline int fm_norm_blocks(int n) { return (n + 64 * FM_NORM_NP - 1) / (64 * FM_NORM_NP); }
+FM_HOST_DEVICE inline int fm_norm_blocks(int n) { return (n + 64 * FM_NORM_NP - 1) / (64 * FM_NORM_NP); }
 inline int64_t fm_norm_stride(int dh, int n, int centre) {
   const int64_t nb = fm_norm_blocks(n);
   return (2 + int64_t(dh) + nb + (centre == 2 ? nb * dh : 0) + 1) / 2 * 2;
@@ -59,16 +59,28 @@ FM_DEVICE void fm_norm_load_centred(const TIO* row, int d0, int centre, const fl
   fm_norm_centre<DH>(v, d0, centre, mean);
 }
 
-// Column sums over the workgroup's 64 * FM_NORM_NP tokens -> out[bh][block][DH]; k_norm_colfinal adds the
-// blocks in a fixed order and divides.  grid (blocks, bh, tensors) and (bh, tensors).
-template <typename TIO, int DH>
-FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_norm_colsum(TRef<const TIO> x0, TRef<const TIO> x1, int n, float* FM_RESTRICT out,
-                                                   int64_t out_stride) {
+// One tensor of a pass.  q and k go through the same launches (the passes are short chains of small kernels: 15 heads of 777 tokens
+// keep 60 workgroups busy for 2 to 10 us a launch on a chip of 256 CUs, and two tensors take hardly longer than one).
+template <typename TIO> struct NormJob {
+  TRef<const TIO> x, dy;               // dy: backward only
+  TRef<TIO> out;                       // y | dx
+  float* stats; int64_t stride;        // scratch and its floats per batch*head
+  float *sums, *mean;                  // within it: the column sums and means of x (and of dy, behind them) of batch*head 0
+  int n;
+};
+
+// Column sums over the workgroup's 64 * FM_NORM_NP tokens -> sums[bh][tensor][block][DH]; k_norm_colfinal adds the
+// blocks in a fixed order and divides.  grid (blocks, bh, jobs * TENSORS) and (bh, jobs * TENSORS); TENSORS: x alone, or x and dy.
+template <typename TIO, int DH, int TENSORS>
+FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_norm_colsum(NormJob<TIO> j0, NormJob<TIO> j1) {
   constexpr int EPT = DH / 4, NP = FM_NORM_NP;
   FM_SHARED float part[64 * (DH + 1)];
-  const int tid = FM_TID_X, bh = FM_BID_Y;
-  const TRef<const TIO> x = FM_BID_Z ? x1 : x0;     // grid z: which tensor
-  out += int64_t(FM_BID_Z) * FM_GDIM_X * DH;
+  const int tid = FM_TID_X, bh = FM_BID_Y, which = int(FM_BID_Z) % TENSORS;
+  const NormJob<TIO> J = int(FM_BID_Z) >= TENSORS ? j1 : j0;
+  const int n = J.n, nblk = fm_norm_blocks(n);
+  if (int(FM_BID_X) >= nblk) return;                // the shorter tensor of the two (workgroup-uniform; here and below)
+  const TRef<const TIO> x = which ? J.dy : J.x;
+  float* FM_RESTRICT out = J.sums + bh * J.stride + int64_t(which) * nblk * DH;
   const int tok0 = FM_BID_X * 64 * NP + (tid >> 2), d0 = (tid & 3) * EPT;
   float v[NP][EPT];
 #pragma unroll
@@ -88,17 +100,18 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_norm_colsum(TRef<const TIO> x0, TRef<cons
   if (tid < DH) {
     float a = 0.f;
     for (int r = 0; r < 64; ++r) a += part[r * (DH + 1) + tid];
-    out[bh * out_stride + int64_t(FM_BID_X) * DH + tid] = a;
+    out[int64_t(FM_BID_X) * DH + tid] = a;
   }
 }
-template <int DH>
-FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_norm_colfinal(const float* FM_RESTRICT sums, int64_t sums_stride, int nblk, int n,
-                                                     float* FM_RESTRICT mean, int64_t mean_stride) {
+template <typename TIO, int DH, int TENSORS>
+FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_norm_colfinal(NormJob<TIO> j0, NormJob<TIO> j1) {
   constexpr int G = 256 / DH;                 // groups of DH threads, each takes every G-th block
   FM_SHARED float part[256];
-  const int tid = FM_TID_X, bh = FM_BID_X, which = FM_BID_Y;     // which: tensor (sums and means of several lie side by side)
+  const int tid = FM_TID_X, bh = FM_BID_X, which = int(FM_BID_Y) % TENSORS;
+  const NormJob<TIO> J = int(FM_BID_Y) >= TENSORS ? j1 : j0;
+  const int n = J.n, nblk = fm_norm_blocks(n);
   const int g = tid / DH, f = tid % DH;
-  sums += bh * sums_stride + int64_t(which) * nblk * DH;
+  const float* FM_RESTRICT sums = J.sums + bh * J.stride + int64_t(which) * nblk * DH;
   float a = 0.f;
   int b = g;
   for (; b + 3 * G < nblk; b += 4 * G) {      // four loads in flight
@@ -113,18 +126,22 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_norm_colfinal(const float* FM_RESTRICT su
     float t = 0.f;
 #pragma unroll
     for (int i = 0; i < G; ++i) t += part[i * DH + tid];
-    mean[bh * mean_stride + which * DH + tid] = t / float(n);
+    J.mean[bh * J.stride + which * DH + tid] = t / float(n);
   }
 }
 
-// grid (ceil(n / (64 * FM_NORM_NP)), bh); four threads per token
+// grid (ceil(n / (64 * FM_NORM_NP)), bh, jobs); four threads per token
 template <typename TIO, int DH>
-FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_norm_maxnorm(TRef<const TIO> x, int n, int centre, float* FM_RESTRICT stats, int64_t stride) {
+FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_norm_maxnorm(NormJob<TIO> j0, NormJob<TIO> j1, int centre) {
   constexpr int EPT = DH / 4, NP = FM_NORM_NP;
   FM_SHARED float wmax[4];
   const int tid = FM_TID_X, bh = FM_BID_Y;
+  const NormJob<TIO> J = FM_BID_Z ? j1 : j0;
+  const TRef<const TIO> x = J.x;
+  const int n = J.n;
+  if (int(FM_BID_X) >= fm_norm_blocks(n)) return;
   const int tok0 = FM_BID_X * 64 * NP + (tid >> 2), d0 = (tid & 3) * EPT;
-  float* st = stats + bh * stride;
+  float* st = J.stats + bh * J.stride;
   float v[NP][EPT];
   // every lane takes part in the shuffles; rows past the end re-read the last row and count as zero
 #pragma unroll
@@ -151,12 +168,15 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_norm_maxnorm(TRef<const TIO> x, int n, in
 }
 
 template <typename TIO, int DH>
-FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_norm_apply(TRef<const TIO> x, TRef<TIO> y, int n, int centre, int max_norm, float scale,
-                                                  const float* FM_RESTRICT stats, int64_t stride) {
+FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_norm_apply(NormJob<TIO> j0, NormJob<TIO> j1, int centre, int max_norm, float scale) {
   constexpr int EPT = DH / 4, NP = FM_NORM_NP;
   const int tid = FM_TID_X, bh = FM_BID_Y;
+  const NormJob<TIO> J = FM_BID_Z ? j1 : j0;
+  const TRef<const TIO> x = J.x;
+  const int n = J.n, nblk = fm_norm_blocks(n);
+  if (int(FM_BID_X) >= nblk) return;
   const int tok0 = FM_BID_X * 64 * NP + (tid >> 2), d0 = (tid & 3) * EPT;
-  const float* st = stats ? stats + bh * stride : nullptr;
+  const float* st = J.stats ? J.stats + bh * J.stride : nullptr;
   float v[NP][EPT];
 #pragma unroll
   for (int p = 0; p < NP; ++p) {
@@ -166,7 +186,6 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_norm_apply(TRef<const TIO> x, TRef<TIO> y
   float f = scale;
   if (max_norm) {
     // the largest of the workgroups' maxima: every lane takes a share, a butterfly joins them
-    const int nblk = int(FM_GDIM_X);
     float m2 = 0.f;
     for (int b = tid & 63; b < nblk; b += 64) m2 = fm_fmaxf(m2, st[2 + DH + b]);
 #pragma unroll
@@ -181,31 +200,42 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_norm_apply(TRef<const TIO> x, TRef<TIO> y
 #pragma unroll
       for (int j = 0; j < EPT; ++j) v[p][j] *= f;
 #pragma unroll
-      for (int j = 0; j < EPT; j += 8) IO<TIO>::st8(y.base(bh) + int64_t(tok) * y.s_n + d0 + j, &v[p][j]);
+      for (int j = 0; j < EPT; j += 8) IO<TIO>::st8(J.out.base(bh) + int64_t(tok) * J.out.s_n + d0 + j, &v[p][j]);
     }
   }
 }
 
+// One tensor (d1 null) or two in the same launches.  q and k of 15 heads of 777 tokens, heads of 64, fp32: 20 us instead of 37 in twice
+// the launches; their backward (fm_normalize_bwd_run) 24 instead of 43.
 template <typename TIO, int DH>
-int fm_normalize_run(const FastmaxNormDesc* d, const void* x, void* y, float* stats, fm_stream_t stream) {
-  const TRef<const TIO> xr = fm_ref<const TIO>(static_cast<const TIO*>(x), d->sx);
-  const TRef<TIO> yr = fm_ref<TIO>(static_cast<TIO*>(y), d->sy);
-  const fm_dim3 grid((d->n + 64 * FM_NORM_NP - 1) / (64 * FM_NORM_NP), d->bh);
-  const int64_t stride = fm_norm_stride(DH, d->n, d->centre);
-  if (d->centre == 2) {
-    float* sums = stats + 2 + DH + grid.x;
-    FM_KERNEL_LAUNCH((k_norm_colsum<TIO, DH>), grid, fm_dim3(256), 0, stream, xr, xr, d->n, sums, stride);
-    FM_KERNEL_LAUNCH((k_norm_colfinal<DH>), fm_dim3(d->bh), fm_dim3(256), 0, stream, sums, stride, int(grid.x), d->n, stats + 2,
-                     stride);
+int fm_normalize_run(const FastmaxNormDesc* d0, const void* x0, void* y0, float* stats0, const FastmaxNormDesc* d1, const void* x1,
+                     void* y1, float* stats1, fm_stream_t stream) {
+  auto job = [](const FastmaxNormDesc* d, const void* x, void* y, float* stats) {
+    NormJob<TIO> j{};
+    j.x = fm_ref<const TIO>(static_cast<const TIO*>(x), d->sx);
+    j.out = fm_ref<TIO>(static_cast<TIO*>(y), d->sy);
+    j.n = d->n; j.stats = stats; j.stride = fm_norm_stride(DH, d->n, d->centre);
+    if (stats) { j.mean = stats + 2; j.sums = stats + 2 + DH + fm_norm_blocks(d->n); }
+    return j;
+  };
+  const NormJob<TIO> j0 = job(d0, x0, y0, stats0), j1 = d1 ? job(d1, x1, y1, stats1) : j0;
+  const int jobs = d1 ? 2 : 1, nb = fm_norm_blocks(j0.n > j1.n ? j0.n : j1.n);
+  const fm_dim3 grid(nb, d0->bh, jobs);
+  if (d0->centre == 2) {
+    FM_KERNEL_LAUNCH((k_norm_colsum<TIO, DH, 1>), grid, fm_dim3(256), 0, stream, j0, j1);
+    FM_KERNEL_LAUNCH((k_norm_colfinal<TIO, DH, 1>), fm_dim3(d0->bh, jobs), fm_dim3(256), 0, stream, j0, j1);
   }
-  if (d->max_norm)
-    FM_KERNEL_LAUNCH((k_norm_maxnorm<TIO, DH>), grid, fm_dim3(256), 0, stream, xr, d->n, d->centre, stats, stride);
-  FM_KERNEL_LAUNCH((k_norm_apply<TIO, DH>), grid, fm_dim3(256), 0, stream, xr, yr, d->n, d->centre, d->max_norm,
-                   d->scale, stats, stride);
+  if (d0->max_norm) FM_KERNEL_LAUNCH((k_norm_maxnorm<TIO, DH>), grid, fm_dim3(256), 0, stream, j0, j1, d0->centre);
+  FM_KERNEL_LAUNCH((k_norm_apply<TIO, DH>), grid, fm_dim3(256), 0, stream, j0, j1, d0->centre, d0->max_norm, d0->scale);
   return fm_after_launch() ? FASTMAX_ERR_LAUNCH : FASTMAX_OK;
 }
 
-inline int fm_normalize_dispatch(const FastmaxNormDesc* d, const void* x, void* y, float* stats, fm_stream_t stream) {
+// a second tensor takes part in the first one's launches: same batch*heads, head size, type and kind of pass
+inline bool fm_norm_same(const FastmaxNormDesc* a, const FastmaxNormDesc* b) {
+  return a->bh == b->bh && a->d == b->d && a->dtype == b->dtype && a->centre == b->centre && a->max_norm == b->max_norm &&
+         a->scale == b->scale;
+}
+inline int fm_norm_check(const FastmaxNormDesc* d, const void* x, const void* y, const float* stats) {
   if (!d || !x || !y) return FASTMAX_ERR_NULL;
   if (d->dtype != FASTMAX_F32 && d->dtype != FASTMAX_BF16) return FASTMAX_ERR_DTYPE;
   if (d->bh <= 0 || d->n <= 0 || d->bh > 65535) return FASTMAX_ERR_SHAPE;
@@ -213,10 +243,20 @@ inline int fm_normalize_dispatch(const FastmaxNormDesc* d, const void* x, void* 
   if (d->centre < 0 || d->centre > 2) return FASTMAX_ERR_UNSUPPORTED;
   if ((d->max_norm || d->centre == 2) && !stats) return FASTMAX_ERR_WORKSPACE;
   if (d->sx.n < d->d || d->sy.n < d->d) return FASTMAX_ERR_SHAPE;
-  if (d->dtype == FASTMAX_BF16) {
-    return d->d == 64 ? fm_normalize_run<fm_bf16, 64>(d, x, y, stats, stream) : fm_normalize_run<fm_bf16, 32>(d, x, y, stats, stream);
-  }
-  return d->d == 64 ? fm_normalize_run<float, 64>(d, x, y, stats, stream) : fm_normalize_run<float, 32>(d, x, y, stats, stream);
+  return FASTMAX_OK;
+}
+
+inline int fm_normalize_dispatch(const FastmaxNormDesc* d0, const void* x0, void* y0, float* stats0, const FastmaxNormDesc* d1,
+                                 const void* x1, void* y1, float* stats1, fm_stream_t stream) {
+  int st = fm_norm_check(d0, x0, y0, stats0);
+  if (!st && d1) st = fm_norm_check(d1, x1, y1, stats1);
+  if (st) return st;
+  if (d1 && !fm_norm_same(d0, d1)) return FASTMAX_ERR_SHAPE;
+  if (d0->dtype == FASTMAX_BF16)
+    return d0->d == 64 ? fm_normalize_run<fm_bf16, 64>(d0, x0, y0, stats0, d1, x1, y1, stats1, stream)
+                       : fm_normalize_run<fm_bf16, 32>(d0, x0, y0, stats0, d1, x1, y1, stats1, stream);
+  return d0->d == 64 ? fm_normalize_run<float, 64>(d0, x0, y0, stats0, d1, x1, y1, stats1, stream)
+                     : fm_normalize_run<float, 32>(d0, x0, y0, stats0, d1, x1, y1, stats1, stream);
 }
 
 // ------------------------------------------------------------------------------
@@ -243,16 +283,19 @@ inline int64_t fm_normb_stride(int dh, int n, int centre) {
   return fm_normb_base(dh, n) + (centre == 2 ? 2 * int64_t(fm_norm_blocks(n)) * dh : 0);
 }
 
-// grid (ceil(n / (64 * FM_NORMB_NP)), bh); four threads per token
+// grid (ceil(n / (64 * FM_NORMB_NP)), bh, jobs); four threads per token
 template <typename TIO, int DH>
-FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_normb_stats(TRef<const TIO> x, TRef<const TIO> dy, int n, int centre, int max_norm,
-                                                   float* FM_RESTRICT stats, int64_t stride) {
+FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_normb_stats(NormJob<TIO> j0, NormJob<TIO> j1, int centre) {
   constexpr int EPT = DH / 4, NP = FM_NORMB_NP;
   FM_SHARED float wsum[NP][4];
   FM_SHARED unsigned long long wkey[4];
   const int tid = FM_TID_X, bh = FM_BID_Y;
+  const NormJob<TIO> J = FM_BID_Z ? j1 : j0;
+  const TRef<const TIO> x = J.x, dy = J.dy;
+  const int n = J.n;
+  if (int(FM_BID_X) >= fm_normb_blocks(n)) return;
   const int tok0 = FM_BID_X * 64 * NP + (tid >> 2), d0 = (tid & 3) * EPT;
-  float* st = stats + bh * stride;
+  float* st = J.stats + bh * J.stride;
   float c[NP][EPT], g[NP][EPT];
 #pragma unroll
   for (int p = 0; p < NP; ++p) {
@@ -302,16 +345,19 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_normb_stats(TRef<const TIO> x, TRef<const
   }
 }
 
-// grid (ceil(n / (64 * FM_NORM_NP)), bh); four threads per token
+// grid (ceil(n / (64 * FM_NORM_NP)), bh, jobs); four threads per token
 template <typename TIO, int DH>
-FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_normb_apply(TRef<const TIO> x, TRef<const TIO> dy, TRef<TIO> dx, int n, int centre,
-                                                   int max_norm, float scale, const float* FM_RESTRICT stats, int64_t stride) {
+FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_normb_apply(NormJob<TIO> j0, NormJob<TIO> j1, int centre, int max_norm, float scale) {
   constexpr int EPT = DH / 4, NP = FM_NORM_NP;
   FM_SHARED float red[256];
   FM_SHARED unsigned long long redk[256];
   const int tid = FM_TID_X, bh = FM_BID_Y;
+  const NormJob<TIO> J = FM_BID_Z ? j1 : j0;
+  const TRef<const TIO> x = J.x, dy = J.dy;
+  const int n = J.n;
+  if (int(FM_BID_X) >= fm_norm_blocks(n)) return;
   const int tok0 = FM_BID_X * 64 * NP + (tid >> 2), d0 = (tid & 3) * EPT;
-  const float* st = stats ? stats + bh * stride : nullptr;
+  const float* st = J.stats ? J.stats + bh * J.stride : nullptr;
   float g[NP][EPT];
 #pragma unroll
   for (int p = 0; p < NP; ++p) {
@@ -365,51 +411,50 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_normb_apply(TRef<const TIO> x, TRef<const
 #pragma unroll
       for (int j = 0; j < EPT; ++j) g[p][j] *= f;
 #pragma unroll
-      for (int j = 0; j < EPT; j += 8) IO<TIO>::st8(dx.base(bh) + int64_t(tok) * dx.s_n + d0 + j, &g[p][j]);
+      for (int j = 0; j < EPT; j += 8) IO<TIO>::st8(J.out.base(bh) + int64_t(tok) * J.out.s_n + d0 + j, &g[p][j]);
     }
   }
 }
 
 template <typename TIO, int DH>
-int fm_normalize_bwd_run(const FastmaxNormDesc* d, const void* x, const void* dy, void* dx, float* stats, fm_stream_t stream) {
-  const TRef<const TIO> xr = fm_ref<const TIO>(static_cast<const TIO*>(x), d->sx);
-  const TRef<const TIO> gr = fm_ref<const TIO>(static_cast<const TIO*>(dy), d->sy);
-  const TRef<TIO> dxr = fm_ref<TIO>(static_cast<TIO*>(dx), d->sx);
-  const fm_dim3 grid_stats((d->n + 64 * FM_NORMB_NP - 1) / (64 * FM_NORMB_NP), d->bh);
-  const fm_dim3 grid((d->n + 64 * FM_NORM_NP - 1) / (64 * FM_NORM_NP), d->bh);
-  const int64_t stride = fm_normb_stride(DH, d->n, d->centre);
-  if (d->max_norm || d->centre == 2) {
-    if (d->centre == 2) {
-      // the means of x and of dy lie side by side: one launch of the last step covers both
-      float* sums = stats + fm_normb_base(DH, d->n);
-      FM_KERNEL_LAUNCH((k_norm_colsum<TIO, DH>), fm_dim3(grid.x, grid.y, 2), fm_dim3(256), 0, stream, xr, gr, d->n, sums, stride);
-      FM_KERNEL_LAUNCH((k_norm_colfinal<DH>), fm_dim3(d->bh, 2), fm_dim3(256), 0, stream, sums, stride, int(grid.x), d->n,
-                       stats + 4, stride);
-    }
-    if (d->max_norm)
-      FM_KERNEL_LAUNCH((k_normb_stats<TIO, DH>), grid_stats, fm_dim3(256), 0, stream, xr, gr, d->n, d->centre, d->max_norm, stats,
-                       stride);
+int fm_normalize_bwd_run(const FastmaxNormDesc* d0, const void* x0, const void* dy0, void* dx0, float* stats0,
+                         const FastmaxNormDesc* d1, const void* x1, const void* dy1, void* dx1, float* stats1, fm_stream_t stream) {
+  auto job = [](const FastmaxNormDesc* d, const void* x, const void* dy, void* dx, float* stats) {
+    NormJob<TIO> j{};
+    j.x = fm_ref<const TIO>(static_cast<const TIO*>(x), d->sx);
+    j.dy = fm_ref<const TIO>(static_cast<const TIO*>(dy), d->sy);
+    j.out = fm_ref<TIO>(static_cast<TIO*>(dx), d->sx);
+    j.n = d->n; j.stats = stats; j.stride = fm_normb_stride(DH, d->n, d->centre);
+    // the means of x and of dy lie side by side: one launch of the last step covers both
+    if (stats) { j.mean = stats + 4; j.sums = stats + fm_normb_base(DH, d->n); }
+    return j;
+  };
+  const NormJob<TIO> j0 = job(d0, x0, dy0, dx0, stats0), j1 = d1 ? job(d1, x1, dy1, dx1, stats1) : j0;
+  const int jobs = d1 ? 2 : 1, nmax = j0.n > j1.n ? j0.n : j1.n;
+  const fm_dim3 grid(fm_norm_blocks(nmax), d0->bh, jobs);
+  if (d0->centre == 2) {
+    FM_KERNEL_LAUNCH((k_norm_colsum<TIO, DH, 2>), fm_dim3(grid.x, grid.y, 2 * jobs), fm_dim3(256), 0, stream, j0, j1);
+    FM_KERNEL_LAUNCH((k_norm_colfinal<TIO, DH, 2>), fm_dim3(d0->bh, 2 * jobs), fm_dim3(256), 0, stream, j0, j1);
   }
-  FM_KERNEL_LAUNCH((k_normb_apply<TIO, DH>), grid, fm_dim3(256), 0, stream, xr, gr, dxr, d->n, d->centre, d->max_norm,
-                   d->scale, stats, stride);
+  if (d0->max_norm)
+    FM_KERNEL_LAUNCH((k_normb_stats<TIO, DH>), fm_dim3(fm_normb_blocks(nmax), d0->bh, jobs), fm_dim3(256), 0, stream, j0, j1, d0->centre);
+  FM_KERNEL_LAUNCH((k_normb_apply<TIO, DH>), grid, fm_dim3(256), 0, stream, j0, j1, d0->centre, d0->max_norm, d0->scale);
   return fm_after_launch() ? FASTMAX_ERR_LAUNCH : FASTMAX_OK;
 }
 
-inline int fm_normalize_bwd_dispatch(const FastmaxNormDesc* d, const void* x, const void* dy, void* dx, float* stats,
+inline int fm_normalize_bwd_dispatch(const FastmaxNormDesc* d0, const void* x0, const void* dy0, void* dx0, float* stats0,
+                                     const FastmaxNormDesc* d1, const void* x1, const void* dy1, void* dx1, float* stats1,
                                      fm_stream_t stream) {
-  if (!d || !x || !dy || !dx) return FASTMAX_ERR_NULL;
-  if (d->dtype != FASTMAX_F32 && d->dtype != FASTMAX_BF16) return FASTMAX_ERR_DTYPE;
-  if (d->bh <= 0 || d->n <= 0 || d->bh > 65535) return FASTMAX_ERR_SHAPE;
-  if (d->d != 32 && d->d != 64) return FASTMAX_ERR_UNSUPPORTED;
-  if (d->centre < 0 || d->centre > 2) return FASTMAX_ERR_UNSUPPORTED;
-  if ((d->max_norm || d->centre == 2) && !stats) return FASTMAX_ERR_WORKSPACE;
-  if (d->sx.n < d->d || d->sy.n < d->d) return FASTMAX_ERR_SHAPE;
-  if (d->dtype == FASTMAX_BF16) {
-    return d->d == 64 ? fm_normalize_bwd_run<fm_bf16, 64>(d, x, dy, dx, stats, stream)
-                      : fm_normalize_bwd_run<fm_bf16, 32>(d, x, dy, dx, stats, stream);
-  }
-  return d->d == 64 ? fm_normalize_bwd_run<float, 64>(d, x, dy, dx, stats, stream)
-                    : fm_normalize_bwd_run<float, 32>(d, x, dy, dx, stats, stream);
+  if (!dx0 || (d1 && !dx1)) return FASTMAX_ERR_NULL;
+  int st = fm_norm_check(d0, x0, dy0, stats0);
+  if (!st && d1) st = fm_norm_check(d1, x1, dy1, stats1);
+  if (st) return st;
+  if (d1 && !fm_norm_same(d0, d1)) return FASTMAX_ERR_SHAPE;
+  if (d0->dtype == FASTMAX_BF16)
+    return d0->d == 64 ? fm_normalize_bwd_run<fm_bf16, 64>(d0, x0, dy0, dx0, stats0, d1, x1, dy1, dx1, stats1, stream)
+                       : fm_normalize_bwd_run<fm_bf16, 32>(d0, x0, dy0, dx0, stats0, d1, x1, dy1, dx1, stats1, stream);
+  return d0->d == 64 ? fm_normalize_bwd_run<float, 64>(d0, x0, dy0, dx0, stats0, d1, x1, dy1, dx1, stats1, stream)
+                     : fm_normalize_bwd_run<float, 32>(d0, x0, dy0, dx0, stats0, d1, x1, dy1, dx1, stats1, stream);
 }
 
 // ------------------------------------------------------------------------------

@@ -199,6 +199,23 @@ def test_score_function_front(sf, normalize, mask, p):
         assert rel_err(got, want) < 2e-5      # the fp32 normalisation backward pass on top of the kernels
 
 
+@pytest.mark.parametrize("d,nq,nk,mask", [(48, 257, 257, True), (20, 65, 65, True), (33, 130, 700, None), (64, 300, 520, True)])
+def test_score_function_front_ragged(sf, d, nq, nk, mask):
+    """Head sizes between the kernels' own, q and k of different lengths, the projection layout; gradients of v alone, too."""
+    shapes = ((nq, 91), (nk, 92), (nk, 93), (nq, 94))
+    q, k, v, go = (rnd(2, n, 3, d, seed=s).transpose(1, 2) for n, s in shapes)
+    qd, kd, vd = (x.to(DEV).requires_grad_(True) for x in (q, k, v))
+    grads = torch.autograd.grad(sf.fastmax(qd, kd, vd, mask=mask, normalize=1, p=2), (qd, kd, vd), go.to(DEV))
+    qr, kr, vr = (x.double().requires_grad_(True) for x in (q, k, v))
+    oref = O.score_function_fastmax(qr, kr, vr, mask=mask, normalize=1, p=2)
+    want = torch.autograd.grad(oref, (qr, kr, vr), go.double())
+    assert rel_err(sf.fastmax(qd, kd, vd, mask=mask, normalize=1, p=2), oref) < 1e-5
+    for a, b in zip(grads, want):
+        assert rel_err(a, b) < 2e-5
+    only_v = torch.autograd.grad(sf.fastmax(q.to(DEV), k.to(DEV), vd, mask=mask, normalize=1, p=2), vd, go.to(DEV))[0]
+    assert torch.equal(only_v, grads[2])
+
+
 def test_rpe_matrix_structured(sf):
     """Sinusoidal relative-position table (reference transformer/model.py:230-241): row n - 1 + t holds
     position -t, row n - 1 - t position +t; checked against the closed form entry by entry."""

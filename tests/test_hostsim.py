@@ -137,6 +137,28 @@ def test_normalize_backward(sim):
     assert O.rel_l2(sim.normalize_backward(x, dy, centre=2, max_norm=True, scale=1.5), xd.grad) < 1e-5
 
 
+@pytest.mark.parametrize("nq,nk,d,centre", [(70, 70, 32, 2), (1, 300, 64, 2), (600, 257, 64, 2), (129, 64, 32, 0)])
+def test_normalize_pair(sim, nq, nk, d, centre):
+    """Two tensors in common launches: the bits of the separate passes, whichever of the two is the longer."""
+    g = torch.Generator().manual_seed(81)
+    q, dq, k, dk = (torch.randn(2, n, d, generator=g) for n in (nq, nq, nk, nk))
+    want = [sim.normalize(x, centre=centre, max_norm=True, scale=1.5) for x in (q, k)]
+    assert all(torch.equal(a, b) for a, b in zip(sim.normalize_pair(q, k, centre=centre, scale=1.5), want))
+    want = [sim.normalize_backward(x, dy, centre=centre, max_norm=True, scale=1.5) for x, dy in ((q, dq), (k, dk))]
+    assert all(torch.equal(a, b) for a, b in zip(sim.normalize_pair(q, k, dq, dk, centre=centre, scale=1.5), want))
+
+
+@pytest.mark.parametrize("d,dpad", [(1, 32), (31, 32), (40, 64), (48, 64), (63, 64), (96, 128), (127, 128)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_pad_features(sim, d, dpad, dtype):
+    g = torch.Generator().manual_seed(82)
+    xs = [torch.randn(2, n, 3, d, generator=g).to(dtype).transpose(1, 2) for n in (1, 70, 33)]
+    xs[1][0, 0, 0, 0] = float("nan")
+    for some in (xs, xs[1:2]):
+        for x, y in zip(some, sim.pad_features(some, dpad)):
+            assert torch.equal(y.nan_to_num(7.0), torch.nn.functional.pad(x, (0, dpad - d)).nan_to_num(7.0))
+
+
 def test_order2_walk_per_value_column(sim):
     """k_walk_sym (D = 64, _Float16): prefix walk for the forward, suffix walk with the weights c for the backward,
     dQ reading the forward's state transposed; with and without the forward's kept workspace, and the one global
