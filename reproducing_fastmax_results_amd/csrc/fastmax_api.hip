@@ -416,25 +416,55 @@ template <typename TIO, typename E> void tok_common(TokArgs<TIO, E>& a, const Fa
   a.out_resid = nullptr; a.own_ores = nullptr; a.state_xscale = 1.0f;
 }
 
+// Launches that go with two groups of wavefronts per workgroup (GRP in fm_tok.h), by their number of workgroups on the chip's 256 CUs.
+// At one workgroup per CU or less every kernel gains (whole calls, microseconds, one group and two; forward of 1 x 8 heads of 64, 4096
+// tokens 54 -> 41.5, of 2 x 8 of 2048 32 -> 27, unmasked 54 -> 45; D = 32 23 -> 19; D = 128 53 -> 48.5; a step with dQ so 174 -> 165,
+// with dK + dV so 174 -> 166).  The causal forward gains up to two per CU where its chains are long, since the light workgroups leave
+// room (16 heads of 3001 tokens 44 -> 37.6, 512 workgroups 61 -> 52 and 40 -> 36; 12 heads of 4096 62.8 -> 63.2; D = 32 25 -> 23; at
+// 512 tokens 19.5 -> 20.0; unmasked 55 -> 55).  Past that the registers hold fewer wavefronts in pairs of groups than in single ones:
+// forward at 1024 workgroups 38 -> 44, dQ at 384 145 -> 145 and 245 -> 253, dK + dV unmasked at 256 191 -> 191 and 114 -> 115.5, at 128
+// 96 -> 93.  Heads of 128: the forward alone (dQ 187 -> 188; dK + dV spills, 187 -> 326), and only up to 256 (at 512 65 -> 72).
+enum { FM_GRP_PV, FM_GRP_DS, FM_GRP_DV };
+inline bool two_groups(int kind, int dh, int64_t workgroups, bool causal, int n_str) {
+  if (kind == FM_GRP_PV) return workgroups <= (causal && dh <= 64 && n_str >= 1024 ? 512 : 256);
+  return dh <= 64 && workgroups <= (kind == FM_GRP_DV && !causal ? 128 : 256);
+}
+
 template <typename TIO, typename E, int DH, int QT, int OWN, int QF = 0>
 int launch_pv(const TokArgs<TIO, E>& a, int bh, int kernel_id, fm_stream_t stream) {
   typedef TokCfg<E, DH, QT> C;
+  ProfScope prof(kernel_id, stream);
+  const fm_dim3 grid((a.n_own + C::QW - 1) / C::QW, bh);
+  if constexpr (sizeof(E) == 2 && QT == 1 && OWN == FM_OWN_Q) {
+    if (!a.use_state && two_groups(FM_GRP_PV, DH, int64_t(grid.x) * bh, a.causal, a.n_str)) {
+      constexpr size_t lds = 2 * C::GRP_PV;
+      fm_allow_lds(reinterpret_cast<const void*>(&k_pv<TIO, E, DH, QT, OWN, QF, 2>), lds);
+      FM_KERNEL_LAUNCH((k_pv<TIO, E, DH, QT, OWN, QF, 2>), grid, fm_dim3(2 * FM_THREADS), lds, stream, a);
+      return fm_launch_status();
+    }
+  }
   const size_t lds = tok_lds_bytes<E, DH, QT>(0);
   fm_allow_lds(reinterpret_cast<const void*>(&k_pv<TIO, E, DH, QT, OWN, QF>), lds);
-  ProfScope prof(kernel_id, stream);
-  FM_KERNEL_LAUNCH((k_pv<TIO, E, DH, QT, OWN, QF>), fm_dim3((a.n_own + C::QW - 1) / C::QW, bh), fm_dim3(FM_THREADS), lds,
-                   stream, a);
+  FM_KERNEL_LAUNCH((k_pv<TIO, E, DH, QT, OWN, QF>), grid, fm_dim3(FM_THREADS), lds, stream, a);
   return fm_launch_status();
 }
 
 template <typename TIO, typename E, int DH, int QT, int OWN, int DV = 0, int PREP = 0, int QF = 0, int STR = 0>
 int launch_ds(const TokArgs<TIO, E>& a, int bh, int kernel_id, fm_stream_t stream) {
   typedef TokCfg<E, DH, QT> C;
+  ProfScope prof(kernel_id, stream);
+  const fm_dim3 grid((a.n_own + C::QW - 1) / C::QW, bh);
+  if constexpr (sizeof(E) == 2 && DH <= 64 && QT == 1 && !STR && (PREP || DV)) {
+    if (!a.use_state && two_groups(DV ? FM_GRP_DV : FM_GRP_DS, DH, int64_t(grid.x) * bh, a.causal, a.n_str)) {
+      constexpr size_t lds = 2 * (DV ? C::GRP_DV : C::GRP_DS);
+      fm_allow_lds(reinterpret_cast<const void*>(&k_ds<TIO, E, DH, QT, OWN, DV, PREP, QF, STR, 2>), lds);
+      FM_KERNEL_LAUNCH((k_ds<TIO, E, DH, QT, OWN, DV, PREP, QF, STR, 2>), grid, fm_dim3(2 * FM_THREADS), lds, stream, a);
+      return fm_launch_status();
+    }
+  }
   const size_t lds = tok_lds_bytes<E, DH, QT>(PREP ? 3 : (DV ? (a.use_state ? 4 : 2) : 1));
   fm_allow_lds(reinterpret_cast<const void*>(&k_ds<TIO, E, DH, QT, OWN, DV, PREP, QF, STR>), lds);
-  ProfScope prof(kernel_id, stream);
-  FM_KERNEL_LAUNCH((k_ds<TIO, E, DH, QT, OWN, DV, PREP, QF, STR>), fm_dim3((a.n_own + C::QW - 1) / C::QW, bh), fm_dim3(FM_THREADS), lds,
-                   stream, a);
+  FM_KERNEL_LAUNCH((k_ds<TIO, E, DH, QT, OWN, DV, PREP, QF, STR>), grid, fm_dim3(FM_THREADS), lds, stream, a);
   return fm_launch_status();
 }
 

@@ -1303,7 +1303,12 @@ struct TokCfg {
   static constexpr int OCC_DS = WIDE ? 1 : (sizeof(E) == 2 ? (QT == 1 ? 3 : 2) : 1);
   static constexpr int OCC_DV = WIDE ? 1 : 2;
   static constexpr int SA = sizeof(E) == 2 ? QT : 2;                      // values of a per state slab
-  static constexpr int KT_PV = sizeof(E) == 2 ? 32 : 64;   // stream tokens per stage of the dense loop, k_pv
+  // Stream tokens per stage of the dense loop, k_pv.  A stage waits for loads that began one stage earlier, so short stages are
+  // bound by that latency: with 64 tokens instead of 32, forward at D = 32, 4 x 8 heads of 4096 tokens 77 -> 53 us, 2 x 8 of 2048
+  // 39.5 -> 22.7 (128 tokens: 58, 23.5); D = 128, 2 x 8 of 2048 57 -> 53.  D = 64 has four workgroups per CU at 32 tokens, which hide
+  // it; 64 tokens leave registers for three: 16 x 8 heads of 1024 tokens 38 -> 42, 4 x 8 of 4096 89 -> 90, and where a CU has one or two
+  // workgroups it gains less than two groups per workgroup do (1 x 8 of 4096 55 -> 48, groups 42).
+  static constexpr int KT_PV = sizeof(E) == 2 && (QT == 2 || DH == 64) ? 32 : 64;
   static constexpr int KT_DS = 64;                        //                                           k_ds
   // the dK + dV pass runs two workgroups per CU whatever its stages are, and 64-token stages
   // halve its barriers (0.163 vs 0.173 ms at the shape above)
@@ -1322,6 +1327,12 @@ struct TokCfg {
   // through transposing LDS reads where the type has them, from two more (transposed) tiles otherwise
   static constexpr int DV_STAGE = 2 * KT_DV * PQ + (M::HAS_TR ? 0 : 2 * DH * PV_DV) + (M::HAS_TR ? 2 : 1) * KT_DV;
   static constexpr int DS_NBUF = sizeof(E) == 2 ? 2 : 1;
+  // Two groups of four wavefronts per workgroup (see fm_join_groups): LDS of one group, and of the sums (ROWS accumulators) that meet
+  static constexpr size_t cmax(size_t a, size_t b) { return a > b ? a : b; }
+  static constexpr size_t GRP_PV = 2 * DH * 4 + sizeof(E) * cmax(QW * PQ, 2 * PV_STAGE);
+  static constexpr size_t GRP_DS = 2 * DH * 4 + cmax(2 * QW * PQ * sizeof(E) + QW * 4, sizeof(E) * DS_NBUF * DS_STAGE);
+  static constexpr size_t GRP_DV = 2 * DH * 4 + sizeof(E) * cmax(QW * PQ, DS_NBUF * DV_STAGE);
+  static constexpr size_t JOIN = size_t(FM_THREADS) * 4 * (16 * NT + 1);
 };
 
 // Moment readout, transposed:  acc[j][ct] (rows c, column = token of tile j) +=

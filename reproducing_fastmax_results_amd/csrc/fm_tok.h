@@ -272,6 +272,23 @@ template <int OWN> FM_DEVICE void fm_tile_window(bool causal, int s0, int lo, in
   }
 }
 
+// GRP = 2: a workgroup of two groups of four wavefronts.  Both hold the same own tokens, each in LDS of its own, and take the stages
+// of the stream in turn; their sums meet here.  For launches of few workgroups (see two_groups in fastmax_api.hip): a causal launch
+// whose workgroups all run at once takes as long as its longest one, and a lone workgroup on a CU waits for every stage's loads; this
+// halves the chain of stages and gives the CU twice the wavefronts.
+template <int NACC> FM_DEVICE void fm_join_groups(float* lds, fm_f32x16* acc, int grp, int tid) {
+  if (grp == 1) {
+#pragma unroll
+    for (int i = 0; i < 16 * NACC; ++i) lds[i * FM_THREADS + tid] = acc[i / 16][i % 16];
+  }
+  FM_SYNC();
+  if (grp == 0) {
+#pragma unroll
+    for (int i = 0; i < 16 * NACC; ++i) acc[i / 16][i % 16] += lds[i * FM_THREADS + tid];
+  }
+  FM_SYNC();
+}
+
 // ------------------------------------------------------------------------------
 // k_pv: forward (own = queries) and dV (own = keys).  grid (ceil(n_own / QW), bh).
 // LDS: va, vb | own rows [QW][PQ] | region (Z, then state slabs); the two dense stages and the
@@ -279,8 +296,10 @@ template <int OWN> FM_DEVICE void fm_tile_window(bool causal, int s0, int lo, in
 // ------------------------------------------------------------------------------
 // QF = 1 (forward of an order-2 problem without states, _Float16): the weights in their completed-square
 // form (see TileMath<fm_half>::wq); the host picks it when a2 is of ordinary size.
-template <typename TIO, typename E, int DH, int QT, int OWN, int QF = 0>
-FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_THREADS, (TokCfg<E, DH, QT>::OCC_PV)) k_pv(TokArgs<TIO, E> A) {
+template <typename TIO, typename E, int DH, int QT, int OWN, int QF = 0, int GRP = 1>
+FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_THREADS * GRP, (TokCfg<E, DH, QT>::OCC_PV)) k_pv(TokArgs<TIO, E> A) {
+  static_assert(GRP == 1 || (QT == 1 && OWN == FM_OWN_Q && sizeof(E) == 2 && TokCfg<E, DH, QT>::JOIN <= 2 * TokCfg<E, DH, QT>::GRP_PV),
+                "two groups: forward without states, one tile per wavefront");
   static_assert(!QF || (QT == 1 && OWN == FM_OWN_Q && sizeof(E) == 2), "completed-square weights: forward, one tile per wavefront");
   typedef TokCfg<E, DH, QT> C;
   typedef Mma<E> M;
@@ -289,10 +308,11 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_THREADS, (TokCfg<E, DH, QT>::OCC_PV)) k_pv(T
   constexpr int NT = C::NT, NKS = C::NKS, QW = C::QW, PQ = C::PQ, KT = C::KT_PV, PV = C::PV_PV;
   constexpr int STAGE = C::PV_STAGE;
   FM_DYN_SMEM(smem);
-  float* vecs = reinterpret_cast<float*>(smem);       // va[DH], vb[DH]
+  const int grp = GRP > 1 ? FM_UNIFORM(int(FM_TID_X) / FM_THREADS) : 0;
+  float* vecs = reinterpret_cast<float*>(smem + grp * C::GRP_PV);   // va[DH], vb[DH]
   E* Own = reinterpret_cast<E*>(vecs + 2 * DH);       // [QW][PQ]
   E* R = Own + QW * PQ;
-  const int tid = FM_TID_X, lane = tid & 63, lr = lane & 31, lh = lane >> 5;
+  const int tid = int(FM_TID_X) % FM_THREADS, lane = tid & 63, lr = lane & 31, lh = lane >> 5;
   const int wave = FM_UNIFORM(tid >> 6);
   TokGeom<OWN, QW, TokArgs<TIO, E> > G;
   G.init(A);
@@ -310,7 +330,7 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_THREADS, (TokCfg<E, DH, QT>::OCC_PV)) k_pv(T
     ro.store(Own, PQ, tid);
   }
   const float* sml = A.small + (int64_t(bh) * A.nslots + G.slot) * StateDims<DH>::SMALL;
-  if (G.use_state) {
+  if (GRP == 1 && G.use_state) {
     // order 1 has no Z (its coefficient is the order-2 one): only the two vectors are staged
     if (OWN == FM_OWN_Q && A.quad) fm_stage_small<E, DH, QT>(sml, R, vecs, tid, 1.0f);
     else if (tid < 2 * DH) vecs[tid] = sml[DH * DH + tid];
@@ -346,7 +366,7 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_THREADS, (TokCfg<E, DH, QT>::OCC_PV)) k_pv(T
 #pragma unroll
   for (int j = 0; j < QT; ++j) gsum[j] = 0.f;
 
-  if (G.use_state) {
+  if (GRP == 1 && G.use_state) {
     if (OWN == FM_OWN_Q && A.quad) {
       // denominator: g_i += sum_m q_im (va[m] + sum_l Z[m][l] q_il)
 #pragma unroll
@@ -402,20 +422,21 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_THREADS, (TokCfg<E, DH, QT>::OCC_PV)) k_pv(T
     // (queries start at the first key of the segment, keys at its last query): blocks that run at
     // the same time then read the same tiles at about the same time and share them in the L2.
     const int nst = (G.send - G.sbeg + KT - 1) / KT;
-    const int s_first = OWN == FM_OWN_Q ? G.sbeg : G.sbeg + KT * (nst - 1);
-    const int s_step = OWN == FM_OWN_Q ? KT : -KT;
+    const int s_end = OWN == FM_OWN_Q ? G.sbeg : G.sbeg + KT * (nst - 1);      // the end of the stream the walk begins at
+    const int s_step = (OWN == FM_OWN_Q ? KT : -KT) * GRP, s_first = s_end + grp * (s_step / GRP);
     // Two stage buffers.  The tiles of stage i+1 travel global memory -> registers during stage i-1
     // and registers -> LDS in the middle of stage i (between the two groups of matrix products),
     // so the only thing left at the top of a stage is the barrier.
     auto more = [&](int sx) { return OWN == FM_OWN_Q ? (sx < G.send) : (sx >= G.sbeg); };
-    fetch(s_first);
+    fetch(GRP == 1 || more(s_first) ? s_first : s_end);
     put(0);
     if (more(s_first + s_step)) fetch(s_first + s_step);
     int buf = 0;
-    for (int s0 = s_first; more(s0); s0 += s_step) {
+    for (int s0 = s_first; more(GRP == 1 ? s0 : s0 - grp * (s_step / GRP)); s0 += s_step) {   // (the groups meet at every barrier)
       E* Xs = Own + buf * STAGE;                        // the own rows and the slabs are spent
       E* Zt = Xs + KT * PQ;
       FM_SYNC();
+      if (GRP > 1 && !more(s0)) break;                  // an odd number of stages: nothing left for the second group
       // One code path for every tile: the products always run, and a tile that touches the mask
       // or the end of the sequence (a wavefront-uniform test) zeroes the entries outside its row
       // window before they are used; a tile wholly outside the mask has an empty window.
@@ -468,6 +489,12 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_THREADS, (TokCfg<E, DH, QT>::OCC_PV)) k_pv(T
       buf ^= 1;
     }
     FM_SYNC();
+    if constexpr (GRP > 1) {
+      float* jl = reinterpret_cast<float*>(smem);
+      if (grp == 1) jl[16 * NT * FM_THREADS + tid] = gsum[0];
+      fm_join_groups<NT>(jl, acc[0], grp, tid);
+      if (grp == 0) gsum[0] += jl[16 * NT * FM_THREADS + tid];
+    }
   }
 
   // ---- epilogue ----
@@ -482,7 +509,7 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_THREADS, (TokCfg<E, DH, QT>::OCC_PV)) k_pv(T
       const float ginv = 1.0f / gt;
       if (QF) gt *= 1.0f / (4.0f * A.a2);              // the constant taken out of the weights (o does not see it)
       const int qi = t0 + xrow[j];
-      const bool in = qi < A.n_own;
+      const bool in = qi < A.n_own && grp == 0;
       if (lh == 0 && in) A.g.base(bh)[int64_t(qi) * A.g.s_n] = gt;
       TIO* orow = ob + int64_t(qi) * A.out.s_n;
       fm_half* rrow = A.out_resid ? A.out_resid + (int64_t(bh) * A.npad_own + qi) * DH : nullptr;
@@ -580,8 +607,10 @@ FM_DEVICE void fm_readout_kv(const E* FM_RESTRICT state2, const E* xs, int xrow,
 // STR = 1 (own = queries, _Float16, two tiles per wavefront): the prefix state is the forward's own layout and is
 // read out transposed (see fm_readout, TRA); the fragments of the dense tiles are fetched behind that readout, so that
 // the kernel holds 64 registers fewer across it.
-template <typename TIO, typename E, int DH, int QT, int OWN, int DV, int PREP, int QF = 0, int STR = 0>
-FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_THREADS, (DV ? TokCfg<E, DH, QT>::OCC_DV : TokCfg<E, DH, QT>::OCC_DS)) k_ds(TokArgs<TIO, E> A) {
+template <typename TIO, typename E, int DH, int QT, int OWN, int DV, int PREP, int QF = 0, int STR = 0, int GRP = 1>
+FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_THREADS * GRP, (DV ? TokCfg<E, DH, QT>::OCC_DV : TokCfg<E, DH, QT>::OCC_DS)) k_ds(TokArgs<TIO, E> A) {
+  static_assert(GRP == 1 || (QT == 1 && sizeof(E) == 2 && !STR && (DV ? 2 : 1) * TokCfg<E, DH, QT>::JOIN <= 2 * (DV ? TokCfg<E, DH, QT>::GRP_DV : TokCfg<E, DH, QT>::GRP_DS)),
+                "two groups: no states, one tile per wavefront");
   static_assert(!STR || (OWN == FM_OWN_Q && sizeof(E) == 2 && !PREP && !QF && !DV), "the transposed readout is dQ's, on _Float16");
   static_assert(!QF || (QT == 1 && sizeof(E) == 2 && (DV != 0 || OWN == FM_OWN_Q)), "completed-square weights: dQ, or dK with dV, one tile per wavefront");
   typedef TokCfg<E, DH, QT> C;
@@ -597,10 +626,11 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_THREADS, (DV ? TokCfg<E, DH, QT>::OCC_DV : T
   // stage, and nobody has to write the transposed copies).  zt and zt2 are not read then.
   constexpr bool TR = M::HAS_TR;
   FM_DYN_SMEM(smem);
-  float* vecs = reinterpret_cast<float*>(smem);
+  const int grp = GRP > 1 ? FM_UNIFORM(int(FM_TID_X) / FM_THREADS) : 0;      // see fm_join_groups
+  float* vecs = reinterpret_cast<float*>(smem + grp * (DV ? C::GRP_DV : C::GRP_DS));
   E* Own = reinterpret_cast<E*>(vecs + 2 * DH);       // [QW][PQ]
   E* R = Own + QW * PQ;
-  const int tid = FM_TID_X, lane = tid & 63, lr = lane & 31, lh = lane >> 5;
+  const int tid = int(FM_TID_X) % FM_THREADS, lane = tid & 63, lr = lane & 31, lh = lane >> 5;
   const int wave = FM_UNIFORM(tid >> 6);
   TokGeom<OWN, QW, TokArgs<TIO, E> > G;
   G.init(A);
@@ -653,14 +683,14 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_THREADS, (DV ? TokCfg<E, DH, QT>::OCC_DV : T
       csum += fm_shfl_xor(csum, 1);
       csum += fm_shfl_xor(csum, 2);
       if (part == 0) {
-        A.w_cv[int64_t(bh) * A.npad_own + t0 + 64 * h + M::tperm(tid >> 2)] = csum;
+        if (grp == 0) A.w_cv[int64_t(bh) * A.npad_own + t0 + 64 * h + M::tperm(tid >> 2)] = csum;
         cl[tok] = csum;
       }
       E* ghrow = A.w_gh + (int64_t(bh) * A.npad_own + row) * DH + d0;
       E* qrrow = A.w_qr + (int64_t(bh) * A.npad_own + row) * DH + d0;
 #pragma unroll
       for (int j = 0; j < EPT; j += 8) {
-        CE<E>::st8(ghrow + j, &vg[j]); CE<E>::st8(qrrow + j, &vq[j]);
+        if (grp == 0) { CE<E>::st8(ghrow + j, &vg[j]); CE<E>::st8(qrrow + j, &vq[j]); }
         CE<E>::st8(R + tok * PQ + d0 + j, &vg[j]); CE<E>::st8(Own + tok * PQ + d0 + j, &vq[j]);
       }
     }
@@ -669,7 +699,7 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_THREADS, (DV ? TokCfg<E, DH, QT>::OCC_DV : T
     ro.load(A.own_r + (int64_t(bh) * A.npad_own + t0) * DH, DH, tid);
     ro.store(Own, PQ, tid);
   }
-  if (G.use_state) {
+  if (GRP == 1 && G.use_state) {
     const float* sml = A.small + (int64_t(bh) * A.nslots + G.slot) * StateDims<DH>::SMALL;
     if (A.quad) fm_stage_small<E, DH, QT>(sml, R, vecs, tid, A.zscale);
     else if (tid < 2 * DH) vecs[tid] = sml[DH * DH + tid];   // order 1 has no Z
@@ -735,7 +765,7 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_THREADS, (DV ? TokCfg<E, DH, QT>::OCC_DV : T
 #pragma unroll
     for (int mt = 0; mt < NT; ++mt) av[j][mt] = fm_zero16();
 
-  if (G.use_state) {
+  if (GRP == 1 && G.use_state) {
     // - c * (va[m] + sum_l Z[m][l] own_l)   (c = c_i for own = queries; folded into Z and va for own = keys)
 #pragma unroll
     for (int j = 0; j < QT; ++j)
@@ -818,8 +848,8 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_THREADS, (DV ? TokCfg<E, DH, QT>::OCC_DV : T
     const E* z2b = DV ? A.zt2 + int64_t(bh) * DH * A.npad_str : nullptr;
     // stage order: see k_pv
     const int nst = (G.send - G.sbeg + KT - 1) / KT;
-    const int s_first = OWN == FM_OWN_Q ? G.sbeg : G.sbeg + KT * (nst - 1);
-    const int s_step = OWN == FM_OWN_Q ? KT : -KT;
+    const int s_end = OWN == FM_OWN_Q ? G.sbeg : G.sbeg + KT * (nst - 1);
+    const int s_step = (OWN == FM_OWN_Q ? KT : -KT) * GRP, s_first = s_end + grp * (s_step / GRP);
     TileRegs<E, KT, DH> rx, ry;
     TileRegs<E, DH, KT> rz, rz2;
     float creg = 0.f;
@@ -842,17 +872,18 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_THREADS, (DV ? TokCfg<E, DH, QT>::OCC_DV : T
     };
     // Two buffers: the tiles of stage i+1 travel global memory -> registers during stage i-1 and
     // registers -> LDS in the middle of stage i (see k_pv).  One buffer (fp32): both at the top.
-    fetch(s_first);
+    fetch(GRP == 1 || more(s_first) ? s_first : s_end);
     if (NBUF == 2) {
       put(0);
       if (more(s_first + s_step)) fetch(s_first + s_step);
     }
     int buf = 0;
-    for (int s0 = s_first; more(s0); s0 += s_step) {
+    for (int s0 = s_first; more(GRP == 1 ? s0 : s0 - grp * (s_step / GRP)); s0 += s_step) {
       E* Xs = Own + buf * STAGE; E* Ys = Xs + KT * PQ; E* Zt = Ys + KT * PQ; E* cs = Zt + (TR ? 0 : DH * PV);
       E* Zt2 = cs + (sizeof(E) == 2 ? 2 : 1) * KT;        // behind the KT floats of -c
       if (NBUF == 1) put(0);
       FM_SYNC();
+      if (GRP > 1 && !more(s0)) break;
       if (NBUF == 1 && more(s0 + s_step)) fetch(s0 + s_step);
       // One code path for every tile (see k_pv).  The score fragments and the transposed fragments
       // serve all own tiles of the wavefront; gh.v is formed per own tile.
@@ -966,6 +997,11 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_THREADS, (DV ? TokCfg<E, DH, QT>::OCC_DV : T
     }
     if (NBUF == 2) FM_SYNC();
   }
+  if constexpr (GRP > 1) {
+    fm_join_groups<NT>(reinterpret_cast<float*>(smem), acc[0], grp, tid);
+    if (DV) fm_join_groups<NT>(reinterpret_cast<float*>(smem), av[0], grp, tid);
+  }
+  const int n_out = grp == 0 ? A.n_own : 0;            // the first group stores
   {
     // with the normalisation's Jacobian: the stored gradient carries lim / max-norm, and the workgroup's part of
     // B = sum dy . y is left for k_norm_fix (the stored values are fac * dy, the copy's rows sc * y)
@@ -973,9 +1009,10 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_THREADS, (DV ? TokCfg<E, DH, QT>::OCC_DV : T
     const E* brows = A.bpart ? (PREP ? A.w_qr : A.brows) + int64_t(bh) * A.npad_own * DH : nullptr;
     float* bout = A.bpart ? A.bpart + int64_t(bh) * ((A.n_own + QW - 1) / QW) + t0 / QW : nullptr;
     fm_store_tokens<TIO, E, DH, QT>(acc, xrow, nullptr, A.out_scale * ginv_sc * fac, reinterpret_cast<float*>(Own), A.out, bh, t0,
-                                    A.n_own, tid, brows, fac > 0.f ? 1.0f / (fac * A.sc) : 0.f, bout);
+                                    n_out, tid, brows, fac > 0.f ? 1.0f / (fac * A.sc) : 0.f, grp == 0 ? bout : nullptr);
+    if (GRP > 1 && grp == 1 && bout) FM_SYNC();        // the barrier of the first group's sum over bout
   }
   if (DV)
     fm_store_tokens<TIO, E, DH, QT>(av, xrow, G.use_state ? vecs + DH : nullptr, A.out2_scale * ginv_sc * (QF ? 1.0f / (4.0f * A.a2) : 1.0f),
-                                    reinterpret_cast<float*>(Own), A.out2, bh, t0, A.n_own, tid);
+                                    reinterpret_cast<float*>(Own), A.out2, bh, t0, n_out, tid);
 }

@@ -40,6 +40,16 @@ def test_mfma_lane_layout(lib):
     assert torch.equal(a32.cpu(), want)
 
 
+@pytest.mark.parametrize("bh,nq,nk,d,mask", [
+    (1, 1, 1, 64, True), (2, 65, 65, 64, True), (3, 97, 97, 32, True), (2, 129, 33, 64, False), (1, 300, 300, 128, True),   # odd and even stages
+    (2, 200, 500, 64, True), (5, 700, 130, 32, False), (2, 520, 70, 128, False), (1, 4096, 4096, 64, True),
+    (128, 129, 129, 64, True), (129, 129, 129, 64, True), (64, 129, 129, 64, False), (65, 129, 129, 64, False),              # 256, 258, 128, 130 workgroups
+    (64, 1024, 1024, 64, True), (65, 1024, 1024, 32, True), (16, 2048, 2048, 128, True), (17, 2048, 2048, 128, True)])       # 512, 520; 256, 272
+def test_groups_of_wavefronts_and_their_limits(lib, bh, nq, nk, d, mask):
+    """Workgroups of one and of two groups of wavefronts on both sides of each limit, stages that do and do not divide among the groups."""
+    check_forward_backward(lib, bh, nq, d, torch.bfloat16, DEV, mask=mask, p=2, nk=nk, seed=160, saved=not (mask and nk > nq))
+
+
 def test_matrix_rate_probe_runs(bench_lib):
     """The bench's yardstick: a register-only loop of matrix products; here only that it runs, writes
     every checksum and reports a rate (16 workgroups, 64 rounds)."""
