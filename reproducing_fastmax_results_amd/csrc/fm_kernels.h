@@ -1287,7 +1287,11 @@ struct TokCfg {
   static constexpr int NT = DH / 32;
   static constexpr int NKS = DH / M::KSTEP;         // k-steps over a feature axis
   static constexpr int QW = 4 * QT * 32;            // tokens per workgroup
-  static constexpr int PQ = DH + M::PAD;            // pitch of row-major token tiles
+  // Pitch of row-major token tiles.  A transposing read takes 16 dwords of each of four rows, a fragment of rows four dwords of each
+  // of 16.  Padded by 16 bytes, rows of 128 begin 4 banks apart and the former met four times in a bank: 42 to 51 % of the LDS
+  // cycles of the wide kernels were conflicts.  12 banks apart they meet twice (21 to 26 %), and fragments of rows never do (2 x 8
+  // heads of 2048 tokens: forward 42.5 -> 38 us, dK + dV 76 -> 66; 20 apart the same).  Rows of 64 meet twice at either padding.
+  static constexpr int PQ = DH + (DH > 64 ? 24 : M::PAD);
   static constexpr int PS = DH + M::PAD;            // pitch of state rows
   // _Float16, QT = 1: one tile per wavefront, small slabs and stages, so that four (k_pv) or three
   // (k_ds) workgroups share a CU: 12 to 16 wavefronts hide each other's LDS and MFMA latency.  On
