@@ -423,11 +423,12 @@ template <typename TIO, typename E> void tok_common(TokArgs<TIO, E>& a, const Fa
 // room (16 heads of 3001 tokens 44 -> 37.6, 512 workgroups 61 -> 52 and 40 -> 36; 12 heads of 4096 62.8 -> 63.2; D = 32 25 -> 23; at
 // 512 tokens 19.5 -> 20.0; unmasked 55 -> 55).  Past that the registers hold fewer wavefronts in pairs of groups than in single ones:
 // forward at 1024 workgroups 38 -> 44, dQ at 384 145 -> 145 and 245 -> 253, dK + dV unmasked at 256 191 -> 191 and 114 -> 115.5, at 128
-// 96 -> 93.  Heads of 128: the forward alone (dQ 187 -> 188; dK + dV spills, 187 -> 326), and only up to 256 (at 512 65 -> 72).
+// 96 -> 93.  Heads of 128 (the step at 256 workgroups): dQ 163 -> 158.5, unmasked 189 -> 187, at 128
+// workgroups 152 -> 147; dK + dV would spill (187 -> 326); and only up to 256 (forward at 512 65 -> 72).
 enum { FM_GRP_PV, FM_GRP_DS, FM_GRP_DV };
 inline bool two_groups(int kind, int dh, int64_t workgroups, bool causal, int n_str) {
   if (kind == FM_GRP_PV) return workgroups <= (causal && dh <= 64 && n_str >= 1024 ? 512 : 256);
-  return dh <= 64 && workgroups <= (kind == FM_GRP_DV && !causal ? 128 : 256);
+  return workgroups <= (kind == FM_GRP_DV && !causal ? 128 : 256);      // (dK + dV of heads of 128 is not built so)
 }
 
 template <typename TIO, typename E, int DH, int QT, int OWN, int QF = 0>
@@ -454,7 +455,7 @@ int launch_ds(const TokArgs<TIO, E>& a, int bh, int kernel_id, fm_stream_t strea
   typedef TokCfg<E, DH, QT> C;
   ProfScope prof(kernel_id, stream);
   const fm_dim3 grid((a.n_own + C::QW - 1) / C::QW, bh);
-  if constexpr (sizeof(E) == 2 && DH <= 64 && QT == 1 && !STR && (PREP || DV)) {
+  if constexpr (sizeof(E) == 2 && (DH <= 64 || PREP) && QT == 1 && !STR && (PREP || DV)) {
     if (!a.use_state && two_groups(DV ? FM_GRP_DV : FM_GRP_DS, DH, int64_t(grid.x) * bh, a.causal, a.n_str)) {
       constexpr size_t lds = 2 * (DV ? C::GRP_DV : C::GRP_DS);
       fm_allow_lds(reinterpret_cast<const void*>(&k_ds<TIO, E, DH, QT, OWN, DV, PREP, QF, STR, 2>), lds);
