@@ -57,14 +57,83 @@ template <int DH> FM_DEVICE void fm_decode_row(int r, bool quad, int& m, int& l,
   } else { m = DH; l = DH; live = false; }
 }
 
+// A thread's rows of a workgroup's [R][4] block (every 512th) in registers, and the tokens added to them one after the other.
+template <typename TIO, int DH> struct DecRows {
+  static constexpr int TB = 16;                          // new tokens staged at a time
+  static constexpr int NI = (int(fm_decode_rows(DH, true)) + FM_DEC_THREADS - 1) / FM_DEC_THREADS;   // rows per thread at most
+  fm_f32x4 acc[NI];
+  float dsum[NI], rmult[NI];
+  int rm[NI], rl[NI];
+  bool rlive[NI];
+  FM_DEVICE void load(const float* num, const float* den, int R, bool quad, bool fresh, int tid) {
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int r = tid + FM_DEC_THREADS * i;
+      rlive[i] = false; rm[i] = DH; rl[i] = DH; rmult[i] = 1.0f; dsum[i] = 0.f;
+      acc[i] = fm_f32x4{0.f, 0.f, 0.f, 0.f};
+      if (r < R) {
+        if (!fresh) {
+          acc[i] = *reinterpret_cast<const fm_f32x4*>(num + int64_t(r) * 4);
+          dsum[i] = den[r];
+        }
+        fm_decode_row<DH>(r, quad, rm[i], rl[i], rlive[i], rmult[i]);
+      }
+    }
+  }
+  // ks: k' of the staged tokens, [DH] = 1; vs: their four value columns (16-byte aligned).  Begins with a barrier.
+  FM_DEVICE void add(const TRef<const TIO>& k, const TRef<const TIO>& v, int bh, int c4, int n_new, float inv_tau, float (*ks)[DH + 1],
+                     float (*vs)[4], int tid) {
+    for (int t0 = 0; t0 < n_new; t0 += TB) {
+      FM_SYNC();
+      for (int i = tid; i < TB * (DH + 1); i += FM_DEC_THREADS) {
+        const int t = i / (DH + 1), f = i % (DH + 1);
+        float x = 0.f;
+        if (t0 + t < n_new) x = f < DH ? IO<TIO>::ld(k.base(bh) + int64_t(t0 + t) * k.s_n + f) * inv_tau : 1.0f;
+        ks[t][f] = x;
+      }
+      if (tid < TB * 4) {
+        const int t = tid / 4, f = tid % 4;
+        vs[t][f] = (t0 + t < n_new) ? IO<TIO>::ld(v.base(bh) + int64_t(t0 + t) * v.s_n + c4 + f) : 0.f;
+      }
+      FM_SYNC();
+      const int nt = n_new - t0 < TB ? n_new - t0 : TB;
+      for (int t = 0; t < nt; ++t) {
+        const fm_f32x4 vc = *reinterpret_cast<const fm_f32x4*>(&vs[t][0]);
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+          const float w = rlive[i] ? ks[t][rm[i]] * ks[t][rl[i]] : 0.f;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) acc[i][j] += w * vc[j];
+          dsum[i] += w;
+        }
+      }
+    }
+  }
+  FM_DEVICE void store(float* num, float* den, int R, int64_t Rp, bool fresh, int tid) const {
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int r = tid + FM_DEC_THREADS * i;
+      if (r < R) {
+        *reinterpret_cast<fm_f32x4*>(num + int64_t(r) * 4) = acc[i];
+        den[r] = dsum[i];
+      }
+    }
+    if (fresh) {                                         // the padding behind the last row
+      for (int64_t r = R + tid; r < Rp; r += FM_DEC_THREADS) {
+        *reinterpret_cast<fm_f32x4*>(num + r * 4) = fm_f32x4{0.f, 0.f, 0.f, 0.f};
+        den[r] = 0.f;
+      }
+    }
+  }
+};
+
 template <typename TIO, int DH>
 FM_GLOBAL void FM_LAUNCH_BOUNDS(FM_DEC_THREADS)
 k_decode(TRef<const TIO> k, TRef<const TIO> v, TRef<const TIO> q, int n_new, int quad, float inv_tau, float a0,
          float a1, float a2, float* FM_RESTRICT state, TRef<TIO> o, TRef<float> g, int has_q, int fresh) {
-  constexpr int TB = 16;                                 // new tokens staged at a time
-  constexpr int NI = (int(fm_decode_rows(DH, true)) + FM_DEC_THREADS - 1) / FM_DEC_THREADS;   // rows per thread at most
-  FM_SHARED float ks[TB][DH + 1];                        // k' of the staged tokens, [DH] = 1
-  FM_SHARED __attribute__((aligned(16))) float vs[TB][4];
+  typedef DecRows<TIO, DH> W;
+  FM_SHARED float ks[W::TB][DH + 1];
+  FM_SHARED __attribute__((aligned(16))) float vs[W::TB][4];
   FM_SHARED float qs[DH + 1];
   FM_SHARED float red[FM_DEC_THREADS / 64][5];
   const int tid = FM_TID_X, cb = FM_BID_X, bh = FM_BID_Y, c4 = 4 * cb;
@@ -72,79 +141,27 @@ k_decode(TRef<const TIO> k, TRef<const TIO> v, TRef<const TIO> q, int n_new, int
   const int64_t Rp = fm_decode_rows_padded(DH, quad != 0);
   float* num = state + (int64_t(bh) * (DH / 4) + cb) * Rp * 5;
   float* den = num + Rp * 4;
-  fm_f32x4 acc[NI];
-  float dsum[NI], rmult[NI];
-  int rm[NI], rl[NI];
-  bool rlive[NI];
+  W w;
   // the query travels with the state's rows (one memory latency for both)
   float qreg = 1.0f;
   if (has_q && tid < DH) qreg = IO<TIO>::ld(q.base(bh) + tid);
-#pragma unroll
-  for (int i = 0; i < NI; ++i) {
-    const int r = tid + FM_DEC_THREADS * i;
-    rlive[i] = false; rm[i] = DH; rl[i] = DH; rmult[i] = 1.0f; dsum[i] = 0.f;
-    acc[i] = fm_f32x4{0.f, 0.f, 0.f, 0.f};
-    if (r < R) {
-      if (!fresh) {
-        acc[i] = *reinterpret_cast<const fm_f32x4*>(num + int64_t(r) * 4);
-        dsum[i] = den[r];
-      }
-      fm_decode_row<DH>(r, quad != 0, rm[i], rl[i], rlive[i], rmult[i]);
-    }
-  }
+  w.load(num, den, R, quad != 0, fresh != 0, tid);
   if (has_q && tid <= DH) qs[tid] = qreg;             // read after the barriers of the token loop
-  for (int t0 = 0; t0 < n_new; t0 += TB) {
-    FM_SYNC();
-    for (int i = tid; i < TB * (DH + 1); i += FM_DEC_THREADS) {
-      const int t = i / (DH + 1), f = i % (DH + 1);
-      float x = 0.f;
-      if (t0 + t < n_new) x = f < DH ? IO<TIO>::ld(k.base(bh) + int64_t(t0 + t) * k.s_n + f) * inv_tau : 1.0f;
-      ks[t][f] = x;
-    }
-    if (tid < TB * 4) {
-      const int t = tid / 4, f = tid % 4;
-      vs[t][f] = (t0 + t < n_new) ? IO<TIO>::ld(v.base(bh) + int64_t(t0 + t) * v.s_n + c4 + f) : 0.f;
-    }
-    FM_SYNC();
-    const int nt = n_new - t0 < TB ? n_new - t0 : TB;
-    for (int t = 0; t < nt; ++t) {
-      const fm_f32x4 vc = *reinterpret_cast<const fm_f32x4*>(&vs[t][0]);
-#pragma unroll
-      for (int i = 0; i < NI; ++i) {
-        const float w = rlive[i] ? ks[t][rm[i]] * ks[t][rl[i]] : 0.f;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] += w * vc[j];
-        dsum[i] += w;
-      }
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < NI; ++i) {
-    const int r = tid + FM_DEC_THREADS * i;
-    if (r < R) {
-      *reinterpret_cast<fm_f32x4*>(num + int64_t(r) * 4) = acc[i];
-      den[r] = dsum[i];
-    }
-  }
-  if (fresh) {                                           // the padding behind the last row
-    for (int64_t r = R + tid; r < Rp; r += FM_DEC_THREADS) {
-      *reinterpret_cast<fm_f32x4*>(num + r * 4) = fm_f32x4{0.f, 0.f, 0.f, 0.f};
-      den[r] = 0.f;
-    }
-  }
+  w.add(k, v, bh, c4, n_new, inv_tau, ks, vs, tid);
+  w.store(num, den, R, Rp, fresh != 0, tid);
   if (!has_q) return;
   // readout of the new token's query: the thread's rows, then the wavefront (a butterfly: every lane ends with the
   // same sum), then the wavefronts in order
   if (n_new <= 0) FM_SYNC();                           // (no token: qs has not met a barrier yet)
   float f[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int i = 0; i < NI; ++i) {
+  for (int i = 0; i < W::NI; ++i) {
     const int r = tid + FM_DEC_THREADS * i;
     const float coef = r == 0 ? a0 : (r <= DH ? a1 : a2);
-    const float w = rlive[i] ? coef * rmult[i] * qs[rm[i]] * qs[rl[i]] : 0.f;
+    const float x = w.rlive[i] ? coef * w.rmult[i] * qs[w.rm[i]] * qs[w.rl[i]] : 0.f;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) f[j] += w * acc[i][j];
-    f[4] += w * dsum[i];
+    for (int j = 0; j < 4; ++j) f[j] += x * w.acc[i][j];
+    f[4] += x * w.dsum[i];
   }
 #pragma unroll
   for (int j = 0; j < 5; ++j) {
@@ -160,7 +177,7 @@ k_decode(TRef<const TIO> k, TRef<const TIO> v, TRef<const TIO> q, int n_new, int
     // each of the four output threads adds its column and the denominator itself (one barrier less than a shared sum)
     float sum = 0.f, gs = 0.f;
 #pragma unroll
-    for (int w = 0; w < FM_DEC_THREADS / 64; ++w) { sum += red[w][tid]; gs += red[w][4]; }
+    for (int i = 0; i < FM_DEC_THREADS / 64; ++i) { sum += red[i][tid]; gs += red[i][4]; }
     IO<TIO>::st(o.base(bh) + c4 + tid, sum / gs);
     if (tid == 0 && cb == 0) g.base(bh)[0] = gs;
   }
@@ -453,6 +470,11 @@ k_decode_absorb_mma(TRef<const TIO> k, TRef<const TIO> v, int n_new, float inv_t
 // The same sums from fp32 products, for fp32 tensors, order 1 and heads of 32.  A matrix instruction takes two tokens; its operands
 // are single floats of the staged rows (key rows [token][feature], x rows [token][8]), read across the lanes without conflicts.
 // The matrix pipe bounds it: 4.5 instructions of 64 cycles per two tokens, wavefront and order-2 problem at D = 64.
+//
+// Its order-2 terms are (k'_a v) k'_b, those of k_decode (k'_a k'_b) v.  A product k'_a v that overflows leaves a sum that is not
+// finite (infinity times a feature of zero is not a number); a workgroup that finds one adds its tokens one after the other
+// after all.  (That code costs 3 of 237 us at 16 heads of 3001 tokens; looking at every product took 73.)  One below 2^-126 is off by
+// at most 2^-150, times k'_b.
 template <int DH> struct DecAbsF32Cfg {
   static constexpr int TT = 64;                        // tokens per tile
   static constexpr int PQ = DH + 4;
@@ -470,6 +492,8 @@ k_decode_absorb_f32(TRef<const TIO> k, TRef<const TIO> v, int n_new, float inv_t
   typedef AbsSums<DH, QUAD> S;
   constexpr int TT = C::TT, PQ = C::PQ, XR = FM_ABS_XR, NT = DH / 32, NG = FM_ABS_GROUPS;
   FM_DYN_SMEM(smem);
+  FM_SHARED int bad;
+  if (QUAD && FM_TID_X == 0) bad = 0;
   const int lane = FM_TID_X & 63, lr = lane & 31, lh = lane >> 5;
   const int wave8 = FM_UNIFORM(FM_TID_X >> 6), wave = wave8 & 3, grp = wave8 >> 2;
   const int tid = FM_TID_X & 255;
@@ -562,6 +586,27 @@ k_decode_absorb_f32(TRef<const TIO> k, TRef<const TIO> v, int n_new, float inv_t
     }
     FM_SYNC_LDS();
     par ^= 1;
+  }
+  if constexpr (QUAD) {
+    float top = 0.f;
+#pragma unroll
+    for (int i = 0; i < S::NP; ++i)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) top += fm_absf(col[i][e]);
+    if (!(top < 0x1p127f)) bad = 1;
+    FM_SYNC_LDS();
+    if (__builtin_expect(FM_UNIFORM(bad) != 0, 0)) {
+      typedef DecRows<TIO, DH> W;
+      static_assert(FM_ABS_THREADS == FM_DEC_THREADS && sizeof(float[W::TB][DH + 1]) % 16 == 0, "the threads and the LDS of k_decode");
+      float (*ks)[DH + 1] = reinterpret_cast<float (*)[DH + 1]>(smem);
+      float (*vs)[4] = reinterpret_cast<float (*)[4]>(smem + sizeof(float[W::TB][DH + 1]));
+      constexpr int R = int(fm_decode_rows(DH, true));
+      W w;
+      w.load(num, den, R, true, fresh != 0, FM_TID_X);
+      w.add(k, v, bh, c4, n_new, inv_tau, ks, vs, FM_TID_X);
+      w.store(num, den, R, Rp, fresh != 0, FM_TID_X);
+      return;
+    }
   }
   fm_absorb_finish<DH, QUAD>(col, sh, reinterpret_cast<float*>(smem), num, den, fresh != 0);
 }

@@ -233,3 +233,35 @@ def check_upstream_gradients_at_the_ends_of_the_range(lib, bh, n, d, device, *, 
         ref = oracle_all(q, k, v, go, mask=False, tau=tau, p=2)
         eq, ev = rel_err(dq, ref[2]), rel_err(dv, ref[4])
         assert eq < TOL[torch.bfloat16] and ev < TOL[torch.bfloat16], f"dO x {go_scale:g}: dq {eq:.3e}, dv {ev:.3e}"
+
+
+def check_prompt_at_the_ends_of_the_range(lib, d, dtype, device, n, *, bh=2, seed=0):
+    """Order-2 sums of a prompt of 64 tokens and more, one token of which has a key of very different features (most of them zero) and
+    a value at an end of the range: products k'_a v overflow where k'_a k'_b v do not.  The state is that of the same tokens
+    added one after the other: every sum within n 2^-23 of the sizes of its terms (two roundings per term, n of the sums), infinite
+    where that one is."""
+    inv_tau = 0.125                                            # exact: k' is what is meant
+    for t, x, big, small in ((n - 2, 1e38, 8.0, 1e-3), (3, 3e38, 1.25, 1e-30), (40, 1e-37, 2.0, 0.5), (5, 1e25, 1e-10, 1e-25)):
+        gen = torch.Generator().manual_seed(seed)
+        k, v = (torch.randn(bh, n, d, generator=gen) for _ in range(2))
+        k[0, t] = 0.0
+        k[0, t, 1], k[0, t, d - 1] = big / inv_tau, small / inv_tau
+        v[0, t] = 0.5
+        v[0, t, 5] = x
+        k, v = k.to(dtype).to(device), v.to(dtype).to(device)
+        if x < 1.0:
+            v[0, :t, 5] = v[0, t + 1:, 5] = 0.0                # nothing beside the tiny terms
+        kw = dict(inv_tau=inv_tau, p=2, a0=1.0, a1=1.0, a2=0.5)
+        one, want, size = (lib.decode_state(k, **kw) for _ in range(3))
+        new = torch.full_like(one, float("nan"))
+        lib.decode_absorb(k, v, one, **kw)
+        lib.decode_absorb(k, v, new, new=True, **kw)
+        for t0 in range(0, n, 48):
+            lib.decode_absorb(k[:, t0:t0 + 48], v[:, t0:t0 + 48], want, **kw)
+            lib.decode_absorb(k[:, t0:t0 + 48].abs(), v[:, t0:t0 + 48].abs(), size, **kw)
+        one, new, want, size = (s.cpu() for s in (one, new, want, size))
+        assert torch.equal(one, new) and not bool(torch.isnan(want).any())
+        assert torch.equal(torch.isinf(one), torch.isinf(want))
+        finite = torch.isfinite(want)
+        off = (one[finite].double() - want[finite].double()).abs() / (n * 2.0 ** -23 * size[finite].double()).clamp_min(1e-44)
+        assert float(off.max()) <= 1.0, f"v = {x:g}: {float(off.max()):g} of the bound"

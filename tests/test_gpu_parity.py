@@ -4,7 +4,7 @@ bf16-rounded inputs)."""
 import pytest
 import torch
 
-from tests.parity import (check_infinite_and_largest_values, check_tiny_values, check_upstream_gradients_at_the_ends_of_the_range, check_batch_head_strides, check_decode, check_forward, check_forward_backward,
+from tests.parity import (check_infinite_and_largest_values, check_prompt_at_the_ends_of_the_range, check_tiny_values, check_upstream_gradients_at_the_ends_of_the_range, check_batch_head_strides, check_decode, check_forward, check_forward_backward,
                           check_norm_fold, make_inputs)
 from reproducing_fastmax_results_amd._capi import FLAG_F32_COMPUTE, FLAG_FORCE_DENSE, FLAG_FORCE_MOMENTS, FLAG_NORM_SELF
 
@@ -488,6 +488,12 @@ def test_prompt_sums(lib, dtype, p, d, n):
     live = small.abs() > 1e-3 * small.abs().max()
     assert float(((one - small).abs() / small.abs().clamp_min(1e-30))[live].max()) < (5e-3 if half else n * 2.0 ** -24 * 1e3)
 
+
+
+@pytest.mark.parametrize("dtype,d,n", [(torch.float32, 64, 64), (torch.float32, 64, 300), (torch.float32, 32, 129), (torch.bfloat16, 32, 200)])
+def test_prompt_at_the_ends_of_the_range(lib, dtype, d, n):
+    print(f"case prompt at the ends of the range {dtype} d={d} n={n}", flush=True)
+    check_prompt_at_the_ends_of_the_range(lib, d, dtype, DEV, n, seed=36)
 
 
 @pytest.mark.parametrize("go_scale", [1e-7, 1e-4, 3e4])

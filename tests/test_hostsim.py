@@ -16,7 +16,7 @@ import pytest
 import torch
 
 from reproducing_fastmax_results_amd import _capi
-from tests.parity import (TOL, check_upstream_gradients_at_the_ends_of_the_range, check_infinite_and_largest_values, check_tiny_values, check_batch_head_strides, check_decode, check_norm_fold, check_forward, check_forward_backward, make_inputs, oracle_all,
+from tests.parity import (TOL, check_upstream_gradients_at_the_ends_of_the_range, check_infinite_and_largest_values, check_tiny_values, check_batch_head_strides, check_decode, check_norm_fold, check_prompt_at_the_ends_of_the_range, check_forward, check_forward_backward, make_inputs, oracle_all,
                           rel_err)
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -302,6 +302,11 @@ def test_prompt_absorbed_with_matrix_instructions(sim):
             sim.decode_absorb(k[:, t0:t0 + 48], v[:, t0:t0 + 48], s2, **kw)
         assert torch.equal(s1, s3)
         assert float((s1 - s2).norm() / s2.norm()) < (1e-5 if dtype == torch.bfloat16 and p == 2 else 1e-6)
+
+
+def test_prompt_at_the_ends_of_the_range(sim):
+    check_prompt_at_the_ends_of_the_range(sim, 32, torch.float32, "cpu", 66, bh=1, seed=34)
+    check_prompt_at_the_ends_of_the_range(sim, 32, torch.bfloat16, "cpu", 66, bh=1, seed=35)
 
 
 def test_bf16_value_range_on_the_cpu(sim):
