@@ -569,6 +569,9 @@ int64_t head_size(const torch::Tensor& t, bool wide) {
 }
 // `ts` (q, k and v, or dO), each padded where it needs it; those that agree in batch*heads, head size and type in one launch.
 void pad_features(std::initializer_list<torch::Tensor*> ts, bool wide) {
+  bool fit = true;
+  for (const torch::Tensor* t : ts) fit = t->size(-1) == head_size(*t, wide) && fit;
+  if (fit) return;
   std::vector<View> views;
   std::vector<FastmaxNormDesc> nds;
   std::vector<torch::Tensor*> todo;
@@ -675,7 +678,10 @@ struct AttentionNode : public torch::autograd::Function<AttentionNode> {
   static torch::Tensor forward(torch::autograd::AutogradContext* ctx, const torch::Tensor& q, const torch::Tensor& k,
                                const torch::Tensor& v, const AttnConfig& c) {
     AttnResult r = attention_forward(q, k, v, c, true);
-    ctx->save_for_backward({r.q, r.k, r.v, r.o, r.g, r.saved, r.qk, r.kk, r.rq, r.rk});
+    // (what a call has, no undefined ones beside it: a classifier layer's step is bound by host time)
+    if (c.norm == kNormCentred) ctx->save_for_backward({r.q, r.k, r.v, r.o, r.g, r.saved, r.rq, r.rk});
+    else if (r.qk.defined()) ctx->save_for_backward({r.q, r.k, r.v, r.o, r.g, r.saved, r.qk, r.kk});
+    else ctx->save_for_backward({r.q, r.k, r.v, r.o, r.g, r.saved});
     ctx->saved_data["d"] = q.size(-1);
     ctx->saved_data["ip"] = std::vector<int64_t>{c.norm, c.p, r.fold, r.self, c.mask};
     ctx->saved_data["fp"] = std::vector<double>{c.inv_tau, c.a0, c.a1, c.a2, c.lim};
@@ -689,11 +695,13 @@ struct AttentionNode : public torch::autograd::Function<AttentionNode> {
     const std::vector<double> fp = ctx->saved_data["fp"].toDoubleVector();
     torch::Tensor go = grads[0];
     if (s[0].size(-1) != d) pad_features({&go}, true);
-    NormArgs na{s[6], s[7], fp[4], ip[0] == kNormGradOfRaw, ip[3] != 0};
+    NormArgs na;
+    na.lim = fp[4]; na.grad = ip[0] == kNormGradOfRaw; na.self = ip[3] != 0;
+    if (fold && !na.self) { na.q_keys = s[6]; na.k_keys = s[7]; }
     std::vector<torch::Tensor> r = backward_any(s[0], s[1], s[2], s[3], s[4], go, &s[5], mask, fp[0], fp[1], fp[2], fp[3], ip[1], 0,
                                                 FASTMAX_FLAG_SAVE_FOR_BACKWARD, fold ? &na : nullptr);
     if (ip[0] == kNormCentred && (ctx->needs_input_grad(0) || ctx->needs_input_grad(1))) {
-      NormPass a = backward_pass(s[8], r[0], kCentreToken, true, fp[4]), b = backward_pass(s[9], r[1], kCentreToken, true, fp[4]);
+      NormPass a = backward_pass(s[6], r[0], kCentreToken, true, fp[4]), b = backward_pass(s[7], r[1], kCentreToken, true, fp[4]);
       run(a, b);
       r[0] = a.out; r[1] = b.out;
     }
