@@ -405,13 +405,13 @@ const NormFold no_fold{nullptr, 0, 1.0f};
 
 template <typename TIO, typename E> void tok_common(TokArgs<TIO, E>& a, const FastmaxDesc* d, const Plan& p) {
   a.own_fold = no_fold; a.out_fold = no_fold; a.brows = nullptr; a.bpart = nullptr;
-  a.own_io = TRef<const TIO>{nullptr, 0, 0, 0, 0, 0};
+  a.own_io = TRef<const TIO>{};
   a.own_r = nullptr; a.own2_r = nullptr; a.cv = nullptr; a.xr = nullptr; a.yr = nullptr; a.zt = nullptr; a.zt2 = nullptr; a.bigb = nullptr;
-  a.out2 = TRef<TIO>{nullptr, 0, 0, 0, 0, 0}; a.out2_scale = 1.0f;
-  a.g = TRef<float>{nullptr, 0, 0, 0, 0, 0};
+  a.out2 = TRef<TIO>{}; a.out2_scale = 1.0f;
+  a.g = TRef<float>{};
   a.nslots = p.nslots; a.L = p.L; a.nseg = p.nseg; a.causal = d->mask != 0; a.use_state = p.use_state;
   a.quad = p.quad; a.a0 = p.a0; a.a1 = p.a1; a.a2 = p.a2; a.sc = p.sc; a.out_scale = 1.0f; a.zscale = 1.0f;
-  a.own_o = TRef<const TIO>{nullptr, 0, 0, 0, 0, 0}; a.own_do = a.own_o;
+  a.own_o = TRef<const TIO>{}; a.own_do = a.own_o;
   a.w_gh = nullptr; a.w_qr = nullptr; a.w_cv = nullptr; a.gpart = nullptr; a.gnblk = 0;
   a.out_resid = nullptr; a.own_ores = nullptr; a.state_xscale = 1.0f;
 }
@@ -491,7 +491,7 @@ template <typename TIO, int DH>
 int o1_key_sums(const FastmaxDesc* d, const Plan& p, const void* k, const void* v, fm_half* big, float* small,
                 float* runtot, fm_half* runhalf, fm_stream_t stream) {
   O1SumArgs<TIO> a;
-  a.x0 = cref<TIO>(k, d->sk); a.x1 = cref<TIO>(v, d->sv); a.o = a.x0; a.g = TRef<const float>{nullptr, 0, 0, 0, 0, 0};
+  a.x0 = cref<TIO>(k, d->sk); a.x1 = cref<TIO>(v, d->sv); a.o = a.x0; a.g = TRef<const float>{};
   a.scale0 = p.sc; a.fold0 = k_fold(d); a.gpart = nullptr; a.gnblk = 0; a.n = d->nk; a.runtot = runtot; a.run_len = p.o1_run;
   BuildArgs<fm_half>& b = a.b;
   b.xt = nullptr; b.pt = nullptr; b.rt = nullptr; b.zt = nullptr; b.pr = nullptr; b.rr = nullptr; b.cw = nullptr;
@@ -534,8 +534,8 @@ inline int x3_split(int bh, int n_own, int tokens) {
 template <typename TIO> X3Args<TIO> x3_args(const FastmaxDesc* d, const Plan& p, const void* q, const void* k, const void* v) {
   X3Args<TIO> a;
   a.q = cref<TIO>(q, d->sq); a.k = cref<TIO>(k, d->sk); a.v = cref<TIO>(v, d->sv);
-  a.o = TRef<const TIO>{nullptr, 0, 0, 0, 0, 0}; a.d_o = a.o; a.out = TRef<TIO>{nullptr, 0, 0, 0, 0, 0}; a.out2 = a.out;
-  a.g = TRef<float>{nullptr, 0, 0, 0, 0, 0};
+  a.o = TRef<const TIO>{}; a.d_o = a.o; a.out = TRef<TIO>{}; a.out2 = a.out;
+  a.g = TRef<float>{};
   a.cv = nullptr; a.out_resid = nullptr; a.ores = nullptr; a.bpart = nullptr;
   a.nq = d->nq; a.nk = d->nk; a.npad_q = p.npad_q; a.causal = d->mask != 0;
   a.a0 = p.a0; a.a1 = p.a1; a.a2 = p.a2; a.sc = p.sc;
@@ -573,9 +573,9 @@ int launch_x3(const X3Args<TIO>& a, int split, int n_own, int bh, fm_stream_t st
 template <typename TIO> SmallArgs<TIO> small_args(const FastmaxDesc* d, const Plan& p, const void* q, const void* k, const void* v) {
   SmallArgs<TIO> a;
   a.q = cref<TIO>(q, d->sq); a.k = cref<TIO>(k, d->sk); a.v = cref<TIO>(v, d->sv);
-  a.o = TRef<const TIO>{nullptr, 0, 0, 0, 0, 0}; a.d_o = a.o;
-  a.out = TRef<TIO>{nullptr, 0, 0, 0, 0, 0}; a.dk = a.out; a.dv = a.out;
-  a.g = TRef<float>{nullptr, 0, 0, 0, 0, 0};
+  a.o = TRef<const TIO>{}; a.d_o = a.o;
+  a.out = TRef<TIO>{}; a.dk = a.out; a.dv = a.out;
+  a.g = TRef<float>{};
   a.out_resid = nullptr; a.ores = nullptr; a.npad_q = d->nq;
   a.nq = d->nq; a.nk = d->nk; a.causal = d->mask != 0;
   a.a0 = p.a0; a.a1 = p.a1; a.a2 = p.a2; a.sc = p.sc;

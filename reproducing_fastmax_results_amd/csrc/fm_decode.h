@@ -645,8 +645,8 @@ int fm_decode_run(const FastmaxDesc* d, const void* q, const void* k, const void
     }
     return fm_absorb_launch_f32<TIO, DH, false>(d, kr, vr, n_new, state, fresh, stream);
   }
-  const TRef<TIO> orf = q ? fm_ref<TIO>(static_cast<TIO*>(o), d->so) : TRef<TIO>{nullptr, 0, 0, 0, 0, 0};
-  const TRef<float> grf = q ? fm_ref<float>(g, d->sg) : TRef<float>{nullptr, 0, 0, 0, 0, 0};
+  const TRef<TIO> orf = q ? fm_ref<TIO>(static_cast<TIO*>(o), d->so) : TRef<TIO>{};
+  const TRef<float> grf = q ? fm_ref<float>(g, d->sg) : TRef<float>{};
   FM_KERNEL_LAUNCH((k_decode<TIO, DH>), fm_dim3(DH / 4, d->bh), fm_dim3(FM_DEC_THREADS), 0, stream, kr, vr, qr, n_new, quad ? 1 : 0,
                    d->inv_tau, d->a0, d->a1, quad ? d->a2 : 0.0f, state, orf, grf, q ? 1 : 0, fresh);
   return fm_after_launch() ? FASTMAX_ERR_LAUNCH : FASTMAX_OK;

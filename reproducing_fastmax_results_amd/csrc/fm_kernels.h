@@ -99,8 +99,8 @@ struct TileRegs {
   }
 };
 
-// Eight elements of row `row` of a caller tensor of n rows; a row outside it reads the nearest one and becomes zeros.  (A branch per
-// row would hold the load and its conversion, and every load would wait for the one before it.)
+// Eight elements of row `row` >= 0 of a caller tensor of n >= 1 rows; a row past the end reads the last one and becomes zeros.  (A
+// branch per row would hold the load and its conversion, and every load would wait for the one before it.)
 template <typename TIO> FM_DEVICE void fm_ld8_row(const TIO* base, int64_t s_n, int row, int n, int col, float v[8]) {
   const int rc = row < n ? row : n - 1;
   IO<TIO>::ld8(base + int64_t(rc) * s_n + col, v);
@@ -143,10 +143,11 @@ struct RowRegs {
   }
 };
 
-// A caller tensor: base pointer, strides in elements, whether 16-byte accesses are aligned.
+// A caller tensor: base pointer and strides in elements.
 template <typename TIO> struct TRef {
-  TIO* p; int64_t s_bh, s_n; int vec; int64_t s_b; int heads;
-  uint32_t inv;                                        // heads > 1: 2^32 / heads rounded up
+  TIO* p = nullptr; int64_t s_bh = 0, s_n = 0, s_b = 0;
+  int heads = 0;
+  uint32_t inv = 0;                                    // heads > 1: 2^32 / heads rounded up
   // First element of batch*head slice bh (one stride, or batch and head strides when heads > 1).  bh / heads is the high half of
   // one product, exact for bh and heads below 2^16 (a division is some 40 instructions one behind the other, per tensor).
   FM_DEVICE TIO* base(int bh) const {
@@ -156,14 +157,9 @@ template <typename TIO> struct TRef {
 };
 
 // host side: TRef of a caller pointer and its FastmaxStrides
-template <typename T> inline bool fm_vec_ok(const void* ptr, const FastmaxStrides& s) {
-  const int64_t a = 16 / int64_t(sizeof(T));          // elements per 16 bytes
-  return (reinterpret_cast<uintptr_t>(ptr) % 16 == 0) && (s.n % a == 0) && (s.bh % a == 0) &&
-         (s.heads <= 1 || s.b % a == 0);
-}
 template <typename T> inline TRef<T> fm_ref(T* ptr, const FastmaxStrides& s) {
   TRef<T> r;
-  r.p = ptr; r.s_bh = s.bh; r.s_n = s.n; r.vec = fm_vec_ok<T>(ptr, s) ? 1 : 0;
+  r.p = ptr; r.s_bh = s.bh; r.s_n = s.n;
   r.s_b = s.heads > 1 ? s.b : 0; r.heads = s.heads > 1 ? s.heads : 0;
   r.inv = s.heads > 1 ? uint32_t(((uint64_t(1) << 32) + uint32_t(s.heads) - 1) / uint32_t(s.heads)) : 0;
   return r;
