@@ -426,7 +426,15 @@ template <typename TIO, typename E> void tok_common(TokArgs<TIO, E>& a, const Fa
 // 96 -> 93.  Heads of 128 (the step at 256 workgroups): dQ 163 -> 158.5, unmasked 189 -> 187, at 128
 // workgroups 152 -> 147; dK + dV would spill (187 -> 326); and only up to 256 (forward at 512 65 -> 72).
 enum { FM_GRP_PV, FM_GRP_DS, FM_GRP_DV };
+#if defined(FM_HOSTSIM)
+// The CPU tests run launches of a few workgroups, which all go with two groups: set, they go with one, as larger launches do.
+static bool fm_hostsim_one_group = false;
+extern "C" void fastmax_hostsim_one_group(int on) { fm_hostsim_one_group = on != 0; }
+#endif
 inline bool two_groups(int kind, int dh, int64_t workgroups, bool causal, int n_str) {
+#if defined(FM_HOSTSIM)
+  if (fm_hostsim_one_group) return false;
+#endif
   if (kind == FM_GRP_PV) return workgroups <= (causal && dh <= 64 && n_str >= 1024 ? 512 : 256);
   return workgroups <= (kind == FM_GRP_DV && !causal ? 128 : 256);      // (dK + dV of heads of 128 is not built so)
 }

@@ -61,7 +61,8 @@ static int run_pointwise(int bh, int n, int d, int dtype) {
   return st;
 }
 // the decoding state: a prompt absorbed, then single-token steps (buffers of exactly the sizes the library names)
-static int run_decode(int bh, int d, int p, int prompt, int steps, int dtype) {
+// fresh: into memory full of NaN that is said to be a new state.  big: a value beside which k' v overflows.
+static int run_decode(int bh, int d, int p, int prompt, int steps, int dtype, int fresh = 0, int big = 0) {
   FastmaxDesc D; memset(&D, 0, sizeof D);
   D.bh = bh; D.nq = 1; D.nk = prompt; D.d = d; D.dtype = dtype; D.mask = 1; D.p = p; D.a0 = 1; D.a1 = 1; D.a2 = .5f;
   D.inv_tau = 1.f / (2.f * std::sqrt(float(d)));
@@ -76,10 +77,12 @@ static int run_decode(int bh, int d, int p, int prompt, int steps, int dtype) {
     }
   };
   fill(k); fill(v); fill(q1); fill(k1); fill(v1);
+  if (big) { reinterpret_cast<float*>(v.data())[5] = 1e38f; reinterpret_cast<float*>(k.data())[1] = 1e3f; }
   const size_t sb = fastmax_decode_state_bytes(&D), cb = fastmax_decode_scratch_bytes(&D);
   if (!sb || !cb) return 99;
   float* state = static_cast<float*>(aligned_alloc(256, (sb + 255) / 256 * 256));
-  memset(state, 0, sb);
+  memset(state, fresh ? 0xff : 0, sb);
+  if (fresh) D.flags = FASTMAX_FLAG_NEW_STATE;
   float* scratch = static_cast<float*>(aligned_alloc(256, (cb + 255) / 256 * 256));
   std::vector<float> g(bh);
   int st = fastmax_decode_absorb(&D, k.data(), v.data(), state, nullptr);
@@ -87,9 +90,62 @@ static int run_decode(int bh, int d, int p, int prompt, int steps, int dtype) {
   for (int i = 0; i < steps && !st; ++i)
     st = fastmax_decode_step(&D, q1.data(), k1.data(), v1.data(), state, o1.data(), g.data(), scratch, nullptr);
   free(state); free(scratch);
-  printf("decode bh=%d d=%d p=%d prompt=%d steps=%d dtype=%d -> status %d, g[0] %.3f\n", bh, d, p, prompt, steps, dtype, st, g[0]);
+  printf("decode bh=%d d=%d p=%d prompt=%d steps=%d dtype=%d fresh=%d big=%d -> status %d, g[0] %.3f\n", bh, d, p, prompt, steps, dtype,
+         fresh, big, st, g[0]);
+  fflush(stdout);
   return st;
 }
+// heads of d features to rows of dpad: up to three tensors of their own lengths in one launch
+static int run_pad(int bh, int d, int dpad, int dtype, int count) {
+  const size_t esz = dtype == FASTMAX_BF16 ? 2 : 4;
+  const int ns[3] = {1, 70, 33};
+  FastmaxNormDesc N[3];
+  const FastmaxNormDesc* D[3];
+  std::vector<unsigned char> x[3], y[3];
+  const void* xp[3]; void* yp[3];
+  for (int i = 0; i < count; ++i) {
+    N[i] = FastmaxNormDesc();
+    N[i].bh = bh; N[i].n = ns[i]; N[i].d = d; N[i].dtype = dtype;
+    N[i].sx.bh = int64_t(ns[i]) * d; N[i].sx.n = d; N[i].sy.bh = int64_t(ns[i]) * dpad; N[i].sy.n = dpad;
+    x[i].assign(size_t(bh) * ns[i] * d * esz, 1); y[i].assign(size_t(bh) * ns[i] * dpad * esz, 7);
+    D[i] = &N[i]; xp[i] = x[i].data(); yp[i] = y[i].data();
+  }
+  const int st = fastmax_pad_features(D, xp, yp, count, dpad, nullptr);
+  printf("pad bh=%d d=%d dpad=%d dtype=%d count=%d -> status %d\n", bh, d, dpad, dtype, count, st);
+  fflush(stdout);
+  return st;
+}
+// two tensors of different lengths through the normalisation passes in common launches
+static int run_norm_pair(int bh, int n0, int n1, int d, int dtype, int centre) {
+  const size_t esz = dtype == FASTMAX_BF16 ? 2 : 4;
+  FastmaxNormDesc N[2];
+  std::vector<unsigned char> x[2], dy[2], y[2];
+  float* stats[2];
+  const int ns[2] = {n0, n1};
+  int st = 0;
+  for (int back = 0; back < 2 && !st; ++back) {
+    for (int i = 0; i < 2; ++i) {
+      N[i] = FastmaxNormDesc();
+      N[i].bh = bh; N[i].n = ns[i]; N[i].d = d; N[i].dtype = dtype; N[i].centre = centre; N[i].max_norm = 1; N[i].scale = 1.5f;
+      N[i].sx.bh = int64_t(ns[i]) * d; N[i].sx.n = d; N[i].sy = N[i].sx;
+      x[i].assign(size_t(bh) * ns[i] * d * esz, 0); dy[i] = x[i]; y[i] = x[i];
+      for (std::vector<unsigned char>* b : {&x[i], &dy[i]})
+        for (size_t j = 0; j < b->size() / esz; ++j) {
+          const float r = frand();
+          if (esz == 2) reinterpret_cast<uint16_t*>(b->data())[j] = bf16(r); else reinterpret_cast<float*>(b->data())[j] = r;
+        }
+      stats[i] = static_cast<float*>(malloc(back ? fastmax_normalize_backward_stats_bytes(&N[i]) : fastmax_normalize_stats_bytes(&N[i])));
+    }
+    st = back ? fastmax_normalize_backward_pair(&N[0], x[0].data(), dy[0].data(), y[0].data(), stats[0], &N[1], x[1].data(), dy[1].data(),
+                                                y[1].data(), stats[1], nullptr)
+              : fastmax_normalize_pair(&N[0], x[0].data(), y[0].data(), stats[0], &N[1], x[1].data(), y[1].data(), stats[1], nullptr);
+    free(stats[0]); free(stats[1]);
+  }
+  printf("norm pair bh=%d n=%d,%d d=%d dtype=%d centre=%d -> status %d\n", bh, n0, n1, d, dtype, centre, st);
+  fflush(stdout);
+  return st;
+}
+extern "C" void fastmax_hostsim_one_group(int on);
 int main() {
   int bad = 0;
   bad |= run_pointwise(3, 333, 64, FASTMAX_BF16);
@@ -97,6 +153,29 @@ int main() {
   bad |= run_decode(2, 64, 2, 37, 2, FASTMAX_BF16);
   bad |= run_decode(3, 32, 1, 5, 2, FASTMAX_F32);
   bad |= run_decode(1, 64, 2, 150, 1, FASTMAX_BF16);  // a prompt summed with matrix instructions (two tiles, the second ragged)
+  // prompts in fp32 products: one and several tiles, ragged, both orders, a new state, a sum that overflows
+  bad |= run_decode(1, 64, 2, 64, 1, FASTMAX_F32);
+  bad |= run_decode(1, 64, 2, 150, 1, FASTMAX_F32, 1);
+  bad |= run_decode(2, 32, 2, 129, 1, FASTMAX_F32, 1);
+  bad |= run_decode(1, 32, 2, 70, 1, FASTMAX_BF16, 1);
+  bad |= run_decode(1, 64, 1, 195, 1, FASTMAX_BF16, 1);
+  bad |= run_decode(1, 32, 2, 70, 1, FASTMAX_F32, 1, 1);
+  bad |= run_decode(1, 64, 2, 150, 1, FASTMAX_BF16, 1);
+  bad |= run_decode(1, 64, 2, 20, 1, FASTMAX_F32, 1);
+  bad |= run_pad(3, 48, 64, FASTMAX_F32, 3);
+  bad |= run_pad(2, 1, 32, FASTMAX_BF16, 3);
+  bad |= run_pad(2, 127, 128, FASTMAX_BF16, 2);
+  bad |= run_norm_pair(2, 70, 300, 64, FASTMAX_F32, 2);
+  bad |= run_norm_pair(1, 257, 1, 32, FASTMAX_BF16, 2);
+  bad |= run_norm_pair(1, 64, 129, 64, FASTMAX_BF16, 1);
+  // one segment in one group of wavefronts per workgroup, as launches of many workgroups run (further down: in two)
+  fastmax_hostsim_one_group(1);
+  bad |= run(2, 200, 64, 2, 0, FASTMAX_BF16, 1);
+  bad |= run(1, 130, 32, 2, 0, FASTMAX_BF16, 0);
+  bad |= run(1, 70, 64, 1, 0, FASTMAX_BF16, 1, opt(75, 0, FASTMAX_FLAG_FORCE_DENSE));
+  bad |= run(1, 200, 128, 2, 0, FASTMAX_BF16, 1);
+  bad |= run(1, 75, 128, 1, 0, FASTMAX_BF16, 0, opt(70, 0));
+  fastmax_hostsim_one_group(0);
   bad |= run(1, 300, 64, 2, 256, FASTMAX_BF16, 1);    // order-2 walk held per value column (two segments), saved and rebuilt
   bad |= run(1, 300, 64, 2, 256, FASTMAX_BF16, 0);
   bad |= run(1, 600, 32, 2, 256, FASTMAX_BF16, 1);    // order-2 walk (a CU to itself: two buffers), both walks

@@ -50,6 +50,28 @@ def test_groups_of_wavefronts_and_their_limits(lib, bh, nq, nk, d, mask):
     check_forward_backward(lib, bh, nq, d, torch.bfloat16, DEV, mask=mask, p=2, nk=nk, seed=160, saved=not (mask and nk > nq))
 
 
+@pytest.mark.parametrize("saved", [False, True])
+@pytest.mark.parametrize("p,a", [(1, (1.0, 1.0, 0.5)), (2, (1.0, 1.0, 0.03)), (2, (1.0, 1.0, 0.5))])
+@pytest.mark.parametrize("bh,nq,nk,d,mask", [(129, 129, 129, 64, True), (129, 130, 200, 32, False), (65, 1024, 1024, 32, True),
+                                             (43, 700, 700, 128, True), (129, 129, 150, 128, False)])
+def test_one_group_of_wavefronts(lib, bh, nq, nk, d, mask, p, a, saved):
+    """Launches above the limits of two groups: plain weights (order 1, and a2 outside the range of completed squares) and completed
+    squares, dQ with its preparation (saved: with what the rounding of o took), dK + dV."""
+    check_forward_backward(lib, bh, nq, d, torch.bfloat16, DEV, mask=mask, p=p, nk=nk, a=a, seed=161, saved=saved,
+                           flags=FLAG_FORCE_DENSE)
+
+
+@pytest.mark.parametrize("d", [32, 64])
+@pytest.mark.parametrize("p", [1, 2])
+def test_one_group_of_wavefronts_normalised_strided_and_small(lib, d, p):
+    """387 workgroups: the folded normalisation with its Jacobian, projection layouts, tiny upstream gradients."""
+    for saved in (False, True):
+        check_norm_fold(lib, 129, 257, d, torch.bfloat16, DEV, mask=True, p=p, seed=162, saved=saved)
+    check_norm_fold(lib, 129, 200, d, torch.bfloat16, DEV, mask=False, p=2, nk=257, seed=163, jacobian=False)
+    check_batch_head_strides(lib, 13, 10, 257, d, torch.bfloat16, DEV, mask=True, p=p, seed=164)
+    check_forward_backward(lib, 129, 257, d, torch.bfloat16, DEV, mask=True, p=p, seed=165, saved=True, go_scale=1e-7)
+
+
 def test_matrix_rate_probe_runs(bench_lib):
     """The bench's yardstick: a register-only loop of matrix products; here only that it runs, writes
     every checksum and reports a rate (16 workgroups, 64 rounds)."""

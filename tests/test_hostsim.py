@@ -57,6 +57,31 @@ def test_dense_forward_backward(sim, dtype):
     check_forward_backward(sim, 1, 33, 32, dtype, "cpu", mask=False, p=1, nk=45, seed=2)
 
 
+@pytest.fixture
+def one_group(sim):
+    sim.lib.fastmax_hostsim_one_group(1)
+    yield
+    sim.lib.fastmax_hostsim_one_group(0)
+
+
+@pytest.mark.parametrize("d,nq,nk,mask,p,saved,a", [
+    (32, 70, 70, True, 2, False, (1.0, 1.0, 0.5)), (64, 130, 130, True, 2, True, (1.0, 1.0, 0.5)),     # completed squares
+    (32, 70, 75, False, 2, True, (1.0, 1.0, 0.03)), (64, 70, 70, True, 1, True, (1.0, 1.0, 0.5)),      # plain weights
+    (64, 75, 70, False, 1, False, (1.0, 1.0, 0.5)), (128, 70, 70, True, 2, True, (1.0, 1.0, 0.5)),
+    (128, 70, 75, False, 1, False, (1.0, 1.0, 0.5))])
+def test_one_group_of_wavefronts(sim, one_group, d, nq, nk, mask, p, saved, a):
+    """The _Float16 kernels of one segment as launches of many workgroups run them."""
+    check_forward_backward(sim, 1, nq, d, torch.bfloat16, "cpu", mask=mask, p=p, nk=nk, a=a, saved=saved,
+                           flags=_capi.FLAG_FORCE_DENSE, seed=68)
+
+
+def test_one_group_of_wavefronts_normalised_strided_and_small(sim, one_group):
+    check_norm_fold(sim, 2, 70, 32, torch.bfloat16, "cpu", mask=True, p=2, seed=69)
+    check_norm_fold(sim, 1, 130, 64, torch.bfloat16, "cpu", mask=True, p=1, seed=70, saved=False)
+    check_batch_head_strides(sim, 2, 2, 70, 32, torch.bfloat16, "cpu", mask=True, p=2, seed=71)
+    check_forward_backward(sim, 1, 70, 32, torch.bfloat16, "cpu", mask=True, p=2, seed=72, go_scale=1e-7)
+
+
 def test_moment_path_forward_backward_bf16(sim):
     # two segments of 256: prefix state for the second, suffix state for the first
     check_forward_backward(sim, 1, 300, 32, torch.bfloat16, "cpu", mask=True, p=2, chunk=256, seed=3)
@@ -305,8 +330,7 @@ def test_prompt_absorbed_with_matrix_instructions(sim):
 
 
 def test_prompt_at_the_ends_of_the_range(sim):
-    check_prompt_at_the_ends_of_the_range(sim, 32, torch.float32, "cpu", 66, bh=1, seed=34)
-    check_prompt_at_the_ends_of_the_range(sim, 32, torch.bfloat16, "cpu", 66, bh=1, seed=35)
+    check_prompt_at_the_ends_of_the_range(sim, 32, torch.float32, "cpu", 66, bh=1, seed=34, cases=1)
 
 
 def test_bf16_value_range_on_the_cpu(sim):
