@@ -45,10 +45,10 @@ PEAK_HBM_GBS = 8000.0
 # (N, order, dtype, --chunk, kernel).  A constant, not a live measurement: it belongs to the kernels as they
 # were when the named summary was made.
 TRAFFIC = {
-    (4096, 2, "bf16", 0, "dkv"): {"bytes": int((42622.6 * 2 + 32768.1) * 1024), "source": "profiles/c2_bf16_hbm_traffic.md"},
-    (65536, 1, "bf16", 0, "dkv"): {"bytes": int((402949.3 * 2 + 393223.9) * 1024), "source": "profiles/long_order1_bf16_hbm_traffic.md"},
+    (4096, 2, "bf16", 0, "dkv"): {"bytes": int((42659.0 * 2 + 32768.0) * 1024), "source": "profiles/c2_bf16_hbm_traffic.md"},
+    (65536, 1, "bf16", 0, "dkv"): {"bytes": int((402845.0 * 2 + 393231.0) * 1024), "source": "profiles/long_order1_bf16_hbm_traffic.md"},
     (65536, 2, "bf16", 0, "build"): {"bytes": int((130128.6 * 2 + 544747.5) * 1024), "source": "profiles/long_order2_bf16_hbm_traffic.md"},
-    (65536, 2, "bf16", 0, "dkv"): {"bytes": int((609337.0 * 2 + 262146.4) * 1024), "source": "profiles/long_order2_bf16_hbm_traffic.md"},
+    (65536, 2, "bf16", 0, "dkv"): {"bytes": int((609633.0 * 2 + 262148.0) * 1024), "source": "profiles/long_order2_bf16_hbm_traffic.md"},
 }
 
 WORKLOAD = dict(name="configs[1]: causal order-2 fwd+bwd", B=4, H=8, N=4096, D=64, p=2, mask=True, scale=1.0)

@@ -66,7 +66,12 @@ enum {
  * with a0 <= 0 the library computes bf16 tensors in fp32 on its own, as if the flag were set.
  * fp32 tensors: every magnitude of fp32, infinities and NaN included, with fp32's 24 bits throughout.  (Dense tiles form fp32
  * products from three bf16 parts of each factor; a workgroup that meets an entry beyond about 1e31 or a sum beyond 1e23, which the
- * parts cannot hold, makes its rows a second time with fp32 products.) */
+ * parts cannot hold, makes its rows a second time with fp32 products.)
+ *
+ * Bits.  A call gives the same bits on every run.  The order in which a sum is added depends on how many workgroups the launch has,
+ * so a batch*head slice can come out with other roundings when nq, nk or the number of slices beside it changes: one-segment
+ * problems of bf16 tensors between launches of up to 128, 256 or 512 workgroups and larger ones, dense fp32 tiles
+ * at 256 and 512, a few queries with the number of parts of the keys. */
 
 /* Where slice i of the batch*head axis, token t, feature f of a tensor lives:
  *   heads <= 1:  i * bh + t * n + f
@@ -184,7 +189,7 @@ int fastmax_backward_saved(const FastmaxDesc* desc, const void* q, const void* k
  *   fastmax_decode_absorb: adds desc->nk tokens (k, v: strides sk, sv) to the state, e.g. a prompt whose
  *     own outputs come from fastmax_forward.  One launch.  64 tokens or more are summed with matrix instructions, on
  *     _Float16 operands (k', and the products v k') with fp32 sums for bf16 tensors at d = 64, order 2, on fp32 operands
- *     otherwise; fewer token after token in fp32.
+ *     otherwise (where a sum is not finite, token after token after all); fewer token after token in fp32.
  *   fastmax_decode_step: adds one token (k, v) and reads the state out for its query q (strides sq; the
  *     query sees its own key, as in causal attention): o (strides so, one token) and g (sg).  scratch is
  *     not used any more (a step is one launch; the argument and fastmax_decode_scratch_bytes stay for

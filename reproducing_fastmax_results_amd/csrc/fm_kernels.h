@@ -1273,10 +1273,6 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS(FM_SCAN_THREADS) k_state_scan(E* FM_RESTRICT big
 // ------------------------------------------------------------------------------
 // LDS sizes (in elements of E) used by k_pv / k_ds; the host computes the dynamic LDS
 // bytes from the same struct.
-// Stream tokens per stage of the dense loops of the _Float16 token kernels.  k_ds stages two row
-// tiles only (its transposed fragments come from transposing LDS reads), so 64-token stages cost it
-// no occupancy and halve its barriers (dQ 0.117 -> 0.114 ms at B*H = 32, N = 4096 on MI355X); k_pv
-// measured slower with them (0.092 vs 0.087 ms).
 template <typename E, int DH, int QT>
 struct TokCfg {
   typedef Mma<E> M;
@@ -1309,7 +1305,9 @@ struct TokCfg {
   // it; 64 tokens leave registers for three: 16 x 8 heads of 1024 tokens 38 -> 42, 4 x 8 of 4096 89 -> 90, and where a CU has one or two
   // workgroups it gains less than two groups per workgroup do (1 x 8 of 4096 55 -> 48, groups 42).
   static constexpr int KT_PV = sizeof(E) == 2 && (QT == 2 || DH == 64) ? 32 : 64;
-  static constexpr int KT_DS = 64;                        //                                           k_ds
+  // k_ds stages two row tiles only (its transposed fragments come from transposing LDS reads): 64-token stages cost it no occupancy and
+  // halve its barriers (dQ 0.117 -> 0.114 ms at B*H = 32, N = 4096)
+  static constexpr int KT_DS = 64;
   // the dK + dV pass runs two workgroups per CU whatever its stages are, and 64-token stages
   // halve its barriers (0.163 vs 0.173 ms at the shape above)
   static constexpr int KT_DV = 64;                        //                                           k_ds with dV

@@ -291,8 +291,8 @@ template <int NACC> FM_DEVICE void fm_join_groups(float* lds, fm_f32x16* acc, in
 
 // ------------------------------------------------------------------------------
 // k_pv: forward (own = queries) and dV (own = keys).  grid (ceil(n_own / QW), bh).
-// LDS: va, vb | own rows [QW][PQ] | region (Z, then state slabs); the two dense stages and the
-// output staging lie over the own rows and the region once they are spent.
+// LDS: va, vb | own rows [QW][PQ] | region (Z, then state slabs); the two dense stages lie over the own rows and the region
+// once they are spent.  Outputs leave straight from the accumulators (fm_each_octet).  GRP = 2 (no states): see fm_join_groups.
 // ------------------------------------------------------------------------------
 // QF = 1 (forward of an order-2 problem without states, _Float16): the weights in their completed-square
 // form (see TileMath<fm_half>::wq); the host picks it when a2 is of ordinary size.
@@ -597,7 +597,8 @@ FM_DEVICE void fm_readout_kv(const E* FM_RESTRICT state2, const E* xs, int xrow,
 // k_ds: dQ (own = queries) and dK (own = keys).  grid (ceil(n_own / QW), bh).
 // LDS: va, vb | own rows [QW][PQ] | region (Z, then state slabs); the dense stages
 // (stream rows for the scores, stream rows for gh.v, stream transposed, c values)
-// and the output staging lie over the own rows and the region once they are spent.
+// lie over the own rows and the region once they are spent; outputs leave straight from the accumulators.
+// GRP = 2 (no states): see fm_join_groups.
 // DV = 1 (own = keys, sequences of one segment): the same pass also forms dV from the
 // score tiles it already has, P = f(S), dV^T += gh^T P, which saves the four score
 // products per tile that a separate k_pv launch would repeat.
