@@ -202,7 +202,9 @@ template <int DH, bool QUAD> struct AbsSums {
   static constexpr int NT = DH / 32;
   static constexpr int NP = QUAD ? NT * (NT + 1) / 2 : 0;        // pair tiles (a <= b): (0,0) or (0,0), (0,1), (1,1)
   static constexpr int NSH = NP + NT + 1;                        // shared: denominators of the pairs, rows 1 .. D, row 0
-  static constexpr int RT = 3;                                   // tiles that meet in LDS at a time
+  // Tiles that meet in LDS at a time: few enough that LDS does not keep a second workgroup off a CU whose registers have room for it
+  // (three everywhere: 98 KB; order 2, 128 heads of 32: 64 tokens 28.9 us, so 21.0, 128 tokens 36.6, so 28.6)
+  static constexpr int RT = DH == 64 ? (QUAD ? 3 : 2) : 1;
   static constexpr size_t red_bytes() { return size_t(4) * FM_ABS_GROUPS * RT * 16 * 64 * 4; }
   static constexpr int pa(int i) { return i == 2 ? 1 : 0; }      // row tile and column tile of pair tile i
   static constexpr int pb(int i) { return i == 0 ? 0 : 1; }
@@ -223,8 +225,8 @@ template <typename TIO, int N> struct Raw {
 };
 
 // Everything accumulated -> state.  col: the wavefront's pair tiles, sh: its part of the shared sums; all LDS from red on is free.
-template <int DH, bool QUAD>
-FM_DEVICE void fm_absorb_finish(const fm_f32x16* col, const fm_f32x16* sh, float* red, float* num, float* den, bool fresh) {
+template <int DH, bool QUAD, bool FRESH>
+FM_DEVICE void fm_absorb_finish(const fm_f32x16* col, const fm_f32x16* sh, float* red, float* num, float* den) {
   typedef AbsSums<DH, QUAD> C;
   constexpr int NP = C::NP, NSH = C::NSH, NW = 4 * FM_ABS_GROUPS;
   const int lane = FM_TID_X & 63, lr = lane & 31, lh = lane >> 5;
@@ -244,14 +246,8 @@ FM_DEVICE void fm_absorb_finish(const fm_f32x16* col, const fm_f32x16* sh, float
       for (int i = 0; i < NP; ++i) {
         live[i][e] = C::pa(i) != C::pb(i) || ra <= lr;
         at[i][e] = num + (live[i][e] ? int64_t(pair_row(32 * C::pa(i) + ra, 32 * C::pb(i) + lr)) * 4 + wave : wave);
-        old[i][e] = 0.f;
+        old[i][e] = FRESH ? 0.f : *at[i][e];
       }
-    }
-    if (!fresh) {
-#pragma unroll
-      for (int i = 0; i < NP; ++i)
-#pragma unroll
-        for (int e = 0; e < 8; ++e) old[i][e] = *at[i][e];
     }
 #pragma unroll
     for (int i = 0; i < NP; ++i)
@@ -288,14 +284,9 @@ FM_DEVICE void fm_absorb_finish(const fm_f32x16* col, const fm_f32x16* sh, float
         else if (lr == 4) p = den;
       }
       sat[i][x] = p;
-      sold[i][x] = 0.f;
+      sold[i][x] = FRESH ? 0.f : *(p ? p : den);
     }
-  if (!fresh) {
-#pragma unroll
-    for (int i = 0; i < NSH; ++i)
-#pragma unroll
-      for (int x = 0; x < EPW; ++x) sold[i][x] = *(sat[i][x] ? sat[i][x] : den);
-  } else {
+  if (FRESH) {
     // the padding behind the last row
     constexpr int R = int(fm_decode_rows(DH, QUAD)), RP = int(fm_decode_rows_padded(DH, QUAD));
     for (int r = R + FM_TID_X; r < RP; r += FM_ABS_THREADS) {
@@ -347,9 +338,9 @@ template <int DH> struct DecAbsCfg {
   }
 };
 
-template <typename TIO, int DH>
+template <typename TIO, int DH, bool FRESH>
 FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_ABS_THREADS, 2)
-k_decode_absorb_mma(TRef<const TIO> k, TRef<const TIO> v, int n_new, float inv_tau, float* FM_RESTRICT state, int fresh) {
+k_decode_absorb_mma(TRef<const TIO> k, TRef<const TIO> v, int n_new, float inv_tau, float* FM_RESTRICT state) {
   static_assert(DH == 64, "two 32-row tiles per feature axis");
   typedef fm_half E;
   typedef Mma<E> M;
@@ -464,7 +455,7 @@ k_decode_absorb_mma(TRef<const TIO> k, TRef<const TIO> v, int n_new, float inv_t
     par ^= 1;
   }
   // the staging buffers are spent: the loop ended on a barrier
-  fm_absorb_finish<DH, true>(col, sh, reinterpret_cast<float*>(smem), num, den, fresh != 0);
+  fm_absorb_finish<DH, true, FRESH>(col, sh, reinterpret_cast<float*>(smem), num, den);
 }
 
 // The same sums from fp32 products, for fp32 tensors, order 1 and heads of 32.  A matrix instruction takes two tokens; its operands
@@ -475,20 +466,20 @@ k_decode_absorb_mma(TRef<const TIO> k, TRef<const TIO> v, int n_new, float inv_t
 // finite (infinity times a feature of zero is not a number); a workgroup that finds one adds its tokens one after the other
 // after all.  (That code costs 3 of 237 us at 16 heads of 3001 tokens; looking at every product took 73.)  One below 2^-126 is off by
 // at most 2^-150, times k'_b.
-template <int DH> struct DecAbsF32Cfg {
+template <int DH, bool QUAD> struct DecAbsF32Cfg {
   static constexpr int TT = 64;                        // tokens per tile
   static constexpr int PQ = DH + 4;
   static constexpr int TILE = TT * PQ + TT * FM_ABS_XR;
   static constexpr size_t lds_bytes() {
-    const size_t st = size_t(FM_ABS_GROUPS) * 2 * TILE * 4, red = AbsSums<DH, true>::red_bytes();
+    const size_t st = size_t(FM_ABS_GROUPS) * 2 * TILE * 4, red = AbsSums<DH, QUAD>::red_bytes();
     return st > red ? st : red;
   }
 };
-template <typename TIO, int DH, bool QUAD>
+template <typename TIO, int DH, bool QUAD, bool FRESH>
 FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_ABS_THREADS, 2)
-k_decode_absorb_f32(TRef<const TIO> k, TRef<const TIO> v, int n_new, float inv_tau, float* FM_RESTRICT state, int fresh) {
+k_decode_absorb_f32(TRef<const TIO> k, TRef<const TIO> v, int n_new, float inv_tau, float* FM_RESTRICT state) {
   typedef Mma<float> M;
-  typedef DecAbsF32Cfg<DH> C;
+  typedef DecAbsF32Cfg<DH, QUAD> C;
   typedef AbsSums<DH, QUAD> S;
   constexpr int TT = C::TT, PQ = C::PQ, XR = FM_ABS_XR, NT = DH / 32, NG = FM_ABS_GROUPS;
   FM_DYN_SMEM(smem);
@@ -602,23 +593,34 @@ k_decode_absorb_f32(TRef<const TIO> k, TRef<const TIO> v, int n_new, float inv_t
       float (*vs)[4] = reinterpret_cast<float (*)[4]>(smem + sizeof(float[W::TB][DH + 1]));
       constexpr int R = int(fm_decode_rows(DH, true));
       W w;
-      w.load(num, den, R, true, fresh != 0, FM_TID_X);
+      w.load(num, den, R, true, FRESH, FM_TID_X);
       w.add(k, v, bh, c4, n_new, inv_tau, ks, vs, FM_TID_X);
-      w.store(num, den, R, Rp, fresh != 0, FM_TID_X);
+      w.store(num, den, R, Rp, FRESH, FM_TID_X);
       return;
     }
   }
-  fm_absorb_finish<DH, QUAD>(col, sh, reinterpret_cast<float*>(smem), num, den, fresh != 0);
+  fm_absorb_finish<DH, QUAD, FRESH>(col, sh, reinterpret_cast<float*>(smem), num, den);
 }
 
-// prompts from this many tokens on are summed with matrix instructions (below it the one launch of k_decode is as quick)
+// Prompts from this many tokens on are summed with matrix instructions.  Into a state that is there, order 2, microseconds with k_decode
+// and with k_decode_absorb_f32: D = 64, 8 heads 64 tokens 27.1 and 15.6, 80 32.7 and 19.8; 64 heads 64 tokens 61.8 and 61.4, 80 73.8
+// and 78.1, 96 86 and 78; D = 32, 128 heads 64 tokens 19.9 and 21.0, 80 23.3 and 28.5, 128 35.2 and 28.6.  A second tile hardly
+// begun on a full chip is the one place k_decode wins; no rule for it, since at 33 heads it loses there too (65.6 and 57.2).
 static constexpr int FM_DEC_MMA_MIN = 64;
-template <typename TIO, int DH, bool QUAD>
-int fm_absorb_launch_f32(const FastmaxDesc* d, const TRef<const TIO>& kr, const TRef<const TIO>& vr, int n_new, float* state, int fresh, fm_stream_t stream) {
-  const size_t lds = DecAbsF32Cfg<DH>::lds_bytes();
-  fm_allow_lds(reinterpret_cast<const void*>(&k_decode_absorb_f32<TIO, DH, QUAD>), lds);
-  FM_KERNEL_LAUNCH((k_decode_absorb_f32<TIO, DH, QUAD>), fm_dim3(DH / 4, d->bh), fm_dim3(FM_ABS_THREADS), lds, stream, kr, vr, n_new,
-                   d->inv_tau, state, fresh);
+// FRESH: a new state.  (With a branch on it at run time, and the addresses of a state's entries made ahead of all their loads, 64 bf16
+// tokens at 64 heads took 47.6 us, so 44.2.)
+template <typename TIO, int DH, bool QUAD, bool FRESH>
+int fm_absorb_launch(const FastmaxDesc* d, const TRef<const TIO>& kr, const TRef<const TIO>& vr, int n_new, float* state, fm_stream_t stream) {
+  const fm_dim3 grid(DH / 4, d->bh);
+  if constexpr (sizeof(TIO) == 2 && DH == 64 && QUAD) {
+    const size_t lds = DecAbsCfg<DH>::lds_bytes();
+    fm_allow_lds(reinterpret_cast<const void*>(&k_decode_absorb_mma<TIO, DH, FRESH>), lds);
+    FM_KERNEL_LAUNCH((k_decode_absorb_mma<TIO, DH, FRESH>), grid, fm_dim3(FM_ABS_THREADS), lds, stream, kr, vr, n_new, d->inv_tau, state);
+  } else {
+    const size_t lds = DecAbsF32Cfg<DH, QUAD>::lds_bytes();
+    fm_allow_lds(reinterpret_cast<const void*>(&k_decode_absorb_f32<TIO, DH, QUAD, FRESH>), lds);
+    FM_KERNEL_LAUNCH((k_decode_absorb_f32<TIO, DH, QUAD, FRESH>), grid, fm_dim3(FM_ABS_THREADS), lds, stream, kr, vr, n_new, d->inv_tau, state);
+  }
   return fm_after_launch() ? FASTMAX_ERR_LAUNCH : FASTMAX_OK;
 }
 
@@ -629,26 +631,17 @@ int fm_decode_run(const FastmaxDesc* d, const void* q, const void* k, const void
   const TRef<const TIO> kr = fm_ref<const TIO>(static_cast<const TIO*>(k), d->sk), vr = fm_ref<const TIO>(static_cast<const TIO*>(v), d->sv);
   const TRef<const TIO> qr = q ? fm_ref<const TIO>(static_cast<const TIO*>(q), d->sq) : kr;
   (void)scratch;
-  const int fresh = !q && (d->flags & FASTMAX_FLAG_NEW_STATE) ? 1 : 0;
+  const bool fresh = !q && (d->flags & FASTMAX_FLAG_NEW_STATE);
   if (!q && n_new >= FM_DEC_MMA_MIN) {
-    if constexpr (sizeof(TIO) == 2 && DH == 64) {
-      if (quad) {
-        const size_t lds = DecAbsCfg<DH>::lds_bytes();
-        fm_allow_lds(reinterpret_cast<const void*>(&k_decode_absorb_mma<TIO, DH>), lds);
-        FM_KERNEL_LAUNCH((k_decode_absorb_mma<TIO, DH>), fm_dim3(DH / 4, d->bh), fm_dim3(FM_ABS_THREADS), lds, stream, kr, vr, n_new,
-                         d->inv_tau, state, fresh);
-        return fm_after_launch() ? FASTMAX_ERR_LAUNCH : FASTMAX_OK;
-      }
-    }
-    if constexpr (sizeof(TIO) == 4 || DH != 64) {
-      if (quad) return fm_absorb_launch_f32<TIO, DH, true>(d, kr, vr, n_new, state, fresh, stream);
-    }
-    return fm_absorb_launch_f32<TIO, DH, false>(d, kr, vr, n_new, state, fresh, stream);
+    if (quad) return fresh ? fm_absorb_launch<TIO, DH, true, true>(d, kr, vr, n_new, state, stream)
+                           : fm_absorb_launch<TIO, DH, true, false>(d, kr, vr, n_new, state, stream);
+    return fresh ? fm_absorb_launch<TIO, DH, false, true>(d, kr, vr, n_new, state, stream)
+                 : fm_absorb_launch<TIO, DH, false, false>(d, kr, vr, n_new, state, stream);
   }
   const TRef<TIO> orf = q ? fm_ref<TIO>(static_cast<TIO*>(o), d->so) : TRef<TIO>{};
   const TRef<float> grf = q ? fm_ref<float>(g, d->sg) : TRef<float>{};
   FM_KERNEL_LAUNCH((k_decode<TIO, DH>), fm_dim3(DH / 4, d->bh), fm_dim3(FM_DEC_THREADS), 0, stream, kr, vr, qr, n_new, quad ? 1 : 0,
-                   d->inv_tau, d->a0, d->a1, quad ? d->a2 : 0.0f, state, orf, grf, q ? 1 : 0, fresh);
+                   d->inv_tau, d->a0, d->a1, quad ? d->a2 : 0.0f, state, orf, grf, q ? 1 : 0, fresh ? 1 : 0);
   return fm_after_launch() ? FASTMAX_ERR_LAUNCH : FASTMAX_OK;
 }
 
