@@ -68,15 +68,21 @@ template <typename TIO> struct NormJob {
   float *sums, *mean;                  // within it: the column sums and means of x (and of dy, behind them) of batch*head 0
   int n;
 };
+// JOBS: one or two.  (One tensor's launches take one job: with two in every launch's arguments the four kernels of a centred pass over
+// 32 heads of 1024 tokens, D = 32, fp32, took 16.5 us for 15.8.)
+template <typename TIO, int JOBS> struct NormJobs {
+  NormJob<TIO> j[JOBS];
+  FM_DEVICE const NormJob<TIO>& pick(bool second) const { return JOBS > 1 && second ? j[JOBS - 1] : j[0]; }
+};
 
 // Column sums over the workgroup's 64 * FM_NORM_NP tokens -> sums[bh][tensor][block][DH]; k_norm_colfinal adds the
-// blocks in a fixed order and divides.  grid (blocks, bh, jobs * TENSORS) and (bh, jobs * TENSORS); TENSORS: x alone, or x and dy.
-template <typename TIO, int DH, int TENSORS>
-FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_norm_colsum(NormJob<TIO> j0, NormJob<TIO> j1) {
+// blocks in a fixed order and divides.  grid (blocks, bh, JOBS * TENSORS) and (bh, JOBS * TENSORS); TENSORS: x alone, or x and dy.
+template <typename TIO, int DH, int TENSORS, int JOBS>
+FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_norm_colsum(NormJobs<TIO, JOBS> jobs) {
   constexpr int EPT = DH / 4, NP = FM_NORM_NP;
   FM_SHARED float part[64 * (DH + 1)];
   const int tid = FM_TID_X, bh = FM_BID_Y, which = int(FM_BID_Z) % TENSORS;
-  const NormJob<TIO> J = int(FM_BID_Z) >= TENSORS ? j1 : j0;
+  const NormJob<TIO> J = jobs.pick(int(FM_BID_Z) >= TENSORS);
   const int n = J.n, nblk = fm_norm_blocks(n);
   if (int(FM_BID_X) >= nblk) return;                // the shorter tensor of the two (workgroup-uniform; here and below)
   const TRef<const TIO> x = which ? J.dy : J.x;
@@ -103,12 +109,12 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_norm_colsum(NormJob<TIO> j0, NormJob<TIO>
     out[int64_t(FM_BID_X) * DH + tid] = a;
   }
 }
-template <typename TIO, int DH, int TENSORS>
-FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_norm_colfinal(NormJob<TIO> j0, NormJob<TIO> j1) {
+template <typename TIO, int DH, int TENSORS, int JOBS>
+FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_norm_colfinal(NormJobs<TIO, JOBS> jobs) {
   constexpr int G = 256 / DH;                 // groups of DH threads, each takes every G-th block
   FM_SHARED float part[256];
   const int tid = FM_TID_X, bh = FM_BID_X, which = int(FM_BID_Y) % TENSORS;
-  const NormJob<TIO> J = int(FM_BID_Y) >= TENSORS ? j1 : j0;
+  const NormJob<TIO> J = jobs.pick(int(FM_BID_Y) >= TENSORS);
   const int n = J.n, nblk = fm_norm_blocks(n);
   const int g = tid / DH, f = tid % DH;
   const float* FM_RESTRICT sums = J.sums + bh * J.stride + int64_t(which) * nblk * DH;
@@ -130,13 +136,13 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_norm_colfinal(NormJob<TIO> j0, NormJob<TI
   }
 }
 
-// grid (ceil(n / (64 * FM_NORM_NP)), bh, jobs); four threads per token
-template <typename TIO, int DH>
-FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_norm_maxnorm(NormJob<TIO> j0, NormJob<TIO> j1, int centre) {
+// grid (ceil(n / (64 * FM_NORM_NP)), bh, JOBS); four threads per token
+template <typename TIO, int DH, int JOBS>
+FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_norm_maxnorm(NormJobs<TIO, JOBS> jobs, int centre) {
   constexpr int EPT = DH / 4, NP = FM_NORM_NP;
   FM_SHARED float wmax[4];
   const int tid = FM_TID_X, bh = FM_BID_Y;
-  const NormJob<TIO> J = FM_BID_Z ? j1 : j0;
+  const NormJob<TIO> J = jobs.pick(FM_BID_Z != 0);
   const TRef<const TIO> x = J.x;
   const int n = J.n;
   if (int(FM_BID_X) >= fm_norm_blocks(n)) return;
@@ -167,11 +173,11 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_norm_maxnorm(NormJob<TIO> j0, NormJob<TIO
   if (tid == 0) st[2 + DH + FM_BID_X] = fm_fmaxf(fm_fmaxf(wmax[0], wmax[1]), fm_fmaxf(wmax[2], wmax[3]));
 }
 
-template <typename TIO, int DH>
-FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_norm_apply(NormJob<TIO> j0, NormJob<TIO> j1, int centre, int max_norm, float scale) {
+template <typename TIO, int DH, int JOBS>
+FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_norm_apply(NormJobs<TIO, JOBS> jobs, int centre, int max_norm, float scale) {
   constexpr int EPT = DH / 4, NP = FM_NORM_NP;
   const int tid = FM_TID_X, bh = FM_BID_Y;
-  const NormJob<TIO> J = FM_BID_Z ? j1 : j0;
+  const NormJob<TIO> J = jobs.pick(FM_BID_Z != 0);
   const TRef<const TIO> x = J.x;
   const int n = J.n, nblk = fm_norm_blocks(n);
   if (int(FM_BID_X) >= nblk) return;
@@ -205,6 +211,18 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_norm_apply(NormJob<TIO> j0, NormJob<TIO> 
   }
 }
 
+template <typename TIO, int DH, int JOBS>
+int fm_normalize_launch(const FastmaxNormDesc* d, const NormJobs<TIO, JOBS>& jobs, fm_stream_t stream) {
+  const int n0 = jobs.j[0].n, n1 = jobs.j[JOBS - 1].n;
+  const fm_dim3 grid(fm_norm_blocks(n0 > n1 ? n0 : n1), d->bh, JOBS);
+  if (d->centre == 2) {
+    FM_KERNEL_LAUNCH((k_norm_colsum<TIO, DH, 1, JOBS>), grid, fm_dim3(256), 0, stream, jobs);
+    FM_KERNEL_LAUNCH((k_norm_colfinal<TIO, DH, 1, JOBS>), fm_dim3(d->bh, JOBS), fm_dim3(256), 0, stream, jobs);
+  }
+  if (d->max_norm) FM_KERNEL_LAUNCH((k_norm_maxnorm<TIO, DH, JOBS>), grid, fm_dim3(256), 0, stream, jobs, d->centre);
+  FM_KERNEL_LAUNCH((k_norm_apply<TIO, DH, JOBS>), grid, fm_dim3(256), 0, stream, jobs, d->centre, d->max_norm, d->scale);
+  return fm_after_launch() ? FASTMAX_ERR_LAUNCH : FASTMAX_OK;
+}
 // One tensor (d1 null) or two in the same launches.  q and k of 15 heads of 777 tokens, heads of 64, fp32: 20 us instead of 37 in twice
 // the launches; their backward (fm_normalize_bwd_run) 24 instead of 43.
 template <typename TIO, int DH>
@@ -218,16 +236,8 @@ int fm_normalize_run(const FastmaxNormDesc* d0, const void* x0, void* y0, float*
     if (stats) { j.mean = stats + 2; j.sums = stats + 2 + DH + fm_norm_blocks(d->n); }
     return j;
   };
-  const NormJob<TIO> j0 = job(d0, x0, y0, stats0), j1 = d1 ? job(d1, x1, y1, stats1) : j0;
-  const int jobs = d1 ? 2 : 1, nb = fm_norm_blocks(j0.n > j1.n ? j0.n : j1.n);
-  const fm_dim3 grid(nb, d0->bh, jobs);
-  if (d0->centre == 2) {
-    FM_KERNEL_LAUNCH((k_norm_colsum<TIO, DH, 1>), grid, fm_dim3(256), 0, stream, j0, j1);
-    FM_KERNEL_LAUNCH((k_norm_colfinal<TIO, DH, 1>), fm_dim3(d0->bh, jobs), fm_dim3(256), 0, stream, j0, j1);
-  }
-  if (d0->max_norm) FM_KERNEL_LAUNCH((k_norm_maxnorm<TIO, DH>), grid, fm_dim3(256), 0, stream, j0, j1, d0->centre);
-  FM_KERNEL_LAUNCH((k_norm_apply<TIO, DH>), grid, fm_dim3(256), 0, stream, j0, j1, d0->centre, d0->max_norm, d0->scale);
-  return fm_after_launch() ? FASTMAX_ERR_LAUNCH : FASTMAX_OK;
+  if (d1) return fm_normalize_launch<TIO, DH, 2>(d0, NormJobs<TIO, 2>{{job(d0, x0, y0, stats0), job(d1, x1, y1, stats1)}}, stream);
+  return fm_normalize_launch<TIO, DH, 1>(d0, NormJobs<TIO, 1>{{job(d0, x0, y0, stats0)}}, stream);
 }
 
 // a second tensor takes part in the first one's launches: same batch*heads, head size, type and kind of pass
@@ -283,14 +293,14 @@ inline int64_t fm_normb_stride(int dh, int n, int centre) {
   return fm_normb_base(dh, n) + (centre == 2 ? 2 * int64_t(fm_norm_blocks(n)) * dh : 0);
 }
 
-// grid (ceil(n / (64 * FM_NORMB_NP)), bh, jobs); four threads per token
-template <typename TIO, int DH>
-FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_normb_stats(NormJob<TIO> j0, NormJob<TIO> j1, int centre) {
+// grid (ceil(n / (64 * FM_NORMB_NP)), bh, JOBS); four threads per token
+template <typename TIO, int DH, int JOBS>
+FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_normb_stats(NormJobs<TIO, JOBS> jobs, int centre) {
   constexpr int EPT = DH / 4, NP = FM_NORMB_NP;
   FM_SHARED float wsum[NP][4];
   FM_SHARED unsigned long long wkey[4];
   const int tid = FM_TID_X, bh = FM_BID_Y;
-  const NormJob<TIO> J = FM_BID_Z ? j1 : j0;
+  const NormJob<TIO> J = jobs.pick(FM_BID_Z != 0);
   const TRef<const TIO> x = J.x, dy = J.dy;
   const int n = J.n;
   if (int(FM_BID_X) >= fm_normb_blocks(n)) return;
@@ -345,14 +355,14 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_normb_stats(NormJob<TIO> j0, NormJob<TIO>
   }
 }
 
-// grid (ceil(n / (64 * FM_NORM_NP)), bh, jobs); four threads per token
-template <typename TIO, int DH>
-FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_normb_apply(NormJob<TIO> j0, NormJob<TIO> j1, int centre, int max_norm, float scale) {
+// grid (ceil(n / (64 * FM_NORM_NP)), bh, JOBS); four threads per token
+template <typename TIO, int DH, int JOBS>
+FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_normb_apply(NormJobs<TIO, JOBS> jobs, int centre, int max_norm, float scale) {
   constexpr int EPT = DH / 4, NP = FM_NORM_NP;
   FM_SHARED float red[256];
   FM_SHARED unsigned long long redk[256];
   const int tid = FM_TID_X, bh = FM_BID_Y;
-  const NormJob<TIO> J = FM_BID_Z ? j1 : j0;
+  const NormJob<TIO> J = jobs.pick(FM_BID_Z != 0);
   const TRef<const TIO> x = J.x, dy = J.dy;
   const int n = J.n;
   if (int(FM_BID_X) >= fm_norm_blocks(n)) return;
@@ -416,6 +426,20 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_normb_apply(NormJob<TIO> j0, NormJob<TIO>
   }
 }
 
+template <typename TIO, int DH, int JOBS>
+int fm_normalize_bwd_launch(const FastmaxNormDesc* d, const NormJobs<TIO, JOBS>& jobs, fm_stream_t stream) {
+  const int n0 = jobs.j[0].n, n1 = jobs.j[JOBS - 1].n, nmax = n0 > n1 ? n0 : n1;
+  const fm_dim3 grid(fm_norm_blocks(nmax), d->bh, JOBS);
+  if (d->centre == 2) {
+    FM_KERNEL_LAUNCH((k_norm_colsum<TIO, DH, 2, JOBS>), fm_dim3(grid.x, grid.y, 2 * JOBS), fm_dim3(256), 0, stream, jobs);
+    FM_KERNEL_LAUNCH((k_norm_colfinal<TIO, DH, 2, JOBS>), fm_dim3(d->bh, 2 * JOBS), fm_dim3(256), 0, stream, jobs);
+  }
+  if (d->max_norm)
+    FM_KERNEL_LAUNCH((k_normb_stats<TIO, DH, JOBS>), fm_dim3(fm_normb_blocks(nmax), d->bh, JOBS), fm_dim3(256), 0, stream, jobs, d->centre);
+  FM_KERNEL_LAUNCH((k_normb_apply<TIO, DH, JOBS>), grid, fm_dim3(256), 0, stream, jobs, d->centre, d->max_norm, d->scale);
+  return fm_after_launch() ? FASTMAX_ERR_LAUNCH : FASTMAX_OK;
+}
+
 template <typename TIO, int DH>
 int fm_normalize_bwd_run(const FastmaxNormDesc* d0, const void* x0, const void* dy0, void* dx0, float* stats0,
                          const FastmaxNormDesc* d1, const void* x1, const void* dy1, void* dx1, float* stats1, fm_stream_t stream) {
@@ -429,17 +453,8 @@ int fm_normalize_bwd_run(const FastmaxNormDesc* d0, const void* x0, const void* 
     if (stats) { j.mean = stats + 4; j.sums = stats + fm_normb_base(DH, d->n); }
     return j;
   };
-  const NormJob<TIO> j0 = job(d0, x0, dy0, dx0, stats0), j1 = d1 ? job(d1, x1, dy1, dx1, stats1) : j0;
-  const int jobs = d1 ? 2 : 1, nmax = j0.n > j1.n ? j0.n : j1.n;
-  const fm_dim3 grid(fm_norm_blocks(nmax), d0->bh, jobs);
-  if (d0->centre == 2) {
-    FM_KERNEL_LAUNCH((k_norm_colsum<TIO, DH, 2>), fm_dim3(grid.x, grid.y, 2 * jobs), fm_dim3(256), 0, stream, j0, j1);
-    FM_KERNEL_LAUNCH((k_norm_colfinal<TIO, DH, 2>), fm_dim3(d0->bh, 2 * jobs), fm_dim3(256), 0, stream, j0, j1);
-  }
-  if (d0->max_norm)
-    FM_KERNEL_LAUNCH((k_normb_stats<TIO, DH>), fm_dim3(fm_normb_blocks(nmax), d0->bh, jobs), fm_dim3(256), 0, stream, j0, j1, d0->centre);
-  FM_KERNEL_LAUNCH((k_normb_apply<TIO, DH>), grid, fm_dim3(256), 0, stream, j0, j1, d0->centre, d0->max_norm, d0->scale);
-  return fm_after_launch() ? FASTMAX_ERR_LAUNCH : FASTMAX_OK;
+  if (d1) return fm_normalize_bwd_launch<TIO, DH, 2>(d0, NormJobs<TIO, 2>{{job(d0, x0, dy0, dx0, stats0), job(d1, x1, dy1, dx1, stats1)}}, stream);
+  return fm_normalize_bwd_launch<TIO, DH, 1>(d0, NormJobs<TIO, 1>{{job(d0, x0, dy0, dx0, stats0)}}, stream);
 }
 
 inline int fm_normalize_bwd_dispatch(const FastmaxNormDesc* d0, const void* x0, const void* dy0, void* dx0, float* stats0,
