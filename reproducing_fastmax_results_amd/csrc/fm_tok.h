@@ -177,15 +177,17 @@ FM_DEVICE void fm_store_tokens(fm_f32x16 (*acc)[DH / 32], const int* xrow, const
 // Placement of the blocks of own tokens.  A causal block's work is its dense part (1 .. L/QW
 // units of QW x QW tiles, growing with the position inside its segment for queries, shrinking
 // for keys) plus the state readout (the same for every block that has a state), so blocks
-// differ by up to an order of magnitude, and at B*H = 32, N = 4096 a launch has exactly as
-// many workgroups as the chip has slots (two per CU): there is no second wave of workgroups
-// to even things out.  Workgroups go round-robin to the 8 XCDs and, inside an XCD, to its
-// 32 CUs in launch order, so the XCD-local launch index j is turned into a weight rank
-// boustrophedon-wise over rounds of 32: the CU that got the heaviest block of one round gets
-// the lightest of the next.  All blocks of one batch*head stay on one XCD (one L2).
-FM_DEVICE int fm_snake_rank(int j, int total) {
+// differ by up to an order of magnitude, and a launch has a few workgroups per place on the chip.
+// Workgroups go round-robin to the 8 XCDs and, inside an XCD, to its 32 CUs in launch order
+// as long as there are free places (slots per CU); those behind them go where a place falls free.  So the
+// XCD-local launch index j is turned into a weight rank boustrophedon-wise over the rounds of 32 that start
+// together (the CU that got the heaviest block of one round gets the lightest of the next), and in order of weight
+// behind them: the first place that falls free gets the heaviest block left.  (With every round turned, the
+// lightest blocks of the last rounds were dealt first: dK + dV of fp32 at 4 x 8 heads of 4096 tokens, two rounds of one
+// workgroup per CU, 423 us, now 365; the bf16 backward 257, now 251.)  All blocks of one batch*head stay on one XCD (one L2).
+FM_DEVICE int fm_snake_rank(int j, int total, int slots) {
   const int r = j >> 5, pos = j & 31, base = r << 5;
-  if ((r & 1) == 0) return j;
+  if ((r & 1) == 0 || r >= slots) return j;
   const int cnt = total - base < 32 ? total - base : 32;
   return base + cnt - 1 - pos;
 }
@@ -222,17 +224,21 @@ template <int OWN, int QW, typename A_>
 struct TokGeom {
   int unit, bh, t0, seg, slot, sbeg, send;
   bool use_state;
-  FM_DEVICE void init(const A_& A) {
+  // slots: workgroups of a CU (see fm_snake_rank)
+  FM_DEVICE void init(const A_& A, int slots) {
     const int nblk = FM_GDIM_X, nbh = FM_GDIM_Y;
     const int id = FM_BID_X + nblk * FM_BID_Y;
     if ((nbh & 7) == 0) {
       const int nb = nbh >> 3;                       // batch*heads per XCD
-      const int rank = fm_snake_rank(id >> 3, nblk * nb);
+      const int rank = fm_snake_rank(id >> 3, nblk * nb, slots);
       unit = rank / nb;
       bh = (id & 7) + 8 * (rank % nb);
     } else {
-      unit = id % nblk;
-      bh = id / nblk;
+      // One segment: in order of weight over all batch*heads.  (Batch*head after batch*head, each one's heaviest block first, the
+      // last heavy blocks started late: bf16, 36 heads of 2000 tokens, forward 57 us, backward 153, now 45 and 98.)
+      const bool by_weight = A.causal && nblk * QW <= A.L;
+      unit = by_weight ? id / nbh : id % nblk;
+      bh = by_weight ? id % nbh : id / nblk;
     }
     // Many segments (a long sequence): the blocks of one segment read the same state, 557 KB at order 2, so
     // they are launched next to each other and run at the same time: the state comes from HBM once and from
@@ -315,7 +321,7 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_THREADS * GRP, (TokCfg<E, DH, QT>::OCC_PV)) 
   const int tid = int(FM_TID_X) % FM_THREADS, lane = tid & 63, lr = lane & 31, lh = lane >> 5;
   const int wave = FM_UNIFORM(tid >> 6);
   TokGeom<OWN, QW, TokArgs<TIO, E> > G;
-  G.init(A);
+  G.init(A, C::OCC_PV / GRP);
   const int bh = G.bh, t0 = G.t0;
   const bool causal = A.causal != 0;
 
@@ -634,7 +640,7 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_THREADS * GRP, (DV ? TokCfg<E, DH, QT>::OCC_
   const int tid = int(FM_TID_X) % FM_THREADS, lane = tid & 63, lr = lane & 31, lh = lane >> 5;
   const int wave = FM_UNIFORM(tid >> 6);
   TokGeom<OWN, QW, TokArgs<TIO, E> > G;
-  G.init(A);
+  G.init(A, DV ? (C::OCC_DV + GRP - 1) / GRP : (C::OCC_DS + GRP - 1) / GRP);
   const int bh = G.bh, t0 = G.t0;
   const bool causal = A.causal != 0;
   const float gsc = fm_grad_scale(A.gpart ? A.gpart + int64_t(bh) * A.gnblk : nullptr, A.gnblk, lane);

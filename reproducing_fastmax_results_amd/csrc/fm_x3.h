@@ -324,11 +324,11 @@ template <typename TIO, int DH, typename R, int ROWS, int NTH> struct X3Stage {
 
 // Block of own tokens and batch*head of a workgroup: heaviest blocks first (late queries, early keys under the causal
 // mask); with a multiple of eight batch*heads all blocks of one run behind one L2, dealt as in TokGeom.
-FM_DEVICE void fm_x3_place(bool late_first, int& blk, int& bh) {
+FM_DEVICE void fm_x3_place(bool late_first, int slots, int& blk, int& bh) {
   const int nblk = FM_GDIM_X, nbh = FM_GDIM_Y, id = FM_BID_X + nblk * FM_BID_Y;
   int unit;
   if ((nbh & 7) == 0) {
-    const int nb = nbh >> 3, rank = fm_snake_rank(id >> 3, nblk * nb);
+    const int nb = nbh >> 3, rank = fm_snake_rank(id >> 3, nblk * nb, slots);
     unit = rank / nb;
     bh = (id & 7) + 8 * (rank % nb);
   } else {
@@ -420,6 +420,7 @@ template <int DH, int NW, int SPLIT> struct X3Cfg {
     const size_t a = size_t(NBUF) * STAGE * 2 + (kind ? size_t(QW) * PQ * 2 + size_t(NBUF) * KT * 4 : 0);
     return a > OS ? a : OS;
   }
+  static constexpr int SLOTS = NW == 8 ? 1 : 2;        // workgroups of a CU, see fm_snake_rank
   static constexpr int OCC = NW == 8 || NBUF == 1 || 2 * (NBUF * STAGE * 2) > 150 * 1024 ? NW / 4 : DH == 32 && SPLIT == 1 ? 3 : 2;   // wavefronts per SIMD
 };
 
@@ -434,7 +435,7 @@ FM_DEVICE void fm_x3_fwd(const X3Args<TIO>& A, uint16_t* st, int* bad, const int
   const int wave = FM_UNIFORM(tid >> 6), own = wave / SPLIT, sub = wave % SPLIT;
   const bool causal = A.causal != 0;
   int blk, bh;
-  fm_x3_place(causal, blk, bh);
+  fm_x3_place(causal, C::SLOTS, blk, bh);
   const int t0 = blk * QW, lo = t0 + 32 * own;
   const float qs = A.sc * fm_norm_factor(A.q_fold, bh, lane) * R::UP, ks_ = A.sc * fm_norm_factor(A.k_fold, bh, lane) * R::UP;
   const X3Coef cf = fm_x3_coef<R>(A.a0, A.a1, A.a2);
@@ -550,7 +551,7 @@ FM_DEVICE void fm_x3_dq(const X3Args<TIO>& A, uint16_t* st, int* bad, const int 
   const int wave = FM_UNIFORM(tid >> 6), own = wave / SPLIT, sub = wave % SPLIT;
   const bool causal = A.causal != 0;
   int blk, bh;
-  fm_x3_place(causal, blk, bh);
+  fm_x3_place(causal, C::SLOTS, blk, bh);
   const int t0 = blk * QW, lo = t0 + 32 * own;
   const float qf = fm_norm_factor(A.q_fold, bh, lane), qs = A.sc * qf * R::UP, ks_ = A.sc * fm_norm_factor(A.k_fold, bh, lane) * R::UP;
   const int send = causal && t0 + QW < A.nk ? t0 + QW : A.nk;
@@ -645,7 +646,7 @@ FM_DEVICE void fm_x3_dkv(const X3Args<TIO>& A, uint16_t* Vs, int* bad, const int
   const int wave = FM_UNIFORM(tid >> 6), own = wave / SPLIT, sub = wave % SPLIT;
   const bool causal = A.causal != 0;
   int blk, bh;
-  fm_x3_place(false, blk, bh);
+  fm_x3_place(false, C::SLOTS, blk, bh);
   const int t0 = blk * QW, lo = t0 + 32 * own;
   const float kf = fm_norm_factor(A.k_fold, bh, lane), ks_ = A.sc * kf * R::UP, qs = A.sc * fm_norm_factor(A.q_fold, bh, lane) * R::UP;
   const int sbeg = causal ? t0 : 0, nst = (A.nq - sbeg + KT - 1) / KT;
