@@ -126,6 +126,12 @@ inline bool half_arithmetic(const FastmaxDesc* d) {
 // Unmasked attention: one total of the moments costs less than products with every key.
 inline bool states_pay_unmasked(const FastmaxDesc* d) { return int64_t(d->nk) > int64_t(d->d) * d->d + d->d; }
 
+// How many wavefronts share an own tile in the fp32 kernels of dense tiles (fm_x3.h): with one each, a launch has blocks of 128
+// own tokens (256 for dK + dV); below two workgroups per CU the own tiles are spread over twice or four times as many.
+inline int x3_split(int bh, int n_own, int tokens) {
+  const int blocks = bh * ((n_own + tokens - 1) / tokens);
+  return blocks >= 512 ? 1 : blocks >= 256 ? 2 : 4;
+}
 int validate(const FastmaxDesc* d) {
   if (!d) return FASTMAX_ERR_NULL;
   if (d->dtype != FASTMAX_F32 && d->dtype != FASTMAX_BF16) return FASTMAX_ERR_DTYPE;
@@ -533,12 +539,6 @@ int run_forward_o1(const FastmaxDesc* d, const Plan& p, const void* q, const voi
 }
 
 // ---- fp32 arithmetic on dense tiles (fm_x3.h) ------------------------------------------------
-// How many wavefronts share an own tile: with one each, a launch has blocks of 128 own tokens (256 for dK + dV); below
-// two workgroups per CU the own tiles are spread over twice or four times as many.
-inline int x3_split(int bh, int n_own, int tokens) {
-  const int blocks = bh * ((n_own + tokens - 1) / tokens);
-  return blocks >= 512 ? 1 : blocks >= 256 ? 2 : 4;
-}
 template <typename TIO> X3Args<TIO> x3_args(const FastmaxDesc* d, const Plan& p, const void* q, const void* k, const void* v) {
   X3Args<TIO> a;
   a.q = cref<TIO>(q, d->sq); a.k = cref<TIO>(k, d->sk); a.v = cref<TIO>(v, d->sv);
@@ -551,19 +551,23 @@ template <typename TIO> X3Args<TIO> x3_args(const FastmaxDesc* d, const Plan& p,
   a.q_fold = q_fold(d); a.k_fold = k_fold(d);
   return a;
 }
-// KIND 0: forward, 1: dQ, 2: dK + dV
-template <typename TIO, int DH, int KIND, int SPLIT>
+// Wavefronts of a workgroup (kind 0: forward, 1: dQ, 2: dK + dV).  Two buffers of a stage for own tiles shared by two wavefronts take 102 KB
+// at D = 64, one workgroup per CU: eight wavefronts rather than four then keep each SIMD two.  (Causal
+// forward in four and in eight: 12 heads of 4096 tokens 237, 168 us, 40 of 1024 64, 46, 64 of 512 36, 27, 100 of 300 25.6, 28.7.)
+inline int x3_waves(int kind, int dh, int split, int n_str) { return kind == 2 || (split == 2 && dh == 64 && n_str >= 512) ? 8 : 4; }
+inline int x3_rows(int kind, int dh, int split, int n_str) { return 32 * x3_waves(kind, dh, split, n_str) / split; }   // own tokens of a workgroup
+template <typename TIO, int DH, int KIND, int SPLIT, int NW>
 int launch_x3_cfg(const X3Args<TIO>& a, int n_own, int bh, fm_stream_t stream) {
-  typedef X3Cfg<DH, KIND == 2 ? 8 : 4, SPLIT> C;
+  typedef X3Cfg<DH, NW, SPLIT> C;
   const size_t lds = C::lds(KIND == 2);
   ProfScope prof(KIND == 0 ? FM_K_FWD : KIND == 1 ? FM_K_DQ : FM_K_DKV, stream);
   const fm_dim3 grid((n_own + C::QW - 1) / C::QW, bh), block(C::NTH);
   if constexpr (KIND == 0) {
-    fm_allow_lds(reinterpret_cast<const void*>(&k_x3_fwd<TIO, DH, SPLIT>), lds);
-    FM_KERNEL_LAUNCH((k_x3_fwd<TIO, DH, SPLIT>), grid, block, lds, stream, a);
+    fm_allow_lds(reinterpret_cast<const void*>(&k_x3_fwd<TIO, DH, SPLIT, NW>), lds);
+    FM_KERNEL_LAUNCH((k_x3_fwd<TIO, DH, SPLIT, NW>), grid, block, lds, stream, a);
   } else if constexpr (KIND == 1) {
-    fm_allow_lds(reinterpret_cast<const void*>(&k_x3_dq<TIO, DH, SPLIT>), lds);
-    FM_KERNEL_LAUNCH((k_x3_dq<TIO, DH, SPLIT>), grid, block, lds, stream, a);
+    fm_allow_lds(reinterpret_cast<const void*>(&k_x3_dq<TIO, DH, SPLIT, NW>), lds);
+    FM_KERNEL_LAUNCH((k_x3_dq<TIO, DH, SPLIT, NW>), grid, block, lds, stream, a);
   } else {
     fm_allow_lds(reinterpret_cast<const void*>(&k_x3_dkv<TIO, DH, SPLIT>), lds);
     FM_KERNEL_LAUNCH((k_x3_dkv<TIO, DH, SPLIT>), grid, block, lds, stream, a);
@@ -571,10 +575,14 @@ int launch_x3_cfg(const X3Args<TIO>& a, int n_own, int bh, fm_stream_t stream) {
   return fm_launch_status();
 }
 template <typename TIO, int DH, int KIND>
-int launch_x3(const X3Args<TIO>& a, int split, int n_own, int bh, fm_stream_t stream) {
-  if (split == 1) return launch_x3_cfg<TIO, DH, KIND, 1>(a, n_own, bh, stream);
-  if (split == 2) return launch_x3_cfg<TIO, DH, KIND, 2>(a, n_own, bh, stream);
-  return launch_x3_cfg<TIO, DH, KIND, 4>(a, n_own, bh, stream);
+int launch_x3(const X3Args<TIO>& a, int split, int n_own, int n_str, int bh, fm_stream_t stream) {
+  constexpr int NW = KIND == 2 ? 8 : 4;
+  if (split == 1) return launch_x3_cfg<TIO, DH, KIND, 1, NW>(a, n_own, bh, stream);
+  if (split == 4) return launch_x3_cfg<TIO, DH, KIND, 4, NW>(a, n_own, bh, stream);
+  if constexpr (KIND < 2 && DH == 64) {
+    if (x3_waves(KIND, DH, split, n_str) == 8) return launch_x3_cfg<TIO, DH, KIND, 2, 8>(a, n_own, bh, stream);
+  }
+  return launch_x3_cfg<TIO, DH, KIND, 2, NW>(a, n_own, bh, stream);
 }
 
 // ---- at most 64 tokens (fm_small.h) ----------------------------------------------------------
@@ -628,7 +636,7 @@ int run_forward(const FastmaxDesc* d, const Plan& p, const void* q, const void* 
       X3Args<TIO> a = x3_args<TIO>(d, p, q, k, v);
       a.out = mref<TIO>(o, d->so); a.g = mref<float>(g, d->sg);
       if (p.keep_resid) a.out_resid = reinterpret_cast<fm_half*>(ws + p.ores);
-      return launch_x3<TIO, DH, 0>(a, x3_split(d->bh, d->nq, 128), d->nq, d->bh, stream);
+      return launch_x3<TIO, DH, 0>(a, x3_split(d->bh, d->nq, 128), d->nq, d->nk, d->bh, stream);
     }
   }
   E* kt = reinterpret_cast<E*>(ws + p.kt);

@@ -425,11 +425,11 @@ template <int DH, int NW, int SPLIT> struct X3Cfg {
 };
 
 // ------------------------------------------------------------------------------
-// forward.  grid (ceil(nq / QW), bh), 256 threads.
+// forward.  grid (ceil(nq / QW), bh).
 // ------------------------------------------------------------------------------
-template <typename TIO, int DH, int SPLIT, typename R>
+template <typename TIO, int DH, int SPLIT, typename R, int NW>
 FM_DEVICE void fm_x3_fwd(const X3Args<TIO>& A, uint16_t* st, int* bad, const int tid) {
-  typedef X3Cfg<DH, 4, SPLIT> C;
+  typedef X3Cfg<DH, NW, SPLIT> C;
   constexpr int NT = DH / 32, PQ = C::PQ, KT = C::KT, QW = C::QW;
   const int lane = tid & 63, lr = lane & 31, lh = lane >> 5;
   const int wave = FM_UNIFORM(tid >> 6), own = wave / SPLIT, sub = wave % SPLIT;
@@ -527,25 +527,25 @@ FM_DEVICE void fm_x3_fwd(const X3Args<TIO>& A, uint16_t* st, int* bad, const int
     if (col == 0) A.g.base(bh)[int64_t(qi) * A.g.s_n] = gt;
   }
 }
-template <typename TIO, int DH, int SPLIT>
-FM_GLOBAL void FM_LAUNCH_BOUNDS2(256, (X3Cfg<DH, 4, SPLIT>::OCC)) k_x3_fwd(X3Args<TIO> A) {
+template <typename TIO, int DH, int SPLIT, int NW>
+FM_GLOBAL void FM_LAUNCH_BOUNDS2(64 * NW, (X3Cfg<DH, NW, SPLIT>::OCC)) k_x3_fwd(X3Args<TIO> A) {
   FM_DYN_SMEM(smem);
   FM_SHARED int bad;
   uint16_t* st = reinterpret_cast<uint16_t*>(smem);
   if (FM_TID_X == 0) bad = 0;
   if (!A.plain) {
-    fm_x3_fwd<TIO, DH, SPLIT, X3Row<DH>>(A, st, &bad, FM_TID_X);
+    fm_x3_fwd<TIO, DH, SPLIT, X3Row<DH>, NW>(A, st, &bad, FM_TID_X);
     if (!fm_x3_again(&bad)) FM_END();
   }
-  fm_x3_fwd<TIO, DH, SPLIT, F32Row<DH>>(FM_ARGS_AGAIN(A), st, &bad, FM_TID_X + FM_OPAQUE_ZERO());
+  fm_x3_fwd<TIO, DH, SPLIT, F32Row<DH>, NW>(FM_ARGS_AGAIN(A), st, &bad, FM_TID_X + FM_OPAQUE_ZERO());
 }
 
 // ------------------------------------------------------------------------------
-// dQ.  grid (ceil(nq / QW), bh), 256 threads.  dS = (a1 + 2 a2 s) (gh . v - c), gh = dO / g, c = gh . o.
+// dQ.  grid (ceil(nq / QW), bh).  dS = (a1 + 2 a2 s) (gh . v - c), gh = dO / g, c = gh . o.
 // ------------------------------------------------------------------------------
-template <typename TIO, int DH, int SPLIT, typename R>
+template <typename TIO, int DH, int SPLIT, typename R, int NW>
 FM_DEVICE void fm_x3_dq(const X3Args<TIO>& A, uint16_t* st, int* bad, const int tid) {
-  typedef X3Cfg<DH, 4, SPLIT> C;
+  typedef X3Cfg<DH, NW, SPLIT> C;
   constexpr int NT = DH / 32, PQ = C::PQ, KT = C::KT, QW = C::QW;
   const int lane = tid & 63, lr = lane & 31, lh = lane >> 5;
   const int wave = FM_UNIFORM(tid >> 6), own = wave / SPLIT, sub = wave % SPLIT;
@@ -619,17 +619,17 @@ FM_DEVICE void fm_x3_dq(const X3Args<TIO>& A, uint16_t* st, int* bad, const int 
   fm_x3_store<TIO, DH, QW, SPLIT, C::NTH, R>(acc, reinterpret_cast<float*>(st), sub, 32 * own + lr, lh, A.sc * (A.bpart ? qf : 1.0f), A.out,
                                           bh, t0, A.nq, tid, A.q, A.bpart ? A.bpart + int64_t(bh) * FM_GDIM_X + blk : nullptr, bad);
 }
-template <typename TIO, int DH, int SPLIT>
-FM_GLOBAL void FM_LAUNCH_BOUNDS2(256, (X3Cfg<DH, 4, SPLIT>::OCC)) k_x3_dq(X3Args<TIO> A) {
+template <typename TIO, int DH, int SPLIT, int NW>
+FM_GLOBAL void FM_LAUNCH_BOUNDS2(64 * NW, (X3Cfg<DH, NW, SPLIT>::OCC)) k_x3_dq(X3Args<TIO> A) {
   FM_DYN_SMEM(smem);
   FM_SHARED int bad;
   uint16_t* st = reinterpret_cast<uint16_t*>(smem);
   if (FM_TID_X == 0) bad = 0;
   if (!A.plain) {
-    fm_x3_dq<TIO, DH, SPLIT, X3Row<DH>>(A, st, &bad, FM_TID_X);
+    fm_x3_dq<TIO, DH, SPLIT, X3Row<DH>, NW>(A, st, &bad, FM_TID_X);
     if (!fm_x3_again(&bad)) FM_END();
   }
-  fm_x3_dq<TIO, DH, SPLIT, F32Row<DH>>(FM_ARGS_AGAIN(A), st, &bad, FM_TID_X + FM_OPAQUE_ZERO());
+  fm_x3_dq<TIO, DH, SPLIT, F32Row<DH>, NW>(FM_ARGS_AGAIN(A), st, &bad, FM_TID_X + FM_OPAQUE_ZERO());
 }
 
 // ------------------------------------------------------------------------------
