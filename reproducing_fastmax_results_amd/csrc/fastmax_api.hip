@@ -11,6 +11,7 @@
 #include "fm_pointwise.h"
 #include "fm_walk_sym.h"
 #include "fm_x3.h"
+#include "fm_x2.h"
 #include "fm_small.h"
 #if defined(FM_BENCH_AIDS)
 #include "fm_bench_aids.h"
@@ -97,6 +98,8 @@ struct Plan {
   bool keep_resid;      // the forward leaves o - bf16(o) for the backward (see TokArgs::out_resid)
   bool tiny;            // at most 64 tokens: fm_small.h
   bool x3;              // fp32 arithmetic without states: the kernels of fm_x3.h (read the caller's tensors, no copies)
+  bool x2;              // of those: the kernels of fm_x2.h
+  int x2_ew; size_t x2r, b_x2r;         // exponent of their weights' factor; ranges of q, k, v (see k_x2_range), of gh, q, k, v
   bool sym;             // order-2 states are built by the walk per value column (k_walk_sym): one layout, no transposed copy   // run, runh: see k_o1_sums
   bool save;
   size_t b_kr, b_vr, b_qr, b_kt, b_vt, b_qt, b_qct, b_gh, b_ght, b_cv, b_bigq, b_smallq, b_bigk, b_smallk, b_bigv, b_gpart, b_bq, b_bk, b_runq, b_runqh, b_runk, b_runkh, bwd_bytes;
@@ -126,12 +129,42 @@ inline bool half_arithmetic(const FastmaxDesc* d) {
 // Unmasked attention: one total of the moments costs less than products with every key.
 inline bool states_pay_unmasked(const FastmaxDesc* d) { return int64_t(d->nk) > int64_t(d->d) * d->d + d->d; }
 
-// How many wavefronts share an own tile in the fp32 kernels of dense tiles (fm_x3.h): with one each, a launch has blocks of 128
+// How many wavefronts share an own tile in the fp32 kernels of dense tiles (fm_x3.h, fm_x2.h): with one each, a launch has blocks of 128
 // own tokens (256 for dK + dV); below two workgroups per CU the own tiles are spread over twice or four times as many.
+#if defined(FM_HOSTSIM)
+// The CPU tests' problems are few and short: set, they go to the kernels of fm_x2.h, with this many wavefronts to an own tile.
+static int fm_hostsim_x2 = 0;
+extern "C" void fastmax_hostsim_x2(int split) { fm_hostsim_x2 = split; }
+#endif
 inline int x3_split(int bh, int n_own, int tokens) {
+#if defined(FM_HOSTSIM)
+  if (fm_hostsim_x2) return fm_hostsim_x2;
+#endif
   const int blocks = bh * ((n_own + tokens - 1) / tokens);
   return blocks >= 512 ? 1 : blocks >= 256 ? 2 : 4;
 }
+// Dense fp32 problems for the kernels of fm_x2.h: not before their error against 64 bits is no larger than that of fm_x3.h's.  Two planes
+// round an operand once more, three products round the sums half as often as six, so sums of enough terms decide it, and
+// sums spread over several wavefronts (sq, sk: x3_split) need more.  Both sides' errors, ratios of o, dq, dk, dv: causal, D = 64, one
+// wavefront per own tile, 512 tokens 1.00 1.01 1.07 1.07, 1024 .91 .92 .93 .91, 4096 .82 .83 .84 .82; two for dK + dV, 777 .94 .91 .99 1.02, 1024
+// .92 .93 .99 .99; two and four, 1536 .95 .96 1.00 1.03, 2048 .92 .90 .96 1.00; four, 2048 1.01 1.02 1.00 1.00, 3000 .96 .95 .95 .95.
+// D = 32: two for dK + dV, 1024 .92 .95 1.04 .99, 1536 .88 .90 .97 .95; four, 3000 .96 1.00 1.01 .96, 4096 .93 .98 .98 .92.  Unmasked: four, 300 keys
+// 1.01 .99 1.00 1.02, 1024 .86 .89 .89 .85; two and four, 512 .85 .87 .95 .94.
+inline bool x2_pays(const FastmaxDesc* d, int sq, int sk) {
+#if defined(FM_HOSTSIM)
+  if (fm_hostsim_x2) return true;
+#endif
+  const int n = d->nq < d->nk ? d->nq : d->nk;
+  if (!d->mask) return n >= (sk == 4 ? 1024 : 512);
+  if (d->d == 32) return n >= (sk == 1 ? 1024 : sk == 2 ? 1536 : 4096);
+  return n >= (sk < 4 ? 1024 : sq < 4 ? 2048 : 3072);
+}
+// own tokens of a workgroup there
+inline int x2_rows(int kind, int split, int bh, int n_own) {
+  if (kind < 2 && split == 1 && bh * ((n_own + 255) / 256) < 512) return 128;
+  return 256 / split;
+}
+
 int validate(const FastmaxDesc* d) {
   if (!d) return FASTMAX_ERR_NULL;
   if (d->dtype != FASTMAX_F32 && d->dtype != FASTMAX_BF16) return FASTMAX_ERR_DTYPE;
@@ -170,6 +203,9 @@ template <int DH> size_t big_array_bytes(int esz, bool quad, size_t slots) {
   if (!slots) return 0;
   return (slots * size_t(StateDims<DH>::stride(quad)) + (quad ? 0 : size_t(StateDims<DH>::PAD_SLABS) * StateDims<DH>::SLAB)) * esz;
 }
+
+// floats of the ranges of q, k and v (see launch_x2_range)
+inline size_t x2_keys(const FastmaxDesc* d) { return size_t(d->bh) * (fm_x2_blocks(d->nq) + 2 * fm_x2_blocks(d->nk)); }
 
 int make_plan(const FastmaxDesc* d, Plan& p) {
   int st = validate(d);
@@ -213,6 +249,9 @@ int make_plan(const FastmaxDesc* d, Plan& p) {
   }
   p.tiny = is_small(d);
   p.x3 = !p.half && !p.use_state && !p.tiny;
+  p.x2_ew = 0;
+  const bool x2_fits = p.x3 && d->dtype == FASTMAX_F32 && x2_coefficients(p.a0, p.a1, p.a2, p.x2_ew);
+  p.x2 = x2_fits && x2_pays(d, x3_split(d->bh, d->nq, 128), x3_split(d->bh, d->nk, 256));
   p.o1 = p.half && p.use_state && !p.quad && d->mask && p.L == FM_O1_SEG && d->nq == d->nk;
   p.rows_build = p.half && p.use_state && !p.quad && d->mask;
   {
@@ -255,6 +294,7 @@ int make_plan(const FastmaxDesc* d, Plan& p) {
   p.run = take(runarr); p.runh = take(runharr);
   p.keep_resid = p.save && d->dtype == FASTMAX_BF16 && !p.o1;
   p.ores = take(p.keep_resid ? size_t(d->bh) * (p.tiny ? d->nq : p.npad_q) * d->d * 2 : 0);
+  p.x2r = take(p.x2 ? x2_keys(d) * 4 : 0);
   p.fwd_bytes = off ? off : 256;
   off = 0;
   p.b_kt = take(tkt); p.b_vt = take(tkt); p.b_qt = take(tqt); p.b_qct = take(tqt);
@@ -270,6 +310,7 @@ int make_plan(const FastmaxDesc* d, Plan& p) {
   p.b_bq = take(jac && d->norm.q_keys ? size_t(d->bh) * ((d->nq + 31) / 32) * 4 : 0);
   p.b_bk = take(jac && d->norm.k_keys ? size_t(d->bh) * ((d->nk + 31) / 32) * 4 : 0);
   p.b_runq = take(runarr); p.b_runqh = take(runharr); p.b_runk = take(runarr); p.b_runkh = take(runharr);
+  p.b_x2r = take(p.x2 ? (x2_keys(d) + size_t(2) * d->bh * fm_x2_blocks(d->nq)) * 4 : 0);
   p.bwd_bytes = off ? off : 256;
   return FASTMAX_OK;
 }
@@ -585,6 +626,55 @@ int launch_x3(const X3Args<TIO>& a, int split, int n_own, int n_str, int bh, fm_
   return launch_x3_cfg<TIO, DH, KIND, 2, NW>(a, n_own, bh, stream);
 }
 
+// Ranges of the tensors that are not null (gh: of d_o / g, its tails behind them; see k_x2_range), in `keys` those of q, k, v; a: where
+// they lie.
+template <int DH>
+int launch_x2_range(const FastmaxDesc* d, const void* q, const void* k, const void* v, const void* d_o, const float* g, float* keys,
+                    float* gh, X2Args& a, fm_stream_t stream) {
+  const int nbq = fm_x2_blocks(d->nq), nbk = fm_x2_blocks(d->nk);
+  float *mq = keys, *mk = mq + size_t(d->bh) * nbq, *mv = mk + size_t(d->bh) * nbk;
+  float* tail = gh ? gh + size_t(d->bh) * nbq : nullptr;
+  a.mq = mq; a.mk = mk; a.mv = mv; a.mg = gh; a.tg = tail; a.nbq = nbq; a.nbk = nbk;
+  X2Job j[4];
+  int n = 0;
+  if (q) j[n++] = X2Job{cref<float>(q, d->sq), TRef<float>{}, mq, nullptr, d->nq, nbq, 0};
+  if (k) j[n++] = X2Job{cref<float>(k, d->sk), TRef<float>{}, mk, nullptr, d->nk, nbk, 0};
+  if (v) j[n++] = X2Job{cref<float>(v, d->sv), TRef<float>{}, mv, nullptr, d->nk, nbk, 0};
+  if (d_o) j[n++] = X2Job{cref<float>(d_o, d->sdo), fm_ref<float>(const_cast<float*>(g), d->sg), gh, tail, d->nq, nbq, 1};
+  const int jobs = n;
+  while (n < 4) { j[n] = j[0]; ++n; }
+  ProfScope prof(FM_K_PREP_BWD, stream);
+  FM_KERNEL_LAUNCH((k_x2_range<DH>), fm_dim3(nbq > nbk ? nbq : nbk, d->bh, jobs), fm_dim3(256), 0, stream, j[0], j[1], j[2], j[3]);
+  return fm_launch_status();
+}
+template <int DH, int KIND, int SPLIT, int NW>
+int launch_x2_cfg(const X2Args& a, int n_own, int bh, fm_stream_t stream) {
+  typedef X2Cfg<DH, NW, SPLIT> C;
+  const size_t lds = C::lds(KIND == 2);
+  ProfScope prof(KIND == 0 ? FM_K_FWD : KIND == 1 ? FM_K_DQ : FM_K_DKV, stream);
+  const fm_dim3 grid((n_own + C::QW - 1) / C::QW, bh), block(C::NTH);
+  if constexpr (KIND == 0) {
+    fm_allow_lds(reinterpret_cast<const void*>(&k_x2_fwd<DH, SPLIT, NW>), lds);
+    FM_KERNEL_LAUNCH((k_x2_fwd<DH, SPLIT, NW>), grid, block, lds, stream, a);
+  } else if constexpr (KIND == 1) {
+    fm_allow_lds(reinterpret_cast<const void*>(&k_x2_dq<DH, SPLIT, NW>), lds);
+    FM_KERNEL_LAUNCH((k_x2_dq<DH, SPLIT, NW>), grid, block, lds, stream, a);
+  } else {
+    fm_allow_lds(reinterpret_cast<const void*>(&k_x2_dkv<DH, SPLIT>), lds);
+    FM_KERNEL_LAUNCH((k_x2_dkv<DH, SPLIT>), grid, block, lds, stream, a);
+  }
+  return fm_launch_status();
+}
+template <int DH, int KIND>
+int launch_x2(const X2Args& a, int split, int n_own, int bh, fm_stream_t stream) {
+  if constexpr (KIND < 2) {
+    if (x2_rows(KIND, split, bh, n_own) == 128 && split == 1) return launch_x2_cfg<DH, KIND, 1, 4>(a, n_own, bh, stream);
+  }
+  if (split == 1) return launch_x2_cfg<DH, KIND, 1, 8>(a, n_own, bh, stream);
+  if (split == 2) return launch_x2_cfg<DH, KIND, 2, 8>(a, n_own, bh, stream);
+  return launch_x2_cfg<DH, KIND, 4, 8>(a, n_own, bh, stream);
+}
+
 // ---- at most 64 tokens (fm_small.h) ----------------------------------------------------------
 template <typename TIO> SmallArgs<TIO> small_args(const FastmaxDesc* d, const Plan& p, const void* q, const void* k, const void* v) {
   SmallArgs<TIO> a;
@@ -632,6 +722,18 @@ int run_forward(const FastmaxDesc* d, const Plan& p, const void* q, const void* 
   if constexpr (sizeof(E) == 2 && DH <= 64) {
     if (p.o1) return run_forward_o1<TIO, DH>(d, p, q, k, v, o, g, ws, stream);
   } else if constexpr (sizeof(E) == 4) {
+    if constexpr (sizeof(TIO) == 4) {
+      if (p.x2) {
+        X2Args a;
+        static_cast<X3Args<float>&>(a) = x3_args<float>(d, p, q, k, v);
+        a.ew = p.x2_ew;
+        a.out = mref<TIO>(o, d->so); a.g = mref<float>(g, d->sg);
+        // (a backward on this workspace reads q's as well)
+        const int st = launch_x2_range<DH>(d, p.save ? q : nullptr, k, v, nullptr, nullptr, reinterpret_cast<float*>(ws + p.x2r), nullptr, a, stream);
+        if (st) return st;
+        return launch_x2<DH, 0>(a, x3_split(d->bh, d->nq, 128), d->nq, d->bh, stream);
+      }
+    }
     if (p.x3) {
       X3Args<TIO> a = x3_args<TIO>(d, p, q, k, v);
       a.out = mref<TIO>(o, d->so); a.g = mref<float>(g, d->sg);

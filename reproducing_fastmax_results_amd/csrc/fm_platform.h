@@ -121,6 +121,7 @@ FM_DEVICE float fm_absf(float x) { return __builtin_fabsf(x); }
 FM_DEVICE float fm_clampf(float x, float lim) { return x > lim ? lim : (x < -lim ? -lim : x); }
 FM_DEVICE float fm_rsqrtf(float a) { return 1.0f / std::sqrt(a); }
 FM_DEVICE float fm_sqrtf(float a) { return std::sqrt(a); }
+FM_DEVICE float fm_rcpf(float a) { return 1.0f / a; }
 
 #else
 // ------------------------------------------------------------------ gfx950
@@ -245,6 +246,8 @@ FM_DEVICE float fm_absf(float x) { return __builtin_fabsf(x); }
 FM_DEVICE float fm_clampf(float x, float lim) { return __builtin_amdgcn_fmed3f(x, -lim, lim); }
 FM_DEVICE float fm_rsqrtf(float a) { return rsqrtf(a); }
 FM_DEVICE float fm_sqrtf(float a) { return sqrtf(a); }
+// 1 / a for an ordinary a, to within a rounding of it (one correction of the instruction's result)
+FM_DEVICE float fm_rcpf(float a) { const float r = __builtin_amdgcn_rcpf(a); return __builtin_fmaf(r, __builtin_fmaf(-a, r, 1.0f), r); }
 #endif
 
 // ---- bf16 <-> f32 (round to nearest even), usable on both builds -------------

@@ -371,10 +371,10 @@ template <int DH, int QW, int SPLIT> FM_DEVICE void fm_x3_sum8(const float* Os, 
   }
 }
 // Gradient rows of the workgroup -> caller's tensor, times scale.  bout: the sum of stored value times raw row (the
-// normalisation's B: stored = fac dy, y = fac x, so dy . y = stored . x), one float per workgroup, or null.  bad: see
-// fm_x3_look.
-template <typename TIO, int DH, int QW, int SPLIT, int NTH, typename R>
-FM_DEVICE void fm_x3_store(const fm_f32x16* acc, float* Os, int sub, int row, int lh, float scale, const TRef<TIO>& out,
+// normalisation's B: stored = fac dy, y = fac x, so dy . y = stored . x), one float per workgroup, or null.  unscale: takes a power
+// of two out of the sums first.  LOOK, bad: see fm_x3_look.
+template <typename TIO, int DH, int QW, int SPLIT, int NTH, bool LOOK>
+FM_DEVICE void fm_x3_store(const fm_f32x16* acc, float* Os, int sub, int row, int lh, float unscale, float scale, const TRef<TIO>& out,
                            int bh, int t0, int n, int tid, const TRef<const TIO>& raw, float* bout, int* bad) {
   FM_SYNC();                                           // whatever lay there has been read
   fm_x3_put<DH, QW>(acc, Os, sub, row, lh);
@@ -385,9 +385,9 @@ FM_DEVICE void fm_x3_store(const fm_f32x16* acc, float* Os, int sub, int row, in
     if (t0 + r >= n) continue;
     float v[8];
     fm_x3_sum8<DH, QW, SPLIT>(Os, r, col, v);
-    if (R::PIPE) fm_x3_look(bad, v, 0.f);
+    if (LOOK) fm_x3_look(bad, v, 0.f);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] = v[i] * (1.0f / (R::UP * R::UP)) * scale;
+    for (int i = 0; i < 8; ++i) v[i] = v[i] * unscale * scale;
     if (bout) {
       float x[8];
       IO<TIO>::ld8(raw.base(bh) + int64_t(t0 + r) * raw.s_n + col, x);
@@ -616,7 +616,7 @@ FM_DEVICE void fm_x3_dq(const X3Args<TIO>& A, uint16_t* st, int* bad, const int 
       }
     } else FM_SYNC();
   }
-  fm_x3_store<TIO, DH, QW, SPLIT, C::NTH, R>(acc, reinterpret_cast<float*>(st), sub, 32 * own + lr, lh, A.sc * (A.bpart ? qf : 1.0f), A.out,
+  fm_x3_store<TIO, DH, QW, SPLIT, C::NTH, R::PIPE>(acc, reinterpret_cast<float*>(st), sub, 32 * own + lr, lh, 1.0f / (R::UP * R::UP), A.sc * (A.bpart ? qf : 1.0f), A.out,
                                           bh, t0, A.nq, tid, A.q, A.bpart ? A.bpart + int64_t(bh) * FM_GDIM_X + blk : nullptr, bad);
 }
 template <typename TIO, int DH, int SPLIT, int NW>
@@ -734,9 +734,9 @@ FM_DEVICE void fm_x3_dkv(const X3Args<TIO>& A, uint16_t* Vs, int* bad, const int
     } else FM_SYNC();
   }
   float* Os = reinterpret_cast<float*>(Vs);
-  fm_x3_store<TIO, DH, QW, SPLIT, C::NTH, R>(acc, Os, sub, 32 * own + lr, lh, A.sc * (A.bpart ? kf : 1.0f), A.out, bh, t0, A.nk, tid, A.k,
+  fm_x3_store<TIO, DH, QW, SPLIT, C::NTH, R::PIPE>(acc, Os, sub, 32 * own + lr, lh, 1.0f / (R::UP * R::UP), A.sc * (A.bpart ? kf : 1.0f), A.out, bh, t0, A.nk, tid, A.k,
                                           A.bpart ? A.bpart + int64_t(bh) * FM_GDIM_X + blk : nullptr, bad);
-  fm_x3_store<TIO, DH, QW, SPLIT, C::NTH, R>(av, Os, sub, 32 * own + lr, lh, 1.0f, A.out2, bh, t0, A.nk, tid, A.k, nullptr, bad);
+  fm_x3_store<TIO, DH, QW, SPLIT, C::NTH, R::PIPE>(av, Os, sub, 32 * own + lr, lh, 1.0f / (R::UP * R::UP), 1.0f, A.out2, bh, t0, A.nk, tid, A.k, nullptr, bad);
 }
 template <typename TIO, int DH, int SPLIT>
 FM_GLOBAL void FM_LAUNCH_BOUNDS2(512, 2) k_x3_dkv(X3Args<TIO> A) {

@@ -265,3 +265,26 @@ def check_prompt_at_the_ends_of_the_range(lib, d, dtype, device, n, *, bh=2, see
         finite = torch.isfinite(want)
         off = (one[finite].double() - want[finite].double()).abs() / (n * 2.0 ** -23 * size[finite].double()).clamp_min(1e-44)
         assert float(off.max()) <= 1.0, f"v = {x:g}: {float(off.max()):g} of the bound"
+
+
+def check_ranges_of_two_planes(lib, bh, n, d, device, *, mask=True, seed=0, tol=2e-6):
+    """fp32, entries far below the rest of their tensor: a column of v and of dO, a row of k and v, the last queries' dO.  Each result that
+    only they reach is held to fp32's bar by itself: the column of o and dv, the first query's o (causal), the last keys' dv."""
+    tau = 8.0 * math.sqrt(d)
+    kw = dict(mask=mask, inv_tau=1.0 / tau, p=2)
+    for which in ("column of v", "column of dO", "first row of v", "last rows of dO"):
+        q, k, v, go = make_inputs(bh, n, n, d, torch.float32, device, seed)
+        if which == "column of v": v[:, :, 3] *= 1e-9
+        if which == "column of dO": go[:, :, 3] *= 1e-9
+        if which == "first row of v": v[:, 0] *= 1e-9
+        if which == "last rows of dO": go[:, -40:] *= 1e-9
+        o, g = lib.forward(q, k, v, **kw)
+        dq, dk, dv = lib.backward(q, k, v, o, g, go, **kw)
+        ref = oracle_all(q, k, v, go, mask=mask, tau=tau, p=2)
+        parts = {"o": (o, ref[0]), "g": (g, ref[1]), "dq": (dq, ref[2]), "dk": (dk, ref[3]), "dv": (dv, ref[4])}
+        if which == "column of v": parts["o there"] = (o[..., 3], ref[0][..., 3])
+        if which == "column of dO": parts["dv there"] = (dv[..., 3], ref[4][..., 3])
+        if which == "first row of v" and mask: parts["o there"] = (o[:, 0], ref[0][:, 0])
+        if which == "last rows of dO" and mask: parts["dv there"] = (dv[:, -40:], ref[4][:, -40:])
+        for m, (x, r) in parts.items():
+            assert rel_err(x, r) < tol, f"{which}: {m} {rel_err(x, r):.3e}"

@@ -4,7 +4,7 @@ bf16-rounded inputs)."""
 import pytest
 import torch
 
-from tests.parity import (check_infinite_and_largest_values, check_prompt_at_the_ends_of_the_range, check_tiny_values, check_upstream_gradients_at_the_ends_of_the_range, check_batch_head_strides, check_decode, check_forward, check_forward_backward,
+from tests.parity import (check_ranges_of_two_planes, check_infinite_and_largest_values, check_prompt_at_the_ends_of_the_range, check_tiny_values, check_upstream_gradients_at_the_ends_of_the_range, check_batch_head_strides, check_decode, check_forward, check_forward_backward,
                           check_norm_fold, make_inputs)
 from reproducing_fastmax_results_amd._capi import FLAG_F32_COMPUTE, FLAG_FORCE_DENSE, FLAG_FORCE_MOMENTS, FLAG_NORM_SELF
 
@@ -316,6 +316,51 @@ def test_fp32_dense_tiles(lib, d, bh, n):
               check_forward_backward(lib, bh, n, d, f, DEV, mask=False, p=2, nk=n + 37, seed=131)):
         assert max(e.values()) < 2e-6, e
     check_forward_backward(lib, bh, n, d, torch.bfloat16, DEV, mask=True, p=2, seed=132, saved=True, flags=FLAG_F32_COMPUTE)
+
+
+@pytest.mark.parametrize("bh,nq,nk,d,mask,p", [
+    (64, 1030, 1030, 64, True, 2), (130, 1024, 1024, 32, True, 1),   # one wavefront per own tile; two and one for dK + dV
+    (32, 4000, 4000, 32, True, 2),                                   # forward and dQ in workgroups of eight
+    (16, 2050, 2050, 64, True, 2), (3, 3100, 3100, 64, True, 2), (2, 4100, 4100, 32, True, 2),   # tiles shared by two and four
+    (1, 1040, 1100, 64, False, 2), (40, 515, 800, 32, False, 1), (70, 1100, 520, 64, False, 2)])
+def test_fp32_as_three_products_of_two_planes(lib, bh, nq, nk, d, mask, p):
+    """fm_x2.h against 64-bit results on the GPU, by the bar of test_fp32_dense_tiles; one batch*head of values that two planes do not
+    hold beside the others, and a saved backward bit by bit as an independent one."""
+    import math
+    from tests.parity import make_inputs
+    print(f"case two planes bh={bh} nq={nq} nk={nk} d={d} mask={mask} p={p}", flush=True)
+    q, k, v, go = make_inputs(bh, nq, nk, d, torch.float32, DEV, 133)
+    v[-1, :, 1] *= 1e-7
+    tau = 8.0 * math.sqrt(d)
+    kw = dict(mask=mask, inv_tau=1.0 / tau, p=p, a2=0.5 if p == 2 else 0.0, flags=FLAG_FORCE_DENSE)
+    o, g, ws = lib.forward(q, k, v, save=True, **kw)
+    grads = lib.backward(q, k, v, o, g, go, saved=ws, **kw)
+    for x, y in zip(grads, lib.backward(q, k, v, o, g, go, **kw)):
+        assert torch.equal(x, y)
+    num, den = [0.0] * 5, [0.0] * 5
+    for b in sorted({0, bh // 2, bh - 1}):
+        Q, K, V, G = (t[b].double() for t in (q, k, v, go))
+        s = Q @ K.T / tau
+        w, dw = 1.0 + s + (0.5 * s * s if p == 2 else 0.0), 1.0 + (s if p == 2 else torch.zeros_like(s))
+        if mask:
+            w, dw = w.tril(), dw.tril()
+        gs = w.sum(1, keepdim=True)
+        out = w @ V / gs
+        gh = G / gs
+        ds = dw * (gh @ V.T - (gh * out).sum(1, keepdim=True))
+        for i, (x, r) in enumerate(zip((o, g, *grads), (out, gs[:, 0], ds @ K / tau, ds.T @ Q / tau, w.T @ gh))):
+            num[i] += float((x[b].double() - r).norm() ** 2)
+            den[i] += float(r.norm() ** 2)
+        if b == bh - 1:
+            assert float((o[b, :, 1].double() - out[:, 1]).norm() / out[:, 1].norm()) < 2e-6
+    errs = [math.sqrt(x / y) for x, y in zip(num, den)]
+    print("errors o g dq dk dv", " ".join(f"{e:.2e}" for e in errs), flush=True)
+    assert max(errs) < 2e-6, errs
+
+
+def test_ranges_of_two_planes(lib):
+    check_ranges_of_two_planes(lib, 2, 3100, 64, DEV, seed=134)
+    check_infinite_and_largest_values(lib, 1, 1040, 64, torch.float32, DEV, seed=135)
 
 
 @pytest.mark.parametrize("d", [32, 64])

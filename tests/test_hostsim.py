@@ -16,7 +16,7 @@ import pytest
 import torch
 
 from reproducing_fastmax_results_amd import _capi
-from tests.parity import (TOL, check_upstream_gradients_at_the_ends_of_the_range, check_infinite_and_largest_values, check_tiny_values, check_batch_head_strides, check_decode, check_norm_fold, check_prompt_at_the_ends_of_the_range, check_forward, check_forward_backward, make_inputs, oracle_all,
+from tests.parity import (TOL, check_ranges_of_two_planes, check_upstream_gradients_at_the_ends_of_the_range, check_infinite_and_largest_values, check_tiny_values, check_batch_head_strides, check_decode, check_norm_fold, check_prompt_at_the_ends_of_the_range, check_forward, check_forward_backward, make_inputs, oracle_all,
                           rel_err)
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -442,3 +442,27 @@ def test_short_sequences_normalised_with_a_nan_row(sim):
         o, g = sim.forward(q, k, v, mask=False, inv_tau=1.0, p=2, flags=flags, norm=(*keys, 1.5, True))
         assert rel_err(o[:, rest], want[0]) < 2e-6 and rel_err(g[:, rest], want[1]) < 2e-6
         assert bool(torch.isnan(o[:, 3]).all())
+
+
+@pytest.fixture
+def two_planes(sim):
+    yield sim.lib.fastmax_hostsim_x2
+    sim.lib.fastmax_hostsim_x2(0)
+
+
+@pytest.mark.parametrize("split", [1, 2, 4])
+def test_fp32_as_three_products_of_two_planes(sim, two_planes, split):
+    """fm_x2.h, which problems of these sizes do not reach by themselves: tile edges, more keys than queries, coefficients of another
+    size, saved and not; and values that two planes do not hold, which go the way of fm_x3.h.  The bar of test_fp32_dense_tiles."""
+    two_planes(split)
+    f = torch.float32
+    for e in (check_forward_backward(sim, 1, 130, 32, f, "cpu", mask=True, p=2, seed=70, saved=True, flags=_capi.FLAG_FORCE_DENSE),
+              check_forward_backward(sim, 2, 70, 64, f, "cpu", mask=False, p=2, nk=97, a=(2.0, 1.5, 0.25), seed=71),
+              check_forward_backward(sim, 1, 97, 32, f, "cpu", mask=True, p=1, a=(0.01, 0.02, 0.0), seed=72)):
+        assert max(e.values()) < 2e-6, e
+    check_norm_fold(sim, 1, 70, 32, f, "cpu", mask=True, p=2, seed=73)
+    check_ranges_of_two_planes(sim, 1, 130, 32, "cpu", seed=74)
+    if split == 1:
+        check_infinite_and_largest_values(sim, 1, 66, 32, f, "cpu", seed=75)
+        check_tiny_values(sim, 1, 66, 32, f, "cpu", tol=2e-6, seed=76)
+        check_forward_backward(sim, 1, 66, 32, f, "cpu", mask=True, p=2, seed=77, scale=30.0)    # weights beyond 65504
