@@ -463,7 +463,8 @@ template <typename TIO, typename E> void tok_common(TokArgs<TIO, E>& a, const Fa
   a.out_resid = nullptr; a.own_ores = nullptr; a.state_xscale = 1.0f;
 }
 
-// Launches that go with two groups of wavefronts per workgroup (GRP in fm_tok.h), by their number of workgroups on the chip's 256 CUs.
+// Launches that go with two groups of wavefronts per workgroup (GRP in fm_tok.h), by their number of workgroups on the chip's 256 CUs:
+// without the causal mask, and the forward of heads of 32 (the others under the mask: half_blocks, which is asked first).
 // At one workgroup per CU or less every kernel gains (whole calls, microseconds, one group and two; forward of 1 x 8 heads of 64, 4096
 // tokens 54 -> 41.5, of 2 x 8 of 2048 32 -> 27, unmasked 54 -> 45; D = 32 23 -> 19; D = 128 53 -> 48.5; a step with dQ so 174 -> 165,
 // with dK + dV so 174 -> 166).  The causal forward gains up to two per CU where its chains are long, since the light workgroups leave
@@ -486,11 +487,32 @@ inline bool two_groups(int kind, int dh, int64_t workgroups, bool causal, int n_
   return workgroups <= (kind == FM_GRP_DV && !causal ? 128 : 256);      // (dK + dV of heads of 128 is not built so)
 }
 
+// Launches under the causal mask that go with blocks of 64 own tokens (HALF in fm_tok.h), by their number of blocks of 128.  Whole calls,
+// microseconds, blocks of 128 (in two groups of wavefronts where those are taken) and of 64: forward of 16 heads of 64, 2048 tokens
+// 27.7, 25.2, 24 heads 32.9, 31.5, 32 36.6, 36.1, 8 of 4096 42.7, 38.6, but D = 32 27.1, 28.7; D = 128 16 heads 44.4, 42.3, 24 52.8, 50.7, 32 60, 62.
+// A backward with dQ so: 16 heads 61.3, 57.9, 24 77.0, 70.4, 32 86.2, 85.8, D = 32 24 heads 50.9, 45.8, D = 128 16 heads 119, 108, 24 132, 128.
+// With dK + dV so: 8 heads 57.0, 52.6, 16 61.3, 57.8, 24 77.0, 76.3, 48 of 1024 49.4, 51.3; D = 128 8 heads 111, 105, 16 119, 122.  (Both at once, four
+// shares of a tile: forward at 128 blocks 23.2, 23.3, at 256 25.2, 27.2, dQ 52.6, 51.4 and 57.9, 65.0.)
+inline bool half_blocks(int kind, int dh, int64_t blocks, bool causal) {
+#if defined(FM_HOSTSIM)
+  if (fm_hostsim_one_group) return false;
+#endif
+  if (kind == FM_GRP_PV) return causal && dh != 32 && blocks <= (dh == 64 ? 512 : 384);
+  return causal && blocks <= (kind == FM_GRP_DS ? 384 : dh > 64 ? 128 : 256);
+}
+
 template <typename TIO, typename E, int DH, int QT, int OWN, int QF = 0>
 int launch_pv(const TokArgs<TIO, E>& a, int bh, int kernel_id, fm_stream_t stream) {
   typedef TokCfg<E, DH, QT> C;
   ProfScope prof(kernel_id, stream);
   const fm_dim3 grid((a.n_own + C::QW - 1) / C::QW, bh);
+  if constexpr (sizeof(E) == 2 && QT == 1 && OWN == FM_OWN_Q && DH != 32) {
+    if (!a.use_state && half_blocks(FM_GRP_PV, DH, int64_t(grid.x) * bh, a.causal)) {
+      fm_allow_lds(reinterpret_cast<const void*>(&k_pv<TIO, E, DH, QT, OWN, QF, 1, 1>), C::HALF_PV);
+      FM_KERNEL_LAUNCH((k_pv<TIO, E, DH, QT, OWN, QF, 1, 1>), fm_dim3((a.n_own + 63) / 64, bh), fm_dim3(FM_THREADS), C::HALF_PV, stream, a);
+      return fm_launch_status();
+    }
+  }
   if constexpr (sizeof(E) == 2 && QT == 1 && OWN == FM_OWN_Q) {
     if (!a.use_state && two_groups(FM_GRP_PV, DH, int64_t(grid.x) * bh, a.causal, a.n_str)) {
       constexpr size_t lds = 2 * C::GRP_PV;
@@ -510,6 +532,14 @@ int launch_ds(const TokArgs<TIO, E>& a, int bh, int kernel_id, fm_stream_t strea
   typedef TokCfg<E, DH, QT> C;
   ProfScope prof(kernel_id, stream);
   const fm_dim3 grid((a.n_own + C::QW - 1) / C::QW, bh);
+  if constexpr (sizeof(E) == 2 && QT == 1 && !STR && (PREP || DV)) {
+    if (!a.use_state && half_blocks(DV ? FM_GRP_DV : FM_GRP_DS, DH, int64_t(grid.x) * bh, a.causal)) {
+      constexpr size_t lds = DV ? C::HALF_DV : C::HALF_DS;
+      fm_allow_lds(reinterpret_cast<const void*>(&k_ds<TIO, E, DH, QT, OWN, DV, PREP, QF, STR, 1, 1>), lds);
+      FM_KERNEL_LAUNCH((k_ds<TIO, E, DH, QT, OWN, DV, PREP, QF, STR, 1, 1>), fm_dim3((a.n_own + 63) / 64, bh), fm_dim3(FM_THREADS), lds, stream, a);
+      return fm_launch_status();
+    }
+  }
   if constexpr (sizeof(E) == 2 && (DH <= 64 || PREP) && QT == 1 && !STR && (PREP || DV)) {
     if (!a.use_state && two_groups(DV ? FM_GRP_DV : FM_GRP_DS, DH, int64_t(grid.x) * bh, a.causal, a.n_str)) {
       constexpr size_t lds = 2 * (DV ? C::GRP_DV : C::GRP_DS);

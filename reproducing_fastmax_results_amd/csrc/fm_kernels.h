@@ -1298,6 +1298,7 @@ struct TokCfg {
   static constexpr int OCC_PV = WIDE ? 2 : (sizeof(E) == 2 ? (QT == 1 ? 4 : 2) : 1);   // workgroups per CU the kernels are sized for
   static constexpr int OCC_DS = WIDE ? 1 : (sizeof(E) == 2 ? (QT == 1 ? 3 : 2) : 1);
   static constexpr int OCC_DV = WIDE ? 1 : 2;
+  static constexpr int OCC_DS_HALF = WIDE ? 2 : OCC_DS;
   static constexpr int SA = sizeof(E) == 2 ? QT : 2;                      // values of a per state slab
   // Stream tokens per stage of the dense loop, k_pv.  A stage waits for loads that began one stage earlier, so short stages are
   // bound by that latency: with 64 tokens instead of 32, forward at D = 32, 4 x 8 heads of 4096 tokens 77 -> 53 us, 2 x 8 of 2048
@@ -1331,6 +1332,11 @@ struct TokCfg {
   static constexpr size_t GRP_DS = 2 * DH * 4 + cmax(2 * QW * PQ * sizeof(E) + QW * 4, sizeof(E) * DS_NBUF * DS_STAGE);
   static constexpr size_t GRP_DV = 2 * DH * 4 + sizeof(E) * cmax(QW * PQ, DS_NBUF * DV_STAGE);
   static constexpr size_t JOIN = size_t(FM_THREADS) * 4 * (16 * NT + 1);
+  // Blocks of 64 own tokens (see fm_join_halves): LDS of a workgroup
+  static constexpr int HALF_STAGE = 2 * 64 * PQ;
+  static constexpr size_t HALF_PV = 2 * DH * 4 + cmax(JOIN / 2, sizeof(E) * cmax(64 * PQ, 2 * HALF_STAGE));
+  static constexpr size_t HALF_DS = 2 * DH * 4 + cmax(cmax(JOIN / 2, 2 * 64 * PQ * sizeof(E) + 64 * 4), sizeof(E) * DS_NBUF * DS_STAGE);
+  static constexpr size_t HALF_DV = 2 * DH * 4 + cmax(JOIN / 2, sizeof(E) * cmax(64 * PQ, DS_NBUF * DV_STAGE));
 };
 
 // Moment readout, transposed:  acc[j][ct] (rows c, column = token of tile j) +=

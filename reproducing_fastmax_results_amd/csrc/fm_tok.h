@@ -295,15 +295,37 @@ template <int NACC> FM_DEVICE void fm_join_groups(float* lds, fm_f32x16* acc, in
   FM_SYNC();
 }
 
+// HALF = 1: a workgroup owns 64 tokens instead of 128; two of its wavefronts hold the same own tile, each takes every other 32-token
+// tile of a stage, and their sums meet here.  A causal launch of about as many workgroups as the chip has places takes as long as its
+// longest one, twice the average; blocks of half the size are twice as many, and heavy and light ones share a CU (see fm_snake_rank).
+// The wavefront holds tile wv and share sub of it; extra: one more sum per lane, or null.
+template <int NACC> FM_DEVICE void fm_join_halves(float* lds, fm_f32x16* acc, float* extra, int sub, int wv, int lane) {
+  float* p = lds + wv * (16 * NACC + 1) * 64 + lane;
+  if (sub == 1) {
+#pragma unroll
+    for (int i = 0; i < 16 * NACC; ++i) p[i * 64] = acc[i / 16][i % 16];
+    if (extra) p[16 * NACC * 64] = *extra;
+  }
+  FM_SYNC();
+  if (sub == 0) {
+#pragma unroll
+    for (int i = 0; i < 16 * NACC; ++i) acc[i / 16][i % 16] += p[i * 64];
+    if (extra) *extra += p[16 * NACC * 64];
+  }
+  FM_SYNC();
+}
+
 // ------------------------------------------------------------------------------
 // k_pv: forward (own = queries) and dV (own = keys).  grid (ceil(n_own / QW), bh).
 // LDS: va, vb | own rows [QW][PQ] | region (Z, then state slabs); the two dense stages lie over the own rows and the region
-// once they are spent.  Outputs leave straight from the accumulators (fm_each_octet).  GRP = 2 (no states): see fm_join_groups.
+// once they are spent.  Outputs leave straight from the accumulators (fm_each_octet).  GRP = 2 and HALF = 1
+// (no states): see fm_join_groups, fm_join_halves.
 // ------------------------------------------------------------------------------
 // QF = 1 (forward of an order-2 problem without states, _Float16): the weights in their completed-square
 // form (see TileMath<fm_half>::wq); the host picks it when a2 is of ordinary size.
-template <typename TIO, typename E, int DH, int QT, int OWN, int QF = 0, int GRP = 1>
+template <typename TIO, typename E, int DH, int QT, int OWN, int QF = 0, int GRP = 1, int HALF = 0>
 FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_THREADS * GRP, (TokCfg<E, DH, QT>::OCC_PV)) k_pv(TokArgs<TIO, E> A) {
+  static_assert(!HALF || (GRP == 1 && QT == 1 && OWN == FM_OWN_Q && sizeof(E) == 2), "blocks of 64: forward without states, one tile per wavefront");
   static_assert(GRP == 1 || (QT == 1 && OWN == FM_OWN_Q && sizeof(E) == 2 && TokCfg<E, DH, QT>::JOIN <= 2 * TokCfg<E, DH, QT>::GRP_PV),
                 "two groups: forward without states, one tile per wavefront");
   static_assert(!QF || (QT == 1 && OWN == FM_OWN_Q && sizeof(E) == 2), "completed-square weights: forward, one tile per wavefront");
@@ -311,15 +333,15 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_THREADS * GRP, (TokCfg<E, DH, QT>::OCC_PV)) 
   typedef Mma<E> M;
   typedef TileMath<E> TM;
   typedef typename M::frag frag;
-  constexpr int NT = C::NT, NKS = C::NKS, QW = C::QW, PQ = C::PQ, KT = C::KT_PV, PV = C::PV_PV;
-  constexpr int STAGE = C::PV_STAGE;
+  constexpr int NT = C::NT, NKS = C::NKS, QW = HALF ? 64 : C::QW, PQ = C::PQ, KT = HALF ? 64 : C::KT_PV, PV = C::PV_PV;
+  constexpr int STAGE = HALF ? C::HALF_STAGE : C::PV_STAGE;
   FM_DYN_SMEM(smem);
   const int grp = GRP > 1 ? FM_UNIFORM(int(FM_TID_X) / FM_THREADS) : 0;
   float* vecs = reinterpret_cast<float*>(smem + grp * C::GRP_PV);   // va[DH], vb[DH]
   E* Own = reinterpret_cast<E*>(vecs + 2 * DH);       // [QW][PQ]
   E* R = Own + QW * PQ;
   const int tid = int(FM_TID_X) % FM_THREADS, lane = tid & 63, lr = lane & 31, lh = lane >> 5;
-  const int wave = FM_UNIFORM(tid >> 6);
+  const int wave = HALF ? FM_UNIFORM(tid >> 6) & 1 : FM_UNIFORM(tid >> 6), sub = HALF ? FM_UNIFORM(tid >> 7) : 0;   // own tile, share
   TokGeom<OWN, QW, TokArgs<TIO, E> > G;
   G.init(A, C::OCC_PV / GRP);
   const int bh = G.bh, t0 = G.t0;
@@ -336,7 +358,7 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_THREADS * GRP, (TokCfg<E, DH, QT>::OCC_PV)) 
     ro.store(Own, PQ, tid);
   }
   const float* sml = A.small + (int64_t(bh) * A.nslots + G.slot) * StateDims<DH>::SMALL;
-  if (GRP == 1 && G.use_state) {
+  if (GRP == 1 && !HALF && G.use_state) {
     // order 1 has no Z (its coefficient is the order-2 one): only the two vectors are staged
     if (OWN == FM_OWN_Q && A.quad) fm_stage_small<E, DH, QT>(sml, R, vecs, tid, 1.0f);
     else if (tid < 2 * DH) vecs[tid] = sml[DH * DH + tid];
@@ -372,7 +394,7 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_THREADS * GRP, (TokCfg<E, DH, QT>::OCC_PV)) 
 #pragma unroll
   for (int j = 0; j < QT; ++j) gsum[j] = 0.f;
 
-  if (GRP == 1 && G.use_state) {
+  if (GRP == 1 && !HALF && G.use_state) {
     if (OWN == FM_OWN_Q && A.quad) {
       // denominator: g_i += sum_m q_im (va[m] + sum_l Z[m][l] q_il)
 #pragma unroll
@@ -447,7 +469,8 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_THREADS * GRP, (TokCfg<E, DH, QT>::OCC_PV)) 
       // or the end of the sequence (a wavefront-uniform test) zeroes the entries outside its row
       // window before they are used; a tile wholly outside the mask has an empty window.
 #pragma unroll
-      for (int st = 0; st < KT / 32; ++st) {
+      for (int st_ = 0; st_ < (HALF ? 1 : KT / 32); ++st_) {
+        const int st = HALF ? sub : st_;
         if (QT == 1) { FM_SCHED_MFMA_DS(0); }
         fm_f32x16 s[QT];
 #pragma unroll
@@ -465,7 +488,7 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_THREADS * GRP, (TokCfg<E, DH, QT>::OCC_PV)) 
           for (int ss = 0; ss < M::ACC_KSTEPS; ++ss)
             zf[ct][ss] = TR ? M::load_tr(Zt, PQ, 32 * st + 16 * ss, 32 * ct, lane)
                             : M::load_perm(Zt + (32 * ct + lr) * PV + 32 * st, ss, lh);
-        if (st == KT / 32 - 1) {
+        if (HALF || st == KT / 32 - 1) {
           // next stage: registers -> the other buffer (its readers finished before this stage's
           // barrier), then the stage after it: global memory -> registers.  No branch (see k_ds): past the last
           // stage the registers go where nobody reads and the current stage is loaded once more.
@@ -495,6 +518,7 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_THREADS * GRP, (TokCfg<E, DH, QT>::OCC_PV)) 
       buf ^= 1;
     }
     FM_SYNC();
+    if constexpr (HALF != 0) fm_join_halves<NT>(vecs, acc[0], &gsum[0], sub, wave, lane);
     if constexpr (GRP > 1) {
       float* jl = reinterpret_cast<float*>(smem);
       if (grp == 1) jl[16 * NT * FM_THREADS + tid] = gsum[0];
@@ -515,7 +539,7 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_THREADS * GRP, (TokCfg<E, DH, QT>::OCC_PV)) 
       const float ginv = 1.0f / gt;
       if (QF) gt *= 1.0f / (4.0f * A.a2);              // the constant taken out of the weights (o does not see it)
       const int qi = t0 + xrow[j];
-      const bool in = qi < A.n_own && grp == 0;
+      const bool in = qi < A.n_own && grp == 0 && sub == 0;
       if (lh == 0 && in) A.g.base(bh)[int64_t(qi) * A.g.s_n] = gt;
       TIO* orow = ob + int64_t(qi) * A.out.s_n;
       fm_half* rrow = A.out_resid ? A.out_resid + (int64_t(bh) * A.npad_own + qi) * DH : nullptr;
@@ -604,7 +628,7 @@ FM_DEVICE void fm_readout_kv(const E* FM_RESTRICT state2, const E* xs, int xrow,
 // LDS: va, vb | own rows [QW][PQ] | region (Z, then state slabs); the dense stages
 // (stream rows for the scores, stream rows for gh.v, stream transposed, c values)
 // lie over the own rows and the region once they are spent; outputs leave straight from the accumulators.
-// GRP = 2 (no states): see fm_join_groups.
+// GRP = 2 and HALF = 1 (no states): see fm_join_groups, fm_join_halves.
 // DV = 1 (own = keys, sequences of one segment): the same pass also forms dV from the
 // score tiles it already has, P = f(S), dV^T += gh^T P, which saves the four score
 // products per tile that a separate k_pv launch would repeat.
@@ -614,17 +638,18 @@ FM_DEVICE void fm_readout_kv(const E* FM_RESTRICT state2, const E* xs, int xrow,
 // STR = 1 (own = queries, _Float16, two tiles per wavefront): the prefix state is the forward's own layout and is
 // read out transposed (see fm_readout, TRA); the fragments of the dense tiles are fetched behind that readout, so that
 // the kernel holds 64 registers fewer across it.
-template <typename TIO, typename E, int DH, int QT, int OWN, int DV, int PREP, int QF = 0, int STR = 0, int GRP = 1>
-FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_THREADS * GRP, (DV ? TokCfg<E, DH, QT>::OCC_DV : TokCfg<E, DH, QT>::OCC_DS)) k_ds(TokArgs<TIO, E> A) {
+template <typename TIO, typename E, int DH, int QT, int OWN, int DV, int PREP, int QF = 0, int STR = 0, int GRP = 1, int HALF = 0>
+FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_THREADS * GRP, (DV ? TokCfg<E, DH, QT>::OCC_DV : HALF ? TokCfg<E, DH, QT>::OCC_DS_HALF : TokCfg<E, DH, QT>::OCC_DS)) k_ds(TokArgs<TIO, E> A) {
   static_assert(GRP == 1 || (QT == 1 && sizeof(E) == 2 && !STR && (DV ? 2 : 1) * TokCfg<E, DH, QT>::JOIN <= 2 * (DV ? TokCfg<E, DH, QT>::GRP_DV : TokCfg<E, DH, QT>::GRP_DS)),
                 "two groups: no states, one tile per wavefront");
+  static_assert(!HALF || (GRP == 1 && QT == 1 && sizeof(E) == 2 && !STR), "blocks of 64: no states, one tile per wavefront");
   static_assert(!STR || (OWN == FM_OWN_Q && sizeof(E) == 2 && !PREP && !QF && !DV), "the transposed readout is dQ's, on _Float16");
   static_assert(!QF || (QT == 1 && sizeof(E) == 2 && (DV != 0 || OWN == FM_OWN_Q)), "completed-square weights: dQ, or dK with dV, one tile per wavefront");
   typedef TokCfg<E, DH, QT> C;
   typedef Mma<E> M;
   typedef TileMath<E> TM;
   typedef typename M::frag frag;
-  constexpr int NT = C::NT, NKS = C::NKS, QW = C::QW, PQ = C::PQ;
+  constexpr int NT = C::NT, NKS = C::NKS, QW = HALF ? 64 : C::QW, PQ = C::PQ;
   constexpr int KT = DV ? C::KT_DV : C::KT_DS, PV = DV ? C::PV_DV : C::PV_DS;
   constexpr int NBUF = C::DS_NBUF;
   constexpr int STAGE = DV ? C::DV_STAGE : C::DS_STAGE;
@@ -638,9 +663,9 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_THREADS * GRP, (DV ? TokCfg<E, DH, QT>::OCC_
   E* Own = reinterpret_cast<E*>(vecs + 2 * DH);       // [QW][PQ]
   E* R = Own + QW * PQ;
   const int tid = int(FM_TID_X) % FM_THREADS, lane = tid & 63, lr = lane & 31, lh = lane >> 5;
-  const int wave = FM_UNIFORM(tid >> 6);
+  const int wave = HALF ? FM_UNIFORM(tid >> 6) & 1 : FM_UNIFORM(tid >> 6), sub = HALF ? FM_UNIFORM(tid >> 7) : 0;   // see fm_join_halves
   TokGeom<OWN, QW, TokArgs<TIO, E> > G;
-  G.init(A, DV ? (C::OCC_DV + GRP - 1) / GRP : (C::OCC_DS + GRP - 1) / GRP);
+  G.init(A, ((DV ? C::OCC_DV : HALF ? C::OCC_DS_HALF : C::OCC_DS) + GRP - 1) / GRP);
   const int bh = G.bh, t0 = G.t0;
   const bool causal = A.causal != 0;
   const float gsc = fm_grad_scale(A.gpart ? A.gpart + int64_t(bh) * A.gnblk : nullptr, A.gnblk, lane);
@@ -706,7 +731,7 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_THREADS * GRP, (DV ? TokCfg<E, DH, QT>::OCC_
     ro.load(A.own_r + (int64_t(bh) * A.npad_own + t0) * DH, DH, tid);
     ro.store(Own, PQ, tid);
   }
-  if (GRP == 1 && G.use_state) {
+  if (GRP == 1 && !HALF && G.use_state) {
     const float* sml = A.small + (int64_t(bh) * A.nslots + G.slot) * StateDims<DH>::SMALL;
     if (A.quad) fm_stage_small<E, DH, QT>(sml, R, vecs, tid, A.zscale);
     else if (tid < 2 * DH) vecs[tid] = sml[DH * DH + tid];   // order 1 has no Z
@@ -772,7 +797,7 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_THREADS * GRP, (DV ? TokCfg<E, DH, QT>::OCC_
 #pragma unroll
     for (int mt = 0; mt < NT; ++mt) av[j][mt] = fm_zero16();
 
-  if (GRP == 1 && G.use_state) {
+  if (GRP == 1 && !HALF && G.use_state) {
     // - c * (va[m] + sum_l Z[m][l] own_l)   (c = c_i for own = queries; folded into Z and va for own = keys)
 #pragma unroll
     for (int j = 0; j < QT; ++j)
@@ -895,7 +920,8 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_THREADS * GRP, (DV ? TokCfg<E, DH, QT>::OCC_
       // One code path for every tile (see k_pv).  The score fragments and the transposed fragments
       // serve all own tiles of the wavefront; gh.v is formed per own tile.
 #pragma unroll
-      for (int st = 0; st < KT / 32; ++st) {
+      for (int st_ = 0; st_ < (HALF ? 1 : KT / 32); ++st_) {
+        const int st = HALF ? sub : st_;
         if (QT == 1) { FM_SCHED_MFMA_DS(DV ? 0 : 1); }   // two tiles per wavefront: measured slower with it
         fm_f32x16 s[QT];
 #pragma unroll
@@ -948,7 +974,7 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_THREADS * GRP, (DV ? TokCfg<E, DH, QT>::OCC_
             zf[mt][ss] = TR ? M::load_tr(Xs, PQ, 32 * st + 16 * ss, 32 * mt, lane)
                             : M::load_perm(Zt + (32 * mt + lr) * PV + 32 * st, ss, lh);
         }
-        if (NBUF == 2 && st == KT / 32 - 1) {
+        if (NBUF == 2 && (HALF || st == KT / 32 - 1)) {
           // the next stage's tiles into the other buffer and the loads of the stage after it, without a branch: past
           // the last stage the registers are stored where nobody reads and the current stage is loaded once more
           const int sn = s0 + s_step, sf = more(sn) && more(sn + s_step) ? sn + s_step : s0;
@@ -1004,11 +1030,15 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(FM_THREADS * GRP, (DV ? TokCfg<E, DH, QT>::OCC_
     }
     if (NBUF == 2) FM_SYNC();
   }
+  if constexpr (HALF != 0) {
+    fm_join_halves<NT>(vecs, acc[0], nullptr, sub, wave, lane);
+    if (DV) fm_join_halves<NT>(vecs, av[0], nullptr, sub, wave, lane);
+  }
   if constexpr (GRP > 1) {
     fm_join_groups<NT>(reinterpret_cast<float*>(smem), acc[0], grp, tid);
     if (DV) fm_join_groups<NT>(reinterpret_cast<float*>(smem), av[0], grp, tid);
   }
-  const int n_out = grp == 0 ? A.n_own : 0;            // the first group stores
+  const int n_out = grp == 0 && sub == 0 ? A.n_own : 0;   // the first group (share) stores
   {
     // with the normalisation's Jacobian: the stored gradient carries lim / max-norm, and the workgroup's part of
     // B = sum dy . y is left for k_norm_fix (the stored values are fac * dy, the copy's rows sc * y)

@@ -358,6 +358,16 @@ def test_fp32_as_three_products_of_two_planes(lib, bh, nq, nk, d, mask, p):
     assert max(errs) < 2e-6, errs
 
 
+@pytest.mark.parametrize("n", [65, 95, 128, 193, 1025])
+@pytest.mark.parametrize("d,p", [(32, 2), (64, 1), (64, 2), (128, 2)])
+def test_blocks_of_64_own_tokens(lib, d, p, n):
+    """Causal bf16 launches of few workgroups: the two shares of an own tile at the edges of tiles, stages and blocks, odd numbers of
+    batch*heads, and more blocks than dK + dV takes so (140 heads of 193 tokens: 280 of 128)."""
+    for bh in (3, 140) if n == 193 and d == 64 else (3,):
+        print(f"case blocks of 64 bh={bh} n={n} d={d} p={p}", flush=True)
+        check_forward_backward(lib, bh, n, d, torch.bfloat16, DEV, mask=True, p=p, seed=136, saved=True, flags=FLAG_FORCE_DENSE)
+
+
 def test_ranges_of_two_planes(lib):
     check_ranges_of_two_planes(lib, 2, 3100, 64, DEV, seed=134)
     check_infinite_and_largest_values(lib, 1, 1040, 64, torch.float32, DEV, seed=135)
