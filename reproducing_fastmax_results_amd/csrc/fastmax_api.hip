@@ -146,18 +146,19 @@ inline int x3_split(int bh, int n_own, int tokens) {
 // Dense fp32 problems for the kernels of fm_x2.h: not before their error against 64 bits is no larger than that of fm_x3.h's.  Two planes
 // round an operand once more, three products round the sums half as often as six, so sums of enough terms decide it, and
 // sums spread over several wavefronts (sq, sk: x3_split) need more.  Both sides' errors, ratios of o, dq, dk, dv: causal, D = 64, one
-// wavefront per own tile, 512 tokens 1.00 1.01 1.07 1.07, 1024 .91 .92 .93 .91, 4096 .82 .83 .84 .82; two for dK + dV, 777 .94 .91 .99 1.02, 1024
-// .92 .93 .99 .99; two and four, 1536 .95 .96 1.00 1.03, 2048 .92 .90 .96 1.00; four, 2048 1.01 1.02 1.00 1.00, 3000 .96 .95 .95 .95.
-// D = 32: two for dK + dV, 1024 .92 .95 1.04 .99, 1536 .88 .90 .97 .95; four, 3000 .96 1.00 1.01 .96, 4096 .93 .98 .98 .92.  Unmasked: four, 300 keys
-// 1.01 .99 1.00 1.02, 1024 .86 .89 .89 .85; two and four, 512 .85 .87 .95 .94.
+// and two wavefronts per own tile for dQ and dK + dV, 512 tokens .79 .97 1.03 .98, 777 .70 .86 .91 .91; one and one, 1024 .64 .85 .86 .83, 4096
+// .48 .74 .74 .72; two and four, 1024 .83 .96 1.00 1.05, 1536 .75 .94 .98 .97; four, 1536 .93 1.02 1.00 1.03, 2048 .86 .99 .97 .99.  D = 32: one and two,
+// 777 .71 .92 .99 .88; two and four, 2048 .69 .96 1.03 .92, 3000 .63 .88 .98 .89; four, 2048 .86 1.04 1.03 .97, 3000 .79 .99 1.00 .94.  Unmasked: four, 300 keys
+// .88 .98 .99 .99; one, 300 .67 .91 1.00 .93, but the pass over the ranges costs small forwards more than it gains (D = 64, 16 heads of 400
+// keys 21.4, 24.5 us, 8 of 700 23.0, 23.8; D = 32, 8 of 1000 20.8, 23.9, 32 of 700 40, 28).
 inline bool x2_pays(const FastmaxDesc* d, int sq, int sk) {
 #if defined(FM_HOSTSIM)
   if (fm_hostsim_x2) return true;
 #endif
   const int n = d->nq < d->nk ? d->nq : d->nk;
-  if (!d->mask) return n >= (sk == 4 ? 1024 : 512);
-  if (d->d == 32) return n >= (sk == 1 ? 1024 : sk == 2 ? 1536 : 4096);
-  return n >= (sk < 4 ? 1024 : sq < 4 ? 2048 : 3072);
+  if (!d->mask) return n >= 640 && int64_t(d->bh) * d->nq * d->nk * d->d >= int64_t(1) << 28;
+  if (sk < 4) return n >= 768;
+  return n >= (d->d == 32 ? 3000 : sq < 4 ? 1536 : 2048);
 }
 // own tokens of a workgroup there
 inline int x2_rows(int kind, int split, int bh, int n_own) {

@@ -7,8 +7,9 @@
 // bf16 planes, whose exponents fit every number; its sums are rounded twice as often.
 //
 // 4 x 8 heads of 4096 tokens, D = 64, causal, fm_x3.h and here: relative error of o, dq, dk, dv against 64-bit results 3.6e-7, 4.3e-7, 4.3e-7, 3.6e-7
-// and 3.0e-7, 3.6e-7, 3.5e-7, 3.0e-7; forward 349 and 220 us (19 of them k_x2_range), backward 1106 and 665 (10).  A few hundred terms
-// give the sums too few roundings for that (see x2_pays), and such problems stay with fm_x3.h.
+// and 1.7e-7, 3.1e-7, 3.1e-7, 2.6e-7 (the forward has the registers for sums of the small terms apart: 3.0e-7 in one sum); forward 349
+// and 220 us (19 of them k_x2_range), backward 1106 and 665 (10).  A few hundred terms give the sums too few roundings for
+// that (see x2_pays), and such problems stay with fm_x3.h.
 // What bounds these kernels is power: the forward keeps the matrix pipe 60 % busy at 1.9 GHz.  Copying ready-made planes to LDS past the
 // registers, without bank conflicts, took 14 % of its cycles away and gave them back as a clock of 1.75 GHz.
 //
@@ -107,7 +108,8 @@ template <int DH> struct X2Row {
       dp = fm_mfma_f16(y.h, of2.f[ks].h, dp);
     }
   }
-  static FM_DEVICE void accum(fm_f32x16* acc, const fm_half* Y, int tok0, const fm_f32x16& s, int lane) {
+  // small: where the sums of the small terms go (acc itself, or sums of their own: a third of acc's roundings then)
+  static FM_DEVICE void accum(fm_f32x16* acc, fm_f32x16* small, const fm_half* Y, int tok0, const fm_f32x16& s, int lane) {
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const X2 pb = fm_x2_split_acc(s, h);
@@ -115,9 +117,9 @@ template <int DH> struct X2Row {
 #pragma unroll
       for (int ct = 0; ct < NT; ++ct) z[ct] = load_tr(Y, tok0 + 16 * h, 32 * ct, lane);
 #pragma unroll
-      for (int ct = 0; ct < NT; ++ct) acc[ct] = fm_mfma_f16(z[ct].l, pb.h, acc[ct]);
+      for (int ct = 0; ct < NT; ++ct) small[ct] = fm_mfma_f16(z[ct].l, pb.h, small[ct]);
 #pragma unroll
-      for (int ct = 0; ct < NT; ++ct) acc[ct] = fm_mfma_f16(z[ct].h, pb.l, acc[ct]);
+      for (int ct = 0; ct < NT; ++ct) small[ct] = fm_mfma_f16(z[ct].h, pb.l, small[ct]);
 #pragma unroll
       for (int ct = 0; ct < NT; ++ct) acc[ct] = fm_mfma_f16(z[ct].h, pb.h, acc[ct]);
     }
@@ -380,10 +382,10 @@ FM_DEVICE bool fm_x2_fwd(const X2Args& A, fm_half* st, int* bad) {
     fm_x2_set<DH>(of, v, fm_x2_scalb(1.0f, eq));
     cf = fm_x2_coef(A.a0, A.a1, A.a2, A.ew, eq + ek);
   }
-  fm_f32x16 acc[NT];
+  fm_f32x16 acc[NT], small[NT];
 #pragma unroll
-  for (int ct = 0; ct < NT; ++ct) acc[ct] = fm_zero16();
-  float gs = 0.f;
+  for (int ct = 0; ct < NT; ++ct) { acc[ct] = fm_zero16(); small[ct] = fm_zero16(); }
+  X3Sum gsum = {0.f, 0.f};
   int buf = 0;
   sg.store(st, st + KT * PQ, ks_, vs, false, tid);
   sg.load(A.k, A.v, nullptr, bh, KT, A.nk, tid);
@@ -398,9 +400,8 @@ FM_DEVICE bool fm_x2_fwd(const X2Args& A, fm_half* st, int* bad) {
 #pragma unroll
       for (int e = 0; e < 16; ++e) s[e] = cf.a0 + s[e] * (cf.a1 + cf.a2 * s[e]);
       if (fm_tile_edge<FM_OWN_Q>(causal, ss0, lo, A.nk)) { FM_KEEP_BRANCH(); fm_x3_window<FM_OWN_Q>(s, causal, ss0, lo, lr, lh, A.nk); }
-#pragma unroll
-      for (int e = 0; e < 16; ++e) gs += s[e];
-      R::accum(acc, Y, 32 * sub, s, lane);
+      gsum.add(s);
+      R::accum(acc, small, Y, 32 * sub, s, lane);
     }
     buf ^= 1;
     if (s0 + KT < send) {
@@ -408,20 +409,19 @@ FM_DEVICE bool fm_x2_fwd(const X2Args& A, fm_half* st, int* bad) {
       sg.load(A.k, A.v, nullptr, bh, s0 + 2 * KT, A.nk, tid);
     }
   }
+#pragma unroll
+  for (int ct = 0; ct < NT; ++ct) acc[ct] += small[ct];
   float* Os = reinterpret_cast<float*>(st);
-  float* Gs = Os + SPLIT * QW * (DH + 4);              // [SPLIT][QW]
   FM_SYNC();
   fm_x3_put<DH, QW>(acc, Os, sub, 32 * own + lr, lh);
-  gs += fm_shfl_xor(gs, 32);
-  if (lh == 0) Gs[sub * QW + 32 * own + lr] = gs;
+  fm_x3_put_sum<DH, QW>(gsum, Os, sub, 32 * own + lr, lh);
   FM_SYNC();
   for (int c = tid; c < QW * (DH / 8); c += C::NTH) {
     const int r = c / (DH / 8), col = (c % (DH / 8)) * 8, qi = t0 + r;
     if (qi >= A.nq) continue;
-    float v[8], gt = 0.f;
+    float v[8];
     fm_x3_sum8<DH, QW, SPLIT>(Os, r, col, v);
-#pragma unroll
-    for (int s = 0; s < SPLIT; ++s) gt += Gs[s * QW + r];
+    const float gt = fm_x3_sum<DH, QW, SPLIT>(Os, r);
     fm_x3_look(bad, v, gt);
     const float gi = 1.0f / gt;
 #pragma unroll
@@ -520,7 +520,7 @@ FM_DEVICE bool fm_x2_dq(const X2Args& A, fm_half* st, int* bad) {
 #pragma unroll
       for (int e = 0; e < 16; ++e) s[e] = (cf.a1 + cf.a2 * s[e]) * dp[e];
       if (fm_tile_edge<FM_OWN_Q>(causal, ss0, lo, A.nk)) { FM_KEEP_BRANCH(); fm_x3_window<FM_OWN_Q>(s, causal, ss0, lo, lr, lh, A.nk); }
-      R::accum(acc, X, 32 * sub, s, lane);
+      R::accum(acc, acc, X, 32 * sub, s, lane);
     }
     buf ^= 1;
     if (s0 + KT < send) {
@@ -642,8 +642,8 @@ FM_DEVICE bool fm_x2_dkv(const X2Args& A, fm_half* st, int* bad) {
         fm_x3_window<FM_OWN_K>(s, causal, ss0, lo, lr, lh, A.nq);
         fm_x3_window<FM_OWN_K>(dp, causal, ss0, lo, lr, lh, A.nq);
       }
-      R::accum(av, Y, 32 * sub, s, lane);
-      R::accum(acc, X, 32 * sub, dp, lane);
+      R::accum(av, av, Y, 32 * sub, s, lane);
+      R::accum(acc, acc, X, 32 * sub, dp, lane);
     }
     buf ^= 1;
     if (s0 - KT >= sbeg) { put(buf); fetch(s0 - 2 * KT); }

@@ -26,6 +26,8 @@
 // workgroups and wavefronts (see x3_split).
 // What bounds them is the matrix pipe and the vector work beside it: per 32 x 32 tile pair and wavefront (D = 64) the
 // forward issues 48 matrix instructions (1536 cycles) and about 140 vector instructions for the weights and their split.
+// Long fp32 problems whose numbers two _Float16 planes hold are fm_x2.h's; short ones, bf16 tensors computed in fp32, unusual
+// coefficients and the numbers that fm_x2.h refuses are made here.
 #pragma once
 #include "fm_kernels.h"
 #include "fm_tok.h"
@@ -346,6 +348,41 @@ template <int OWN> FM_DEVICE void fm_x3_window(fm_f32x16& p, bool causal, int s0
   for (int e = 0; e < 16; ++e) { const int r = fm_acc_row(e, lh); if (r < wlo || r > whi) p[e] = 0.f; }
 }
 
+// Sum of many weights: a tile's sixteen as a tree, the tiles with the rounding of each addition carried on.  Denominators of 4096 weights are
+// off by 2.3e-8 so, which is the rounding of the result; one weight after the other by 3.9e-7, a tree without the carry by 1.0e-7.
+struct X3Sum {
+  float s, c;
+  FM_DEVICE void add(const fm_f32x16& w) {
+    float t[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) t[i] = w[i] + w[i + 8];
+#pragma unroll
+    for (int n = 4; n > 0; n >>= 1)
+#pragma unroll
+      for (int i = 0; i < n; ++i) t[i] += t[i + n];
+    const float y = t[0] - c, z = s + y;
+    const float r = (z - s) - y;
+    c = fm_absf(z) < 0x1p127f ? r : 0.f;               // a sum past fp32 stays what it is
+    s = z;
+  }
+};
+// The sums of a row's two lanes and SPLIT parts meet in the four floats behind Os's rows, added in 64 bits: what is rounded is g itself.
+template <int DH, int QW> FM_DEVICE void fm_x3_put_sum(const X3Sum& w, float* Os, int sub, int row, int lh) {
+  float* p = Os + (sub * QW + row) * (DH + 4) + DH + 2 * lh;
+  p[0] = w.s; p[1] = w.c;
+}
+template <int DH, int QW, int SPLIT> FM_DEVICE float fm_x3_sum(const float* Os, int row) {
+  double s = 0.0;
+  float c = 0.f;
+#pragma unroll
+  for (int i = 0; i < SPLIT; ++i) {
+    const fm_f32x4 w = *reinterpret_cast<const fm_f32x4*>(Os + (i * QW + row) * (DH + 4) + DH);
+    s += double(w[0]) + double(w[2]);
+    c += w[1] + w[3];
+  }
+  return float(s - double(c));
+}
+
 // Accumulators of all wavefronts -> Os [SPLIT][QW][DH + 4], rows summed over the SPLIT parts by fm_x3_sum8.
 template <int DH, int QW>
 FM_DEVICE void fm_x3_put(const fm_f32x16* acc, float* Os, int sub, int row, int lh) {
@@ -414,7 +451,7 @@ template <int DH, int NW, int SPLIT> struct X3Cfg {
   static constexpr int NTH = 64 * NW, OT = NW / SPLIT, QW = 32 * OT, KT = 32 * SPLIT, PQ = X3Row<DH>::PQ;
   static constexpr int STAGE = 2 * KT * PQ;            // u16 elements of one stage buffer
   static constexpr int NBUF = 2 * STAGE * 2 <= 112 * 1024 ? 2 : 1;
-  static constexpr size_t OS = size_t(SPLIT) * QW * (DH + 4) * 4 + size_t(SPLIT) * QW * 4;
+  static constexpr size_t OS = size_t(SPLIT) * QW * (DH + 4) * 4;
   // kind 0: forward, dQ; 1: dK + dV (own v rows and the stages' c values as well)
   static constexpr size_t lds(int kind) {
     const size_t a = size_t(NBUF) * STAGE * 2 + (kind ? size_t(QW) * PQ * 2 + size_t(NBUF) * KT * 4 : 0);
@@ -460,7 +497,7 @@ FM_DEVICE void fm_x3_fwd(const X3Args<TIO>& A, uint16_t* st, int* bad, const int
   fm_f32x16 acc[NT];
 #pragma unroll
   for (int ct = 0; ct < NT; ++ct) acc[ct] = fm_zero16();
-  float gs = 0.f;
+  X3Sum gsum = {0.f, 0.f};
   constexpr bool TWO = R::PIPE && C::NBUF == 2;
   // Shared own tiles are short problems, bound by their straight code: there the walk starts one stage early, for that stage's
   // store alone, and the code of a store is there once (570 of 3090 instructions; 256 tokens, D = 32, B*H = 2, whole call 8.98 ->
@@ -486,8 +523,7 @@ FM_DEVICE void fm_x3_fwd(const X3Args<TIO>& A, uint16_t* st, int* bad, const int
 #pragma unroll
       for (int e = 0; e < 16; ++e) s[e] = cf.a0 + s[e] * (cf.a1 + cf.a2 * s[e]);
       if (fm_tile_edge<FM_OWN_Q>(causal, ss0, lo, A.nk)) { FM_KEEP_BRANCH(); fm_x3_window<FM_OWN_Q>(s, causal, ss0, lo, lr, lh, A.nk); }
-#pragma unroll
-      for (int e = 0; e < 16; ++e) gs += s[e];
+      gsum.add(s);
       R::accum(acc, Y, 32 * sub, s, lane);
     }
     if (TWO) {
@@ -499,19 +535,16 @@ FM_DEVICE void fm_x3_fwd(const X3Args<TIO>& A, uint16_t* st, int* bad, const int
     } else FM_SYNC();
   }
   float* Os = reinterpret_cast<float*>(st);
-  float* Gs = Os + SPLIT * QW * (DH + 4);              // [SPLIT][QW]
   FM_SYNC();
   fm_x3_put<DH, QW>(acc, Os, sub, 32 * own + lr, lh);
-  gs += fm_shfl_xor(gs, 32);
-  if (lh == 0) Gs[sub * QW + 32 * own + lr] = gs;
+  fm_x3_put_sum<DH, QW>(gsum, Os, sub, 32 * own + lr, lh);
   FM_SYNC();
   for (int c = tid; c < QW * (DH / 8); c += C::NTH) {
     const int r = c / (DH / 8), col = (c % (DH / 8)) * 8, qi = t0 + r;
     if (qi >= A.nq) continue;
-    float v[8], gt = 0.f;
+    float v[8];
     fm_x3_sum8<DH, QW, SPLIT>(Os, r, col, v);
-#pragma unroll
-    for (int s = 0; s < SPLIT; ++s) gt += Gs[s * QW + r];
+    float gt = fm_x3_sum<DH, QW, SPLIT>(Os, r);
     if (R::PIPE) fm_x3_look(bad, v, gt);
     gt *= 1.0f / R::UP;
     const float gi = 1.0f / gt;
