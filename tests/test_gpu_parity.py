@@ -368,6 +368,20 @@ def test_blocks_of_64_own_tokens(lib, d, p, n):
         check_forward_backward(lib, bh, n, d, torch.bfloat16, DEV, mask=True, p=p, seed=136, saved=True, flags=FLAG_FORCE_DENSE)
 
 
+@pytest.mark.parametrize("bh,nq,nk,d,p,dtype", [
+    (2, 1057, 1057, 32, 2, torch.float32), (56, 1100, 1152, 32, 2, torch.float32), (57, 1100, 1152, 32, 2, torch.float32),   # 504 and 513 blocks
+    (14, 77, 1100, 32, 1, torch.float32), (15, 1152, 1060, 32, 1, torch.float32), (1, 4170, 4161, 64, 2, torch.float32),
+    (3, 4700, 4800, 32, 2, torch.bfloat16), (2, 4700, 4800, 32, 2, torch.bfloat16)])                              # 2^26 products and less
+def test_unmasked_fp32_on_tiles_and_states(lib, bh, nq, nk, d, p, dtype):
+    """Long unmasked fp32 problems on dense tiles while those do not fill the chip, on the total of the moments beyond: both sides of the
+    limits, each against float64 by the bar of test_fp32_dense_tiles."""
+    print(f"case unmasked fp32 bh={bh} nq={nq} nk={nk} d={d} p={p} {dtype}", flush=True)
+    flags = FLAG_F32_COMPUTE if dtype is torch.bfloat16 else 0
+    e = check_forward_backward(lib, bh, nq, d, dtype, DEV, mask=False, p=p, nk=nk, seed=137, saved=True, flags=flags)
+    if dtype is torch.float32:
+        assert max(e.values()) < 2e-6, e
+
+
 def test_ranges_of_two_planes(lib):
     check_ranges_of_two_planes(lib, 2, 3100, 64, DEV, seed=134)
     check_infinite_and_largest_values(lib, 1, 1040, 64, torch.float32, DEV, seed=135)
