@@ -182,6 +182,28 @@ inline int x2_rows(int kind, int split, int bh, int n_own) {
   return 256 / split;
 }
 
+// dK + dV of long causal problems on fm_x2.h: two wavefronts to an own tile at least, whose sums are half as long.
+inline int x2_key_split(const FastmaxDesc* d) {
+  const int s = x3_split(d->bh, d->nk, 256);
+  return s == 1 && d->mask && d->nq > 6144 ? 2 : s;
+}
+// Causal problems in fp32 arithmetic that keep dense tiles past the lengths at which _Float16 ones go to states (see make_plan): the state
+// kernels' products are fp32's, a sixth of the rate of fm_x2.h's.  Forward and backward on states and on tiles, microseconds: order 2,
+// D = 64, fp32 tensors, 16 heads of 8192 1419 and 3254, 402 and 1272, 2 of 6200 316 and 865, 96 and 265, 4 of 16000 862 and 1935, 416 and 1365, 2 of 32000
+// 857 and 1902, 788 and 2646; D = 32, 16 of 7000 303 and 716, 206 and 570, 128 of 7000 1813 and 4489, 1311 and 4485, 4 of 12000 191 and 470, 197 and
+// 492.  bf16 tensors (fm_x3.h), D = 64, 16 of 7000 1200 and 2735, 481 and 1578, 3 of 8192 434 and 976, 472 and 914.  The limits are also where the
+// tiles' error against 64 bits is below the states': D = 64, 8192 tokens, o, dq, dk, dv 3.0, 4.7, 4.9, 3.3e-7 and 2.0, 4.0, 3.1, 2.6e-7 (dv 3.5e-7 with one
+// wavefront to an own tile: x2_key_split); a full chip's dq is past it from about 10000 tokens.  Order 1 keeps its 1024: at 1280 tokens the tiles
+// are faster for few heads and for many, not between (24 heads 65 and 153, 84 and 178).
+inline bool tiles_pay_causal(const FastmaxDesc* d) {
+  int ew;
+  const int64_t n = d->nq;
+  if (half_arithmetic(d) || d->p != 2 || d->a2 == 0.0f || d->d > 64) return false;
+  if (d->dtype != FASTMAX_F32) return d->d == 64 && n <= 7168;
+  if (!x2_coefficients(d->a0, d->a1, d->a2, ew)) return false;
+  return d->d == 64 ? n <= 8192 || (n <= 16384 && d->bh * ((n + 127) / 128) < 512) : n <= 7168;
+}
+
 int validate(const FastmaxDesc* d) {
   if (!d) return FASTMAX_ERR_NULL;
   if (d->dtype != FASTMAX_F32 && d->dtype != FASTMAX_BF16) return FASTMAX_ERR_DTYPE;
@@ -247,10 +269,9 @@ int make_plan(const FastmaxDesc* d, Plan& p) {
     // beyond; order 1 (one D x D state per segment): one segment up to 1024 tokens (0.150 against 0.159 ms
     // per step at B*H = 128; at 1536 tokens, B*H = 96: 0.209 against 0.190),
     // 256-token segments beyond.
-    // fp32 arithmetic keeps the same limits: they were not measured for it (its dense tiles, fm_x3.h, run at about a quarter
-    // of the _Float16 rate, its state kernels at fp32's).
+    // fp32 arithmetic: one segment for longer (tiles_pay_causal).
     // Order 1 on _Float16: 128-token segments, so that the backward of a segment is one workgroup's work (k_o1_bwd).
-    const int auto_L = p.quad ? (d->nq > 6144 ? 1024 : p.npad_q) : (d->nq > 1024 ? (p.half ? 128 : 256) : p.npad_q);
+    const int auto_L = tiles_pay_causal(d) ? p.npad_q : p.quad ? (d->nq > 6144 ? 1024 : p.npad_q) : (d->nq > 1024 ? (p.half ? 128 : 256) : p.npad_q);
     int L = d->chunk > 0 ? (d->chunk >= d->nq ? p.npad_q : int(round_up(d->chunk, 256))) : auto_L;
     if (force_dense || L > p.npad_q) L = p.npad_q;
     p.L = L;
@@ -268,7 +289,7 @@ int make_plan(const FastmaxDesc* d, Plan& p) {
   p.x3 = !p.half && !p.use_state && !p.tiny;
   p.x2_ew = 0;
   const bool x2_fits = p.x3 && d->dtype == FASTMAX_F32 && x2_coefficients(p.a0, p.a1, p.a2, p.x2_ew);
-  p.x2 = x2_fits && x2_pays(d, x3_split(d->bh, d->nq, 128), x3_split(d->bh, d->nk, 256));
+  p.x2 = x2_fits && x2_pays(d, x3_split(d->bh, d->nq, 128), x2_key_split(d));
   p.o1 = p.half && p.use_state && !p.quad && d->mask && p.L == FM_O1_SEG && d->nq == d->nk;
   p.rows_build = p.half && p.use_state && !p.quad && d->mask;
   {

@@ -321,6 +321,7 @@ def test_fp32_dense_tiles(lib, d, bh, n):
 @pytest.mark.parametrize("bh,nq,nk,d,mask,p", [
     (64, 1030, 1030, 64, True, 2), (130, 769, 769, 32, True, 1),   # one wavefront per own tile; two and one for dK + dV
     (32, 4000, 4000, 32, True, 2),                                   # forward and dQ in workgroups of eight
+    (18, 7300, 7300, 64, True, 2),                                   # dK + dV by two although the chip is full
     (16, 2050, 2050, 64, True, 2), (3, 3100, 3100, 64, True, 2), (2, 4100, 4100, 32, True, 2),   # tiles shared by two and four
     (1, 1040, 1100, 64, False, 2), (40, 645, 800, 32, False, 1), (70, 1100, 650, 64, False, 2)])
 def test_fp32_as_three_products_of_two_planes(lib, bh, nq, nk, d, mask, p):
@@ -366,6 +367,18 @@ def test_blocks_of_64_own_tokens(lib, d, p, n):
     for bh in (3, 140) if n == 193 and d == 64 else (3,):
         print(f"case blocks of 64 bh={bh} n={n} d={d} p={p}", flush=True)
         check_forward_backward(lib, bh, n, d, torch.bfloat16, DEV, mask=True, p=p, seed=136, saved=True, flags=FLAG_FORCE_DENSE)
+
+
+@pytest.mark.parametrize("bh,n,d,dtype", [
+    (1, 6145, 64, torch.float32), (2, 8193, 64, torch.float32), (9, 8192, 64, torch.float32), (9, 8193, 64, torch.float32),
+    (1, 7168, 32, torch.float32), (1, 7169, 32, torch.float32), (2, 7168, 64, torch.bfloat16), (2, 7169, 64, torch.bfloat16)])
+def test_long_causal_fp32_on_tiles_and_states(lib, bh, n, d, dtype):
+    """Long causal order-2 problems in fp32 arithmetic on both sides of the limits of the dense tiles, against float64."""
+    print(f"case long causal fp32 bh={bh} n={n} d={d} {dtype}", flush=True)
+    flags = FLAG_F32_COMPUTE if dtype is torch.bfloat16 else 0
+    e = check_forward_backward(lib, bh, n, d, dtype, DEV, mask=True, p=2, seed=138, saved=True, flags=flags)
+    if dtype is torch.float32:
+        assert max(e.values()) < 2e-6, e
 
 
 @pytest.mark.parametrize("bh,nq,nk,d,p,dtype", [
