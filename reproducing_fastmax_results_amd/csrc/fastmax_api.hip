@@ -663,8 +663,21 @@ template <typename TIO> X3Args<TIO> x3_args(const FastmaxDesc* d, const Plan& p,
 // Wavefronts of a workgroup (kind 0: forward, 1: dQ, 2: dK + dV).  Two buffers of a stage for own tiles shared by two wavefronts take 102 KB
 // at D = 64, one workgroup per CU: eight wavefronts rather than four then keep each SIMD two.  (Causal
 // forward in four and in eight: 12 heads of 4096 tokens 237, 168 us, 40 of 1024 64, 46, 64 of 512 36, 27, 100 of 300 25.6, 28.7.)
-inline int x3_waves(int kind, int dh, int split, int n_str) { return kind == 2 || (split == 2 && dh == 64 && n_str >= 512) ? 8 : 4; }
-inline int x3_rows(int kind, int dh, int split, int n_str) { return 32 * x3_waves(kind, dh, split, n_str) / split; }   // own tokens of a workgroup
+// Own tiles shared by four leave one workgroup per CU too, and one of four wavefronts is one tile: with more tiles than CUs the rest are a
+// second round, in eight (two tiles) none is.  Causal, the light tiles of a head fit behind the heavy ones of others, the better the
+// longer the heads are: hence the 4.  Forward and backward in four and in eight, causal: 24 heads of 640 tokens (480
+// tiles) 32.9 and 74.5, 22.5 and 63.2 us, 15 of 777 (375) 28.4 and 78.6, 26.0 and 76.8, 24 of 400 (312) 21.1 and 53.5, 21.1 and 50.8, 12 of 1030 (396)
+// 33.0 and 93.4, 31.0 and 92.7; 11 of 777 (275) 25.5 and 72.7, 25.3 and 76.0, 9 of 1300 (369) 36.6 and 106, 36.9 and 111; unmasked, 17 of 500 (272) 32.9 and 70.9,
+// 21.1 and 56.6.
+inline int x3_waves(int kind, int dh, int split, int n_str, int n_own, int bh, bool causal) {
+  if (kind == 2) return 8;
+  if (dh != 64 || split == 1) return 4;
+  if (split == 2) return n_str >= 512 ? 8 : 4;
+  return (bh - (causal ? 4 : 0)) * ((n_own + 31) / 32) > 256 ? 8 : 4;
+}
+inline int x3_rows(int kind, int dh, int split, int n_str, int n_own, int bh, bool causal) {    // own tokens of a workgroup
+  return 32 * x3_waves(kind, dh, split, n_str, n_own, bh, causal) / split;
+}
 template <typename TIO, int DH, int KIND, int SPLIT, int NW>
 int launch_x3_cfg(const X3Args<TIO>& a, int n_own, int bh, fm_stream_t stream) {
   typedef X3Cfg<DH, NW, SPLIT> C;
@@ -687,10 +700,11 @@ template <typename TIO, int DH, int KIND>
 int launch_x3(const X3Args<TIO>& a, int split, int n_own, int n_str, int bh, fm_stream_t stream) {
   constexpr int NW = KIND == 2 ? 8 : 4;
   if (split == 1) return launch_x3_cfg<TIO, DH, KIND, 1, NW>(a, n_own, bh, stream);
-  if (split == 4) return launch_x3_cfg<TIO, DH, KIND, 4, NW>(a, n_own, bh, stream);
   if constexpr (KIND < 2 && DH == 64) {
-    if (x3_waves(KIND, DH, split, n_str) == 8) return launch_x3_cfg<TIO, DH, KIND, 2, 8>(a, n_own, bh, stream);
+    if (x3_waves(KIND, DH, split, n_str, n_own, bh, a.causal) == 8)
+      return split == 2 ? launch_x3_cfg<TIO, DH, KIND, 2, 8>(a, n_own, bh, stream) : launch_x3_cfg<TIO, DH, KIND, 4, 8>(a, n_own, bh, stream);
   }
+  if (split == 4) return launch_x3_cfg<TIO, DH, KIND, 4, NW>(a, n_own, bh, stream);
   return launch_x3_cfg<TIO, DH, KIND, 2, NW>(a, n_own, bh, stream);
 }
 

@@ -369,6 +369,19 @@ def test_blocks_of_64_own_tokens(lib, d, p, n):
         check_forward_backward(lib, bh, n, d, torch.bfloat16, DEV, mask=True, p=p, seed=136, saved=True, flags=FLAG_FORCE_DENSE)
 
 
+@pytest.mark.parametrize("bh,nq,nk,mask", [
+    (90, 65, 65, True), (30, 290, 290, True), (24, 639, 639, True), (24, 672, 672, True), (12, 1030, 1030, True),   # 258 .. 420 tiles beside four heads'
+    (87, 66, 70, False), (17, 500, 129, False)])                                                 # 261, 272
+def test_fp32_own_tiles_of_four_in_workgroups_of_eight(lib, bh, nq, nk, mask):
+    """Two own tiles, each shared by four wavefronts, to a workgroup: one, two and odd numbers of tiles per head; with the Jacobian's
+    partial sums, whose number follows the workgroups."""
+    print(f"case tiles of four, eight wavefronts bh={bh} nq={nq} nk={nk} mask={mask}", flush=True)
+    e = check_forward_backward(lib, bh, nq, 64, torch.float32, DEV, mask=mask, p=2, nk=nk, seed=139, saved=True)
+    assert max(e.values()) < 2e-6, e
+    if nq == nk:
+        check_norm_fold(lib, bh, nq, 64, torch.float32, DEV, mask=mask, p=2, seed=140)
+
+
 @pytest.mark.parametrize("bh,n,d,dtype", [
     (1, 6145, 64, torch.float32), (2, 8193, 64, torch.float32), (9, 8192, 64, torch.float32), (9, 8193, 64, torch.float32),
     (1, 7168, 32, torch.float32), (1, 7169, 32, torch.float32), (2, 7168, 64, torch.bfloat16), (2, 7169, 64, torch.bfloat16)])
