@@ -36,8 +36,8 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 if ROOT not in sys.path:
     sys.path.insert(0, ROOT)
 
-# MI355X dense matrix peaks (published); an fp32 product of the dense tiles is six bf16 ones
-PEAK_TFLOPS = {"bf16": 2500.0, "f32": 2500.0 / 6}
+# MI355X dense matrix peaks (published); an fp32 product of long dense tiles is three _Float16 ones
+PEAK_TFLOPS = {"bf16": 2500.0, "f32": 2500.0 / 3}
 PEAK_HBM_GBS = 8000.0
 
 # HBM bytes per launch of the dominant kernel, from rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE runs of this file

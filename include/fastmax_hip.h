@@ -41,7 +41,7 @@ enum {
                                         forward_bytes grows accordingly */
   FASTMAX_FLAG_F32_COMPUTE = 8,      /* bf16 tensors: do all arithmetic in fp32 (matrix products included)
                                         instead of _Float16; for inputs outside the range stated below.
-                                        A training step takes four to five times as long; workspace sizes differ.
+                                        A training step takes about four times as long; workspace sizes differ.
                                         Ignored for fp32 tensors. */
   FASTMAX_FLAG_NORM_SELF = 16,       /* nq, nk <= 64 (and not causal with nk > nq): q and k are max-normalised with norm.lim and
                                         the kernels find the norms themselves; norm.q_keys and norm.k_keys are null */
@@ -64,14 +64,16 @@ enum {
  * backward rescales dO / g per batch*head to the _Float16 range and back).  The 2e-2 accuracy of this
  * path also rests on weights f(s) that add up without cancelling, as the Taylor weights do (f > 0):
  * with a0 <= 0 the library computes bf16 tensors in fp32 on its own, as if the flag were set.
- * fp32 tensors: every magnitude of fp32, infinities and NaN included, with fp32's 24 bits throughout.  (Dense tiles form fp32
- * products from three bf16 parts of each factor; a workgroup that meets an entry beyond about 1e31 or a sum beyond 1e23, which the
- * parts cannot hold, makes its rows a second time with fp32 products.)
+ * fp32 tensors: every magnitude of fp32, infinities and NaN included, at fp32's accuracy throughout.  (Dense tiles form fp32
+ * products from three bf16 parts of each factor, all 24 bits; a workgroup that meets an entry beyond about 1e31 or a sum beyond 1e23,
+ * which the parts cannot hold, makes its rows a second time with fp32 products.  Long problems, whose sums round more than their
+ * operands, form them from two _Float16 parts, about 23 bits, where the largest entries of the tensors' rows and columns lie
+ * within 2^13 of each other; a workgroup whose tensors do not keep to that makes its rows from the three parts.)
  *
  * Bits.  A call gives the same bits on every run.  The order in which a sum is added depends on how many workgroups the launch has,
  * so a batch*head slice can come out with other roundings when nq, nk or the number of slices beside it changes: one-segment
  * problems of bf16 tensors between launches of up to 128, 256 or 512 workgroups and larger ones, dense fp32 tiles
- * at 256 and 512, a few queries with the number of parts of the keys. */
+ * at 256 and 512 (and where three parts or two are taken, or states or tiles), a few queries with the number of parts of the keys. */
 
 /* Where slice i of the batch*head axis, token t, feature f of a tensor lives:
  *   heads <= 1:  i * bh + t * n + f
