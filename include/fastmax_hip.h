@@ -41,7 +41,7 @@ enum {
                                         forward_bytes grows accordingly */
   FASTMAX_FLAG_F32_COMPUTE = 8,      /* bf16 tensors: do all arithmetic in fp32 (matrix products included)
                                         instead of _Float16; for inputs outside the range stated below.
-                                        A training step takes about four times as long; workspace sizes differ.
+                                        A training step takes four to five times as long; workspace sizes differ.
                                         Ignored for fp32 tensors. */
   FASTMAX_FLAG_NORM_SELF = 16,       /* nq, nk <= 64 (and not causal with nk > nq): q and k are max-normalised with norm.lim and
                                         the kernels find the norms themselves; norm.q_keys and norm.k_keys are null */
