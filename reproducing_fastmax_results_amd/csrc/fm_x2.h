@@ -580,11 +580,12 @@ FM_DEVICE bool fm_x2_dkv(const X2Args& A, fm_half* st, int* bad) {
   fetch(s_last);
   const float kf = fm_norm_factor(A.k_fold, bh, lane), qf = A.sc * fm_norm_factor(A.q_fold, bh, lane);
   const X2Max xq = fm_x2_join(A.mq + int64_t(bh) * A.nbq, 0, A.nbq, lane), xv = fm_x2_join(A.mv + int64_t(bh) * A.nbk, 0, A.nbk, lane);
-  // gh: of the queries that the block's keys see; what the last key sees has to be within the range of it
+  // gh: of the queries that the block's keys see; what the last key sees has to be within the range of it: the blocks behind its own, or,
+  // where those are zero, the last row of its own that is not (the row before that it may not see)
   const int tl = (t0 + QW < A.nk ? t0 + QW : A.nk) - 1;
   const int b0 = causal ? fm_x2_block(t0, A.nbq) : 0, b1 = causal ? fm_x2_block(tl, A.nbq) : 0;
   const X2Max xg = fm_x2_join(A.mg + int64_t(bh) * A.nbq, b0, A.nbq, lane), xl = fm_x2_join(A.mg + int64_t(bh) * A.nbq, b1 + 1, A.nbq, lane);
-  const float seen = fm_fmaxf(xl.mx, A.tg[int64_t(bh) * A.nbq + b1]);
+  const float seen = xl.mx > 0.f ? xl.mx : A.tg[int64_t(bh) * A.nbq + b1];
   bool ok = xq.ok && xv.ok && !(causal && seen > 0.f && seen * 2048.0f < xg.mx);
   const int eq = FM_UNIFORM(fm_x2_exp(xq.mx * qf, ok)), ev = FM_UNIFORM(fm_x2_exp(xv.mx, ok)), eg = FM_UNIFORM(fm_x2_exp(xg.mx, ok));
   if (!ok) return true;

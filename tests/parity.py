@@ -288,3 +288,21 @@ def check_ranges_of_two_planes(lib, bh, n, d, device, *, mask=True, seed=0, tol=
         if which == "last rows of dO" and mask: parts["dv there"] = (dv[:, -40:], ref[4][:, -40:])
         for m, (x, r) in parts.items():
             assert rel_err(x, r) < tol, f"{which}: {m} {rel_err(x, r):.3e}"
+
+
+def check_keys_that_see_small_gradients(lib, bh, n, d, device, *, end, zeros, seed=0, tol=2e-6):
+    """fp32, causal: dO is zero in the `zeros` rows up to `end` (tokens left out of a loss) and far smaller behind them, so that the keys of
+    those rows see small gradients alone.  Their dk and dv are held to the bar by themselves."""
+    tau = 8.0 * math.sqrt(d)
+    kw = dict(mask=True, inv_tau=1.0 / tau, p=2)
+    rows = slice(end - zeros, end)
+    for scale in (1e-5, 1e-9):
+        q, k, v, go = make_inputs(bh, n, n, d, torch.float32, device, seed)
+        go[:, rows] = 0.0
+        go[:, end:] *= scale
+        o, g = lib.forward(q, k, v, **kw)
+        grads = lib.backward(q, k, v, o, g, go, **kw)
+        ref = oracle_all(q, k, v, go, mask=True, tau=tau, p=2)[2:]
+        errs = {m: rel_err(x, r) for m, x, r in zip(("dq", "dk", "dv"), grads, ref)}
+        errs.update({m + " there": rel_err(x[:, rows], r[:, rows]) for m, x, r in zip(("dk", "dv"), grads[1:], ref[1:])})
+        assert max(errs.values()) < tol, f"dO x {scale:g} behind token {end}: {errs}"

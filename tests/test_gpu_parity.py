@@ -4,7 +4,7 @@ bf16-rounded inputs)."""
 import pytest
 import torch
 
-from tests.parity import (check_ranges_of_two_planes, check_infinite_and_largest_values, check_prompt_at_the_ends_of_the_range, check_tiny_values, check_upstream_gradients_at_the_ends_of_the_range, check_batch_head_strides, check_decode, check_forward, check_forward_backward,
+from tests.parity import (check_keys_that_see_small_gradients, check_ranges_of_two_planes, check_infinite_and_largest_values, check_prompt_at_the_ends_of_the_range, check_tiny_values, check_upstream_gradients_at_the_ends_of_the_range, check_batch_head_strides, check_decode, check_forward, check_forward_backward,
                           check_norm_fold, make_inputs)
 from reproducing_fastmax_results_amd._capi import FLAG_F32_COMPUTE, FLAG_FORCE_DENSE, FLAG_FORCE_MOMENTS, FLAG_NORM_SELF
 
@@ -411,6 +411,13 @@ def test_unmasked_fp32_on_tiles_and_states(lib, bh, nq, nk, d, p, dtype):
 def test_ranges_of_two_planes(lib):
     check_ranges_of_two_planes(lib, 2, 3100, 64, DEV, seed=134)
     check_infinite_and_largest_values(lib, 1, 1040, 64, torch.float32, DEV, seed=135)
+
+
+@pytest.mark.parametrize("bh,n,d,end", [(128, 1030, 64, 512), (32, 1540, 64, 128), (2, 2100, 64, 1984), (2, 3100, 32, 64)])
+def test_keys_that_see_small_gradients(lib, bh, n, d, end):
+    """dK + dV of fm_x2.h with blocks of 256, 128 and 64 own keys."""
+    print(f"case keys that see small gradients bh={bh} n={n} d={d} end={end}", flush=True)
+    check_keys_that_see_small_gradients(lib, bh, n, d, DEV, end=end, zeros=9, seed=141)
 
 
 @pytest.mark.parametrize("d", [32, 64])

@@ -16,7 +16,7 @@ import pytest
 import torch
 
 from reproducing_fastmax_results_amd import _capi
-from tests.parity import (TOL, check_ranges_of_two_planes, check_upstream_gradients_at_the_ends_of_the_range, check_infinite_and_largest_values, check_tiny_values, check_batch_head_strides, check_decode, check_norm_fold, check_prompt_at_the_ends_of_the_range, check_forward, check_forward_backward, make_inputs, oracle_all,
+from tests.parity import (TOL, check_keys_that_see_small_gradients, check_ranges_of_two_planes, check_upstream_gradients_at_the_ends_of_the_range, check_infinite_and_largest_values, check_tiny_values, check_batch_head_strides, check_decode, check_norm_fold, check_prompt_at_the_ends_of_the_range, check_forward, check_forward_backward, make_inputs, oracle_all,
                           rel_err)
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -466,3 +466,10 @@ def test_fp32_as_three_products_of_two_planes(sim, two_planes, split):
         check_infinite_and_largest_values(sim, 1, 66, 32, f, "cpu", seed=75)
         check_tiny_values(sim, 1, 66, 32, f, "cpu", tol=2e-6, seed=76)
         check_forward_backward(sim, 1, 66, 32, f, "cpu", mask=True, p=2, seed=77, scale=30.0)    # weights beyond 65504
+
+
+@pytest.mark.parametrize("split,n,end,zeros", [(1, 322, 256, 6), (2, 194, 128, 1), (4, 130, 64, 1)])
+def test_two_planes_keys_that_see_small_gradients(sim, two_planes, split, n, end, zeros):
+    """The last keys of a workgroup's block see none of the block's large gradients."""
+    two_planes(split)
+    check_keys_that_see_small_gradients(sim, 1, n, 32, "cpu", end=end, zeros=zeros, seed=78)
