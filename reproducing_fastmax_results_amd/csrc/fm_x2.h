@@ -246,8 +246,14 @@ FM_DEVICE float fm_x2_scalb(float x, int e) {
   return __builtin_amdgcn_ldexpf(x, e);
 #endif
 }
-// Own rows that only form scores: no more than leaves the coefficients their range (a smaller score has no bits beside a0).
-FM_DEVICE int fm_x2_score_exp(int e, int stream) { return e + stream > 56 ? 56 - stream : e; }
+// Own rows that only form scores: no more than leaves the coefficients their range (a smaller score has no bits beside a0).  A row that has no
+// exponent is a workgroup for fm_x3.h, but for one so small that its scores are (64 products with numbers below 2^(15 - stream): 2^-60).
+FM_DEVICE int fm_x2_row_exp(float m, int stream, int* bad) {
+  bool ok = true;
+  const int e = fm_x2_exp(m, ok);
+  if (!ok && (m > 1.0f || stream < -18)) *bad = 1;     // (looked at behind the stores)
+  return e + stream > 56 ? 56 - stream : e;
+}
 
 struct X2Args : X3Args<float> {
   const float *mq, *mk, *mv, *mg, *tg;  // partial maxima, and gh's tails: see k_x2_range
@@ -377,8 +383,7 @@ FM_DEVICE bool fm_x2_fwd(const X2Args& A, fm_half* st, int* bad) {
     float v[DH / 16][8];
     const bool in = lo + lr < A.nq;
     fm_x2_own<DH>(A.q, bh, in ? lo + lr : A.nq - 1, in, lh, qs, v);
-    bool fine = true;
-    const int eq = fm_x2_score_exp(fm_x2_exp(fm_x2_largest<DH>(v), fine), ek);
+    const int eq = fm_x2_row_exp(fm_x2_largest<DH>(v), ek, bad);
     fm_x2_set<DH>(of, v, fm_x2_scalb(1.0f, eq));
     cf = fm_x2_coef(A.a0, A.a1, A.a2, A.ew, eq + ek);
   }
@@ -436,6 +441,7 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(64 * NW, 2) k_x2_fwd(X2Args A) {
   FM_DYN_SMEM(smem);
   FM_SHARED int bad;
   if (FM_TID_X == 0) bad = 0;
+  FM_SYNC();                                           // (the flag is set before the first barrier of the walk)
   if (!fm_x2_fwd<DH, SPLIT, NW>(A, reinterpret_cast<fm_half*>(smem), &bad)) FM_END();
   FM_SYNC();
   if (FM_TID_X == 0) bad = 0;
@@ -479,8 +485,7 @@ FM_DEVICE bool fm_x2_dq(const X2Args& A, fm_half* st, int* bad) {
     const int64_t row = in ? lo + lr : A.nq - 1;
     float v[DH / 16][8];
     fm_x2_own<DH>(A.q, bh, row, in, lh, A.sc * qf, v);
-    bool fine = true;
-    const int eq = fm_x2_score_exp(fm_x2_exp(fm_x2_largest<DH>(v), fine), ek);
+    const int eq = fm_x2_row_exp(fm_x2_largest<DH>(v), ek, bad);
     fm_x2_set<DH>(of, v, fm_x2_scalb(1.0f, eq));
     fm_x2_own<DH>(A.d_o, bh, row, in, lh, in ? 1.0f / A.g.base(bh)[row * A.g.s_n] : 0.f, v);
     const float* po = A.o.base(bh) + row * A.o.s_n + 8 * lh;
@@ -491,9 +496,9 @@ FM_DEVICE bool fm_x2_dq(const X2Args& A, fm_half* st, int* bad) {
 #pragma unroll
       for (int i = 0; i < 8; ++i) cs += v[c][i] * o[i];
     }
-    fine = true;
+    bool fine = true;
     const int eg = fm_x2_exp(fm_x2_largest<DH>(v), fine);
-    if (!fine) *bad = 1;                               // (looked at behind the stores)
+    if (!fine) *bad = 1;
     fm_x2_set<DH>(of2, v, fm_x2_pow(eg));
     cs += fm_shfl_xor(cs, 32);
     if (sub == 0 && lh == 0 && in) A.cv[int64_t(bh) * A.npad_q + row] = cs;
@@ -541,7 +546,7 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(64 * NW, 2) k_x2_dq(X2Args A) {
   FM_DYN_SMEM(smem);
   FM_SHARED int bad;
   if (FM_TID_X == 0) bad = 0;
-  FM_SYNC();                                           // (the flag is set before the first barrier of the walk)
+  FM_SYNC();                                           // (see k_x2_fwd)
   if (!fm_x2_dq<DH, SPLIT, NW>(A, reinterpret_cast<fm_half*>(smem), &bad)) FM_END();
   FM_SYNC();
   if (FM_TID_X == 0) bad = 0;
@@ -602,8 +607,7 @@ FM_DEVICE bool fm_x2_dkv(const X2Args& A, fm_half* st, int* bad) {
     const int64_t row = in ? lo + lr : A.nk - 1;
     float v[DH / 16][8];
     fm_x2_own<DH>(A.k, bh, row, in, lh, A.sc * kf, v);
-    bool fine = true;
-    const int ek = fm_x2_score_exp(fm_x2_exp(fm_x2_largest<DH>(v), fine), eq);
+    const int ek = fm_x2_row_exp(fm_x2_largest<DH>(v), eq, bad);
     fm_x2_set<DH>(of, v, fm_x2_scalb(1.0f, ek));
     fm_x2_own<DH>(A.v, bh, row, in, lh, fm_x2_pow(ev), v);
     fm_x2_set<DH>(of2, v, 1.0f);
@@ -665,6 +669,7 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(512, 2) k_x2_dkv(X2Args A) {
   FM_DYN_SMEM(smem);
   FM_SHARED int bad;
   if (FM_TID_X == 0) bad = 0;
+  FM_SYNC();                                           // (see k_x2_fwd)
   if (!fm_x2_dkv<DH, SPLIT>(A, reinterpret_cast<fm_half*>(smem), &bad)) FM_END();
   FM_SYNC();
   if (FM_TID_X == 0) bad = 0;

@@ -306,3 +306,18 @@ def check_keys_that_see_small_gradients(lib, bh, n, d, device, *, end, zeros, se
         errs = {m: rel_err(x, r) for m, x, r in zip(("dq", "dk", "dv"), grads, ref)}
         errs.update({m + " there": rel_err(x[:, rows], r[:, rows]) for m, x, r in zip(("dk", "dv"), grads[1:], ref[1:])})
         assert max(errs.values()) < tol, f"dO x {scale:g} behind token {end}: {errs}"
+
+
+def check_small_tensor_against_a_large_one(lib, bh, n, d, device, *, p, seed=0, tol=2e-6, ends=((2e-31, 2e29), (2e29, 2e-31))):
+    """fp32: q near one end of the range and k near the other, so that their scores are ordinary numbers."""
+    kw = dict(mask=True, inv_tau=1.0, p=p, a2=0.5 if p == 2 else 0.0, flags=2)        # FASTMAX_FLAG_FORCE_DENSE
+    for q_scale, k_scale in ends:
+        q, k, v, go = make_inputs(bh, n, n, d, torch.float32, device, seed)
+        q, k = q * q_scale, k * k_scale
+        if p == 1:
+            k, q = k.abs(), q.abs()                    # (weights that add up)
+        o, g = lib.forward(q, k, v, **kw)
+        grads = lib.backward(q, k, v, o, g, go, **kw)
+        ref = oracle_all(q, k, v, go, mask=True, tau=1.0, p=p)
+        errs = {m: rel_err(x, r) for m, x, r in zip(("o", "g", "dq", "dk", "dv"), (o, g, *grads), ref)}
+        assert max(errs.values()) < tol, f"q x {q_scale:g}, k x {k_scale:g}, order {p}: {errs}"

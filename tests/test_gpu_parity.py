@@ -4,7 +4,7 @@ bf16-rounded inputs)."""
 import pytest
 import torch
 
-from tests.parity import (check_keys_that_see_small_gradients, check_ranges_of_two_planes, check_infinite_and_largest_values, check_prompt_at_the_ends_of_the_range, check_tiny_values, check_upstream_gradients_at_the_ends_of_the_range, check_batch_head_strides, check_decode, check_forward, check_forward_backward,
+from tests.parity import (check_small_tensor_against_a_large_one, check_keys_that_see_small_gradients, check_ranges_of_two_planes, check_infinite_and_largest_values, check_prompt_at_the_ends_of_the_range, check_tiny_values, check_upstream_gradients_at_the_ends_of_the_range, check_batch_head_strides, check_decode, check_forward, check_forward_backward,
                           check_norm_fold, make_inputs)
 from reproducing_fastmax_results_amd._capi import FLAG_F32_COMPUTE, FLAG_FORCE_DENSE, FLAG_FORCE_MOMENTS, FLAG_NORM_SELF
 
@@ -418,6 +418,13 @@ def test_keys_that_see_small_gradients(lib, bh, n, d, end):
     """dK + dV of fm_x2.h with blocks of 256, 128 and 64 own keys."""
     print(f"case keys that see small gradients bh={bh} n={n} d={d} end={end}", flush=True)
     check_keys_that_see_small_gradients(lib, bh, n, d, DEV, end=end, zeros=9, seed=141)
+
+
+@pytest.mark.parametrize("p", [1, 2])
+@pytest.mark.parametrize("bh,n,d", [(64, 1030, 64), (2, 3100, 32)])
+def test_two_planes_small_tensor_against_a_large_one(lib, bh, n, d, p):
+    print(f"case small against large bh={bh} n={n} d={d} p={p}", flush=True)
+    check_small_tensor_against_a_large_one(lib, bh, n, d, DEV, p=p, seed=142)
 
 
 @pytest.mark.parametrize("d", [32, 64])

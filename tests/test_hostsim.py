@@ -16,7 +16,7 @@ import pytest
 import torch
 
 from reproducing_fastmax_results_amd import _capi
-from tests.parity import (TOL, check_keys_that_see_small_gradients, check_ranges_of_two_planes, check_upstream_gradients_at_the_ends_of_the_range, check_infinite_and_largest_values, check_tiny_values, check_batch_head_strides, check_decode, check_norm_fold, check_prompt_at_the_ends_of_the_range, check_forward, check_forward_backward, make_inputs, oracle_all,
+from tests.parity import (TOL, check_small_tensor_against_a_large_one, check_keys_that_see_small_gradients, check_ranges_of_two_planes, check_upstream_gradients_at_the_ends_of_the_range, check_infinite_and_largest_values, check_tiny_values, check_batch_head_strides, check_decode, check_norm_fold, check_prompt_at_the_ends_of_the_range, check_forward, check_forward_backward, make_inputs, oracle_all,
                           rel_err)
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -473,3 +473,11 @@ def test_two_planes_keys_that_see_small_gradients(sim, two_planes, split, n, end
     """The last keys of a workgroup's block see none of the block's large gradients."""
     two_planes(split)
     check_keys_that_see_small_gradients(sim, 1, n, 32, "cpu", end=end, zeros=zeros, seed=78)
+
+
+@pytest.mark.parametrize("p", [1, 2])
+@pytest.mark.parametrize("split", [1, 4])
+def test_two_planes_small_tensor_against_a_large_one(sim, two_planes, split, p):
+    """Own rows whose power of two leaves the range: their scores are not zero."""
+    two_planes(split)
+    check_small_tensor_against_a_large_one(sim, 1, 70, 32, "cpu", p=p, seed=79)
