@@ -25,7 +25,7 @@
 // block's largest entry, and a block that is not zero 2^-6 of the tensor's; then the largest entry of every row and every column of
 // a block is at least 2^-13 of the tensor's largest, and is held to 2^-26 of itself.  A workgroup whose tensors do not keep to
 // that, and one with a sum that is not finite (an infinity, a weight beyond 65504), makes its rows as fm_x3.h does (and so, where
-// its sums are not finite either, with fp32 matrix products).
+// its sums are not finite either, or where fm_x3.h's planes would lose a coefficient, with fp32 matrix products).
 #pragma once
 #include "fm_x3.h"
 #include <cmath>
@@ -446,8 +446,10 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(64 * NW, 2) k_x2_fwd(X2Args A) {
   FM_SYNC();
   if (FM_TID_X == 0) bad = 0;
   FM_SYNC();
-  fm_x3_fwd<float, DH, SPLIT, X3Row<DH>, NW>(FM_ARGS_AGAIN(A), reinterpret_cast<uint16_t*>(smem), &bad, FM_TID_X + FM_OPAQUE_ZERO());
-  if (!fm_x3_again(&bad)) FM_END();
+  if (!A.plain) {
+    fm_x3_fwd<float, DH, SPLIT, X3Row<DH>, NW>(FM_ARGS_AGAIN(A), reinterpret_cast<uint16_t*>(smem), &bad, FM_TID_X + FM_OPAQUE_ZERO());
+    if (!fm_x3_again(&bad)) FM_END();
+  }
   fm_x3_fwd<float, DH, SPLIT, F32Row<DH>, NW>(FM_ARGS_AGAIN(A), reinterpret_cast<uint16_t*>(smem), &bad, FM_TID_X + FM_OPAQUE_ZERO());
 }
 
@@ -551,8 +553,10 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(64 * NW, 2) k_x2_dq(X2Args A) {
   FM_SYNC();
   if (FM_TID_X == 0) bad = 0;
   FM_SYNC();
-  fm_x3_dq<float, DH, SPLIT, X3Row<DH>, NW>(FM_ARGS_AGAIN(A), reinterpret_cast<uint16_t*>(smem), &bad, FM_TID_X + FM_OPAQUE_ZERO());
-  if (!fm_x3_again(&bad)) FM_END();
+  if (!A.plain) {
+    fm_x3_dq<float, DH, SPLIT, X3Row<DH>, NW>(FM_ARGS_AGAIN(A), reinterpret_cast<uint16_t*>(smem), &bad, FM_TID_X + FM_OPAQUE_ZERO());
+    if (!fm_x3_again(&bad)) FM_END();
+  }
   fm_x3_dq<float, DH, SPLIT, F32Row<DH>, NW>(FM_ARGS_AGAIN(A), reinterpret_cast<uint16_t*>(smem), &bad, FM_TID_X + FM_OPAQUE_ZERO());
 }
 
@@ -674,7 +678,9 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(512, 2) k_x2_dkv(X2Args A) {
   FM_SYNC();
   if (FM_TID_X == 0) bad = 0;
   FM_SYNC();
-  fm_x3_dkv<float, DH, SPLIT, X3Row<DH>>(FM_ARGS_AGAIN(A), reinterpret_cast<uint16_t*>(smem), &bad, FM_TID_X + FM_OPAQUE_ZERO());
-  if (!fm_x3_again(&bad)) FM_END();
+  if (!A.plain) {
+    fm_x3_dkv<float, DH, SPLIT, X3Row<DH>>(FM_ARGS_AGAIN(A), reinterpret_cast<uint16_t*>(smem), &bad, FM_TID_X + FM_OPAQUE_ZERO());
+    if (!fm_x3_again(&bad)) FM_END();
+  }
   fm_x3_dkv<float, DH, SPLIT, F32Row<DH>>(FM_ARGS_AGAIN(A), reinterpret_cast<uint16_t*>(smem), &bad, FM_TID_X + FM_OPAQUE_ZERO());
 }

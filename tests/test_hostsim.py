@@ -8,6 +8,7 @@ FASTMAX_HOSTSIM_ASAN=1 (minutes of compile and run time, so not by default), und
 AddressSanitizer through a driver of its own (tests/hostsim/asan_driver.cpp).  It is a test build
 only: the package never loads it.  Sizes are tiny because every work-item is a thread.
 """
+import math
 import os
 import shutil
 import subprocess
@@ -481,3 +482,21 @@ def test_two_planes_small_tensor_against_a_large_one(sim, two_planes, split, p):
     """Own rows whose power of two leaves the range: their scores are not zero."""
     two_planes(split)
     check_small_tensor_against_a_large_one(sim, 1, 70, 32, "cpu", p=p, seed=79)
+
+
+@pytest.mark.parametrize("split", [1, 4])
+def test_two_planes_small_coefficient(sim, two_planes, split):
+    """a2 = 1e-20 beside weights that two planes do not hold: three planes would lose the coefficient, so their turn is left out.  (dS is a
+    difference of near numbers here: the errors are held to those of the fp32 products that the call takes without two planes.)"""
+    d, tau, a = 32, 8.0 * math.sqrt(32), (1.0, 1.0, 1e-20)
+    q, k, v, go = make_inputs(1, 70, 70, d, torch.float32, "cpu", 80)
+    q, k = q * 1e11, k * 1e11
+    kw = dict(mask=True, inv_tau=1.0 / tau, p=2, a2=a[2], flags=_capi.FLAG_FORCE_DENSE)
+    ref = oracle_all(q, k, v, go, mask=True, tau=tau, p=2, a=a)
+    errs = {}
+    for planes in (0, split):
+        two_planes(planes)
+        o, g = sim.forward(q, k, v, **kw)
+        grads = sim.backward(q, k, v, o, g, go, **kw)
+        errs[planes] = [rel_err(x, r) for x, r in zip((o, g, *grads), ref)]
+    assert all(x < 2 * y for x, y in zip(errs[split], errs[0])), errs
