@@ -20,8 +20,8 @@
 //   weights      f(s) as it is, times the power of two that brings a0 to [1, 2); dS times 2^-19 (of products of two scaled rows)
 // The powers are taken out of the polynomials' coefficients and of the sums, exactly.
 //
-// Which problems these kernels may take is decided in two places.  x2_coefficients (host): a0 > 0 and the other coefficients of its
-// size.  k_x2_range and its readers, per batch*head: a row or a column of a 64-token block that is not zero reaches 2^-7 of the
+// Which problems these kernels may take is decided in two places.  x2_coefficients (host): a0 > 0, a1 of its
+// size and a2 no larger than that.  k_x2_range and its readers, per batch*head: a row or a column of a 64-token block that is not zero reaches 2^-7 of the
 // block's largest entry, and a block that is not zero 2^-6 of the tensor's; then the largest entry of every row and every column of
 // a block is at least 2^-13 of the tensor's largest, and is held to 2^-26 of itself.  A workgroup whose tensors do not keep to
 // that, and one with a sum that is not finite (an infinity, a weight beyond 65504), makes its rows as fm_x3.h does (and so, where
@@ -270,11 +270,11 @@ FM_DEVICE X3Coef fm_x2_dcoef(float a1, float a2, int ew, int es) {
   const X3Coef c = {0.f, fm_x2_scalb(a1, ew + FM_X2_DS), fm_x2_scalb(2.0f * a2, ew + FM_X2_DS - es)};
   return c;
 }
-// Coefficients that these kernels take; ew as above.
+// Coefficients that these kernels take; ew as above.  (A score too small to be seen beside a0 is the whole of f'(s) where a1 is zero.)
 inline bool x2_coefficients(float a0, float a1, float a2, int& ew) {
   const float b1 = std::fabs(a1), b2 = std::fabs(a2), big = b1 > b2 ? b1 : b2;
   ew = 0;
-  if (!(a0 > 0x1p-40f && a0 < 0x1p40f) || !(big <= 16.0f * a0) || !(big >= a0 * 0.0625f)) return false;
+  if (!(a0 > 0x1p-40f && a0 < 0x1p40f) || !(big <= 16.0f * a0) || !(b1 >= a0 * 0.0625f)) return false;
   int e;
   std::frexp(a0, &e);
   ew = 1 - e;

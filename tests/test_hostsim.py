@@ -500,3 +500,17 @@ def test_two_planes_small_coefficient(sim, two_planes, split):
         grads = sim.backward(q, k, v, o, g, go, **kw)
         errs[planes] = [rel_err(x, r) for x, r in zip((o, g, *grads), ref)]
     assert all(x < 2 * y for x, y in zip(errs[split], errs[0])), errs
+
+
+@pytest.mark.parametrize("a1", [0.0, 1e-6])
+def test_two_planes_scores_are_all_of_the_derivative(sim, two_planes, a1):
+    """Without a1, f'(s) is the score itself, however small."""
+    two_planes(1)
+    d, tau, a = 32, 8.0 * math.sqrt(32), (1.0, a1, 0.5)
+    q, k, v, go = make_inputs(1, 70, 70, d, torch.float32, "cpu", 81)
+    q = q * 1e-7
+    kw = dict(mask=True, inv_tau=1.0 / tau, p=2, a1=a1, flags=_capi.FLAG_FORCE_DENSE)
+    o, g = sim.forward(q, k, v, **kw)
+    grads = sim.backward(q, k, v, o, g, go, **kw)
+    errs = [rel_err(x, r) for x, r in zip((o, g, *grads), oracle_all(q, k, v, go, mask=True, tau=tau, p=2, a=a))]
+    assert max(errs) < 2e-6, errs
