@@ -243,8 +243,9 @@ template <int DH> size_t big_array_bytes(int esz, bool quad, size_t slots) {
   return (slots * size_t(StateDims<DH>::stride(quad)) + (quad ? 0 : size_t(StateDims<DH>::PAD_SLABS) * StateDims<DH>::SLAB)) * esz;
 }
 
-// floats of the ranges of q, k and v (see launch_x2_range)
+// floats of the ranges of q, k and v, and of gh (see launch_x2_range)
 inline size_t x2_keys(const FastmaxDesc* d) { return size_t(d->bh) * (fm_x2_blocks(d->nq) + 2 * fm_x2_blocks(d->nk)); }
+inline size_t x2_gradients(const FastmaxDesc* d) { return size_t(4) * d->bh * fm_x2_blocks(d->nq); }
 
 int make_plan(const FastmaxDesc* d, Plan& p) {
   int st = validate(d);
@@ -348,7 +349,7 @@ int make_plan(const FastmaxDesc* d, Plan& p) {
   p.b_bq = take(jac && d->norm.q_keys ? size_t(d->bh) * ((d->nq + 31) / 32) * 4 : 0);
   p.b_bk = take(jac && d->norm.k_keys ? size_t(d->bh) * ((d->nk + 31) / 32) * 4 : 0);
   p.b_runq = take(runarr); p.b_runqh = take(runharr); p.b_runk = take(runarr); p.b_runkh = take(runharr);
-  p.b_x2r = take(p.x2 ? (x2_keys(d) + size_t(2) * d->bh * fm_x2_blocks(d->nq)) * 4 : 0);
+  p.b_x2r = take(p.x2 ? (x2_keys(d) + x2_gradients(d)) * 4 : 0);
   p.bwd_bytes = off ? off : 256;
   return FASTMAX_OK;
 }
@@ -708,7 +709,7 @@ int launch_x3(const X3Args<TIO>& a, int split, int n_own, int n_str, int bh, fm_
   return launch_x3_cfg<TIO, DH, KIND, 2, NW>(a, n_own, bh, stream);
 }
 
-// Ranges of the tensors that are not null (gh: of d_o / g, its tails behind them; see k_x2_range), in `keys` those of q, k, v; a: where
+// Ranges of the tensors that are not null (gh: of d_o / g, its tails and columns behind them; see k_x2_range), in `keys` those of q, k, v; a: where
 // they lie.
 template <int DH>
 int launch_x2_range(const FastmaxDesc* d, const void* q, const void* k, const void* v, const void* d_o, const float* g, float* keys,
@@ -716,13 +717,14 @@ int launch_x2_range(const FastmaxDesc* d, const void* q, const void* k, const vo
   const int nbq = fm_x2_blocks(d->nq), nbk = fm_x2_blocks(d->nk);
   float *mq = keys, *mk = mq + size_t(d->bh) * nbq, *mv = mk + size_t(d->bh) * nbk;
   float* tail = gh ? gh + size_t(d->bh) * nbq : nullptr;
-  a.mq = mq; a.mk = mk; a.mv = mv; a.mg = gh; a.tg = tail; a.nbq = nbq; a.nbk = nbk;
+  unsigned long long* cols = gh ? reinterpret_cast<unsigned long long*>(gh + size_t(2) * d->bh * nbq) : nullptr;
+  a.mq = mq; a.mk = mk; a.mv = mv; a.mg = gh; a.tg = tail; a.cg = cols; a.nbq = nbq; a.nbk = nbk;
   X2Job j[4];
   int n = 0;
-  if (q) j[n++] = X2Job{cref<float>(q, d->sq), TRef<float>{}, mq, nullptr, d->nq, nbq, 0};
-  if (k) j[n++] = X2Job{cref<float>(k, d->sk), TRef<float>{}, mk, nullptr, d->nk, nbk, 0};
-  if (v) j[n++] = X2Job{cref<float>(v, d->sv), TRef<float>{}, mv, nullptr, d->nk, nbk, 0};
-  if (d_o) j[n++] = X2Job{cref<float>(d_o, d->sdo), fm_ref<float>(const_cast<float*>(g), d->sg), gh, tail, d->nq, nbq, 1};
+  if (q) j[n++] = X2Job{cref<float>(q, d->sq), TRef<float>{}, mq, nullptr, nullptr, d->nq, nbq, 0};
+  if (k) j[n++] = X2Job{cref<float>(k, d->sk), TRef<float>{}, mk, nullptr, nullptr, d->nk, nbk, 0};
+  if (v) j[n++] = X2Job{cref<float>(v, d->sv), TRef<float>{}, mv, nullptr, nullptr, d->nk, nbk, 0};
+  if (d_o) j[n++] = X2Job{cref<float>(d_o, d->sdo), fm_ref<float>(const_cast<float*>(g), d->sg), gh, tail, cols, d->nq, nbq, 1};
   const int jobs = n;
   while (n < 4) { j[n] = j[0]; ++n; }
   ProfScope prof(FM_K_PREP_BWD, stream);

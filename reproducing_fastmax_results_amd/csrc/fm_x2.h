@@ -23,7 +23,8 @@
 // Which problems these kernels may take is decided in two places.  x2_coefficients (host): a0 > 0, a1 of its
 // size and a2 no larger than that.  k_x2_range and its readers, per batch*head: a row or a column of a 64-token block that is not zero reaches 2^-7 of the
 // block's largest entry, and a block that is not zero 2^-6 of the tensor's; then the largest entry of every row and every column of
-// a block is at least 2^-13 of the tensor's largest, and is held to 2^-26 of itself.  A workgroup whose tensors do not keep to
+// a block is at least 2^-13 of the tensor's largest, and is held to 2^-26 of itself.  (gh: whole rows and blocks may be smaller, they
+// add little to sums over rows; a column may not lie in them alone.)  A workgroup whose tensors do not keep to
 // that, and one with a sum that is not finite (an infinity, a weight beyond 65504), makes its rows as fm_x3.h does (and so, where
 // its sums are not finite either, or where fm_x3.h's planes would lose a coefficient, with fp32 matrix products).
 #pragma once
@@ -130,11 +131,12 @@ template <int DH> struct X2Row {
 static constexpr int FM_X2_TOKENS = 64;                // rows of a partial maximum; the last takes the rest (up to 127)
 FM_DEVICE int fm_x2_block(int row, int nblk) { return row / FM_X2_TOKENS < nblk ? row / FM_X2_TOKENS : nblk - 1; }
 inline int fm_x2_blocks(int n) { return n < FM_X2_TOKENS ? 1 : n / FM_X2_TOKENS; }
-struct X2Job { TRef<const float> x; TRef<float> g; float *part, *tail; int n, nblk, divide; };   // part, tail [bh][nblk]
+struct X2Job { TRef<const float> x; TRef<float> g; float *part, *tail; unsigned long long* cols; int n, nblk, divide; };   // [bh][nblk] each
 
 // Largest |x| (divide: |x / g|) of a block of rows, or infinity where the block does not keep to the range (see above).  Where rows are
 // divided their sizes are left out of that (a small row adds little to sums over rows, and its own workgroup scales it by itself), but
 // a key that sees the sequence's end alone must not find it small: tail is the largest entry of the block's last row that is not zero.
+// cols: one bit per column that is not zero (see fm_x2_columns).
 // grid (blocks, bh, jobs), 256 threads.  Reads its tensors once: three of 4 x 8 heads of 4096 x 64 (101 MB).
 template <int DH>
 FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_x2_range(X2Job j0, X2Job j1, X2Job j2, X2Job j3) {
@@ -196,9 +198,11 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_x2_range(X2Job j0, X2Job j1, X2Job j2, X2
   float m = 0.f;
   if (tid < DH) m = fm_fmaxf(fm_fmaxf(cm[0][tid], cm[1][tid]), fm_fmaxf(cm[2][tid], cm[3][tid]));
   float all = m, least = m > 0.f ? m : 0x1p127f;
+  unsigned long long bits = m > 0.f ? 1ull << tid : 0ull;
 #pragma unroll
   for (int s = 1; s < 64; s <<= 1) {
     all = fm_fmaxf(all, fm_shfl_xor(all, s));
+    bits |= fm_shfl_xor_u64(bits, s);
     const float o = fm_shfl_xor(least, s);
     least = o < least ? o : least;
   }
@@ -208,6 +212,7 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_x2_range(X2Job j0, X2Job j1, X2Job j2, X2
       last = wt[w] > last ? wt[w] : last;
     }
     if (J.tail) J.tail[int64_t(bh) * J.nblk + blk] = fm_bits_f32(uint32_t(last));
+    if (J.cols) J.cols[int64_t(bh) * J.nblk + blk] = bits;
     J.part[int64_t(bh) * J.nblk + blk] = least * 128.0f < all ? __builtin_inff() : all;
   }
 }
@@ -229,6 +234,19 @@ FM_DEVICE X2Max fm_x2_join(const float* part, int b0, int nblk, int lane) {
   }
   const X2Max r = {m, !(least * 64.0f < m)};
   return r;
+}
+// Whether every column of blocks b0 .. nblk - 1 that is not zero is of the size of mx (a block near mx has all of them), where the blocks
+// themselves are not.
+FM_DEVICE bool fm_x2_columns(const float* part, const unsigned long long* cols, int b0, int nblk, float mx, int lane) {
+  unsigned long long all = 0;
+  for (int i = b0 + lane; i < nblk; i += 64) all |= cols[i];
+#pragma unroll
+  for (int s = 1; s < 64; s <<= 1) all |= fm_shfl_xor_u64(all, s);
+  unsigned long long one = 0;
+  for (int i = b0 + lane; i < nblk; i += 64) one |= part[i] * 64.0f >= mx && cols[i] == all ? 1 : 0;
+#pragma unroll
+  for (int s = 1; s < 64; s <<= 1) one |= fm_shfl_xor_u64(one, s);
+  return one != 0;
 }
 // Exponent e that brings m to [2^14, 2^15): m 2^e (0 for m = 0); ok cleared where that power or its inverse would leave fp32's
 // normal numbers.
@@ -256,7 +274,8 @@ FM_DEVICE int fm_x2_row_exp(float m, int stream, int* bad) {
 }
 
 struct X2Args : X3Args<float> {
-  const float *mq, *mk, *mv, *mg, *tg;  // partial maxima, and gh's tails: see k_x2_range
+  const float *mq, *mk, *mv, *mg, *tg;  // partial maxima, and gh's tails and columns: see k_x2_range
+  const unsigned long long* cg;
   int nbq, nbk;
   int ew;                               // exponent of the weights' factor (a0 2^ew in [1, 2))
 };
@@ -596,6 +615,7 @@ FM_DEVICE bool fm_x2_dkv(const X2Args& A, fm_half* st, int* bad) {
   const X2Max xg = fm_x2_join(A.mg + int64_t(bh) * A.nbq, b0, A.nbq, lane), xl = fm_x2_join(A.mg + int64_t(bh) * A.nbq, b1 + 1, A.nbq, lane);
   const float seen = xl.mx > 0.f ? xl.mx : A.tg[int64_t(bh) * A.nbq + b1];
   bool ok = xq.ok && xv.ok && !(causal && seen > 0.f && seen * 2048.0f < xg.mx);
+  ok = ok && (xg.ok || fm_x2_columns(A.mg + int64_t(bh) * A.nbq, A.cg + int64_t(bh) * A.nbq, b0, A.nbq, xg.mx, lane));
   const int eq = FM_UNIFORM(fm_x2_exp(xq.mx * qf, ok)), ev = FM_UNIFORM(fm_x2_exp(xv.mx, ok)), eg = FM_UNIFORM(fm_x2_exp(xg.mx, ok));
   if (!ok) return true;
   const float qs = qf * fm_x2_pow(eq), gsc = fm_x2_pow(eg), cl = fm_x2_scalb(1.0f, eg + ev);

@@ -321,3 +321,21 @@ def check_small_tensor_against_a_large_one(lib, bh, n, d, device, *, p, seed=0, 
         ref = oracle_all(q, k, v, go, mask=True, tau=1.0, p=p)
         errs = {m: rel_err(x, r) for m, x, r in zip(("o", "g", "dq", "dk", "dv"), (o, g, *grads), ref)}
         assert max(errs.values()) < tol, f"q x {q_scale:g}, k x {k_scale:g}, order {p}: {errs}"
+
+
+def check_column_of_small_gradients(lib, bh, n, d, device, *, mask, seed=0, tol=2e-6):
+    """fp32: a column of dO is zero in the first tokens and dO far smaller behind them, so that this column of dv is made of small
+    gradients alone.  It is held to the bar by itself."""
+    tau = 8.0 * math.sqrt(d)
+    kw = dict(mask=mask, inv_tau=1.0 / tau, p=2, flags=2)      # FASTMAX_FLAG_FORCE_DENSE
+    for scale in (1e-8, 1e-12):
+        q, k, v, go = make_inputs(bh, n, n, d, torch.float32, device, seed)
+        go[:, 64:] *= scale
+        go[:, :64, 3] = 0.0
+        go[:, :, 7] = 0.0                              # (zero everywhere: not a column of small numbers)
+        o, g = lib.forward(q, k, v, **kw)
+        grads = lib.backward(q, k, v, o, g, go, **kw)
+        ref = oracle_all(q, k, v, go, mask=mask, tau=tau, p=2)[2:]
+        errs = {m: rel_err(x, r) for m, x, r in zip(("dq", "dk", "dv"), grads, ref)}
+        errs["dv there"] = rel_err(grads[2][..., 3], ref[2][..., 3])
+        assert max(errs.values()) < tol and not bool(grads[2][..., 7].any()), f"dO x {scale:g}: {errs}"

@@ -17,7 +17,7 @@ import pytest
 import torch
 
 from reproducing_fastmax_results_amd import _capi
-from tests.parity import (TOL, check_small_tensor_against_a_large_one, check_keys_that_see_small_gradients, check_ranges_of_two_planes, check_upstream_gradients_at_the_ends_of_the_range, check_infinite_and_largest_values, check_tiny_values, check_batch_head_strides, check_decode, check_norm_fold, check_prompt_at_the_ends_of_the_range, check_forward, check_forward_backward, make_inputs, oracle_all,
+from tests.parity import (TOL, check_column_of_small_gradients, check_small_tensor_against_a_large_one, check_keys_that_see_small_gradients, check_ranges_of_two_planes, check_upstream_gradients_at_the_ends_of_the_range, check_infinite_and_largest_values, check_tiny_values, check_batch_head_strides, check_decode, check_norm_fold, check_prompt_at_the_ends_of_the_range, check_forward, check_forward_backward, make_inputs, oracle_all,
                           rel_err)
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -514,3 +514,9 @@ def test_two_planes_scores_are_all_of_the_derivative(sim, two_planes, a1):
     grads = sim.backward(q, k, v, o, g, go, **kw)
     errs = [rel_err(x, r) for x, r in zip((o, g, *grads), oracle_all(q, k, v, go, mask=True, tau=tau, p=2, a=a))]
     assert max(errs) < 2e-6, errs
+
+
+@pytest.mark.parametrize("split,mask", [(1, False), (2, True), (4, False), (4, True)])
+def test_two_planes_column_of_small_gradients(sim, two_planes, split, mask):
+    two_planes(split)
+    check_column_of_small_gradients(sim, 1, 150, 32, "cpu", mask=mask, seed=82)
