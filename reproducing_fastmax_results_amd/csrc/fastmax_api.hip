@@ -151,6 +151,7 @@ inline bool states_pay_unmasked(const FastmaxDesc* d) {
 // The CPU tests' problems are few and short: set, they go to the kernels of fm_x2.h, with this many wavefronts to an own tile.
 static int fm_hostsim_x2 = 0;
 extern "C" void fastmax_hostsim_x2(int split) { fm_hostsim_x2 = split; }
+extern "C" int fastmax_hostsim_x2_left(int walked) { const int n = fm_hostsim_x2_left[walked]; fm_hostsim_x2_left[walked] = 0; return n; }
 #endif
 inline int x3_split(int bh, int n_own, int tokens) {
 #if defined(FM_HOSTSIM)
@@ -244,8 +245,8 @@ template <int DH> size_t big_array_bytes(int esz, bool quad, size_t slots) {
 }
 
 // floats of the ranges of q, k and v, and of gh (see launch_x2_range)
-inline size_t x2_keys(const FastmaxDesc* d) { return size_t(d->bh) * (fm_x2_blocks(d->nq) + 2 * fm_x2_blocks(d->nk)); }
-inline size_t x2_gradients(const FastmaxDesc* d) { return size_t(4) * d->bh * fm_x2_blocks(d->nq); }
+inline size_t x2_keys(const FastmaxDesc* d) { return size_t(2) * d->bh * (fm_x2_blocks(d->nq) + 2 * fm_x2_blocks(d->nk)); }
+inline size_t x2_gradients(const FastmaxDesc* d) { return size_t(6) * d->bh * fm_x2_blocks(d->nq); }
 
 int make_plan(const FastmaxDesc* d, Plan& p) {
   int st = validate(d);
@@ -715,16 +716,18 @@ template <int DH>
 int launch_x2_range(const FastmaxDesc* d, const void* q, const void* k, const void* v, const void* d_o, const float* g, float* keys,
                     float* gh, X2Args& a, fm_stream_t stream) {
   const int nbq = fm_x2_blocks(d->nq), nbk = fm_x2_blocks(d->nk);
-  float *mq = keys, *mk = mq + size_t(d->bh) * nbq, *mv = mk + size_t(d->bh) * nbk;
-  float* tail = gh ? gh + size_t(d->bh) * nbq : nullptr;
-  unsigned long long* cols = gh ? reinterpret_cast<unsigned long long*>(gh + size_t(2) * d->bh * nbq) : nullptr;
-  a.mq = mq; a.mk = mk; a.mv = mv; a.mg = gh; a.tg = tail; a.cg = cols; a.nbq = nbq; a.nbk = nbk;
+  const size_t tq = size_t(d->bh) * nbq, tk = size_t(d->bh) * nbk;
+  float *mq = keys, *mk = mq + tq, *mv = mk + tk, *sq = mv + tk, *sk = sq + tq, *sv = sk + tk;
+  float *sg = nullptr, *tail = nullptr;
+  unsigned long long* cols = nullptr;
+  if (gh) { sg = gh + tq; tail = sg + tq; cols = reinterpret_cast<unsigned long long*>(tail + 2 * tq); }
+  a.mq = mq; a.mk = mk; a.mv = mv; a.mg = gh; a.sq = sq; a.sk = sk; a.sv = sv; a.sg = sg; a.tg = tail; a.cg = cols; a.nbq = nbq; a.nbk = nbk;
   X2Job j[4];
   int n = 0;
-  if (q) j[n++] = X2Job{cref<float>(q, d->sq), TRef<float>{}, mq, nullptr, nullptr, d->nq, nbq, 0};
-  if (k) j[n++] = X2Job{cref<float>(k, d->sk), TRef<float>{}, mk, nullptr, nullptr, d->nk, nbk, 0};
-  if (v) j[n++] = X2Job{cref<float>(v, d->sv), TRef<float>{}, mv, nullptr, nullptr, d->nk, nbk, 0};
-  if (d_o) j[n++] = X2Job{cref<float>(d_o, d->sdo), fm_ref<float>(const_cast<float*>(g), d->sg), gh, tail, cols, d->nq, nbq, 1};
+  if (q) j[n++] = X2Job{cref<float>(q, d->sq), TRef<float>{}, mq, sq, nullptr, nullptr, d->nq, nbq, 0};
+  if (k) j[n++] = X2Job{cref<float>(k, d->sk), TRef<float>{}, mk, sk, nullptr, nullptr, d->nk, nbk, 0};
+  if (v) j[n++] = X2Job{cref<float>(v, d->sv), TRef<float>{}, mv, sv, nullptr, nullptr, d->nk, nbk, 0};
+  if (d_o) j[n++] = X2Job{cref<float>(d_o, d->sdo), fm_ref<float>(const_cast<float*>(g), d->sg), gh, sg, tail, cols, d->nq, nbq, 1};
   const int jobs = n;
   while (n < 4) { j[n] = j[0]; ++n; }
   ProfScope prof(FM_K_PREP_BWD, stream);

@@ -21,11 +21,10 @@
 // The powers are taken out of the polynomials' coefficients and of the sums, exactly.
 //
 // Which problems these kernels may take is decided in two places.  x2_coefficients (host): a0 > 0, a1 of its
-// size and a2 no larger than that.  k_x2_range and its readers, per batch*head: a row or a column of a 64-token block that is not zero reaches 2^-7 of the
-// block's largest entry, and a block that is not zero 2^-6 of the tensor's; then the largest entry of every row and every column of
-// a block is at least 2^-13 of the tensor's largest, and is held to 2^-26 of itself.  (gh: whole rows and blocks may be smaller, they
-// add little to sums over rows; a column may not lie in them alone.)  A workgroup whose tensors do not keep to
-// that, and one with a sum that is not finite (an infinity, a weight beyond 65504), makes its rows as fm_x3.h does (and so, where
+// size and a2 no larger than that.  k_x2_range and its readers, per batch*head: the largest entry of every row and every column of
+// a block of 64 tokens that is not zero is at least 2^-14 of the tensor's largest, and so is held to 2^-25 of itself.  (gh: whole rows
+// and blocks may be smaller, they add little to sums over rows; a column may not lie in them alone.)  A workgroup whose tensors do not
+// keep to that, and one with a sum that is not finite (an infinity, a weight beyond 65504), makes its rows as fm_x3.h does (and so, where
 // its sums are not finite either, or where fm_x3.h's planes would lose a coefficient, with fp32 matrix products).
 #pragma once
 #include "fm_x3.h"
@@ -131,10 +130,10 @@ template <int DH> struct X2Row {
 static constexpr int FM_X2_TOKENS = 64;                // rows of a partial maximum; the last takes the rest (up to 127)
 FM_DEVICE int fm_x2_block(int row, int nblk) { return row / FM_X2_TOKENS < nblk ? row / FM_X2_TOKENS : nblk - 1; }
 inline int fm_x2_blocks(int n) { return n < FM_X2_TOKENS ? 1 : n / FM_X2_TOKENS; }
-struct X2Job { TRef<const float> x; TRef<float> g; float *part, *tail; unsigned long long* cols; int n, nblk, divide; };   // [bh][nblk] each
+struct X2Job { TRef<const float> x; TRef<float> g; float *part, *least, *tail; unsigned long long* cols; int n, nblk, divide; };   // [bh][nblk] each
 
-// Largest |x| (divide: |x / g|) of a block of rows, or infinity where the block does not keep to the range (see above).  Where rows are
-// divided their sizes are left out of that (a small row adds little to sums over rows, and its own workgroup scales it by itself), but
+// part: largest |x| (divide: |x / g|) of a block of rows.  least: the smallest largest entry of its rows and columns that are not zero.  Where
+// rows are divided their sizes are left out of that (a small row adds little to sums over rows, and its own workgroup scales it by itself), but
 // a key that sees the sequence's end alone must not find it small: tail is the largest entry of the block's last row that is not zero.
 // cols: one bit per column that is not zero (see fm_x2_columns).
 // grid (blocks, bh, jobs), 256 threads.  Reads its tensors once: three of 4 x 8 heads of 4096 x 64 (101 MB).
@@ -213,18 +212,20 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_x2_range(X2Job j0, X2Job j1, X2Job j2, X2
     }
     if (J.tail) J.tail[int64_t(bh) * J.nblk + blk] = fm_bits_f32(uint32_t(last));
     if (J.cols) J.cols[int64_t(bh) * J.nblk + blk] = bits;
-    J.part[int64_t(bh) * J.nblk + blk] = least * 128.0f < all ? __builtin_inff() : all;
+    J.part[int64_t(bh) * J.nblk + blk] = all;
+    J.least[int64_t(bh) * J.nblk + blk] = least;
   }
 }
 
-// Largest of the partial maxima b0 .. nblk - 1 and whether every one that is not zero reaches 2^-6 of it.  (Whole wavefronts.)
+// Largest of the partial maxima of blocks b0 .. nblk - 1, and whether what is not zero there reaches FM_X2_SPREAD of it.  (Whole wavefronts.)
+static constexpr float FM_X2_SPREAD = 0x1p-14f;
 struct X2Max { float mx; bool ok; };
-FM_DEVICE X2Max fm_x2_join(const float* part, int b0, int nblk, int lane) {
+FM_DEVICE X2Max fm_x2_join(const float* part, const float* small, int b0, int nblk, int lane) {
   float m = 0.f, least = 0x1p127f;
   for (int i = b0 + lane; i < nblk; i += 64) {
-    const float x = part[i];
+    const float x = part[i], y = small[i];
     m = fm_fmaxf(m, x);
-    least = x > 0.f && x < least ? x : least;
+    least = y < least ? y : least;
   }
 #pragma unroll
   for (int s = 1; s < 64; s <<= 1) {
@@ -232,18 +233,17 @@ FM_DEVICE X2Max fm_x2_join(const float* part, int b0, int nblk, int lane) {
     const float o = fm_shfl_xor(least, s);
     least = o < least ? o : least;
   }
-  const X2Max r = {m, !(least * 64.0f < m)};
+  const X2Max r = {m, least >= m * FM_X2_SPREAD};
   return r;
 }
-// Whether every column of blocks b0 .. nblk - 1 that is not zero is of the size of mx (a block near mx has all of them), where the blocks
-// themselves are not.
-FM_DEVICE bool fm_x2_columns(const float* part, const unsigned long long* cols, int b0, int nblk, float mx, int lane) {
+// Whether every column of blocks b0 .. nblk - 1 that is not zero reaches that part of mx (one block has all of them so), where not every block does.
+FM_DEVICE bool fm_x2_columns(const float* small, const unsigned long long* cols, int b0, int nblk, float mx, int lane) {
   unsigned long long all = 0;
   for (int i = b0 + lane; i < nblk; i += 64) all |= cols[i];
 #pragma unroll
   for (int s = 1; s < 64; s <<= 1) all |= fm_shfl_xor_u64(all, s);
   unsigned long long one = 0;
-  for (int i = b0 + lane; i < nblk; i += 64) one |= part[i] * 64.0f >= mx && cols[i] == all ? 1 : 0;
+  for (int i = b0 + lane; i < nblk; i += 64) one |= small[i] >= mx * FM_X2_SPREAD && cols[i] == all ? 1 : 0;
 #pragma unroll
   for (int s = 1; s < 64; s <<= 1) one |= fm_shfl_xor_u64(one, s);
   return one != 0;
@@ -273,8 +273,17 @@ FM_DEVICE int fm_x2_row_exp(float m, int stream, int* bad) {
   return e + stream > 56 ? 56 - stream : e;
 }
 
+#if defined(FM_HOSTSIM)
+// Workgroups of these kernels whose rows fm_x3.h made: without a walk, and after one.
+inline int fm_hostsim_x2_left[2] = {0, 0};
+FM_DEVICE bool fm_x2_leave(int walked) { if (FM_TID_X == 0) ++fm_hostsim_x2_left[walked]; return true; }
+#else
+FM_DEVICE bool fm_x2_leave(int) { return true; }
+#endif
+
 struct X2Args : X3Args<float> {
-  const float *mq, *mk, *mv, *mg, *tg;  // partial maxima, and gh's tails and columns: see k_x2_range
+  const float *mq, *mk, *mv, *mg;       // partial maxima, least entries, gh's tails and columns: see k_x2_range
+  const float *sq, *sk, *sv, *sg, *tg;
   const unsigned long long* cg;
   int nbq, nbk;
   int ew;                               // exponent of the weights' factor (a0 2^ew in [1, 2))
@@ -391,10 +400,10 @@ FM_DEVICE bool fm_x2_fwd(const X2Args& A, fm_half* st, int* bad) {
   Stage sg;
   sg.load(A.k, A.v, nullptr, bh, 0, A.nk, tid);
   const float kf = A.sc * fm_norm_factor(A.k_fold, bh, lane), qs = A.sc * fm_norm_factor(A.q_fold, bh, lane);
-  const X2Max xk = fm_x2_join(A.mk + int64_t(bh) * A.nbk, 0, A.nbk, lane), xv = fm_x2_join(A.mv + int64_t(bh) * A.nbk, 0, A.nbk, lane);
+  const X2Max xk = fm_x2_join(A.mk + int64_t(bh) * A.nbk, A.sk + int64_t(bh) * A.nbk, 0, A.nbk, lane), xv = fm_x2_join(A.mv + int64_t(bh) * A.nbk, A.sv + int64_t(bh) * A.nbk, 0, A.nbk, lane);
   bool ok = xk.ok && xv.ok;
   const int ek = FM_UNIFORM(fm_x2_exp(xk.mx * kf, ok)), ev = FM_UNIFORM(fm_x2_exp(xv.mx, ok));
-  if (!ok) return true;                                // the same for all of the batch*head
+  if (!ok) return fm_x2_leave(0);                      // the same for all of the batch*head
   const float ks_ = kf * fm_x2_pow(ek), vs = fm_x2_pow(ev);
   typename R::Own of;
   X3Coef cf;
@@ -453,7 +462,7 @@ FM_DEVICE bool fm_x2_fwd(const X2Args& A, fm_half* st, int* bad) {
     IO<float>::st8(A.out.base(bh) + int64_t(qi) * A.out.s_n + col, v);
     if (col == 0) A.g.base(bh)[int64_t(qi) * A.g.s_n] = fm_x2_scalb(gt, -A.ew);
   }
-  return fm_x3_again(bad);
+  return fm_x3_again(bad) && fm_x2_leave(1);
 }
 template <int DH, int SPLIT, int NW>
 FM_GLOBAL void FM_LAUNCH_BOUNDS2(64 * NW, 2) k_x2_fwd(X2Args A) {
@@ -491,10 +500,10 @@ FM_DEVICE bool fm_x2_dq(const X2Args& A, fm_half* st, int* bad) {
   Stage sg;
   sg.load(A.k, A.v, nullptr, bh, 0, A.nk, tid);
   const float kf = A.sc * fm_norm_factor(A.k_fold, bh, lane), qf = fm_norm_factor(A.q_fold, bh, lane);
-  const X2Max xk = fm_x2_join(A.mk + int64_t(bh) * A.nbk, 0, A.nbk, lane), xv = fm_x2_join(A.mv + int64_t(bh) * A.nbk, 0, A.nbk, lane);
+  const X2Max xk = fm_x2_join(A.mk + int64_t(bh) * A.nbk, A.sk + int64_t(bh) * A.nbk, 0, A.nbk, lane), xv = fm_x2_join(A.mv + int64_t(bh) * A.nbk, A.sv + int64_t(bh) * A.nbk, 0, A.nbk, lane);
   bool ok = xk.ok && xv.ok;
   const int ek = FM_UNIFORM(fm_x2_exp(xk.mx * kf, ok)), ev = FM_UNIFORM(fm_x2_exp(xv.mx, ok));
-  if (!ok) return true;
+  if (!ok) return fm_x2_leave(0);
   const float ks_ = kf * fm_x2_pow(ek), vs = fm_x2_pow(ev);
   typename R::Own of, of2;
   X3Coef cf;
@@ -560,7 +569,7 @@ FM_DEVICE bool fm_x2_dq(const X2Args& A, fm_half* st, int* bad) {
     for (int e = 0; e < 16; ++e) acc[ct][e] = fm_x2_scalb(acc[ct][e], eout);
   fm_x3_store<float, DH, QW, SPLIT, C::NTH, true>(acc, reinterpret_cast<float*>(st), sub, 32 * own + lr, lh, 1.0f, A.sc * (A.bpart ? qf : 1.0f), A.out,
                                           bh, t0, A.nq, tid, A.q, A.bpart ? A.bpart + int64_t(bh) * FM_GDIM_X + blk : nullptr, bad);
-  return fm_x3_again(bad);
+  return fm_x3_again(bad) && fm_x2_leave(1);
 }
 template <int DH, int SPLIT, int NW>
 FM_GLOBAL void FM_LAUNCH_BOUNDS2(64 * NW, 2) k_x2_dq(X2Args A) {
@@ -607,17 +616,17 @@ FM_DEVICE bool fm_x2_dkv(const X2Args& A, fm_half* st, int* bad) {
   };
   fetch(s_last);
   const float kf = fm_norm_factor(A.k_fold, bh, lane), qf = A.sc * fm_norm_factor(A.q_fold, bh, lane);
-  const X2Max xq = fm_x2_join(A.mq + int64_t(bh) * A.nbq, 0, A.nbq, lane), xv = fm_x2_join(A.mv + int64_t(bh) * A.nbk, 0, A.nbk, lane);
+  const X2Max xq = fm_x2_join(A.mq + int64_t(bh) * A.nbq, A.sq + int64_t(bh) * A.nbq, 0, A.nbq, lane), xv = fm_x2_join(A.mv + int64_t(bh) * A.nbk, A.sv + int64_t(bh) * A.nbk, 0, A.nbk, lane);
   // gh: of the queries that the block's keys see; what the last key sees has to be within the range of it: the blocks behind its own, or,
   // where those are zero, the last row of its own that is not (the row before that it may not see)
   const int tl = (t0 + QW < A.nk ? t0 + QW : A.nk) - 1;
   const int b0 = causal ? fm_x2_block(t0, A.nbq) : 0, b1 = causal ? fm_x2_block(tl, A.nbq) : 0;
-  const X2Max xg = fm_x2_join(A.mg + int64_t(bh) * A.nbq, b0, A.nbq, lane), xl = fm_x2_join(A.mg + int64_t(bh) * A.nbq, b1 + 1, A.nbq, lane);
+  const X2Max xg = fm_x2_join(A.mg + int64_t(bh) * A.nbq, A.sg + int64_t(bh) * A.nbq, b0, A.nbq, lane), xl = fm_x2_join(A.mg + int64_t(bh) * A.nbq, A.sg + int64_t(bh) * A.nbq, b1 + 1, A.nbq, lane);
   const float seen = xl.mx > 0.f ? xl.mx : A.tg[int64_t(bh) * A.nbq + b1];
-  bool ok = xq.ok && xv.ok && !(causal && seen > 0.f && seen * 2048.0f < xg.mx);
-  ok = ok && (xg.ok || fm_x2_columns(A.mg + int64_t(bh) * A.nbq, A.cg + int64_t(bh) * A.nbq, b0, A.nbq, xg.mx, lane));
+  bool ok = xq.ok && xv.ok && !(causal && seen > 0.f && seen < xg.mx * FM_X2_SPREAD);
+  ok = ok && (xg.ok || fm_x2_columns(A.sg + int64_t(bh) * A.nbq, A.cg + int64_t(bh) * A.nbq, b0, A.nbq, xg.mx, lane));
   const int eq = FM_UNIFORM(fm_x2_exp(xq.mx * qf, ok)), ev = FM_UNIFORM(fm_x2_exp(xv.mx, ok)), eg = FM_UNIFORM(fm_x2_exp(xg.mx, ok));
-  if (!ok) return true;
+  if (!ok) return fm_x2_leave(0);
   const float qs = qf * fm_x2_pow(eq), gsc = fm_x2_pow(eg), cl = fm_x2_scalb(1.0f, eg + ev);
   auto put = [&](int b) FM_ALWAYS_INLINE {
     fm_half* X = st + b * C::STAGE;
@@ -686,7 +695,7 @@ FM_DEVICE bool fm_x2_dkv(const X2Args& A, fm_half* st, int* bad) {
   fm_x3_store<float, DH, QW, SPLIT, C::NTH, true>(acc, Os, sub, 32 * own + lr, lh, 1.0f, A.sc * (A.bpart ? kf : 1.0f), A.out, bh, t0, A.nk, tid, A.k,
                                           A.bpart ? A.bpart + int64_t(bh) * FM_GDIM_X + blk : nullptr, bad);
   fm_x3_store<float, DH, QW, SPLIT, C::NTH, true>(av, Os, sub, 32 * own + lr, lh, 1.0f, 1.0f, A.out2, bh, t0, A.nk, tid, A.k, nullptr, bad);
-  return fm_x3_again(bad);
+  return fm_x3_again(bad) && fm_x2_leave(1);
 }
 template <int DH, int SPLIT>
 FM_GLOBAL void FM_LAUNCH_BOUNDS2(512, 2) k_x2_dkv(X2Args A) {

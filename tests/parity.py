@@ -339,3 +339,22 @@ def check_column_of_small_gradients(lib, bh, n, d, device, *, mask, seed=0, tol=
         errs = {m: rel_err(x, r) for m, x, r in zip(("dq", "dk", "dv"), grads, ref)}
         errs["dv there"] = rel_err(grads[2][..., 3], ref[2][..., 3])
         assert max(errs.values()) < tol and not bool(grads[2][..., 7].any()), f"dO x {scale:g}: {errs}"
+
+
+def check_numbers_within_two_planes(lib, bh, n, d, device, *, mask, seed=0, tol=2e-6):
+    """fp32: a first token with a value near zero and a feature of k far larger than the others, both common in trained models.  What only
+    those reach is held to the bar by itself."""
+    tau = 8.0 * math.sqrt(d)
+    q, k, v, go = make_inputs(bh, n, n, d, torch.float32, device, seed)
+    v[:, 0] *= 1e-3
+    k[..., 5] *= 300.0
+    q[..., 5] /= 300.0
+    kw = dict(mask=mask, inv_tau=1.0 / tau, p=2, flags=2)      # FASTMAX_FLAG_FORCE_DENSE
+    o, g = lib.forward(q, k, v, **kw)
+    grads = lib.backward(q, k, v, o, g, go, **kw)
+    ref = oracle_all(q, k, v, go, mask=mask, tau=tau, p=2)
+    errs = {m: rel_err(x, r) for m, x, r in zip(("o", "g", "dq", "dk", "dv"), (o, g, *grads), ref)}
+    errs["first o"] = rel_err(o[:, 0], ref[0][:, 0])
+    errs["other dq"] = rel_err(grads[0][..., :5], ref[2][..., :5])
+    errs["dk there"] = rel_err(grads[1][..., 5], ref[3][..., 5])
+    assert max(errs.values()) < tol, errs

@@ -4,7 +4,7 @@ bf16-rounded inputs)."""
 import pytest
 import torch
 
-from tests.parity import (check_column_of_small_gradients, check_small_tensor_against_a_large_one, check_keys_that_see_small_gradients, check_ranges_of_two_planes, check_infinite_and_largest_values, check_prompt_at_the_ends_of_the_range, check_tiny_values, check_upstream_gradients_at_the_ends_of_the_range, check_batch_head_strides, check_decode, check_forward, check_forward_backward,
+from tests.parity import (check_numbers_within_two_planes, check_column_of_small_gradients, check_small_tensor_against_a_large_one, check_keys_that_see_small_gradients, check_ranges_of_two_planes, check_infinite_and_largest_values, check_prompt_at_the_ends_of_the_range, check_tiny_values, check_upstream_gradients_at_the_ends_of_the_range, check_batch_head_strides, check_decode, check_forward, check_forward_backward,
                           check_norm_fold, make_inputs)
 from reproducing_fastmax_results_amd._capi import FLAG_F32_COMPUTE, FLAG_FORCE_DENSE, FLAG_FORCE_MOMENTS, FLAG_NORM_SELF
 
@@ -431,6 +431,12 @@ def test_two_planes_small_tensor_against_a_large_one(lib, bh, n, d, p):
 def test_two_planes_column_of_small_gradients(lib, bh, n, d, mask):
     print(f"case column of small gradients bh={bh} n={n} d={d} mask={mask}", flush=True)
     check_column_of_small_gradients(lib, bh, n, d, DEV, mask=mask, seed=143)
+
+
+@pytest.mark.parametrize("bh,n,d,mask", [(128, 1030, 64, True), (16, 1030, 64, False), (2, 3100, 32, True)])
+def test_numbers_within_two_planes(lib, bh, n, d, mask):
+    print(f"case numbers within two planes bh={bh} n={n} d={d} mask={mask}", flush=True)
+    check_numbers_within_two_planes(lib, bh, n, d, DEV, mask=mask, seed=144)
 
 
 @pytest.mark.parametrize("d", [32, 64])

@@ -17,7 +17,7 @@ import pytest
 import torch
 
 from reproducing_fastmax_results_amd import _capi
-from tests.parity import (TOL, check_column_of_small_gradients, check_small_tensor_against_a_large_one, check_keys_that_see_small_gradients, check_ranges_of_two_planes, check_upstream_gradients_at_the_ends_of_the_range, check_infinite_and_largest_values, check_tiny_values, check_batch_head_strides, check_decode, check_norm_fold, check_prompt_at_the_ends_of_the_range, check_forward, check_forward_backward, make_inputs, oracle_all,
+from tests.parity import (TOL, check_numbers_within_two_planes, check_column_of_small_gradients, check_small_tensor_against_a_large_one, check_keys_that_see_small_gradients, check_ranges_of_two_planes, check_upstream_gradients_at_the_ends_of_the_range, check_infinite_and_largest_values, check_tiny_values, check_batch_head_strides, check_decode, check_norm_fold, check_prompt_at_the_ends_of_the_range, check_forward, check_forward_backward, make_inputs, oracle_all,
                           rel_err)
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -520,3 +520,23 @@ def test_two_planes_scores_are_all_of_the_derivative(sim, two_planes, a1):
 def test_two_planes_column_of_small_gradients(sim, two_planes, split, mask):
     two_planes(split)
     check_column_of_small_gradients(sim, 1, 150, 32, "cpu", mask=mask, seed=82)
+
+
+def left_two_planes(sim):
+    """Workgroups that fm_x3.h made since the last call: without a walk over two planes, and after one."""
+    return sim.lib.fastmax_hostsim_x2_left(0), sim.lib.fastmax_hostsim_x2_left(1)
+
+
+@pytest.mark.parametrize("split,mask", [(1, True), (4, False)])
+def test_two_planes_hold_ordinary_numbers(sim, two_planes, split, mask):
+    """Ordinary numbers, and those of trained models, stay with two planes; far smaller rows do not."""
+    two_planes(split)
+    left_two_planes(sim)
+    check_forward_backward(sim, 1, 130, 64, torch.float32, "cpu", mask=mask, p=2, seed=83, saved=True, flags=_capi.FLAG_FORCE_DENSE)
+    check_numbers_within_two_planes(sim, 1, 130, 32, "cpu", mask=mask, seed=84)
+    assert left_two_planes(sim) == (0, 0)
+    q, k, v, _ = make_inputs(1, 130, 130, 32, torch.float32, "cpu", 85)
+    v[:, 100] *= 1e-9
+    sim.forward(q, k, v, mask=mask, inv_tau=0.02, p=2, flags=_capi.FLAG_FORCE_DENSE)
+    refused, walked = left_two_planes(sim)
+    assert refused > 0 and walked == 0
