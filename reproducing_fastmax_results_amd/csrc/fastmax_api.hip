@@ -245,7 +245,7 @@ template <int DH> size_t big_array_bytes(int esz, bool quad, size_t slots) {
 }
 
 // floats of the ranges of q, k and v, and of gh (see launch_x2_range)
-inline size_t x2_keys(const FastmaxDesc* d) { return size_t(2) * d->bh * (fm_x2_blocks(d->nq) + 2 * fm_x2_blocks(d->nk)); }
+inline size_t x2_keys(const FastmaxDesc* d) { return size_t(d->bh) * (3 * fm_x2_blocks(d->nq) + 5 * fm_x2_blocks(d->nk)); }
 inline size_t x2_gradients(const FastmaxDesc* d) { return size_t(6) * d->bh * fm_x2_blocks(d->nq); }
 
 int make_plan(const FastmaxDesc* d, Plan& p) {
@@ -717,17 +717,17 @@ int launch_x2_range(const FastmaxDesc* d, const void* q, const void* k, const vo
                     float* gh, X2Args& a, fm_stream_t stream) {
   const int nbq = fm_x2_blocks(d->nq), nbk = fm_x2_blocks(d->nk);
   const size_t tq = size_t(d->bh) * nbq, tk = size_t(d->bh) * nbk;
-  float *mq = keys, *mk = mq + tq, *mv = mk + tk, *sq = mv + tk, *sk = sq + tq, *sv = sk + tk;
+  float *mq = keys, *mk = mq + tq, *mv = mk + tk, *sq = mv + tk, *sk = sq + tq, *sv = sk + tk, *lq = sv + tk, *lk = lq + tq;
   float *sg = nullptr, *tail = nullptr;
   unsigned long long* cols = nullptr;
   if (gh) { sg = gh + tq; tail = sg + tq; cols = reinterpret_cast<unsigned long long*>(tail + 2 * tq); }
-  a.mq = mq; a.mk = mk; a.mv = mv; a.mg = gh; a.sq = sq; a.sk = sk; a.sv = sv; a.sg = sg; a.tg = tail; a.cg = cols; a.nbq = nbq; a.nbk = nbk;
+  a.mq = mq; a.mk = mk; a.mv = mv; a.mg = gh; a.sq = sq; a.sk = sk; a.sv = sv; a.sg = sg; a.tg = tail; a.cg = cols; a.lq = lq; a.lk = lk; a.nbq = nbq; a.nbk = nbk;
   X2Job j[4];
   int n = 0;
-  if (q) j[n++] = X2Job{cref<float>(q, d->sq), TRef<float>{}, mq, sq, nullptr, nullptr, d->nq, nbq, 0};
-  if (k) j[n++] = X2Job{cref<float>(k, d->sk), TRef<float>{}, mk, sk, nullptr, nullptr, d->nk, nbk, 0};
-  if (v) j[n++] = X2Job{cref<float>(v, d->sv), TRef<float>{}, mv, sv, nullptr, nullptr, d->nk, nbk, 0};
-  if (d_o) j[n++] = X2Job{cref<float>(d_o, d->sdo), fm_ref<float>(const_cast<float*>(g), d->sg), gh, sg, tail, cols, d->nq, nbq, 1};
+  if (q) j[n++] = X2Job{cref<float>(q, d->sq), TRef<float>{}, mq, sq, lq, nullptr, nullptr, d->nq, nbq, 0};
+  if (k) j[n++] = X2Job{cref<float>(k, d->sk), TRef<float>{}, mk, sk, lk, nullptr, nullptr, d->nk, nbk, 0};
+  if (v) j[n++] = X2Job{cref<float>(v, d->sv), TRef<float>{}, mv, sv, nullptr, nullptr, nullptr, d->nk, nbk, 0};
+  if (d_o) j[n++] = X2Job{cref<float>(d_o, d->sdo), fm_ref<float>(const_cast<float*>(g), d->sg), gh, sg, nullptr, tail, cols, d->nq, nbq, 1};
   const int jobs = n;
   while (n < 4) { j[n] = j[0]; ++n; }
   ProfScope prof(FM_K_PREP_BWD, stream);

@@ -117,6 +117,10 @@ FM_DEVICE void fm_swap_halves(uint32_t& a, uint32_t& b) {
   if (l < 32) b = oa; else a = ob;
 }
 FM_DEVICE float fm_fmaxf(float a, float b) { return a != a ? b : (b != b ? a : (a > b ? a : b)); }   // drops a NaN, like fmaxf
+template <int FROM, int TO> FM_DEVICE float fm_lanes_max(float v) {
+  for (int m = FROM; m < TO; m <<= 1) v = fm_fmaxf(v, fm_shfl_xor(v, m));
+  return v;
+}
 FM_DEVICE float fm_absf(float x) { return __builtin_fabsf(x); }
 FM_DEVICE float fm_clampf(float x, float lim) { return x > lim ? lim : (x < -lim ? -lim : x); }
 FM_DEVICE float fm_rsqrtf(float a) { return 1.0f / std::sqrt(a); }
@@ -241,6 +245,27 @@ FM_DEVICE void fm_swap_halves(uint32_t& a, uint32_t& b) {
   a = r[0]; b = r[1];
 }
 FM_DEVICE float fm_fmaxf(float a, float b) { return fmaxf(a, b); }
+// Largest of the values of the lanes that differ in the bits FROM .. TO / 2 of their number, in each of them, without the LDS pipe but for
+// bit 2 alone: data-parallel primitives inside rows of 16, then rows and halves exchanged.
+template <int FROM, int TO> FM_DEVICE float fm_lanes_max(float v) {
+  typedef uint32_t fm_u2 __attribute__((ext_vector_type(2)));
+#define FM_DPP_MAX(ctrl) v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), (ctrl), 0xf, 0xf, true)))
+  if (FROM <= 1 && TO > 1) FM_DPP_MAX(0xB1);           // quad_perm [1,0,3,2]
+  if (FROM <= 2 && TO > 2) FM_DPP_MAX(0x4E);           // quad_perm [2,3,0,1]
+  if (FROM == 1 && TO > 4) FM_DPP_MAX(0x141);          // row_half_mirror: the other quad
+  else if (FROM <= 4 && TO > 4) v = fmaxf(v, fm_shfl_xor(v, 4));
+  if (FROM <= 8 && TO > 8) FM_DPP_MAX(0x128);          // row_ror:8
+#undef FM_DPP_MAX
+  if (FROM <= 16 && TO > 16) {
+    const fm_u2 r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  }
+  if (FROM <= 32 && TO > 32) {
+    const fm_u2 r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  }
+  return v;
+}
 FM_DEVICE float fm_absf(float x) { return __builtin_fabsf(x); }
 // clamp to [-lim, lim] in one instruction (v_med3_f32)
 FM_DEVICE float fm_clampf(float x, float lim) { return __builtin_amdgcn_fmed3f(x, -lim, lim); }

@@ -17,15 +17,16 @@
 //   own rows     the row's largest entry (the lane holds the row)
 //   stream rows  the largest entry of the batch*head (k, v, q) or of what a block of keys sees (gh = dO / g, which falls like the
 //                reciprocal of the token index): partial maxima per 64 tokens, written by k_x2_range and joined by every workgroup
-//   weights      f(s) as it is, times the power of two that brings a0 to [1, 2); dS times 2^-19 (of products of two scaled rows)
+//   weights      f(s) as it is, times the power of two that brings a0 to [1, 2); dS times 2^-19 (of products of two scaled rows), less
+//                where scores are large (fm_x2_ds_exp)
 // The powers are taken out of the polynomials' coefficients and of the sums, exactly.
 //
 // Which problems these kernels may take is decided in two places.  x2_coefficients (host): a0 > 0, a1 of its
 // size and a2 no larger than that.  k_x2_range and its readers, per batch*head: the largest entry of every row and every column of
 // a block of 64 tokens that is not zero is at least 2^-14 of the tensor's largest, and so is held to 2^-25 of itself.  (gh: whole rows
 // and blocks may be smaller, they add little to sums over rows; a column may not lie in them alone.)  A workgroup whose tensors do not
-// keep to that, and one with a sum that is not finite (an infinity, a weight beyond 65504), makes its rows as fm_x3.h does (and so, where
-// its sums are not finite either, or where fm_x3.h's planes would lose a coefficient, with fp32 matrix products).
+// keep to that, one whose weights may pass 65504 (fm_x2_weights) and one with a sum that is not finite make their rows as fm_x3.h does (and so,
+// where those sums are not finite either, or where fm_x3.h's planes would lose a coefficient, with fp32 matrix products).
 #pragma once
 #include "fm_x3.h"
 #include <cmath>
@@ -130,23 +131,23 @@ template <int DH> struct X2Row {
 static constexpr int FM_X2_TOKENS = 64;                // rows of a partial maximum; the last takes the rest (up to 127)
 FM_DEVICE int fm_x2_block(int row, int nblk) { return row / FM_X2_TOKENS < nblk ? row / FM_X2_TOKENS : nblk - 1; }
 inline int fm_x2_blocks(int n) { return n < FM_X2_TOKENS ? 1 : n / FM_X2_TOKENS; }
-struct X2Job { TRef<const float> x; TRef<float> g; float *part, *least, *tail; unsigned long long* cols; int n, nblk, divide; };   // [bh][nblk] each
+struct X2Job { TRef<const float> x; TRef<float> g; float *part, *least, *norm, *tail; unsigned long long* cols; int n, nblk, divide; };   // [bh][nblk] each
 
 // part: largest |x| (divide: |x / g|) of a block of rows.  least: the smallest largest entry of its rows and columns that are not zero.  Where
 // rows are divided their sizes are left out of that (a small row adds little to sums over rows, and its own workgroup scales it by itself), but
 // a key that sees the sequence's end alone must not find it small: tail is the largest entry of the block's last row that is not zero.
-// cols: one bit per column that is not zero (see fm_x2_columns).
+// cols: one bit per column that is not zero (see fm_x2_columns).  norm: the largest Euclidean norm of a row.
 // grid (blocks, bh, jobs), 256 threads.  Reads its tensors once: three of 4 x 8 heads of 4096 x 64 (101 MB).
 template <int DH>
 FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_x2_range(X2Job j0, X2Job j1, X2Job j2, X2Job j3) {
   constexpr int CPR = DH / 8, RPP = 256 / CPR;         // threads of a row, rows of a pass
-  FM_SHARED float cm[4][DH], wr[4];
+  FM_SHARED float cm[4][DH], wr[4], wn[4];
   FM_SHARED unsigned long long wt[4];
   const X2Job& J = FM_BID_Z == 0 ? j0 : FM_BID_Z == 1 ? j1 : FM_BID_Z == 2 ? j2 : j3;
   const int tid = FM_TID_X, bh = FM_BID_Y, blk = FM_BID_X;
   if (blk >= J.nblk) return;
   const int r0 = blk * FM_X2_TOKENS, r1 = blk == J.nblk - 1 ? J.n : r0 + FM_X2_TOKENS, col = (tid % CPR) * 8;
-  float c[8], rmin = 0x1p127f;
+  float c[8], rmin = 0x1p127f, n2 = 0.f;
   unsigned long long last = 0;                         // row and bits of its largest entry
 #pragma unroll
   for (int i = 0; i < 8; ++i) c[i] = 0.f;
@@ -165,11 +166,11 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_x2_range(X2Job j0, X2Job j1, X2Job j2, X2
     }
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
-      float m = 0.f;
+      float m = 0.f, q = 0.f;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) { const float a = fm_absf(v[u][i]); c[i] = fm_fmaxf(c[i], a); m = fm_fmaxf(m, a); }
-#pragma unroll
-      for (int s = 1; s < CPR; s <<= 1) m = fm_fmaxf(m, fm_shfl_xor(m, s));
+      for (int i = 0; i < 8; ++i) { const float a = fm_absf(v[u][i]); c[i] = fm_fmaxf(c[i], a); m = fm_fmaxf(m, a); q += a * a; }
+      m = fm_lanes_max<1, CPR>(m);
+      n2 = fm_fmaxf(n2, fm_group_sum<CPR>(q));
       if (m > 0.f && m < rmin) rmin = m;
       uint32_t b;
       __builtin_memcpy(&b, &m, 4);
@@ -178,38 +179,40 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_x2_range(X2Job j0, X2Job j1, X2Job j2, X2
     }
   }
 #pragma unroll
-  for (int s = CPR; s < 64; s <<= 1) {
+  for (int i = 0; i < 8; ++i) c[i] = fm_lanes_max<CPR, 64>(c[i]);
+  rmin = -fm_lanes_max<CPR, 64>(-rmin);
+  n2 = fm_lanes_max<CPR, 64>(n2);
+  if (J.tail) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) c[i] = fm_fmaxf(c[i], fm_shfl_xor(c[i], s));
-    const float o = fm_shfl_xor(rmin, s);
-    rmin = o < rmin ? o : rmin;
-    const unsigned long long l = fm_shfl_xor_u64(last, s);
-    last = l > last ? l : last;
+    for (int s = CPR; s < 64; s <<= 1) {
+      const unsigned long long l = fm_shfl_xor_u64(last, s);
+      last = l > last ? l : last;
+    }
   }
   const int wave = tid >> 6, lane = tid & 63;
   if (lane < CPR) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) cm[wave][col + i] = c[i];
   }
-  if (lane == 0) { wr[wave] = rmin; wt[wave] = last; }
+  if (lane == 0) { wr[wave] = rmin; wn[wave] = n2; wt[wave] = last; }
   FM_SYNC();
   if (tid >= 64) return;
   float m = 0.f;
   if (tid < DH) m = fm_fmaxf(fm_fmaxf(cm[0][tid], cm[1][tid]), fm_fmaxf(cm[2][tid], cm[3][tid]));
   float all = m, least = m > 0.f ? m : 0x1p127f;
   unsigned long long bits = m > 0.f ? 1ull << tid : 0ull;
+  all = fm_lanes_max<1, 64>(all);
+  least = -fm_lanes_max<1, 64>(-least);
+  if (J.cols) {
 #pragma unroll
-  for (int s = 1; s < 64; s <<= 1) {
-    all = fm_fmaxf(all, fm_shfl_xor(all, s));
-    bits |= fm_shfl_xor_u64(bits, s);
-    const float o = fm_shfl_xor(least, s);
-    least = o < least ? o : least;
+    for (int s = 1; s < 64; s <<= 1) bits |= fm_shfl_xor_u64(bits, s);
   }
   if (tid == 0) {
     for (int w = 0; w < 4; ++w) {
       if (!J.divide) least = wr[w] < least ? wr[w] : least;
       last = wt[w] > last ? wt[w] : last;
     }
+    if (J.norm) J.norm[int64_t(bh) * J.nblk + blk] = fm_sqrtf(fm_fmaxf(fm_fmaxf(wn[0], wn[1]), fm_fmaxf(wn[2], wn[3])));
     if (J.tail) J.tail[int64_t(bh) * J.nblk + blk] = fm_bits_f32(uint32_t(last));
     if (J.cols) J.cols[int64_t(bh) * J.nblk + blk] = bits;
     J.part[int64_t(bh) * J.nblk + blk] = all;
@@ -219,7 +222,7 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS(256) k_x2_range(X2Job j0, X2Job j1, X2Job j2, X2
 
 // Largest of the partial maxima of blocks b0 .. nblk - 1, and whether what is not zero there reaches FM_X2_SPREAD of it.  (Whole wavefronts.)
 static constexpr float FM_X2_SPREAD = 0x1p-14f;
-struct X2Max { float mx; bool ok; };
+struct X2Max { float mx, least; bool ok; };
 FM_DEVICE X2Max fm_x2_join(const float* part, const float* small, int b0, int nblk, int lane) {
   float m = 0.f, least = 0x1p127f;
   for (int i = b0 + lane; i < nblk; i += 64) {
@@ -227,14 +230,16 @@ FM_DEVICE X2Max fm_x2_join(const float* part, const float* small, int b0, int nb
     m = fm_fmaxf(m, x);
     least = y < least ? y : least;
   }
-#pragma unroll
-  for (int s = 1; s < 64; s <<= 1) {
-    m = fm_fmaxf(m, fm_shfl_xor(m, s));
-    const float o = fm_shfl_xor(least, s);
-    least = o < least ? o : least;
-  }
-  const X2Max r = {m, least >= m * FM_X2_SPREAD};
+  m = fm_lanes_max<1, 64>(m);
+  least = -fm_lanes_max<1, 64>(-least);
+  const X2Max r = {m, least, least >= m * FM_X2_SPREAD};
   return r;
+}
+// Largest of the norms.
+FM_DEVICE float fm_x2_longest(const float* norm, int nblk, int lane) {
+  float m = 0.f;
+  for (int i = lane; i < nblk; i += 64) m = fm_fmaxf(m, norm[i]);
+  return fm_lanes_max<1, 64>(m);
 }
 // Whether every column of blocks b0 .. nblk - 1 that is not zero reaches that part of mx (one block has all of them so), where not every block does.
 FM_DEVICE bool fm_x2_columns(const float* small, const unsigned long long* cols, int b0, int nblk, float mx, int lane) {
@@ -269,7 +274,7 @@ FM_DEVICE float fm_x2_scalb(float x, int e) {
 FM_DEVICE int fm_x2_row_exp(float m, int stream, int* bad) {
   bool ok = true;
   const int e = fm_x2_exp(m, ok);
-  if (!ok && (m > 1.0f || stream < -18)) *bad = 1;     // (looked at behind the stores)
+  if (!ok && (m > 1.0f || stream < -18)) *bad = 1;
   return e + stream > 56 ? 56 - stream : e;
 }
 
@@ -281,21 +286,38 @@ FM_DEVICE bool fm_x2_leave(int walked) { if (FM_TID_X == 0) ++fm_hostsim_x2_left
 FM_DEVICE bool fm_x2_leave(int) { return true; }
 #endif
 
+static constexpr int FM_X2_DS = -19;                   // dS's power of two, see fm_x2_ds_exp
 struct X2Args : X3Args<float> {
   const float *mq, *mk, *mv, *mg;       // partial maxima, least entries, gh's tails and columns: see k_x2_range
   const float *sq, *sk, *sv, *sg, *tg;
   const unsigned long long* cg;
+  const float *lq, *lk;                 // largest norms of q and k rows per block
   int nbq, nbk;
   int ew;                               // exponent of the weights' factor (a0 2^ew in [1, 2))
 };
-// The polynomials' coefficients: f(s) 2^ew, and f'(s) 2^(ew - 22), s = score 2^-es.
-static constexpr int FM_X2_DS = -19;
+// A score is at most the product of its rows' norms: b, the lane's own row with the longest stream row.
+//   weights      one beyond _Float16 would be infinite: the workgroup leaves them to fm_x3.h before it makes any
+//   dS           large derivatives take their size out of dS's power of two (an ordinary product of rows leaves them a factor of 8).  What
+//                that costs the small entries of dS is taken from the spread that v's rows may have.
+FM_DEVICE void fm_x2_weights(const X2Args& A, float b, int* bad) {
+  const float w = fm_absf(A.a0) + b * (fm_absf(A.a1) + b * fm_absf(A.a2));
+  if (!(fm_x2_scalb(w, A.ew) < 65000.0f)) *bad = 1;
+}
+FM_DEVICE int fm_x2_ds_exp(const X2Args& A, float b, const X2Max& v, int* bad) {
+  const float w = fm_x2_scalb(fm_absf(A.a1) + 2.0f * b * fm_absf(A.a2), A.ew);
+  uint32_t u;
+  __builtin_memcpy(&u, &w, 4);
+  const int over = int(u >> 23) - 127 - 2, e = over > 0 ? over : 0;
+  if (e > 0 && v.least < v.mx * fm_x2_scalb(FM_X2_SPREAD, e)) *bad = 1;
+  return FM_X2_DS - e;
+}
+// The polynomials' coefficients: f(s) 2^ew, and f'(s) 2^(ew + ds), s = score 2^-es.
 FM_DEVICE X3Coef fm_x2_coef(float a0, float a1, float a2, int ew, int es) {
   const X3Coef c = {fm_x2_scalb(a0, ew), fm_x2_scalb(a1, ew - es), fm_x2_scalb(a2, ew - 2 * es)};
   return c;
 }
-FM_DEVICE X3Coef fm_x2_dcoef(float a1, float a2, int ew, int es) {
-  const X3Coef c = {0.f, fm_x2_scalb(a1, ew + FM_X2_DS), fm_x2_scalb(2.0f * a2, ew + FM_X2_DS - es)};
+FM_DEVICE X3Coef fm_x2_dcoef(float a1, float a2, int ew, int ds, int es) {
+  const X3Coef c = {0.f, fm_x2_scalb(a1, ew + ds), fm_x2_scalb(2.0f * a2, ew + ds - es)};
   return c;
 }
 // Coefficients that these kernels take; ew as above.  (A score too small to be seen beside a0 is the whole of f'(s) where a1 is zero.)
@@ -363,6 +385,14 @@ template <int DH> FM_DEVICE void fm_x2_own(const TRef<const float>& t, int bh, i
     for (int i = 0; i < 8; ++i) v[c][i] = in ? v[c][i] * f : 0.f;
   }
 }
+template <int DH> FM_DEVICE float fm_x2_norm(const float (*v)[8]) {
+  float q = 0.f;
+#pragma unroll
+  for (int c = 0; c < DH / 16; ++c)
+#pragma unroll
+    for (int i = 0; i < 8; ++i) q += v[c][i] * v[c][i];
+  return fm_sqrtf(q + fm_shfl_xor(q, 32));
+}
 template <int DH> FM_DEVICE float fm_x2_largest(const float (*v)[8]) {
   float m = 0.f;
 #pragma unroll
@@ -404,7 +434,7 @@ FM_DEVICE bool fm_x2_fwd(const X2Args& A, fm_half* st, int* bad) {
   bool ok = xk.ok && xv.ok;
   const int ek = FM_UNIFORM(fm_x2_exp(xk.mx * kf, ok)), ev = FM_UNIFORM(fm_x2_exp(xv.mx, ok));
   if (!ok) return fm_x2_leave(0);                      // the same for all of the batch*head
-  const float ks_ = kf * fm_x2_pow(ek), vs = fm_x2_pow(ev);
+  const float ks_ = kf * fm_x2_pow(ek), vs = fm_x2_pow(ev), kn = kf * fm_x2_longest(A.lk + int64_t(bh) * A.nbk, A.nbk, lane);
   typename R::Own of;
   X3Coef cf;
   {
@@ -414,6 +444,7 @@ FM_DEVICE bool fm_x2_fwd(const X2Args& A, fm_half* st, int* bad) {
     const int eq = fm_x2_row_exp(fm_x2_largest<DH>(v), ek, bad);
     fm_x2_set<DH>(of, v, fm_x2_scalb(1.0f, eq));
     cf = fm_x2_coef(A.a0, A.a1, A.a2, A.ew, eq + ek);
+    fm_x2_weights(A, kn * fm_x2_norm<DH>(v), bad);
   }
   fm_f32x16 acc[NT], small[NT];
 #pragma unroll
@@ -422,10 +453,11 @@ FM_DEVICE bool fm_x2_fwd(const X2Args& A, fm_half* st, int* bad) {
   int buf = 0;
   sg.store(st, st + KT * PQ, ks_, vs, false, tid);
   sg.load(A.k, A.v, nullptr, bh, KT, A.nk, tid);
+  if (fm_x3_again(bad)) return fm_x2_leave(0);         // (the first stage's barrier)
   for (int s0 = 0; s0 < send; s0 += KT) {
     const fm_half* X = st + buf * C::STAGE;
     const fm_half* Y = X + KT * PQ;
-    FM_SYNC();
+    if (s0 > 0) FM_SYNC();
     const int ss0 = s0 + 32 * sub;
     if (ss0 < A.nk && !(causal && ss0 > lo + 31)) {
       fm_f32x16 s = fm_zero16();
@@ -465,7 +497,7 @@ FM_DEVICE bool fm_x2_fwd(const X2Args& A, fm_half* st, int* bad) {
   return fm_x3_again(bad) && fm_x2_leave(1);
 }
 template <int DH, int SPLIT, int NW>
-FM_GLOBAL void FM_LAUNCH_BOUNDS2(64 * NW, 2) k_x2_fwd(X2Args A) {
+FM_GLOBAL void FM_LAUNCH_BOUNDS2(64 * NW, (DH == 32 && SPLIT == 2 ? 4 : 2)) k_x2_fwd(X2Args A) {   // (28 heads of 2200 tokens, unmasked, 78 us, with 133 registers 85)
   FM_DYN_SMEM(smem);
   FM_SHARED int bad;
   if (FM_TID_X == 0) bad = 0;
@@ -504,7 +536,7 @@ FM_DEVICE bool fm_x2_dq(const X2Args& A, fm_half* st, int* bad) {
   bool ok = xk.ok && xv.ok;
   const int ek = FM_UNIFORM(fm_x2_exp(xk.mx * kf, ok)), ev = FM_UNIFORM(fm_x2_exp(xv.mx, ok));
   if (!ok) return fm_x2_leave(0);
-  const float ks_ = kf * fm_x2_pow(ek), vs = fm_x2_pow(ev);
+  const float ks_ = kf * fm_x2_pow(ek), vs = fm_x2_pow(ev), kn = kf * fm_x2_longest(A.lk + int64_t(bh) * A.nbk, A.nbk, lane);
   typename R::Own of, of2;
   X3Coef cf;
   float cs = 0.f;
@@ -517,6 +549,7 @@ FM_DEVICE bool fm_x2_dq(const X2Args& A, fm_half* st, int* bad) {
     fm_x2_own<DH>(A.q, bh, row, in, lh, A.sc * qf, v);
     const int eq = fm_x2_row_exp(fm_x2_largest<DH>(v), ek, bad);
     fm_x2_set<DH>(of, v, fm_x2_scalb(1.0f, eq));
+    const int ds = fm_x2_ds_exp(A, kn * fm_x2_norm<DH>(v), xv, bad);
     fm_x2_own<DH>(A.d_o, bh, row, in, lh, in ? 1.0f / A.g.base(bh)[row * A.g.s_n] : 0.f, v);
     const float* po = A.o.base(bh) + row * A.o.s_n + 8 * lh;
 #pragma unroll
@@ -535,8 +568,8 @@ FM_DEVICE bool fm_x2_dq(const X2Args& A, fm_half* st, int* bad) {
     cs = fm_x2_scalb(cs, eg + ev);                     // as gh . v
 #pragma unroll
     for (int e = 0; e < 16; ++e) seed[e] = -cs;
-    cf = fm_x2_dcoef(A.a1, A.a2, A.ew, eq + ek);
-    eout = -(eg + ev + ek + A.ew + FM_X2_DS);
+    cf = fm_x2_dcoef(A.a1, A.a2, A.ew, ds, eq + ek);
+    eout = -(eg + ev + ek + A.ew + ds);
   }
   fm_f32x16 acc[NT];
 #pragma unroll
@@ -544,10 +577,11 @@ FM_DEVICE bool fm_x2_dq(const X2Args& A, fm_half* st, int* bad) {
   int buf = 0;
   sg.store(st, st + KT * PQ, ks_, vs, false, tid);
   sg.load(A.k, A.v, nullptr, bh, KT, A.nk, tid);
+  if (fm_x3_again(bad)) return fm_x2_leave(0);         // (the first stage's barrier)
   for (int s0 = 0; s0 < send; s0 += KT) {
     const fm_half* X = st + buf * C::STAGE;
     const fm_half* Y = X + KT * PQ;
-    FM_SYNC();
+    if (s0 > 0) FM_SYNC();
     const int ss0 = s0 + 32 * sub;
     if (ss0 < A.nk && !(causal && ss0 > lo + 31)) {
       fm_f32x16 s = fm_zero16(), dp = seed;
@@ -627,7 +661,7 @@ FM_DEVICE bool fm_x2_dkv(const X2Args& A, fm_half* st, int* bad) {
   ok = ok && (xg.ok || fm_x2_columns(A.sg + int64_t(bh) * A.nbq, A.cg + int64_t(bh) * A.nbq, b0, A.nbq, xg.mx, lane));
   const int eq = FM_UNIFORM(fm_x2_exp(xq.mx * qf, ok)), ev = FM_UNIFORM(fm_x2_exp(xv.mx, ok)), eg = FM_UNIFORM(fm_x2_exp(xg.mx, ok));
   if (!ok) return fm_x2_leave(0);
-  const float qs = qf * fm_x2_pow(eq), gsc = fm_x2_pow(eg), cl = fm_x2_scalb(1.0f, eg + ev);
+  const float qs = qf * fm_x2_pow(eq), gsc = fm_x2_pow(eg), cl = fm_x2_scalb(1.0f, eg + ev), qn = qf * fm_x2_longest(A.lq + int64_t(bh) * A.nbq, A.nbq, lane);
   auto put = [&](int b) FM_ALWAYS_INLINE {
     fm_half* X = st + b * C::STAGE;
     sg.store(X, X + KT * PQ, qs, gsc, true, tid);
@@ -635,6 +669,7 @@ FM_DEVICE bool fm_x2_dkv(const X2Args& A, fm_half* st, int* bad) {
   };
   typename R::Own of, of2;
   X3Coef cp, cd;
+  int ds;
   {
     const bool in = lo + lr < A.nk;
     const int64_t row = in ? lo + lr : A.nk - 1;
@@ -642,10 +677,13 @@ FM_DEVICE bool fm_x2_dkv(const X2Args& A, fm_half* st, int* bad) {
     fm_x2_own<DH>(A.k, bh, row, in, lh, A.sc * kf, v);
     const int ek = fm_x2_row_exp(fm_x2_largest<DH>(v), eq, bad);
     fm_x2_set<DH>(of, v, fm_x2_scalb(1.0f, ek));
+    const float b = qn * fm_x2_norm<DH>(v);
+    fm_x2_weights(A, b, bad);
+    ds = fm_x2_ds_exp(A, b, xv, bad);
     fm_x2_own<DH>(A.v, bh, row, in, lh, fm_x2_pow(ev), v);
     fm_x2_set<DH>(of2, v, 1.0f);
     cp = fm_x2_coef(A.a0, A.a1, A.a2, A.ew, ek + eq);
-    cd = fm_x2_dcoef(A.a1, A.a2, A.ew, ek + eq);
+    cd = fm_x2_dcoef(A.a1, A.a2, A.ew, ds, ek + eq);
   }
   fm_f32x16 acc[NT], av[NT];
 #pragma unroll
@@ -653,10 +691,11 @@ FM_DEVICE bool fm_x2_dkv(const X2Args& A, fm_half* st, int* bad) {
   int buf = 0;
   put(0);
   fetch(s_last - KT);
+  if (fm_x3_again(bad)) return fm_x2_leave(0);         // (the first stage's barrier)
   for (int s0 = s_last; s0 >= sbeg; s0 -= KT) {
     const fm_half* X = st + buf * C::STAGE;
     const fm_half* Y = X + KT * PQ;
-    FM_SYNC();
+    if (s0 < s_last) FM_SYNC();
     const int ss0 = s0 + 32 * sub;
     if (ss0 < A.nq && !(causal && ss0 + 31 < lo)) {
       fm_f32x16 s = fm_zero16(), dp;                   // gh . v starts from -c
@@ -686,7 +725,7 @@ FM_DEVICE bool fm_x2_dkv(const X2Args& A, fm_half* st, int* bad) {
     buf ^= 1;
     if (s0 - KT >= sbeg) { put(buf); fetch(s0 - 2 * KT); }
   }
-  const int edk = -(eg + ev + eq + A.ew + FM_X2_DS), edv = -(eg + A.ew);
+  const int edk = -(eg + ev + eq + A.ew + ds), edv = -(eg + A.ew);
 #pragma unroll
   for (int ct = 0; ct < NT; ++ct)
 #pragma unroll

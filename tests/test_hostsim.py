@@ -540,3 +540,24 @@ def test_two_planes_hold_ordinary_numbers(sim, two_planes, split, mask):
     sim.forward(q, k, v, mask=mask, inv_tau=0.02, p=2, flags=_capi.FLAG_FORCE_DENSE)
     refused, walked = left_two_planes(sim)
     assert refused > 0 and walked == 0
+
+
+@pytest.mark.parametrize("split,mask", [(1, True), (4, False)])
+def test_two_planes_large_scores(sim, two_planes, split, mask):
+    """Scores of plain numbers without a temperature: nothing that two planes make overflows, in the weights or in dS.  Weights that would are
+    left to three planes before any is made."""
+    two_planes(split)
+    left_two_planes(sim)
+    for which in ("q", "v"):
+        q, k, v, go = make_inputs(1, 130, 130, 64, torch.float32, "cpu", 86)
+        q, k = q * 1.5, k * 1.2
+        if which == "v": v[:, 70] *= 50.0              # one token's value far longer than the others'
+        kw = dict(mask=mask, inv_tau=1.0, p=2, flags=_capi.FLAG_FORCE_DENSE)
+        o, g = sim.forward(q, k, v, **kw)
+        grads = sim.backward(q, k, v, o, g, go, **kw)
+        errs = [rel_err(x, r) for x, r in zip((o, g, *grads), oracle_all(q, k, v, go, mask=mask, tau=1.0, p=2))]
+        assert max(errs) < 2e-6, errs
+    assert left_two_planes(sim) == (0, 0)
+    check_forward_backward(sim, 1, 70, 32, torch.float32, "cpu", mask=mask, p=2, seed=87, scale=30.0, flags=_capi.FLAG_FORCE_DENSE)
+    refused, walked = left_two_planes(sim)
+    assert refused > 0 and walked == 0
