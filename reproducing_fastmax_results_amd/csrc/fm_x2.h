@@ -297,19 +297,17 @@ struct X2Args : X3Args<float> {
 };
 // A score is at most the product of its rows' norms: b, the lane's own row with the longest stream row.
 //   weights      one beyond _Float16 would be infinite: the workgroup leaves them to fm_x3.h before it makes any
-//   dS           large derivatives take their size out of dS's power of two (an ordinary product of rows leaves them a factor of 8).  What
-//                that costs the small entries of dS is taken from the spread that v's rows may have.
+//   dS           large derivatives take their size out of dS's power of two (an ordinary product of rows leaves them a factor of 8)
 FM_DEVICE void fm_x2_weights(const X2Args& A, float b, int* bad) {
   const float w = fm_absf(A.a0) + b * (fm_absf(A.a1) + b * fm_absf(A.a2));
   if (!(fm_x2_scalb(w, A.ew) < 65000.0f)) *bad = 1;
 }
-FM_DEVICE int fm_x2_ds_exp(const X2Args& A, float b, const X2Max& v, int* bad) {
+FM_DEVICE int fm_x2_ds_exp(const X2Args& A, float b) {
   const float w = fm_x2_scalb(fm_absf(A.a1) + 2.0f * b * fm_absf(A.a2), A.ew);
   uint32_t u;
   __builtin_memcpy(&u, &w, 4);
-  const int over = int(u >> 23) - 127 - 2, e = over > 0 ? over : 0;
-  if (e > 0 && v.least < v.mx * fm_x2_scalb(FM_X2_SPREAD, e)) *bad = 1;
-  return FM_X2_DS - e;
+  const int over = int(u >> 23) - 127 - 2;
+  return FM_X2_DS - (over > 0 ? over : 0);
 }
 // The polynomials' coefficients: f(s) 2^ew, and f'(s) 2^(ew + ds), s = score 2^-es.
 FM_DEVICE X3Coef fm_x2_coef(float a0, float a1, float a2, int ew, int es) {
@@ -549,7 +547,13 @@ FM_DEVICE bool fm_x2_dq(const X2Args& A, fm_half* st, int* bad) {
     fm_x2_own<DH>(A.q, bh, row, in, lh, A.sc * qf, v);
     const int eq = fm_x2_row_exp(fm_x2_largest<DH>(v), ek, bad);
     fm_x2_set<DH>(of, v, fm_x2_scalb(1.0f, eq));
-    const int ds = fm_x2_ds_exp(A, kn * fm_x2_norm<DH>(v), xv, bad);
+    const int ds = fm_x2_ds_exp(A, kn * fm_x2_norm<DH>(v));
+    if (causal) {
+      // What that costs the small entries of dS is taken from the spread that v's rows may have, where the query sees none but small ones:
+      // the largest of the blocks before its own, or the smallest of all.
+      const float first = fm_x2_join(A.mv + int64_t(bh) * A.nbk, A.sv + int64_t(bh) * A.nbk, 0, fm_x2_block(t0, A.nbk), lane).mx;
+      if (ds < FM_X2_DS && fm_fmaxf(first, xv.least) < xv.mx * fm_x2_scalb(FM_X2_SPREAD, FM_X2_DS - ds)) *bad = 1;
+    }
     fm_x2_own<DH>(A.d_o, bh, row, in, lh, in ? 1.0f / A.g.base(bh)[row * A.g.s_n] : 0.f, v);
     const float* po = A.o.base(bh) + row * A.o.s_n + 8 * lh;
 #pragma unroll
@@ -651,14 +655,11 @@ FM_DEVICE bool fm_x2_dkv(const X2Args& A, fm_half* st, int* bad) {
   fetch(s_last);
   const float kf = fm_norm_factor(A.k_fold, bh, lane), qf = A.sc * fm_norm_factor(A.q_fold, bh, lane);
   const X2Max xq = fm_x2_join(A.mq + int64_t(bh) * A.nbq, A.sq + int64_t(bh) * A.nbq, 0, A.nbq, lane), xv = fm_x2_join(A.mv + int64_t(bh) * A.nbk, A.sv + int64_t(bh) * A.nbk, 0, A.nbk, lane);
-  // gh: of the queries that the block's keys see; what the last key sees has to be within the range of it: the blocks behind its own, or,
-  // where those are zero, the last row of its own that is not (the row before that it may not see)
-  const int tl = (t0 + QW < A.nk ? t0 + QW : A.nk) - 1;
-  const int b0 = causal ? fm_x2_block(t0, A.nbq) : 0, b1 = causal ? fm_x2_block(tl, A.nbq) : 0;
-  const X2Max xg = fm_x2_join(A.mg + int64_t(bh) * A.nbq, A.sg + int64_t(bh) * A.nbq, b0, A.nbq, lane), xl = fm_x2_join(A.mg + int64_t(bh) * A.nbq, A.sg + int64_t(bh) * A.nbq, b1 + 1, A.nbq, lane);
-  const float seen = xl.mx > 0.f ? xl.mx : A.tg[int64_t(bh) * A.nbq + b1];
-  bool ok = xq.ok && xv.ok && !(causal && seen > 0.f && seen < xg.mx * FM_X2_SPREAD);
-  ok = ok && (xg.ok || fm_x2_columns(A.sg + int64_t(bh) * A.nbq, A.cg + int64_t(bh) * A.nbq, b0, A.nbq, xg.mx, lane));
+  // gh: of the queries that the block's keys see
+  const float *mg = A.mg + int64_t(bh) * A.nbq, *sg_ = A.sg + int64_t(bh) * A.nbq;
+  const int b0 = causal ? fm_x2_block(t0, A.nbq) : 0;
+  const X2Max xg = fm_x2_join(mg, sg_, b0, A.nbq, lane);
+  bool ok = xq.ok && xv.ok && (xg.ok || fm_x2_columns(sg_, A.cg + int64_t(bh) * A.nbq, b0, A.nbq, xg.mx, lane));
   const int eq = FM_UNIFORM(fm_x2_exp(xq.mx * qf, ok)), ev = FM_UNIFORM(fm_x2_exp(xv.mx, ok)), eg = FM_UNIFORM(fm_x2_exp(xg.mx, ok));
   if (!ok) return fm_x2_leave(0);
   const float qs = qf * fm_x2_pow(eq), gsc = fm_x2_pow(eg), cl = fm_x2_scalb(1.0f, eg + ev), qn = qf * fm_x2_longest(A.lq + int64_t(bh) * A.nbq, A.nbq, lane);
@@ -679,7 +680,20 @@ FM_DEVICE bool fm_x2_dkv(const X2Args& A, fm_half* st, int* bad) {
     fm_x2_set<DH>(of, v, fm_x2_scalb(1.0f, ek));
     const float b = qn * fm_x2_norm<DH>(v);
     fm_x2_weights(A, b, bad);
-    ds = fm_x2_ds_exp(A, b, xv, bad);
+    ds = fm_x2_ds_exp(A, b);
+    if (causal) {
+      // What the wavefront's keys see of gh falls like 1 / i: the power of two of what its first key sees.  What its last key sees has to be
+      // within the range of that: the blocks of 64 behind its own, or, where those are zero, the last row of its own that is not (the row
+      // before that it may not see).  As dS, 2^-11 less what its scores take (with 2^-14 and tau = 1, where g falls from one query to the next by any
+      // factor: keys 16 - 63 of a head 9e-7 off, 2.3e-7 so); as gh by itself, the range of every tensor.
+      const int last = (lo + 31 < A.nk ? lo + 31 : A.nk - 1), bl = fm_x2_block(last, A.nbq);
+      const X2Max xw = fm_x2_join(mg, sg_, fm_x2_block(lo < last ? lo : last, A.nbq), A.nbq, lane), xl = fm_x2_join(mg, sg_, bl + 1, A.nbq, lane);
+      const float seen = xl.mx > 0.f ? xl.mx : A.tg[int64_t(bh) * A.nbq + bl];
+      if (seen > 0.f && (seen < xw.mx * fm_x2_scalb(0x1p-11f, FM_X2_DS - ds) || seen < xg.mx * FM_X2_SPREAD)) *bad = 1;
+      bool fine = true;
+      const int ew = fm_x2_exp(xw.mx, fine);
+      if (xw.mx > 0.f && fine) ds += ew - eg;
+    }
     fm_x2_own<DH>(A.v, bh, row, in, lh, fm_x2_pow(ev), v);
     fm_x2_set<DH>(of2, v, 1.0f);
     cp = fm_x2_coef(A.a0, A.a1, A.a2, A.ew, ek + eq);

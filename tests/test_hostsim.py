@@ -533,8 +533,10 @@ def test_two_planes_hold_ordinary_numbers(sim, two_planes, split, mask):
     two_planes(split)
     left_two_planes(sim)
     check_forward_backward(sim, 1, 130, 64, torch.float32, "cpu", mask=mask, p=2, seed=83, saved=True, flags=_capi.FLAG_FORCE_DENSE)
-    check_numbers_within_two_planes(sim, 1, 130, 32, "cpu", mask=mask, seed=84)
     assert left_two_planes(sim) == (0, 0)
+    check_numbers_within_two_planes(sim, 1, 130, 32, "cpu", mask=mask, seed=84)
+    refused, walked = left_two_planes(sim)
+    assert walked == 0 and (mask or refused == 0)      # (causal: see test_two_planes_large_scores)
     q, k, v, _ = make_inputs(1, 130, 130, 32, torch.float32, "cpu", 85)
     v[:, 100] *= 1e-9
     sim.forward(q, k, v, mask=mask, inv_tau=0.02, p=2, flags=_capi.FLAG_FORCE_DENSE)
@@ -557,7 +559,25 @@ def test_two_planes_large_scores(sim, two_planes, split, mask):
         grads = sim.backward(q, k, v, o, g, go, **kw)
         errs = [rel_err(x, r) for x, r in zip((o, g, *grads), oracle_all(q, k, v, go, mask=mask, tau=1.0, p=2))]
         assert max(errs) < 2e-6, errs
-    assert left_two_planes(sim) == (0, 0)
+    refused, walked = left_two_planes(sim)
+    assert walked == 0 and (mask or refused == 0)      # (causal: dO / g of the first queries differ by more than large scores leave room for)
     check_forward_backward(sim, 1, 70, 32, torch.float32, "cpu", mask=mask, p=2, seed=87, scale=30.0, flags=_capi.FLAG_FORCE_DENSE)
     refused, walked = left_two_planes(sim)
     assert refused > 0 and walked == 0
+
+
+@pytest.mark.parametrize("split", [1, 4])
+def test_two_planes_one_large_gradient(sim, two_planes, split):
+    """A first query whose weight is small has a dO / g a thousand times the next ones': the keys that do not see it keep the bits of theirs."""
+    q, k, v, go = make_inputs(1, 130, 130, 64, torch.float32, "cpu", 88)
+    q[:, 0] = -k[:, 0] / k[:, 0].pow(2).sum(-1, keepdim=True)
+    kw = dict(mask=True, inv_tau=1.0, p=2, flags=_capi.FLAG_FORCE_DENSE)
+    ref = oracle_all(q, k, v, go, mask=True, tau=1.0, p=2)
+    keys, errs = slice(8, 64), {}
+    for planes in (0, split):
+        two_planes(planes)
+        o, g = sim.forward(q, k, v, **kw)
+        _, dk, dv = sim.backward(q, k, v, o, g, go, **kw)
+        errs[planes] = [rel_err(x[:, keys], r[:, keys]) for x, r in ((dk, ref[3]), (dv, ref[4]))]
+    # two planes and three round alike here, to within the roundings of a few hundred terms
+    assert all(x < 2 * y for x, y in zip(errs[split], errs[0])), errs
