@@ -399,13 +399,23 @@ template <int DH> FM_DEVICE float fm_x2_largest(const float (*v)[8]) {
     for (int i = 0; i < 8; ++i) m = fm_fmaxf(m, fm_absf(v[c][i]));
   return fm_fmaxf(m, fm_shfl_xor(m, 32));
 }
-template <int DH> FM_DEVICE void fm_x2_set(typename X2Row<DH>::Own& o, const float (*v)[8], float f) {
+// Own rows, times f.  A quarter of the numbers lie half way between two that the planes hold, and what rounding does to an own row is the same
+// for every stream token: it does not average out where the tokens have something in common.  So of the wavefronts that share an own tile every
+// other one (other) rounds such numbers the other way, and what is left meets its opposite in the sums.
+template <int DH> FM_DEVICE void fm_x2_set(typename X2Row<DH>::Own& o, const float (*v)[8], float f, bool other) {
 #pragma unroll
   for (int c = 0; c < DH / 16; ++c) {
     float w[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) w[i] = v[c][i] * f;
     o.f[c] = fm_x2_split(w);
+    if (other) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float l = fm_x2_minus(w[i], o.f[c].h[i]);
+        o.f[c].l[i] = fm_half(l + (l - float(o.f[c].l[i])));
+      }
+    }
   }
 }
 
@@ -440,7 +450,7 @@ FM_DEVICE bool fm_x2_fwd(const X2Args& A, fm_half* st, int* bad) {
     const bool in = lo + lr < A.nq;
     fm_x2_own<DH>(A.q, bh, in ? lo + lr : A.nq - 1, in, lh, qs, v);
     const int eq = fm_x2_row_exp(fm_x2_largest<DH>(v), ek, bad);
-    fm_x2_set<DH>(of, v, fm_x2_scalb(1.0f, eq));
+    fm_x2_set<DH>(of, v, fm_x2_scalb(1.0f, eq), SPLIT > 1 && (sub & 1));
     cf = fm_x2_coef(A.a0, A.a1, A.a2, A.ew, eq + ek);
     fm_x2_weights(A, kn * fm_x2_norm<DH>(v), bad);
   }
@@ -546,7 +556,7 @@ FM_DEVICE bool fm_x2_dq(const X2Args& A, fm_half* st, int* bad) {
     float v[DH / 16][8];
     fm_x2_own<DH>(A.q, bh, row, in, lh, A.sc * qf, v);
     const int eq = fm_x2_row_exp(fm_x2_largest<DH>(v), ek, bad);
-    fm_x2_set<DH>(of, v, fm_x2_scalb(1.0f, eq));
+    fm_x2_set<DH>(of, v, fm_x2_scalb(1.0f, eq), SPLIT > 1 && (sub & 1));
     const int ds = fm_x2_ds_exp(A, kn * fm_x2_norm<DH>(v));
     if (causal) {
       // What that costs the small entries of dS is taken from the spread that v's rows may have, where the query sees none but small ones:
@@ -566,7 +576,7 @@ FM_DEVICE bool fm_x2_dq(const X2Args& A, fm_half* st, int* bad) {
     bool fine = true;
     const int eg = fm_x2_exp(fm_x2_largest<DH>(v), fine);
     if (!fine) *bad = 1;
-    fm_x2_set<DH>(of2, v, fm_x2_pow(eg));
+    fm_x2_set<DH>(of2, v, fm_x2_pow(eg), SPLIT > 1 && (sub & 1));
     cs += fm_shfl_xor(cs, 32);
     if (sub == 0 && lh == 0 && in) A.cv[int64_t(bh) * A.npad_q + row] = cs;
     cs = fm_x2_scalb(cs, eg + ev);                     // as gh . v
@@ -677,7 +687,7 @@ FM_DEVICE bool fm_x2_dkv(const X2Args& A, fm_half* st, int* bad) {
     float v[DH / 16][8];
     fm_x2_own<DH>(A.k, bh, row, in, lh, A.sc * kf, v);
     const int ek = fm_x2_row_exp(fm_x2_largest<DH>(v), eq, bad);
-    fm_x2_set<DH>(of, v, fm_x2_scalb(1.0f, ek));
+    fm_x2_set<DH>(of, v, fm_x2_scalb(1.0f, ek), SPLIT > 1 && (sub & 1));
     const float b = qn * fm_x2_norm<DH>(v);
     fm_x2_weights(A, b, bad);
     ds = fm_x2_ds_exp(A, b);
@@ -695,7 +705,7 @@ FM_DEVICE bool fm_x2_dkv(const X2Args& A, fm_half* st, int* bad) {
       if (xw.mx > 0.f && fine) ds += ew - eg;
     }
     fm_x2_own<DH>(A.v, bh, row, in, lh, fm_x2_pow(ev), v);
-    fm_x2_set<DH>(of2, v, 1.0f);
+    fm_x2_set<DH>(of2, v, 1.0f, SPLIT > 1 && (sub & 1));
     cp = fm_x2_coef(A.a0, A.a1, A.a2, A.ew, ek + eq);
     cd = fm_x2_dcoef(A.a1, A.a2, A.ew, ds, ek + eq);
   }

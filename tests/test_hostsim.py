@@ -581,3 +581,22 @@ def test_two_planes_one_large_gradient(sim, two_planes, split):
         errs[planes] = [rel_err(x[:, keys], r[:, keys]) for x, r in ((dk, ref[3]), (dv, ref[4]))]
     # two planes and three round alike here, to within the roundings of a few hundred terms
     assert all(x < 2 * y for x, y in zip(errs[split], errs[0])), errs
+
+
+@pytest.mark.parametrize("split", [2, 4])
+def test_two_planes_tokens_with_something_in_common(sim, two_planes, split):
+    """Every token of q, k, v and dO has a part that all others share: the rounding of an own row does not average out over those.  dk and g
+    are held to what three planes, which do not round it, leave of the sums' roundings."""
+    d, tau = 32, 8.0 * math.sqrt(32)
+    x = make_inputs(1, 256, 256, d, torch.float32, "cpu", 1)
+    gen = torch.Generator().manual_seed(51)
+    q, k, v, go = (t + 4 * torch.randn(1, 1, d, generator=gen) for t in x)
+    kw = dict(mask=False, inv_tau=1.0 / tau, p=2, flags=_capi.FLAG_FORCE_DENSE)
+    ref = oracle_all(q, k, v, go, mask=False, tau=tau, p=2)
+    errs = {}
+    for planes in (0, split):
+        two_planes(planes)
+        o, g = sim.forward(q, k, v, **kw)
+        _, dk, _ = sim.backward(q, k, v, o, g, go, **kw)
+        errs[planes] = [rel_err(g, ref[1]), rel_err(dk, ref[3])]
+    assert all(x < 1.5 * y for x, y in zip(errs[split], errs[0])), errs
