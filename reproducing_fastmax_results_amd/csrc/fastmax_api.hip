@@ -126,23 +126,21 @@ inline bool is_small(const FastmaxDesc* d) {
 inline bool half_arithmetic(const FastmaxDesc* d) {
   return d->dtype == FASTMAX_BF16 && !(d->flags & FASTMAX_FLAG_F32_COMPUTE) && d->a0 > 0.0f;
 }
-// Unmasked attention: one total of the moments costs less than products with every key.  In fp32 arithmetic not before the dense tiles
-// (fm_x2.h; fm_x3.h for bf16 tensors computed in fp32) fill the chip: the states are summed by a few workgroups per batch*head, one chain over
-// the keys, and their matrix products are fp32's.  Forward and backward on states and on tiles, microseconds, fp32 tensors, order 2: D = 32, 2
+// Unmasked attention: one total of the moments costs less than products with every key.  In fp32 arithmetic of order 2 not before the dense
+// tiles (fm_x2.h; fm_x3.h for bf16 tensors computed in fp32) fill the chip: the states are summed by a few workgroups per batch*head, one chain over
+// the keys, and their matrix products are fp32's.  Forward and backward on states and on tiles, microseconds, fp32 tensors: D = 32, 2
 // heads of 1100 keys 100 and 159, 22 and 56, 28 of 2200 172 and 273, 79 and 252, 8 of 5700 352 and 454, 158 and 451, 4 of 9000 526 and 629, 218 and 684;
-// D = 64, 2 of 4300 569 and 880, 70 and 188, 15 of 4300 690 and 1334, 247 and 798, 4 of 14000 1693 and 2339, 642 and 2235.  Order 1: D = 32, 7 of 2000
-// 92 and 121, 32 and 76, 32 of 3000 148 and 198, 149 and 415; D = 64, 3 of 5000 467 and 531, 95 and 252.  bf16 tensors, order 2: D = 32, 4 of 4096 248
-// and 312, 145 and 259, 4 of 5700 343 and 410, 289 and 584; D = 64, 8 of 4300 676 and 1289, 364 and 977, 4 of 9000 1183 and 1799, 745 and 2069;
-// order 1, D = 32, 3 of 4000 167 and 209, 139 and 250.  On a full chip the tiles of fm_x2.h are faster for a while too, but one accumulator loses more of
-// thousands of terms there than the states do (64 heads of 2000, D = 32: error of dq 5.2e-7, 4.4e-7).
+// D = 64, 2 of 4300 569 and 880, 70 and 188, 15 of 4300 690 and 1334, 247 and 798, 4 of 14000 1693 and 2339, 642 and 2235.  bf16 tensors: D = 32, 4 of 4096 248
+// and 312, 145 and 259, 4 of 5700 343 and 410, 289 and 584; D = 64, 8 of 4300 676 and 1289, 364 and 977, 4 of 9000 1183 and 1799, 745 and 2069.  On a
+// full chip the tiles of fm_x2.h are faster for a while too, but one accumulator loses more of thousands of terms there than the states do
+// (64 heads of 2000, D = 32: error of dq 5.2e-7, 4.4e-7).
 inline bool states_pay_unmasked(const FastmaxDesc* d) {
   if (int64_t(d->nk) <= int64_t(d->d) * d->d + d->d) return false;
-  const bool quad = d->p == 2 && d->a2 != 0.0f;
   int ew;
-  const bool x2 = d->dtype == FASTMAX_F32 && x2_coefficients(d->a0, d->a1, quad ? d->a2 : 0.0f, ew);
-  if (half_arithmetic(d) || d->d > 64 || !(x2 || quad)) return true;
+  if (half_arithmetic(d) || d->d > 64 || d->p != 2 || d->a2 == 0.0f) return true;
+  const bool x2 = d->dtype == FASTMAX_F32 && x2_coefficients(d->a0, d->a1, d->a2, ew);
   const int64_t blocks = d->bh * ((int64_t(d->nq > d->nk ? d->nq : d->nk) + 127) / 128);
-  return blocks >= (quad ? 512 : 128) || d->bh * int64_t(d->nq) * d->nk > int64_t(1) << ((d->d == 64 ? 30 : 28) - (x2 ? 0 : 2));
+  return blocks >= 512 || d->bh * int64_t(d->nq) * d->nk > int64_t(1) << ((d->d == 64 ? 30 : 28) - (x2 ? 0 : 2));
 }
 
 // How many wavefronts share an own tile in the fp32 kernels of dense tiles (fm_x3.h, fm_x2.h): with one each, a launch has blocks of 128

@@ -22,7 +22,7 @@
 // The powers are taken out of the polynomials' coefficients and of the sums, exactly.
 //
 // Which problems these kernels may take is decided in two places.  x2_coefficients (host): a0 > 0, a1 of its
-// size and a2 no larger than that.  k_x2_range and its readers, per batch*head: the largest entry of every row and every column of
+// size and weights that do not change their sign.  k_x2_range and its readers, per batch*head: the largest entry of every row and every column of
 // a block of 64 tokens that is not zero is at least 2^-14 of the tensor's largest, and so is held to 2^-25 of itself.  (gh: whole rows
 // and blocks may be smaller, they add little to sums over rows; a column may not lie in them alone.)  A workgroup whose tensors do not
 // keep to that, one whose weights may pass 65504 (fm_x2_weights) and one with a sum that is not finite make their rows as fm_x3.h does (and so,
@@ -318,11 +318,14 @@ FM_DEVICE X3Coef fm_x2_dcoef(float a1, float a2, int ew, int ds, int es) {
   const X3Coef c = {0.f, fm_x2_scalb(a1, ew + ds), fm_x2_scalb(2.0f * a2, ew + ds - es)};
   return c;
 }
-// Coefficients that these kernels take; ew as above.  (A score too small to be seen beside a0 is the whole of f'(s) where a1 is zero.)
+// Coefficients that these kernels take; ew as above.  A score too small to be seen beside a0 is the whole of f'(s) where a1 is zero.  And f(s) is
+// to stay away from zero (a0 / 2 at least: a1^2 <= 2 a0 a2, as the Taylor weights have it): weights of both signs cancel in the denominators and
+// leave the roundings of the scores, which are two planes' there.  (Order 1, q and k with a common component that takes weights through zero,
+// 176 heads of 780 tokens: o off by 9e-5, three planes 1.3e-5; 32 of 7000, D = 32, 3e-4 and 5e-5.)
 inline bool x2_coefficients(float a0, float a1, float a2, int& ew) {
-  const float b1 = std::fabs(a1), b2 = std::fabs(a2), big = b1 > b2 ? b1 : b2;
+  const float b1 = std::fabs(a1), big = b1 > a2 ? b1 : a2;
   ew = 0;
-  if (!(a0 > 0x1p-40f && a0 < 0x1p40f) || !(big <= 16.0f * a0) || !(b1 >= a0 * 0.0625f)) return false;
+  if (!(a0 > 0x1p-40f && a0 < 0x1p40f) || !(big <= 16.0f * a0) || !(b1 >= a0 * 0.0625f) || !(b1 * b1 <= 2.0f * a0 * a2)) return false;
   int e;
   std::frexp(a0, &e);
   ew = 1 - e;

@@ -600,3 +600,21 @@ def test_two_planes_tokens_with_something_in_common(sim, two_planes, split):
         _, dk, _ = sim.backward(q, k, v, o, g, go, **kw)
         errs[planes] = [rel_err(g, ref[1]), rel_err(dk, ref[3])]
     assert all(x < 1.5 * y for x, y in zip(errs[split], errs[0])), errs
+
+
+def test_two_planes_weights_of_both_signs(sim, two_planes):
+    """Order 1, scores around -1: the weights cancel in the denominators and leave the roundings of the scores (two planes in one wavefront
+    per tile: o off by 1.1e-4 where three give 1.9e-5), so such coefficients keep the three planes: the same bits."""
+    d, tau = 32, 8.0 * math.sqrt(32)
+    q, k, v, go = make_inputs(1, 130, 130, d, torch.float32, "cpu", 4)
+    qc, kc = 4 * torch.randn(2, d, generator=torch.Generator().manual_seed(54))
+    q, k = q + qc, k + kc - qc * ((qc @ kc + tau) / (qc @ qc))      # q . k = -tau on average
+    kw = dict(mask=False, inv_tau=1.0 / tau, p=1, a2=0.0, flags=_capi.FLAG_FORCE_DENSE)
+    got = []
+    for planes in (0, 4):                              # (so few tokens are shared by four wavefronts in any case)
+        two_planes(planes)
+        o, g = sim.forward(q, k, v, **kw)
+        got.append((o, g, *sim.backward(q, k, v, o, g, go, **kw)))
+    assert all(torch.equal(x, y) for x, y in zip(*got))
+    ref = oracle_all(q, k, v, go, mask=False, tau=tau, p=1, a=(1.0, 1.0, 0.0))
+    assert rel_err(got[0][0], ref[0]) < 1e-4
