@@ -181,26 +181,32 @@ inline int x2_rows(int kind, int split, int bh, int n_own) {
   return 256 / split;
 }
 
-// dK + dV of long causal problems on fm_x2.h: two wavefronts to an own tile at least, whose sums are half as long.
+// Own tiles of long causal problems on fm_x2.h: shared by more wavefronts than a full chip asks for, whose sums are shorter.  Where the tokens share
+// a component, sums of 8192 have their own size at every step and their roundings add up: dv 2.6e-7 off with two wavefronts to a tile, 1.3e-7 with
+// four, states 1.3 - 2.2e-7 (backward of 16 heads 1290, 1420 us, states 3420); o at D = 32, 7000 tokens, 3.1e-7 with one, 1.6e-7 with two, states
+// 2.6e-7 (forward of 32 heads 354, 355 us); at D = 64 the forward adds its sums up in parts of 1024 by itself.
 inline int x2_key_split(const FastmaxDesc* d) {
-  const int s = x3_split(d->bh, d->nk, 256);
-  return s == 1 && d->mask && d->nq > 6144 ? 2 : s;
+  return d->mask && d->nq > 6144 ? 4 : x3_split(d->bh, d->nk, 256);
+}
+inline int x2_forward_split(const FastmaxDesc* d) {
+  const int s = x3_split(d->bh, d->nq, 128);
+  return s == 1 && d->d == 32 && d->mask && d->nq > 6144 ? 2 : s;
 }
 // Causal problems in fp32 arithmetic that keep dense tiles past the lengths at which _Float16 ones go to states (see make_plan): the state
 // kernels' products are fp32's, a sixth of the rate of fm_x2.h's.  Forward and backward on states and on tiles, microseconds: order 2,
-// D = 64, fp32 tensors, 16 heads of 8192 1419 and 3254, 402 and 1272, 2 of 6200 316 and 865, 96 and 265, 4 of 16000 862 and 1935, 416 and 1365, 2 of 32000
-// 857 and 1902, 788 and 2646; D = 32, 16 of 7000 303 and 716, 206 and 570, 128 of 7000 1813 and 4489, 1311 and 4485, 4 of 12000 191 and 470, 197 and
-// 492.  bf16 tensors (fm_x3.h), D = 64, 16 of 7000 1200 and 2735, 481 and 1578, 3 of 8192 434 and 976, 472 and 914.  The limits are also where the
-// tiles' error against 64 bits is below the states': D = 64, 8192 tokens, o, dq, dk, dv 3.0, 4.7, 4.9, 3.3e-7 and 2.0, 4.0, 3.1, 2.6e-7 (dv 3.5e-7 with one
-// wavefront to an own tile: x2_key_split); a full chip's dq is past it from about 10000 tokens.  Order 1 keeps its 1024: at 1280 tokens the tiles
-// are faster for few heads and for many, not between (24 heads 65 and 153, 84 and 178).
+// D = 64, fp32 tensors, 16 heads of 8192 1450 and 3420, 397 and 1420, 2 of 6200 316 and 865, 96 and 265; D = 32, 16 of 7000 303 and 716, 206 and 570, 32
+// of 7000 612 and 1390, 355 and 1230, 4 of 12000 191 and 470, 197 and 492.  bf16 tensors (fm_x3.h), D = 64, 16 of 7000 1200 and 2735, 481 and 1578, 3 of
+// 8192 434 and 976, 472 and 914.  The limits are also where the tiles' error against 64 bits is below the states': D = 64, 8192 tokens, o, dq, dk, dv
+// 2.6, 4.1, 4.4, 2.8e-7 and 1.6, 4.0, 2.6, 1.9e-7, with a component that all tokens share 1.6, 52, 45, 1.3e-7 and 1.1, 11, 8.3, 1.3e-7; of 16000 tokens
+// dv is past it (1.0 and 1.8e-7).  Order 1 keeps its 1024: at 1280 tokens the tiles are faster for few heads and for many, not between (24 heads 65 and
+// 153, 84 and 178).
 inline bool tiles_pay_causal(const FastmaxDesc* d) {
   int ew;
   const int64_t n = d->nq;
   if (half_arithmetic(d) || d->p != 2 || d->a2 == 0.0f || d->d > 64) return false;
   if (d->dtype != FASTMAX_F32) return d->d == 64 && n <= 7168;
   if (!x2_coefficients(d->a0, d->a1, d->a2, ew)) return false;
-  return d->d == 64 ? n <= 8192 || (n <= 16384 && d->bh * ((n + 127) / 128) < 512) : n <= 7168;
+  return n <= (d->d == 64 ? 8192 : 7168);
 }
 
 int validate(const FastmaxDesc* d) {
@@ -289,7 +295,7 @@ int make_plan(const FastmaxDesc* d, Plan& p) {
   p.x3 = !p.half && !p.use_state && !p.tiny;
   p.x2_ew = 0;
   const bool x2_fits = p.x3 && d->dtype == FASTMAX_F32 && x2_coefficients(p.a0, p.a1, p.a2, p.x2_ew);
-  p.x2 = x2_fits && x2_pays(d, x3_split(d->bh, d->nq, 128), x2_key_split(d));
+  p.x2 = x2_fits && x2_pays(d, x3_split(d->bh, d->nq, 128), x3_split(d->bh, d->nk, 256));
   p.o1 = p.half && p.use_state && !p.quad && d->mask && p.L == FM_O1_SEG && d->nq == d->nk;
   p.rows_build = p.half && p.use_state && !p.quad && d->mask;
   {
@@ -816,7 +822,7 @@ int run_forward(const FastmaxDesc* d, const Plan& p, const void* q, const void* 
         // (a backward on this workspace reads q's as well)
         const int st = launch_x2_range<DH>(d, p.save ? q : nullptr, k, v, nullptr, nullptr, reinterpret_cast<float*>(ws + p.x2r), nullptr, a, stream);
         if (st) return st;
-        return launch_x2<DH, 0>(a, x3_split(d->bh, d->nq, 128), d->nq, d->bh, stream);
+        return launch_x2<DH, 0>(a, x2_forward_split(d), d->nq, d->bh, stream);
       }
     }
     if (p.x3) {

@@ -439,6 +439,44 @@ def test_numbers_within_two_planes(lib, bh, n, d, mask):
     check_numbers_within_two_planes(lib, bh, n, d, DEV, mask=mask, seed=144)
 
 
+def fp32_errors(lib, q, k, v, go, heads, **kw):
+    """Relative errors of o, g, dq, dk, dv of some heads against 64-bit results on the GPU (order 2, Taylor weights)."""
+    o, g, ws = lib.forward(q, k, v, save=True, **kw)
+    got = (o, g, *lib.backward(q, k, v, o, g, go, saved=ws, **kw))
+    num, den = [0.0] * 5, [0.0] * 5
+    for b in heads:
+        Q, K, V, G = (t[b].double() for t in (q, k, v, go))
+        s = Q @ K.T * kw["inv_tau"]
+        w = 1.0 + s + 0.5 * s * s
+        if kw["mask"]:
+            w = w.tril()
+        gs = w.sum(1, keepdim=True)
+        out, gh = w @ V / gs, G / gs
+        ds = (1.0 + s) * (gh @ V.T - (gh * out).sum(1, keepdim=True))
+        if kw["mask"]:
+            ds = ds.tril()
+        for i, (x, r) in enumerate(zip(got, (out, gs[:, 0], ds @ K * kw["inv_tau"], ds.T @ Q * kw["inv_tau"], w.T @ gh))):
+            num[i] += float((x[b].double() - r).norm() ** 2)
+            den[i] += float(r.norm() ** 2)
+    return [(x / y) ** 0.5 for x, y in zip(num, den)]
+
+
+@pytest.mark.parametrize("bh,n,d", [(9, 8192, 64), (16, 8192, 64), (32, 7000, 32)])
+@pytest.mark.parametrize("common", [0.0, 1.0])
+def test_long_causal_fp32_is_no_less_accurate_than_on_states(lib, bh, n, d, common):
+    """Problems that dense tiles keep past the length at which states begin: each error no larger than the states', also where all tokens
+    share a component (one standard deviation) and the sums' roundings add up.  A tenth above is what two sets of roundings differ by."""
+    print(f"case long causal fp32 against states bh={bh} n={n} d={d} common={common}", flush=True)
+    x = make_inputs(bh, n, n, d, torch.float32, DEV, 145)
+    gen = torch.Generator().manual_seed(146)
+    q, k, v, go = (t + common * torch.randn(1, 1, d, generator=gen).to(DEV) for t in x)
+    kw = dict(mask=True, inv_tau=1.0 / (8.0 * d ** 0.5), p=2)
+    tiles = fp32_errors(lib, q, k, v, go, (0, bh - 1), **kw)
+    states = fp32_errors(lib, q, k, v, go, (0, bh - 1), **kw, flags=FLAG_FORCE_MOMENTS, chunk=1024)
+    print("errors o g dq dk dv, tiles", " ".join(f"{e:.2e}" for e in tiles), "states", " ".join(f"{e:.2e}" for e in states), flush=True)
+    assert all(x < 1.1 * y for x, y in zip(tiles, states)), (tiles, states)
+
+
 @pytest.mark.parametrize("d", [32, 64])
 @pytest.mark.parametrize("bh", [3, 256, 512])
 def test_infinite_and_largest_values_on_fp32_dense_tiles(lib, d, bh):
