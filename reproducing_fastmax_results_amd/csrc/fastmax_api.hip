@@ -160,20 +160,19 @@ inline int x3_split(int bh, int n_own, int tokens) {
 }
 // Dense fp32 problems for the kernels of fm_x2.h: not before their error against 64 bits is no larger than that of fm_x3.h's.  Two planes
 // round an operand once more, three products round the sums half as often as six, so sums of enough terms decide it, and
-// sums spread over several wavefronts (sq, sk: x3_split) need more.  Both sides' errors, ratios of o, dq, dk, dv: causal, D = 64, one
-// and two wavefronts per own tile for dQ and dK + dV, 512 tokens .79 .97 1.03 .98, 777 .70 .86 .91 .91; one and one, 1024 .64 .85 .86 .83, 4096
-// .48 .74 .74 .72; two and four, 1024 .83 .96 1.00 1.05, 1536 .75 .94 .98 .97; four, 1536 .93 1.02 1.00 1.03, 2048 .86 .99 .97 .99.  D = 32: one and two,
-// 777 .71 .92 .99 .88; two and four, 2048 .69 .96 1.03 .92, 3000 .63 .88 .98 .89; four, 2048 .86 1.04 1.03 .97, 3000 .79 .99 1.00 .94.  Unmasked: four, 300 keys
-// .88 .98 .99 .99; one, 300 .67 .91 1.00 .93, but the pass over the ranges costs small forwards more than it gains (D = 64, 16 heads of 400
-// keys 21.4, 24.5 us, 8 of 700 23.0, 23.8; D = 32, 8 of 1000 20.8, 23.9, 32 of 700 40, 28).
+// sums spread over several wavefronts (sq, sk: x3_split) need more.  Largest ratio of the errors of o, dq, dk, dv, N(0, 1) tokens with tau = 8 sqrt(D),
+// sqrt(D) and 1, causal: D = 64, 32 heads of 4096 .87, 64 of 2000 .93, 12 of 4096 .96, 4 of 4096 .97, 4 of 2100 1.07 (dk), but 128 of 1030 1.26 (dq, tau = 1;
+// .97 with the others); D = 32, 64 of 2000 .96, 4 of 3100 1.08 (dk), but 128 of 1030 1.03 and 176 of 780 1.13; unmasked at most .88.  Tokens with a common
+// component, uniform, repeated or of mixed sizes: at most 1.0 but dk, where v and dO have one, 1.15 for 4 of 2100.
+// Unmasked, the pass over the ranges costs small forwards more than it gains (D = 64, 16 heads of 400 keys 21.4, 24.5 us, 8 of 700 23.0, 23.8; D = 32, 8 of
+// 1000 20.8, 23.9, 32 of 700 40, 28).
 inline bool x2_pays(const FastmaxDesc* d, int sq, int sk) {
 #if defined(FM_HOSTSIM)
   if (fm_hostsim_x2) return true;
 #endif
   const int n = d->nq < d->nk ? d->nq : d->nk;
   if (!d->mask) return n >= 640 && int64_t(d->bh) * d->nq * d->nk * d->d >= int64_t(1) << 28;
-  if (sk < 4) return n >= 768;
-  return n >= (d->d == 32 ? 3000 : sq < 4 ? 1536 : 2048);
+  return n >= (sk < 4 || (sq < 4 && d->d == 64) ? 1536 : d->d == 64 ? 2048 : 3000);
 }
 // own tokens of a workgroup there
 inline int x2_rows(int kind, int split, int bh, int n_own) {
@@ -187,6 +186,13 @@ inline int x2_rows(int kind, int split, int bh, int n_own) {
 // 2.6e-7 (forward of 32 heads 354, 355 us); at D = 64 the forward adds its sums up in parts of 1024 by itself.
 inline int x2_key_split(const FastmaxDesc* d) {
   return d->mask && d->nq > 6144 ? 4 : x3_split(d->bh, d->nk, 256);
+}
+// whether the first block of queries goes to three planes (see fm_x2_dq)
+inline int x2_first(const FastmaxDesc* d, int split) {
+#if defined(FM_HOSTSIM)
+  if (fm_hostsim_x2) return d->mask && split == 4;     // (the first block of fewer wavefronts is all that a test's problem has)
+#endif
+  return d->mask && (split > 1 || d->nq < 4096);
 }
 inline int x2_forward_split(const FastmaxDesc* d) {
   const int s = x3_split(d->bh, d->nq, 128);
@@ -662,7 +668,7 @@ template <typename TIO> X3Args<TIO> x3_args(const FastmaxDesc* d, const Plan& p,
   a.cv = nullptr; a.out_resid = nullptr; a.ores = nullptr; a.bpart = nullptr;
   a.nq = d->nq; a.nk = d->nk; a.npad_q = p.npad_q; a.causal = d->mask != 0;
   a.a0 = p.a0; a.a1 = p.a1; a.a2 = p.a2; a.sc = p.sc;
-  a.plain = fm_x3_coef_lost(p.a1, p.a2);
+  a.plain = fm_x3_coef_lost(p.a1, p.a2); a.first = 0;
   a.q_fold = q_fold(d); a.k_fold = k_fold(d);
   return a;
 }
@@ -817,12 +823,13 @@ int run_forward(const FastmaxDesc* d, const Plan& p, const void* q, const void* 
       if (p.x2) {
         X2Args a;
         static_cast<X3Args<float>&>(a) = x3_args<float>(d, p, q, k, v);
-        a.ew = p.x2_ew;
+        const int split = x2_forward_split(d);
+        a.ew = p.x2_ew; a.first = x2_first(d, split);
         a.out = mref<TIO>(o, d->so); a.g = mref<float>(g, d->sg);
         // (a backward on this workspace reads q's as well)
         const int st = launch_x2_range<DH>(d, p.save ? q : nullptr, k, v, nullptr, nullptr, reinterpret_cast<float*>(ws + p.x2r), nullptr, a, stream);
         if (st) return st;
-        return launch_x2<DH, 0>(a, x2_forward_split(d), d->nq, d->bh, stream);
+        return launch_x2<DH, 0>(a, split, d->nq, d->bh, stream);
       }
     }
     if (p.x3) {

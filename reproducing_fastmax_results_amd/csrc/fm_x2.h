@@ -434,9 +434,10 @@ FM_DEVICE bool fm_x2_fwd(const X2Args& A, fm_half* st, int* bad) {
   const int wave = FM_UNIFORM(tid >> 6), own = wave / SPLIT, sub = wave % SPLIT;
   const bool causal = A.causal != 0;
   int blk, bh;
-  fm_x3_place(causal, C::SLOTS, blk, bh);
+  fm_x3_place(causal, A.first != 0, C::SLOTS, blk, bh);
   const int t0 = blk * QW, lo = t0 + 32 * own;
   const int send = causal && t0 + QW < A.nk ? t0 + QW : A.nk;
+  if (A.first && blk == 0) return fm_x2_leave(0);      // see fm_x2_dq
   typedef X2Stage<DH, KT, C::NTH> Stage;
   Stage sg;
   sg.load(A.k, A.v, nullptr, bh, 0, A.nk, tid);
@@ -549,9 +550,15 @@ FM_DEVICE bool fm_x2_dq(const X2Args& A, fm_half* st, int* bad) {
   const int wave = FM_UNIFORM(tid >> 6), own = wave / SPLIT, sub = wave % SPLIT;
   const bool causal = A.causal != 0;
   int blk, bh;
-  fm_x3_place(causal, C::SLOTS, blk, bh);
+  fm_x3_place(causal, A.first != 0, C::SLOTS, blk, bh);
   const int t0 = blk * QW, lo = t0 + 32 * own;
   const int send = causal && t0 + QW < A.nk ? t0 + QW : A.nk;
+  // Causal: the first queries have most of dq and, seen by the first keys, of dk, in few terms, which are as well rounded as their operands: gh . (v - o)
+  // is small beside both factors there.  The first block of queries is short work, so it keeps three planes, forward and here, and starts first.
+  // Without a temperature, errors of dq, dk, dv and three planes': 4 heads of 4096 tokens 3.1, 3.3, 2.8e-7, 2.7, 2.8, 2.6e-7, now 2.5, 2.6, 2.4e-7, 64 of
+  // 2000 3.8, 5.1, 3.4e-7, 4.0, 4.0, 3.3e-7, now 3.5, 3.7, 3.0e-7.  Not where one wavefront sums 4096 tokens and more, whose roundings hide it (32 heads of
+  // 4096: 3.8, 3.9, 3.7e-7, three planes 4.5, 4.4, 4.1e-7; step 866 us, with the block 881).
+  if (A.first && blk == 0) return fm_x2_leave(0);
   typedef X2Stage<DH, KT, C::NTH> Stage;
   Stage sg;
   sg.load(A.k, A.v, nullptr, bh, 0, A.nk, tid);
@@ -665,7 +672,7 @@ FM_DEVICE bool fm_x2_dkv(const X2Args& A, fm_half* st, int* bad) {
   const int wave = FM_UNIFORM(tid >> 6), own = wave / SPLIT, sub = wave % SPLIT;
   const bool causal = A.causal != 0;
   int blk, bh;
-  fm_x3_place(false, C::SLOTS, blk, bh);
+  fm_x3_place(false, false, C::SLOTS, blk, bh);
   const int t0 = blk * QW, lo = t0 + 32 * own;
   const int sbeg = causal ? t0 : 0, nst = (A.nq - sbeg + KT - 1) / KT;
   const int s_last = sbeg + (nst - 1) * KT;            // the stream is walked from its end: see k_ds

@@ -263,6 +263,7 @@ template <typename TIO> struct X3Args {
   int nq, nk, npad_q, causal;
   float a0, a1, a2, sc;                 // sc = sqrt(1/tau), on q and on k
   int plain;                            // see fm_x3_coef_lost
+  int first;                            // causal, own queries: block 0 starts first, on three planes (see fm_x2_dq)
   NormFold q_fold, k_fold;
   float* bpart;                         // the Jacobian's partial sums (see TokArgs::bpart), or null
 };
@@ -326,7 +327,7 @@ template <typename TIO, int DH, typename R, int ROWS, int NTH> struct X3Stage {
 
 // Block of own tokens and batch*head of a workgroup: heaviest blocks first (late queries, early keys under the causal
 // mask); with a multiple of eight batch*heads all blocks of one run behind one L2, dealt as in TokGeom.
-FM_DEVICE void fm_x3_place(bool late_first, int slots, int& blk, int& bh) {
+FM_DEVICE void fm_x3_place(bool late_first, bool zero_first, int slots, int& blk, int& bh) {
   const int nblk = FM_GDIM_X, nbh = FM_GDIM_Y, id = FM_BID_X + nblk * FM_BID_Y;
   int unit;
   if ((nbh & 7) == 0) {
@@ -337,7 +338,7 @@ FM_DEVICE void fm_x3_place(bool late_first, int slots, int& blk, int& bh) {
     unit = id / nbh;
     bh = id % nbh;
   }
-  blk = late_first ? nblk - 1 - unit : unit;
+  blk = !late_first ? unit : !zero_first ? nblk - 1 - unit : unit == 0 ? 0 : nblk - unit;
 }
 
 // rows of the stream tile (starting at s0) that the lane's own token (lo + lr) may see
@@ -472,7 +473,7 @@ FM_DEVICE void fm_x3_fwd(const X3Args<TIO>& A, uint16_t* st, int* bad, const int
   const int wave = FM_UNIFORM(tid >> 6), own = wave / SPLIT, sub = wave % SPLIT;
   const bool causal = A.causal != 0;
   int blk, bh;
-  fm_x3_place(causal, C::SLOTS, blk, bh);
+  fm_x3_place(causal, A.first != 0, C::SLOTS, blk, bh);
   const int t0 = blk * QW, lo = t0 + 32 * own;
   const float qs = A.sc * fm_norm_factor(A.q_fold, bh, lane) * R::UP, ks_ = A.sc * fm_norm_factor(A.k_fold, bh, lane) * R::UP;
   const X3Coef cf = fm_x3_coef<R>(A.a0, A.a1, A.a2);
@@ -584,7 +585,7 @@ FM_DEVICE void fm_x3_dq(const X3Args<TIO>& A, uint16_t* st, int* bad, const int 
   const int wave = FM_UNIFORM(tid >> 6), own = wave / SPLIT, sub = wave % SPLIT;
   const bool causal = A.causal != 0;
   int blk, bh;
-  fm_x3_place(causal, C::SLOTS, blk, bh);
+  fm_x3_place(causal, A.first != 0, C::SLOTS, blk, bh);
   const int t0 = blk * QW, lo = t0 + 32 * own;
   const float qf = fm_norm_factor(A.q_fold, bh, lane), qs = A.sc * qf * R::UP, ks_ = A.sc * fm_norm_factor(A.k_fold, bh, lane) * R::UP;
   const int send = causal && t0 + QW < A.nk ? t0 + QW : A.nk;
@@ -679,7 +680,7 @@ FM_DEVICE void fm_x3_dkv(const X3Args<TIO>& A, uint16_t* Vs, int* bad, const int
   const int wave = FM_UNIFORM(tid >> 6), own = wave / SPLIT, sub = wave % SPLIT;
   const bool causal = A.causal != 0;
   int blk, bh;
-  fm_x3_place(false, C::SLOTS, blk, bh);
+  fm_x3_place(false, false, C::SLOTS, blk, bh);
   const int t0 = blk * QW, lo = t0 + 32 * own;
   const float kf = fm_norm_factor(A.k_fold, bh, lane), ks_ = A.sc * kf * R::UP, qs = A.sc * fm_norm_factor(A.q_fold, bh, lane) * R::UP;
   const int sbeg = causal ? t0 : 0, nst = (A.nq - sbeg + KT - 1) / KT;
