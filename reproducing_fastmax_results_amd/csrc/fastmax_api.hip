@@ -514,15 +514,12 @@ template <typename TIO, typename E> void tok_common(TokArgs<TIO, E>& a, const Fa
 }
 
 // Launches that go with two groups of wavefronts per workgroup (GRP in fm_tok.h), by their number of workgroups on the chip's 256 CUs:
-// without the causal mask, and the forward of heads of 32 (the others under the mask: half_blocks, which is asked first).
-// At one workgroup per CU or less every kernel gains (whole calls, microseconds, one group and two; forward of 1 x 8 heads of 64, 4096
-// tokens 54 -> 41.5, of 2 x 8 of 2048 32 -> 27, unmasked 54 -> 45; D = 32 23 -> 19; D = 128 53 -> 48.5; a step with dQ so 174 -> 165,
-// with dK + dV so 174 -> 166).  The causal forward gains up to two per CU where its chains are long, since the light workgroups leave
-// room (16 heads of 3001 tokens 44 -> 37.6, 512 workgroups 61 -> 52 and 40 -> 36; 12 heads of 4096 62.8 -> 63.2; D = 32 25 -> 23; at
-// 512 tokens 19.5 -> 20.0; unmasked 55 -> 55).  Past that the registers hold fewer wavefronts in pairs of groups than in single ones:
-// forward at 1024 workgroups 38 -> 44, dQ at 384 145 -> 145 and 245 -> 253, dK + dV unmasked at 256 191 -> 191 and 114 -> 115.5, at 128
-// 96 -> 93.  Heads of 128 (the step at 256 workgroups): dQ 163 -> 158.5, unmasked 189 -> 187, at 128
-// workgroups 152 -> 147; dK + dV would spill (187 -> 326); and only up to 256 (forward at 512 65 -> 72).
+// without the causal mask, and the causal forward of heads of 32 (the others under the mask: half_blocks).
+// At one workgroup per CU or less every kernel gains (whole calls, microseconds, one group and two; unmasked forward of 1 x 8 heads of 64, 4096
+// tokens 54 -> 45, causal at D = 32 23 -> 19).  The causal forward gains up to two per CU where its chains are long, since the light workgroups leave
+// room (D = 32, 16 heads of 3001 tokens 25 -> 23; at 512 tokens none; unmasked 55 -> 55).  Past that the registers hold fewer wavefronts in pairs of groups
+// than in single ones: dK + dV unmasked at 256 191 -> 191 and 114 -> 115.5, at 128 96 -> 93.  Heads of 128, unmasked, the step at 256 workgroups 189 -> 187;
+// their dK + dV would spill (187 -> 326).
 enum { FM_GRP_PV, FM_GRP_DS, FM_GRP_DV };
 #if defined(FM_HOSTSIM)
 // The CPU tests run launches of a few workgroups, which all go with two groups: set, they go with one, as larger launches do.
@@ -533,8 +530,8 @@ inline bool two_groups(int kind, int dh, int64_t workgroups, bool causal, int n_
 #if defined(FM_HOSTSIM)
   if (fm_hostsim_one_group) return false;
 #endif
-  if (kind == FM_GRP_PV) return workgroups <= (causal && dh <= 64 && n_str >= 1024 ? 512 : 256);
-  return workgroups <= (kind == FM_GRP_DV && !causal ? 128 : 256);      // (dK + dV of heads of 128 is not built so)
+  if (causal) return kind == FM_GRP_PV && dh == 32 && workgroups <= (n_str >= 1024 ? 512 : 256);
+  return workgroups <= (kind == FM_GRP_DV ? 128 : 256);                 // (dK + dV of heads of 128 is not built so)
 }
 
 // Launches under the causal mask that go with blocks of 64 own tokens (HALF in fm_tok.h), by their number of blocks of 128.  Whole calls,
@@ -680,7 +677,8 @@ template <typename TIO> X3Args<TIO> x3_args(const FastmaxDesc* d, const Plan& p,
 // longer the heads are: hence the 4.  Forward and backward in four and in eight, causal: 24 heads of 640 tokens (480
 // tiles) 32.9 and 74.5, 22.5 and 63.2 us, 15 of 777 (375) 28.4 and 78.6, 26.0 and 76.8, 24 of 400 (312) 21.1 and 53.5, 21.1 and 50.8, 12 of 1030 (396)
 // 33.0 and 93.4, 31.0 and 92.7; 11 of 777 (275) 25.5 and 72.7, 25.3 and 76.0, 9 of 1300 (369) 36.6 and 106, 36.9 and 111; unmasked, 17 of 500 (272) 32.9 and 70.9,
-// 21.1 and 56.6.
+// 21.1 and 56.6.  Of 48 problems of 260 to 420 tiles (9 to 90 heads, masked and not) the rule takes the slower one twice: 40 causal heads of 220 (6 %), 24
+// of 350 (1 %).
 inline int x3_waves(int kind, int dh, int split, int n_str, int n_own, int bh, bool causal) {
   if (kind == 2) return 8;
   if (dh != 64 || split == 1) return 4;

@@ -26,7 +26,7 @@
 // a block of 64 tokens that is not zero is at least 2^-14 of the tensor's largest, and so is held to 2^-25 of itself.  (gh: whole rows
 // and blocks may be smaller, they add little to sums over rows; a column may not lie in them alone.)  A workgroup whose tensors do not
 // keep to that, one whose weights may pass 65504 (fm_x2_weights) and one with a sum that is not finite make their rows as fm_x3.h does (and so,
-// where those sums are not finite either, or where fm_x3.h's planes would lose a coefficient, with fp32 matrix products).
+// where those sums are not finite either, with fp32 matrix products).
 #pragma once
 #include "fm_x3.h"
 #include <cmath>
@@ -321,7 +321,8 @@ FM_DEVICE X3Coef fm_x2_dcoef(float a1, float a2, int ew, int ds, int es) {
 // Coefficients that these kernels take; ew as above.  A score too small to be seen beside a0 is the whole of f'(s) where a1 is zero.  And f(s) is
 // to stay away from zero (a0 / 2 at least: a1^2 <= 2 a0 a2, as the Taylor weights have it): weights of both signs cancel in the denominators and
 // leave the roundings of the scores, which are two planes' there.  (Order 1, q and k with a common component that takes weights through zero,
-// 176 heads of 780 tokens: o off by 9e-5, three planes 1.3e-5; 32 of 7000, D = 32, 3e-4 and 5e-5.)
+// 176 heads of 780 tokens: o off by 9e-5, three planes 1.3e-5; 32 of 7000, D = 32, 3e-4 and 5e-5.)  So a2 is at least a0 / 512, and fm_x3.h's planes, which
+// make what these kernels leave, do not lose it (see fm_x3_coef_lost).
 inline bool x2_coefficients(float a0, float a1, float a2, int& ew) {
   const float b1 = std::fabs(a1), big = b1 > a2 ? b1 : a2;
   ew = 0;
@@ -531,10 +532,8 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(64 * NW, (DH == 32 && SPLIT == 2 ? 4 : 2)) k_x2
   FM_SYNC();
   if (FM_TID_X == 0) bad = 0;
   FM_SYNC();
-  if (!A.plain) {
-    fm_x3_fwd<float, DH, SPLIT, X3Row<DH>, NW>(FM_ARGS_AGAIN(A), reinterpret_cast<uint16_t*>(smem), &bad, FM_TID_X + FM_OPAQUE_ZERO());
-    if (!fm_x3_again(&bad)) FM_END();
-  }
+  fm_x3_fwd<float, DH, SPLIT, X3Row<DH>, NW>(FM_ARGS_AGAIN(A), reinterpret_cast<uint16_t*>(smem), &bad, FM_TID_X + FM_OPAQUE_ZERO());
+  if (!fm_x3_again(&bad)) FM_END();
   fm_x3_fwd<float, DH, SPLIT, F32Row<DH>, NW>(FM_ARGS_AGAIN(A), reinterpret_cast<uint16_t*>(smem), &bad, FM_TID_X + FM_OPAQUE_ZERO());
 }
 
@@ -652,10 +651,8 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(64 * NW, 2) k_x2_dq(X2Args A) {
   FM_SYNC();
   if (FM_TID_X == 0) bad = 0;
   FM_SYNC();
-  if (!A.plain) {
-    fm_x3_dq<float, DH, SPLIT, X3Row<DH>, NW>(FM_ARGS_AGAIN(A), reinterpret_cast<uint16_t*>(smem), &bad, FM_TID_X + FM_OPAQUE_ZERO());
-    if (!fm_x3_again(&bad)) FM_END();
-  }
+  fm_x3_dq<float, DH, SPLIT, X3Row<DH>, NW>(FM_ARGS_AGAIN(A), reinterpret_cast<uint16_t*>(smem), &bad, FM_TID_X + FM_OPAQUE_ZERO());
+  if (!fm_x3_again(&bad)) FM_END();
   fm_x3_dq<float, DH, SPLIT, F32Row<DH>, NW>(FM_ARGS_AGAIN(A), reinterpret_cast<uint16_t*>(smem), &bad, FM_TID_X + FM_OPAQUE_ZERO());
 }
 
@@ -793,9 +790,7 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(512, 2) k_x2_dkv(X2Args A) {
   FM_SYNC();
   if (FM_TID_X == 0) bad = 0;
   FM_SYNC();
-  if (!A.plain) {
-    fm_x3_dkv<float, DH, SPLIT, X3Row<DH>>(FM_ARGS_AGAIN(A), reinterpret_cast<uint16_t*>(smem), &bad, FM_TID_X + FM_OPAQUE_ZERO());
-    if (!fm_x3_again(&bad)) FM_END();
-  }
+  fm_x3_dkv<float, DH, SPLIT, X3Row<DH>>(FM_ARGS_AGAIN(A), reinterpret_cast<uint16_t*>(smem), &bad, FM_TID_X + FM_OPAQUE_ZERO());
+  if (!fm_x3_again(&bad)) FM_END();
   fm_x3_dkv<float, DH, SPLIT, F32Row<DH>>(FM_ARGS_AGAIN(A), reinterpret_cast<uint16_t*>(smem), &bad, FM_TID_X + FM_OPAQUE_ZERO());
 }
