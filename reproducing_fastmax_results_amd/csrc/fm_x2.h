@@ -532,9 +532,9 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(64 * NW, (DH == 32 && SPLIT == 2 ? 4 : 2)) k_x2
   FM_SYNC();
   if (FM_TID_X == 0) bad = 0;
   FM_SYNC();
-  fm_x3_fwd<float, DH, SPLIT, X3Row<DH>, NW>(FM_ARGS_AGAIN(A), reinterpret_cast<uint16_t*>(smem), &bad, FM_TID_X + FM_OPAQUE_ZERO());
+  fm_x3_fwd<float, DH, SPLIT, X3Row<DH>, NW, true>(FM_ARGS_AGAIN(A), reinterpret_cast<uint16_t*>(smem), &bad, FM_TID_X + FM_OPAQUE_ZERO());
   if (!fm_x3_again(&bad)) FM_END();
-  fm_x3_fwd<float, DH, SPLIT, F32Row<DH>, NW>(FM_ARGS_AGAIN(A), reinterpret_cast<uint16_t*>(smem), &bad, FM_TID_X + FM_OPAQUE_ZERO());
+  fm_x3_fwd<float, DH, SPLIT, F32Row<DH>, NW, true>(FM_ARGS_AGAIN(A), reinterpret_cast<uint16_t*>(smem), &bad, FM_TID_X + FM_OPAQUE_ZERO());
 }
 
 // ------------------------------------------------------------------------------
@@ -651,9 +651,9 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(64 * NW, 2) k_x2_dq(X2Args A) {
   FM_SYNC();
   if (FM_TID_X == 0) bad = 0;
   FM_SYNC();
-  fm_x3_dq<float, DH, SPLIT, X3Row<DH>, NW>(FM_ARGS_AGAIN(A), reinterpret_cast<uint16_t*>(smem), &bad, FM_TID_X + FM_OPAQUE_ZERO());
+  fm_x3_dq<float, DH, SPLIT, X3Row<DH>, NW, true>(FM_ARGS_AGAIN(A), reinterpret_cast<uint16_t*>(smem), &bad, FM_TID_X + FM_OPAQUE_ZERO());
   if (!fm_x3_again(&bad)) FM_END();
-  fm_x3_dq<float, DH, SPLIT, F32Row<DH>, NW>(FM_ARGS_AGAIN(A), reinterpret_cast<uint16_t*>(smem), &bad, FM_TID_X + FM_OPAQUE_ZERO());
+  fm_x3_dq<float, DH, SPLIT, F32Row<DH>, NW, true>(FM_ARGS_AGAIN(A), reinterpret_cast<uint16_t*>(smem), &bad, FM_TID_X + FM_OPAQUE_ZERO());
 }
 
 // ------------------------------------------------------------------------------

@@ -465,7 +465,8 @@ template <int DH, int NW, int SPLIT> struct X3Cfg {
 // ------------------------------------------------------------------------------
 // forward.  grid (ceil(nq / QW), bh).
 // ------------------------------------------------------------------------------
-template <typename TIO, int DH, int SPLIT, typename R, int NW>
+// FIRST: called by a kernel of fm_x2.h, whose order of blocks A.first names.
+template <typename TIO, int DH, int SPLIT, typename R, int NW, bool FIRST = false>
 FM_DEVICE void fm_x3_fwd(const X3Args<TIO>& A, uint16_t* st, int* bad, const int tid) {
   typedef X3Cfg<DH, NW, SPLIT> C;
   constexpr int NT = DH / 32, PQ = C::PQ, KT = C::KT, QW = C::QW;
@@ -473,7 +474,7 @@ FM_DEVICE void fm_x3_fwd(const X3Args<TIO>& A, uint16_t* st, int* bad, const int
   const int wave = FM_UNIFORM(tid >> 6), own = wave / SPLIT, sub = wave % SPLIT;
   const bool causal = A.causal != 0;
   int blk, bh;
-  fm_x3_place(causal, A.first != 0, C::SLOTS, blk, bh);
+  fm_x3_place(causal, FIRST && A.first != 0, C::SLOTS, blk, bh);
   const int t0 = blk * QW, lo = t0 + 32 * own;
   const float qs = A.sc * fm_norm_factor(A.q_fold, bh, lane) * R::UP, ks_ = A.sc * fm_norm_factor(A.k_fold, bh, lane) * R::UP;
   const X3Coef cf = fm_x3_coef<R>(A.a0, A.a1, A.a2);
@@ -577,7 +578,7 @@ FM_GLOBAL void FM_LAUNCH_BOUNDS2(64 * NW, (X3Cfg<DH, NW, SPLIT>::OCC)) k_x3_fwd(
 // ------------------------------------------------------------------------------
 // dQ.  grid (ceil(nq / QW), bh).  dS = (a1 + 2 a2 s) (gh . v - c), gh = dO / g, c = gh . o.
 // ------------------------------------------------------------------------------
-template <typename TIO, int DH, int SPLIT, typename R, int NW>
+template <typename TIO, int DH, int SPLIT, typename R, int NW, bool FIRST = false>
 FM_DEVICE void fm_x3_dq(const X3Args<TIO>& A, uint16_t* st, int* bad, const int tid) {
   typedef X3Cfg<DH, NW, SPLIT> C;
   constexpr int NT = DH / 32, PQ = C::PQ, KT = C::KT, QW = C::QW;
@@ -585,7 +586,7 @@ FM_DEVICE void fm_x3_dq(const X3Args<TIO>& A, uint16_t* st, int* bad, const int 
   const int wave = FM_UNIFORM(tid >> 6), own = wave / SPLIT, sub = wave % SPLIT;
   const bool causal = A.causal != 0;
   int blk, bh;
-  fm_x3_place(causal, A.first != 0, C::SLOTS, blk, bh);
+  fm_x3_place(causal, FIRST && A.first != 0, C::SLOTS, blk, bh);
   const int t0 = blk * QW, lo = t0 + 32 * own;
   const float qf = fm_norm_factor(A.q_fold, bh, lane), qs = A.sc * qf * R::UP, ks_ = A.sc * fm_norm_factor(A.k_fold, bh, lane) * R::UP;
   const int send = causal && t0 + QW < A.nk ? t0 + QW : A.nk;
