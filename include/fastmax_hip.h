@@ -67,8 +67,9 @@ enum {
  * fp32 tensors: every magnitude of fp32, infinities and NaN included, at fp32's accuracy throughout.  (Dense tiles form fp32
  * products from three bf16 parts of each factor, all 24 bits; a workgroup that meets an entry beyond about 1e31 or a sum beyond 1e23,
  * which the parts cannot hold, makes its rows a second time with fp32 products.  Long problems, whose sums round more than their
- * operands, form them from two _Float16 parts, about 23 bits, where the largest entries of the tensors' rows and columns lie
- * within 2^14 of each other; a workgroup whose tensors do not keep to that makes its rows from the three parts.)
+ * operands, form them from two _Float16 parts, 23 bits and the sign, where f(s) stays above a0 / 2 and the largest entries of the tensors' rows and
+ * columns lie within 2^14 of each other; a workgroup whose tensors do not keep to that, one whose scores may give weights beyond 65504 a0 and, causal, one of
+ * the first queries make their rows from the three parts.)
  *
  * Bits.  A call gives the same bits on every run.  The order in which a sum is added depends on how many workgroups the launch has,
  * so a batch*head slice can come out with other roundings when nq, nk or the number of slices beside it changes: one-segment

@@ -7,10 +7,10 @@
 // bf16 planes, whose exponents fit every number; its sums are rounded twice as often.
 //
 // 4 x 8 heads of 4096 tokens, D = 64, causal, fm_x3.h and here: relative error of o, dq, dk, dv against 64-bit results 3.6e-7, 4.3e-7, 4.3e-7, 3.6e-7
-// and 1.7e-7, 3.1e-7, 3.1e-7, 2.6e-7 (the forward has the registers for sums of the small terms apart: 3.0e-7 in one sum); forward 349
-// and 220 us (19 of them k_x2_range), backward 1106 and 665 (10).  A few hundred terms give the sums too few roundings for
+// and 1.5e-7, 3.1e-7, 3.1e-7, 2.6e-7 (the forward has the registers for sums of the small terms apart: 3.0e-7 in one sum); forward 349
+// and 220 us (24 of them k_x2_range), backward 1106 and 650 (16).  A few hundred terms give the sums too few roundings for
 // that (see x2_pays), and such problems stay with fm_x3.h.
-// What bounds these kernels is power: the forward keeps the matrix pipe 60 % busy at 1.9 GHz.  Copying ready-made planes to LDS past the
+// What bounds these kernels is power: the forward keeps the matrix pipe 52 % busy at 1.9 GHz.  Copying ready-made planes to LDS past the
 // registers, without bank conflicts, took 14 % of its cycles away and gave them back as a clock of 1.75 GHz.
 //
 // What the powers of two are taken from.
@@ -26,7 +26,9 @@
 // a block of 64 tokens that is not zero is at least 2^-14 of the tensor's largest, and so is held to 2^-25 of itself.  (gh: whole rows
 // and blocks may be smaller, they add little to sums over rows; a column may not lie in them alone.)  A workgroup whose tensors do not
 // keep to that, one whose weights may pass 65504 (fm_x2_weights) and one with a sum that is not finite make their rows as fm_x3.h does (and so,
-// where those sums are not finite either, with fp32 matrix products).
+// where those sums are not finite either, with fp32 matrix products).  What that costs, forward and backward, us, v's first row 1e-9 of the others, and
+// the same problem on fm_x3.h's own launches: 32 heads of 4096 tokens 368 and 1169, 365 and 1243, 12 of 4096 205 and 632, 170 and 543, 4 of 2100 75 and 205,
+// 53 and 153, unmasked 16 of 1024 48 and 122, 35 and 100.
 #pragma once
 #include "fm_x3.h"
 #include <cmath>

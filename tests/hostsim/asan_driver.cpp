@@ -146,6 +146,7 @@ static int run_norm_pair(int bh, int n0, int n1, int d, int dtype, int centre) {
   return st;
 }
 extern "C" void fastmax_hostsim_one_group(int on);
+extern "C" void fastmax_hostsim_x2(int split);
 int main() {
   int bad = 0;
   bad |= run_pointwise(3, 333, 64, FASTMAX_BF16);
@@ -195,6 +196,15 @@ int main() {
   bad |= run(1, 70, 64, 2, 0, FASTMAX_BF16, 1, opt(0, 1, FASTMAX_FLAG_F32_COMPUTE));
   bad |= run(1, 70, 64, 2, 0, FASTMAX_F32, 1, opt(0, 1, 0, 0, 1));
   bad |= run(1, 70, 32, 2, 0, FASTMAX_F32, 0, opt(0, 0, 0, 0, 1));
+  // fp32 on two planes (fm_x2.h): one, two and four wavefronts to a tile, square and not, normalised, refused
+  for (int split : {1, 2, 4}) {
+    fastmax_hostsim_x2(split);
+    bad |= run(1, 130, 64, 2, 0, FASTMAX_F32, 1, opt(0, 1, FASTMAX_FLAG_FORCE_DENSE));
+    bad |= run(2, 70, 32, 2, 0, FASTMAX_F32, 0, opt(97, 0, FASTMAX_FLAG_FORCE_DENSE));
+    bad |= run(1, 97, 64, 2, 0, FASTMAX_F32, 1, opt(0, 1, FASTMAX_FLAG_FORCE_DENSE, 1));
+    bad |= run(1, 70, 32, 2, 0, FASTMAX_F32, 1, opt(0, 0, FASTMAX_FLAG_FORCE_DENSE, 0, 1));
+  }
+  fastmax_hostsim_x2(0);
   // at most 64 tokens (fm_small.h): normalised by the kernels, causal with more keys, fp32 arithmetic, the second pass
   for (int dtype : {FASTMAX_F32, FASTMAX_BF16})
     for (int n : {1, 33, 50, 64}) bad |= run(2, n, n == 50 ? 32 : 64, 2, 0, dtype, 1, opt(0, 0, 0, 1));

@@ -439,6 +439,36 @@ def test_numbers_within_two_planes(lib, bh, n, d, mask):
     check_numbers_within_two_planes(lib, bh, n, d, DEV, mask=mask, seed=144)
 
 
+@pytest.mark.parametrize("bh,n,d", [(65, 700, 128), (129, 513, 64), (129, 513, 32)])
+def test_causal_launches_past_blocks_of_64(lib, bh, n, d):
+    """Causal bf16 launches of more workgroups than blocks of 64 own tokens are for: one group of wavefronts, forward, dQ and dK + dV."""
+    print(f"case past blocks of 64 bh={bh} n={n} d={d}", flush=True)
+    check_forward_backward(lib, bh, n, d, torch.bfloat16, DEV, mask=True, p=2, seed=149, saved=True)
+
+
+@pytest.mark.parametrize("bh,n,d", [(46, 1540, 64), (88, 1540, 64), (88, 1540, 32), (2, 6200, 64)])
+def test_two_planes_jacobian_of_the_normalisation(lib, bh, n, d):
+    """The Jacobian's partial sums, one per workgroup: blocks of 128 and 256 queries, and of 64; of 128, 256 and 64 keys.  Two heads against autograd
+    in float64 on the GPU."""
+    from oracle import fastmax_oracle as O
+    print(f"case two planes with the normalisation's Jacobian bh={bh} n={n} d={d}", flush=True)
+    lim = 4.0
+    q, k, v, go = make_inputs(bh, n, n, d, torch.float32, DEV, 150)
+    keys = lib.maxnorm_stats(q, k)
+    kw = dict(mask=True, inv_tau=1.0, p=2, norm=(*keys, lim, True))
+    o, g, ws = lib.forward(q, k, v, save=True, **kw)
+    got = (o, *lib.backward(q, k, v, o, g, go, saved=ws, **kw))
+    for b in (0, bh - 1):
+        x = [t[b:b + 1].double().requires_grad_(True) for t in (q, k, v)]
+        s = O.normalize_lim(x[0], lim)[0] @ O.normalize_lim(x[1], lim)[0].T
+        w = (1.0 + s + 0.5 * s * s).tril()
+        out = (w @ x[2][0] / w.sum(1, keepdim=True))[None]
+        ref = (out, *torch.autograd.grad(out, x, go[b:b + 1].double()))
+        errs = [float((y[b:b + 1].double() - r).norm() / r.norm()) for y, r in zip(got, ref)]
+        print("errors o dq dk dv", " ".join(f"{e:.2e}" for e in errs), flush=True)
+        assert max(errs) < 2e-6, errs
+
+
 def fp32_errors(lib, q, k, v, go, heads, a2=0.5, **kw):
     """Relative errors of o, g, dq, dk, dv of some heads against 64-bit results on the GPU (order 2, weights 1 + s + a2 s^2)."""
     kw["a2"] = a2
