@@ -215,6 +215,13 @@ inline bool tiles_pay_causal(const FastmaxDesc* d) {
   return n <= (d->d == 64 ? 8192 : 7168);
 }
 
+// Forwards alone past that, where the chip is not full: o is as accurate on tiles to 16384 tokens and beyond.
+inline bool tiles_hold_forward(const FastmaxDesc* d) {
+  int ew;
+  return d->dtype == FASTMAX_F32 && d->mask && d->d == 64 && d->p == 2 && d->chunk == 0 && !(d->flags & FASTMAX_FLAG_FORCE_MOMENTS) &&
+         x2_coefficients(d->a0, d->a1, d->a2, ew) && d->nq <= 16384 && int64_t(d->bh) * ((int64_t(d->nq) + 127) / 128) < 512;
+}
+
 int validate(const FastmaxDesc* d) {
   if (!d) return FASTMAX_ERR_NULL;
   if (d->dtype != FASTMAX_F32 && d->dtype != FASTMAX_BF16) return FASTMAX_ERR_DTYPE;
@@ -1132,13 +1139,20 @@ int fastmax_forward_static(const FastmaxDesc* desc, const void* q, const void* k
   // a few queries whose general route needs more than the buffer take theirs, which needs next to nothing
   const bool few = need > size_t(FASTMAX_STATIC_SCRATCH_BYTES) && desc->nq <= 16 && few_possible(desc) &&
                    few_bytes(desc) <= size_t(FASTMAX_STATIC_SCRATCH_BYTES);
-  if (need > size_t(FASTMAX_STATIC_SCRATCH_BYTES) && !few) return FASTMAX_ERR_TOO_LARGE;
+  // and causal fp32 problems of few heads whose states do not fit stay on dense tiles for twice as long as others: it is dv that asks for states
+  // there (see tiles_pay_causal), and this is a forward
+  FastmaxDesc dense = *desc;
+  if (need > size_t(FASTMAX_STATIC_SCRATCH_BYTES) && !few) {
+    if (!tiles_hold_forward(desc)) return FASTMAX_ERR_TOO_LARGE;
+    dense.flags |= FASTMAX_FLAG_FORCE_DENSE;
+    if (fastmax_workspace_bytes(&dense, &need, nullptr) || need > size_t(FASTMAX_STATIC_SCRATCH_BYTES)) return FASTMAX_ERR_TOO_LARGE;
+  }
   void* ws = nullptr;
   const int sa = fm_static_scratch(&ws);
   if (sa) return sa;
   // nothing in the scratch has to start at zero: every kernel of the forward writes what a later one reads
   if (few) return forward_few(desc, q, k, v, o, g, ws, size_t(FASTMAX_STATIC_SCRATCH_BYTES), hip_stream);
-  return fastmax_forward(desc, q, k, v, o, g, ws, size_t(FASTMAX_STATIC_SCRATCH_BYTES), hip_stream);
+  return fastmax_forward(&dense, q, k, v, o, g, ws, size_t(FASTMAX_STATIC_SCRATCH_BYTES), hip_stream);
 }
 
 static int backward_one(const FastmaxDesc* desc, const void* q, const void* k, const void* v, const void* o,

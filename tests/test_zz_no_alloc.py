@@ -74,3 +74,14 @@ def test_static_scratch_takes_a_few_queries_on_many_keys(lib):
     lib.forward_static(q, k, v, o2, g2, **kw)
     assert float((o1.double() - o2.double()).norm() / o1.double().norm()) < 4e-3
     assert float((g1.double() - g2.double()).norm() / g1.double().norm()) < 1e-3
+
+
+def test_static_scratch_takes_long_fp32_problems_of_few_heads(lib):
+    """States of 9000 tokens do not fit the buffer; the forward alone stays on dense tiles, whose bits it gives."""
+    gen = torch.Generator().manual_seed(5)
+    q, k, v = (torch.randn(4, 9000, 64, generator=gen).to(DEV) for _ in range(3))
+    kw = dict(mask=True, inv_tau=1.0 / 64, p=2)
+    o, g = lib.forward(q, k, v, flags=_capi.FLAG_FORCE_DENSE, **kw)
+    o2, g2 = torch.empty_like(o), torch.empty_like(g)
+    lib.forward_static(q, k, v, o2, g2, **kw)
+    assert torch.equal(o, o2) and torch.equal(g, g2)
