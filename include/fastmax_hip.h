@@ -150,7 +150,8 @@ int fastmax_forward(const FastmaxDesc* desc, const void* q, const void* k, const
  * process ends); the call allocates and frees nothing.  A problem whose forward_bytes
  * (fastmax_workspace_bytes) exceed that size is refused with FASTMAX_ERR_TOO_LARGE before anything is
  * launched, unless it has at most 16 queries (nq) and takes the kernels for a few queries, which need no
- * such workspace.  All calls on one GPU share that GPU's buffer: calls that overlap in time on one GPU (two
+ * such workspace, or is a causal fp32 problem of order 2 with D = 64, at most 16384 queries and few batch*heads, which goes as with
+ * FASTMAX_FLAG_FORCE_DENSE.  All calls on one GPU share that GPU's buffer: calls that overlap in time on one GPU (two
  * streams, two threads) race and give wrong results; calls on one stream are ordered and safe.  The
  * buffer keeps the last call's contents; nothing in it needs clearing between calls.
  * FASTMAX_FLAG_SAVE_FOR_BACKWARD is honoured (the saved data then lives in the static buffer, until the
